@@ -180,6 +180,23 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_native = None
+
+
+def native():
+    """The extension behind the module-level calls (``csrc/native.cpp``): takes tensors as they are and returns ``None``
+    for whatever it leaves to the Python path of the caller."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as ext
+        except ImportError as e:
+            raise RuntimeError(f"daisy_amd/_native.so is not usable ({e}); build it with: python -m daisy_amd.build") from e
+        _native = ext
+    return _native
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load().daisy_last_error().decode("utf-8", "replace")

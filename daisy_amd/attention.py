@@ -24,7 +24,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from . import ops
+from . import _lib, ops
 from .functional import NORM_EPS_BF16, init_linear, norm
 from .kv_cache import RingContext
 
@@ -313,8 +313,12 @@ STEP_ROWS_KERNEL_MAX = 4
 
 
 def step_linear(x: Tensor, w: Tensor) -> Tensor:
-    """``F.linear(x, w)`` for the activations of a decode step (models/daisy/attention.py:119-120, :201).
-    The kernel has no backward: where autograd would record the product, the library op stays."""
+    """``F.linear(x, w)`` for the activations of a decode step or a short prompt (models/daisy/attention.py:119-120, :201).
+    The kernels have no backward: where autograd would record the product, the library op stays."""
+    if x.is_cuda:
+        y = _lib.native().linear(x, w, None, STEP_ROWS_KERNEL_MAX, 0)
+        if y is not None:
+            return y
     if (x.numel() <= STEP_ROWS_KERNEL_MAX * x.shape[-1] and ops.linear_rows_ok(x, w)
             and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
         return ops.linear_rows(x, w)
@@ -414,6 +418,14 @@ class CausalSelfAttention(nn.Module):
             mask = WindowMask(mask.window, mask.doc_start.to(x.device), mask.kv_out)
         dest = kv_out if kv_out is not None else mask.kv_out
         if self._fused_prep_ok():
+            rot = self.rotary
+            k_dest, v_dest = dest if dest is not None else (None, None)
+            fast = _lib.native().layer_prefill(
+                x, self.qkvo_w, rot.cos, rot.sin, self.num_heads, self.head_dim, mask.window or 0, mask.doc_start,
+                ve if self.receives_ve else None, self.g_ve, k_dest, v_dest, float(self.attn_scale), NORM_EPS_BF16,
+                STEP_ROWS_KERNEL_MAX, want_q)
+            if fast is not None:
+                return fast
             q, k_rot, v = self._project_qkv_fused(x, ve, 0, *(dest or (None, None)))
             o, _ = ops.prefill_attention(q, k_rot, v, window=mask.window, scale=self.attn_scale, doc_start=mask.doc_start)
             y = F.linear(o.view(B, T, self.m_dim), self.qkvo_w[3])
@@ -561,6 +573,13 @@ class CausalSelfAttention(nn.Module):
         rows' way into slot ``pos % W`` and the attention over the ring all happen in
         ``ops.attn_step``.  Returns the new rows as views of the ring, or ``None, None`` when only
         the device knows the position."""
+        rot = self.rotary
+        fast = _lib.native().layer_step(x, self.qkvo_w, ring.k, ring.v, pos, rot.cos, rot.sin, ve if self.receives_ve else None,
+                                        self.g_ve, ring.status if isinstance(pos, Tensor) else None, float(self.attn_scale),
+                                        NORM_EPS_BF16, STEP_ROWS_KERNEL_MAX)
+        if fast is not None:
+            ring.mark_written()
+            return fast
         B, H, D = x.size(0), self.num_heads, self.head_dim
         x = x.to(self.qkvo_w.dtype)
         ve_rows = gate = None

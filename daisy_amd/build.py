@@ -15,7 +15,7 @@ from concurrent.futures import ThreadPoolExecutor
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_NAME = "libdaisy_hip.so"
 LIB_PATH = os.path.join(CSRC, LIB_NAME)
-SOURCES = ["abi.hip", "decode.hip", "prefill.hip", "kda.hip", "kda_step.hip", "prep.hip", "kimi.hip", "linear.hip", "layer_step.hip"]
+SOURCES = ["abi.hip", "decode.hip", "prefill.hip", "kda.hip", "kda_step.hip", "prep.hip", "proj.hip", "kimi.hip", "linear.hip", "layer_step.hip"]
 # Diagnostic kernels of the benchmark (matrix-pipe and read-stream ceilings): not part of the product.  Their source
 # sits next to bench.py at the repository root and is built into a library of its own there, which only bench.py loads.
 ROOT = os.path.dirname(os.path.dirname(CSRC))
@@ -60,6 +60,39 @@ def _compile(src: str, verbose: bool) -> str:
     return obj
 
 
+# The call path from torch tensors to the kernels (a CPython extension linked against the product library and torch).
+NATIVE_SOURCE = os.path.join(CSRC, "native.cpp")
+NATIVE_PATH = os.path.join(os.path.dirname(CSRC), "_native.so")
+
+
+def _compile_native(verbose: bool) -> str:
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    obj = os.path.splitext(NATIVE_SOURCE)[0] + ".o"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for inc in (*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]):
+        cmd += ["-isystem", inc]
+    _run([*cmd, "-c", NATIVE_SOURCE, "-o", obj], "native.cpp", verbose)
+    return obj
+
+
+def _link_native(obj: str, verbose: bool) -> None:
+    import torch
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    _run(["g++", "-shared", "-o", NATIVE_PATH, obj, "-L", CSRC, f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN/csrc", "-L", lib,
+          "-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lc10"], "native.cpp", verbose)
+
+
+def _run(cmd, what: str, verbose: bool) -> None:
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"building {what} failed:\n{r.stdout}\n{r.stderr}")
+
+
 def _link(objs, out: str, verbose: bool) -> None:
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", *objs, "-o", out]
     if verbose:
@@ -76,9 +109,11 @@ def build(verbose: bool = True, sources=None) -> str:
     every = srcs + ([PROBE_SOURCE] if os.path.exists(PROBE_SOURCE) else [])
     if "abi.hip" not in every:
         every.append("abi.hip")
-    with ThreadPoolExecutor(max_workers=min(4, len(every))) as ex:
+    with ThreadPoolExecutor(max_workers=min(6, len(every) + 1)) as ex:
+        native = ex.submit(_compile_native, verbose)
         objs = dict(zip(every, ex.map(lambda s: _compile(s, verbose), every)))
     _link([objs[s] for s in srcs], LIB_PATH, verbose)
+    _link_native(native.result(), verbose)
     if PROBE_SOURCE in objs:
         _link([objs["abi.hip"], objs[PROBE_SOURCE]], PROBE_LIB_PATH, verbose)
     return LIB_PATH

@@ -6,7 +6,7 @@
 #include <stdio.h>
 #include <stdarg.h>
 
-#include "../../include/daisy_hip.h"
+#include "internal.h"
 
 namespace daisy {
 
@@ -36,6 +36,13 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
 }
 __device__ __forceinline__ float round_bf16(float a) {
   return bf16lo_to_f32(pack_bf16x2(a, 0.f));
+}
+
+// The value of a gate on the device.
+__device__ __forceinline__ float gate_value(const GateSource& g) {
+  if (g.kind == GateSource::kValue) return *(const float*)g.p;
+  const float x = g.kind == GateSource::kLogitBf16 ? bf16lo_to_f32(*(const uint16_t*)g.p) : *(const float*)g.p;
+  return round_bf16(1.f / (1.f + expf(-x)));
 }
 
 // Unpack 8 bf16 held in a 16-byte register quad into 8 floats.

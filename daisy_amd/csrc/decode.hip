@@ -42,8 +42,9 @@ struct DecodeParams {
   // and k_new at the step's position, value-embedding mix): the position when it is a launch
   // argument, the rotation tables, and the optional second value row with its gate.
   int pos_host; const float* cos_tab; const float* sin_tab; int table_rows; float eps;
-  const uint16_t* ve; int64_t ve_sb, ve_sh; const float* gate;
+  const uint16_t* ve; int64_t ve_sb, ve_sh; GateSource gate;
   int32_t* status;   // optional: receives DAISY_STATUS_* bits the kernel raises (never cleared by it)
+  uint16_t* k_rows; uint16_t* v_rows;   // optional: bf16 copies of the new rows, [B, H, D]
 };
 
 struct DecodeRange { int n_rows, new_idx, rows_per_split; };
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(DecodeParams p) 
     vn_raw = *reinterpret_cast<const u32x4*>((holds_new ? vn_row : q_row) + dl);
     if (p.ve != nullptr) {
       ve_raw = *reinterpret_cast<const u32x4*>((holds_new ? p.ve + b * p.ve_sb + h * p.ve_sh : q_row) + dl);
-      gate = p.gate[0];
+      gate = gate_value(p.gate);
     }
   } else {
     static_assert(!F16C, "fp16 cache rows come with the kernel-side preparation only");
@@ -335,6 +336,14 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(DecodeParams p) 
         if (p.write_back) {
           *reinterpret_cast<u32x4*>(kbase + (int64_t)row * p.kc_sr) = kn_packed;
           *reinterpret_cast<u32x4*>(vbase + (int64_t)row * p.vc_sr) = vn_packed;
+        }
+        if (PREP && p.k_rows != nullptr) {
+          float f[8];
+          const int64_t at = ((int64_t)b * p.H + h) * D + dl;
+          unpack8_cache<F16C>(kn_packed, f);
+          *reinterpret_cast<u32x4*>(p.k_rows + at) = pack8(f);
+          unpack8_cache<F16C>(vn_packed, f);
+          *reinterpret_cast<u32x4*>(p.v_rows + at) = pack8(f);
         }
       }
       float kf[8];
@@ -601,27 +610,20 @@ extern "C" size_t daisy_decode_workspace_bytes(int B, int H, int D, int n_rows, 
   return (size_t)B * H * ns * (D + 2) * sizeof(float);
 }
 
-// What daisy_attn_step_fwd adds to a decode launch: the kernel prepares the rows itself.
-struct StepPrep {
-  int pos_host; const float* cos; const float* sin; int table_rows; float eps;
-  const void* ve; const int64_t* ve_strides; const float* gate;
-  int cache_f16; int32_t* status;
-};
-
+namespace daisy {
 // Shared by the entry points.  With pos_dev set, n_rows is the ring's slot count (it fixes the
 // split count and the grid) and the kernel derives the live rows and the new row's slot from *pos_dev.
-static int decode_launch(const void* q, const int64_t* q_strides,
-                         const void* k_new, const int64_t* k_new_strides,
-                         const void* v_new, const int64_t* v_new_strides,
-                         void* k_cache, const int64_t* k_cache_strides,
-                         void* v_cache, const int64_t* v_cache_strides,
-                         const float* cos_row, const float* sin_row,
-                         void* o, const int64_t* o_strides,
-                         int B, int H, int D,
-                         int n_rows, int new_idx, const int32_t* pos_dev, int write_back,
-                         float scale, int nsplit,
-                         void* workspace, size_t workspace_bytes, void* stream, const StepPrep* prep = nullptr,
-                         bool f32_io = false) {
+int decode_launch(const void* q, const int64_t* q_strides,
+                  const void* k_new, const int64_t* k_new_strides,
+                  const void* v_new, const int64_t* v_new_strides,
+                  void* k_cache, const int64_t* k_cache_strides,
+                  void* v_cache, const int64_t* v_cache_strides,
+                  const float* cos_row, const float* sin_row,
+                  void* o, const int64_t* o_strides,
+                  int B, int H, int D,
+                  int n_rows, int new_idx, const int32_t* pos_dev, int write_back,
+                  float scale, int nsplit,
+                  void* workspace, size_t workspace_bytes, void* stream, const StepPrep* prep, bool f32_io) {
   DAISY_CHECK_ARG(q && k_new && v_new && o, "decode: q, k_new, v_new and o must be non-NULL");
   DAISY_CHECK_ARG(q_strides && k_new_strides && v_new_strides && o_strides, "decode: stride arrays must be non-NULL");
   DAISY_CHECK_ARG(B > 0 && H > 0, "decode: B=%d and H=%d must be positive", B, H);
@@ -668,10 +670,11 @@ static int decode_launch(const void* q, const int64_t* q_strides,
   p.rows_per_split = (n_rows + p.nsplit - 1) / p.nsplit;
   p.pos_dev = pos_dev; p.ring_rows = n_rows;
   p.pos_host = 0; p.cos_tab = p.sin_tab = nullptr; p.table_rows = 0; p.eps = 0.f;
-  p.ve = nullptr; p.ve_sb = p.ve_sh = 0; p.gate = nullptr; p.status = nullptr;
+  p.ve = nullptr; p.ve_sb = p.ve_sh = 0; p.gate = GateSource{nullptr, 0}; p.status = nullptr; p.k_rows = p.v_rows = nullptr;
   if (prep != nullptr) {
     p.pos_host = prep->pos_host; p.cos_tab = prep->cos; p.sin_tab = prep->sin; p.table_rows = prep->table_rows;
     p.eps = prep->eps; p.ve = (const uint16_t*)prep->ve; p.gate = prep->gate; p.status = prep->status;
+    p.k_rows = prep->k_rows; p.v_rows = prep->v_rows;
     if (prep->ve) { p.ve_sb = prep->ve_strides[0]; p.ve_sh = prep->ve_strides[1]; }
   }
   p.scale_log2e = scale * kLog2e;
@@ -714,6 +717,35 @@ static int decode_launch(const void* q, const int64_t* q_strides,
   }
   return DAISY_OK;
 }
+
+// Everything CausalSelfAttention.step does between its two projections; the checks of daisy_attn_step_fwd.
+int attn_step_launch(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                     const void* v, const int64_t* v_strides, void* k_cache, const int64_t* k_cache_strides,
+                     void* v_cache, const int64_t* v_cache_strides, void* o, const int64_t* o_strides,
+                     int B, int H, int D, int ring_rows, const int32_t* pos_dev, float scale, int nsplit,
+                     void* workspace, size_t workspace_bytes, void* stream, const StepPrep& prep) {
+  const int pos = prep.pos_host, table_rows = prep.table_rows;
+  DAISY_CHECK_SUPPORTED(D == 64 || D == 128, "attn_step: head_dim %d not supported (64 or 128)", D);
+  DAISY_CHECK_ARG(k_cache && v_cache && k_cache_strides && v_cache_strides, "attn_step: the ring cache is required");
+  DAISY_CHECK_ARG(ring_rows >= 1, "attn_step: ring_rows=%d must be >= 1", ring_rows);
+  DAISY_CHECK_ARG(prep.cos && prep.sin && table_rows >= 1, "attn_step: the rotary tables are required");
+  DAISY_CHECK_ARG((prep.ve == nullptr) == (prep.gate.p == nullptr), "attn_step: ve and gate must both be given or both NULL");
+  DAISY_CHECK_ARG(prep.ve == nullptr || prep.ve_strides != nullptr, "attn_step: ve needs ve_strides");
+  DAISY_CHECK_ARG(pos_dev != nullptr || (pos >= 0 && pos < table_rows),
+                  "attn_step: position %d outside the rotary tables (%d rows)", pos, table_rows);
+  auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
+  DAISY_CHECK_ARG(al16(prep.ve) && (!prep.ve || (prep.ve_strides[0] % 8 == 0 && prep.ve_strides[1] % 8 == 0)),
+                  "attn_step: ve must be 16-byte aligned with strides that are multiples of 8 elements");
+  // With the position on the host the live rows and the slot are launch arguments (and the split
+  // count follows the live rows); with the position on the device the kernel derives them.
+  const int n_rows = pos_dev ? ring_rows : (pos + 1 < ring_rows ? pos + 1 : ring_rows);
+  const int new_idx = pos_dev ? 0 : pos % ring_rows;
+  return decode_launch(q, q_strides, k, k_strides, v, v_strides, k_cache, k_cache_strides, v_cache, v_cache_strides,
+                       nullptr, nullptr, o, o_strides, B, H, D, n_rows, new_idx, pos_dev, /*write_back=*/1, scale, nsplit,
+                       workspace, workspace_bytes, stream, &prep);
+}
+
+}  // namespace daisy
 
 extern "C" int daisy_decode_fwd(const void* q, const int64_t* q_strides,
                                 const void* k_new, const int64_t* k_new_strides,
@@ -858,23 +890,8 @@ extern "C" int daisy_attn_step_fwd(const void* q, const int64_t* q_strides,
                                    int B, int H, int D, int ring_rows,
                                    float scale, int nsplit,
                                    void* workspace, size_t workspace_bytes, void* stream) {
-  DAISY_CHECK_SUPPORTED(D == 64 || D == 128, "attn_step: head_dim %d not supported (64 or 128)", D);
-  DAISY_CHECK_ARG(k_cache && v_cache && k_cache_strides && v_cache_strides, "attn_step: the ring cache is required");
-  DAISY_CHECK_ARG(ring_rows >= 1, "attn_step: ring_rows=%d must be >= 1", ring_rows);
-  DAISY_CHECK_ARG(cos && sin && table_rows >= 1, "attn_step: the rotary tables are required");
-  DAISY_CHECK_ARG((ve == nullptr) == (gate == nullptr), "attn_step: ve and gate must both be given or both NULL");
-  DAISY_CHECK_ARG(ve == nullptr || ve_strides != nullptr, "attn_step: ve needs ve_strides");
-  DAISY_CHECK_ARG(pos_dev != nullptr || (pos >= 0 && pos < table_rows),
-                  "attn_step: position %d outside the rotary tables (%d rows)", pos, table_rows);
-  auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
-  DAISY_CHECK_ARG(al16(ve) && (!ve || (ve_strides[0] % 8 == 0 && ve_strides[1] % 8 == 0)),
-                  "attn_step: ve must be 16-byte aligned with strides that are multiples of 8 elements");
-  StepPrep prep{pos, cos, sin, table_rows, eps, ve, ve_strides, gate, cache_is_f16 != 0, status};
-  // With the position on the host the live rows and the slot are launch arguments (and the split
-  // count follows the live rows); with the position on the device the kernel derives them.
-  const int n_rows = pos_dev ? ring_rows : (pos + 1 < ring_rows ? pos + 1 : ring_rows);
-  const int new_idx = pos_dev ? 0 : pos % ring_rows;
-  return decode_launch(q, q_strides, k, k_strides, v, v_strides, k_cache, k_cache_strides, v_cache, v_cache_strides,
-                       nullptr, nullptr, o, o_strides, B, H, D, n_rows, new_idx, pos_dev, /*write_back=*/1, scale, nsplit,
-                       workspace, workspace_bytes, stream, &prep);
+  const StepPrep prep{pos, cos, sin, table_rows, eps, ve, ve_strides, GateSource{gate, GateSource::kValue}, cache_is_f16 != 0,
+                      status, nullptr, nullptr};
+  return attn_step_launch(q, q_strides, k, k_strides, v, v_strides, k_cache, k_cache_strides, v_cache, v_cache_strides,
+                          o, o_strides, B, H, D, ring_rows, pos_dev, scale, nsplit, workspace, workspace_bytes, stream, prep);
 }

@@ -1,0 +1,79 @@
+// Kernels of this library that the package's native glue (native.cpp) launches directly, beside the C ABI.
+// Host code only: the glue is compiled by the host compiler.
+#pragma once
+
+#include <hip/hip_runtime_api.h>
+#include <stdint.h>
+
+#include "../../include/daisy_hip.h"
+
+namespace daisy {
+
+// The value-embedding gate of a layer: sigmoid(logit) rounded to bf16, the dtype in which the mix is evaluated.
+// Either the value itself (fp32, as the C ABI takes it) or the layer's logit, which a kernel turns into the value
+// where it is needed instead of three launches of a tensor library in front of it.
+struct GateSource {
+  enum Kind { kValue = 0, kLogitF32 = 1, kLogitBf16 = 2 };
+  const void* p;
+  int kind;
+};
+
+// Everything between the QKV projection and the attention: RMS norm of q, k, v, RoPE of q, k at rows pos0 + t of the
+// tables, gate * v + (1 - gate) * ve; outputs [B, T, H, D] with {batch, token, head} strides in elements.
+struct QkvEpilogue {
+  uint16_t* q; int64_t q_sb, q_st, q_sh;
+  uint16_t* k; int64_t k_sb, k_st, k_sh;
+  uint16_t* v; int64_t v_sb, v_st, v_sh;
+  const uint16_t* ve; int64_t ve_sb, ve_st, ve_sh;
+  GateSource gate;
+  const float* cos; const float* sin;
+  int pos0, H, T;
+  float eps;
+};
+
+// y [M, N] = x [M, K] w [N, K]^T (+ bias), fp32 accumulation, one rounding.  tile: 0 = by the sizes.
+int proj_linear(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const uint16_t* bias,
+                uint16_t* y, int64_t y_sm, int M, int N, int K, hipStream_t s, int tile = 0);
+// Whether the tiled kernel is the better choice for these sizes than the library GEMM (and, for the QKV projection, than
+// the library GEMM with qkv_prep_kernel behind it).
+bool proj_wanted(int M, int N, int K);
+bool proj_qkv_wanted(int M, int N, int K);
+// The QKV projection of x [B * T, K] with its epilogue.
+int proj_qkv(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const QkvEpilogue& e,
+             int B, int K, int D, hipStream_t s, int tile = 0);
+
+// What a one-launch attention step adds to a decode launch: the kernel prepares the rows of the projection itself.
+// k_rows / v_rows: NULL, or bf16 [B, H, D] contiguous copies of the new rows as the ring holds them (an fp16 ring's
+// rows in the model's dtype, without another pass over them).
+struct StepPrep {
+  int pos_host; const float* cos; const float* sin; int table_rows; float eps;
+  const void* ve; const int64_t* ve_strides; GateSource gate;
+  int cache_f16; int32_t* status;
+  uint16_t* k_rows; uint16_t* v_rows;
+};
+int decode_launch(const void* q, const int64_t* q_strides,
+                  const void* k_new, const int64_t* k_new_strides,
+                  const void* v_new, const int64_t* v_new_strides,
+                  void* k_cache, const int64_t* k_cache_strides,
+                  void* v_cache, const int64_t* v_cache_strides,
+                  const float* cos_row, const float* sin_row,
+                  void* o, const int64_t* o_strides,
+                  int B, int H, int D,
+                  int n_rows, int new_idx, const int32_t* pos_dev, int write_back,
+                  float scale, int nsplit,
+                  void* workspace, size_t workspace_bytes, void* stream, const StepPrep* prep = nullptr,
+                  bool f32_io = false);
+int attn_step_launch(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                     const void* v, const int64_t* v_strides, void* k_cache, const int64_t* k_cache_strides,
+                     void* v_cache, const int64_t* v_cache_strides, void* o, const int64_t* o_strides,
+                     int B, int H, int D, int ring_rows, const int32_t* pos_dev, float scale, int nsplit,
+                     void* workspace, size_t workspace_bytes, void* stream, const StepPrep& prep);
+
+// qkv_prep_kernel with the gate as the layer holds it.
+int prep_launch(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                const void* v, const int64_t* v_strides, const void* ve, const int64_t* ve_strides, GateSource gate,
+                const float* cos, const float* sin, int pos0, const int32_t* pos0_dev, int table_rows, int32_t* status,
+                void* q_out, const int64_t* q_out_strides, void* k_out, const int64_t* k_out_strides,
+                void* v_out, const int64_t* v_out_strides, int B, int T, int H, int D, float eps, void* stream);
+
+}  // namespace daisy

@@ -18,7 +18,7 @@ struct PrepParams {
   const uint16_t* k; int64_t k_sb, k_st, k_sh;
   const uint16_t* v; int64_t v_sb, v_st, v_sh;
   const uint16_t* ve; int64_t e_sb, e_st, e_sh;
-  const float* gate;
+  GateSource gate;
   const float* cos; const float* sin;
   uint16_t* qo; int64_t qo_sb, qo_st, qo_sh;
   uint16_t* ko; int64_t ko_sb, ko_st, ko_sh;
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256) void qkv_prep_kernel(PrepParams p) {
   if (p.ve != nullptr) {
     // g*v + (1-g)*ve the way a bf16 tensor library evaluates it: each product, the
     // difference and the sum are separate bf16 results.
-    const float g = p.gate[0];
+    const float g = gate_value(p.gate);
     const float og = round_bf16(1.0f - g);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -137,25 +137,17 @@ __global__ __launch_bounds__(256) void qkv_prep_kernel(PrepParams p) {
   }
 }
 
-}  // namespace daisy
-
-using namespace daisy;
-
-static int prep_launch(const void* q, const int64_t* q_strides,
-                       const void* k, const int64_t* k_strides,
-                       const void* v, const int64_t* v_strides,
-                       const void* ve, const int64_t* ve_strides, const float* gate,
-                       const float* cos, const float* sin, int pos0, const int32_t* pos0_dev, int table_rows, int32_t* status,
-                       void* q_out, const int64_t* q_out_strides,
-                       void* k_out, const int64_t* k_out_strides,
-                       void* v_out, const int64_t* v_out_strides,
-                       int B, int T, int H, int D, float eps, void* stream) {
+int prep_launch(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                const void* v, const int64_t* v_strides, const void* ve, const int64_t* ve_strides, GateSource gate,
+                const float* cos, const float* sin, int pos0, const int32_t* pos0_dev, int table_rows, int32_t* status,
+                void* q_out, const int64_t* q_out_strides, void* k_out, const int64_t* k_out_strides,
+                void* v_out, const int64_t* v_out_strides, int B, int T, int H, int D, float eps, void* stream) {
   DAISY_CHECK_ARG(q && k && v && q_out && k_out && v_out, "qkv_prep: q, k, v and the three outputs must be non-NULL");
   DAISY_CHECK_ARG(q_strides && k_strides && v_strides && q_out_strides && k_out_strides && v_out_strides,
                   "qkv_prep: stride arrays must be non-NULL");
   DAISY_CHECK_ARG(B > 0 && T > 0 && H > 0, "qkv_prep: B=%d, T=%d, H=%d must be positive", B, T, H);
   DAISY_CHECK_ARG((cos == nullptr) == (sin == nullptr), "qkv_prep: cos and sin must both be given or both NULL");
-  DAISY_CHECK_ARG((ve == nullptr) == (gate == nullptr), "qkv_prep: ve and gate must both be given or both NULL");
+  DAISY_CHECK_ARG((ve == nullptr) == (gate.p == nullptr), "qkv_prep: ve and gate must both be given or both NULL");
   DAISY_CHECK_ARG(ve == nullptr || ve_strides != nullptr, "qkv_prep: ve needs ve_strides");
   DAISY_CHECK_ARG(pos0 >= 0, "qkv_prep: pos0=%d must be >= 0", pos0);
   DAISY_CHECK_SUPPORTED(D == 64 || D == 128, "qkv_prep: head_dim %d not supported (64 or 128)", D);
@@ -192,6 +184,10 @@ static int prep_launch(const void* q, const int64_t* q_strides,
   return DAISY_OK;
 }
 
+}  // namespace daisy
+
+using namespace daisy;
+
 extern "C" int daisy_qkv_prep_fwd(const void* q, const int64_t* q_strides,
                                   const void* k, const int64_t* k_strides,
                                   const void* v, const int64_t* v_strides,
@@ -201,7 +197,7 @@ extern "C" int daisy_qkv_prep_fwd(const void* q, const int64_t* q_strides,
                                   void* k_out, const int64_t* k_out_strides,
                                   void* v_out, const int64_t* v_out_strides,
                                   int B, int T, int H, int D, float eps, void* stream) {
-  return prep_launch(q, q_strides, k, k_strides, v, v_strides, ve, ve_strides, gate, cos, sin, pos0, nullptr, 0, nullptr,
+  return prep_launch(q, q_strides, k, k_strides, v, v_strides, ve, ve_strides, GateSource{gate, GateSource::kValue}, cos, sin, pos0, nullptr, 0, nullptr,
                      q_out, q_out_strides, k_out, k_out_strides, v_out, v_out_strides, B, T, H, D, eps, stream);
 }
 
@@ -217,6 +213,6 @@ extern "C" int daisy_qkv_prep_fwd_at(const void* q, const int64_t* q_strides,
   DAISY_CHECK_ARG(pos0 != nullptr, "qkv_prep_at: the device position pointer must be non-NULL");
   DAISY_CHECK_ARG(cos && sin, "qkv_prep_at: the rotary tables are required");
   DAISY_CHECK_ARG(table_rows >= T, "qkv_prep_at: table_rows=%d must cover the %d rows of the call", table_rows, T);
-  return prep_launch(q, q_strides, k, k_strides, v, v_strides, ve, ve_strides, gate, cos, sin, 0, pos0, table_rows, status,
+  return prep_launch(q, q_strides, k, k_strides, v, v_strides, ve, ve_strides, GateSource{gate, GateSource::kValue}, cos, sin, 0, pos0, table_rows, status,
                      q_out, q_out_strides, k_out, k_out_strides, v_out, v_out_strides, B, T, H, D, eps, stream);
 }

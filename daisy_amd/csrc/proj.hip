@@ -1,0 +1,338 @@
+// Projections of a few hundred activation rows for gfx950: y = x W^T on the matrix cores, and the QKV projection
+// with everything that follows it up to the attention (models/daisy/attention.py:116-135) in its epilogue.
+//
+// What bounds it.  A prompt of a few hundred tokens (or a decode step of a few dozen sequences) has too few output
+// tiles to give every compute unit several workgroups, so nothing hides a workgroup's own latencies: with one K step in
+// flight, a step lasts a memory round trip (about 0.7 us) where its matrix instructions take 0.2 us.  The kernel
+// keeps up to three K steps in flight (asynchronous global -> LDS copies; a wavefront waits with vmcnt for the oldest
+// step only), reads the operands of a step before it issues the next copies, and the tile shape follows the number of
+// tiles (kProjTiles).  Large products are bound by the matrix cores and by what the compute units can pull through the
+// L2, hence the order of the tiles (below).  Reading the operands of a step ahead of the barrier in front of it
+// was tried: 10 % slower on the small shapes, no different on the large ones.
+//
+// Operands: both x [M, K] and W [N, K] have K contiguous, so both tiles are rows of 64 or 128 bf16 in LDS, their
+// 16-byte chunks XOR-swizzled so that 16 rows read side by side fall into 16 different slots of the 256-byte bank
+// window.  v_mfma_f32_16x16x32_bf16 with W as left operand: a lane's accumulator holds four
+// consecutive output columns of one row, which go through LDS once and leave as whole rows.
+#include "common.h"
+
+#include <type_traits>
+
+namespace daisy {
+
+struct ProjParams {
+  const uint16_t* x; int64_t x_sm;     // [M, K]
+  const uint16_t* w; int64_t w_sn;     // [N, K]
+  const uint16_t* bias;                // [N] or NULL (plain epilogue)
+  uint16_t* y; int64_t y_sm;           // [M, N] (plain epilogue)
+  int M, N, K, MT, NT;
+  QkvEpilogue e;                       // QKV epilogue
+};
+
+// At most N vector-memory operations outstanding (bits 3:0 and 15:14 of the immediate) and every LDS read back.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
+}
+
+// EPI 0: y = x W^T (+ bias), bf16.  EPI 1 / 2: the QKV epilogue for heads of 64 / 128 channels.
+// WVM x WVN wavefronts; BK elements of K per step.
+template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI>
+__global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
+  constexpr int NW = WVM * WVN, NTHR = 64 * NW;
+  constexpr int WM = BM / WVM, WN = BN / WVN, MI = WM / 16, NI = WN / 16, KK = BK / 32;
+  constexpr int RB = 2 * BK, CPRW = BK / 8, RPC = 64 / CPRW;   // bytes and 16-byte chunks per tile row, rows per copy
+  constexpr int CA = BM / RPC / NW, CB = BN / RPC / NW;        // copies per wavefront and step
+  constexpr int CPW = CA + CB;
+  constexpr int ABYTES = BM * RB, STAGE = (BM + BN) * RB;
+  static_assert(CA >= 1 && CB >= 1 && MI >= 1 && NI >= 1, "every wavefront copies and multiplies");
+  static_assert(STAGES <= 4 && CPW * (STAGES - 2) < 64, "vmcnt counts to 63");
+  static_assert(STAGES * STAGE >= BM * BN * 2, "the output tile passes through the stages");
+  __shared__ __attribute__((aligned(1024))) char smem[STAGES * STAGE];
+  // swizzle of a row's chunks: 16 rows read side by side must fall into 16 slots of the 256-byte bank window
+  auto swz = [](int r) { return BK == 128 ? (r & 15) : ((r >> 1) & 7); };
+
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 15, q4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WVM, wn = wave / WVM;
+
+  // Workgroups are dealt round-robin to the 8 XCDs: an XCD takes a contiguous run of tiles, in panels of eight rows of
+  // tiles walked column by column, so that the tiles in flight on an XCD share rows of x and of W in its L2 (32 of them
+  // at a time: 8 x 4 tiles read 12 strips, a column of 32 would read 33 and be bound by the bandwidth behind the L2).
+  const int total = p.MT * p.NT, per = total >> 3, rest = total & 7;
+  const int xcd = blockIdx.x & 7, vid = xcd * per + min(xcd, rest) + (blockIdx.x >> 3);
+  const int panel = vid / (8 * p.NT), in_panel = vid - panel * 8 * p.NT, rows = min(8, p.MT - 8 * panel);
+  const int mt = 8 * panel + in_panel % rows, nt = in_panel / rows;
+  const int m0 = mt * BM, n0 = nt * BN;
+
+  // Copy j of this wavefront covers tile rows RPC (wave + NW j) ..: lane i lands at row i / CPRW, chunk position i % CPRW and
+  // fetches the chunk that belongs there.  Rows past the end re-read the last row (their results are not stored).
+  const int cr = lane / CPRW, cp = lane % CPRW;
+  int offa[CA], offb[CB];
+#pragma unroll
+  for (int j = 0; j < CA; ++j) {
+    const int r = RPC * (wave + NW * j) + cr;
+    offa[j] = 2 * (int)((min(m0 + r, p.M - 1) - m0) * p.x_sm) + 16 * (cp ^ swz(r));
+  }
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    const int r = RPC * (wave + NW * j) + cr;
+    offb[j] = 2 * (int)((min(n0 + r, p.N - 1) - n0) * p.w_sn) + 16 * (cp ^ swz(r));
+  }
+  const uint16_t* xa = p.x + (int64_t)m0 * p.x_sm;
+  const uint16_t* wb = p.w + (int64_t)n0 * p.w_sn;
+  const uint32_t lds0 = lds_address(smem) + 1024 * wave;
+  auto issue = [&](int st) {
+    const uint32_t dst = lds0 + st * STAGE;
+#pragma unroll
+    for (int j = 0; j < CB; ++j) copy16_to_lds_async(wb, offb[j], dst + ABYTES + 1024 * NW * j);
+#pragma unroll
+    for (int j = 0; j < CA; ++j) copy16_to_lds_async(xa, offa[j], dst + 1024 * NW * j);
+    xa += BK;
+    wb += BK;
+  };
+
+  f32x4 acc[NI][MI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int nk = p.K / BK;
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < nk) issue(s);
+
+  // Fragment addresses inside a stage: chunk (4 kk + q4) ^ swizzle of its row; rows 16 apart share a swizzle.
+  const uint32_t fa = lds_address(smem) + (WM * wm + ln) * RB + 16 * (q4 ^ swz(ln));
+  const uint32_t fb = lds_address(smem) + ABYTES + (WN * wn + ln) * RB + 16 * (q4 ^ swz(ln));
+  auto frag = [&](uint32_t a) { return __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)(size_t)a); };
+
+  int st = 0;
+  for (int k = 0; k < nk; ++k) {
+    // the copies of step k have landed when at most those of the steps behind it are outstanding
+    const int behind = nk - 1 - k;
+    if (STAGES == 2 || behind == 0) wait_vmcnt<0>();
+    else if (behind >= STAGES - 2) wait_vmcnt<CPW * (STAGES - 2)>();
+    else wait_vmcnt<CPW>();                  // STAGES <= 4: one step behind
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint32_t so = st * STAGE;
+    bf16x8 a[KK][NI], b[KK][MI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) a[0][i] = frag(fb + so + 16 * RB * i);
+#pragma unroll
+    for (int j = 0; j < MI; ++j) b[0][j] = frag(fa + so + 16 * RB * j);
+    __builtin_amdgcn_sched_barrier(0);
+    // every wavefront is done with step k - 1: its stage takes step k + STAGES - 1
+    if (k + STAGES - 1 < nk) issue(st == 0 ? STAGES - 1 : st - 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      if (kk + 1 < KK) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) a[kk + 1][i] = frag((fb ^ (64u * (kk + 1))) + so + 16 * RB * i);
+#pragma unroll
+        for (int j = 0; j < MI; ++j) b[kk + 1][j] = frag((fa ^ (64u * (kk + 1))) + so + 16 * RB * j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < MI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][i], b[kk][j], acc[i][j], 0, 0, 0);
+    }
+    st = st + 1 == STAGES ? 0 : st + 1;
+  }
+  __syncthreads();
+
+  // Output tile [BM][BN] bf16 in LDS, 16-byte chunks swizzled by the row.
+  constexpr int CHN = BN / 8;                      // chunks per row
+  auto tile_at = [&](int m, int c) { return smem + m * (2 * BN) + 16 * (c ^ (m & (CHN - 1))); };
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int n = WN * wn + 16 * i + 4 * q4;       // four consecutive columns
+    float bv[4] = {0.f, 0.f, 0.f, 0.f};
+    if (EPI == 0 && p.bias != nullptr) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bv[r] = bf16lo_to_f32(p.bias[min(n0 + n + r, p.N - 1)]);
+    }
+#pragma unroll
+    for (int j = 0; j < MI; ++j) {
+      const int m = WM * wm + 16 * j + ln;
+      const u32x2 v = {pack_bf16x2(acc[i][j][0] + bv[0], acc[i][j][1] + bv[1]), pack_bf16x2(acc[i][j][2] + bv[2], acc[i][j][3] + bv[3])};
+      *reinterpret_cast<u32x2*>(tile_at(m, n >> 3) + 2 * (n & 7)) = v;
+    }
+  }
+  __syncthreads();
+
+  if constexpr (EPI == 0) {
+#pragma unroll
+    for (int it = 0; it < (BM * CHN + NTHR - 1) / NTHR; ++it) {
+      const int idx = tid + NTHR * it, m = idx / CHN, c = idx % CHN;
+      if (BM * CHN % NTHR != 0 && m >= BM) break;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(tile_at(m, c));
+      if (m0 + m < p.M && n0 + 8 * c < p.N) *reinterpret_cast<u32x4*>(p.y + (int64_t)(m0 + m) * p.y_sm + n0 + 8 * c) = v;
+    }
+  } else {
+    constexpr int D = EPI == 1 ? 64 : 128, HALF = D / 2, LPR = D / 16, HPT = BN / D;
+    static_assert(BN % D == 0, "a tile holds whole heads");
+    const QkvEpilogue& e = p.e;
+    static_assert(BM * BN / 16 % 64 == 0, "whole wavefronts");
+    constexpr int PASSES = (BM * BN / 16 + NTHR - 1) / NTHR;
+#pragma unroll(PASSES < 4 ? PASSES : 4)
+    for (int it = 0; it < PASSES; ++it) {
+      // LPR lanes share one (row, head): lane c holds channels [8c, 8c + 8) and their rotation partners
+      const int idx = tid + NTHR * it, c = idx % LPR, hh = (idx / LPR) % HPT, m = idx / (LPR * HPT);
+      if (BM * BN / 16 % NTHR != 0 && m >= BM) break;
+      const int n = n0 + hh * D;
+      const bool live = m0 + m < p.M && n < p.N;
+      const int row = min(m0 + m, p.M - 1);
+      const int third = min(n / (e.H * D), 2), h = min(n / D - third * e.H, e.H - 1);
+      const int t = row % e.T, b = row / e.T;
+      float lo[8], hi[8];
+      unpack8(*reinterpret_cast<const u32x4*>(tile_at(m, hh * (D / 8) + c)), lo);
+      unpack8(*reinterpret_cast<const u32x4*>(tile_at(m, hh * (D / 8) + LPR + c)), hi);
+      // x * rsqrt(mean(x^2) + eps), rounded to bf16 like the norm's output tensor
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss += lo[i] * lo[i];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss += hi[i] * hi[i];
+      ss = group_sum<LPR>(ss);
+      const float rstd = rsqrtf(ss / (float)D + e.eps);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) { lo[i] = round_bf16(lo[i] * rstd); hi[i] = round_bf16(hi[i] * rstd); }
+      uint16_t* dst;
+      if (third < 2) {
+        const int64_t off = (int64_t)(e.pos0 + t) * HALF + 8 * c;
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          const f32x4 cs = *reinterpret_cast<const f32x4*>(e.cos + off + 4 * v), sn = *reinterpret_cast<const f32x4*>(e.sin + off + 4 * v);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float x1 = lo[4 * v + i], x2 = hi[4 * v + i];
+            lo[4 * v + i] = rope_lo(x1, x2, cs[i], sn[i]);
+            hi[4 * v + i] = rope_hi(x1, x2, cs[i], sn[i]);
+          }
+        }
+        dst = third == 0 ? e.q + b * e.q_sb + t * e.q_st + h * e.q_sh : e.k + b * e.k_sb + t * e.k_st + h * e.k_sh;
+      } else {
+        if (e.ve != nullptr) {
+          // g*v + (1-g)*ve with every product, the difference and the sum rounded to bf16
+          const float g = gate_value(e.gate), og = round_bf16(1.0f - g);
+          const uint16_t* vp = e.ve + b * e.ve_sb + t * e.ve_st + h * e.ve_sh + 8 * c;
+          float el[8], eh[8];
+          unpack8(*reinterpret_cast<const u32x4*>(vp), el);
+          unpack8(*reinterpret_cast<const u32x4*>(vp + HALF), eh);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            lo[i] = round_bf16(g * lo[i]) + round_bf16(og * el[i]);
+            hi[i] = round_bf16(g * hi[i]) + round_bf16(og * eh[i]);
+          }
+        }
+        dst = e.v + b * e.v_sb + t * e.v_st + h * e.v_sh;
+      }
+      if (live) {
+        *reinterpret_cast<u32x4*>(dst + 8 * c) = pack8(lo);
+        *reinterpret_cast<u32x4*>(dst + 8 * c + HALF) = pack8(hi);
+      }
+    }
+  }
+}
+
+// The tile shapes, and what choosing one costs.  `per_cu` workgroups of a shape fit a compute unit; one round of a
+// workgroup on every compute unit takes `one` us at K = 2048 (measured with the operands behind the L2; the time is
+// proportional to K), a round with all of them `full`.  A product of n tiles then costs about 1.5 us plus its rounds, and
+// the shape with the least cost is taken: the small ones while their tiles fit one round, the large ones from there on.
+// (M = 777, N = 4608, K = 1536: 16.6 us with 128 x 128 and 8 wavefronts, 18.6 us with 64 x 128, 24.4 us with 64 x 64,
+// 17.9 us in the library; M = 64, N = 6144, K = 2048: 7.3 us with 32 x 64, 9.7 us in the library; M = 8192,
+// N = 6144, K = 2048: 155 us with 256 x 256, 178 us with 128 x 128, 141 us in the library.)
+struct ProjTile { int code, bm, bn, bk, per_cu; float one, full; };
+constexpr ProjTile kProjTiles[] = {
+    {1, 32, 64, 128, 2, 5.8f, 8.0f},      // 4 wavefronts, 3 stages
+    {2, 64, 64, 128, 1, 7.2f, 7.2f},      // 8 wavefronts, 4 stages
+    {3, 64, 128, 128, 1, 10.3f, 10.3f},   // 8 wavefronts, 3 stages
+    {4, 64, 128, 64, 2, 12.3f, 19.0f},    // 4 wavefronts, 3 stages
+    {5, 128, 128, 64, 1, 15.8f, 15.8f},   // 8 wavefronts, 4 stages
+    {6, 128, 128, 64, 2, 20.2f, 25.3f},   // 4 wavefronts, 2 stages
+    {7, 256, 256, 64, 1, 42.0f, 42.0f},   // 8 wavefronts, 2 stages
+};
+static int proj_tile(int M, int N, int K, int head) {
+  int best = 0;
+  float least = 0.f;
+  for (const ProjTile& t : kProjTiles) {
+    if (K % t.bk != 0 || t.bn % head != 0) continue;    // (head: a tile of the QKV projection holds whole heads)
+    const int64_t n = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), round = 256 * t.per_cu;
+    const int64_t tail = n % round;
+    const float cost = (float)(n / round) * t.full + (tail > 256 ? t.full : tail > 0 ? t.one : 0.f);
+    if (best == 0 || cost < least) { best = t.code; least = cost; }
+  }
+  return best;
+}
+
+// Against the library GEMM: level or ahead (1.0 to 1.7 times as fast) up to about four million outputs, and for short
+// rows at any size; 0.9 beyond that.  With the QKV epilogue it replaces the library GEMM and qkv_prep_kernel behind it
+// (another read and write of every row, 62 us of 228 us at M = 32768, N = 3072, K = 1024), which it beats at every size.
+bool proj_wanted(int M, int N, int K) { return K % 64 == 0 && N % 8 == 0 && (K <= 512 || (int64_t)M * N <= 4300000); }
+bool proj_qkv_wanted(int M, int N, int K) { return K % 64 == 0; }
+
+template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI>
+static int launch_proj(ProjParams p, hipStream_t s) {
+  p.MT = (p.M + BM - 1) / BM;
+  p.NT = (p.N + BN - 1) / BN;
+  hipLaunchKernelGGL((proj_kernel<BM, BN, WVM, WVN, BK, STAGES, EPI>), dim3((unsigned)(p.MT * p.NT)), dim3(64 * WVM * WVN), 0, s, p);
+  DAISY_CHECK_LAUNCH("proj_kernel");
+  return DAISY_OK;
+}
+
+template <int EPI>
+static int dispatch_proj(int tile, const ProjParams& p, hipStream_t s) {
+  for (const ProjTile& t : kProjTiles)
+    DAISY_CHECK_SUPPORTED(t.code != tile || (p.K % t.bk == 0 && !(EPI == 2 && t.bn % 128 != 0)), "proj: tile %d does not serve K=%d", tile, p.K);
+  if constexpr (EPI != 2) {
+    if (tile == 1) return launch_proj<32, 64, 2, 2, 128, 3, EPI>(p, s);
+    if (tile == 2) return launch_proj<64, 64, 2, 4, 128, 4, EPI>(p, s);
+  }
+  switch (tile) {
+    case 3: return launch_proj<64, 128, 2, 4, 128, 3, EPI>(p, s);
+    case 4: return launch_proj<64, 128, 2, 2, 64, 3, EPI>(p, s);
+    case 5: return launch_proj<128, 128, 4, 2, 64, 4, EPI>(p, s);
+    case 6: return launch_proj<128, 128, 2, 2, 64, 2, EPI>(p, s);
+    case 7: return launch_proj<256, 256, 2, 4, 64, 2, EPI>(p, s);
+    default: DAISY_CHECK_SUPPORTED(false, "proj: no tile %d", tile);
+  }
+}
+
+static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+int proj_linear(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const uint16_t* bias,
+                uint16_t* y, int64_t y_sm, int M, int N, int K, hipStream_t s, int tile) {
+  DAISY_CHECK_ARG(x && w && y && M > 0 && N > 0 && K > 0, "proj_linear: NULL tensor or M=%d, N=%d, K=%d", M, N, K);
+  DAISY_CHECK_SUPPORTED(K % 64 == 0 && N % 8 == 0, "proj_linear: K=%d must be a multiple of 64 and N=%d of 8", K, N);
+  DAISY_CHECK_ARG(aligned16(x) && aligned16(w) && aligned16(y) && x_sm % 8 == 0 && w_sn % 8 == 0 && y_sm % 8 == 0,
+                  "proj_linear: rows must start on 16-byte boundaries");
+  DAISY_CHECK_ARG(x_sm < (1 << 22) && w_sn < (1 << 22), "proj_linear: row strides too long");
+  ProjParams p{};
+  p.x = x; p.x_sm = x_sm; p.w = w; p.w_sn = w_sn; p.bias = bias; p.y = y; p.y_sm = y_sm; p.M = M; p.N = N; p.K = K;
+  return dispatch_proj<0>(tile ? tile : proj_tile(M, N, K, 8), p, s);
+}
+
+int proj_qkv(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const QkvEpilogue& e,
+             int B, int K, int D, hipStream_t s, int tile) {
+  const int M = B * e.T, N = 3 * e.H * D;
+  DAISY_CHECK_ARG(x && w && e.q && e.k && e.v && e.cos && e.sin && M > 0 && K > 0, "proj_qkv: NULL tensor or empty shape");
+  DAISY_CHECK_SUPPORTED(K % 64 == 0 && (D == 64 || D == 128), "proj_qkv: K=%d must be a multiple of 64 and D=%d 64 or 128", K, D);
+  DAISY_CHECK_ARG(aligned16(x) && aligned16(w) && aligned16(e.q) && aligned16(e.k) && aligned16(e.v) && aligned16(e.ve) &&
+                      aligned16(e.cos) && aligned16(e.sin) && x_sm % 8 == 0 && w_sn % 8 == 0,
+                  "proj_qkv: tensors must be 16-byte aligned");
+  const int64_t st[] = {e.q_sb, e.q_st, e.q_sh, e.k_sb, e.k_st, e.k_sh, e.v_sb, e.v_st, e.v_sh, e.ve_sb, e.ve_st, e.ve_sh};
+  for (int64_t v : st) DAISY_CHECK_ARG(v % 8 == 0, "proj_qkv: strides must be multiples of 8 elements");
+  DAISY_CHECK_ARG(x_sm < (1 << 22) && w_sn < (1 << 22), "proj_qkv: row strides too long");
+  ProjParams p{};
+  p.x = x; p.x_sm = x_sm; p.w = w; p.w_sn = w_sn; p.M = M; p.N = N; p.K = K; p.e = e;
+  if (!tile) tile = proj_tile(M, N, K, D);
+  return D == 128 ? dispatch_proj<2>(tile, p, s) : dispatch_proj<1>(tile, p, s);
+}
+
+}  // namespace daisy

@@ -40,6 +40,9 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     picks the key tiles of a block of queries from the block's first row).  It is not checked
     here, since that would synchronise; ``check_doc_start`` does, for callers that want it.
     """
+    fast = _lib.native().prefill_attention(q, k, v, 0 if window is None else int(window), float(scale), cos, sin, doc_start, out, k_out)
+    if fast is not None:
+        return fast
     dev = _lib.require_gpu(q, k, v, cos, sin, doc_start, out, k_out)
     for name, t in (("q", q), ("k", k), ("v", v)):
         _check_bf16(name, t, 4)
@@ -464,6 +467,11 @@ def kda_chunk_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     holds N sequences packed along T, each with its own state ``[N, H, Dk, Dv]``.  The kernels read
     the bounds on the device; the host never does, so the call does not synchronise.
     """
+    if workspace is None and chunk == 64:
+        fast = _lib.native().kda_chunk(q, k, v, g, beta, scale, initial_state, bool(output_final_state), bool(use_qk_l2norm_in_kernel),
+                                       float(l2_eps), cu_seqlens)
+        if fast is not None:
+            return fast
     dev = _lib.require_gpu(q, k, v, g, beta, initial_state, workspace, cu_seqlens)
     B, T, H, Dk = q.shape
     Dv = v.shape[-1]

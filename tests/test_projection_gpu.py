@@ -1,0 +1,75 @@
+"""The tiled projection kernel (``csrc/proj.hip``) at the edges of its tiles, with and without the QKV epilogue, and
+the attention kernel for few query blocks around its tile edges and on both sides of the rule that picks it."""
+import pytest
+import torch
+
+import oracle
+from daisy_amd import CausalSelfAttention, WindowMask, _lib, ops
+from tests.helpers import assert_close_bf16
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("tile,K", [(0, 128), (1, 384), (2, 128), (3, 256), (4, 64), (5, 192), (6, 64), (7, 192)])
+@pytest.mark.parametrize("M,N", [(1, 8), (31, 64), (33, 72), (127, 136), (129, 256), (257, 520)])
+def test_tiles_against_fp64(tile, K, M, N):
+    g = torch.Generator().manual_seed(M * 1000 + N)
+    x, w, b = (torch.randn(*s, generator=g).bfloat16() for s in ((M, K), (N, K), (N,)))
+    ref = x.double() @ w.double().t()
+    xd = torch.zeros(M, K + 8, dtype=torch.bfloat16, device=DEV)[:, :K].copy_(x)      # rows at a stride of their own
+    for bias in (None, b):
+        y = _lib.native().linear(xd, w.to(DEV), None if bias is None else bias.to(DEV), 4, tile)
+        if y is None:
+            assert tile == 0 and M <= 4 or bias is not None     # the rule left the product to another kernel
+            continue
+        r = ref if bias is None else ref + bias.double()
+        err = (y.cpu().double() - r).abs()
+        assert (err <= r.abs() * 2 ** -8 + K ** 0.5 * 1e-5 + 1e-3).all(), err.max().item()
+
+
+@pytest.mark.parametrize("H,D", [(2, 128), (6, 64), (3, 64)])
+@pytest.mark.parametrize("B,T", [(1, 5), (2, 64), (1, 129), (3, 200), (1, 1100)])
+@pytest.mark.parametrize("ve", [False, True])
+def test_layer_prefill_matches_the_oracle(H, D, B, T, ve):
+    dim = H * D
+    torch.manual_seed(T)
+    attn = CausalSelfAttention(dim, H, D, receives_ve=ve, layer_idx=0, max_seq_len=T)
+    with torch.no_grad():
+        attn.qkvo_w.copy_((torch.randn(4, dim, dim) * 0.05).bfloat16())
+    x, vals = torch.randn(B, T, dim).bfloat16(), torch.randn(B, T, dim).bfloat16()
+    y_ref, k_ref, v_ref = oracle.attn_prefill(x, attn.qkvo_w.detach(), H, D, attn.rotary.cos, attn.rotary.sin, 70,
+                                              ve=vals if ve else None, g_ve=0.3228 if ve else None)
+    attn = attn.to(DEV).eval()
+    with torch.no_grad():
+        y, k, v = attn.prefill(x.to(DEV), vals.to(DEV) if ve else None, attn_mask=WindowMask(70), debug=True)
+        assert attn.last_q is not None and attn.last_q.shape == (B, T, H, D)
+        y2 = attn(x.to(DEV), vals.to(DEV) if ve else None, attn_mask=WindowMask(70))
+    assert torch.equal(y, y2)                     # the output may or may not take the queries' place
+    assert_close_bf16(k, k_ref, "k", max_abs=4e-2)
+    assert_close_bf16(v, v_ref, "v", max_abs=4e-2)
+    assert_close_bf16(y, y_ref, "y")
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H", [(1, 1), (2, 4), (8, 33)])      # few blocks; few blocks in XCD groups; many blocks
+@pytest.mark.parametrize("T,window,docs", [(1, None, False), (32, None, False), (33, 5, False), (127, 64, True), (161, None, True),
+                                           (300, 33, False)])
+def test_attention_on_both_sides_of_the_block_rule(D, B, H, T, window, docs):
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q, k, v = (torch.randn(B, T, H, D, generator=g, device=DEV).bfloat16() for _ in range(3))
+    doc = None
+    if docs:
+        doc = torch.zeros(T, dtype=torch.int32, device=DEV)
+        doc[T // 3:] = T // 3
+        doc[T - 2:] = T - 2
+    o, _ = ops.prefill_attention(q, k, v, window=window, doc_start=doc)
+    pos = torch.arange(T, device=DEV)
+    lo = torch.zeros_like(pos) if window is None else (pos - window + 1).clamp_min(0)
+    if doc is not None:
+        lo = torch.maximum(lo, doc.long())
+    seen = (pos[None, :] <= pos[:, None]) & (pos[None, :] >= lo[:, None])
+    s = torch.matmul(q.float().transpose(1, 2), k.float().transpose(1, 2).transpose(2, 3).contiguous()) * 0.12
+    p = s.masked_fill(~seen, float("-inf")).softmax(-1)
+    ref = torch.matmul(p, v.float().transpose(1, 2).contiguous()).transpose(1, 2)
+    assert_close_bf16(o, ref, f"o T={T}")
