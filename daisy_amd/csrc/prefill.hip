@@ -420,6 +420,251 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   }
 }
 
+// Few workgroups (a prompt of one or two thousand tokens of one sequence): blocks of 128 queries leave most compute
+// units idle and the last block walks all of its keys with one step in flight.  Here a workgroup is 32 queries, its
+// four wavefronts take every fourth key tile each -- tiles of their own, copied into LDS areas of their own, no
+// barrier in the loop -- and the four partial results (maximum, sum, O^T) meet in LDS at the end.  K(n+1) is copied
+// while the softmax and the second product of tile n run, V(n+1) while the scores of tile n+1 do (in-order vmcnt:
+// at most one tensor's copies stay outstanding).  A tile is fetched once per 32 queries instead of once per 128, so
+// long grids are better off with prefill_tile_kernel (the rule stands at launch_mfma).
+template <int D>
+__global__ __launch_bounds__(kPrefillThreads, 2) void prefill_split_kernel(PrefillParams p) {
+  constexpr int NS = D / 16, NDT = D / 32, HALF = D / 2, CPR = D / 8;
+  constexpr int RPL = 64 / CPR, NCP = kTBN / RPL, TILE = kTBN * D;    // NCP copies of 1 KiB per tile
+  auto swz_k = [](int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); };
+  auto swz_v = [](int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
+  __shared__ __attribute__((aligned(1024))) uint16_t tiles[4][2][TILE];   // [wavefront][K, V]; the fp32 partial O at the end
+  __shared__ float part_m[4][32], part_l[4][32];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lq = lane & 31, lh = lane >> 5;
+
+  // (batch, head) pairs in contiguous groups per XCD; inside a pair the block with the most keys first
+  const int nbh = p.B * p.H, nqb = (p.T + 31) >> 5;
+  int bh, qb;
+  if ((nbh & 7) == 0) {
+    const int g = nbh >> 3, idx = blockIdx.x >> 3;
+    bh = (blockIdx.x & 7) * g + idx % g;
+    qb = nqb - 1 - idx / g;
+  } else {
+    bh = blockIdx.x % nbh;
+    qb = nqb - 1 - blockIdx.x / nbh;
+  }
+  const int h = bh % p.H, b = bh / p.H;
+  const int q0 = qb * 32;
+  const int qrow = min(q0 + lq, p.T - 1);
+  const int lo_q = row_lo(p, qrow);
+  const int lo_min = __builtin_amdgcn_readlane(lo_q, 0), lo_max = __builtin_amdgcn_readlane(lo_q, 31);
+  const int q_max = min(q0 + 31, p.T - 1);
+  const int t_lo = lo_min / kTBN, t_hi = q_max / kTBN;
+
+  const uint16_t* kbase = p.k + b * p.k_sb + h * p.k_sh;
+  const uint16_t* vbase = p.v + b * p.v_sb + h * p.v_sh;
+  const int ld_row = lane / CPR, ld_pos = lane % CPR;
+  const uint32_t k_lds = lds_address(&tiles[wave][0][0]), v_lds = lds_address(&tiles[wave][1][0]);
+  // copy j moves rows RPL * j .. of a tile; rows past the sequence re-read its last row (masked by causality)
+  auto copy_k = [&](int t) {
+    const int kv0 = t * kTBN;
+    const uint16_t* src = kbase + (int64_t)kv0 * p.k_st;
+#pragma unroll
+    for (int j = 0; j < NCP; ++j) {
+      const int r = RPL * j + ld_row;
+      copy16_to_lds_async(src, 2 * (min(r, p.T - 1 - kv0) * (int)p.k_st + 8 * (ld_pos ^ swz_k(r))), k_lds + 1024 * j);
+    }
+  };
+  auto copy_v = [&](int t) {
+    const int kv0 = t * kTBN;
+    const uint16_t* src = vbase + (int64_t)kv0 * p.v_st;
+#pragma unroll
+    for (int j = 0; j < NCP; ++j) {
+      const int r = RPL * j + ld_row;
+      copy16_to_lds_async(src, 2 * (min(r, p.T - 1 - kv0) * (int)p.v_st + 8 * (ld_pos ^ swz_v(r))), v_lds + 1024 * j);
+    }
+  };
+  int t = t_lo + wave;
+  const bool any = t <= t_hi;
+
+  // ---- Q fragments: whole rows from global memory, rotated, through this wavefront's V area -----------------
+  constexpr int CH = HALF / 8, QRI = 64 / CH, QT = 32 / QRI;
+  bf16x8 qreg[NS];
+  {
+    const int qr = lane / CH, qc = lane % CH;
+    u32x4 x1[QT], x2[QT];
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+      const int row = min(q0 + QRI * j + qr, p.T - 1);
+      const uint16_t* qptr = p.q + b * p.q_sb + (int64_t)row * p.q_st + h * p.q_sh + 8 * qc;
+      x1[j] = *reinterpret_cast<const u32x4*>(qptr);
+      x2[j] = *reinterpret_cast<const u32x4*>(qptr + HALF);
+    }
+    if (p.cos != nullptr) {
+#pragma unroll
+      for (int j = 0; j < QT; ++j) {
+        const int row = min(q0 + QRI * j + qr, p.T - 1);
+        const float* cr = p.cos + (int64_t)row * HALF + 8 * qc;
+        const float* sr = p.sin + (int64_t)row * HALF + 8 * qc;
+        float a1[8], a2[8], y1[8], y2[8];
+        unpack8(x1[j], a1);
+        unpack8(x2[j], a2);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          y1[e] = rope_lo(a1[e], a2[e], cr[e], sr[e]);
+          y2[e] = rope_hi(a1[e], a2[e], cr[e], sr[e]);
+        }
+        x1[j] = pack8(y1);
+        x2[j] = pack8(y2);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+      const int r = QRI * j + qr;
+      *(u32x4 __attribute__((address_space(3)))*)(size_t)(v_lds + 2 * (r * D + 8 * (qc ^ swz_k(r)))) = x1[j];
+      *(u32x4 __attribute__((address_space(3)))*)(size_t)(v_lds + 2 * (r * D + 8 * ((CH + qc) ^ swz_k(r)))) = x2[j];
+    }
+    const uint32_t q_a0 = v_lds + 2 * (lq * D + 8 * (lh ^ swz_k(lq)));
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      qreg[s] = __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)(size_t)(q_a0 ^ (32u * s)));
+    // the fragments are in registers (and the global loads behind them done) before the first copies go out
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    asm volatile("" ::: "memory");
+  }
+  if (any) { copy_k(t); copy_v(t); }
+
+  const uint32_t k_a0 = k_lds + 2 * (lq * D + 8 * (lh ^ swz_k(lq)));
+  uint32_t v_a0;
+  {
+    const int i16 = lane & 15, vrow = 4 * lh + (i16 >> 2);
+    const int chunk = 2 * ((lane >> 4) & 1) + ((i16 & 3) >> 1);
+    v_a0 = v_lds + 2 * (vrow * D + 8 * (chunk ^ swz_v(vrow)) + 4 * (i16 & 1));
+  }
+  f32x16 oacc[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+
+  for (; t <= t_hi; t += 4) {
+    const int kv0 = t * kTBN;
+    const bool more = t + 4 <= t_hi;
+    // K(n) has landed when only V(n)'s copies are outstanding
+    __builtin_amdgcn_s_waitcnt(0x0F70 | NCP);
+    asm volatile("" ::: "memory");
+    f32x16 sacc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
+    bf16x8 kf[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      kf[s] = __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)(size_t)(k_a0 ^ (32u * s)));
+    __builtin_amdgcn_s_waitcnt(0xC07F);    // lgkmcnt(0): the fragments are out of LDS, the area takes the next tile
+    asm volatile("" ::: "memory");
+    if (more) copy_k(t + 4);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qreg[s], sacc, 0, 0, 0);
+    if (!(kv0 + kTBN - 1 <= min(q0, p.T - 1) && kv0 >= lo_max)) {
+      const int hi = qrow - (kv0 + 4 * lh), lo = lo_q - (kv0 + 4 * lh);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int c = 8 * (r >> 2) + (r & 3);
+        if (c > hi || c < lo) sacc[r] = -INFINITY;
+      }
+    }
+    // online softmax with the lazy rescale of prefill_tile_kernel
+    float mt = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[r]);
+    mt = pair_max(mt) * p.scale_log2e;
+    if (__builtin_amdgcn_ballot_w64(mt > m_run + 8.f) != 0) {
+      const float m_new = fmaxf(m_run, mt);
+      const float mu = (m_new == -INFINITY) ? 0.f : m_new;
+      const float alpha = fast_exp2(m_run - mu);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+    }
+    const float mu = (m_run == -INFINITY) ? 0.f : m_run;
+    bf16x8 pfrag[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      float pv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        pv[e] = fast_exp2(fmaf(sacc[8 * m + e], p.scale_log2e, -mu));
+        l_run += pv[e];
+      }
+      pfrag[m] = __builtin_bit_cast(bf16x8, pack8(pv));
+    }
+    // V(n) has landed when only K(n + 1)'s copies are outstanding
+    if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | NCP);
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) {
+        lds_u16_ptr vp = (lds_u16_ptr)(size_t)((v_a0 ^ (64u * dt)) + 2 * (16 * m * D));
+        const u32x2 a0 = lds_read_tr16_as3(vp), a1 = lds_read_tr16_as3(vp + 8 * D);
+        const u32x4 av = {a0.x, a0.y, a1.x, a1.y};
+        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), pfrag[m], oacc[dt], 0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);    // the V fragments are out of LDS
+    asm volatile("" ::: "memory");
+    if (more) copy_v(t + 4);
+  }
+
+  // Partial results: each lane of a pair holds its share of the row sum; O^T as [query][channel] fp32 in the
+  // wavefront's own tile area, 16-byte pieces swizzled by the query.
+  const float l_tot = pair_sum(l_run);
+  if (lh == 0) { part_m[wave][lq] = m_run; part_l[wave][lq] = l_tot; }
+  float* const po = reinterpret_cast<float*>(&tiles[wave][0][0]);
+  constexpr int PC = D / 4;
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int piece = 8 * dt + 2 * g + lh;      // channels 32 dt + 8 g + 4 lh + 0..3
+      *reinterpret_cast<f32x4*>(po + lq * D + 4 * (piece ^ (lq & (PC - 1)))) =
+          f32x4{oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+    }
+  __syncthreads();
+  // 8 channels per thread and pass
+#pragma unroll
+  for (int it = 0; it < 32 * CPR / kPrefillThreads; ++it) {
+    const int idx = tid + kPrefillThreads * it, row = idx / CPR, c = idx % CPR;
+    float m = part_m[0][row];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) m = fmaxf(m, part_m[w][row]);
+    const float mu = (m == -INFINITY) ? 0.f : m;
+    float l = 0.f, acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float a = fast_exp2(part_m[w][row] - mu);
+      l = fmaf(part_l[w][row], a, l);
+      const float* src = reinterpret_cast<const float*>(&tiles[w][0][0]) + row * D;
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        const f32x4 o4 = *reinterpret_cast<const f32x4*>(src + 4 * ((2 * c + v) ^ (row & (PC - 1))));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[4 * v + i] = fmaf(o4[i], a, acc[4 * v + i]);
+      }
+    }
+    const float inv = 1.f / l;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] *= inv;
+    if (q0 + row < p.T)
+      *reinterpret_cast<u32x4*>(p.o + b * p.o_sb + (int64_t)(q0 + row) * p.o_st + h * p.o_sh + 8 * c) = pack8(acc);
+  }
+}
+
 // Rotates keys once and stores them with the caller's output strides.  A thread takes one pair chunk
 // (8 + 8 channels) of HPT heads of one position: the cos and sin values are fetched once for them.
 template <int D, int HPT>
@@ -534,6 +779,18 @@ __global__ __launch_bounds__(64) void prefill_scalar_kernel(PrefillParams p) {
   }
 }
 
+// Up to how many blocks of 128 queries the kernel with four wavefronts per 32 queries is the faster one.  From a sweep
+// over B * H = 4 ... 64, T = 64 ... 8192, windows of 128, 1024 and 8192, both head dims: 1.4 to 2.4 times as fast
+// while the blocks leave compute units idle (12 heads of 128, T = 777: 19.4 -> 11.0 us; 8 heads of 64, T = 2048:
+// 32.7 -> 14.4 us), level at the limits below and slower beyond (it fetches every key tile four times as often).  Full
+// causal blocks differ in length, which favours it longer than windowed ones; wide heads less than narrow ones.
+template <int D>
+static int64_t split_limit(const PrefillParams& p) {
+  const bool full = p.doc_start == nullptr && (p.window <= 0 || p.window >= p.T);
+  if (D == 64) return full ? 768 : 320;
+  return full && p.T >= 1024 ? 384 : p.window <= 0 || p.window >= 1024 ? 192 : 144;
+}
+
 template <int D>
 static int launch_mfma(PrefillParams p, hipStream_t s) {
   const int64_t nwg = (int64_t)p.nqb * p.H * p.B;
@@ -549,6 +806,12 @@ static int launch_mfma(PrefillParams p, hipStream_t s) {
     else hipLaunchKernelGGL((rope_k_kernel<D, 1>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p);
     DAISY_CHECK_LAUNCH("rope_k_kernel");
     p.k = p.k_out; p.k_sb = p.ko_sb; p.k_st = p.ko_st; p.k_sh = p.ko_sh;
+  }
+  if (nwg <= split_limit<D>(p)) {
+    const int64_t nsw = (int64_t)((p.T + 31) / 32) * p.H * p.B;
+    hipLaunchKernelGGL((prefill_split_kernel<D>), dim3((unsigned)nsw), dim3(kPrefillThreads), 0, s, p);
+    DAISY_CHECK_LAUNCH("prefill_split_kernel");
+    return DAISY_OK;
   }
   hipLaunchKernelGGL((prefill_tile_kernel<D>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
   DAISY_CHECK_LAUNCH("prefill_tile_kernel");
