@@ -65,68 +65,77 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 
 
 // ===========================================================================
-// Chunked forward.  Per (batch, head), chunk of C = 64 positions.  The kernels work on 128 key
-// channels and 128 value columns; a smaller Dk (a multiple of 8) is served by reading the missing
-// channels as zeros (zero channels of q, k and g change nothing: they add nothing to any dot product
-// or norm, and their state rows stay zero), and value columns are independent of each other, so any
-// Dv (a multiple of 8) is served in passes of up to 128 columns, a short last pass reading zeros.
+// Chunked forward.  Per (batch, head), chunk of C = 32 positions.  The kernels work on KD = 64 or 128 key
+// channels; a smaller Dk (a multiple of 8) is served by reading the missing channels as zeros (zero channels of q, k
+// and g change nothing: they add nothing to any dot product or norm, and their state rows stay zero), and value
+// columns are independent of each other, so any Dv (a multiple of 8) is served in groups of 32.
 //
-// With G_i the inclusive running sum of the log-decay g inside the chunk (per
-// channel), S0 the state at the chunk start, and (per channel products written
-// with (.)):
+// With G_i the inclusive running sum of the log-decay g inside the chunk (per channel), S0 the state at the chunk
+// start, and (per channel products written with (.)):
 //   A_ij = beta_i sum_d k_id k_jd exp(G_id - G_jd)     (j <  i)
 //   P_ij =        sum_d q_id k_jd exp(G_id - G_jd)     (j <= i)
-//   (I + A) [W | U0] = diag(beta) [exp(G) (.) K | V]
-//   U  = U0 - W S0
-//   O  = scale ((exp(G) (.) Q) S0 + P U)
-//   S' = diag(exp(G_last)) S0 + (exp(G_last - G) (.) K)^T U
+//   T  = (I + A)^-1 diag(beta)
+//   X  = V - (exp(G) (.) K) S0
+//   O  = scale ((exp(G) (.) Q) S0 + (P T) X)
+//   S' = diag(exp(G_last)) S0 + ((exp(G_last - G) (.) K)^T T) X
 //
-// kda_prep_kernel (one workgroup per chunk, all chunks in parallel) produces
-// everything that does not depend on S0 into the workspace:
-//   Wn  = -W                        bf16 [64][128]   contraction index (channel) permuted
-//   Qg  = scale exp(G) (.) Q        bf16 [64][128]   channel permuted
-//   Pm  = scale tril(P)             bf16 [64][64]    column (position) permuted
-//   KtH + KtL = (exp(G_last - G) (.) K)^T split into two bf16 terms, [128][64], position permuted
-//   U0T = U0^T                      fp32 [128][64]
-//   dec = exp(G_last)               fp32 [128]
-// kda_state_kernel (one workgroup per (batch, head, 32 value columns): two computing
-// wavefronts per tile of 16 columns, four data-moving wavefronts that fill the
-// double-buffered LDS stages with the chunk data) then walks the chunks in order
-// with the fp32 state in registers; every product in it is a
-// v_mfma_f32_16x16x32_bf16 whose B operand is an accumulator (S0 or U)
-// converted to bf16 in place: in the 16x16 accumulator layout lane l holds
-// column l%16 and rows 4*(l/16)+r of each tile, so two stacked tiles give the
-// lane 8 contraction indices 16*t + 4*(l/16) + r (t = 0,1; r = 0..3).  The A
-// operands are stored with their contraction index permuted inside every
-// aligned group of 32 (perm32) so that those 8 indices are 8 consecutive
-// elements, one 16-byte load.
+// kda_prep_kernel (all chunks in parallel) produces everything that depends on neither S0 nor V, one block of
+// KdaBlob<KD>::kBytes per chunk, laid out as the other kernel wants it in LDS:
+//   Kg  = -exp(G) (.) K             bf16 [32][KD]   contraction index (channel) permuted
+//   Qg  = scale exp(G) (.) Q        bf16 [32][KD]   channel permuted
+//   Mh + Ml = (exp(G_last - G) (.) K)^T T split into two bf16 terms, [KD][32], column (position) permuted
+//   Ph + Pl = scale tril(P) T       the same, [32][32]
+//   dec = exp(G_last)               fp32 [KD]
+// kda_state_kernel (one workgroup per (batch, head, 32 value columns)) then walks the chunks in order with the fp32
+// state in registers; every product in it is a v_mfma_f32_16x16x32_bf16 whose B operand is an accumulator (S0 or X)
+// converted to bf16 in place: in the 16x16 accumulator layout lane l holds column l%16 and rows 4*(l/16)+r of each
+// tile, so two stacked tiles give the lane 8 contraction indices 16*t + 4*(l/16) + r (t = 0,1; r = 0..3).  The A
+// operands are stored with their contraction index permuted inside every aligned group of 32 (perm32) so that those 8
+// indices are 8 consecutive elements, one 16-byte load.
 //
-// Numerics: the 16x16 blocks of A and P run on MFMA with both operands
-// referenced to the row before the block (every exponent <= 0 off the diagonal);
-// a diagonal block whose total decay exceeds exp(-80) is instead accumulated in
-// fp32 pair by pair with exp(G_i - G_j), j < i (no exponent is ever positive, so strong
-// decays cannot overflow).  The triangular solve works on 16-row blocks: fp32
-// inverses of the diagonal blocks, everything else as products of two-term bf16
-// splits (three MFMAs each, relative error ~2^-17).  The state update uses the
-// same two-term split of both operands, which keeps the state error near fp32.
+// What bounds it.  The first kernel moves bytes, with the conversions in between: 1.0 GB in 217 us at B4 T8192 H16 (4.7 TB/s);
+// with chunks of 64 and W = T K, U0 = T V in the workspace (107 KB per 64 positions, from a solve with 256 right-hand
+// sides) it took 355 us.  The second kernel is a serial chain of chunks, bound by the latency of a link: folding T into
+// the two matrices above takes a product and a conversion out of it, and chunks of 32 let three stages of everything the
+// chain needs fit the LDS, so that no computing wavefront waits for global memory (those loads alone were 90 us of 284).
+// It takes 230 us at that size, 0.9 us per chunk; 165 us of them remain without the copies into the LDS.
+//
+// Numerics: the 16x16 blocks of A and P run on MFMA with both operands referenced to the row before the block (every
+// exponent <= 0 off the diagonal); a diagonal block whose total decay exceeds exp(-80) is instead accumulated in
+// fp32 pair by pair with exp(G_i - G_j), j < i (no exponent is ever positive, so strong decays cannot overflow).
+// T is computed in fp32; the products with T, the state update and the output's second term use two-term bf16 splits of
+// both operands (three MFMAs each, relative error ~2^-17), which keeps the state error near fp32.
 // ===========================================================================
-constexpr int KC = 64;    // chunk length
-constexpr int KD = 128;   // Dk = Dv
+constexpr int KC = 32;    // chunk length
+constexpr int KDMAX = 128;
 constexpr int KVS = 16;   // value columns per state wavefront
-constexpr size_t kChunkBytes = (size_t)KC * KD * 2 * 2 + KC * KC * 2 + (size_t)KD * KC * 2 * 2 + (size_t)KD * KC * 4 + KD * 4;
+
+// One chunk's block in the workspace: byte offsets of its parts; rows of 16-byte pieces XOR-swizzled (below).
+template <int KD> struct KdaBlob {
+  static constexpr int kKg = 0, kQg = KC * KD * 2, kMh = 2 * KC * KD * 2, kMl = 3 * KC * KD * 2;
+  static constexpr int kPh = 4 * KC * KD * 2, kPl = kPh + KC * KC * 2, kDec = kPl + KC * KC * 2;
+  static constexpr int kBytes = (kDec + KD * 4 + 1023) & ~1023;     // whole 1 KiB copies
+};
+static_assert(KdaBlob<128>::kBytes == 37 * 1024 && KdaBlob<64>::kBytes == 21 * 1024, "");
+// Swizzle of a row's 16-byte pieces: the 16 lanes that a 16-byte LDS read serves together must fall into 16 different slots
+// of the 256-byte bank window.  Those are not 16 consecutive lanes but lanes 0-3, 12-15 and 20-27 (and so on): rows 0-3
+// and 12-15 of one k-group with rows 4-11 of the next.  For rows of 64 bytes (row >> 2) & 3 itself puts two of them into every
+// slot (256 of 930 LDS cycles per chunk); the permutation 0 2 3 1 of it puts one.  Rows of 256, 128 and 64 bytes:
+template <int ROWBYTES> __host__ __device__ constexpr int piece_swizzle(int row) {
+  return ROWBYTES == 256 ? (row & 15) : ROWBYTES == 128 ? ((row >> 1) & 7) : ((row >> 3) & 1) | (((row >> 2) ^ (row >> 3)) & 1) << 1;
+}
 
 struct KdaParams {
   const uint16_t* q; const uint16_t* k; const uint16_t* v;
   const void* g; int g_bf16; const float* beta;
   const float* s0; uint16_t* o; float* s_out;
   int B, T, H, NC; float scale; int l2norm; float l2eps;
-  int Dk, Dv;     // the tensors' own widths: Dk <= 128 key channels, Dv value columns
-  int v0, nv;     // this pass covers value columns v0 .. v0 + nv - 1 (nv <= 128)
-  uint16_t* Wn; uint16_t* Qg; uint16_t* Pm; uint16_t* KtH; uint16_t* KtL; float* U0T; float* dec;
+  int Dk, Dv;     // the tensors' own widths: Dk <= KD key channels, Dv value columns
+  char* blobs;    // [H][nc_total][KdaBlob<KD>::kBytes]
   // Sequences packed along the token axis of a batch of one (B == 1, T = all tokens): n_seq > 0,
   // bounds [n_seq + 1] = sanitised running lengths, seq_chunk0 [n_seq + 1] = first chunk slot of
   // every sequence, chunk_seq [NC] = sequence of every chunk slot; all three are written on the
-  // device by kda_chunk_table_kernel, NC is the host's upper bound T / 64 + n_seq on the slots.
+  // device by kda_chunk_table_kernel, NC is the host's upper bound T / 32 + n_seq on the slots.
   int n_seq; const int32_t* bounds; const int32_t* seq_chunk0; const int32_t* chunk_seq;
   int nc_total;   // chunk slots per head in the workspace: B * NC, or NC for a packed batch
 };
@@ -148,7 +157,7 @@ __device__ __forceinline__ SeqSpan seq_span(const KdaParams& p, int seq) {
 
 // Chunk slots of packed sequences, built on the device so that the host never reads the bounds.
 // bounds = cu_seqlens forced to start at 0, to stay within 0..T and not to decrease (whatever the
-// caller passed, no kernel then leaves the tensors); seq_chunk0 = running sum of ceil(len / 64);
+// caller passed, no kernel then leaves the tensors); seq_chunk0 = running sum of ceil(len / 32);
 // chunk_seq = the sequence of every slot.  One workgroup; thread i takes a run of sequences.
 __global__ __launch_bounds__(256) void kda_chunk_table_kernel(const int32_t* cu, int n_seq, int T, int nc_max,
                                                               int32_t* bounds, int32_t* seq_chunk0, int32_t* chunk_seq) {
@@ -193,157 +202,176 @@ __host__ __device__ constexpr int perm32_inv(int p) { return (p & ~0x1c) | ((p &
 
 __device__ __forceinline__ f32x4 lds_f4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
-// Off-diagonal 16x16 blocks of A in LDS: block (I, J), J < I, has index I(I-1)/2 + J.
-__host__ __device__ constexpr int off_block(int I, int J) { return I * (I - 1) / 2 + J; }
-
 // A float as two bf16 terms (value = hi + lo up to 2^-17 relative).
 __device__ __forceinline__ void split_bf16(float x, float& hi, float& lo) { hi = round_bf16(x); lo = x - hi; }
+// Eight floats as two 16-byte pieces of bf16 terms.
+__device__ __forceinline__ void split_pack8(const float* x, u32x4& hi, u32x4& lo) {
+  float h[8], l[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) split_bf16(x[e], h[e], l[e]);
+  hi = pack8(h);
+  lo = pack8(l);
+}
+// LDS writes of a wavefront before this point are seen by all of its lanes after it.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ uint32_t dpp_xor2(uint32_t x) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, false); }
 
-__global__ __launch_bounds__(256, 2) void kda_prep_kernel(KdaParams p) {
-  __shared__ __attribute__((aligned(16))) float G[KC][KD + 4];       // inclusive running log-decay (rows 4 banks apart: 16 rows read side by side do not collide); later staging for Wn
-  __shared__ __attribute__((aligned(16))) uint16_t Kr[KC][KD + 8];   // k as given (bf16)
-  __shared__ __attribute__((aligned(16))) uint16_t QV[KC][KD + 8];   // q as given; v as given once A and P are done
-  __shared__ __attribute__((aligned(16))) float Ad[4][16][16];       // diagonal blocks of A, [block][column j][row i]; later T = (I + A_II)^-1 as bf16 hi | lo
-  __shared__ __attribute__((aligned(16))) uint16_t AoH[6][16][16];   // -A, off-diagonal blocks (off_block), [row][column], bf16 high term
-  __shared__ __attribute__((aligned(16))) uint16_t AoL[6][16][16];   //   ... low term
-  __shared__ float rk[KC], rq[KC], bt[KC];                           // 1/|k|, 1/|q|, beta (0 for padded rows)
-  __shared__ int steep[4];                                           // per 16-row block: total decay beyond exp(-80); 2 when some 4 rows of it alone go beyond
-  auto& Qr = QV;
-  auto& Vr = QV;
+// A workgroup makes two neighbouring chunk slots (64 rows; they may belong to different sequences).
+template <int KD>
+__global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaParams p) {
+  using Blob = KdaBlob<KD>;
+  constexpr int CPR = KD / 8, RPP = 256 / CPR, NP = 64 / RPP;         // 16-byte pieces per row, rows per pass, passes
+  constexpr int NM = KD / 32;                                         // contraction groups of 32 channels
+  __shared__ __attribute__((aligned(16))) float G[64][KD + 4];        // inclusive running log-decay (rows 4 banks apart: 16 rows read side by side do not collide)
+  __shared__ __attribute__((aligned(16))) uint16_t Kr[64][KD + 8];    // k as given (bf16)
+  __shared__ __attribute__((aligned(16))) uint16_t Qr[64][KD + 8];    // q as given
+  __shared__ __attribute__((aligned(16))) float Ad[4][16][16];        // diagonal blocks of A, [block][column j][row i]; later scratch of that wavefront
+  __shared__ __attribute__((aligned(16))) float Ao[2][16][20];        // the block A_10 of either chunk, [row][column]
+  __shared__ __attribute__((aligned(16))) float Td[4][16][20];        // (I + A_II)^-1, [block][row][column]
+  __shared__ __attribute__((aligned(16))) float rk[64], rq[64], bt[64];   // 1/|k|, 1/|q|, beta (0 for padded rows)
+  __shared__ int steep[4];                                            // per 16-row block: total decay beyond exp(-80); 2 when some 4 rows of it alone go beyond
 
-  // Chunk slot gc of the workspace; token rows t0 .. t_end - 1 of the flattened token axis are this
-  // chunk's share of its sequence (t_end = end of the sequence: the last chunk may be short).
   const int h = blockIdx.y;
-  const int gc = blockIdx.z * p.NC + blockIdx.x;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  int t0, t_end;
-  if (p.n_seq > 0) {
-    if (gc >= p.seq_chunk0[p.n_seq]) return;      // a surplus slot (the grid covers the upper bound)
-    const SeqSpan sp = seq_span(p, p.chunk_seq[gc]);
-    t0 = sp.tok0 + (gc - sp.c0) * KC;
-    t_end = sp.tok_end;
-  } else {
-    t0 = blockIdx.z * p.T + blockIdx.x * KC;
-    t_end = (blockIdx.z + 1) * p.T;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  // First token row and live rows of the two chunks.  A slot without a chunk has no live rows and is not stored; its
+  // loads go to the first chunk's first row.
+  int t0[2], n_live[2];
+  int64_t ci[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int slot = 2 * blockIdx.x + c;
+    t0[c] = 0;
+    n_live[c] = 0;
+    int gc = slot;
+    if (p.n_seq > 0) {
+      if (slot < p.seq_chunk0[p.n_seq]) {
+        const SeqSpan sp = seq_span(p, p.chunk_seq[slot]);
+        t0[c] = sp.tok0 + (slot - sp.c0) * KC;
+        n_live[c] = min(sp.tok_end - t0[c], KC);
+      }
+    } else {
+      gc = blockIdx.z * p.NC + slot;
+      if (slot < p.NC) {
+        t0[c] = blockIdx.z * p.T + slot * KC;
+        n_live[c] = min((int)(blockIdx.z + 1) * p.T - t0[c], KC);
+      }
+    }
+    if (c == 0 && n_live[0] <= 0) return;      // surplus slots (the grid covers the upper bound)
+    if (n_live[c] <= 0) { t0[c] = t0[0]; n_live[c] = 0; }
+    ci[c] = (int64_t)h * p.nc_total + gc;
   }
-  const int n_live = t_end - t0;                  // live rows of the chunk when < 64
-  const int64_t ci = (int64_t)h * p.nc_total + gc;
-  // Addresses: a wavefront-uniform 64-bit base per array (the chunk's first token row of this head, or
-  // the chunk's slot in the workspace) plus a 32-bit offset per lane.  Written out once here: as one
-  // 64-bit expression per access the row products were rebuilt per lane and load (seven vector
-  // instructions each, three of them at a quarter of the rate).
+  // Addresses: a wavefront-uniform 64-bit base per array and chunk plus a 32-bit offset per lane.
   const uint32_t row_stride = (uint32_t)p.H * (uint32_t)p.Dk;     // elements between token rows of one head (q, k, g)
-  const uint32_t row_stride_v = (uint32_t)p.H * (uint32_t)p.Dv;   //   ... of v
-  const int64_t tok_base = ((int64_t)t0 * p.H + h) * p.Dk;        // first element of the chunk's first row
-  const uint16_t* const q_c = p.q + tok_base;
-  const uint16_t* const k_c = p.k + tok_base;
-  const uint16_t* const v_c = p.v + ((int64_t)t0 * p.H + h) * p.Dv + p.v0;
-  const float* const beta_c = p.beta + ((int64_t)t0 * p.H + h);
-  uint16_t* const qg_c = p.Qg + ci * KC * KD;
-  uint16_t* const pm_c = p.Pm + ci * KC * KC;
-  float* const u0_c = p.U0T + ci * KD * KC;
+  const int64_t tok_base[2] = {((int64_t)t0[0] * p.H + h) * p.Dk, ((int64_t)t0[1] * p.H + h) * p.Dk};
+  char* const blob[2] = {p.blobs + ci[0] * Blob::kBytes, p.blobs + ci[1] * Blob::kBytes};
 
   // ---- phase 0a: G = cumsum(g) -----------------------------------------------
-  // Every global load of the chunk (g here, then q, k, v and beta of phase 0b) goes out before
-  // the first result is used, so that the memory latency is paid once.  Inputs are read once and
-  // the workspace is written once: both as streaming (non-temporal) accesses.
+  // Every global load of the chunks (g here, then q, k and beta of phase 0b) goes out before the first result is used,
+  // so that the memory latency is paid once.  Inputs are read once and the workspace is written once: both as streaming
+  // (non-temporal) accesses.
   if (tid < 4) steep[tid] = 0;
   __syncthreads();
-  const int cc = tid & 15, r4 = tid >> 4;
-  u32x4 qraw[4], vraw[4], kraw[4];
-  float btv[4];
+  const int cc = tid % CPR, r4 = tid / CPR;
+  u32x4 qraw[NP], kraw[NP];
+  float btv[NP];
+  constexpr int GR = 64 * KD / 256;               // rows of one channel per thread: a whole chunk (128) or half of one (64)
   {
-    const int d = tid & 127, half = __builtin_amdgcn_readfirstlane(tid >> 7);   // the row of a g load is wavefront-uniform
+    const int d = tid % KD, part = __builtin_amdgcn_readfirstlane(tid / KD);   // the row of a g load is wavefront-uniform
+    const int c = part * GR / KC, row0 = part * GR % KC;
     const bool d_live = d < p.Dk;                 // channels beyond Dk read as zero (their loads re-read the last channel)
     const int dl = min(d, p.Dk - 1);
-    float gv[32];
-    // Rows past the end re-read the last row (always valid) and are zeroed afterwards, so that
-    // the loads carry no branches and all go out together; the dtype is decided once, outside
-    // the loops, for the same reason.  bf16 g: the two channels of a pair read the same dword
-    // (no sub-dword loads) and take their half.
-    uint32_t graw[32];
+    // Rows past the end re-read the last row (always valid) and are zeroed afterwards, so that the loads carry no
+    // branches and all go out together; the dtype is decided once, outside the loops, for the same reason.  bf16 g: the
+    // two channels of a pair read the same dword (no sub-dword loads) and take their half.
+    const int last = max((c ? n_live[1] : n_live[0]) - 1, 0), live = c ? n_live[1] : n_live[0];
+    const int64_t base = c ? tok_base[1] : tok_base[0];
+    uint32_t graw[GR];
     if (p.g_bf16) {
 #pragma unroll
-      for (int i = 0; i < 32; ++i) {
-        const uint32_t* row = reinterpret_cast<const uint32_t*>(p.g) + ((tok_base + (uint32_t)min(32 * half + i, n_live - 1) * row_stride) >> 1);
+      for (int i = 0; i < GR; ++i) {
+        const uint32_t* row = reinterpret_cast<const uint32_t*>(p.g) + ((base + (uint32_t)min(row0 + i, last) * row_stride) >> 1);
         graw[i] = __builtin_nontemporal_load(row + (uint32_t)(dl >> 1));
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < 32; ++i) {
-        const uint32_t* row = reinterpret_cast<const uint32_t*>(p.g) + (tok_base + (uint32_t)min(32 * half + i, n_live - 1) * row_stride);
+      for (int i = 0; i < GR; ++i) {
+        const uint32_t* row = reinterpret_cast<const uint32_t*>(p.g) + (base + (uint32_t)min(row0 + i, last) * row_stride);
         graw[i] = __builtin_nontemporal_load(row + (uint32_t)dl);
       }
     }
-    const bool g16 = p.g_bf16 != 0, odd = (d & 1) != 0;
+    const int ccl = min(cc, p.Dk / 8 - 1);
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      const float x = g16 ? (odd ? bf16hi_to_f32(graw[i]) : bf16lo_to_f32(graw[i])) : __uint_as_float(graw[i]);
-      gv[i] = (32 * half + i < n_live && d_live) ? x : 0.f;
-    }
-    const int ccl = min(cc, p.Dk / 8 - 1), ccv = min(cc, p.nv / 8 - 1);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = r4 + 16 * i;
-      const int rc = min(r, n_live - 1);
-      const uint32_t off = (uint32_t)rc * row_stride + 8u * ccl;
-      kraw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(k_c + off));
-      vraw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(v_c + (uint32_t)rc * row_stride_v + 8u * ccv));
-      qraw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(q_c + off));
-      btv[i] = beta_c[(uint32_t)rc * (uint32_t)p.H];
+    for (int i = 0; i < NP; ++i) {
+      const int r = r4 + RPP * i, rc = r >> 5;    // (a pass of 16 or 32 rows lies inside one chunk)
+      const uint32_t row = (uint32_t)min(r & 31, max((rc ? n_live[1] : n_live[0]) - 1, 0));
+      const int64_t at = (rc ? tok_base[1] : tok_base[0]) + row * row_stride + 8u * ccl;
+      kraw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.k + at));
+      qraw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.q + at));
+      btv[i] = p.beta[(int64_t)((rc ? t0[1] : t0[0]) + row) * p.H + h];
     }
     __builtin_amdgcn_sched_barrier(0);
-    // G holds the running sum in units of log 2 (g * log2(e)): every exponential below is a bare
-    // v_exp_f32.
+    float gv[GR];
+    const bool g16 = p.g_bf16 != 0, odd = (d & 1) != 0;
+#pragma unroll
+    for (int i = 0; i < GR; ++i) {
+      const float x = g16 ? (odd ? bf16hi_to_f32(graw[i]) : bf16lo_to_f32(graw[i])) : __uint_as_float(graw[i]);
+      gv[i] = (row0 + i < live && d_live) ? x : 0.f;
+    }
+    // G holds the running sum in units of log 2 (g * log2(e)): every exponential below is a bare v_exp_f32.
     float acc = 0.f;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < GR; ++i) {
       acc += gv[i] * kLog2e;
-      G[32 * half + i][d] = acc;
+      G[part * GR + i][d] = acc;
     }
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
+    for (int blk = 0; blk < GR / 16; ++blk) {
       float tot = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; ++i) tot += gv[16 * blk + i];
-      if (tot < -80.f) atomicMax(&steep[2 * half + blk], 1);
-      // ... and whether four consecutive rows alone decay that far (then no reference row per
-      // group of four keeps the exponents of the matrix-core path in range)
+      const int sb = part * GR / 16 + blk;
+      if (tot < -80.f) atomicMax(&steep[sb], 1);
+      // ... and whether four consecutive rows alone decay that far (then no reference row per group of four keeps
+      // the exponents of the matrix-core path in range)
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
         const float t4 = gv[16 * blk + 4 * g4] + gv[16 * blk + 4 * g4 + 1] + gv[16 * blk + 4 * g4 + 2] + gv[16 * blk + 4 * g4 + 3];
-        if (t4 < -80.f) atomicMax(&steep[2 * half + blk], 2);
+        if (t4 < -80.f) atomicMax(&steep[sb], 2);
       }
     }
-    __syncthreads();
-    if (half == 1) {
-      const float add = G[31][d];
+    if constexpr (GR < KC) {                      // the second half of a chunk continues from the first
+      __syncthreads();
+      if (row0 != 0) {
+        const float add = G[part * GR - 1][d];
 #pragma unroll
-      for (int i = 0; i < 32; ++i) G[32 + i][d] += add;
+        for (int i = 0; i < GR; ++i) G[part * GR + i][d] += add;
+      }
     }
   }
 
   // ---- phase 0b: raw q, k to LDS, row norms, beta ---------------------------
-  float rqv[4];
+  float rkv[NP], rqv[NP];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = r4 + 16 * i;
-    const bool live = r < n_live;
+  for (int i = 0; i < NP; ++i) {
+    const int r = r4 + RPP * i;
+    const bool live = (r & 31) < ((r >> 5) ? n_live[1] : n_live[0]);
     const u32x4 zero4 = {0, 0, 0, 0};
     if (!live || 8 * cc >= p.Dk) { kraw[i] = zero4; qraw[i] = zero4; }
-    if (!live || 8 * cc >= p.nv) vraw[i] = zero4;
     float kf[8], qf[8];
     unpack8(kraw[i], kf);
     unpack8(qraw[i], qf);
     float sk = 0.f, sq = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) { sk = fmaf(kf[e], kf[e], sk); sq = fmaf(qf[e], qf[e], sq); }
-    sk = group_sum<16>(sk);
-    sq = group_sum<16>(sq);
-    const float nk = p.l2norm ? rsqrtf(sk + p.l2eps) : 1.f;
+    sk = group_sum<CPR>(sk);
+    sq = group_sum<CPR>(sq);
+    rkv[i] = p.l2norm ? rsqrtf(sk + p.l2eps) : 1.f;
     rqv[i] = p.l2norm ? rsqrtf(sq + p.l2eps) : 1.f;
     if (cc == 0) {
-      rk[r] = nk;
+      rk[r] = rkv[i];
       rq[r] = rqv[i];
       bt[r] = live ? btv[i] : 0.f;
     }
@@ -352,52 +380,66 @@ __global__ __launch_bounds__(256, 2) void kda_prep_kernel(KdaParams p) {
   }
   __syncthreads();
 
-  // ---- phase 1: Qg = scale exp(G) q/|q| (channel permuted), dec = exp(G_last) ----
+  // ---- phase 1: Kg = -exp(G) k/|k|, Qg = scale exp(G) q/|q| (channel permuted), dec = exp(G_last) ----
   {
-    const int pos0 = ((cc >> 2) << 5) | ((cc & 1) << 4) | (((cc >> 1) & 1) << 2);  // perm32(8*cc)
+    // The stored 16-byte piece a of a group of 32 channels holds channels 4a..+3 and 16 + 4a..+3: lanes cc and cc ^ 2 each
+    // own half of two pieces and swap one half.
+    const int b2 = cc & 3;
+    const bool low = b2 < 2;
+    const int piece = (cc & ~3) + 2 * (b2 & 1) + (low ? 0 : 1);
+    auto join = [&](const u32x4& pk) -> u32x4 {
+      const uint32_t s0 = low ? pk.z : pk.x, s1 = low ? pk.w : pk.y;
+      const uint32_t x0 = dpp_xor2(s0), x1 = dpp_xor2(s1);
+      return low ? u32x4{pk.x, pk.y, x0, x1} : u32x4{x0, x1, pk.z, pk.w};
+    };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = r4 + 16 * i;
-      float qf[8], o8[8];
+    for (int i = 0; i < NP; ++i) {
+      const int r = r4 + RPP * i, rc = r >> 5, row = r & 31;
+      float qf[8], kf[8], o8[8], k8[8];
       unpack8(qraw[i], qf);
+      unpack8(kraw[i], kf);
       const f32x4 g0 = lds_f4(&G[r][8 * cc]), g1 = lds_f4(&G[r][8 * cc + 4]);
-      const float sc = p.scale * rqv[i];
+      const float sq = p.scale * rqv[i], sk = -rkv[i];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        o8[e] = sc * __builtin_amdgcn_exp2f(g0[e]) * qf[e];
-        o8[4 + e] = sc * __builtin_amdgcn_exp2f(g1[e]) * qf[4 + e];
+      for (int e = 0; e < 8; ++e) {
+        const float f = __builtin_amdgcn_exp2f(e < 4 ? g0[e & 3] : g1[e & 3]);
+        o8[e] = sq * f * qf[e];
+        k8[e] = sk * f * kf[e];
       }
-      const u32x4 pk = pack8(o8);
-      uint16_t* dst = qg_c + (uint32_t)(r * KD + pos0);
-      u32x2 lo2 = {pk.x, pk.y}, hi2 = {pk.z, pk.w};
-      __builtin_nontemporal_store(lo2, reinterpret_cast<u32x2*>(dst));        // channels 8cc+0..3
-      __builtin_nontemporal_store(hi2, reinterpret_cast<u32x2*>(dst + 8));    // channels 8cc+4..7
+      const uint32_t at = (uint32_t)(row * 2 * KD + 16 * (piece ^ piece_swizzle<2 * KD>(row)));
+      const u32x4 kp = join(pack8(k8)), qp = join(pack8(o8));
+      if (rc == 0 || n_live[1] > 0) {
+        char* dst = (rc ? blob[1] : blob[0]) + at;
+        __builtin_nontemporal_store(kp, reinterpret_cast<u32x4*>(dst + Blob::kKg));
+        __builtin_nontemporal_store(qp, reinterpret_cast<u32x4*>(dst + Blob::kQg));
+      }
     }
-    if (r4 == 0) {
-      const f32x4 g0 = lds_f4(&G[KC - 1][8 * cc]), g1 = lds_f4(&G[KC - 1][8 * cc + 4]);
-      f32x4 d0, d1;
+    if (tid < 2 * KD / 4) {
+      const int c = tid / (KD / 4), d4 = 4 * (tid % (KD / 4));
+      const f32x4 gl = lds_f4(&G[KC * c + KC - 1][d4]);
+      f32x4 dv;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { d0[e] = __builtin_amdgcn_exp2f(g0[e]); d1[e] = __builtin_amdgcn_exp2f(g1[e]); }
-      float* dd = p.dec + ci * KD + 8 * cc;
-      *reinterpret_cast<f32x4*>(dd) = d0;
-      *reinterpret_cast<f32x4*>(dd + 4) = d1;
+      for (int e = 0; e < 4; ++e) dv[e] = __builtin_amdgcn_exp2f(gl[e]);
+      if (c == 0 || n_live[1] > 0) *reinterpret_cast<f32x4*>((c ? blob[1] : blob[0]) + Blob::kDec + 4 * d4) = dv;
     }
   }
 
-  // ---- phase 2a: 16x16 blocks of A and P on MFMA --------------------------------
-  // Block (I, J), J <= I: both operands are referenced to the row before block I, so the row
-  // factor exp(G_i - G_ref) is <= 1 and, for J < I, so is the column factor exp(G_ref - G_j).
-  // For a diagonal block (J == I) the column factor grows to exp(total decay of the block); the
-  // block takes this path only when that total stays below 80 (flag `steep` otherwise).
-  // The row operands (k_i f_i, q_i f_i with f_i = exp(G_i - G_ref)) of a block row are made once
-  // and serve every block of the row.
-  bf16x8 va[4], vq[4];
-  auto row_operands = [&](int I) {
-    const int li = lane & 15, q4 = lane >> 4;
-    const int ref = 16 * I - 1;   // -1 for the first block: G_ref = 0
-    const int ri = 16 * I + li;
+  // ---- phase 2: 16x16 blocks of A and P on MFMA --------------------------------
+  // Block rows bi = 0..3 of the 64 rows (chunk bi / 2, I = bi % 2).  Block (I, J), J <= I: both operands are referenced to
+  // the row before block I (the chunk's start for I = 0: G_ref = 0), so the row factor exp(G_i - G_ref) is <= 1 and, for J < I,
+  // so is the column factor exp(G_ref - G_j).  For a diagonal block (J == I) the column factor grows to exp(total decay
+  // of the block); the block takes this path only when that total stays below 80 (flag `steep` otherwise).
+  // Wavefront w takes block row w: its diagonal block and, in the second block row of a chunk, block (1, 0).
+  const int li = lane & 15, q4 = lane >> 4;
+  const int chunk = wave >> 1, I = wave & 1;
+  const int ri = 16 * wave + li;
+  char* const my_blob = chunk ? blob[1] : blob[0];
+  const bool stored = chunk == 0 || n_live[1] > 0;
+  bf16x8 va[NM], vq[NM];
+  // Row operands k_i f_i, q_i f_i with f_i = exp(G_i - G_ref(i)); `ref` is the lane's reference row (-1: G_ref = 0).
+  auto row_operands = [&](int ref) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < NM; ++m) {
       const int d0 = 32 * m + 8 * q4;
       float ki[8], qi[8], ak[8], aq[8];
       unpack8(*reinterpret_cast<const u32x4*>(&Kr[ri][d0]), ki);
@@ -418,13 +460,15 @@ __global__ __launch_bounds__(256, 2) void kda_prep_kernel(KdaParams p) {
       vq[m] = __builtin_bit_cast(bf16x8, pack8(aq));
     }
   };
-  auto mfma_block = [&](int I, int J) {
-    const int li = lane & 15, q4 = lane >> 4;
-    const int ref = 16 * I - 1;
-    const int rj = 16 * J + li;
+  // This wavefront's rows of scale tril(P), as a product's operand wants them: row 16 I + li, columns 4 q4 + r of either
+  // column block.
+  f32x4 P[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  auto mfma_block = [&](int J) {
+    const int ref = I ? 16 * wave - 1 : -1;
+    const int rj = 32 * chunk + 16 * J + li;
     f32x4 accA = {0.f, 0.f, 0.f, 0.f}, accP = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < NM; ++m) {
       const int d0 = 32 * m + 8 * q4;
       float kj[8], bk[8];
       unpack8(*reinterpret_cast<const u32x4*>(&Kr[rj][d0]), kj);
@@ -439,64 +483,52 @@ __global__ __launch_bounds__(256, 2) void kda_prep_kernel(KdaParams p) {
       const bf16x8 vb = __builtin_bit_cast(bf16x8, pack8(bk));
       accA = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[m], vb, accA, 0, 0, 0);
       // P comes out transposed (operands swapped: both operand layouts hold 8 contraction indices of
-      // one row / column per lane): a lane then owns four consecutive columns of one row of P, one
-      // 8-byte store instead of four 2-byte ones.
+      // one row / column per lane): a lane then owns four consecutive columns of one row of P.
       accP = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb, vq[m], accP, 0, 0, 0);
     }
     // accA: lane holds column j = 16J + li, rows i = 16I + 4*q4 + r
-    const int j = 16 * J + li;
-    const float rkj = rk[j];
+    const float rkj = rk[rj];
     f32x4 av;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = 16 * I + 4 * q4 + r;
+      const int i = 16 * wave + 4 * q4 + r;
       av[r] = bt[i] * rk[i] * rkj * accA[r];
     }
     {
-      // accP: lane holds row i = 16I + li, columns j = 16J + 4*q4 + r (stored positions perm32(j): the
-      // four are consecutive, perm32 keeps the low two bits)
+      // accP: lane holds row i = 16I + li, columns j = 16J + 4*q4 + r
       const int ip = 16 * I + li, jp = 16 * J + 4 * q4;
-      const f32x4 rk4 = lds_f4(&rk[jp]);
-      const float qs = p.scale * rq[ip];
-      float pv[4];
+      const f32x4 rk4 = lds_f4(&rk[32 * chunk + jp]);
+      const float qs = p.scale * rq[ri];
+      f32x4 pv;
 #pragma unroll
       for (int r = 0; r < 4; ++r) pv[r] = (jp + r <= ip) ? qs * rk4[r] * accP[r] : 0.f;
-      const u32x2 w = {pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3])};
-      *reinterpret_cast<u32x2*>(pm_c + (uint32_t)(ip * KC + perm32(jp))) = w;
+      if (J == 0) P[0] = pv; else P[1] = pv;
     }
     if (I == J) {
-      *reinterpret_cast<f32x4*>(&Ad[I][li][4 * q4]) = av;   // entries with i <= j are never read
+      *reinterpret_cast<f32x4*>(&Ad[wave][li][4 * q4]) = av;   // entries with i <= j are never read
     } else {
-      const int ob = off_block(I, J);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float hi, lo;
-        split_bf16(-av[r], hi, lo);
-        AoH[ob][4 * q4 + r][li] = (uint16_t)(pack_bf16x2(hi, 0.f) & 0xffffu);
-        AoL[ob][4 * q4 + r][li] = (uint16_t)(pack_bf16x2(lo, 0.f) & 0xffffu);
-      }
+      for (int r = 0; r < 4; ++r) Ao[chunk][4 * q4 + r][li] = av[r];
     }
   };
-  // Blocks by wavefront, normally: 0 -> (0,0), (3,3); 1 -> (1,0), (1,1); 2 -> (2,0), (2,1), (2,2);
-  // 3 -> (3,0), (3,1), (3,2).  A diagonal block whose decay is too steep for the MFMA path (some
-  // channel beyond exp(-80) across the block: the column factors could overflow) is accumulated
+  // A diagonal block whose decay is too steep for the MFMA path even with a reference row per four rows is accumulated
   // in fp32 pair by pair with exp(G_i - G_j), j < i, where no exponent is ever positive.
-  auto steep_diagonal = [&](int I) {
+  auto steep_diagonal = [&]() {
     const int il = lane >> 2, dq = lane & 3;
-    const int ri = 16 * I + il;
+    const int rr = 16 * wave + il;
     float a[16], pp[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) { a[j] = 0.f; pp[j] = 0.f; }
 #pragma unroll 1
-    for (int dc = 0; dc < 4; ++dc) {
-      const int d0 = 32 * dq + 8 * dc;
+    for (int dc = 0; dc < KD / 32; ++dc) {
+      const int d0 = (KD / 4) * dq + 8 * dc;
       float ki[8], qi[8];
-      unpack8(*reinterpret_cast<const u32x4*>(&Kr[ri][d0]), ki);
-      unpack8(*reinterpret_cast<const u32x4*>(&Qr[ri][d0]), qi);
-      const f32x4 gi0 = lds_f4(&G[ri][d0]), gi1 = lds_f4(&G[ri][d0 + 4]);
+      unpack8(*reinterpret_cast<const u32x4*>(&Kr[rr][d0]), ki);
+      unpack8(*reinterpret_cast<const u32x4*>(&Qr[rr][d0]), qi);
+      const f32x4 gi0 = lds_f4(&G[rr][d0]), gi1 = lds_f4(&G[rr][d0 + 4]);
 #pragma unroll
       for (int j = 15; j >= 0; --j) {
-        const int rj = 16 * I + j;
+        const int rj = 16 * wave + j;
         float kj[8];
         unpack8(*reinterpret_cast<const u32x4*>(&Kr[rj][d0]), kj);
         // exp(G_i - G_j) for j < i: the exponent is a sum of log-decays, never positive; rows at or
@@ -512,65 +544,34 @@ __global__ __launch_bounds__(256, 2) void kda_prep_kernel(KdaParams p) {
         }
       }
     }
-    const float bi = bt[ri] * rk[ri], qs = p.scale * rq[ri];
+    const float bi = bt[rr] * rk[rr], qs = p.scale * rq[rr];
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-      float av = dpp_add<0x4E>(dpp_add<0xB1>(a[j]));    // sum over the 4 channel quarters
+      float av = dpp_add<0x4E>(dpp_add<0xB1>(a[j]));         // sum over the 4 channel quarters
       float pv = dpp_add<0x4E>(dpp_add<0xB1>(pp[j]));
-      if ((j & 3) == dq) {
-        const int rj = 16 * I + j;
-        const float rkj = rk[rj];
-        if (j < il) Ad[I][j][il] = bi * rkj * av;
-        pv = (j <= il) ? qs * rkj * pv : 0.f;
-        pm_c[(uint32_t)(ri * KC + perm32(rj))] = (uint16_t)(pack_bf16x2(pv, 0.f) & 0xffffu);
-      }
+      const float rkj = rk[16 * wave + j];
+      if ((j & 3) == dq && j < il) Ad[wave][j][il] = bi * rkj * av;
+      if ((j & 3) == dq) Td[wave][il][j] = (j <= il) ? qs * rkj * pv : 0.f;   // (on the way to the operand layout)
     }
+    wave_lds_fence();
+    if (I == 0) P[0] = lds_f4(&Td[wave][li][4 * q4]); else P[1] = lds_f4(&Td[wave][li][4 * q4]);
+    wave_lds_fence();
   };
   // A steep diagonal block on the matrix cores after all: with one reference row per group of four
   // rows (the row before the group) every row factor exp(G_i - G_ref(i)) is <= 1, and the column
   // factors exp(G_ref - G_j) are <= 1 for columns of earlier groups and at most the decay of four
   // rows inside the group.  Pass r multiplies all rows by the columns scaled for the reference of
-  // group r; the accumulator layout gives rows 4r..4r+3 to the lanes with q4 == r, which keep
-  // that pass's result.  Four passes, a fifth of the exponentials of the pairwise path.
-  auto steep_diagonal_mfma = [&](int I) {
-    const int li = lane & 15, q4 = lane >> 4;
-    const int ri = 16 * I + li;
-    // The diagonal block is the last of its segment: the row operands of the block row are not needed
-    // again and their registers take the ones made here.
-    bf16x8 (&sa)[4] = va;
-    bf16x8 (&sq)[4] = vq;
-    {
-      const int ref = 16 * I + (li & ~3) - 1;   // -1: the chunk's first rows, G_ref = 0
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const int d0 = 32 * m + 8 * q4;
-        float ki[8], qi[8], ak[8], aq[8];
-        unpack8(*reinterpret_cast<const u32x4*>(&Kr[ri][d0]), ki);
-        unpack8(*reinterpret_cast<const u32x4*>(&Qr[ri][d0]), qi);
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-          const f32x4 gi = lds_f4(&G[ri][d0 + 4 * hf]);
-          const f32x4 gr = (ref >= 0) ? lds_f4(&G[max(ref, 0)][d0 + 4 * hf]) : zero;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float fi = __builtin_amdgcn_exp2f(gi[e] - gr[e]);
-            ak[4 * hf + e] = ki[4 * hf + e] * fi;
-            aq[4 * hf + e] = qi[4 * hf + e] * fi;
-          }
-        }
-        sa[m] = __builtin_bit_cast(bf16x8, pack8(ak));
-        sq[m] = __builtin_bit_cast(bf16x8, pack8(aq));
-      }
-    }
+  // group r; the accumulator layout gives rows 4r..4r+3 (A) resp. the lanes of those rows (P, transposed) that pass's result.
+  auto steep_diagonal_mfma = [&]() {
+    row_operands((I == 0 && li < 4) ? -1 : 16 * wave + (li & ~3) - 1);
     f32x4 accA = {0.f, 0.f, 0.f, 0.f}, accP = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int r = 0; r < 4; ++r) {
-      const int ref = 16 * I + 4 * r - 1;
+      const int ref = (I == 0 && r == 0) ? -1 : 16 * wave + 4 * r - 1;
       const bool live = (li >> 2) <= r;     // later columns are above the diagonal for every row of the group
       f32x4 pa = {0.f, 0.f, 0.f, 0.f}, pp = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
+      for (int m = 0; m < NM; ++m) {
         const int d0 = 32 * m + 8 * q4;
         float kj[8], bk[8];
         unpack8(*reinterpret_cast<const u32x4*>(&Kr[ri][d0]), kj);
@@ -584,229 +585,153 @@ __global__ __launch_bounds__(256, 2) void kda_prep_kernel(KdaParams p) {
             bk[4 * hf + e] = live ? kj[4 * hf + e] * __builtin_amdgcn_exp2f(fminf(gr[e] - gj[e], 120.f)) : 0.f;
         }
         const bf16x8 vb = __builtin_bit_cast(bf16x8, pack8(bk));
-        pa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sa[m], vb, pa, 0, 0, 0);
-        pp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sq[m], vb, pp, 0, 0, 0);
+        pa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[m], vb, pa, 0, 0, 0);
+        pp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb, vq[m], pp, 0, 0, 0);
       }
-      if (q4 == r) { accA = pa; accP = pp; }
+      if (q4 == r) accA = pa;               // rows 4 q4 .. of A
+      if ((li >> 2) == r) accP = pp;        // row li of P
     }
-    // accumulator: lane holds column j = 16I + li, rows i = 16I + 4*q4 + r
-    const int j = 16 * I + li;
-    const float rkj = rk[j];
+    const float rkj = rk[ri];
     f32x4 av;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = 16 * I + 4 * q4 + r;
+      const int i = 16 * wave + 4 * q4 + r;
       av[r] = bt[i] * rk[i] * rkj * accA[r];
-      const float pv = (j <= i) ? p.scale * rq[i] * rkj * accP[r] : 0.f;
-      pm_c[(uint32_t)(i * KC + perm32(j))] = (uint16_t)(pack_bf16x2(pv, 0.f) & 0xffffu);
     }
-    *reinterpret_cast<f32x4*>(&Ad[I][li][4 * q4]) = av;   // entries with i <= j are never read
+    *reinterpret_cast<f32x4*>(&Ad[wave][li][4 * q4]) = av;   // entries with i <= j are never read
+    const f32x4 rk4 = lds_f4(&rk[16 * wave + 4 * q4]);
+    const float qs = p.scale * rq[ri];
+    f32x4 pv;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) pv[r] = (4 * q4 + r <= li) ? qs * rk4[r] * accP[r] : 0.f;
+    if (I == 0) P[0] = pv; else P[1] = pv;
   };
   {
-    // Segments (block row I, columns jlo..jhi) per wavefront, 4 bits each, two per wavefront
-    // (0xf.. = none).  A steep diagonal block costs about as much as five others, so when there
-    // is one the blocks are dealt differently: 0 -> (0,0), (3,0..1); 1 -> (1,1), (3,2);
-    // 2 -> (2,0..2); 3 -> (3,3), (1,0).
-    const bool any_steep = (steep[0] | steep[1] | steep[2] | steep[3]) != 0;
-    constexpr uint32_t kPlain[4] = {0x333000u, 0xfff101u, 0xfff202u, 0xfff203u};   // (jhi, jlo, I) second | first
-    constexpr uint32_t kSteep[4] = {0x103000u, 0x223111u, 0xfff202u, 0x001333u};
-    uint32_t plan = any_steep ? kSteep[0] : kPlain[0];
+    const int sp = __builtin_amdgcn_readfirstlane(steep[wave]);
+    if (I == 1 || sp == 0) row_operands(I ? 16 * wave - 1 : -1);
+    if (I == 1) mfma_block(0);
+    if (sp == 2) steep_diagonal();
+    else if (sp == 1) steep_diagonal_mfma();
+    else mfma_block(I);
+  }
+
+  // ---- phase 3: T = (I + A)^-1 diag(beta).  The inverse of diagonal block `wave` in fp32, one column per lane (lanes
+  // 16.. repeat the work of lane & 15).
+  wave_lds_fence();
+  {
+    float tc[16];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) if (wave == w) plan = any_steep ? kSteep[w] : kPlain[w];
-    for (int sg = 0; sg < 2; ++sg, plan >>= 12) {
-      const int I = plan & 15, jlo = (plan >> 4) & 15, jhi = (plan >> 8) & 15;
-      if (I == 15) break;
-      row_operands(I);
-      for (int J = jlo; J <= jhi; ++J) {
-        if (J == I && steep[I] == 2) steep_diagonal(I);
-        else if (J == I && steep[I] == 1) steep_diagonal_mfma(I);
-        else mfma_block(I, J);
-      }
+    for (int i = 0; i < 16; ++i) tc[i] = (i == li) ? 1.f : 0.f;
+#pragma unroll
+    for (int j = 0; j < 15; ++j) {
+      f32x4 ar[4];
+#pragma unroll
+      for (int i4 = (j + 1) / 4; i4 < 4; ++i4) ar[i4] = lds_f4(&Ad[wave][j][4 * i4]);
+      const float xj = tc[j];
+#pragma unroll
+      for (int i = j + 1; i < 16; ++i) tc[i] = fmaf(-ar[i >> 2][i & 3], xj, tc[i]);
     }
-    // The state kernel reads P in 16x32 pieces; blocks (0,1) and (2,3) lie above the diagonal.
-    if (wave == 1) {
-      const int li = lane & 15, q4 = lane >> 4;
+    if (lane < 16) {
 #pragma unroll
-      for (int I = 0; I < 4; I += 2)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) pm_c[(uint32_t)((16 * I + 4 * q4 + r) * KC + perm32(16 * (I + 1) + li))] = 0;
+      for (int i = 0; i < 16; ++i) Td[wave][i][li] = tc[i];
     }
   }
-  __syncthreads();
-
-  // Q is no longer needed: V takes its place in LDS (right-hand side of the solve).
-#pragma unroll
-  for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(&Vr[r4 + 16 * i][8 * cc]) = vraw[i];
-
-  __syncthreads();   // V is in place
-
-  // ---- phase 4: (I + A) X = diag(beta) [exp(G) K | V] by blocks of 16 rows on MFMA ----
-  //     X_I = T_I (B_I - sum_{J<I} A_IJ X_J),   T_I = (I + A_II)^-1.
-  // The 256 right-hand-side columns form 16 tiles of 16; wavefront w solves tiles w, w+4 (W part)
-  // and w+8, w+12 (U part).  In the 16x16x32 MFMA a lane's accumulator holds rows 4q..4q+3 of a
-  // block for one column; the same four values, split into two bf16 terms, are that lane's
-  // share of the next product's right operand when contraction slot (q, e) stands for row
-  // 4q+e of block J (e < 4) and of block J+1 (e >= 4) -- so X never leaves the registers.  The left
-  // operands (T and -A, two bf16 terms each) come from LDS in that slot order; every product is
-  // three MFMAs (hi*hi, hi*lo, lo*hi).
+  __syncthreads();   // both inverses and A_10 of either chunk are in place
+  // T_10 = -T_11 (A_10 T_00): lane (row li, columns 4 q4 .. + 3); the two wavefronts of a chunk both make all of it, in a
+  // scratch area of their own (A_II is no longer needed).
   {
-    const int li = lane & 15, q4 = lane >> 4;
-    // 4a: T of diagonal block `wave`, one column per lane (lanes 16.. repeat the work of lane & 15).
-    {
-      float tc[16];
+    f32x4 m1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 16; ++i) tc[i] = (i == li) ? 1.f : 0.f;
+    for (int j4 = 0; j4 < 4; ++j4) {
+      const f32x4 a4 = lds_f4(&Ao[chunk][li][4 * j4]);
 #pragma unroll
-      for (int j = 0; j < 15; ++j) {
-        f32x4 ar[4];
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 t4 = lds_f4(&Td[2 * chunk][4 * j4 + e][4 * q4]);
 #pragma unroll
-        for (int i4 = (j + 1) / 4; i4 < 4; ++i4) ar[i4] = lds_f4(&Ad[wave][j][4 * i4]);
-        const float xj = tc[j];
-#pragma unroll
-        for (int i = j + 1; i < 16; ++i) tc[i] = fmaf(-ar[i >> 2][i & 3], xj, tc[i]);
-      }
-      // The wavefront has read all of its block before any lane writes: T replaces A_II in place.
-      uint16_t* Th = reinterpret_cast<uint16_t*>(&Ad[wave][0][0]);   // [16][16] high terms, then [16][16] low terms
-      if (lane < 16) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          float hi, lo;
-          split_bf16(tc[i], hi, lo);
-          Th[i * 16 + li] = (uint16_t)(pack_bf16x2(hi, 0.f) & 0xffffu);
-          Th[256 + i * 16 + li] = (uint16_t)(pack_bf16x2(lo, 0.f) & 0xffffu);
-        }
+        for (int r = 0; r < 4; ++r) m1[r] = fmaf(a4[e], t4[r], m1[r]);
       }
     }
-    // 4b: right-hand sides in accumulator layout: C[tile][block][r] = B[16*block + 4*q4 + r][column].
-    f32x4 C[4][4];
+    *reinterpret_cast<f32x4*>(&Ad[wave][li][4 * q4]) = m1;
+    wave_lds_fence();
+    f32x4 t10 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      const int col = 16 * (wave + 4 * (tt & 1)) + li;
+    for (int j4 = 0; j4 < 4; ++j4) {
+      const f32x4 a4 = lds_f4(&Td[2 * chunk + 1][li][4 * j4]);
 #pragma unroll
-      for (int I = 0; I < 4; ++I) {
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 x4 = lds_f4(&Ad[wave][4 * j4 + e][4 * q4]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int i = 16 * I + 4 * q4 + r;
-          C[tt][I][r] = (tt < 2) ? bt[i] * rk[i] * __builtin_amdgcn_exp2f(G[i][col]) * bf16lo_to_f32(Kr[i][col])
-                                 : bt[i] * bf16lo_to_f32(Vr[i][col]);
-        }
+        for (int r = 0; r < 4; ++r) t10[r] = fmaf(-a4[e], x4[r], t10[r]);
       }
     }
-    // ---- phase 3 (placed here, where few registers are live): (exp(G_last - G) k/|k|)^T as two
-    // bf16 terms, position permuted.  Thread (d, gh) makes four 16-byte pieces of row d; stored
-    // from here they would hit 64 different lines per instruction, so they go through LDS (the
-    // space of G and of K, both dead after the barrier) and leave as whole rows.
-    u32x4 kth[4], ktl[4];
-    const int kd = tid & 127, kgh = tid >> 7;
-    {
-      const float glast = G[KC - 1][kd];
+    wave_lds_fence();
+    *reinterpret_cast<f32x4*>(&Ad[wave][li][4 * q4]) = t10;
+    wave_lds_fence();
+  }
+  // T^T as left operand: row (column of T) 16 J + li, contraction slots (q4, e): positions 4 q4 + e for e < 4,
+  // 16 + 4 q4 + (e - 4) for e >= 4; two bf16 terms.
+  bf16x8 th[2], tl[2];
+  {
+    const float b0 = bt[32 * chunk + li], b1 = bt[32 * chunk + 16 + li];
+    float v0[8], v1[8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int g8 = 4 * kgh + i;   // group of 8 stored positions
-        float hi[8], lo[8];
+    for (int e = 0; e < 4; ++e) {
+      v0[e] = b0 * Td[2 * chunk][4 * q4 + e][li];
+      v0[4 + e] = b0 * Ad[wave][4 * q4 + e][li];
+      v1[e] = 0.f;
+      v1[4 + e] = b1 * Td[2 * chunk + 1][4 * q4 + e][li];
+    }
+    u32x4 hi, lo;
+    split_pack8(v0, hi, lo);
+    th[0] = __builtin_bit_cast(bf16x8, hi);
+    tl[0] = __builtin_bit_cast(bf16x8, lo);
+    split_pack8(v1, hi, lo);
+    th[1] = __builtin_bit_cast(bf16x8, hi);
+    tl[1] = __builtin_bit_cast(bf16x8, lo);
+  }
+  // Row `row` of (right operand)^T T: the products come out with four consecutive columns of T per lane and column block,
+  // which is the stored piece q4 of that row; both terms of it leave from here, 16 whole rows per instruction.
+  auto times_t = [&](const float* r8, char* dst_hi, char* dst_lo, int row) {
+    u32x4 hi, lo;
+    split_pack8(r8, hi, lo);
+    const bf16x8 rh = __builtin_bit_cast(bf16x8, hi), rl = __builtin_bit_cast(bf16x8, lo);
+    float out[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int pos = perm32_inv(8 * g8 + e);
-          const float val = __builtin_amdgcn_exp2f(glast - G[pos][kd]) * bf16lo_to_f32(Kr[pos][kd]) * rk[pos];
-          hi[e] = round_bf16(val);
-          lo[e] = val - hi[e];
-        }
-        kth[i] = pack8(hi);
-        ktl[i] = pack8(lo);
+    for (int J = 0; J < 2; ++J) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tl[J], rh, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(th[J], rl, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(th[J], rh, acc, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[4 * J + r] = acc[r];
+    }
+    split_pack8(out, hi, lo);
+    const int at = row * 64 + 16 * (q4 ^ piece_swizzle<64>(row));
+    if (stored) {
+      __builtin_nontemporal_store(hi, reinterpret_cast<u32x4*>(dst_hi + at));
+      __builtin_nontemporal_store(lo, reinterpret_cast<u32x4*>(dst_lo + at));
+    }
+  };
+  {
+    float pv[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { pv[e] = P[0][e]; pv[4 + e] = P[1][e]; }
+    times_t(pv, my_blob + Blob::kPh, my_blob + Blob::kPl, 16 * I + li);
+  }
+  // ---- phase 4: M = (exp(G_last - G) k/|k|)^T T, half of the chunk's channels per wavefront
+  {
+    const f32x4 r0 = lds_f4(&rk[32 * chunk + 4 * q4]), r1 = lds_f4(&rk[32 * chunk + 16 + 4 * q4]);
+#pragma unroll
+    for (int i = 0; i < KD / 32; ++i) {
+      const int d = 16 * (KD / 32 * I + i) + li;
+      const float glast = G[32 * chunk + 31][d];
+      float kv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int r = 32 * chunk + (e < 4 ? 4 * q4 + e : 12 + 4 * q4 + e);
+        kv[e] = __builtin_amdgcn_exp2f(glast - G[r][d]) * bf16lo_to_f32(Kr[r][d]) * (e < 4 ? r0[e & 3] : r1[e & 3]);
       }
-    }
-    __syncthreads();   // G, K and V have been read by everyone (their space becomes staging); T is in place
-    char* KtHst = reinterpret_cast<char*>(&G[0][0]) + KC * KD * 2;   // [128][64] bf16 behind the Wn tile
-    char* KtLst = reinterpret_cast<char*>(&Kr[0][0]);                // [128][64] bf16
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int off = kd * 128 + 16 * ((4 * kgh + i) ^ (kd & 7));    // pieces of a row swizzled against bank conflicts
-      *reinterpret_cast<u32x4*>(KtHst + off) = kth[i];
-      *reinterpret_cast<u32x4*>(KtLst + off) = ktl[i];
-    }
-    // 4c: left operands.  Slot (q4, e): e < 4 -> column 4*q4+e of the first block, e >= 4 -> of the second.
-    auto lds_half = [&](const uint16_t* row) -> u32x2 { return *reinterpret_cast<const u32x2*>(row + 4 * q4); };
-    auto frag = [&](u32x2 a, u32x2 b) -> bf16x8 { u32x4 w = {a.x, a.y, b.x, b.y}; return __builtin_bit_cast(bf16x8, w); };
-    const u32x2 none = {0u, 0u};
-    bf16x8 Tf[4][2], Af[4][2];   // Af: (1,0) | (2,0)(2,1) | (3,0)(3,1) | (3,2)
-#pragma unroll
-    for (int I = 0; I < 4; ++I) {
-      const uint16_t* Th = reinterpret_cast<const uint16_t*>(&Ad[I][0][0]);
-      Tf[I][0] = frag(lds_half(Th + li * 16), none);
-      Tf[I][1] = frag(lds_half(Th + 256 + li * 16), none);
-    }
-    Af[0][0] = frag(lds_half(&AoH[off_block(1, 0)][li][0]), none);
-    Af[0][1] = frag(lds_half(&AoL[off_block(1, 0)][li][0]), none);
-    Af[1][0] = frag(lds_half(&AoH[off_block(2, 0)][li][0]), lds_half(&AoH[off_block(2, 1)][li][0]));
-    Af[1][1] = frag(lds_half(&AoL[off_block(2, 0)][li][0]), lds_half(&AoL[off_block(2, 1)][li][0]));
-    Af[2][0] = frag(lds_half(&AoH[off_block(3, 0)][li][0]), lds_half(&AoH[off_block(3, 1)][li][0]));
-    Af[2][1] = frag(lds_half(&AoL[off_block(3, 0)][li][0]), lds_half(&AoL[off_block(3, 1)][li][0]));
-    Af[3][0] = frag(lds_half(&AoH[off_block(3, 2)][li][0]), none);
-    Af[3][1] = frag(lds_half(&AoL[off_block(3, 2)][li][0]), none);
-
-    // Two bf16 terms of an accumulator as halves of a right operand.
-    auto split_acc = [&](const f32x4& x, u32x2& hi, u32x2& lo) {
-      float h[4], l[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) split_bf16(x[e], h[e], l[e]);
-      hi.x = pack_bf16x2(h[0], h[1]); hi.y = pack_bf16x2(h[2], h[3]);
-      lo.x = pack_bf16x2(l[0], l[1]); lo.y = pack_bf16x2(l[2], l[3]);
-    };
-    // acc += L * R with L = Lf[0] + Lf[1], R = (hi | lo)
-    auto mul3 = [&](const bf16x8 (&Lf)[2], bf16x8 Rh, bf16x8 Rl, f32x4 acc) -> f32x4 {
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Lf[1], Rh, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Lf[0], Rl, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Lf[0], Rh, acc, 0, 0, 0);
-      return acc;
-    };
-    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    uint16_t* Wst = reinterpret_cast<uint16_t*>(&G[0][0]);   // [64][128] bf16 staging
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      f32x4 X[4];
-      u32x2 xh[4], xl[4], ch, cl;
-      split_acc(C[tt][0], ch, cl);
-      X[0] = mul3(Tf[0], frag(ch, none), frag(cl, none), zero4);
-      split_acc(X[0], xh[0], xl[0]);
-      C[tt][1] = mul3(Af[0], frag(xh[0], none), frag(xl[0], none), C[tt][1]);
-      split_acc(C[tt][1], ch, cl);
-      X[1] = mul3(Tf[1], frag(ch, none), frag(cl, none), zero4);
-      split_acc(X[1], xh[1], xl[1]);
-      C[tt][2] = mul3(Af[1], frag(xh[0], xh[1]), frag(xl[0], xl[1]), C[tt][2]);
-      C[tt][3] = mul3(Af[2], frag(xh[0], xh[1]), frag(xl[0], xl[1]), C[tt][3]);
-      split_acc(C[tt][2], ch, cl);
-      X[2] = mul3(Tf[2], frag(ch, none), frag(cl, none), zero4);
-      split_acc(X[2], xh[2], xl[2]);
-      C[tt][3] = mul3(Af[3], frag(xh[2], none), frag(xl[2], none), C[tt][3]);
-      split_acc(C[tt][3], ch, cl);
-      X[3] = mul3(Tf[3], frag(ch, none), frag(cl, none), zero4);
-
-      const int col = 16 * (wave + 4 * (tt & 1)) + li;
-      if (tt < 2) {
-        const int pc = perm32(col);
-#pragma unroll
-        for (int I = 0; I < 4; ++I)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            Wst[(16 * I + 4 * q4 + r) * KD + pc] = (uint16_t)(pack_bf16x2(-X[I][r], 0.f) & 0xffffu);
-      } else {
-        float* dst = u0_c + (uint32_t)(col * KC + 4 * q4);
-#pragma unroll
-        for (int I = 0; I < 4; ++I) __builtin_nontemporal_store(X[I], reinterpret_cast<f32x4*>(dst + 16 * I));
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ch = tid + 256 * i;   // 16-byte chunk of the [64][128] bf16 tile
-      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(Wst + 8 * ch), reinterpret_cast<u32x4*>(p.Wn + ci * KC * KD + 8 * ch));
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ch = tid + 256 * i;   // 16-byte chunk of a [128][64] bf16 tile
-      const int off = (ch >> 3) * 128 + 16 * ((ch & 7) ^ ((ch >> 3) & 7));
-      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(KtHst + off), reinterpret_cast<u32x4*>(p.KtH + ci * KD * KC + 8 * ch));
-      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(KtLst + off), reinterpret_cast<u32x4*>(p.KtL + ci * KD * KC + 8 * ch));
+      times_t(kv, my_blob + Blob::kMh, my_blob + Blob::kMl, d);
     }
   }
 }
@@ -817,48 +742,59 @@ __device__ __forceinline__ bf16x8 pack_acc2(const f32x4& t0, const f32x4& t1) {
   r.z = pack_bf16x2(t1[0], t1[1]); r.w = pack_bf16x2(t1[2], t1[3]);
   return __builtin_bit_cast(bf16x8, r);
 }
-
-// LDS stage of the state kernel: everything of one chunk that does not depend on the value
-// column, copied with asynchronous global->LDS copies while the previous chunk is computed.
-// Rows are stored with their 16-byte chunks XOR-swizzled (chunk c of row r at position
-// c ^ f(r)) so that the 16-byte operand reads of 16 consecutive rows fall into 16 different
-// slots of the 256-byte bank window: f(r) = r & 15 for 256-byte rows, (r >> 1) & 7 for 128-byte
-// rows (two rows per window).
-constexpr int KCT = 2;                        // tiles of 16 value columns per workgroup
-constexpr int KSW = 2 * KCT;                  // computing wavefronts per workgroup: two per column tile
-constexpr int KPW = 4;                        // data-moving wavefronts per workgroup
-constexpr int kStageWn = 0;                   // [64][128] bf16
-constexpr int kStageQg = 16384;               // [64][128] bf16
-constexpr int kStageKtH = 32768;              // [128][64] bf16
-constexpr int kStageKtL = 49152;              // [128][64] bf16
-constexpr int kStageDec = 65536;               // [128] fp32: the chunk's total decay per key channel
-constexpr int kStageBytes = 65536 + 1024;
+// ... and what the rounding left over, as a second operand.
+__device__ __forceinline__ bf16x8 pack_rest2(const f32x4& t0, const f32x4& t1, bf16x8 high) {
+  const u32x4 hb = __builtin_bit_cast(u32x4, high);
+  f32x4 l0, l1;
+  l0[0] = t0[0] - bf16lo_to_f32(hb.x); l0[1] = t0[1] - bf16hi_to_f32(hb.x);
+  l0[2] = t0[2] - bf16lo_to_f32(hb.y); l0[3] = t0[3] - bf16hi_to_f32(hb.y);
+  l1[0] = t1[0] - bf16lo_to_f32(hb.z); l1[1] = t1[1] - bf16hi_to_f32(hb.z);
+  l1[2] = t1[2] - bf16lo_to_f32(hb.w); l1[3] = t1[3] - bf16hi_to_f32(hb.w);
+  return pack_acc2(l0, l1);
+}
 
 typedef __attribute__((address_space(3))) const char* lds_cptr;
 __device__ __forceinline__ bf16x8 lds_bf16x8(lds_cptr p) {
   return __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)p);
 }
+__device__ __forceinline__ f32x4 lds_f32x4(lds_cptr p) { return *(const f32x4 __attribute__((address_space(3)))*)p; }
+// LDS transpose read: inside a block of 16 lanes that address, lane i, row i / 4 and columns 4 (i % 4) .. + 3 of a bf16
+// tile, lane i receives column i of the four rows.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x2 lds_column4(lds_cptr p) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)p));
+}
 
-// The chunk-to-chunk chain sets the time of this kernel.  Two measures shorten a link:
-//  * the work of one tile of 16 value columns is shared by two wavefronts: wavefront `hf` keeps
-//    the state rows (key channels) [64 hf, 64 hf + 64) and produces the output rows (positions)
-//    [32 hf, 32 hf + 32) of the chunk.  Both need all of U = U0 - W S0, whose contraction runs
-//    over every key channel: each computes it in full (16 MFMAs, duplicated) from its own half of
-//    the state and a bf16 copy of the partner's half, handed over through LDS at the barrier
-//    that ends a chunk -- no barrier inside a chunk;
-//  * a fifth wavefront does nothing but move data: it issues the global->LDS copies of the next
-//    chunk (a CU takes in only ~30 bytes per cycle, so issuing 64 KB blocks a wavefront for
-//    longer than the arithmetic of a chunk lasts) and stores the previous chunk's output rows,
-//    which the computing wavefronts leave in LDS, as whole 64-byte row pieces.
-__global__ __launch_bounds__(64 * (KSW + KPW), 1) void kda_state_kernel(KdaParams p) {
-  __shared__ __attribute__((aligned(1024))) char stage[2][kStageBytes];
-  __shared__ __attribute__((aligned(16))) u32x4 xch[2][KSW][2][64];           // [chunk parity][wavefront][k-group][lane]
-  __shared__ __attribute__((aligned(16))) uint16_t ost[2][KC][KVS * KCT];      // [chunk parity][position][value column]
+constexpr int KCT = 2;                        // tiles of 16 value columns per workgroup
+constexpr int KPW = 4;                        // data-moving wavefronts per workgroup
+constexpr int KSTAGES = 3;                    // LDS stages of chunk data
+constexpr int kStateThreads = 64 * (2 * KCT + KPW);
+
+// The chunk-to-chunk chain sets the time of this kernel once its data are there, and next to it what the CU's LDS can
+// deliver (about 110 KB of operands and copies per chunk).  So:
+//  * one wavefront owns one tile of 16 value columns with all of its state rows: the state never leaves its registers
+//    (as right operand it is the accumulators converted in place), nothing of the chain waits for another wavefront,
+//    and every operand of the chain is read once per column tile.  Two wavefronts per tile with half of the state each,
+//    both computing X and handing state halves over through LDS, took 250 us instead of 230 (B4 T8192 H16, 128 x 128);
+//  * the outputs are not part of the chain: a second wavefront per tile makes Qg S0 of the chunk from the bf16 state
+//    the first one left in LDS, adds (P T) X when X has arrived, and stores the rows one chunk later;
+//  * neither waits for global memory: four further wavefronts issue the asynchronous copies of the chunk two ahead (the
+//    chunk's block is one linear copy of 37 or 21 KiB, V 32 rows of 64 bytes).
+template <int KD>
+__global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p) {
+  using Blob = KdaBlob<KD>;
+  constexpr int NM = KD / 32, NS = KD / 16;                    // channel groups of 32, state tiles of 16 rows
+  constexpr int kV = Blob::kBytes, kStage = Blob::kBytes + KC * KVS * KCT * 2;
+  constexpr int NCP = Blob::kBytes / 1024;
+  __shared__ __attribute__((aligned(1024))) char stage[KSTAGES][kStage];
+  __shared__ __attribute__((aligned(16))) u32x4 xs[2][KCT][NM][64];           // [chunk parity][column tile][channel group][lane]: S0 as right operand
+  __shared__ __attribute__((aligned(16))) u32x4 xx[2][KCT][2][64];            // X as right operand, two terms
+  __shared__ __attribute__((aligned(16))) uint16_t ost[KCT][KC][KVS];         // output rows on their way out
 
   // Keep the column groups of one (batch, head) on one XCD: they read the same chunk data.
   int vid = blockIdx.x;
   if ((gridDim.x & 7) == 0) vid = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const int NGRP = (p.nv + KVS * KCT - 1) / (KVS * KCT);   // groups of 32 value columns in this pass
+  const int NGRP = (p.Dv + KVS * KCT - 1) / (KVS * KCT);       // groups of 32 value columns
   const int grp = vid % NGRP, bh = vid / NGRP;
   const int h = bh % p.H, b = bh / p.H;     // b: batch element, or sequence of a packed batch
   const SeqSpan sp = seq_span(p, b);
@@ -867,258 +803,208 @@ __global__ __launch_bounds__(64 * (KSW + KPW), 1) void kda_state_kernel(KdaParam
   const int lane = threadIdx.x & 63, ln = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-  if (wave >= KSW) {
-    const int pw = wave - KSW;
+  if (wave >= 2 * KCT) {
     // ================= data-moving wavefront =================
+    const int pw = wave - 2 * KCT;
     const uint32_t stage_lds = lds_address(&stage[0][0]);
-    // 256-byte rows: a wavefront copy moves 4 rows; lane i lands at row i/16, position i%16.
-    // 128-byte rows: 8 rows per copy; lane i lands at row i/8, position i%8.
-    int src256[4], src128[2];   // source byte offsets inside a group of 16 rows, by (copy index & 3) / (& 1)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) src256[v] = (4 * v + (lane >> 4)) * 256 + 16 * ((lane & 15) ^ ((4 * v + (lane >> 4)) & 15));
-#pragma unroll
-    for (int v = 0; v < 2; ++v) src128[v] = (8 * v + (lane >> 3)) * 128 + 16 * ((lane & 7) ^ ((4 * v + (lane >> 4)) & 7));
+    // V: a copy moves 16 rows of 64 bytes; lane i lands at row i / 4, piece i % 4.  Pieces past the last column re-read
+    // the last one (columns are independent and dead ones are not stored).
+    const int v_row = lane >> 2, v_piece = min(KVS * KCT * grp / 8 + (lane & 3), p.Dv / 8 - 1);
+    const char* const my_blobs = p.blobs + ci0 * Blob::kBytes;
     auto issue_copies = [&](int n, int st) {
-      const int64_t ci = ci0 + n;
-      const uint32_t dst = stage_lds + st * kStageBytes;
-      const uint16_t* wn = p.Wn + ci * KC * KD;
-      const uint16_t* qg = p.Qg + ci * KC * KD;
-      const uint16_t* kh = p.KtH + ci * KD * KC;
-      const uint16_t* kl = p.KtL + ci * KD * KC;
+      const uint16_t* src = reinterpret_cast<const uint16_t*>(my_blobs + (int64_t)n * Blob::kBytes);
+      const uint32_t dst = stage_lds + st * kStage;
 #pragma unroll
-      for (int j = pw; j < 16; j += KPW) {
-        copy16_to_lds_async(wn + (j >> 2) * 2048, src256[j & 3], dst + kStageWn + j * 1024);
-        copy16_to_lds_async(qg + (j >> 2) * 2048, src256[j & 3], dst + kStageQg + j * 1024);
+      for (int j = pw; j < NCP; j += KPW) copy16_to_lds_async(src + 512 * j, 16 * lane, dst + 1024 * j);
+      if (pw >= 2) {
+        const int tok = sp.tok0 + n * KC;
+        const int row = min(16 * (pw - 2) + v_row, sp.tok_end - 1 - tok);
+        copy16_to_lds_async(p.v + ((int64_t)tok * p.H + h) * p.Dv, 2 * (row * p.H * p.Dv + 8 * v_piece), dst + kV + 1024 * (pw - 2));
       }
-#pragma unroll
-      for (int j = pw; j < 16; j += KPW) {
-        copy16_to_lds_async(kh + (j >> 1) * 1024, src128[j & 1], dst + kStageKtH + j * 1024);
-        copy16_to_lds_async(kl + (j >> 1) * 1024, src128[j & 1], dst + kStageKtL + j * 1024);
-      }
-      // the 512 bytes of the chunk's decay ride along (half a copy): fetched by the computing wavefronts
-      // themselves they were four more vector-memory instructions per wavefront and chunk, and the number
-      // of such instructions a CU issues per chunk is what the chunk time follows
-      if (pw == 0 && lane < 32) copy16_to_lds_async(reinterpret_cast<const uint16_t*>(p.dec + ci * KD), lane * 16, dst + kStageDec);
     };
-    // The four workgroups of a (batch, head) copy the same 64 KB per chunk at about the same
-    // time and would all wait out the full HBM latency.  Each touches a quarter of a later chunk
-    // (this wavefront 4 KB of it, one dword per 64 bytes) so that the copies find their lines in
-    // L2.  The touching load is the youngest of an iteration: vmcnt(1) then means that every copy
-    // has landed (loads return in order) while the touch stays in flight.  Its target register
-    // is tied up for the whole loop.
+    // The workgroups of a (batch, head) copy the same blocks at about the same time; each asks for its share of the block
+    // two chunks beyond the copies (one dword per 128-byte line, by wavefronts 0 and 1) so that the copies find it in
+    // the L2.  The target register is tied up for the whole loop.
+    constexpr int kAhead = 4;                 // (6 and 8 gave the same time)
     uint32_t touched = 0;
-    constexpr int kAhead = 3;
+    const int t_line = (64 * pw + lane) * NGRP + grp;
+    const int t_off = 128 * min(t_line, Blob::kBytes / 128 - 1);
     auto touch_ahead = [&](int n) {
-      const int64_t ci = ci0 + n;
-      const uint16_t* base = (grp == 0) ? p.Wn + ci * KC * KD : (grp == 1) ? p.Qg + ci * KC * KD
-                           : (grp == 2) ? p.KtH + ci * KD * KC : p.KtL + ci * KD * KC;
-      asm volatile("global_load_dword %0, %1, %2" : "+v"(touched) : "v"(pw * 4096 + lane * 64), "s"(base) : "memory");
+      asm volatile("global_load_dword %0, %1, %2" : "+v"(touched) : "v"(t_off), "s"(my_blobs + (int64_t)n * Blob::kBytes) : "memory");
     };
-    // Output rows of chunk n: 64 rows x 64 bytes, 16 bytes per lane and pass.
-    auto store_o = [&](int n) {
-#pragma unroll
-      for (int k = pw; k < 4; k += KPW) {
-        const int idx = 64 * k + lane, row = idx >> 2, piece = idx & 3;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(&ost[n & 1][row][8 * piece]);
-        const int tok = sp.tok0 + n * KC + row;
-        if (tok < sp.tok_end && KVS * KCT * grp + 8 * piece < p.nv)
-          *reinterpret_cast<u32x4*>(p.o + ((int64_t)tok * p.H + h) * p.Dv + p.v0 + KVS * KCT * grp + 8 * piece) = v;
-      }
+    // Copies of one chunk that this wavefront has in flight: they are its youngest when it waits for the chunk before.
+    static_assert(NCP % KPW == 1 && NCP / KPW + 2 < 16, "copies per wavefront: base + 1 (0), base (1), base + 1 (2, 3: V)");
+    auto older_landed = [&](bool more, bool touching) {
+      constexpr int base = NCP / KPW;
+      if (!more) __builtin_amdgcn_s_waitcnt(0x0F70);
+      else if (pw == 0 && touching) __builtin_amdgcn_s_waitcnt(0x0F70 | (base + 2));
+      else if (pw != 1 || touching) __builtin_amdgcn_s_waitcnt(0x0F70 | (base + 1));
+      else __builtin_amdgcn_s_waitcnt(0x0F70 | base);
+      asm volatile("" ::: "memory");
     };
     if (nc > 0) issue_copies(0, 0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-    asm volatile("" ::: "memory");
+    if (nc > 1) issue_copies(1, 1);
+    older_landed(nc > 1, false);
     __syncthreads();
+    int st = 2;                               // stage of chunk n + 2
     for (int n = 0; n < nc; ++n) {
-      if (n > 0) store_o(n - 1);
-      if (n + 1 < nc) issue_copies(n + 1, (n + 1) & 1);
-      if (NGRP == 4 && n + kAhead < nc) {
-        touch_ahead(n + kAhead);
-        __builtin_amdgcn_s_waitcnt(0x0F71);   // vmcnt(1)
-      } else {
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-      }
-      asm volatile("" ::: "memory");
+      const bool touching = n + kAhead < nc;
+      if (n + 2 < nc) issue_copies(n + 2, st);
+      if (touching && pw < 2) touch_ahead(n + kAhead);
+      older_landed(n + 2 < nc, touching);
+      st = st == KSTAGES - 1 ? 0 : st + 1;
       __syncthreads();
     }
-    if (nc > 0) store_o(nc - 1);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     asm volatile("" :: "v"(touched));
     return;
   }
 
-  // ================= computing wavefronts =================
-  const int ct = wave >> 1, hf = wave & 1;
-  const int vcol = KVS * (KCT * grp + ct) + ln;
-
   // ---- per-lane LDS read offsets (bytes, inside a stage) ------------------------------------
-  // A operand of a 16x16x32 MFMA: lane (row ln, k-group q4) reads chunk 4m + q4 of its row.
-  // Groups of 32 key channels are taken own half first: local group mm is channel group
-  // 2 hf + mm for mm < 2 and 2 (1 - hf) + mm - 2 after that.
-  int rdk[4], rd128[2];
+  // A operand of a 16x16x32 MFMA: lane (row ln, k-group q4) reads piece 4m + q4 of its row; rows 16 apart share a swizzle.
+  const int ct = wave % KCT;
+  int rdk[NM];
 #pragma unroll
-  for (int mm = 0; mm < 4; ++mm) {
-    const int m = (mm < 2) ? 2 * hf + mm : 2 * (1 - hf) + (mm - 2);
-    rdk[mm] = ln * 256 + 16 * ((4 * m + q4) ^ ln);
-  }
-#pragma unroll
-  for (int m = 0; m < 2; ++m) rd128[m] = ln * 128 + 16 * ((4 * m + q4) ^ ((ln >> 1) & 7));
+  for (int m = 0; m < NM; ++m) rdk[m] = ln * 2 * KD + 16 * ((4 * m + q4) ^ piece_swizzle<2 * KD>(ln));
+  const int rd64 = ln * 64 + 16 * (q4 ^ piece_swizzle<64>(ln));
   lds_cptr stage0 = (lds_cptr)&stage[0][0];
+  int so = 0;                                 // stage of the chunk at hand
 
-  // State tile i: rows (key channels) 16*(4 hf + i) + 4*q4 + r, column vcol of this pass; rows beyond Dk and
-  // columns beyond Dv do not exist in the caller's [Dk, Dv] state: they are zero and stay zero.
-  const bool col_live = vcol < p.nv;
-  f32x4 S[4];
+  if (wave >= KCT) {
+    // ================= output wavefront =================
+    const int piece = lane & 1, col = KVS * (KCT * grp + ct) + 8 * piece;
+    f32x4 O[2];
+    bf16x8 ph[2], pl[2];
+    // O(n) += (P T) X, then the 32 rows of 32 bytes leave: two lanes per row
+    auto finish = [&](int n) {
+      const bf16x8 Xh = __builtin_bit_cast(bf16x8, xx[n & 1][ct][0][lane]), Xl = __builtin_bit_cast(bf16x8, xx[n & 1][ct][1][lane]);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+      for (int mt = 0; mt < 2; ++mt) {
+        O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[mt], Xh, O[mt], 0, 0, 0);
+        O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph[mt], Xl, O[mt], 0, 0, 0);
+        O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph[mt], Xh, O[mt], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ost[ct][16 * mt + 4 * q4 + r][ln] = (uint16_t)(pack_bf16x2(O[mt][r], 0.f) & 0xffffu);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const u32x4 v = *reinterpret_cast<const u32x4*>(&ost[ct][lane >> 1][8 * piece]);
+      const int tok = sp.tok0 + n * KC + (lane >> 1);
+      if (tok < sp.tok_end && col < p.Dv) *reinterpret_cast<u32x4*>(p.o + ((int64_t)tok * p.H + h) * p.Dv + col) = v;
+    };
+    __syncthreads();
+    for (int n = 0; n < nc; ++n) {
+      lds_cptr sb = stage0 + so;
+      so = so == (KSTAGES - 1) * kStage ? 0 : so + kStage;
+      if (n > 0) finish(n - 1);
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+        ph[mt] = lds_bf16x8(sb + Blob::kPh + 16 * mt * 64 + rd64);
+        pl[mt] = lds_bf16x8(sb + Blob::kPl + 16 * mt * 64 + rd64);
+        O[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        const bf16x8 Sb = __builtin_bit_cast(bf16x8, xs[n & 1][ct][m][lane]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+          O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds_bf16x8(sb + Blob::kQg + 16 * mt * 2 * KD + rdk[m]), Sb, O[mt], 0, 0, 0);
+      }
+      __syncthreads();
+    }
+    if (nc > 0) finish(nc - 1);
+    return;
+  }
+
+  // ================= chain wavefront =================
+  const int vcol = KVS * (KCT * grp + ct) + ln;
+  const int rdv = kV + (4 * q4 + (ln >> 2)) * 64 + 2 * (KVS * ct + 4 * (ln & 3));
+  // State tile i: rows (key channels) 16*i + 4*q4 + r, column vcol; rows beyond Dk and columns beyond Dv do not
+  // exist in the caller's [Dk, Dv] state: they are zero and stay zero.
+  const bool col_live = vcol < p.Dv;
+  f32x4 S[NS];
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = 16 * (4 * hf + i) + 4 * q4 + r;
-      S[i][r] = (p.s0 && col_live && row < p.Dk) ? p.s0[((int64_t)bh * p.Dk + row) * p.Dv + p.v0 + vcol] : 0.f;
+      const int row = 16 * i + 4 * q4 + r;
+      S[i][r] = (p.s0 && col_live && row < p.Dk) ? p.s0[((int64_t)bh * p.Dk + row) * p.Dv + vcol] : 0.f;
     }
   }
-
-  // What depends on the value column comes straight from global memory, one chunk ahead: U0
-  // (accumulator initial value of U) and this wavefront's rows of P as left operand.
-  auto load_direct = [&](int n, f32x4* u0, bf16x8 (*pa)[2]) {
-    const int64_t ci = ci0 + n;
-    const float* src = p.U0T + (ci * KD + vcol) * KC + 4 * q4;
+  bf16x8 Sb[NM];   // the state as right operand, by channel group
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) u0[mt] = *reinterpret_cast<const f32x4*>(src + 16 * mt);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int m = 0; m < 2; ++m)
-        pa[i][m] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(p.Pm + (ci * KC + 16 * (2 * hf + i) + ln) * KC + 32 * m + 8 * q4));
-  };
-  // Two sets, used in turn by even and odd chunks (the chunk loop is unrolled by two so that no
-  // register copy, which would have to wait for the loads, sits between them and their use).
-  f32x4 u0[2][4];
-  bf16x8 pa[2][2][2];
-  bf16x8 Sb[4];   // the state as right operand, by local channel group
-  Sb[0] = pack_acc2(S[0], S[1]);
-  Sb[1] = pack_acc2(S[2], S[3]);
-  xch[0][wave][0][lane] = __builtin_bit_cast(u32x4, Sb[0]);
-  xch[0][wave][1][lane] = __builtin_bit_cast(u32x4, Sb[1]);
-  if (nc > 0) load_direct(0, u0[0], pa[0]);
+  for (int m = 0; m < NM; ++m) {
+    Sb[m] = pack_acc2(S[2 * m], S[2 * m + 1]);
+    xs[0][ct][m][lane] = __builtin_bit_cast(u32x4, Sb[m]);
+  }
   __syncthreads();
 
-  auto chunk_step = [&](int n, auto parity) {
-    constexpr int st = decltype(parity)::value;
-    f32x4 (&u0c)[4] = u0[st];
-    f32x4 dcc[4];
-    bf16x8 (&pac)[2][2] = pa[st];
-    // The direct loads of the next chunk go out first thing, ahead of the burst of copies of the
-    // data-moving wavefronts (the memory pipeline of a CU is one queue: behind that burst they
-    // would block this wavefront for thousands of cycles), and are waited for at the end of the
-    // chunk, so that no wait for them can end up behind newer loads.
-    if (n + 1 < nc) load_direct(n + 1, u0[st ^ 1], pa[st ^ 1]);
-    __builtin_amdgcn_sched_barrier(0);
-    lds_cptr sb = stage0 + st * kStageBytes;
+  for (int n = 0; n < nc; ++n) {
+    const int par = n & 1;
+    lds_cptr sb = stage0 + so;
+    so = so == (KSTAGES - 1) * kStage ? 0 : so + kStage;
 
-    // LDS operands are read in two batches ahead of the MFMAs that use them instead of each next
-    // to its MFMA, where every MFMA waited for a full LDS latency.
-    Sb[2] = __builtin_bit_cast(bf16x8, xch[st][wave ^ 1][0][lane]);
-    Sb[3] = __builtin_bit_cast(bf16x8, xch[st][wave ^ 1][1][lane]);
-    bf16x8 wa[4][4], qa[2][4], kh[4][2], kl[4][2];
+    // A 16-byte LDS read keeps a wavefront's port for 16 cycles and this wavefront needs forty of them per chunk: what
+    // X needs is read first, everything else between the products and the conversions that do not need it.
+    bf16x8 ka[2][NM], mh[NS], ml[NS];
+    u32x2 vr[2];
+    f32x4 dcc[NS];
 #pragma unroll
-    for (int mm = 0; mm < 4; ++mm) {
+    for (int mt = 0; mt < 2; ++mt) vr[mt] = lds_column4(sb + rdv + 16 * mt * 64);
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) wa[mt][mm] = lds_bf16x8(sb + kStageWn + 4096 * mt + rdk[mm]);
+    for (int m = 0; m < NM; ++m) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) qa[i][mm] = lds_bf16x8(sb + kStageQg + 4096 * (2 * hf + i) + rdk[mm]);
+      for (int mt = 0; mt < 2; ++mt) ka[mt][m] = lds_bf16x8(sb + Blob::kKg + 16 * mt * 2 * KD + rdk[m]);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dcc[i] = *(const f32x4 __attribute__((address_space(3)))*)(sb + kStageDec + 4 * (16 * (4 * hf + i) + 4 * q4));
     __builtin_amdgcn_sched_barrier(0);
 
-    // U = U0 + (-W) S0 (all four row tiles) and O = Qg S0 (this wavefront's two row tiles).
-    // Row tile mt: positions 16*mt + 4*q4 + r, column vcol.
-    f32x4 U[4], O[2];
+    // X = V + (-exp(G) K) S0, row tile mt: positions 16*mt + 4*q4 + r, column vcol
+    f32x4 X[2];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) U[mt] = u0c[mt];
+    for (int mt = 0; mt < 2; ++mt) X[mt] = f32x4{bf16lo_to_f32(vr[mt].x), bf16hi_to_f32(vr[mt].x), bf16lo_to_f32(vr[mt].y), bf16hi_to_f32(vr[mt].y)};
 #pragma unroll
-    for (int i = 0; i < 2; ++i) O[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < NM; ++m) {
 #pragma unroll
-    for (int mm = 0; mm < 4; ++mm) {
+      for (int mt = 0; mt < 2; ++mt) X[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[mt][m], Sb[m], X[mt], 0, 0, 0);
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) U[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[mt][mm], Sb[mm], U[mt], 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[i][mm], Sb[mm], O[i], 0, 0, 0);
+      for (int i = m * NS / NM; i < (m + 1) * NS / NM; ++i) dcc[i] = lds_f32x4(sb + Blob::kDec + 4 * (16 * i + 4 * q4));
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // The operands of the state update are read while those MFMAs run.
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        kh[i][m] = lds_bf16x8(sb + kStageKtH + 2048 * (4 * hf + i) + rd128[m]);
-        kl[i][m] = lds_bf16x8(sb + kStageKtL + 2048 * (4 * hf + i) + rd128[m]);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    bf16x8 Uh[2], Ul[2];
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      Uh[m] = pack_acc2(U[2 * m], U[2 * m + 1]);
-      f32x4 l0, l1;
-      const u32x4 hb = __builtin_bit_cast(u32x4, Uh[m]);
-      l0[0] = U[2 * m][0] - bf16lo_to_f32(hb.x); l0[1] = U[2 * m][1] - bf16hi_to_f32(hb.x);
-      l0[2] = U[2 * m][2] - bf16lo_to_f32(hb.y); l0[3] = U[2 * m][3] - bf16hi_to_f32(hb.y);
-      l1[0] = U[2 * m + 1][0] - bf16lo_to_f32(hb.z); l1[1] = U[2 * m + 1][1] - bf16hi_to_f32(hb.z);
-      l1[2] = U[2 * m + 1][2] - bf16lo_to_f32(hb.w); l1[3] = U[2 * m + 1][3] - bf16hi_to_f32(hb.w);
-      Ul[m] = pack_acc2(l0, l1);
-    }
-
-    // S = exp(G_last) (.) S + Kt^T U, with both operands split into two bf16 terms.
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NS; ++i) {
+      ml[i] = lds_bf16x8(sb + Blob::kMl + 16 * i * 64 + rd64);
+      mh[i] = lds_bf16x8(sb + Blob::kMh + 16 * i * 64 + rd64);
 #pragma unroll
       for (int r = 0; r < 4; ++r) S[i][r] *= dcc[i][r];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // S = exp(G_last) (.) S + M X, both operands split into two bf16 terms
+    const bf16x8 Xh = pack_acc2(X[0], X[1]);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ml[i], Xh, S[i], 0, 0, 0);
+    const bf16x8 Xl = pack_rest2(X[0], X[1], Xh);
+    {
+      xx[par][ct][0][lane] = __builtin_bit_cast(u32x4, Xh);
+      xx[par][ct][1][lane] = __builtin_bit_cast(u32x4, Xl);
     }
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int i = 0; i < NS; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mh[i], Xh, S[i], 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh[i][m], Uh[m], S[i], 0, 0, 0);
-        S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh[i][m], Ul[m], S[i], 0, 0, 0);
-        S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl[i][m], Uh[m], S[i], 0, 0, 0);
-      }
+    for (int i = 0; i < NS; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mh[i], Xl, S[i], 0, 0, 0);
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      Sb[m] = pack_acc2(S[2 * m], S[2 * m + 1]);
+      xs[par ^ 1][ct][m][lane] = __builtin_bit_cast(u32x4, Sb[m]);
     }
-    // O += Pm U (scale already folded into Qg and Pm).  Positions 32..63 of U only reach the
-    // output rows of the second half (P is zero above the diagonal).
-#pragma unroll
-    for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pac[i][0], Uh[0], O[i], 0, 0, 0);
-    if (hf) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pac[i][1], Uh[1], O[i], 0, 0, 0);
-    }
-    // The new state goes to the partner as soon as it exists.
-    Sb[0] = pack_acc2(S[0], S[1]);
-    Sb[1] = pack_acc2(S[2], S[3]);
-    xch[st ^ 1][wave][0][lane] = __builtin_bit_cast(u32x4, Sb[0]);
-    xch[st ^ 1][wave][1][lane] = __builtin_bit_cast(u32x4, Sb[1]);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        ost[st][16 * (2 * hf + i) + 4 * q4 + r][KVS * ct + ln] = (uint16_t)(pack_bf16x2(O[i][r], 0.f) & 0xffffu);
-    }
-
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the direct loads of the next chunk
     __syncthreads();
-  };
-  for (int n = 0; n < nc; n += 2) {
-    chunk_step(n, std::integral_constant<int, 0>{});
-    if (n + 1 < nc) chunk_step(n + 1, std::integral_constant<int, 1>{});
   }
   if (p.s_out != nullptr && col_live) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NS; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = 16 * (4 * hf + i) + 4 * q4 + r;
-        if (row < p.Dk) p.s_out[((int64_t)bh * p.Dk + row) * p.Dv + p.v0 + vcol] = S[i][r];
+        const int row = 16 * i + 4 * q4 + r;
+        if (row < p.Dk) p.s_out[((int64_t)bh * p.Dk + row) * p.Dv + vcol] = S[i][r];
       }
   }
 }
@@ -1149,8 +1035,8 @@ extern "C" int daisy_kda_gate_fwd(const void* g, const float* A_log, const float
 }
 
 
-// Chunk slots of the workspace: B * ceil(T / 64), or for n_seq packed sequences of T tokens in all
-// the upper bound T / 64 + n_seq on sum(ceil(len / 64)).
+// Chunk slots of the workspace: B * ceil(T / 32), or for n_seq packed sequences of T tokens in all
+// the upper bound T / 32 + n_seq on sum(ceil(len / 32)).
 static size_t kda_chunk_slots(int B, int T, int n_seq) {
   return n_seq > 0 ? (size_t)T / KC + (size_t)n_seq : (size_t)B * ((size_t)(T + KC - 1) / KC);
 }
@@ -1159,18 +1045,31 @@ static size_t kda_table_bytes(int T, int n_seq) {
   const size_t ints = 2 * ((size_t)n_seq + 1) + kda_chunk_slots(1, T, n_seq);
   return (ints * sizeof(int32_t) + 255) & ~(size_t)255;
 }
+static size_t kda_blob_bytes(int Dk) { return Dk <= 64 ? KdaBlob<64>::kBytes : KdaBlob<128>::kBytes; }
 
-// Head widths the kernels serve: Dk a multiple of 8 up to 128, Dv any multiple of 8.
-static bool kda_dims_ok(int Dk, int Dv) { return Dk >= 8 && Dk <= KD && Dk % 8 == 0 && Dv >= 8 && Dv % 8 == 0; }
+// Head widths the kernels serve: Dk a multiple of 8 up to 128, Dv any multiple of 8.  `chunk` is the caller's idea of the
+// algorithm's chunk (64); the result does not depend on where the chunks lie, and the kernels use 32.
+constexpr int kApiChunk = 64;
+static bool kda_dims_ok(int Dk, int Dv) { return Dk >= 8 && Dk <= KDMAX && Dk % 8 == 0 && Dv >= 8 && Dv % 8 == 0; }
 
 extern "C" size_t daisy_kda_workspace_bytes(int B, int T, int H, int Dk, int Dv, int chunk) {
-  if (B <= 0 || T <= 0 || H <= 0 || !kda_dims_ok(Dk, Dv) || chunk != KC) return 0;
-  return kda_chunk_slots(B, T, 0) * H * kChunkBytes;
+  if (B <= 0 || T <= 0 || H <= 0 || !kda_dims_ok(Dk, Dv) || chunk != kApiChunk) return 0;
+  return kda_chunk_slots(B, T, 0) * H * kda_blob_bytes(Dk);
 }
 
 extern "C" size_t daisy_kda_varlen_workspace_bytes(int T, int n_seq, int H, int Dk, int Dv, int chunk) {
-  if (T <= 0 || n_seq <= 0 || H <= 0 || !kda_dims_ok(Dk, Dv) || chunk != KC) return 0;
-  return kda_chunk_slots(1, T, n_seq) * H * kChunkBytes + kda_table_bytes(T, n_seq);
+  if (T <= 0 || n_seq <= 0 || H <= 0 || !kda_dims_ok(Dk, Dv) || chunk != kApiChunk) return 0;
+  return kda_chunk_slots(1, T, n_seq) * H * kda_blob_bytes(Dk) + kda_table_bytes(T, n_seq);
+}
+
+template <int KD>
+static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
+  const int groups = (p.Dv + KVS * KCT - 1) / (KVS * KCT);
+  hipLaunchKernelGGL(kda_prep_kernel<KD>, dim3((p.NC + 1) / 2, p.H, p.n_seq > 0 ? 1 : p.B), dim3(256), 0, s, p);
+  DAISY_CHECK_LAUNCH("kda_prep_kernel");
+  hipLaunchKernelGGL(kda_state_kernel<KD>, dim3((unsigned)(n_streams * p.H * groups)), dim3(kStateThreads), 0, s, p);
+  DAISY_CHECK_LAUNCH("kda_state_kernel");
+  return DAISY_OK;
 }
 
 // Shared by the batched and the packed entry point (n_seq == 0: batched).
@@ -1181,22 +1080,23 @@ static int kda_chunk_launch(const void* q, const void* k, const void* v,
                             int B, int T, int H, int Dk, int Dv, int chunk,
                             float scale, int l2norm_qk, float l2_eps,
                             void* workspace, size_t workspace_bytes, void* stream) {
-  DAISY_CHECK_SUPPORTED(kda_dims_ok(Dk, Dv), "kda: Dk=%d, Dv=%d not supported (Dk: a multiple of 8 up to %d; Dv: a multiple of 8)", Dk, Dv, KD);
-  DAISY_CHECK_SUPPORTED(chunk == KC, "kda: chunk=%d not supported (must be %d)", chunk, KC);
+  DAISY_CHECK_SUPPORTED(kda_dims_ok(Dk, Dv), "kda: Dk=%d, Dv=%d not supported (Dk: a multiple of 8 up to %d; Dv: a multiple of 8)", Dk, Dv, KDMAX);
+  DAISY_CHECK_SUPPORTED(chunk == kApiChunk, "kda: chunk=%d not supported (must be %d)", chunk, kApiChunk);
   DAISY_CHECK_ARG(q && k && v && g && beta && o, "kda: q, k, v, g, beta and o must be non-NULL");
   DAISY_CHECK_ARG(B > 0 && T > 0 && H > 0, "kda: B=%d, T=%d, H=%d must be positive", B, T, H);
   DAISY_CHECK_ARG(B <= 65535 && H <= 65535, "kda: B and H must each be <= 65535");
   DAISY_CHECK_ARG((int64_t)B * T <= 0x7fffffff, "kda: B*T too large");
+  DAISY_CHECK_ARG((int64_t)H * Dk * KC < 0x7fffffff && (int64_t)H * Dv * KC * 2 < 0x7fffffff, "kda: token rows too long");
   auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
   DAISY_CHECK_ARG(al16(q) && al16(k) && al16(v) && al16(g) && al16(o) && al16(workspace),
                   "kda: tensors and workspace must be 16-byte aligned");
   const size_t slots = kda_chunk_slots(B, T, n_seq);
-  const size_t need = slots * H * kChunkBytes + kda_table_bytes(T, n_seq);
+  const size_t need = slots * H * kda_blob_bytes(Dk) + kda_table_bytes(T, n_seq);
   if (!workspace || workspace_bytes < need) {
     set_error("kda: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
     return DAISY_ERR_WORKSPACE;
   }
-  DAISY_CHECK_ARG(slots <= 0x7fffffff && (int64_t)(n_seq > 0 ? n_seq : B) * H * (KD / (KVS * KCT)) <= 0x7fffffff,
+  DAISY_CHECK_ARG(slots <= 0x7fffffff && (int64_t)(n_seq > 0 ? n_seq : B) * H * ((Dv + KVS * KCT - 1) / (KVS * KCT)) <= 0x7fffffff,
                   "kda: too many chunks or sequences");
   KdaParams p;
   p.q = (const uint16_t*)q; p.k = (const uint16_t*)k; p.v = (const uint16_t*)v;
@@ -1206,15 +1106,9 @@ static int kda_chunk_launch(const void* q, const void* k, const void* v,
   p.NC = n_seq > 0 ? (int)slots : (T + KC - 1) / KC;
   p.nc_total = (int)slots;
   p.scale = scale; p.l2norm = l2norm_qk; p.l2eps = l2_eps;
-  const size_t chunks = slots * H;
   char* w = (char*)workspace;
-  p.Wn = (uint16_t*)w;  w += chunks * KC * KD * 2;
-  p.Qg = (uint16_t*)w;  w += chunks * KC * KD * 2;
-  p.KtH = (uint16_t*)w; w += chunks * KD * KC * 2;
-  p.KtL = (uint16_t*)w; w += chunks * KD * KC * 2;
-  p.U0T = (float*)w;    w += chunks * KD * KC * 4;
-  p.Pm = (uint16_t*)w;  w += chunks * KC * KC * 2;
-  p.dec = (float*)w;    w += chunks * KD * 4;
+  p.blobs = w;
+  w += slots * H * kda_blob_bytes(Dk);
   p.n_seq = n_seq; p.bounds = p.seq_chunk0 = p.chunk_seq = nullptr;
   hipStream_t s = (hipStream_t)stream;
   if (n_seq > 0) {
@@ -1226,17 +1120,7 @@ static int kda_chunk_launch(const void* q, const void* k, const void* v,
   }
   const int n_streams = n_seq > 0 ? n_seq : B;    // independent recurrences per head
   p.Dk = Dk; p.Dv = Dv;
-  // Value columns are independent: passes of up to 128 columns, each through the same workspace (the
-  // launches of one stream run in order).
-  for (int v0 = 0; v0 < Dv; v0 += KD) {
-    p.v0 = v0; p.nv = Dv - v0 < KD ? Dv - v0 : KD;
-    const int groups = (p.nv + KVS * KCT - 1) / (KVS * KCT);
-    hipLaunchKernelGGL(kda_prep_kernel, dim3(p.NC, H, n_seq > 0 ? 1 : B), dim3(256), 0, s, p);
-    DAISY_CHECK_LAUNCH("kda_prep_kernel");
-    hipLaunchKernelGGL(kda_state_kernel, dim3((unsigned)(n_streams * H * groups)), dim3(64 * (KSW + KPW)), 0, s, p);
-    DAISY_CHECK_LAUNCH("kda_state_kernel");
-  }
-  return DAISY_OK;
+  return Dk <= 64 ? kda_launch_width<64>(p, n_streams, s) : kda_launch_width<128>(p, n_streams, s);
 }
 
 extern "C" int daisy_kda_chunk_fwd(const void* q, const void* k, const void* v,

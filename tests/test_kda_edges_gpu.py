@@ -1,0 +1,59 @@
+"""Chunked KDA at the edges of its tiling: chunks of 32 positions handled in pairs, key widths of 64 and 128 channels, groups
+of 32 value columns, and keys that overlap so strongly that the triangle's inverse carries the result."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import oracle
+from daisy_amd import chunk_kda
+from helpers import assert_close_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(B, T, H, Dk, Dv, seed, overlap=0.0):
+    g = torch.Generator().manual_seed(seed)
+    q, k = (F.normalize(torch.randn(B, T, H, Dk, generator=g), dim=-1) for _ in range(2))
+    k = F.normalize((1 - overlap) * k + overlap * k[:, :1], dim=-1)
+    v = torch.randn(B, T, H, Dv, generator=g)
+    gl = F.logsigmoid(torch.randn(B, T, H, Dk, generator=g) + 3 * overlap)
+    beta = torch.sigmoid(torch.randn(B, T, H, generator=g) + 3 * overlap)
+    return q.bfloat16(), k.bfloat16(), v.bfloat16(), gl, beta
+
+
+def _run(q, k, v, gl, beta, **kw):
+    o, S = chunk_kda(q.cuda(), k.cuda(), v.cuda(), gl.cuda(), beta.cuda(), output_final_state=True, use_qk_l2norm_in_kernel=True, **kw)
+    return o.cpu(), S.cpu()
+
+
+@pytest.mark.parametrize("Dk,Dv", [(64, 32), (72, 40), (128, 128)])
+@pytest.mark.parametrize("T", [1, 16, 31, 32, 33, 63, 65, 96, 97, 161])
+def test_kda_chunk_edges(T, Dk, Dv):
+    q, k, v, gl, beta = _inputs(2, T, 2, Dk, Dv, seed=T + Dk)
+    o_ref, S_ref = oracle.kda_recurrent(q, k, v, gl, beta)
+    o, S = _run(q, k, v, gl, beta)
+    assert_close_bf16(o, o_ref, "o")
+    assert ((S - S_ref).norm() / S_ref.norm()).item() <= 1e-3
+
+
+@pytest.mark.parametrize("overlap", [0.5, 0.9])
+def test_kda_overlapping_keys(overlap):
+    q, k, v, gl, beta = _inputs(1, 160, 2, 128, 64, seed=3, overlap=overlap)
+    o_ref, S_ref = oracle.kda_recurrent(q, k, v, gl, beta)
+    o, S = _run(q, k, v, gl, beta)
+    assert_close_bf16(o, o_ref, "o")
+    assert ((S - S_ref).norm() / S_ref.norm()).item() <= 1e-3
+
+
+@pytest.mark.parametrize("lengths", [(1, 31, 0, 32, 33, 64, 5), (97,), (32, 32)])
+def test_kda_packed_chunk_slots(lengths):
+    q, k, v, gl, beta = _inputs(1, sum(lengths), 3, 64, 64, seed=sum(lengths))
+    cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32)
+    o, S = _run(q, k, v, gl, beta, cu_seqlens=cu.cuda())
+    for i, n in enumerate(lengths):
+        a = int(cu[i])
+        if n == 0:
+            continue
+        o_ref, S_ref = oracle.kda_recurrent(*(t[:, a:a + n] for t in (q, k, v, gl, beta)))
+        assert_close_bf16(o[:, a:a + n], o_ref, f"sequence {i}: o")
+        assert ((S[i:i + 1] - S_ref).norm() / S_ref.norm()).item() <= 1e-3
