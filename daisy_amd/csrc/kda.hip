@@ -1045,7 +1045,8 @@ static size_t kda_table_bytes(int T, int n_seq) {
   const size_t ints = 2 * ((size_t)n_seq + 1) + kda_chunk_slots(1, T, n_seq);
   return (ints * sizeof(int32_t) + 255) & ~(size_t)255;
 }
-static size_t kda_blob_bytes(int Dk) { return Dk <= 64 ? KdaBlob<64>::kBytes : KdaBlob<128>::kBytes; }
+// The workspace is sized for the widest heads whatever the width (part of the contract); narrower ones leave its end untouched.
+constexpr size_t kBlobBytes = KdaBlob<128>::kBytes;
 
 // Head widths the kernels serve: Dk a multiple of 8 up to 128, Dv any multiple of 8.  `chunk` is the caller's idea of the
 // algorithm's chunk (64); the result does not depend on where the chunks lie, and the kernels use 32.
@@ -1054,12 +1055,12 @@ static bool kda_dims_ok(int Dk, int Dv) { return Dk >= 8 && Dk <= KDMAX && Dk % 
 
 extern "C" size_t daisy_kda_workspace_bytes(int B, int T, int H, int Dk, int Dv, int chunk) {
   if (B <= 0 || T <= 0 || H <= 0 || !kda_dims_ok(Dk, Dv) || chunk != kApiChunk) return 0;
-  return kda_chunk_slots(B, T, 0) * H * kda_blob_bytes(Dk);
+  return kda_chunk_slots(B, T, 0) * H * kBlobBytes;
 }
 
 extern "C" size_t daisy_kda_varlen_workspace_bytes(int T, int n_seq, int H, int Dk, int Dv, int chunk) {
   if (T <= 0 || n_seq <= 0 || H <= 0 || !kda_dims_ok(Dk, Dv) || chunk != kApiChunk) return 0;
-  return kda_chunk_slots(1, T, n_seq) * H * kda_blob_bytes(Dk) + kda_table_bytes(T, n_seq);
+  return kda_chunk_slots(1, T, n_seq) * H * kBlobBytes + kda_table_bytes(T, n_seq);
 }
 
 template <int KD>
@@ -1091,7 +1092,7 @@ static int kda_chunk_launch(const void* q, const void* k, const void* v,
   DAISY_CHECK_ARG(al16(q) && al16(k) && al16(v) && al16(g) && al16(o) && al16(workspace),
                   "kda: tensors and workspace must be 16-byte aligned");
   const size_t slots = kda_chunk_slots(B, T, n_seq);
-  const size_t need = slots * H * kda_blob_bytes(Dk) + kda_table_bytes(T, n_seq);
+  const size_t need = slots * H * kBlobBytes + kda_table_bytes(T, n_seq);
   if (!workspace || workspace_bytes < need) {
     set_error("kda: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
     return DAISY_ERR_WORKSPACE;
@@ -1108,7 +1109,7 @@ static int kda_chunk_launch(const void* q, const void* k, const void* v,
   p.scale = scale; p.l2norm = l2norm_qk; p.l2eps = l2_eps;
   char* w = (char*)workspace;
   p.blobs = w;
-  w += slots * H * kda_blob_bytes(Dk);
+  w += slots * H * kBlobBytes;
   p.n_seq = n_seq; p.bounds = p.seq_chunk0 = p.chunk_seq = nullptr;
   hipStream_t s = (hipStream_t)stream;
   if (n_seq > 0) {

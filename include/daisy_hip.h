@@ -256,7 +256,7 @@ int daisy_attn_step_fwd(const void* q, const int64_t* q_strides,
  * initial_state : fp32 [B, H, Dk, Dv] or NULL (zeros).
  * final_state   : fp32 [B, H, Dk, Dv] or NULL (not wanted).
  * Dk: a multiple of 8 up to 128.  Dv: any multiple of 8 (value columns are independent).  chunk = 64
- * (the size of the workspace and the result do not depend on it).  T is arbitrary.  The kernels are laid out for
+ * (the result does not depend on it).  T is arbitrary.  The kernels are laid out for
  * 64 or 128 key channels (narrower heads cost what the next width costs) and groups of 32 value columns.
  * l2norm_qk : normalise q and k rows as x / sqrt(sum(x^2) + l2_eps) first.
  * workspace : >= daisy_kda_workspace_bytes(...) bytes, 256-byte aligned.
