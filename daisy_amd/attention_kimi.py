@@ -31,7 +31,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from . import ops
+from . import _lib, ops
 from . import attention as _attention
 from .attention import step_linear
 from .kda import chunk_kda, fused_kda_gate, fused_recurrent_kda
@@ -84,6 +84,11 @@ def _project(lin: nn.Linear, x: Tensor) -> Tensor:
     if lin.bias is None:
         return step_linear(x, lin.weight)
     return lin(x)
+
+
+def _plain(module: nn.Module, cls: type) -> bool:
+    """Whether calling ``module`` is calling ``cls.forward`` and nothing else."""
+    return type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks
 
 
 class KimiLinearSelfAttention(nn.Module):
@@ -223,10 +228,54 @@ class KimiLinearSelfAttention(nn.Module):
             return home
         return fresh
 
+    def _fast(self, x: Tensor, use_cache: bool) -> Optional[Tensor]:
+        """The whole layer through one call of the native extension (a decode step: three launches; a prompt: the library's large
+        products and seven launches), or None: autograd, other dtypes or layouts, replaced submodules or hooks."""
+        m = self._modules
+        try:
+            lins = (m["q_proj"], m["k_proj"], m["v_proj"], m["f_proj"]._modules["0"], m["g_proj"]._modules["0"], m["b_proj"],
+                    m["f_proj"]._modules["1"], m["o_proj"])
+            g1, convs, norm = m["g_proj"]._modules["1"], (m["q_conv1d"], m["k_conv1d"], m["v_conv1d"]), m["o_norm"]
+            if not (_plain(g1, nn.Linear) and _plain(norm, GatedRMSNorm) and all([_plain(c, ShortConvolution) for c in convs])
+                    and all([l._parameters["bias"] is None for l in lins])):
+                return None
+            w = [l._parameters["weight"] for l in lins]
+            weights = (*w[:7], g1._parameters["weight"], g1._parameters["bias"], w[7], *[c._parameters["weight"] for c in convs],
+                       *[c._parameters.get("bias") for c in convs], self._parameters["A_log"], self._parameters["dt_bias"],
+                       norm._parameters["weight"])
+        except (KeyError, AttributeError):
+            return None
+        state = windows = None
+        homes = (None, None, None, None)
+        if use_cache:
+            state, windows = self._recurrent_state, self._conv_state
+            if self._state_homes:
+                homes = self._state_homes.get(x.shape[0], homes)
+        out = _lib.native().kda_layer(x.contiguous(), weights, self.num_heads, self.head_k_dim, self.head_v_dim, self.conv_size, state,
+                                      windows or (None, None, None), homes, use_cache, norm.eps, _attention.STEP_ROWS_KERNEL_MAX)
+        if out is None:
+            return None
+        if use_cache:
+            if out[1] is not state or out[2] is not windows[0]:     # (a step updates what is carried in place)
+                self._keep(x.shape[0], out[1], out[2:])
+            self._seen += x.shape[1]
+        return out[0]
+
+    def _keep(self, states: int, state: Tensor, windows) -> None:
+        """Stores the states after a prompt where those of the last prompt of that batch size were."""
+        homes = self._state_homes.get(states, (None, None, None, None))
+        self._recurrent_state = self._store(homes[0], state)
+        self._conv_state = tuple(self._store(h, c) for h, c in zip(homes[1:], windows))
+        self._state_homes[states] = (self._recurrent_state,) + self._conv_state
+
     def _core(self, x: Tensor, ve: Optional[Tensor], use_cache: bool, attn_mask=None) -> Tensor:
         B0, S0, _ = x.shape
         H, Dk, Dv = self.num_heads, self.head_k_dim, self.head_v_dim
         x = x.to(self.q_proj.weight.dtype)
+        if x.is_cuda and self.use_short_conv and not self.receives_ve and not (isinstance(attn_mask, Tensor) and attn_mask.ndim == 2):
+            y = self._fast(x, use_cache)
+            if y is not None:
+                return y
         indices = cu_seqlens = None
         if isinstance(attn_mask, Tensor) and attn_mask.ndim == 2:
             # get_unpad_data of the reference's dependency, restated: positions of the tokens in the
@@ -265,10 +314,7 @@ class KimiLinearSelfAttention(nn.Module):
             o, state = chunk_kda(q, k, v, g, beta, initial_state=state, output_final_state=use_cache,
                                  use_qk_l2norm_in_kernel=True, cu_seqlens=cu_seqlens)
         if use_cache:
-            homes = self._state_homes.get(state.shape[0], (None, None, None, None))
-            self._recurrent_state = self._store(homes[0], state)
-            self._conv_state = tuple(self._store(h, c) for h, c in zip(homes[1:], (cq, ck, cv)))
-            self._state_homes[state.shape[0]] = (self._recurrent_state,) + self._conv_state
+            self._keep(state.shape[0], state, (cq, ck, cv))
             self._seen += T
         # (contiguous rows: the library adds the bias inside the product then, as it does for the reference's tensors)
         gate = self.g_proj[1](g_low.contiguous()).view(B, T, H, Dv)

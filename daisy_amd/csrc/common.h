@@ -91,6 +91,15 @@ template <typename E> __device__ __forceinline__ float round_elem(float x);
 template <> __device__ __forceinline__ float round_elem<uint16_t>(float x) { return round_bf16(x); }
 template <> __device__ __forceinline__ float round_elem<float>(float x) { return x; }
 
+// softplus(v) with slope `beta`, linear above the threshold: (max(bx, 0) + log1p(exp(-|bx|))) / beta with bx = beta v; log1p
+// by its series below 1/64 (error < 1e-6 of the value), by the hardware logarithm above (1 + t is exact enough there).
+__device__ __forceinline__ float softplus(float v, float beta, float threshold, float inv_beta) {
+  const float bx = v * beta;
+  const float t = __expf(-fabsf(bx));
+  const float l = (t < 0.015625f) ? t * (1.f - t * (0.5f - 0.33333334f * t)) : __logf(1.f + t);
+  return (bx > threshold) ? v : (fmaxf(bx, 0.f) + l) * inv_beta;
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // ---- cross-lane sums with DPP (no LDS traffic) -------------------------------

@@ -34,6 +34,19 @@ struct QkvEpilogue {
 // y [M, N] = x [M, K] w [N, K]^T (+ bias), fp32 accumulation, one rounding.  tile: 0 = by the sizes.
 int proj_linear(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const uint16_t* bias,
                 uint16_t* y, int64_t y_sm, int M, int N, int K, hipStream_t s, int tile = 0);
+// One of several products over the same number of rows M and the same K that share a launch: y = x w^T (+ bias).  N need not be a
+// multiple of 8 where y's rows have room for it (y_sm >= N rounded up to 8; the columns from N on are then scribbled over).
+struct ProjSegment {
+  const uint16_t* x; int64_t x_sm;
+  const uint16_t* w; int64_t w_sn;
+  const uint16_t* bias;
+  uint16_t* y; int64_t y_sm;
+  int N, tile_end;      // tile_end: filled in by the launch
+};
+constexpr int kMaxSegments = 6;
+int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, int tile = 0);
+// The same through the weight-streaming kernel of linear.hip, M <= 8 (no bias); every row as daisy_linear_rows_fwd computes it.
+int linear_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s);
 // Whether the tiled kernel is the better choice for these sizes than the library GEMM (and, for the QKV projection, than
 // the library GEMM with qkv_prep_kernel behind it).
 bool proj_wanted(int M, int N, int K);
@@ -75,5 +88,25 @@ int prep_launch(const void* q, const int64_t* q_strides, const void* k, const in
                 const float* cos, const float* sin, int pos0, const int32_t* pos0_dev, int table_rows, int32_t* status,
                 void* q_out, const int64_t* q_out_strides, void* k_out, const int64_t* k_out_strides,
                 void* v_out, const int64_t* v_out_strides, int B, int T, int H, int D, float eps, void* stream);
+
+// A decode step of the KDA layer (attention_kimi.py) between its first and its last projection, one token per sequence: short
+// convolutions with SiLU (windows shifted in place), the second halves of the two low-rank projections, decay gate,
+// beta, delta-rule update of the state (in place), gated RMS norm.  Rows of q, k, v, f, g, b: one per sequence, `row`
+// elements apart.
+struct KdaLayerStep {
+  const uint16_t *q, *k, *v, *f, *g, *b; int64_t q_row, k_row, v_row, f_row, g_row, b_row;
+  const uint16_t* conv_w[3]; const uint16_t* conv_bias[3]; uint16_t* window[3]; int taps;     // [C, taps], [C] or NULL, [B, C, taps]
+  const uint16_t *wf, *wg, *g_bias;       // [H * Dk, Dv], [H * Dv, Dv], [H * Dv] or NULL
+  const float *A_log, *dt_bias;           // [H], [H * Dk]
+  const uint16_t* norm_w;                 // [Dv]
+  float* state;                           // [B, H, Dk, Dv]
+  uint16_t* o; int64_t o_row;             // [B, H * Dv]
+  int H, Dk; float scale, l2_eps, norm_eps;
+};
+// daisy_kda_gate_fwd (bf16, slope 1, threshold 20) and beta = bf16(sigmoid(logits)) as fp32 [rows, H] in one launch; out may be g.
+int kda_gate_beta(const uint16_t* g, const float* A_log, const float* bias, uint16_t* out, const uint16_t* logits, int64_t logits_row,
+                  float* beta, int64_t rows, int H, int Dk, hipStream_t s);
+bool kda_layer_step_serves(int Dk, int Dv, int taps);
+int kda_layer_step(const KdaLayerStep& p, int B, int Dv, hipStream_t s);
 
 }  // namespace daisy

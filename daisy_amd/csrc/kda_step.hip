@@ -16,6 +16,8 @@
 // 8 dq lanes of a column group with cross-lane moves.
 #include "common.h"
 
+#include <type_traits>
+
 namespace daisy {
 
 constexpr int RD = 128;   // key channels and value columns a workgroup works on
@@ -146,6 +148,256 @@ __global__ __launch_bounds__(256) void kda_recurrent_kernel(KdaStepParams p) {
     for (int i = 0; i < 16; ++i)
       if (16 * dq + i < p.Dk) __builtin_nontemporal_store(S[i], reinterpret_cast<f32x4*>(p.s_out + sbase + (int64_t)i * p.Dv));
   }
+}
+
+// The same step with everything of the KDA layer that lies between its projections.
+//
+// What bounds it: HBM, the state in and out (134 MB for 64 sequences of 16 heads of 128 x 128: 27.6 us at what a copy
+// reaches, 33 us measured).  As separate launches the token passed through eleven kernels (three convolutions, two
+// projections from the low rank, gate, two for beta, recurrence, copy, norm), 70 us of GPU time and as much again between them.  Here one
+// workgroup per (sequence, head) requests its inputs, then its state, and does the small work while the state arrives:
+// the two products from the low rank are 32 KB of weights per head and matrix, read through the L2 by all sequences.
+// VD / 16 wavefronts; wavefront w owns value columns [32 (w / 2), .. + 32) of half w % 2 of the key channels, lane (dq, jc)
+// channels KD / 16 dq .. of that half and columns 4 jc ..: rows of 128 bytes as in kda_recurrent_kernel (with 64-byte
+// rows the step of 64 sequences took 3 us more), and half as much state per lane, so that the weights fit beside it in
+// 128 registers.  The
+// products run on the matrix cores, weights as left operand straight from memory and all sixteen columns of the right
+// operand the same row: fifteen of them are waste, but nothing is unpacked and nothing summed across lanes.
+__device__ __forceinline__ float sum_over_rows(float x) {          // lane bits 3, 4, 5
+  x = dpp_add<0x128>(x);                 // row_ror 8
+  u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+  x = __uint_as_float(t.x) + __uint_as_float(t.y);
+  t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+  return __uint_as_float(t.x) + __uint_as_float(t.y);
+}
+template <int KD, int VD>
+__global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep p) {
+  constexpr int NW = VD / 16, NT = 64 * NW, ROWS = KD / 16;
+  // Outputs of the low-rank products: tiles of 16 decay channels, then of 16 gate channels; wavefront w makes tiles w + NW t.
+  constexpr int SLOTS = KD + VD, TILES = SLOTS / 16, TPW = (TILES + NW - 1) / NW, KS = VD / 32;
+  constexpr int CH = 2 * KD + VD, CROUNDS = (CH + NT - 1) / NT;   // convolution channels: q, k, v
+  __shared__ __attribute__((aligned(16))) float qkv[CH];
+  __shared__ __attribute__((aligned(16))) float eg_gate[SLOTS];   // exp(g), then sigmoid(gate)
+  __shared__ __attribute__((aligned(16))) f32x4 part[2][2][VD / 4];   // [half][prediction, read-out][columns]
+  __shared__ float red[VD / 32];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = wave & 1, dq = lane >> 3, jc = lane & 7, d0 = KD / 2 * half + ROWS * dq;     // d0: this lane's first key channel
+  const int ln = lane & 15, q4 = lane >> 4;                       // matrix operands: row or column ln, contraction group q4
+  const int h = blockIdx.x % p.H, b = blockIdx.x / p.H;
+  const int Dk = p.Dk;
+
+  // ---- requests: the low-rank rows and weights, the convolutions' inputs, the state --------------------------------
+  u32x4 low_f[KS], low_g[KS], wv[TPW][KS];
+#pragma unroll
+  for (int m = 0; m < KS; ++m) {
+    low_f[m] = *reinterpret_cast<const u32x4*>(p.f + b * p.f_row + 32 * m + 8 * q4);
+    low_g[m] = *reinterpret_cast<const u32x4*>(p.g + b * p.g_row + 32 * m + 8 * q4);
+  }
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) {
+    const int s0 = 16 * min(wave + NW * t, TILES - 1);            // (surplus tiles redo the last one)
+    const uint16_t* w = s0 < KD ? p.wf + ((int64_t)h * Dk + min(s0 + ln, Dk - 1)) * VD    // (channels beyond Dk re-read the last row)
+                                : p.wg + ((int64_t)h * VD + s0 - KD + ln) * VD;
+#pragma unroll
+    for (int m = 0; m < KS; ++m) wv[t][m] = *reinterpret_cast<const u32x4*>(w + 32 * m + 8 * q4);
+  }
+  // Taps and window of a channel as four bf16 aligned at the newest end: tap 3 meets the new input, window entry j tap j - 1.
+  float xin[CROUNDS], cb[CROUNDS];
+  u32x2 cw[CROUNDS], win[CROUNDS];
+#pragma unroll
+  for (int r = 0; r < CROUNDS; ++r) {
+    const int c = tid + NT * r, kind = c < KD ? 0 : c < 2 * KD ? 1 : 2, d = c - KD * kind, D = kind == 2 ? VD : Dk;
+    xin[r] = 0.f;
+    if (c >= CH || d >= D) continue;                              // (channels beyond Dk: zeros)
+    const int ch = h * D + d;
+    const uint16_t* x = kind == 0 ? p.q + b * p.q_row : kind == 1 ? p.k + b * p.k_row : p.v + b * p.v_row;
+    const uint16_t *wp = p.conv_w[kind] + (int64_t)ch * p.taps, *cp = p.window[kind] + ((int64_t)b * p.H * D + ch) * p.taps;
+    xin[r] = bf16lo_to_f32(x[ch]);
+    cb[r] = p.conv_bias[kind] != nullptr ? bf16lo_to_f32(p.conv_bias[kind][ch]) : 0.f;
+    if (p.taps == 4) {
+      cw[r] = *reinterpret_cast<const u32x2*>(wp);
+      win[r] = *reinterpret_cast<const u32x2*>(cp);
+    } else {
+      const uint32_t w0 = p.taps == 3 ? wp[0] : 0, c0 = p.taps == 3 ? cp[0] : 0;
+      cw[r] = u32x2{w0 << 16, (uint32_t)wp[p.taps - 2] | (uint32_t)wp[p.taps - 1] << 16};
+      win[r] = u32x2{c0 << 16, (uint32_t)cp[p.taps - 2] | (uint32_t)cp[p.taps - 1] << 16};
+    }
+  }
+  const float b_logit = bf16lo_to_f32(p.b[b * p.b_row + h]);
+  const int col = 32 * (wave >> 1) + 4 * jc;
+  float* const state = p.state + ((int64_t)blockIdx.x * Dk + d0) * VD + col;
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 S[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (d0 + i < Dk) S[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(state + i * VD));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- convolutions ----------------------------------------------------------------------------------------------
+#pragma unroll
+  for (int r = 0; r < CROUNDS; ++r) {
+    const int c = tid + NT * r, kind = c < KD ? 0 : c < 2 * KD ? 1 : 2, d = c - KD * kind, D = kind == 2 ? VD : Dk;
+    if (c >= CH) continue;
+    float a = 0.f;
+    if (d < D) {
+      a = cb[r];
+      a = fmaf(bf16lo_to_f32(cw[r].x), bf16hi_to_f32(win[r].x), a);
+      a = fmaf(bf16hi_to_f32(cw[r].x), bf16lo_to_f32(win[r].y), a);
+      a = fmaf(bf16lo_to_f32(cw[r].y), bf16hi_to_f32(win[r].y), a);
+      a = round_bf16(fmaf(bf16hi_to_f32(cw[r].y), xin[r], a));
+      a = round_bf16(a * __builtin_amdgcn_rcpf(1.f + __expf(-a)));
+      uint16_t* cp = p.window[kind] + ((int64_t)b * p.H * D + h * D + d) * p.taps;
+      const u32x2 next = {win[r].x >> 16 | win[r].y << 16, win[r].y >> 16 | __float_as_uint(xin[r])};
+      if (p.taps == 4) *reinterpret_cast<u32x2*>(cp) = next;
+      else {
+        if (p.taps == 3) cp[0] = (uint16_t)(next.x >> 16);
+        cp[p.taps - 2] = (uint16_t)next.y;
+        cp[p.taps - 1] = (uint16_t)(next.y >> 16);
+      }
+    }
+    qkv[c] = a;
+  }
+  // ---- g = f wf^T and gate = g wg^T + bias: every column of a tile is the same; lane (ln, q4) takes row 4 q4 + ln % 4 of
+  // tile ln / 4 of every four
+#pragma unroll
+  for (int t0 = 0; t0 < TPW; t0 += 4) {
+    f32x4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (t0 + t >= TPW) continue;
+      const bool decay = 16 * (wave + NW * (t0 + t)) < KD;
+#pragma unroll
+      for (int m = 0; m < KS; ++m)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[t0 + t][m]),
+                                                         __builtin_bit_cast(bf16x8, decay ? low_f[m] : low_g[m]), acc[t], 0, 0, 0);
+    }
+    f32x4 mine = acc[0];
+#pragma unroll
+    for (int t = 1; t < 4; ++t) mine = (ln >> 2) == t ? acc[t] : mine;
+    float x = mine[0];
+#pragma unroll
+    for (int r = 1; r < 4; ++r) x = (ln & 3) == r ? mine[r] : x;
+    const int t = t0 + (ln >> 2), slot = 16 * (wave + NW * t) + 4 * q4 + (ln & 3);
+    if (t < TPW && slot < SLOTS) {
+      float y;
+      if (slot < KD) {
+        // every intermediate rounded as the tensor that holds it in the layer
+        const int d = min(slot, Dk - 1);
+        const float gl = -expf(p.A_log[h]) * softplus(round_bf16(x) + p.dt_bias[h * Dk + d], 1.f, 20.f, 1.f);
+        y = slot < Dk ? __expf(round_bf16(gl)) : 1.f;
+      } else {
+        if (p.g_bias != nullptr) x += bf16lo_to_f32(p.g_bias[h * VD + slot - KD]);
+        y = __builtin_amdgcn_rcpf(1.f + __expf(-round_bf16(x)));
+      }
+      eg_gate[slot] = y;
+    }
+  }
+  const float beta = round_bf16(1.f / (1.f + expf(-b_logit)));
+  __syncthreads();
+
+  // ---- the delta rule; q and k L2-normalised (every wavefront sums for itself) ---------------------------------------
+  float qs = 0.f, ks = 0.f, kq = 0.f;
+#pragma unroll
+  for (int e = 0; e < KD / 64; ++e) {
+    const float q1 = qkv[lane + 64 * e], k1 = qkv[KD + lane + 64 * e];
+    qs = fmaf(q1, q1, qs);
+    ks = fmaf(k1, k1, ks);
+    kq = fmaf(k1, q1, kq);
+  }
+  qs = sum_over_rows(group_sum<8>(qs));
+  ks = sum_over_rows(group_sum<8>(ks));
+  kq = sum_over_rows(group_sum<8>(kq));
+  const float qn = rsqrtf(qs + p.l2_eps), kn = rsqrtf(ks + p.l2_eps);
+  kq *= kn * qn;
+  // With S the decayed state: pred = S^T k, delta = beta (v - pred), the new state S + k delta^T and its read-out
+  // S^T q + (k . q) delta: both products over the old state in one pass and one round of cross-lane sums.
+  f32x4 pred = {0.f, 0.f, 0.f, 0.f}, out = {0.f, 0.f, 0.f, 0.f};
+  float kk[ROWS];
+#pragma unroll
+  for (int i4 = 0; i4 < ROWS / 4; ++i4) {
+    const f32x4 e4 = *reinterpret_cast<const f32x4*>(&eg_gate[d0 + 4 * i4]);
+    const f32x4 k4 = *reinterpret_cast<const f32x4*>(&qkv[KD + d0 + 4 * i4]);
+    const f32x4 q4v = *reinterpret_cast<const f32x4*>(&qkv[d0 + 4 * i4]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 4 * i4 + e;
+      const float qq = q4v[e] * qn;
+      kk[i] = k4[e] * kn;
+      S[i] *= e4[e];
+      pred += S[i] * kk[i];
+      out += S[i] * qq;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    pred[c] = sum_over_rows(pred[c]);
+    out[c] = sum_over_rows(out[c]);
+  }
+  if (dq == 0) {
+    part[half][0][col >> 2] = pred;
+    part[half][1][col >> 2] = out;
+  }
+  __syncthreads();
+  pred = part[0][0][col >> 2] + part[1][0][col >> 2];
+  out = part[0][1][col >> 2] + part[1][1][col >> 2];
+  const f32x4 v4 = *reinterpret_cast<const f32x4*>(&qkv[2 * KD + col]);
+  const f32x4 delta = (v4 - pred) * beta;
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    S[i] += delta * kk[i];
+    if (d0 + i < Dk) __builtin_nontemporal_store(S[i], reinterpret_cast<f32x4*>(state + i * VD));
+  }
+  // ---- gated RMS norm over the head's columns ------------------------------------
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    out[c] = round_bf16(fmaf(kq, delta[c], out[c]) * p.scale);
+    ss = fmaf(out[c], out[c], ss);
+  }
+  ss = group_sum<8>(ss);
+  if (lane == 0 && half == 0) red[wave >> 1] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int w = 0; w < VD / 32; ++w) ss += red[w];
+  const float rstd = rsqrtf(ss / (float)VD + p.norm_eps);
+  if (dq == 0 && half == 0) {
+    const u32x2 nw = *reinterpret_cast<const u32x2*>(p.norm_w + col);
+    const f32x4 gt = *reinterpret_cast<const f32x4*>(&eg_gate[KD + col]);
+    const float w4[4] = {bf16lo_to_f32(nw.x), bf16hi_to_f32(nw.x), bf16lo_to_f32(nw.y), bf16hi_to_f32(nw.y)};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) out[c] *= rstd * w4[c] * gt[c];
+    *reinterpret_cast<u32x2*>(p.o + b * p.o_row + h * VD + col) = u32x2{pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3])};
+  }
+}
+
+bool kda_layer_step_serves(int Dk, int Dv, int taps) {
+  return Dk >= 8 && Dk <= 128 && Dk % 8 == 0 && (Dv == 32 || Dv == 64 || Dv == 128) && taps >= 2 && taps <= 4;
+}
+
+int kda_layer_step(const KdaLayerStep& p, int B, int Dv, hipStream_t s) {
+  DAISY_CHECK_SUPPORTED(kda_layer_step_serves(p.Dk, Dv, p.taps), "kda_layer_step: Dk=%d, Dv=%d, %d taps not supported", p.Dk, Dv, p.taps);
+  DAISY_CHECK_ARG(B > 0 && p.H > 0 && (int64_t)B * p.H <= 0x7fffffff, "kda_layer_step: B=%d, H=%d", B, p.H);
+  for (const void* t : {(const void*)p.f, (const void*)p.g, (const void*)p.wf, (const void*)p.wg, (const void*)p.state, (const void*)p.norm_w,
+                        (const void*)p.o, (const void*)p.window[0], (const void*)p.window[1], (const void*)p.window[2],
+                        (const void*)p.conv_w[0], (const void*)p.conv_w[1], (const void*)p.conv_w[2]})
+    DAISY_CHECK_ARG(t != nullptr && (reinterpret_cast<uintptr_t>(t) & 15) == 0, "kda_layer_step: NULL or unaligned tensor");
+  DAISY_CHECK_ARG(p.q && p.k && p.v && p.b && p.A_log && p.dt_bias && p.f_row % 8 == 0 && p.g_row % 8 == 0 && p.o_row % 8 == 0,
+                  "kda_layer_step: NULL tensor or row stride");
+  const dim3 grid((unsigned)(B * p.H));
+  auto launch = [&](auto kd) {
+    constexpr int KD = decltype(kd)::value;
+    if (Dv == 128) hipLaunchKernelGGL((kda_layer_step_kernel<KD, 128>), grid, dim3(512), 0, s, p);
+    else if (Dv == 64) hipLaunchKernelGGL((kda_layer_step_kernel<KD, 64>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((kda_layer_step_kernel<KD, 32>), grid, dim3(128), 0, s, p);
+  };
+  if (p.Dk <= 64) launch(std::integral_constant<int, 64>()); else launch(std::integral_constant<int, 128>());
+  DAISY_CHECK_LAUNCH("kda_layer_step_kernel");
+  return DAISY_OK;
 }
 
 }  // namespace daisy

@@ -140,6 +140,50 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// linears(x, weights, biases, max_rows, tile): the products of x with several matrices in one launch, as a tuple, or None.
+// Arguments as for linear; weights and biases: tuples (a bias may be None).
+PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 5 || !is_tensor(a[0]) || !PyTuple_Check(a[1]) || !PyTuple_Check(a[2])) return none();
+  const Py_ssize_t count = PyTuple_GET_SIZE(a[1]);
+  if (count < 1 || count > daisy::kMaxSegments || PyTuple_GET_SIZE(a[2]) != count) return none();
+  const Tensor& x = THPVariable_Unpack(a[0]);
+  const int max_rows = (int)PyLong_AsLong(a[3]), tile = (int)PyLong_AsLong(a[4]);
+  const int dev = gpu_of(x);
+  Rows r;
+  if (dev < 0 || !as_rows(x, dev, r)) return none();
+  daisy::ProjSegment seg[daisy::kMaxSegments];
+  int64_t pitch = 0;
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    PyObject *wo = PyTuple_GET_ITEM(a[1], i), *bo = PyTuple_GET_ITEM(a[2], i);
+    if (!is_tensor(wo) || !tensor_or_none(bo)) return none();
+    const Tensor& w = THPVariable_Unpack(wo);
+    const Tensor* bias = opt_tensor(bo);
+    if (!rows_bf16(w, 2, dev) || w.size(1) != r.K || w.stride(0) < r.K || needs_autograd({&x, &w, bias})) return none();
+    if (bias && (!on_gpu(*bias, dev) || !bf16(*bias) || bias->numel() != w.size(0) || !bias->is_contiguous())) return none();
+    seg[i] = daisy::ProjSegment{r.p, r.stride, (const uint16_t*)ptr(w), w.stride(0), (const uint16_t*)ptr(bias), nullptr, 0, (int)w.size(0), 0};
+    pitch += (w.size(0) + 7) / 8 * 8;
+  }
+  Tensor y = empty({(int64_t)r.M, pitch}, at::kBFloat16, x);
+  int64_t at = 0;
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    seg[i].y = (uint16_t*)ptr(y) + at;
+    seg[i].y_sm = pitch;
+    at += (seg[i].N + 7) / 8 * 8;
+  }
+  const hipStream_t s = stream_of(dev);
+  const int rc = r.M <= max_rows && !tile ? daisy::linear_segments(seg, (int)count, r.M, r.K, s) : daisy::proj_segments(seg, (int)count, r.M, r.K, s, tile);
+  if (rc != DAISY_OK) return none();
+  PyObject* res = PyTuple_New(count);
+  at = 0;
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    PyTuple_SET_ITEM(res, i, wrap(y.narrow(1, at, seg[i].N)));
+    at += (seg[i].N + 7) / 8 * 8;
+  }
+  return res;
+  END_HANDLE_TH_ERRORS
+}
+
 // ---- attention ----------------------------------------------------------------------------------------------------
 // prefill_attention(q, k, v, window, scale, cos, sin, doc_start, out, k_out) -> (out, k_out)
 PyObject* py_prefill_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -408,8 +452,160 @@ PyObject* py_kda_chunk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// kda_layer(x, weights, H, Dk, Dv, taps, state, windows, homes, keep, norm_eps, max_rows) -> (y, state, wq, wk, wv)
+// KimiLinearSelfAttention on bf16 weights without value embeddings or padding.  weights: tuple of q, k, v, f0, g0, b, f1, g1
+// projections, g1's bias, output projection, the three convolutions' weights and biases, A_log, dt_bias, norm weight.
+// state / windows (tuple of three): what the layer carries, or None.  keep: return the states after the last token; homes: tuple of
+// four tensors (state, windows) to store them in where they fit, or None each.  One token with carried states updates them in place.
+PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  constexpr int kWeights = 19;
+  if (n != 12 || !is_tensor(a[0]) || !PyTuple_Check(a[1]) || PyTuple_GET_SIZE(a[1]) != kWeights || !tensor_or_none(a[6])) return none();
+  if (!PyTuple_Check(a[7]) || PyTuple_GET_SIZE(a[7]) != 3 || !PyTuple_Check(a[8]) || PyTuple_GET_SIZE(a[8]) != 4) return none();
+  const Tensor* w[kWeights];
+  for (int i = 0; i < kWeights; ++i) {
+    PyObject* o = PyTuple_GET_ITEM(a[1], i);
+    const bool optional = i == 8 || i == 13 || i == 14 || i == 15;
+    if (!(is_tensor(o) || (optional && o == Py_None))) return none();
+    w[i] = opt_tensor(o);
+  }
+  const Tensor* win[3]; const Tensor* home[4];
+  for (int i = 0; i < 3; ++i) {
+    PyObject* o = PyTuple_GET_ITEM(a[7], i);
+    if (!tensor_or_none(o)) return none();
+    win[i] = opt_tensor(o);
+  }
+  for (int i = 0; i < 4; ++i) {
+    PyObject* o = PyTuple_GET_ITEM(a[8], i);
+    if (!tensor_or_none(o)) return none();
+    home[i] = opt_tensor(o);
+  }
+  const Tensor& x = THPVariable_Unpack(a[0]);
+  const Tensor* state = opt_tensor(a[6]);
+  const int64_t H = PyLong_AsLong(a[2]), Dk = PyLong_AsLong(a[3]), Dv = PyLong_AsLong(a[4]), taps = PyLong_AsLong(a[5]);
+  const bool keep = a[9] == Py_True;
+  const float norm_eps = (float)PyFloat_AsDouble(a[10]);
+  const int max_rows = (int)PyLong_AsLong(a[11]);
+  if (PyErr_Occurred()) { PyErr_Clear(); return none(); }
+  const int dev = gpu_of(x);
+  if (dev < 0 || max_rows <= 0 || taps < 2 || taps > 4) return none();
+  Rows r;
+  if (x.dim() != 3 || !as_rows(x, dev, r)) return none();
+  const int64_t B = x.size(0), T = x.size(1), dim = r.K, M = r.M, kd = H * Dk, vd = H * Dv;
+  if (c10::GradMode::is_enabled()) {
+    if (x.requires_grad()) return none();
+    for (const Tensor* t : w)
+      if (t && t->requires_grad()) return none();
+  }
+  auto matrix = [&](const Tensor* t, int64_t rows, int64_t cols) {
+    return rows_bf16(*t, 2, dev) && t->is_contiguous() && t->size(0) == rows && t->size(1) == cols && (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0;
+  };
+  auto vector = [&](const Tensor* t, int64_t len, at::ScalarType type) {
+    return on_gpu(*t, dev) && t->scalar_type() == type && t->numel() == len && t->is_contiguous();
+  };
+  const int64_t widths[6] = {kd, kd, vd, Dv, Dv, H};
+  for (int i = 0; i < 6; ++i)
+    if (!matrix(w[i], widths[i], dim)) return none();
+  if (!matrix(w[6], kd, Dv) || !matrix(w[7], vd, Dv) || (w[8] && !vector(w[8], vd, at::kBFloat16)) || !matrix(w[9], dim, vd)) return none();
+  for (int i = 0; i < 3; ++i) {
+    if (!vector(w[10 + i], widths[i] * taps, at::kBFloat16) || (w[13 + i] && !vector(w[13 + i], widths[i], at::kBFloat16))) return none();
+    if (win[i] && !(vector(win[i], B * widths[i] * taps, at::kBFloat16) && win[i]->dim() == 3 && win[i]->size(0) == B)) return none();
+  }
+  if (!vector(w[16], H, at::kFloat) || !vector(w[17], kd, at::kFloat) || !vector(w[18], Dv, at::kBFloat16)) return none();
+  if (state && !(vector(state, B * kd * Dv, at::kFloat) && state->dim() == 4 && state->size(0) == B && state->size(1) == H && state->size(2) == Dk)) return none();
+  const bool step = keep && T == 1 && state;
+  if (step ? !(win[0] && win[1] && win[2] && daisy::kda_layer_step_serves((int)Dk, (int)Dv, (int)taps)) : (dim % 64 != 0 || Dv % 64 != 0)) return none();
+
+  // ---- the projections of the input ---------------------------------------------------------------------------------
+  const hipStream_t s = stream_of(dev);
+  const uint16_t* W[kWeights];
+  for (int i = 0; i < kWeights; ++i) W[i] = (const uint16_t*)ptr(w[i]);
+  const int64_t pitch = (2 * kd + vd + 2 * Dv + H + 7) / 8 * 8, small = (2 * Dv + H + 7) / 8 * 8;
+  const bool rows_kernel = M <= max_rows, together = rows_kernel || daisy::proj_wanted((int)M, (int)pitch, (int)dim);
+  Tensor proj, big[3];
+  daisy::ProjSegment seg[6];
+  proj = empty({M, together ? pitch : small}, at::kBFloat16, x);
+  {
+    uint16_t* y = (uint16_t*)ptr(proj);
+    for (int i = 0; i < 6; ++i) {
+      seg[i] = daisy::ProjSegment{r.p, r.stride, W[i], dim, nullptr, y, together ? pitch : small, (int)widths[i], 0};
+      if (together || i >= 3) y += widths[i];
+    }
+  }
+  if (rows_kernel) {
+    if (daisy::linear_segments(seg, 6, (int)M, (int)dim, s) != DAISY_OK) return none();
+  } else if (together) {
+    if (daisy::proj_segments(seg, 6, (int)M, (int)dim, s) != DAISY_OK) return none();
+  } else {
+    for (int i = 0; i < 3; ++i) {
+      big[i] = at::linear(x, *w[i]);
+      seg[i].y = (uint16_t*)ptr(big[i]);
+      seg[i].y_sm = widths[i];
+    }
+    if (daisy::proj_segments(seg + 3, 3, (int)M, (int)dim, s) != DAISY_OK) return none();
+  }
+
+  // ---- one token: everything up to the output projection in one launch ----------------------------------------------
+  const float scale = (float)(1.0 / std::sqrt((double)Dk));
+  constexpr float kL2Eps = 1e-6f;
+  Tensor o, st, new_win[3];
+  if (step) {
+    o = empty({B, 1, vd}, at::kBFloat16, x);
+    daisy::KdaLayerStep p{seg[0].y, seg[1].y, seg[2].y, seg[3].y, seg[4].y, seg[5].y, seg[0].y_sm, seg[1].y_sm, seg[2].y_sm, seg[3].y_sm,
+                          seg[4].y_sm, seg[5].y_sm, {W[10], W[11], W[12]}, {W[13], W[14], W[15]}, {}, (int)taps, W[6], W[7], W[8],
+                          (const float*)ptr(w[16]), (const float*)ptr(w[17]), W[18], (float*)ptr(state), (uint16_t*)ptr(o), vd,
+                          (int)H, (int)Dk, scale, kL2Eps, norm_eps};
+    for (int i = 0; i < 3; ++i) p.window[i] = (uint16_t*)ptr(win[i]);
+    if (daisy::kda_layer_step(p, (int)B, (int)Dv, s) != DAISY_OK) return none();
+  } else {
+    // Where a state is kept: in its home when that has the shape, else in a new tensor.
+    auto keeper = [&](const Tensor* h, at::IntArrayRef shape, at::ScalarType type) {
+      return h && on_gpu(*h, dev) && h->scalar_type() == type && h->is_contiguous() && h->sizes() == shape ? *h : empty(shape, type, x);
+    };
+    Tensor conv[3];
+    for (int i = 0; i < 3; ++i) {
+      conv[i] = empty({B, T, widths[i]}, at::kBFloat16, x);
+      const std::array<int64_t, 3> shape{B, widths[i], taps};
+      // (a window is updated in place for short inputs only)
+      if (keep) new_win[i] = win[i] && home[i + 1] && win[i]->data_ptr() == home[i + 1]->data_ptr() && T > 32 ? empty(shape, at::kBFloat16, x)
+                                                                                                             : keeper(home[i + 1], shape, at::kBFloat16);
+      const int64_t in[2] = {T * seg[i].y_sm, seg[i].y_sm}, out[2] = {T * widths[i], widths[i]};
+      if (daisy_short_conv_fwd(seg[i].y, in, W[10 + i], W[13 + i], ptr(win[i]), ptr(conv[i]), out, keep ? ptr(new_win[i]) : nullptr,
+                               (int)B, (int)T, (int)widths[i], (int)taps, 1, s) != DAISY_OK) return none();
+      big[i] = Tensor();
+    }
+    Tensor g = empty({M, kd}, at::kBFloat16, x), gate = empty({M, vd}, at::kBFloat16, x), beta = empty({M, H}, at::kFloat, x);
+    const daisy::ProjSegment low[2] = {{seg[3].y, seg[3].y_sm, W[6], Dv, nullptr, (uint16_t*)ptr(g), kd, (int)kd, 0},
+                                       {seg[4].y, seg[4].y_sm, W[7], Dv, W[8], (uint16_t*)ptr(gate), vd, (int)vd, 0}};
+    if (daisy::proj_segments(low, 2, (int)M, (int)Dv, s) != DAISY_OK) return none();
+    if (daisy::kda_gate_beta((const uint16_t*)ptr(g), (const float*)ptr(w[16]), (const float*)ptr(w[17]), (uint16_t*)ptr(g), seg[5].y, seg[5].y_sm,
+                             (float*)ptr(beta), M, (int)H, (int)Dk, s) != DAISY_OK) return none();
+    o = empty({B, T, vd}, at::kBFloat16, x);
+    if (keep) st = keeper(home[0], {B, H, Dk, Dv}, at::kFloat);
+    const size_t need = daisy_kda_workspace_bytes((int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64);
+    Tensor ws = empty({(int64_t)need}, at::kByte, x);
+    if (daisy_kda_chunk_fwd(ptr(conv[0]), ptr(conv[1]), ptr(conv[2]), ptr(g), 1, (const float*)ptr(beta), (const float*)ptr(state), ptr(o),
+                            keep ? (float*)ptr(st) : nullptr, (int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64, scale, 1, kL2Eps, ptr(ws), need, s) != DAISY_OK)
+      return none();
+    if (daisy_gated_rmsnorm_fwd(ptr(o), ptr(gate), W[18], ptr(o), M * H, (int)Dv, norm_eps, s) != DAISY_OK) return none();
+  }
+  Tensor y;
+  if (M <= max_rows || daisy::proj_wanted((int)M, (int)dim, (int)vd)) {
+    y = empty({B, T, dim}, at::kBFloat16, x);
+    if (!own_linear(Rows{(const uint16_t*)ptr(o), vd, (int)M, (int)vd}, W[9], vd, (int)dim, nullptr, (uint16_t*)ptr(y), dim, max_rows, s)) return none();
+  } else {
+    y = at::linear(o, *w[9]);
+  }
+  PyObject* res = PyTuple_New(5);
+  PyTuple_SET_ITEM(res, 0, wrap(y));
+  PyTuple_SET_ITEM(res, 1, !keep ? none() : wrap(step ? *state : st));
+  for (int i = 0; i < 3; ++i) PyTuple_SET_ITEM(res, 2 + i, !keep ? none() : wrap(step ? *win[i] : new_win[i]));
+  return res;
+  END_HANDLE_TH_ERRORS
+}
+
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {FAST(linear), FAST(prefill_attention), FAST(layer_prefill), FAST(layer_step), FAST(kda_chunk),
+PyMethodDef kMethods[] = {FAST(linear), FAST(linears), FAST(prefill_attention), FAST(layer_prefill), FAST(layer_step), FAST(kda_chunk), FAST(kda_layer),
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -21,12 +21,14 @@
 namespace daisy {
 
 struct ProjParams {
-  const uint16_t* x; int64_t x_sm;     // [M, K]
-  const uint16_t* w; int64_t w_sn;     // [N, K]
-  const uint16_t* bias;                // [N] or NULL (plain epilogue)
-  uint16_t* y; int64_t y_sm;           // [M, N] (plain epilogue)
-  int M, N, K, MT, NT;
+  ProjSegment one;                     // the product (bias and y: plain epilogue only)
+  int M, K, MT, NT;
   QkvEpilogue e;                       // QKV epilogue
+};
+// Several products, told apart by the column of tiles.
+struct ProjSegmentsParams {
+  ProjSegment seg[kMaxSegments];
+  int n, M, K, MT, NT;
 };
 
 // At most N vector-memory operations outstanding (bits 3:0 and 15:14 of the immediate) and every LDS read back.
@@ -35,10 +37,10 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
 }
 
-// EPI 0: y = x W^T (+ bias), bf16.  EPI 1 / 2: the QKV epilogue for heads of 64 / 128 channels.
+// EPI 0: y = x W^T (+ bias), bf16, of one or (SEGMENTS) several products.  EPI 1 / 2: the QKV epilogue for heads of 64 / 128 channels.
 // WVM x WVN wavefronts; BK elements of K per step.
-template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI>
-__global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
+template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI, bool SEGMENTS = false>
+__global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t<SEGMENTS, ProjSegmentsParams, ProjParams> p) {
   constexpr int NW = WVM * WVN, NTHR = 64 * NW;
   constexpr int WM = BM / WVM, WN = BN / WVN, MI = WM / 16, NI = WN / 16, KK = BK / 32;
   constexpr int RB = 2 * BK, CPRW = BK / 8, RPC = 64 / CPRW;   // bytes and 16-byte chunks per tile row, rows per copy
@@ -62,7 +64,18 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
   const int total = p.MT * p.NT, per = total >> 3, rest = total & 7;
   const int xcd = blockIdx.x & 7, vid = xcd * per + min(xcd, rest) + (blockIdx.x >> 3);
   const int panel = vid / (8 * p.NT), in_panel = vid - panel * 8 * p.NT, rows = min(8, p.MT - 8 * panel);
-  const int mt = 8 * panel + in_panel % rows, nt = in_panel / rows;
+  const int mt = 8 * panel + in_panel % rows;
+  int nt = in_panel / rows;
+  const ProjSegment* gp;
+  if constexpr (SEGMENTS) {
+    int i = 0;
+    while (i + 1 < p.n && nt >= p.seg[i].tile_end) ++i;
+    if (i > 0) nt -= p.seg[i - 1].tile_end;
+    gp = &p.seg[i];
+  } else {
+    gp = &p.one;
+  }
+  const ProjSegment g = *gp;
   const int m0 = mt * BM, n0 = nt * BN;
 
   // Copy j of this wavefront covers tile rows RPC (wave + NW j) ..: lane i lands at row i / CPRW, chunk position i % CPRW and
@@ -72,15 +85,15 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
 #pragma unroll
   for (int j = 0; j < CA; ++j) {
     const int r = RPC * (wave + NW * j) + cr;
-    offa[j] = 2 * (int)((min(m0 + r, p.M - 1) - m0) * p.x_sm) + 16 * (cp ^ swz(r));
+    offa[j] = 2 * (int)((min(m0 + r, p.M - 1) - m0) * g.x_sm) + 16 * (cp ^ swz(r));
   }
 #pragma unroll
   for (int j = 0; j < CB; ++j) {
     const int r = RPC * (wave + NW * j) + cr;
-    offb[j] = 2 * (int)((min(n0 + r, p.N - 1) - n0) * p.w_sn) + 16 * (cp ^ swz(r));
+    offb[j] = 2 * (int)((min(n0 + r, g.N - 1) - n0) * g.w_sn) + 16 * (cp ^ swz(r));
   }
-  const uint16_t* xa = p.x + (int64_t)m0 * p.x_sm;
-  const uint16_t* wb = p.w + (int64_t)n0 * p.w_sn;
+  const uint16_t* xa = g.x + (int64_t)m0 * g.x_sm;
+  const uint16_t* wb = g.w + (int64_t)n0 * g.w_sn;
   const uint32_t lds0 = lds_address(smem) + 1024 * wave;
   auto issue = [&](int st) {
     const uint32_t dst = lds0 + st * STAGE;
@@ -153,9 +166,9 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
   for (int i = 0; i < NI; ++i) {
     const int n = WN * wn + 16 * i + 4 * q4;       // four consecutive columns
     float bv[4] = {0.f, 0.f, 0.f, 0.f};
-    if (EPI == 0 && p.bias != nullptr) {
+    if (EPI == 0 && g.bias != nullptr) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bv[r] = bf16lo_to_f32(p.bias[min(n0 + n + r, p.N - 1)]);
+      for (int r = 0; r < 4; ++r) bv[r] = bf16lo_to_f32(g.bias[min(n0 + n + r, g.N - 1)]);
     }
 #pragma unroll
     for (int j = 0; j < MI; ++j) {
@@ -172,7 +185,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
       const int idx = tid + NTHR * it, m = idx / CHN, c = idx % CHN;
       if (BM * CHN % NTHR != 0 && m >= BM) break;
       const u32x4 v = *reinterpret_cast<const u32x4*>(tile_at(m, c));
-      if (m0 + m < p.M && n0 + 8 * c < p.N) *reinterpret_cast<u32x4*>(p.y + (int64_t)(m0 + m) * p.y_sm + n0 + 8 * c) = v;
+      if (m0 + m < p.M && n0 + 8 * c < g.N) *reinterpret_cast<u32x4*>(g.y + (int64_t)(m0 + m) * g.y_sm + n0 + 8 * c) = v;
     }
   } else {
     constexpr int D = EPI == 1 ? 64 : 128, HALF = D / 2, LPR = D / 16, HPT = BN / D;
@@ -186,7 +199,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
       const int idx = tid + NTHR * it, c = idx % LPR, hh = (idx / LPR) % HPT, m = idx / (LPR * HPT);
       if (BM * BN / 16 % NTHR != 0 && m >= BM) break;
       const int n = n0 + hh * D;
-      const bool live = m0 + m < p.M && n < p.N;
+      const bool live = m0 + m < p.M && n < g.N;
       const int row = min(m0 + m, p.M - 1);
       const int third = min(n / (e.H * D), 2), h = min(n / D - third * e.H, e.H - 1);
       const int t = row % e.T, b = row / e.T;
@@ -220,15 +233,15 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
       } else {
         if (e.ve != nullptr) {
           // g*v + (1-g)*ve with every product, the difference and the sum rounded to bf16
-          const float g = gate_value(e.gate), og = round_bf16(1.0f - g);
+          const float gv = gate_value(e.gate), og = round_bf16(1.0f - gv);
           const uint16_t* vp = e.ve + b * e.ve_sb + t * e.ve_st + h * e.ve_sh + 8 * c;
           float el[8], eh[8];
           unpack8(*reinterpret_cast<const u32x4*>(vp), el);
           unpack8(*reinterpret_cast<const u32x4*>(vp + HALF), eh);
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            lo[i] = round_bf16(g * lo[i]) + round_bf16(og * el[i]);
-            hi[i] = round_bf16(g * hi[i]) + round_bf16(og * eh[i]);
+            lo[i] = round_bf16(gv * lo[i]) + round_bf16(og * el[i]);
+            hi[i] = round_bf16(gv * hi[i]) + round_bf16(og * eh[i]);
           }
         }
         dst = e.v + b * e.v_sb + t * e.v_st + h * e.v_sh;
@@ -246,7 +259,8 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(ProjParams p) {
 // proportional to K), a round with all of them `full`.  A product of n tiles then costs about 1.5 us plus its rounds, and
 // the shape with the least cost is taken: the small ones while their tiles fit one round, the large ones from there on.
 // (M = 777, N = 4608, K = 1536: 16.6 us with 128 x 128 and 8 wavefronts, 18.6 us with 64 x 128, 24.4 us with 64 x 64,
-// 17.9 us in the library; M = 64, N = 6144, K = 2048: 7.3 us with 32 x 64, 9.7 us in the library; M = 8192,
+// 17.9 us in the library; M = 64, N = 6144, K = 2048: 7.3 us with 32 x 64, 9.7 us in the library (a KDA decode step's six input projections in
+// one launch: 8.3 us, one by one 42 us); M = 8192,
 // N = 6144, K = 2048: 155 us with 256 x 256, 178 us with 128 x 128, 141 us in the library.)
 struct ProjTile { int code, bm, bn, bk, per_cu; float one, full; };
 constexpr ProjTile kProjTiles[] = {
@@ -258,12 +272,13 @@ constexpr ProjTile kProjTiles[] = {
     {6, 128, 128, 64, 2, 20.2f, 25.3f},   // 4 wavefronts, 2 stages
     {7, 256, 256, 64, 1, 42.0f, 42.0f},   // 8 wavefronts, 2 stages
 };
-static int proj_tile(int M, int N, int K, int head) {
+template <typename COLUMNS>      // columns(bn): columns of tiles of that width
+static int proj_tile(int M, int K, int head, COLUMNS columns) {
   int best = 0;
   float least = 0.f;
   for (const ProjTile& t : kProjTiles) {
     if (K % t.bk != 0 || t.bn % head != 0) continue;    // (head: a tile of the QKV projection holds whole heads)
-    const int64_t n = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), round = 256 * t.per_cu;
+    const int64_t n = (int64_t)((M + t.bm - 1) / t.bm) * columns(t.bn), round = 256 * t.per_cu;
     const int64_t tail = n % round;
     const float cost = (float)(n / round) * t.full + (tail > 256 ? t.full : tail > 0 ? t.one : 0.f);
     if (best == 0 || cost < least) { best = t.code; least = cost; }
@@ -278,16 +293,25 @@ bool proj_wanted(int M, int N, int K) { return K % 64 == 0 && N % 8 == 0 && (K <
 bool proj_qkv_wanted(int M, int N, int K) { return K % 64 == 0; }
 
 template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI>
-static int launch_proj(ProjParams p, hipStream_t s) {
+static int launch_proj(ProjParams& p, hipStream_t s) {
   p.MT = (p.M + BM - 1) / BM;
-  p.NT = (p.N + BN - 1) / BN;
+  p.NT = (p.one.N + BN - 1) / BN;
   hipLaunchKernelGGL((proj_kernel<BM, BN, WVM, WVN, BK, STAGES, EPI>), dim3((unsigned)(p.MT * p.NT)), dim3(64 * WVM * WVN), 0, s, p);
   DAISY_CHECK_LAUNCH("proj_kernel");
   return DAISY_OK;
 }
+template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI>
+static int launch_proj(ProjSegmentsParams& p, hipStream_t s) {
+  p.MT = (p.M + BM - 1) / BM;
+  p.NT = 0;
+  for (int i = 0; i < p.n; ++i) p.seg[i].tile_end = p.NT += (p.seg[i].N + BN - 1) / BN;
+  hipLaunchKernelGGL((proj_kernel<BM, BN, WVM, WVN, BK, STAGES, EPI, true>), dim3((unsigned)(p.MT * p.NT)), dim3(64 * WVM * WVN), 0, s, p);
+  DAISY_CHECK_LAUNCH("proj_kernel");
+  return DAISY_OK;
+}
 
-template <int EPI>
-static int dispatch_proj(int tile, const ProjParams& p, hipStream_t s) {
+template <int EPI, typename PARAMS>
+static int dispatch_proj(int tile, PARAMS& p, hipStream_t s) {
   for (const ProjTile& t : kProjTiles)
     DAISY_CHECK_SUPPORTED(t.code != tile || (p.K % t.bk == 0 && !(EPI == 2 && t.bn % 128 != 0)), "proj: tile %d does not serve K=%d", tile, p.K);
   if constexpr (EPI != 2) {
@@ -314,8 +338,29 @@ int proj_linear(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn
                   "proj_linear: rows must start on 16-byte boundaries");
   DAISY_CHECK_ARG(x_sm < (1 << 22) && w_sn < (1 << 22), "proj_linear: row strides too long");
   ProjParams p{};
-  p.x = x; p.x_sm = x_sm; p.w = w; p.w_sn = w_sn; p.bias = bias; p.y = y; p.y_sm = y_sm; p.M = M; p.N = N; p.K = K;
-  return dispatch_proj<0>(tile ? tile : proj_tile(M, N, K, 8), p, s);
+  p.one = ProjSegment{x, x_sm, w, w_sn, bias, y, y_sm, N, 0}; p.M = M; p.K = K;
+  return dispatch_proj<0>(tile ? tile : proj_tile(M, K, 8, [&](int bn) { return (N + bn - 1) / bn; }), p, s);
+}
+
+int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, int tile) {
+  DAISY_CHECK_ARG(seg && n >= 1 && n <= kMaxSegments && M > 0 && K > 0, "proj_segments: %d products, M=%d, K=%d", n, M, K);
+  DAISY_CHECK_SUPPORTED(K % 64 == 0, "proj_segments: K=%d must be a multiple of 64", K);
+  ProjSegmentsParams p{};
+  for (int i = 0; i < n; ++i) {
+    const ProjSegment& g = seg[i];
+    DAISY_CHECK_ARG(g.x && g.w && g.y && g.N > 0, "proj_segments: NULL tensor or N=%d", g.N);
+    DAISY_CHECK_ARG(aligned16(g.x) && aligned16(g.w) && aligned16(g.y) && g.x_sm % 8 == 0 && g.w_sn % 8 == 0 && g.y_sm % 8 == 0 &&
+                        g.y_sm >= ((g.N + 7) & ~7) && g.x_sm < (1 << 22) && g.w_sn < (1 << 22),
+                    "proj_segments: rows must start on 16-byte boundaries, with room for whole 16-byte pieces");
+    p.seg[i] = g;
+  }
+  p.n = n; p.M = M; p.K = K;
+  auto columns = [&](int bn) {
+    int c = 0;
+    for (int i = 0; i < n; ++i) c += (seg[i].N + bn - 1) / bn;
+    return c;
+  };
+  return dispatch_proj<0>(tile ? tile : proj_tile(M, K, 8, columns), p, s);
 }
 
 int proj_qkv(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const QkvEpilogue& e,
@@ -330,8 +375,8 @@ int proj_qkv(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, c
   for (int64_t v : st) DAISY_CHECK_ARG(v % 8 == 0, "proj_qkv: strides must be multiples of 8 elements");
   DAISY_CHECK_ARG(x_sm < (1 << 22) && w_sn < (1 << 22), "proj_qkv: row strides too long");
   ProjParams p{};
-  p.x = x; p.x_sm = x_sm; p.w = w; p.w_sn = w_sn; p.M = M; p.N = N; p.K = K; p.e = e;
-  if (!tile) tile = proj_tile(M, N, K, D);
+  p.one = ProjSegment{x, x_sm, w, w_sn, nullptr, nullptr, 0, N, 0}; p.M = M; p.K = K; p.e = e;
+  if (!tile) tile = proj_tile(M, K, D, [&](int bn) { return (N + bn - 1) / bn; });
   return D == 128 ? dispatch_proj<2>(tile, p, s) : dispatch_proj<1>(tile, p, s);
 }
 

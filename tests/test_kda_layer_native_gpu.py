@@ -1,0 +1,75 @@
+"""The KDA layer's one-call path against the layer's own Python path (the same kernels one by one), and the products that share a
+launch against separate ones."""
+import pytest
+import torch
+
+from daisy_amd import KimiLinearSelfAttention, _lib
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _layer(H, D, expand_v, taps, conv_bias):
+    torch.manual_seed(H * D + taps)
+    with torch.device(DEV):
+        m = KimiLinearSelfAttention(H * D, H, max_seq_len=1024, head_dim=D, expand_v=expand_v, conv_size=taps, conv_bias=conv_bias)
+    with torch.no_grad():
+        m.dt_bias.normal_()
+        m.g_proj[1].bias.normal_(std=0.3)
+        m.o_norm.weight.normal_(1, 0.2)
+        for c in (m.q_conv1d, m.k_conv1d, m.v_conv1d):
+            if c.bias is not None:
+                c.bias.normal_(std=0.2)
+    return m.eval()
+
+
+@pytest.mark.parametrize("H,D,expand_v,taps,conv_bias", [(16, 128, 1.0, 4, False), (12, 64, 1.0, 4, True), (4, 64, 2.0, 3, True),
+                                                         (4, 128, 0.5, 2, False), (12, 96, 4 / 3, 4, False), (8, 40, 1.6, 3, False)])
+@pytest.mark.parametrize("B,T", [(1, 1), (1, 37), (3, 70), (33, 2)])
+def test_layer_in_one_call_equals_its_kernels_one_by_one(H, D, expand_v, taps, conv_bias, B, T, monkeypatch):
+    m = _layer(H, D, expand_v, taps, conv_bias)
+    g = torch.Generator(device=DEV).manual_seed(B + T)
+    x = torch.randn(B, T, H * D, generator=g, device=DEV).bfloat16()
+    steps = torch.randn(3, B, 1, H * D, generator=g, device=DEV).bfloat16()
+
+    @torch.no_grad()
+    def run(fast):
+        taken = []
+        whole = KimiLinearSelfAttention._fast
+        monkeypatch.setattr(KimiLinearSelfAttention, "_fast",
+                            (lambda self, *a: taken.append(whole(self, *a)) or taken[-1]) if fast else (lambda self, *a: None))
+        m._recurrent_state = m._conv_state = None
+        m._state_homes = {}
+        outs = [m(x, None), m.prefill(x, None)[0], m.prefill(x[:, :max(1, T // 2)], None)[0]]
+        outs += [m.step(s, None, None, T + i, None, None)[0] for i, s in enumerate(steps)]
+        outs += [t.clone() for t in m.state_tensors()]
+        addresses = [t.data_ptr() for t in m.state_tensors()]
+        m.reset_history()
+        outs += [m.prefill(x, None)[0]] + [t.clone() for t in m.state_tensors()]
+        assert [t.data_ptr() for t in m.state_tensors()] == addresses
+        monkeypatch.undo()
+        return outs, taken
+
+    ref, _ = run(False)
+    got, taken = run(True)
+    served = m.head_v_dim % 64 == 0 and (H * D) % 64 == 0
+    assert all((t is not None) == served for t in taken[:3]) and all(t is not None for t in taken[3:6])
+    for a, b in zip(ref, got):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert ((a.float() - b.float()).norm() / a.float().norm().clamp_min(1e-9)).item() < 5e-3
+
+
+@pytest.mark.parametrize("M,K,Ns", [(1, 256, (256, 64, 12)), (4, 128, (100, 8, 1)), (5, 64, (64, 200)), (70, 768, (768, 64, 64, 12)),
+                                    (300, 128, (2048, 2048)), (513, 2048, (128, 128, 16))])
+def test_products_in_one_launch_equal_separate_ones(M, K, Ns):
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    ws = tuple(torch.randn(n, K, generator=g, device=DEV).bfloat16() for n in Ns)
+    bs = tuple(torch.randn(n, generator=g, device=DEV).bfloat16() if M > 4 and i % 2 else None for i, n in enumerate(Ns))
+    native = _lib.native()
+    for tile in [0] + [t for t, bk in ((1, 128), (2, 128), (3, 128), (4, 64), (5, 64), (6, 64), (7, 64)) if K % bk == 0]:
+        ys = native.linears(x, ws, bs, 4, tile)
+        assert ys is not None
+        for y, w, b in zip(ys, ws, bs):
+            ref = x.float() @ w.float().T + (b.float() if b is not None else 0.0)
+            assert ((y.float() - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-3 * K ** 0.5).all(), tile
