@@ -101,8 +101,10 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 // It takes 230 us at that size, 0.9 us per chunk; 165 us of them remain without the copies into the LDS.
 //
 // Numerics: the 16x16 blocks of A and P run on MFMA with both operands referenced to the row before the block (every
-// exponent <= 0 off the diagonal); a diagonal block whose total decay exceeds exp(-80) is instead accumulated in
-// fp32 pair by pair with exp(G_i - G_j), j < i (no exponent is ever positive, so strong decays cannot overflow).
+// exponent <= 0 off the diagonal); a diagonal block whose total decay exceeds exp(-80) is referenced to its middle row
+// instead (exponents up to the decay of 8 rows either way), when those go beyond exp(-80) to four rows in four passes, and
+// when four rows do, it is accumulated in fp32 pair by pair with exp(G_i - G_j), j < i (no exponent is ever positive, so
+// strong decays cannot overflow).
 // T is computed in fp32; the products with T, the state update and the output's second term use two-term bf16 splits of
 // both operands (three MFMAs each, relative error ~2^-17), which keeps the state error near fp32.
 // ===========================================================================
@@ -132,30 +134,70 @@ struct KdaParams {
   int B, T, H, NC; float scale; int l2norm; float l2eps;
   int Dk, Dv;     // the tensors' own widths: Dk <= KD key channels, Dv value columns
   char* blobs;    // [H][nc_total][KdaBlob<KD>::kBytes]
-  // Sequences packed along the token axis of a batch of one (B == 1, T = all tokens): n_seq > 0,
-  // bounds [n_seq + 1] = sanitised running lengths, seq_chunk0 [n_seq + 1] = first chunk slot of
-  // every sequence, chunk_seq [NC] = sequence of every chunk slot; all three are written on the
-  // device by kda_chunk_table_kernel, NC is the host's upper bound T / 32 + n_seq on the slots.
-  int n_seq; const int32_t* bounds; const int32_t* seq_chunk0; const int32_t* chunk_seq;
+  // Sequences packed along the token axis of a batch of one (B == 1, T = all tokens): n_seq > 0, cu [n_seq + 1] = the
+  // caller's running lengths; NC is the host's upper bound T / 32 + n_seq on the chunk slots.  Up to kScanSeqs sequences a
+  // wavefront finds its way by itself (packed_span); beyond, kda_chunk_table_kernel writes bounds [n_seq + 1] = sanitised
+  // running lengths, seq_chunk0 [n_seq + 1] = first chunk slot of every sequence, chunk_seq [NC] = sequence of every slot.
+  int n_seq; const int32_t* cu; const int32_t* bounds; const int32_t* seq_chunk0; const int32_t* chunk_seq;
   int nc_total;   // chunk slots per head in the workspace: B * NC, or NC for a packed batch
 };
 
 // Where a sequence lives: token rows [tok0, tok_end) of the flattened [B * T] token axis and
 // chunk slots [c0, c0 + nc) of the workspace.  A batch element is a sequence of its own.
 struct SeqSpan { int tok0, tok_end, c0, nc; };
-__device__ __forceinline__ SeqSpan seq_span(const KdaParams& p, int seq) {
-  SeqSpan s;
-  if (p.n_seq > 0) {
-    s.tok0 = p.bounds[seq]; s.tok_end = p.bounds[seq + 1];
-    s.c0 = p.seq_chunk0[seq]; s.nc = p.seq_chunk0[seq + 1] - s.c0;
-  } else {
-    s.tok0 = seq * p.T; s.tok_end = s.tok0 + p.T;
-    s.c0 = seq * p.NC; s.nc = p.NC;
+
+// Sequence `key` of a packed batch, or (by_slot) the one that owns chunk slot `key`: nc == 0 when there is none.  `rows_end`
+// gets the end of the last sequence.  Bounds = the caller's, forced to start at 0, to stay within 0..T and not to decrease
+// (whatever was passed, no kernel then leaves the tensors); chunk slots = running sum of ceil(len / 32).  A lane per
+// sequence, two scans: about 0.5 us in every workgroup of both kernels instead of a launch of one workgroup in front of
+// them (6 us).
+constexpr int kScanSeqs = 64;
+__device__ __forceinline__ SeqSpan packed_span(const KdaParams& p, int key, bool by_slot, int& rows_end) {
+  SeqSpan s{0, 0, 0, 0};
+  if (p.bounds != nullptr) {
+    rows_end = p.bounds[p.n_seq];
+    if (by_slot) {
+      if (key >= p.seq_chunk0[p.n_seq]) return s;
+      key = p.chunk_seq[key];
+    }
+    s.tok0 = p.bounds[key]; s.tok_end = p.bounds[key + 1];
+    s.c0 = p.seq_chunk0[key]; s.nc = p.seq_chunk0[key + 1] - s.c0;
+    return s;
   }
+  const int lane = threadIdx.x & 63;
+  int end = min(max(p.cu[min(lane + 1, p.n_seq)], p.cu[0]), p.T);
+  end = max(end, 0);
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int left = __shfl_up(end, off);
+    if (lane >= off) end = max(end, left);
+  }
+  int begin = __shfl_up(end, 1);
+  begin = lane == 0 ? 0 : begin;
+  const int nc = lane < p.n_seq ? (end - begin + KC - 1) / KC : 0;
+  int upto = nc;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int left = __shfl_up(upto, off);
+    if (lane >= off) upto += left;
+  }
+  rows_end = __builtin_amdgcn_readlane(end, 63);     // (lanes past the last sequence repeat its end)
+  if (by_slot) {
+    const uint64_t owner = __ballot(key >= upto - nc && key < upto);
+    if (owner == 0) return s;
+    key = __builtin_ctzll(owner);
+  }
+  s.tok0 = __builtin_amdgcn_readlane(begin, key); s.tok_end = __builtin_amdgcn_readlane(end, key);
+  s.nc = __builtin_amdgcn_readlane(nc, key); s.c0 = __builtin_amdgcn_readlane(upto, key) - s.nc;
   return s;
 }
+__device__ __forceinline__ SeqSpan seq_span(const KdaParams& p, int seq, int& rows_end) {
+  if (p.n_seq > 0) return packed_span(p, seq, false, rows_end);
+  rows_end = p.B * p.T;
+  return SeqSpan{seq * p.T, (seq + 1) * p.T, seq * p.NC, p.NC};
+}
 
-// Chunk slots of packed sequences, built on the device so that the host never reads the bounds.
+// Chunk slots of more than kScanSeqs packed sequences, built on the device so that the host never reads the bounds.
 // bounds = cu_seqlens forced to start at 0, to stay within 0..T and not to decrease (whatever the
 // caller passed, no kernel then leaves the tensors); seq_chunk0 = running sum of ceil(len / 32);
 // chunk_seq = the sequence of every slot.  One workgroup; thread i takes a run of sequences.
@@ -228,11 +270,11 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
   __shared__ __attribute__((aligned(16))) float G[64][KD + 4];        // inclusive running log-decay (rows 4 banks apart: 16 rows read side by side do not collide)
   __shared__ __attribute__((aligned(16))) uint16_t Kr[64][KD + 8];    // k as given (bf16)
   __shared__ __attribute__((aligned(16))) uint16_t Qr[64][KD + 8];    // q as given
-  __shared__ __attribute__((aligned(16))) float Ad[4][16][16];        // diagonal blocks of A, [block][column j][row i]; later scratch of that wavefront
+  __shared__ __attribute__((aligned(16))) float Ad[4][16][16];        // diagonal blocks of A, [block][column j][row i]
   __shared__ __attribute__((aligned(16))) float Ao[2][16][20];        // the block A_10 of either chunk, [row][column]
   __shared__ __attribute__((aligned(16))) float Td[4][16][20];        // (I + A_II)^-1, [block][row][column]
   __shared__ __attribute__((aligned(16))) float rk[64], rq[64], bt[64];   // 1/|k|, 1/|q|, beta (0 for padded rows)
-  __shared__ int steep[4];                                            // per 16-row block: total decay beyond exp(-80); 2 when some 4 rows of it alone go beyond
+  __shared__ int steep[4];      // per 16-row block: decay beyond exp(-80) over all of it (1), over 8 of its rows (2), over 4 (3)
 
   const int h = blockIdx.y;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -247,8 +289,9 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
     n_live[c] = 0;
     int gc = slot;
     if (p.n_seq > 0) {
-      if (slot < p.seq_chunk0[p.n_seq]) {
-        const SeqSpan sp = seq_span(p, p.chunk_seq[slot]);
+      int rows_end;
+      const SeqSpan sp = packed_span(p, slot, true, rows_end);
+      if (sp.nc > 0) {
         t0[c] = sp.tok0 + (slot - sp.c0) * KC;
         n_live[c] = min(sp.tok_end - t0[c], KC);
       }
@@ -329,17 +372,13 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
     }
 #pragma unroll
     for (int blk = 0; blk < GR / 16; ++blk) {
-      float tot = 0.f;
+      float t4[4];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) tot += gv[16 * blk + i];
-      const int sb = part * GR / 16 + blk;
-      if (tot < -80.f) atomicMax(&steep[sb], 1);
-      // ... and whether four consecutive rows alone decay that far (then no reference row per group of four keeps
-      // the exponents of the matrix-core path in range)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const float t4 = gv[16 * blk + 4 * g4] + gv[16 * blk + 4 * g4 + 1] + gv[16 * blk + 4 * g4 + 2] + gv[16 * blk + 4 * g4 + 3];
-        if (t4 < -80.f) atomicMax(&steep[sb], 2);
+      for (int f = 0; f < 4; ++f) t4[f] = gv[16 * blk + 4 * f] + gv[16 * blk + 4 * f + 1] + gv[16 * blk + 4 * f + 2] + gv[16 * blk + 4 * f + 3];
+      const float lo = t4[0] + t4[1], hi = t4[2] + t4[3];
+      if (__any(lo + hi < -80.f)) {
+        const bool four = __any(fminf(fminf(t4[0], t4[1]), fminf(t4[2], t4[3])) < -80.f), eight = __any(fminf(lo, hi) < -80.f);
+        if ((tid & 63) == 0) atomicMax(&steep[part * GR / 16 + blk], four ? 3 : eight ? 2 : 1);
       }
     }
     if constexpr (GR < KC) {                      // the second half of a chunk continues from the first
@@ -428,7 +467,8 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
   // Block rows bi = 0..3 of the 64 rows (chunk bi / 2, I = bi % 2).  Block (I, J), J <= I: both operands are referenced to
   // the row before block I (the chunk's start for I = 0: G_ref = 0), so the row factor exp(G_i - G_ref) is <= 1 and, for J < I,
   // so is the column factor exp(G_ref - G_j).  For a diagonal block (J == I) the column factor grows to exp(total decay
-  // of the block); the block takes this path only when that total stays below 80 (flag `steep` otherwise).
+  // of the block); beyond exp(80) the block's middle row is the reference, each factor then growing to the decay of 8 rows
+  // (four passes took 60 us more per 32768 rows of 16 heads with the decays of a freshly initialised layer).
   // Wavefront w takes block row w: its diagonal block and, in the second block row of a chunk, block (1, 0).
   const int li = lane & 15, q4 = lane >> 4;
   const int chunk = wave >> 1, I = wave & 1;
@@ -463,8 +503,7 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
   // This wavefront's rows of scale tril(P), as a product's operand wants them: row 16 I + li, columns 4 q4 + r of either
   // column block.
   f32x4 P[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  auto mfma_block = [&](int J) {
-    const int ref = I ? 16 * wave - 1 : -1;
+  auto mfma_block = [&](int J, int ref) {
     const int rj = 32 * chunk + 16 * J + li;
     f32x4 accA = {0.f, 0.f, 0.f, 0.f}, accP = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -607,12 +646,16 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
     if (I == 0) P[0] = pv; else P[1] = pv;
   };
   {
-    const int sp = __builtin_amdgcn_readfirstlane(steep[wave]);
-    if (I == 1 || sp == 0) row_operands(I ? 16 * wave - 1 : -1);
-    if (I == 1) mfma_block(0);
-    if (sp == 2) steep_diagonal();
-    else if (sp == 1) steep_diagonal_mfma();
-    else mfma_block(I);
+    const int sp = __builtin_amdgcn_readfirstlane(steep[wave]), before = I ? 16 * wave - 1 : -1, middle = 16 * wave + 7;
+    if (I == 1 || sp == 0) row_operands(before);
+    if (I == 1) mfma_block(0, before);
+    if (sp == 3) steep_diagonal();
+    else if (sp == 2) steep_diagonal_mfma();
+    else {
+      // With the middle row as reference the entries above the diagonal may overflow; nothing reads them.
+      if (sp == 1) row_operands(middle);
+      mfma_block(I, sp == 1 ? middle : before);
+    }
   }
 
   // ---- phase 3: T = (I + A)^-1 diag(beta).  The inverse of diagonal block `wave` in fp32, one column per lane (lanes
@@ -637,36 +680,23 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
     }
   }
   __syncthreads();   // both inverses and A_10 of either chunk are in place
-  // T_10 = -T_11 (A_10 T_00): lane (row li, columns 4 q4 .. + 3); the two wavefronts of a chunk both make all of it, in a
-  // scratch area of their own (A_II is no longer needed).
+  // T_10 = -T_11 (A_10 T_00) in two fp32 matrix products, both wavefronts of a chunk all of it.  As right operand (lane
+  // (column li, rows 4 q4 + e)) and as result the layout is the same, and it is also the one T^T is wanted in below.  (As
+  // multiply-adds from LDS this took 3400 of the workgroup's 27000 cycles.)
+  f32x4 t00, t10, t11;
   {
+    const f32x4 a10 = lds_f4(&Ao[chunk][li][4 * q4]), r11 = lds_f4(&Td[2 * chunk + 1][li][4 * q4]);
     f32x4 m1 = {0.f, 0.f, 0.f, 0.f};
+    t10 = m1;
 #pragma unroll
-    for (int j4 = 0; j4 < 4; ++j4) {
-      const f32x4 a4 = lds_f4(&Ao[chunk][li][4 * j4]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const f32x4 t4 = lds_f4(&Td[2 * chunk][4 * j4 + e][4 * q4]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) m1[r] = fmaf(a4[e], t4[r], m1[r]);
-      }
+    for (int e = 0; e < 4; ++e) {
+      t00[e] = Td[2 * chunk][4 * q4 + e][li];
+      t11[e] = Td[2 * chunk + 1][4 * q4 + e][li];
     }
-    *reinterpret_cast<f32x4*>(&Ad[wave][li][4 * q4]) = m1;
-    wave_lds_fence();
-    f32x4 t10 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j4 = 0; j4 < 4; ++j4) {
-      const f32x4 a4 = lds_f4(&Td[2 * chunk + 1][li][4 * j4]);
+    for (int e = 0; e < 4; ++e) m1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a10[e], t00[e], m1, 0, 0, 0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const f32x4 x4 = lds_f4(&Ad[wave][4 * j4 + e][4 * q4]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) t10[r] = fmaf(-a4[e], x4[r], t10[r]);
-      }
-    }
-    wave_lds_fence();
-    *reinterpret_cast<f32x4*>(&Ad[wave][li][4 * q4]) = t10;
-    wave_lds_fence();
+    for (int e = 0; e < 4; ++e) t10 = __builtin_amdgcn_mfma_f32_16x16x4f32(-r11[e], m1[e], t10, 0, 0, 0);
   }
   // T^T as left operand: row (column of T) 16 J + li, contraction slots (q4, e): positions 4 q4 + e for e < 4,
   // 16 + 4 q4 + (e - 4) for e >= 4; two bf16 terms.
@@ -676,10 +706,10 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
     float v0[8], v1[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      v0[e] = b0 * Td[2 * chunk][4 * q4 + e][li];
-      v0[4 + e] = b0 * Ad[wave][4 * q4 + e][li];
+      v0[e] = b0 * t00[e];
+      v0[4 + e] = b0 * t10[e];
       v1[e] = 0.f;
-      v1[4 + e] = b1 * Td[2 * chunk + 1][4 * q4 + e][li];
+      v1[4 + e] = b1 * t11[e];
     }
     u32x4 hi, lo;
     split_pack8(v0, hi, lo);
@@ -797,7 +827,8 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
   const int NGRP = (p.Dv + KVS * KCT - 1) / (KVS * KCT);       // groups of 32 value columns
   const int grp = vid % NGRP, bh = vid / NGRP;
   const int h = bh % p.H, b = bh / p.H;     // b: batch element, or sequence of a packed batch
-  const SeqSpan sp = seq_span(p, b);
+  int rows_end;
+  const SeqSpan sp = seq_span(p, b, rows_end);
   const int nc = sp.nc;                      // chunks of this sequence (0 for an empty one)
   const int64_t ci0 = (int64_t)h * p.nc_total + sp.c0;
   const int lane = threadIdx.x & 63, ln = lane & 15, q4 = lane >> 4;
@@ -913,6 +944,9 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
       __syncthreads();
     }
     if (nc > 0) finish(nc - 1);
+    // rows behind the last sequence of a packed batch belong to none: zeros
+    if (p.n_seq > 0 && b == p.n_seq - 1 && col < p.Dv)
+      for (int tok = rows_end + (lane >> 1); tok < p.T; tok += 32) *reinterpret_cast<u32x4*>(p.o + ((int64_t)tok * p.H + h) * p.Dv + col) = u32x4{0u, 0u, 0u, 0u};
     return;
   }
 
@@ -1121,9 +1155,9 @@ static int kda_chunk_launch(const void* q, const void* k, const void* v,
   char* w = (char*)workspace;
   p.blobs = w;
   w += slots * H * kBlobBytes;
-  p.n_seq = n_seq; p.bounds = p.seq_chunk0 = p.chunk_seq = nullptr;
+  p.n_seq = n_seq; p.cu = cu_seqlens; p.bounds = p.seq_chunk0 = p.chunk_seq = nullptr;
   hipStream_t s = (hipStream_t)stream;
-  if (n_seq > 0) {
+  if (n_seq > kScanSeqs) {
     int32_t* tab = (int32_t*)w;
     int32_t* bounds = tab; int32_t* seq_chunk0 = tab + n_seq + 1; int32_t* chunk_seq = tab + 2 * (n_seq + 1);
     hipLaunchKernelGGL(kda_chunk_table_kernel, dim3(1), dim3(256), 0, s, cu_seqlens, n_seq, T, (int)slots, bounds, seq_chunk0, chunk_seq);

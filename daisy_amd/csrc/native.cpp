@@ -434,7 +434,6 @@ PyObject* py_kda_chunk(PyObject*, PyObject* const* a, Py_ssize_t n) {
                             : daisy_kda_workspace_bytes((int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64);
   if (need == 0) return none();
   Tensor o = empty({B, T, H, Dv}, at::kBFloat16, q), st;
-  if (n_seq) o.zero_();      // rows that belong to no sequence are not written by the kernels
   if (want_state) st = empty({states, H, Dk, Dv}, at::kFloat, q);
   Tensor ws = empty({(int64_t)need}, at::kByte, q);
   const hipStream_t s = stream_of(dev);

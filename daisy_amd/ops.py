@@ -478,8 +478,7 @@ def kda_chunk_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     n_seq = _check_cu_seqlens(cu_seqlens, B) if cu_seqlens is not None else 0
     n_states = n_seq if n_seq else B
     q, k, v, g, beta, initial_state, scale = _kda_inputs(q, k, v, g, beta, initial_state, n_states, scale)
-    # rows that belong to no sequence (bounds that stop short of T) are not written by the kernels
-    o = (torch.zeros if n_seq else torch.empty)((B, T, H, Dv), dtype=torch.bfloat16, device=dev)
+    o = torch.empty((B, T, H, Dv), dtype=torch.bfloat16, device=dev)
     final = torch.empty((n_states, H, Dk, Dv), dtype=torch.float32, device=dev) if output_final_state else None
     lib = _lib.load()
     if n_seq:

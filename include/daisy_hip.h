@@ -278,7 +278,7 @@ int daisy_kda_chunk_fwd(const void* q, const void* k, const void* v,
  * (empty sequences allowed).  The bounds are read by the kernels, never by the host.  Every packed-
  * sequence kernel of this library (this one, daisy_kda_recurrent_varlen_fwd, daisy_short_conv_varlen_fwd)
  * forces each bound into 0..T, so that no bound can lead outside the tensors; rows that belong to no
- * sequence are left unwritten.  Bounds that DECREASE break the contract: every kernel stays inside the
+ * sequence are left unwritten (by this one: o is zero behind the last bound).  Bounds that DECREASE break the contract: every kernel stays inside the
  * tensors, but how tokens are then assigned to sequences differs between the kernels (this one takes
  * the running maximum of the bounds, the recurrent one clamps each pair, the convolution bisects over
  * them as they are) -- the three kernels of one layer agree only on bounds that honour the contract.

@@ -36,6 +36,18 @@ def test_kda_chunk_edges(T, Dk, Dv):
     assert ((S - S_ref).norm() / S_ref.norm()).item() <= 1e-3
 
 
+@pytest.mark.parametrize("decay", [3.0, 6.0, 9.0, 13.0, 22.0, 60.0])
+def test_kda_decays_around_the_limits(decay):
+    """Per-row decays whose sums over 16, 8 and 4 rows fall on either side of exp(-80)."""
+    q, k, v, _, beta = _inputs(1, 96, 2, 128, 32, seed=4)
+    g = torch.Generator().manual_seed(9)
+    gl = -decay * (0.5 + torch.rand(1, 96, 2, 128, generator=g)) * torch.rand(1, 1, 2, 128, generator=g).round()
+    o_ref, S_ref = oracle.kda_recurrent(q, k, v, gl, beta)
+    o, S = _run(q, k, v, gl, beta)
+    assert_close_bf16(o, o_ref, "o")
+    assert ((S - S_ref).norm() / S_ref.norm()).item() <= 1e-3
+
+
 @pytest.mark.parametrize("overlap", [0.5, 0.9])
 def test_kda_overlapping_keys(overlap):
     q, k, v, gl, beta = _inputs(1, 160, 2, 128, 64, seed=3, overlap=overlap)
@@ -45,11 +57,15 @@ def test_kda_overlapping_keys(overlap):
     assert ((S - S_ref).norm() / S_ref.norm()).item() <= 1e-3
 
 
-@pytest.mark.parametrize("lengths", [(1, 31, 0, 32, 33, 64, 5), (97,), (32, 32)])
-def test_kda_packed_chunk_slots(lengths):
-    q, k, v, gl, beta = _inputs(1, sum(lengths), 3, 64, 64, seed=sum(lengths))
+# 64 sequences: the most that a wavefront looks up by itself; 65 and more: from a table.  `behind`: rows after the last sequence.
+@pytest.mark.parametrize("lengths,behind", [((1, 31, 0, 32, 33, 64, 5), 0), ((97,), 3), ((32, 32), 65), ((3, 0, 33) * 21 + (1,), 7),
+                                            ((3, 0, 33) * 21 + (1, 40), 7), ((2,) * 130, 0)])
+def test_kda_packed_chunk_slots(lengths, behind):
+    q, k, v, gl, beta = _inputs(1, sum(lengths) + behind, 3, 64, 64, seed=sum(lengths))
     cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32)
+    torch.full((sum(lengths) + behind, 3, 64), float("nan"), dtype=torch.bfloat16, device="cuda")     # (what fresh memory may hold)
     o, S = _run(q, k, v, gl, beta, cu_seqlens=cu.cuda())
+    assert not o[:, sum(lengths):].any()
     for i, n in enumerate(lengths):
         a = int(cu[i])
         if n == 0:
