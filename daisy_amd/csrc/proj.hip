@@ -288,9 +288,11 @@ static int proj_tile(int M, int K, int head, COLUMNS columns) {
 
 // Against the library GEMM: level or ahead (1.0 to 1.7 times as fast) up to about four million outputs, and for short
 // rows at any size; 0.9 beyond that.  With the QKV epilogue it replaces the library GEMM and qkv_prep_kernel behind it
-// (another read and write of every row, 62 us of 228 us at M = 32768, N = 3072, K = 1024), which it beats at every size.
+// (another read and write of every row, 62 us of 228 us at M = 32768, N = 3072, K = 1024).  That pass is a fixed price per
+// output and the library's lead grows with K: ahead at every M up to K = 1536 (whole layer, M = 32768: 640 against 655 us),
+// behind from K = 2048 on where the product is large (M = 32768: 1014 against 981 us; M = 8192: 251 against 257 us).
 bool proj_wanted(int M, int N, int K) { return K % 64 == 0 && N % 8 == 0 && (K <= 512 || (int64_t)M * N <= 4300000); }
-bool proj_qkv_wanted(int M, int N, int K) { return K % 64 == 0; }
+bool proj_qkv_wanted(int M, int N, int K) { return K % 64 == 0 && (K <= 1536 || (int64_t)M * N <= 80000000); }
 
 template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI>
 static int launch_proj(ProjParams& p, hipStream_t s) {
