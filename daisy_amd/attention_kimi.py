@@ -88,7 +88,7 @@ def _project(lin: nn.Linear, x: Tensor) -> Tensor:
 
 def _plain(module: nn.Module, cls: type) -> bool:
     """Whether calling ``module`` is calling ``cls.forward`` and nothing else."""
-    return type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks
+    return type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__
 
 
 class KimiLinearSelfAttention(nn.Module):

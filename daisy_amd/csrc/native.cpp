@@ -8,12 +8,16 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <algorithm>
 #include <array>
@@ -27,9 +31,22 @@ using at::Tensor;
 using daisy::GateSource;
 
 // ---- arguments ----------------------------------------------------------------------------------------------------
+// A tensor whose operations nothing intercepts: no Python subclass, and none of the dispatch keys of vmap, function
+// transforms, fake or lazily conjugated or negated tensors, no tangent of forward-mode differentiation.
+bool is_tensor(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) return false;
+  constexpr c10::DispatchKeySet plain = c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::AutocastCUDA,
+                                                             c10::DispatchKey::ADInplaceOrView});
+  const Tensor& t = THPVariable_Unpack(o);
+  return t.defined() && (t.key_set() - plain).empty() && !t._fw_grad(0).defined();
+}
+bool tensor_or_none(PyObject* o) { return o == Py_None || is_tensor(o); }
 const Tensor* opt_tensor(PyObject* o) { return o == Py_None ? nullptr : &THPVariable_Unpack(o); }
-bool is_tensor(PyObject* o) { return THPVariable_Check(o); }
-bool tensor_or_none(PyObject* o) { return o == Py_None || THPVariable_Check(o); }
+// Whether someone watches or redirects the calls of this thread: those have to reach the library's operators one by one.
+bool intercepted() {
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing() ||
+         at::autocast::is_autocast_enabled(at::kCUDA);
+}
 
 // The current device when the tensor lives there, else -1 (asked of CPU tensors' processes too, which may have no device).
 int gpu_of(const Tensor& t) {
@@ -75,7 +92,24 @@ void* ptr(const Tensor& t) { return t.data_ptr(); }
 void* ptr(const Tensor* t) { return t ? t->data_ptr() : nullptr; }
 hipStream_t stream_of(int dev) { return c10::hip::getCurrentHIPStream(dev).stream(); }
 
-PyObject* none() { Py_RETURN_NONE; }
+// "Not here": borrowed, also without the interpreter lock (the method table's wrapper adds the reference).
+PyObject* none() { return Py_None; }
+PyObject* new_none() { Py_RETURN_NONE; }
+
+// The interpreter lock is given up while memory is allocated and kernels are launched, as the library's operators do.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  ~Unlocked() { end(); }
+  void end() {
+    if (state_) PyEval_RestoreThread(state_);
+    state_ = nullptr;
+  }
+
+ private:
+  PyThreadState* state_;
+};
+
 PyObject* wrap(const Tensor& t) { return THPVariable_Wrap(t); }
 
 // The gate logit of a layer with value embeddings; false when it is not a lone fp32 or bf16 number on the GPU.
@@ -117,7 +151,7 @@ bool own_linear(const Rows& x, const uint16_t* w, int64_t w_sn, int N, const uin
 // with that tile (tests and sweeps).
 PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 5 || !is_tensor(a[0]) || !is_tensor(a[1]) || !tensor_or_none(a[2])) return none();
+  if (intercepted() || n != 5 || !is_tensor(a[0]) || !is_tensor(a[1]) || !tensor_or_none(a[2])) return none();
   const Tensor &x = THPVariable_Unpack(a[0]), &w = THPVariable_Unpack(a[1]);
   const Tensor* bias = opt_tensor(a[2]);
   const int max_rows = (int)PyLong_AsLong(a[3]), tile = (int)PyLong_AsLong(a[4]);
@@ -131,11 +165,13 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!tile && !(r.M <= max_rows && !bias) && !(max_rows > 0 && daisy::proj_wanted(r.M, N, r.K))) return none();
   c10::SmallVector<int64_t, 5> sizes(x.sizes().begin(), x.sizes().end());
   sizes.back() = N;
+  Unlocked unlocked;
   Tensor y = empty(sizes, at::kBFloat16, x);
   const uint16_t* wp = (const uint16_t*)ptr(w);
   const hipStream_t s = stream_of(dev);
   const bool ok = tile ? daisy::proj_linear(r.p, r.stride, wp, w.stride(0), (const uint16_t*)ptr(bias), (uint16_t*)ptr(y), N, r.M, N, r.K, s, tile) == DAISY_OK
                        : own_linear(r, wp, w.stride(0), N, (const uint16_t*)ptr(bias), (uint16_t*)ptr(y), N, max_rows, s);
+  unlocked.end();
   return ok ? wrap(y) : none();
   END_HANDLE_TH_ERRORS
 }
@@ -144,7 +180,7 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // Arguments as for linear; weights and biases: tuples (a bias may be None).
 PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 5 || !is_tensor(a[0]) || !PyTuple_Check(a[1]) || !PyTuple_Check(a[2])) return none();
+  if (intercepted() || n != 5 || !is_tensor(a[0]) || !PyTuple_Check(a[1]) || !PyTuple_Check(a[2])) return none();
   const Py_ssize_t count = PyTuple_GET_SIZE(a[1]);
   if (count < 1 || count > daisy::kMaxSegments || PyTuple_GET_SIZE(a[2]) != count) return none();
   const Tensor& x = THPVariable_Unpack(a[0]);
@@ -164,6 +200,7 @@ PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
     seg[i] = daisy::ProjSegment{r.p, r.stride, (const uint16_t*)ptr(w), w.stride(0), (const uint16_t*)ptr(bias), nullptr, 0, (int)w.size(0), 0};
     pitch += (w.size(0) + 7) / 8 * 8;
   }
+  Unlocked unlocked;
   Tensor y = empty({(int64_t)r.M, pitch}, at::kBFloat16, x);
   int64_t at = 0;
   for (Py_ssize_t i = 0; i < count; ++i) {
@@ -174,6 +211,7 @@ PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const hipStream_t s = stream_of(dev);
   const int rc = r.M <= max_rows && !tile ? daisy::linear_segments(seg, (int)count, r.M, r.K, s) : daisy::proj_segments(seg, (int)count, r.M, r.K, s, tile);
   if (rc != DAISY_OK) return none();
+  unlocked.end();
   PyObject* res = PyTuple_New(count);
   at = 0;
   for (Py_ssize_t i = 0; i < count; ++i) {
@@ -188,7 +226,7 @@ PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // prefill_attention(q, k, v, window, scale, cos, sin, doc_start, out, k_out) -> (out, k_out)
 PyObject* py_prefill_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 10) return none();
+  if (intercepted() || n != 10) return none();
   for (int i : {0, 1, 2})
     if (!is_tensor(a[i])) return none();
   for (int i : {5, 6, 7, 8, 9})
@@ -208,6 +246,7 @@ PyObject* py_prefill_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (doc && !(int32_vector(*doc, T, dev) && doc->dim() == 1)) return none();
   for (const Tensor* t : {out, ko})
     if (t && (!rows_bf16(*t, 4, dev) || t->sizes() != q.sizes())) return none();
+  Unlocked unlocked;
   Tensor o = out ? *out : empty(q.sizes(), at::kBFloat16, q), kr;
   if (ko) kr = *ko;
   else if (cos) kr = empty(q.sizes(), at::kBFloat16, q);
@@ -216,9 +255,10 @@ PyObject* py_prefill_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                    (const int32_t*)ptr(doc), ptr(o), os.s, kr.defined() ? ptr(kr) : nullptr, kos.s,
                                    (int)B, (int)T, (int)H, (int)D, window, scale, 0, stream_of(dev));
   if (rc != DAISY_OK) return none();
+  unlocked.end();
   PyObject* r = PyTuple_New(2);
   PyTuple_SET_ITEM(r, 0, wrap(o));
-  PyTuple_SET_ITEM(r, 1, kr.defined() ? wrap(kr) : none());
+  PyTuple_SET_ITEM(r, 1, kr.defined() ? wrap(kr) : new_none());
   return r;
   END_HANDLE_TH_ERRORS
 }
@@ -228,7 +268,7 @@ PyObject* py_prefill_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // CausalSelfAttention.prefill on bf16 weights: QKV projection, norm + RoPE + value mix, attention, output projection.
 PyObject* py_layer_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 16) return none();
+  if (intercepted() || n != 16) return none();
   for (int i : {0, 1, 2, 3})
     if (!is_tensor(a[i])) return none();
   for (int i : {7, 8, 9, 10, 11})
@@ -256,6 +296,7 @@ PyObject* py_layer_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   for (const Tensor* t : {k_out, v_out})
     if (t && (!rows_bf16(*t, 4, dev) || t->size(0) != B || t->size(1) != T || t->size(2) != H || t->size(3) != D)) return none();
 
+  Unlocked unlocked;
   const hipStream_t s = stream_of(dev);
   const uint16_t* wp = (const uint16_t*)ptr(w);
   const std::array<int64_t, 4> shape{B, T, H, D};
@@ -296,9 +337,10 @@ PyObject* py_layer_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   } else {
     y = at::linear(o.view({B, T, (int64_t)dim}), w.select(0, 3));
   }
+  unlocked.end();
   PyObject* res = PyTuple_New(4);
   PyTuple_SET_ITEM(res, 0, wrap(y));
-  PyTuple_SET_ITEM(res, 1, want_q ? wrap(q) : none());
+  PyTuple_SET_ITEM(res, 1, want_q ? wrap(q) : new_none());
   PyTuple_SET_ITEM(res, 2, wrap(k));
   PyTuple_SET_ITEM(res, 3, wrap(v));
   return res;
@@ -310,7 +352,7 @@ PyObject* py_layer_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // CausalSelfAttention.step on a ring: QKV projection, the one-launch attention step, output projection.
 PyObject* py_layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 13) return none();
+  if (intercepted() || n != 13) return none();
   for (int i : {0, 1, 2, 3, 5, 6})
     if (!is_tensor(a[i])) return none();
   for (int i : {7, 8, 9})
@@ -340,6 +382,7 @@ PyObject* py_layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   GateSource gate{nullptr, 0};
   if (ve && !(gate_source(*g_ve, dev, gate) && on_gpu(*ve, dev) && bf16(*ve) && ve->is_contiguous() && ve->numel() == B * dim)) return none();
 
+  Unlocked unlocked;
   const hipStream_t s = stream_of(dev);
   const uint16_t* wp = (const uint16_t*)ptr(w);
   Tensor qkv;
@@ -378,11 +421,12 @@ PyObject* py_layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   } else {
     y = at::linear(o, w.select(0, 3));
   }
+  unlocked.end();
   PyObject* res = PyTuple_New(3);
   PyTuple_SET_ITEM(res, 0, wrap(y));
   if (pos_dev) {
-    PyTuple_SET_ITEM(res, 1, none());
-    PyTuple_SET_ITEM(res, 2, none());
+    PyTuple_SET_ITEM(res, 1, new_none());
+    PyTuple_SET_ITEM(res, 2, new_none());
   } else {
     if (!f16) {
       const int64_t slot = pos % W;
@@ -403,7 +447,7 @@ PyObject* py_layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // kda_chunk(q, k, v, g, beta, scale, initial_state, want_state, l2norm, l2_eps, cu_seqlens) -> (o, state or None)
 PyObject* py_kda_chunk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 11) return none();
+  if (intercepted() || n != 11) return none();
   for (int i : {0, 1, 2, 3, 4})
     if (!is_tensor(a[i])) return none();
   if (!tensor_or_none(a[6]) || !tensor_or_none(a[10])) return none();
@@ -433,6 +477,7 @@ PyObject* py_kda_chunk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const size_t need = n_seq ? daisy_kda_varlen_workspace_bytes((int)T, (int)n_seq, (int)H, (int)Dk, (int)Dv, 64)
                             : daisy_kda_workspace_bytes((int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64);
   if (need == 0) return none();
+  Unlocked unlocked;
   Tensor o = empty({B, T, H, Dv}, at::kBFloat16, q), st;
   if (want_state) st = empty({states, H, Dk, Dv}, at::kFloat, q);
   Tensor ws = empty({(int64_t)need}, at::kByte, q);
@@ -444,9 +489,10 @@ PyObject* py_kda_chunk(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                              want_state ? (float*)ptr(st) : nullptr, (int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64, scale,
                                              l2norm, l2_eps, ptr(ws), need, s);
   if (rc != DAISY_OK) return none();
+  unlocked.end();
   PyObject* r = PyTuple_New(2);
   PyTuple_SET_ITEM(r, 0, wrap(o));
-  PyTuple_SET_ITEM(r, 1, want_state ? wrap(st) : none());
+  PyTuple_SET_ITEM(r, 1, want_state ? wrap(st) : new_none());
   return r;
   END_HANDLE_TH_ERRORS
 }
@@ -459,7 +505,7 @@ PyObject* py_kda_chunk(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   constexpr int kWeights = 19;
-  if (n != 12 || !is_tensor(a[0]) || !PyTuple_Check(a[1]) || PyTuple_GET_SIZE(a[1]) != kWeights || !tensor_or_none(a[6])) return none();
+  if (intercepted() || n != 12 || !is_tensor(a[0]) || !PyTuple_Check(a[1]) || PyTuple_GET_SIZE(a[1]) != kWeights || !tensor_or_none(a[6])) return none();
   if (!PyTuple_Check(a[7]) || PyTuple_GET_SIZE(a[7]) != 3 || !PyTuple_Check(a[8]) || PyTuple_GET_SIZE(a[8]) != 4) return none();
   const Tensor* w[kWeights];
   for (int i = 0; i < kWeights; ++i) {
@@ -513,9 +559,11 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!vector(w[16], H, at::kFloat) || !vector(w[17], kd, at::kFloat) || !vector(w[18], Dv, at::kBFloat16)) return none();
   if (state && !(vector(state, B * kd * Dv, at::kFloat) && state->dim() == 4 && state->size(0) == B && state->size(1) == H && state->size(2) == Dk)) return none();
   const bool step = keep && T == 1 && state;
-  if (step ? !(win[0] && win[1] && win[2] && daisy::kda_layer_step_serves((int)Dk, (int)Dv, (int)taps)) : (dim % 64 != 0 || Dv % 64 != 0)) return none();
+  const size_t need = step ? 0 : daisy_kda_workspace_bytes((int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64);
+  if (step ? !(win[0] && win[1] && win[2] && daisy::kda_layer_step_serves((int)Dk, (int)Dv, (int)taps)) : (need == 0 || dim % 64 != 0 || Dv % 64 != 0)) return none();
 
   // ---- the projections of the input ---------------------------------------------------------------------------------
+  Unlocked unlocked;
   const hipStream_t s = stream_of(dev);
   const uint16_t* W[kWeights];
   for (int i = 0; i < kWeights; ++i) W[i] = (const uint16_t*)ptr(w[i]);
@@ -581,7 +629,6 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
                              (float*)ptr(beta), M, (int)H, (int)Dk, s) != DAISY_OK) return none();
     o = empty({B, T, vd}, at::kBFloat16, x);
     if (keep) st = keeper(home[0], {B, H, Dk, Dv}, at::kFloat);
-    const size_t need = daisy_kda_workspace_bytes((int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64);
     Tensor ws = empty({(int64_t)need}, at::kByte, x);
     if (daisy_kda_chunk_fwd(ptr(conv[0]), ptr(conv[1]), ptr(conv[2]), ptr(g), 1, (const float*)ptr(beta), (const float*)ptr(state), ptr(o),
                             keep ? (float*)ptr(st) : nullptr, (int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64, scale, 1, kL2Eps, ptr(ws), need, s) != DAISY_OK)
@@ -595,15 +642,22 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   } else {
     y = at::linear(o, *w[9]);
   }
+  unlocked.end();
   PyObject* res = PyTuple_New(5);
   PyTuple_SET_ITEM(res, 0, wrap(y));
-  PyTuple_SET_ITEM(res, 1, !keep ? none() : wrap(step ? *state : st));
-  for (int i = 0; i < 3; ++i) PyTuple_SET_ITEM(res, 2 + i, !keep ? none() : wrap(step ? *win[i] : new_win[i]));
+  PyTuple_SET_ITEM(res, 1, !keep ? new_none() : wrap(step ? *state : st));
+  for (int i = 0; i < 3; ++i) PyTuple_SET_ITEM(res, 2 + i, !keep ? new_none() : wrap(step ? *win[i] : new_win[i]));
   return res;
   END_HANDLE_TH_ERRORS
 }
 
-#define FAST(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyObject* call(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  PyObject* r = F(self, a, n);
+  if (r == Py_None) Py_INCREF(r);
+  return r;
+}
+#define FAST(name) {#name, (PyCFunction)(void (*)(void))call<py_##name>, METH_FASTCALL, nullptr}
 PyMethodDef kMethods[] = {FAST(linear), FAST(linears), FAST(prefill_attention), FAST(layer_prefill), FAST(layer_step), FAST(kda_chunk), FAST(kda_layer),
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

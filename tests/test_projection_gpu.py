@@ -73,3 +73,24 @@ def test_attention_on_both_sides_of_the_block_rule(D, B, H, T, window, docs):
     p = s.masked_fill(~seen, float("-inf")).softmax(-1)
     ref = torch.matmul(p, v.float().transpose(1, 2).contiguous()).transpose(1, 2)
     assert_close_bf16(o, ref, f"o T={T}")
+
+
+def test_calls_that_something_intercepts_reach_the_library_op():
+    """Tangents, subclasses, vmap and autocast of a decode batch's projection (64 rows: above the few-rows kernel)."""
+    from daisy_amd.attention import step_linear
+    g = torch.Generator().manual_seed(7)
+    x, w, dx = (torch.randn(*s, generator=g).bfloat16().to(DEV) for s in ((64, 256), (512, 256), (64, 256)))
+    with torch.no_grad():
+        assert _lib.native().linear(x, w, None, 4, 0) is not None
+        import torch.autograd.forward_ad as fwad
+        with fwad.dual_level():
+            y = fwad.unpack_dual(step_linear(fwad.make_dual(x, dx), w))
+            assert torch.equal(y.tangent, torch.nn.functional.linear(dx, w))
+        assert torch.equal(torch.vmap(lambda a: step_linear(a, w))(x[None]), torch.nn.functional.linear(x[None], w))
+
+        class Sub(torch.Tensor):
+            pass
+
+        assert type(step_linear(x.as_subclass(Sub), w)) is Sub
+        with torch.autocast("cuda", torch.float16):
+            assert step_linear(x, w).dtype == torch.float16
