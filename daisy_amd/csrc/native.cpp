@@ -38,7 +38,7 @@ bool is_tensor(PyObject* o) {
   constexpr c10::DispatchKeySet plain = c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::AutocastCUDA,
                                                              c10::DispatchKey::ADInplaceOrView});
   const Tensor& t = THPVariable_Unpack(o);
-  return t.defined() && (t.key_set() - plain).empty() && !t._fw_grad(0).defined();
+  return t.defined() && (t.key_set().raw_repr() & ~plain.raw_repr()) == 0 && !t._fw_grad(0).defined();
 }
 bool tensor_or_none(PyObject* o) { return o == Py_None || is_tensor(o); }
 const Tensor* opt_tensor(PyObject* o) { return o == Py_None ? nullptr : &THPVariable_Unpack(o); }
