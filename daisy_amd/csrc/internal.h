@@ -34,6 +34,14 @@ struct QkvEpilogue {
 // y [M, N] = x [M, K] w [N, K]^T (+ bias), fp32 accumulation, one rounding.  tile: 0 = by the sizes.
 int proj_linear(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const uint16_t* bias,
                 uint16_t* y, int64_t y_sm, int M, int N, int K, hipStream_t s, int tile = 0);
+// The decay gate of the KDA layer as a product's epilogue: y = -exp(A_log[h]) * softplus(y + dt_bias) on the bf16 product, heads of Dk
+// channels (a multiple of 8), and beside it beta [M, H] = bf16(sigmoid(logits)) as fp32, logits rows `logits_row` elements apart.
+struct KdaGates {
+  const float *A_log, *dt_bias;      // [H], [H * Dk]
+  int H, Dk;
+  const uint16_t* logits; int64_t logits_row;
+  float* beta;
+};
 // One of several products over the same number of rows M and the same K that share a launch: y = x w^T (+ bias).  N need not be a
 // multiple of 8 where y's rows have room for it (y_sm >= N rounded up to 8; the columns from N on are then scribbled over).
 struct ProjSegment {
@@ -44,7 +52,8 @@ struct ProjSegment {
   int N, tile_end;      // tile_end: filled in by the launch
 };
 constexpr int kMaxSegments = 6;
-int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, int tile = 0);
+// gates: what becomes of the first product on its way out (its N is H Dk).
+int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, int tile = 0, const KdaGates* gates = nullptr);
 // The same through the weight-streaming kernel of linear.hip, M <= 8 (no bias); every row as daisy_linear_rows_fwd computes it.
 int linear_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s);
 // Whether the tiled kernel is the better choice for these sizes than the library GEMM (and, for the QKV projection, than
@@ -103,9 +112,17 @@ struct KdaLayerStep {
   uint16_t* o; int64_t o_row;             // [B, H * Dv]
   int H, Dk; float scale, l2_eps, norm_eps;
 };
-// daisy_kda_gate_fwd (bf16, slope 1, threshold 20) and beta = bf16(sigmoid(logits)) as fp32 [rows, H] in one launch; out may be g.
-int kda_gate_beta(const uint16_t* g, const float* A_log, const float* bias, uint16_t* out, const uint16_t* logits, int64_t logits_row,
-                  float* beta, int64_t rows, int H, int Dk, hipStream_t s);
+// daisy_short_conv_fwd for one to three inputs of the same B, T and number of taps in one launch.
+struct ConvPart {
+  const uint16_t* x; int64_t x_sb, x_st;       // [B, T, C], channel stride 1
+  const uint16_t* w;                           // [C, K]
+  const uint16_t* bias;                        // [C] or null
+  const uint16_t* cache_in;                    // [B, C, K] or null: the last K inputs before t = 0 (the first is unused)
+  uint16_t* y; int64_t y_sb, y_st;             // [B, T, C]
+  uint16_t* cache_out;                         // [B, C, K] or null: the last K inputs of the extended sequence
+  int C;
+};
+int short_conv_group(const ConvPart* parts, int n, int B, int T, int K, int silu, hipStream_t s);
 bool kda_layer_step_serves(int Dk, int Dv, int taps);
 int kda_layer_step(const KdaLayerStep& p, int B, int Dv, hipStream_t s);
 

@@ -4,20 +4,11 @@
 
 namespace daisy {
 
-// beta = sigmoid(logit) in the layer's bf16, as the fp32 the delta rule takes: rows of H logits `row` elements apart.
-struct BetaRows { const uint16_t* logits; int64_t row; float* out; int64_t total; };
-
 // out = -exp(A_log[h]) * softplus(g + bias[h, d]).  VEC = 8: a thread takes 8 consecutive channels
-// (Dk a multiple of 8), 16-byte accesses; VEC = 1: one element per thread, any Dk.  Workgroups from gate_blocks on make beta.
+// (Dk a multiple of 8), 16-byte accesses; VEC = 1: one element per thread, any Dk.
 template <bool BF16, int VEC>
 __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const float* A_log, const float* bias, void* out,
-                                                       int64_t total, int H, int Dk, float sp_beta, float threshold,
-                                                       uint32_t gate_blocks, BetaRows br) {
-  if (blockIdx.x >= gate_blocks) {
-    const int64_t i = (int64_t)(blockIdx.x - gate_blocks) * blockDim.x + threadIdx.x;
-    if (i < br.total) br.out[i] = round_bf16(1.f / (1.f + expf(-bf16lo_to_f32(br.logits[i / H * br.row + i % H]))));
-    return;
-  }
+                                                       int64_t total, int H, int Dk, float sp_beta, float threshold) {
   const uint32_t vi = blockIdx.x * blockDim.x + threadIdx.x;   // 32-bit index arithmetic (64-bit division is slow)
   const int64_t i = (int64_t)vi * VEC;
   if (i >= total) return;
@@ -1047,36 +1038,25 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
 
 using namespace daisy;
 
-static int gate_launch(const void* g, const float* A_log, const float* bias, void* out, int64_t rows, int H, int Dk, int io_is_bf16,
-                       float softplus_beta, float threshold, const BetaRows& br, hipStream_t s) {
+extern "C" int daisy_kda_gate_fwd(const void* g, const float* A_log, const float* bias, void* out,
+                                  int64_t rows, int H, int Dk, int io_is_bf16,
+                                  float softplus_beta, float threshold, void* stream) {
   DAISY_CHECK_ARG(g && A_log && out, "kda_gate: g, A_log and out must be non-NULL");
   DAISY_CHECK_ARG(rows >= 0 && H > 0 && Dk > 0, "kda_gate: rows=%lld, H=%d, Dk=%d invalid", (long long)rows, H, Dk);
   DAISY_CHECK_ARG(softplus_beta > 0.f, "kda_gate: softplus beta must be positive");
   const int64_t total = rows * H * Dk;
   if (total == 0) return DAISY_OK;
+  hipStream_t s = (hipStream_t)stream;
   const bool vec = Dk % 8 == 0 && (reinterpret_cast<uintptr_t>(g) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  const int64_t nblk = ((vec ? total / 8 : total) + 255) / 256, all = nblk + (br.total + 255) / 256;
-  DAISY_CHECK_ARG(all <= 0x7fffffff, "kda_gate: too many elements");
-  const dim3 grid((unsigned)all), block(256);
-  const uint32_t nb = (uint32_t)nblk;
-  if (vec && io_is_bf16) hipLaunchKernelGGL((kda_gate_kernel<true, 8>), grid, block, 0, s, g, A_log, bias, out, total, H, Dk, softplus_beta, threshold, nb, br);
-  else if (vec) hipLaunchKernelGGL((kda_gate_kernel<false, 8>), grid, block, 0, s, g, A_log, bias, out, total, H, Dk, softplus_beta, threshold, nb, br);
-  else if (io_is_bf16) hipLaunchKernelGGL((kda_gate_kernel<true, 1>), grid, block, 0, s, g, A_log, bias, out, total, H, Dk, softplus_beta, threshold, nb, br);
-  else hipLaunchKernelGGL((kda_gate_kernel<false, 1>), grid, block, 0, s, g, A_log, bias, out, total, H, Dk, softplus_beta, threshold, nb, br);
+  const int64_t nblk = ((vec ? total / 8 : total) + 255) / 256;
+  DAISY_CHECK_ARG(nblk <= 0x7fffffff, "kda_gate: too many elements");
+  const dim3 grid((unsigned)nblk), block(256);
+  if (vec && io_is_bf16) hipLaunchKernelGGL((kda_gate_kernel<true, 8>), grid, block, 0, s, g, A_log, bias, out, total, H, Dk, softplus_beta, threshold);
+  else if (vec) hipLaunchKernelGGL((kda_gate_kernel<false, 8>), grid, block, 0, s, g, A_log, bias, out, total, H, Dk, softplus_beta, threshold);
+  else if (io_is_bf16) hipLaunchKernelGGL((kda_gate_kernel<true, 1>), grid, block, 0, s, g, A_log, bias, out, total, H, Dk, softplus_beta, threshold);
+  else hipLaunchKernelGGL((kda_gate_kernel<false, 1>), grid, block, 0, s, g, A_log, bias, out, total, H, Dk, softplus_beta, threshold);
   DAISY_CHECK_LAUNCH("kda_gate_kernel");
   return DAISY_OK;
-}
-
-extern "C" int daisy_kda_gate_fwd(const void* g, const float* A_log, const float* bias, void* out,
-                                  int64_t rows, int H, int Dk, int io_is_bf16,
-                                  float softplus_beta, float threshold, void* stream) {
-  return gate_launch(g, A_log, bias, out, rows, H, Dk, io_is_bf16, softplus_beta, threshold, BetaRows{nullptr, 0, nullptr, 0}, (hipStream_t)stream);
-}
-
-int daisy::kda_gate_beta(const uint16_t* g, const float* A_log, const float* bias, uint16_t* out, const uint16_t* logits, int64_t logits_row,
-                         float* beta, int64_t rows, int H, int Dk, hipStream_t s) {
-  DAISY_CHECK_ARG(logits && beta, "kda_gate_beta: logits and beta must be non-NULL");
-  return gate_launch(g, A_log, bias, out, rows, H, Dk, 1, 1.f, 20.f, BetaRows{logits, logits_row, beta, rows * H}, s);
 }
 
 

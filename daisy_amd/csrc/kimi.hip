@@ -12,6 +12,7 @@
 
 namespace daisy {
 
+// The varlen kernel's arguments.
 struct ConvParams {
   const uint16_t* x; int64_t x_sb, x_st;       // [B, T, C], channel stride 1
   const uint16_t* w;                           // [C, K]
@@ -21,21 +22,32 @@ struct ConvParams {
   uint16_t* cache_out;                         // [B, C, K] or null: the last K inputs of the extended sequence
   int B, T, C, silu;
 };
+// Up to three convolutions over the same positions in one launch, told apart by the column of workgroups.
+struct ConvGroup {
+  ConvPart part[3];
+  int block_end[3];      // first column of workgroups behind each part
+  int T, silu, seg;      // seg: time steps per thread
+};
 
-constexpr int kConvSeg = 32;   // time steps per thread
+constexpr int kConvSeg = 32;        // time steps per thread
+constexpr int kConvSegShort = 8;    // ... of a short input
 
-// A thread owns 8 consecutive channels and kConvSeg consecutive time steps; the K-1 inputs
+// A thread owns 8 consecutive channels and `seg` consecutive time steps; the K-1 inputs
 // before its first step come from the sequence itself or from the carried window.  The sum is
 // taken in fp32 and rounded to bf16 before the activation, which is again evaluated in fp32 and
 // rounded (the two roundings of a bf16 convolution followed by a bf16 SiLU).
 template <int K>
-__global__ __launch_bounds__(256) void short_conv_kernel(ConvParams p) {
-  const int cg = blockIdx.x * 256 + threadIdx.x;        // group of 8 channels
+__global__ __launch_bounds__(256) void short_conv_kernel(ConvGroup group) {
+  int part = 0;
+  while (part < 2 && (int)blockIdx.x >= group.block_end[part]) ++part;
+  const ConvPart p = group.part[part];
+  const int T = group.T;
+  const int cg = (blockIdx.x - (part > 0 ? group.block_end[part - 1] : 0)) * 256 + threadIdx.x;        // group of 8 channels
   const int c0 = 8 * cg;
   if (c0 >= p.C) return;
   const int b = blockIdx.z;
-  const int t0 = blockIdx.y * kConvSeg;
-  const int t1 = min(t0 + kConvSeg, p.T);
+  const int t0 = blockIdx.y * group.seg;
+  const int t1 = min(t0 + group.seg, T);
 
   float w[K][8], acc0[8];
   {
@@ -103,7 +115,7 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParams p) {
     u32x4 raw[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int t = min(tb + u, p.T - 1);   // steps past the end re-read the last row and are not stored
+      const int t = min(tb + u, T - 1);   // steps past the end re-read the last row and are not stored
       raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.x + b * p.x_sb + (int64_t)t * p.x_st + c0));
     }
 #pragma unroll
@@ -116,7 +128,7 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParams p) {
 #pragma unroll
         for (int j = 0; j < K - 1; ++j) a = fmaf(w[j][e], win[j][e], a);
         a = round_bf16(fmaf(w[K - 1][e], xin[e], a));
-        if (p.silu) a = a * __builtin_amdgcn_rcpf(1.f + __expf(-a));
+        if (group.silu) a = a * __builtin_amdgcn_rcpf(1.f + __expf(-a));
         out[e] = a;
       }
       if (tb + u < t1) *reinterpret_cast<u32x4*>(p.y + b * p.y_sb + (int64_t)(tb + u) * p.y_st + c0) = pack8(out);
@@ -129,10 +141,10 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvParams p) {
     }
   }
   // The thread that reaches the end of the sequence leaves the window for the next call.
-  if (p.cache_out != nullptr && t1 == p.T) {
+  if (p.cache_out != nullptr && t1 == T) {
     float last[K][8];
 #pragma unroll
-    for (int j = 0; j < K; ++j) input_at(p.T - K + j, last[j]);
+    for (int j = 0; j < K; ++j) input_at(T - K + j, last[j]);
     if (K == 4) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -266,36 +278,53 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(GatedNormParams p) {
 
 using namespace daisy;
 
+// A thread walks its steps eight inputs at a time, so a short input, whose threads do not fill the chip, lasts as long as one
+// thread's chain of loads: threads of eight steps there (three more rows read per eight, all cached).  LINE_FIGURES
+int daisy::short_conv_group(const ConvPart* parts, int n, int B, int T, int K, int silu, hipStream_t s) {
+  DAISY_CHECK_ARG(parts && n >= 1 && n <= 3 && B > 0 && T > 0, "short_conv: %d parts, B=%d, T=%d", n, B, T);
+  DAISY_CHECK_SUPPORTED(K >= 2 && K <= 4, "short_conv: kernel size %d not supported (2..4)", K);
+  DAISY_CHECK_ARG(B <= 65535, "short_conv: B must be <= 65535");
+  auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
+  ConvGroup g{};
+  int columns = 0;
+  bool in_place = false;
+  for (int i = 0; i < 3; ++i) {
+    if (i < n) {
+      const ConvPart& p = parts[i];
+      DAISY_CHECK_ARG(p.x && p.w && p.y && p.C > 0, "short_conv: x, weight and y must be non-NULL, C=%d positive", p.C);
+      DAISY_CHECK_SUPPORTED(p.C % 8 == 0, "short_conv: channels (%d) must be a multiple of 8", p.C);
+      DAISY_CHECK_ARG(al16(p.x) && al16(p.y) && al16(p.bias) && al16(p.w) && al16(p.cache_in) && al16(p.cache_out),
+                      "short_conv: x, y, weight, bias and the windows must be 16-byte aligned");
+      DAISY_CHECK_ARG(p.x_sb % 8 == 0 && p.x_st % 8 == 0 && p.y_sb % 8 == 0 && p.y_st % 8 == 0, "short_conv: strides must be multiples of 8 elements");
+      // Updating the window in place is safe only while the thread that writes it is the one that read it.
+      const bool same = p.cache_out != nullptr && p.cache_out == p.cache_in;
+      DAISY_CHECK_ARG(!same || T <= kConvSeg, "short_conv: the window can be updated in place for T <= %d only (T=%d)", kConvSeg, T);
+      in_place |= same;
+      g.part[i] = p;
+      columns += (p.C / 8 + 255) / 256;
+    }
+    g.block_end[i] = columns;
+  }
+  g.T = T; g.silu = silu;
+  const int64_t workgroups = (int64_t)columns * B * ((T + kConvSeg - 1) / kConvSeg);
+  g.seg = workgroups < 256 && !in_place ? kConvSegShort : kConvSeg;
+  const dim3 grid((unsigned)columns, (unsigned)((T + g.seg - 1) / g.seg), (unsigned)B);
+  DAISY_CHECK_ARG(grid.y <= 65535, "short_conv: T=%d too long for one launch", T);
+  if (K == 4) hipLaunchKernelGGL(short_conv_kernel<4>, grid, dim3(256), 0, s, g);
+  else if (K == 3) hipLaunchKernelGGL(short_conv_kernel<3>, grid, dim3(256), 0, s, g);
+  else hipLaunchKernelGGL(short_conv_kernel<2>, grid, dim3(256), 0, s, g);
+  DAISY_CHECK_LAUNCH("short_conv_kernel");
+  return DAISY_OK;
+}
+
 extern "C" int daisy_short_conv_fwd(const void* x, const int64_t* x_strides, const void* weight, const void* bias,
                                     const void* cache_in, void* y, const int64_t* y_strides, void* cache_out,
                                     int B, int T, int C, int K, int apply_silu, void* stream) {
   DAISY_CHECK_ARG(x && weight && y && x_strides && y_strides, "short_conv: x, weight, y and the stride arrays must be non-NULL");
   DAISY_CHECK_ARG(B > 0 && T > 0 && C > 0, "short_conv: B=%d, T=%d, C=%d must be positive", B, T, C);
-  DAISY_CHECK_SUPPORTED(K >= 2 && K <= 4, "short_conv: kernel size %d not supported (2..4)", K);
-  DAISY_CHECK_SUPPORTED(C % 8 == 0, "short_conv: channels (%d) must be a multiple of 8", C);
-  DAISY_CHECK_ARG(B <= 65535, "short_conv: B must be <= 65535");
-  auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
-  DAISY_CHECK_ARG(al16(x) && al16(y) && al16(bias) && al16(weight) && al16(cache_in) && al16(cache_out),
-                  "short_conv: x, y, weight, bias and the windows must be 16-byte aligned");
-  for (int i = 0; i < 2; ++i)
-    DAISY_CHECK_ARG(x_strides[i] % 8 == 0 && y_strides[i] % 8 == 0, "short_conv: strides must be multiples of 8 elements");
-  // Updating the window in place is safe only while the thread that writes it is the one that read it.
-  DAISY_CHECK_ARG(cache_out == nullptr || cache_out != cache_in || T <= kConvSeg,
-                  "short_conv: the window can be updated in place for T <= %d only (T=%d)", kConvSeg, T);
-  ConvParams p;
-  p.x = (const uint16_t*)x; p.x_sb = x_strides[0]; p.x_st = x_strides[1];
-  p.w = (const uint16_t*)weight; p.bias = (const uint16_t*)bias; p.cache_in = (const uint16_t*)cache_in;
-  p.y = (uint16_t*)y; p.y_sb = y_strides[0]; p.y_st = y_strides[1];
-  p.cache_out = (uint16_t*)cache_out;
-  p.B = B; p.T = T; p.C = C; p.silu = apply_silu;
-  const dim3 grid((unsigned)((C / 8 + 255) / 256), (unsigned)((T + kConvSeg - 1) / kConvSeg), (unsigned)B);
-  DAISY_CHECK_ARG(grid.y <= 65535, "short_conv: T=%d too long for one launch", T);
-  hipStream_t s = (hipStream_t)stream;
-  if (K == 4) hipLaunchKernelGGL(short_conv_kernel<4>, grid, dim3(256), 0, s, p);
-  else if (K == 3) hipLaunchKernelGGL(short_conv_kernel<3>, grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL(short_conv_kernel<2>, grid, dim3(256), 0, s, p);
-  DAISY_CHECK_LAUNCH("short_conv_kernel");
-  return DAISY_OK;
+  const ConvPart p{(const uint16_t*)x, x_strides[0], x_strides[1], (const uint16_t*)weight, (const uint16_t*)bias, (const uint16_t*)cache_in,
+                   (uint16_t*)y, y_strides[0], y_strides[1], (uint16_t*)cache_out, C};
+  return daisy::short_conv_group(&p, 1, B, T, K, apply_silu, (hipStream_t)stream);
 }
 
 extern "C" int daisy_short_conv_varlen_fwd(const void* x, int64_t x_row_stride, const void* weight, const void* bias,

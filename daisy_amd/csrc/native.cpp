@@ -610,23 +610,23 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return h && on_gpu(*h, dev) && h->scalar_type() == type && h->is_contiguous() && h->sizes() == shape ? *h : empty(shape, type, x);
     };
     Tensor conv[3];
+    daisy::ConvPart parts[3];
     for (int i = 0; i < 3; ++i) {
       conv[i] = empty({B, T, widths[i]}, at::kBFloat16, x);
       const std::array<int64_t, 3> shape{B, widths[i], taps};
       // (a window is updated in place for short inputs only)
       if (keep) new_win[i] = win[i] && home[i + 1] && win[i]->data_ptr() == home[i + 1]->data_ptr() && T > 32 ? empty(shape, at::kBFloat16, x)
-                                                                                                             : keeper(home[i + 1], shape, at::kBFloat16);
-      const int64_t in[2] = {T * seg[i].y_sm, seg[i].y_sm}, out[2] = {T * widths[i], widths[i]};
-      if (daisy_short_conv_fwd(seg[i].y, in, W[10 + i], W[13 + i], ptr(win[i]), ptr(conv[i]), out, keep ? ptr(new_win[i]) : nullptr,
-                               (int)B, (int)T, (int)widths[i], (int)taps, 1, s) != DAISY_OK) return none();
-      big[i] = Tensor();
+                                                                                                           : keeper(home[i + 1], shape, at::kBFloat16);
+      parts[i] = daisy::ConvPart{seg[i].y, T * seg[i].y_sm, seg[i].y_sm, W[10 + i], W[13 + i], (const uint16_t*)ptr(win[i]), (uint16_t*)ptr(conv[i]),
+                                 T * widths[i], widths[i], keep ? (uint16_t*)ptr(new_win[i]) : nullptr, (int)widths[i]};
     }
+    if (daisy::short_conv_group(parts, 3, (int)B, (int)T, (int)taps, 1, s) != DAISY_OK) return none();
+    for (Tensor& t : big) t = Tensor();
     Tensor g = empty({M, kd}, at::kBFloat16, x), gate = empty({M, vd}, at::kBFloat16, x), beta = empty({M, H}, at::kFloat, x);
     const daisy::ProjSegment low[2] = {{seg[3].y, seg[3].y_sm, W[6], Dv, nullptr, (uint16_t*)ptr(g), kd, (int)kd, 0},
                                        {seg[4].y, seg[4].y_sm, W[7], Dv, W[8], (uint16_t*)ptr(gate), vd, (int)vd, 0}};
-    if (daisy::proj_segments(low, 2, (int)M, (int)Dv, s) != DAISY_OK) return none();
-    if (daisy::kda_gate_beta((const uint16_t*)ptr(g), (const float*)ptr(w[16]), (const float*)ptr(w[17]), (uint16_t*)ptr(g), seg[5].y, seg[5].y_sm,
-                             (float*)ptr(beta), M, (int)H, (int)Dk, s) != DAISY_OK) return none();
+    const daisy::KdaGates gates{(const float*)ptr(w[16]), (const float*)ptr(w[17]), (int)H, (int)Dk, seg[5].y, seg[5].y_sm, (float*)ptr(beta)};
+    if (daisy::proj_segments(low, 2, (int)M, (int)Dv, s, 0, &gates) != DAISY_OK) return none();
     o = empty({B, T, vd}, at::kBFloat16, x);
     if (keep) st = keeper(home[0], {B, H, Dk, Dv}, at::kFloat);
     Tensor ws = empty({(int64_t)need}, at::kByte, x);

@@ -29,6 +29,7 @@ struct ProjParams {
 struct ProjSegmentsParams {
   ProjSegment seg[kMaxSegments];
   int n, M, K, MT, NT;
+  KdaGates gates;                      // EPI 3
 };
 
 // At most N vector-memory operations outstanding (bits 3:0 and 15:14 of the immediate) and every LDS read back.
@@ -38,6 +39,7 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 
 // EPI 0: y = x W^T (+ bias), bf16, of one or (SEGMENTS) several products.  EPI 1 / 2: the QKV epilogue for heads of 64 / 128 channels.
+// EPI 3: as 0, the first product through the KDA layer's decay gate.
 // WVM x WVN wavefronts; BK elements of K per step.
 template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI, bool SEGMENTS = false>
 __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t<SEGMENTS, ProjSegmentsParams, ProjParams> p) {
@@ -67,11 +69,13 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
   const int mt = 8 * panel + in_panel % rows;
   int nt = in_panel / rows;
   const ProjSegment* gp;
+  [[maybe_unused]] bool gated = false;
   if constexpr (SEGMENTS) {
     int i = 0;
     while (i + 1 < p.n && nt >= p.seg[i].tile_end) ++i;
     if (i > 0) nt -= p.seg[i - 1].tile_end;
     gp = &p.seg[i];
+    gated = EPI == 3 && i == 0;
   } else {
     gp = &p.one;
   }
@@ -166,7 +170,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
   for (int i = 0; i < NI; ++i) {
     const int n = WN * wn + 16 * i + 4 * q4;       // four consecutive columns
     float bv[4] = {0.f, 0.f, 0.f, 0.f};
-    if (EPI == 0 && g.bias != nullptr) {
+    if ((EPI == 0 || EPI == 3) && g.bias != nullptr) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) bv[r] = bf16lo_to_f32(g.bias[min(n0 + n + r, g.N - 1)]);
     }
@@ -179,7 +183,36 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
   }
   __syncthreads();
 
-  if constexpr (EPI == 0) {
+  if constexpr (EPI == 3) {
+    // The gate was a kernel of its own behind the product: 134 MB read and written once more for 32768 rows of 16 heads of 128.
+    if (gated) {
+      const KdaGates& kg = p.gates;
+      static_assert(NTHR % CHN == 0, "a thread keeps its channels");
+      const int c = tid % CHN, col = n0 + 8 * c;
+      if (col < g.N) {
+        const float scale = -expf(kg.A_log[col / kg.Dk]);
+        float bv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bv[e] = kg.dt_bias[col + e];
+        for (int m = tid / CHN; m < min(BM, p.M - m0); m += NTHR / CHN) {
+          float f[8];
+          unpack8(*reinterpret_cast<const u32x4*>(tile_at(m, c)), f);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] = scale * softplus(f[e] + bv[e], 1.f, 20.f, 1.f);
+          *reinterpret_cast<u32x4*>(g.y + (int64_t)(m0 + m) * g.y_sm + col) = pack8(f);
+        }
+      }
+      if (n0 == 0) {                         // beta of these rows
+        const int count = min(BM, p.M - m0) * kg.H;
+        for (int i = tid; i < count; i += NTHR) {
+          const float logit = bf16lo_to_f32(kg.logits[(int64_t)(m0 + i / kg.H) * kg.logits_row + i % kg.H]);
+          kg.beta[(int64_t)m0 * kg.H + i] = round_bf16(1.f / (1.f + expf(-logit)));
+        }
+      }
+      return;
+    }
+  }
+  if constexpr (EPI == 0 || EPI == 3) {
 #pragma unroll
     for (int it = 0; it < (BM * CHN + NTHR - 1) / NTHR; ++it) {
       const int idx = tid + NTHR * it, m = idx / CHN, c = idx % CHN;
@@ -344,7 +377,7 @@ int proj_linear(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn
   return dispatch_proj<0>(tile ? tile : proj_tile(M, K, 8, [&](int bn) { return (N + bn - 1) / bn; }), p, s);
 }
 
-int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, int tile) {
+int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, int tile, const KdaGates* gates) {
   DAISY_CHECK_ARG(seg && n >= 1 && n <= kMaxSegments && M > 0 && K > 0, "proj_segments: %d products, M=%d, K=%d", n, M, K);
   DAISY_CHECK_SUPPORTED(K % 64 == 0, "proj_segments: K=%d must be a multiple of 64", K);
   ProjSegmentsParams p{};
@@ -362,7 +395,12 @@ int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, in
     for (int i = 0; i < n; ++i) c += (seg[i].N + bn - 1) / bn;
     return c;
   };
-  return dispatch_proj<0>(tile ? tile : proj_tile(M, K, 8, columns), p, s);
+  if (!tile) tile = proj_tile(M, K, 8, columns);
+  if (!gates) return dispatch_proj<0>(tile, p, s);
+  DAISY_CHECK_ARG(gates->A_log && gates->dt_bias && gates->logits && gates->beta && gates->H > 0 && gates->Dk % 8 == 0 && seg[0].N == gates->H * gates->Dk,
+                  "proj_segments: gate of %d heads of %d channels on a product of %d", gates->H, gates->Dk, seg[0].N);
+  p.gates = *gates;
+  return dispatch_proj<3>(tile, p, s);
 }
 
 int proj_qkv(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const QkvEpilogue& e,
