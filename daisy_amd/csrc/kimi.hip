@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(GatedNormParams p) {
 using namespace daisy;
 
 // A thread walks its steps eight inputs at a time, so a short input, whose threads do not fill the chip, lasts as long as one
-// thread's chain of loads: threads of eight steps there (three more rows read per eight, all cached).  LINE_FIGURES
+// thread's chain of loads: threads of eight steps there (three more rows read per eight, all cached).FIG
 int daisy::short_conv_group(const ConvPart* parts, int n, int B, int T, int K, int silu, hipStream_t s) {
   DAISY_CHECK_ARG(parts && n >= 1 && n <= 3 && B > 0 && T > 0, "short_conv: %d parts, B=%d, T=%d", n, B, T);
   DAISY_CHECK_SUPPORTED(K >= 2 && K <= 4, "short_conv: kernel size %d not supported (2..4)", K);

@@ -224,64 +224,75 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
     constexpr int D = EPI == 1 ? 64 : 128, HALF = D / 2, LPR = D / 16, HPT = BN / D;
     static_assert(BN % D == 0, "a tile holds whole heads");
     const QkvEpilogue& e = p.e;
-    static_assert(BM * BN / 16 % 64 == 0, "whole wavefronts");
-    constexpr int PASSES = (BM * BN / 16 + NTHR - 1) / NTHR;
-#pragma unroll(PASSES < 4 ? PASSES : 4)
+    // A thread takes the same channels of all heads of its row where that still gives every thread a row: it then fetches the
+    // rotation (four times the bytes of the channels it turns) once.
+    constexpr int HS = BM * LPR % NTHR == 0 ? HPT : 1;
+    static_assert(BM * BN / 16 / HS % 64 == 0, "whole wavefronts");
+    constexpr int PASSES = (BM * BN / 16 / HS + NTHR - 1) / NTHR, UNROLL = 4 / HS > 0 ? 4 / HS : 1;
+#pragma unroll(PASSES < UNROLL ? PASSES : UNROLL)
     for (int it = 0; it < PASSES; ++it) {
       // LPR lanes share one (row, head): lane c holds channels [8c, 8c + 8) and their rotation partners
-      const int idx = tid + NTHR * it, c = idx % LPR, hh = (idx / LPR) % HPT, m = idx / (LPR * HPT);
-      if (BM * BN / 16 % NTHR != 0 && m >= BM) break;
-      const int n = n0 + hh * D;
-      const bool live = m0 + m < p.M && n < g.N;
+      const int idx = tid + NTHR * it, c = idx % LPR, h0 = idx / LPR % (HPT / HS) * HS, m = idx / (LPR * (HPT / HS));
+      if (BM * BN / 16 / HS % NTHR != 0 && m >= BM) break;
       const int row = min(m0 + m, p.M - 1);
-      const int third = min(n / (e.H * D), 2), h = min(n / D - third * e.H, e.H - 1);
       const int t = row % e.T, b = row / e.T;
-      float lo[8], hi[8];
-      unpack8(*reinterpret_cast<const u32x4*>(tile_at(m, hh * (D / 8) + c)), lo);
-      unpack8(*reinterpret_cast<const u32x4*>(tile_at(m, hh * (D / 8) + LPR + c)), hi);
-      // x * rsqrt(mean(x^2) + eps), rounded to bf16 like the norm's output tensor
-      float ss = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) ss += lo[i] * lo[i];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) ss += hi[i] * hi[i];
-      ss = group_sum<LPR>(ss);
-      const float rstd = rsqrtf(ss / (float)D + e.eps);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) { lo[i] = round_bf16(lo[i] * rstd); hi[i] = round_bf16(hi[i] * rstd); }
-      uint16_t* dst;
-      if (third < 2) {
+      f32x4 cs[2], sn[2];
+      if (n0 + h0 * D < 2 * e.H * D) {
         const int64_t off = (int64_t)(e.pos0 + t) * HALF + 8 * c;
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-          const f32x4 cs = *reinterpret_cast<const f32x4*>(e.cos + off + 4 * v), sn = *reinterpret_cast<const f32x4*>(e.sin + off + 4 * v);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float x1 = lo[4 * v + i], x2 = hi[4 * v + i];
-            lo[4 * v + i] = rope_lo(x1, x2, cs[i], sn[i]);
-            hi[4 * v + i] = rope_hi(x1, x2, cs[i], sn[i]);
-          }
+          cs[v] = *reinterpret_cast<const f32x4*>(e.cos + off + 4 * v);
+          sn[v] = *reinterpret_cast<const f32x4*>(e.sin + off + 4 * v);
         }
-        dst = third == 0 ? e.q + b * e.q_sb + t * e.q_st + h * e.q_sh : e.k + b * e.k_sb + t * e.k_st + h * e.k_sh;
-      } else {
-        if (e.ve != nullptr) {
-          // g*v + (1-g)*ve with every product, the difference and the sum rounded to bf16
-          const float gv = gate_value(e.gate), og = round_bf16(1.0f - gv);
-          const uint16_t* vp = e.ve + b * e.ve_sb + t * e.ve_st + h * e.ve_sh + 8 * c;
-          float el[8], eh[8];
-          unpack8(*reinterpret_cast<const u32x4*>(vp), el);
-          unpack8(*reinterpret_cast<const u32x4*>(vp + HALF), eh);
+      }
+#pragma unroll
+      for (int j = 0; j < HS; ++j) {
+        const int hh = h0 + j;
+        const int n = n0 + hh * D;
+        const bool live = m0 + m < p.M && n < g.N;
+        const int third = min(n / (e.H * D), 2), h = min(n / D - third * e.H, e.H - 1);
+        float lo[8], hi[8];
+        unpack8(*reinterpret_cast<const u32x4*>(tile_at(m, hh * (D / 8) + c)), lo);
+        unpack8(*reinterpret_cast<const u32x4*>(tile_at(m, hh * (D / 8) + LPR + c)), hi);
+        // x * rsqrt(mean(x^2) + eps), rounded to bf16 like the norm's output tensor
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += lo[i] * lo[i];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss += hi[i] * hi[i];
+        ss = group_sum<LPR>(ss);
+        const float rstd = rsqrtf(ss / (float)D + e.eps);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) { lo[i] = round_bf16(lo[i] * rstd); hi[i] = round_bf16(hi[i] * rstd); }
+        uint16_t* dst;
+        if (third < 2) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            lo[i] = round_bf16(gv * lo[i]) + round_bf16(og * el[i]);
-            hi[i] = round_bf16(gv * hi[i]) + round_bf16(og * eh[i]);
+            const float x1 = lo[i], x2 = hi[i];
+            lo[i] = rope_lo(x1, x2, cs[i / 4][i % 4], sn[i / 4][i % 4]);
+            hi[i] = rope_hi(x1, x2, cs[i / 4][i % 4], sn[i / 4][i % 4]);
           }
+          dst = third == 0 ? e.q + b * e.q_sb + t * e.q_st + h * e.q_sh : e.k + b * e.k_sb + t * e.k_st + h * e.k_sh;
+        } else {
+          if (e.ve != nullptr) {
+            // g*v + (1-g)*ve with every product, the difference and the sum rounded to bf16
+            const float gv = gate_value(e.gate), og = round_bf16(1.0f - gv);
+            const uint16_t* vp = e.ve + b * e.ve_sb + t * e.ve_st + h * e.ve_sh + 8 * c;
+            float el[8], eh[8];
+            unpack8(*reinterpret_cast<const u32x4*>(vp), el);
+            unpack8(*reinterpret_cast<const u32x4*>(vp + HALF), eh);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              lo[i] = round_bf16(gv * lo[i]) + round_bf16(og * el[i]);
+              hi[i] = round_bf16(gv * hi[i]) + round_bf16(og * eh[i]);
+            }
+          }
+          dst = e.v + b * e.v_sb + t * e.v_st + h * e.v_sh;
         }
-        dst = e.v + b * e.v_sb + t * e.v_st + h * e.v_sh;
-      }
-      if (live) {
-        *reinterpret_cast<u32x4*>(dst + 8 * c) = pack8(lo);
-        *reinterpret_cast<u32x4*>(dst + 8 * c + HALF) = pack8(hi);
+        if (live) {
+          *reinterpret_cast<u32x4*>(dst + 8 * c) = pack8(lo);
+          *reinterpret_cast<u32x4*>(dst + 8 * c + HALF) = pack8(hi);
+        }
       }
     }
   }
@@ -400,6 +411,8 @@ int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, in
   DAISY_CHECK_ARG(gates->A_log && gates->dt_bias && gates->logits && gates->beta && gates->H > 0 && gates->Dk % 8 == 0 && seg[0].N == gates->H * gates->Dk,
                   "proj_segments: gate of %d heads of %d channels on a product of %d", gates->H, gates->Dk, seg[0].N);
   p.gates = *gates;
+  // (two workgroups to a compute unit: the gate of one runs beside the copies of the other; 32768 rows, whole layer: 1674 against 1680 us)
+  if (tile == 7) tile = 6;
   return dispatch_proj<3>(tile, p, s);
 }
 
