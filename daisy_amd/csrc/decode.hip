@@ -498,6 +498,120 @@ __global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(DecodeP
   p.o[b * p.o_sb + h * p.o_sh + d] = (uint16_t)(pack_bf16x2(r, 0.f) & 0xffffu);
 }
 
+// The combine of one sequence's splits and the projection of the row it gives, y [N] = o [H D] w^T, in one launch: with one
+// sequence both kernels are a memory round trip each, and so is the gap between them.  Every workgroup combines the whole row o
+// into LDS (a thread four channels), and each of its wavefronts multiplies it with one weight row.  What bounds it is what a
+// compute unit pulls out of the L2 (98 KB of partials for 12 heads of 128 and 16 splits), so all of a thread's partials and its
+// pieces of the weight row are requested first, and the splits' weights are worked out meanwhile, once per workgroup
+// (a first version, every thread on its own, took 1.5 us longer).  Sums in the order of decode_combine_kernel and
+// linear_rows_kernel: the results are the same bits.
+// 12 heads of 128, ring of 8192: one layer's step launched eagerly 22.6 to 24.9 -> 21.4 us; twelve of them in a recorded step
+// 381.3 -> 381.0 us (6.1 us for this kernel where the two took 2.5 and 3.3 and a gap: a graph's nodes follow each other closely).
+struct CombineProjectParams {
+  const float* partials;     // [H, nsplit, D + 2]
+  int HD, nsplit;
+  StepProjection out;
+};
+constexpr int kProjectThreads = 512;
+constexpr int kProjectRows = kProjectThreads / 64;
+constexpr int kProjectChannels = 4 * kProjectThreads;      // H D at most
+constexpr int kProjectSplits = 32;                         // and H nsplit at most kProjectThreads
+// G groups of up to eight splits, as decode_combine_kernel forms them: split s belongs to group s % G.
+template <int D, int G>
+__global__ __launch_bounds__(kProjectThreads) void decode_combine_project_kernel(CombineProjectParams p) {
+  constexpr int S = 8 * G, PIECES = kProjectChannels / 8 / 64;
+  __shared__ __attribute__((aligned(16))) uint32_t row[kProjectChannels / 2];
+  __shared__ f32x2 ml[kProjectThreads];                 // [H][nsplit] maximum and sum of a split
+  __shared__ float ws[kProjectChannels / D * S];        // [H][S] weight of a split in its group (0: no such split)
+  __shared__ float wg[kProjectChannels / D * (G + 1)];  // [H][G + 1] weight of a group; the sum
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int H = p.HD / D, ns = p.nsplit, pieces = p.HD / 8;
+  const f32x2 my_ml = *reinterpret_cast<const f32x2*>(p.partials + (int64_t)min(tid, H * ns - 1) * (D + 2));
+  const int c = min(4 * tid, p.HD - 4), h = c / D;      // (threads past the end redo the last channels)
+  const float* part = p.partials + (int64_t)h * ns * (D + 2) + 2 + c % D;
+  f32x2 as[S][2];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const float* at = part + min(s, ns - 1) * (D + 2);  // 8-byte aligned
+    as[s][0] = *reinterpret_cast<const f32x2*>(at);
+    as[s][1] = *reinterpret_cast<const f32x2*>(at + 2);
+  }
+  const int n = blockIdx.x * kProjectRows + wave;
+  const uint16_t* wr = p.out.w + (int64_t)min(n, p.out.N - 1) * p.out.w_sn;
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  u32x4 wv[PIECES];
+#pragma unroll
+  for (int j = 0; j < PIECES; ++j) wv[j] = lane + 64 * j < pieces ? *reinterpret_cast<const u32x4*>(wr + 8 * (lane + 64 * j)) : zero;
+  __builtin_amdgcn_sched_barrier(0);
+
+  // The barriers wait for LDS only: the loads stay in flight.
+  auto publish = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  if (tid < H * ns) ml[tid] = my_ml;
+  publish();
+  for (int i = tid; i < H * S; i += kProjectThreads) {
+    const int hh = i / S, s = i % S, g = s % G;
+    float m = -INFINITY;
+    for (int u = g; u < ns; u += G) m = fmaxf(m, ml[hh * ns + u][0]);
+    const float mu = (m == -INFINITY) ? 0.f : m;
+    ws[i] = s < ns ? fast_exp2(ml[hh * ns + s][0] - mu) : 0.f;
+    if (s < G) {
+      float mt = m;
+      for (int u = 0; u < ns; ++u) mt = fmaxf(mt, ml[hh * ns + u][0]);
+      const float mut = (mt == -INFINITY) ? 0.f : mt;
+      wg[hh * (G + 1) + s] = fast_exp2(m - mut);
+    }
+  }
+  publish();
+  if (tid < H) {
+    float lt = 0.f;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float l = 0.f;
+      for (int u = g; u < ns; u += G) l = fmaf(ml[tid * ns + u][1], ws[tid * S + u], l);
+      lt = G > 1 ? fmaf(l, wg[tid * (G + 1) + g], lt) : l;
+    }
+    wg[tid * (G + 1) + G] = lt;
+  }
+  publish();
+
+  float t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int s = g + u * G;
+      const float w = ws[h * S + s];
+      if (s < ns) {          // (an infinite value of the last split must not meet a weight of 0)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = fmaf(as[s][e / 2][e % 2], w, a[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = G > 1 ? fmaf(a[e], wg[h * (G + 1) + g], t[e]) : a[e];
+  }
+  const float lt = wg[h * (G + 1) + G];
+  if (4 * tid < p.HD) *reinterpret_cast<u32x2*>(&row[2 * tid]) = u32x2{pack_bf16x2(t[0] / lt, t[1] / lt), pack_bf16x2(t[2] / lt, t[3] / lt)};
+  publish();
+  float acc = 0.f;
+#pragma unroll
+  for (int j = 0; j < PIECES; ++j) {
+    const u32x4 xv = lane + 64 * j < pieces ? *reinterpret_cast<const u32x4*>(&row[4 * (lane + 64 * j)]) : zero;
+    float xf[8], wf[8];
+    unpack8(xv, xf);
+    unpack8(wv[j], wf);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc = fmaf(wf[i], xf[i], acc);
+  }
+  acc = group_sum<32>(acc);
+  acc += __shfl_xor(acc, 32);
+  if (lane == 0 && n < p.out.N) p.out.y[n] = (uint16_t)(pack_bf16x2(acc, 0.f) & 0xffffu);
+}
+
 static int choose_nsplit(int B, int H, int n_rows) {
   // About 512 rows per workgroup (two full iterations of every wavefront and some), as long as that does not make
   // more than about 1024 workgroups; when it leaves fewer than 192 workgroups on the 256 compute units (a few
@@ -525,6 +639,25 @@ static int resolve_nsplit(int B, int H, int n_rows, int nsplit) {
   const int rps = (n_rows + nsplit - 1) / nsplit;
   // Drop splits that would be empty after rounding rows_per_split up.
   return (n_rows + rps - 1) / rps;
+}
+
+bool step_projects(int B, int H, int D, int n_rows) {
+  if (B != 1 || (D != 64 && D != 128) || H * D > kProjectChannels) return false;
+  const int ns = resolve_nsplit(B, H, n_rows, 0);
+  return ns > 1 && ns <= kProjectSplits && H * ns <= kProjectThreads;
+}
+template <int D, int G>
+static void launch_combine_project(const DecodeParams& p, const StepProjection& out, hipStream_t s) {
+  hipLaunchKernelGGL((decode_combine_project_kernel<D, G>), dim3((out.N + kProjectRows - 1) / kProjectRows), dim3(kProjectThreads), 0, s,
+                     CombineProjectParams{p.partials, p.H * D, p.nsplit, out});
+}
+template <int D>
+static void launch_combine_project(const DecodeParams& p, const StepProjection& out, hipStream_t s) {
+  const int groups = (p.nsplit + 7) / 8;
+  if (groups == 1) launch_combine_project<D, 1>(p, out, s);
+  else if (groups == 2) launch_combine_project<D, 2>(p, out, s);
+  else if (groups == 3) launch_combine_project<D, 3>(p, out, s);
+  else launch_combine_project<D, 4>(p, out, s);
 }
 
 // Any even head dim up to 256 (the reference's unit tests use 2 and 8): one wavefront per
@@ -688,6 +821,10 @@ int decode_launch(const void* q, const int64_t* q_strides,
     p.partials = (float*)workspace;
   }
 
+  const bool projects = prep != nullptr && prep->out.w != nullptr;
+  DAISY_CHECK_ARG(!projects || (nsplit == 0 && step_projects(B, H, D, n_rows) && prep->out.y && prep->out.N > 0 && prep->out.w_sn % 8 == 0 &&
+                                al16(prep->out.w) && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0),
+                  "decode: a projection of one sequence's split row only, weights on 16-byte boundaries");
   hipStream_t s = (hipStream_t)stream;
   if (!fast) {
     if (f32_io) hipLaunchKernelGGL(decode_scalar_kernel<float>, dim3(H, B), dim3(64), 0, s, p, D);
@@ -701,7 +838,10 @@ int decode_launch(const void* q, const int64_t* q_strides,
     else if (prep) hipLaunchKernelGGL((decode_kernel<128, true>), grid, dim3(kDecodeThreads), 0, s, p);
     else hipLaunchKernelGGL((decode_kernel<128, false>), grid, dim3(kDecodeThreads), 0, s, p);
     DAISY_CHECK_LAUNCH("decode_kernel");
-    if (p.nsplit > 1) {
+    if (projects) {
+      launch_combine_project<128>(p, prep->out, s);
+      DAISY_CHECK_LAUNCH("decode_combine_project_kernel");
+    } else if (p.nsplit > 1) {
       hipLaunchKernelGGL(decode_combine_kernel<128>, dim3(H, B), dim3(combine_threads(128, p.nsplit)), 0, s, p);
       DAISY_CHECK_LAUNCH("decode_combine_kernel");
     }
@@ -710,7 +850,10 @@ int decode_launch(const void* q, const int64_t* q_strides,
     else if (prep) hipLaunchKernelGGL((decode_kernel<64, true>), grid, dim3(kDecodeThreads), 0, s, p);
     else hipLaunchKernelGGL((decode_kernel<64, false>), grid, dim3(kDecodeThreads), 0, s, p);
     DAISY_CHECK_LAUNCH("decode_kernel");
-    if (p.nsplit > 1) {
+    if (projects) {
+      launch_combine_project<64>(p, prep->out, s);
+      DAISY_CHECK_LAUNCH("decode_combine_project_kernel");
+    } else if (p.nsplit > 1) {
       hipLaunchKernelGGL(decode_combine_kernel<64>, dim3(H, B), dim3(combine_threads(64, p.nsplit)), 0, s, p);
       DAISY_CHECK_LAUNCH("decode_combine_kernel");
     }

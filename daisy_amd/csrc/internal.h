@@ -67,11 +67,16 @@ int proj_qkv(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, c
 // What a one-launch attention step adds to a decode launch: the kernel prepares the rows of the projection itself.
 // k_rows / v_rows: NULL, or bf16 [B, H, D] contiguous copies of the new rows as the ring holds them (an fp16 ring's
 // rows in the model's dtype, without another pass over them).
+// out: a product y [N] = o [H * D] w [N, H * D]^T that takes the attention's place in memory (o is then not written), for the calls that
+// step_projects says it serves: one sequence whose ring is split.
+struct StepProjection { const uint16_t* w; int64_t w_sn; uint16_t* y; int N; };
+bool step_projects(int B, int H, int D, int n_rows);
 struct StepPrep {
   int pos_host; const float* cos; const float* sin; int table_rows; float eps;
   const void* ve; const int64_t* ve_strides; GateSource gate;
   int cache_f16; int32_t* status;
   uint16_t* k_rows; uint16_t* v_rows;
+  StepProjection out = {nullptr, 0, nullptr, 0};
 };
 int decode_launch(const void* q, const int64_t* q_strides,
                   const void* k_new, const int64_t* k_new_strides,

@@ -394,7 +394,7 @@ PyObject* py_layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   } else {
     qkv = at::linear(x, w.narrow(0, 0, 3).view({3 * dim, dim}));
   }
-  Tensor o = empty({B, 1, dim}, at::kBFloat16, x), k_new, v_new;
+  Tensor o, y, k_new, v_new;
   if (f16 && !pos_dev) {
     k_new = empty({B, 1, H, D}, at::kBFloat16, x);
     v_new = empty({B, 1, H, D}, at::kBFloat16, x);
@@ -404,22 +404,28 @@ PyObject* py_layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor ws;
   if (need) ws = empty({(int64_t)need}, at::kByte, x);
   const uint16_t* base = (const uint16_t*)ptr(qkv);
+  const uint16_t* wo = wp + 3 * dim * dim;
+  // one sequence with a split ring: the output projection combines the splits itself, and no attention row is written
+  const bool projects = max_rows > 0 && daisy::step_projects((int)B, (int)H, (int)D, live);
+  if (projects) y = empty({B, 1, dim}, at::kBFloat16, x);
+  else o = empty({B, 1, dim}, at::kBFloat16, x);
   const int64_t rs[2] = {3 * dim, D}, os[2] = {dim, D};
   const Strides3 krs(kr), vrs(vr);
   const daisy::StepPrep prep{pos, (const float*)ptr(cos), (const float*)ptr(sin), (int)cos.size(0), eps, ptr(ve), os, gate, f16,
                              (int32_t*)ptr(status), k_new.defined() ? (uint16_t*)ptr(k_new) : nullptr,
-                             v_new.defined() ? (uint16_t*)ptr(v_new) : nullptr};
-  if (daisy::attn_step_launch(base, rs, base + dim, rs, base + 2 * dim, rs, ptr(kr), krs.s, ptr(vr), vrs.s, ptr(o), os, (int)B, (int)H,
+                             v_new.defined() ? (uint16_t*)ptr(v_new) : nullptr,
+                             projects ? daisy::StepProjection{wo, dim, (uint16_t*)ptr(y), (int)dim} : daisy::StepProjection{nullptr, 0, nullptr, 0}};
+  if (daisy::attn_step_launch(base, rs, base + dim, rs, base + 2 * dim, rs, ptr(kr), krs.s, ptr(vr), vrs.s, projects ? ptr(qkv) : ptr(o), os, (int)B, (int)H,
                               (int)D, (int)W, pos_dev ? (const int32_t*)ptr(*pos_dev) : nullptr, scale, 0, need ? ptr(ws) : nullptr, need, s,
                               prep) != DAISY_OK) return none();
-  const Rows orow{(const uint16_t*)ptr(o), dim, (int)B, (int)dim};
-  const uint16_t* wo = wp + 3 * dim * dim;
-  Tensor y;
-  if (max_rows > 0 && (B <= max_rows || daisy::proj_wanted((int)B, (int)dim, (int)dim))) {
-    y = empty({B, 1, dim}, at::kBFloat16, x);
-    if (!own_linear(orow, wo, dim, (int)dim, nullptr, (uint16_t*)ptr(y), dim, max_rows, s)) return none();
-  } else {
-    y = at::linear(o, w.select(0, 3));
+  if (!projects) {
+    const Rows orow{(const uint16_t*)ptr(o), dim, (int)B, (int)dim};
+    if (max_rows > 0 && (B <= max_rows || daisy::proj_wanted((int)B, (int)dim, (int)dim))) {
+      y = empty({B, 1, dim}, at::kBFloat16, x);
+      if (!own_linear(orow, wo, dim, (int)dim, nullptr, (uint16_t*)ptr(y), dim, max_rows, s)) return none();
+    } else {
+      y = at::linear(o, w.select(0, 3));
+    }
   }
   unlocked.end();
   PyObject* res = PyTuple_New(3);

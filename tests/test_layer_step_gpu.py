@@ -69,3 +69,18 @@ def test_layer_step_refusals():
         int(cos.shape[0]), 3, None, None, 1e-6, kr.data_ptr(), _lib.strides(kr, (0, 1, 2)), vr.data_ptr(),
         _lib.strides(vr, (0, 1, 2)), 0, x.data_ptr(), 128, 2, 2, 64, 128, 16, 0.12, 0, small.data_ptr(), 256, None)
     assert rc != 0 and "workspace" in lib.daisy_last_error().decode()
+
+
+# splits of the ring (groups of eight) x channel pairs per thread of the kernel that combines and projects, live rows that leave splits empty
+@pytest.mark.parametrize("H,D,W,t,on_device", [(12, 128, 8192, 8292, False), (16, 128, 8192, 8292, True), (12, 128, 1024, 700, False),
+                                               (8, 128, 8192, 9000, True), (6, 128, 8192, 9000, False), (12, 64, 8192, 300, True),
+                                               (3, 64, 600, 599, False), (31, 64, 8192, 9001, True), (16, 128, 300, 299, True)])
+@pytest.mark.parametrize("ring_dtype", [torch.bfloat16, torch.float16])
+def test_projection_that_combines_the_splits_equals_the_two_kernels(H, D, W, t, on_device, ring_dtype):
+    x, w, kr, vr, _, _, cos, sin = _setup(1, H, D, W, seed=H, ring_dtype=ring_dtype)
+    pos = torch.tensor([t], dtype=torch.int32, device="cuda") if on_device else t
+    k1, v1, k2, v2 = kr.clone(), vr.clone(), kr.clone(), vr.clone()
+    ref = ops.attn_layer_step(x, w[:3].flatten(end_dim=1), w[3], k1, v1, pos, cos=cos, sin=sin, eps=NORM_EPS_BF16, scale=0.12)
+    with torch.no_grad():
+        y = _lib.native().layer_step(x, w, k2, v2, pos, cos, sin, None, None, None, 0.12, NORM_EPS_BF16, 4)[0]
+    assert torch.equal(y, ref) and torch.equal(k1, k2) and torch.equal(v1, v2)
