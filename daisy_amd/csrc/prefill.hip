@@ -48,6 +48,8 @@ struct PrefillParams {
   int B, T, H, D, window, nqb;
   int period;    // 32-key tiles in a full window's range (0 = no window): the rotation period of the tile order
   int n_light;   // leading query blocks that see fewer keys than a full window (0 = order by block only)
+  int order_shift;   // documents: query blocks in the order of their lengths, in units of 2^order_shift tiles; -1: by block
+  int order_bit;     // the highest bit of such a length
   float scale_log2e;
 };
 
@@ -60,18 +62,79 @@ __device__ __forceinline__ int row_lo(const PrefillParams& p, int q) {
   return lo;
 }
 
+// With documents the length of a block depends on where its document starts, which only the device knows: item `idx` of a group of
+// gsize (batch, head) pairs in the order of decreasing length, pair by pair from the last block down within a length.  Block by
+// block from the end, the last workgroups of the grid were those of the first two documents, of any length (T = 20001, 16 heads
+// of 64, window 4096, seven documents: 183 -> 161 us; T = 65536, 4 heads of 64, five documents: 520 -> 453 us).  One wavefront works it out: it holds the lengths of up to 512 blocks, and counts
+// with ballots; any lengths give every block once.
+constexpr int kOrderChunks = 8;
+__device__ __forceinline__ void block_by_length(const PrefillParams& p, int gsize, int idx, int& local, int& qb, int& lo) {
+  const int lane = threadIdx.x & 63;
+  int len[kOrderChunks];     // 0..2 order_bit - 1, -1 past the last block
+  int first[kOrderChunks];   // the first key of a block
+#pragma unroll
+  for (int c = 0; c < kOrderChunks; ++c) {
+    len[c] = -1;
+    if (64 * c < p.nqb) {
+      const int i = 64 * c + lane, q0 = min(i, p.nqb - 1) * kBM;
+      first[c] = row_lo(p, q0);
+      const int n = min(q0 + kBM - 1, p.T - 1) / 32 - first[c] / 32 + 1;
+      if (i < p.nqb) len[c] = min(max(n, 0) >> p.order_shift, 2 * p.order_bit - 1);
+    }
+  }
+  auto at_least = [&](int v) {
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < kOrderChunks; ++c)
+      if (64 * c < p.nqb) n += __popcll(__ballot(len[c] >= v));
+    return n;
+  };
+  int v = 0;                 // the largest length with more than idx items at least as long
+  for (int bit = p.order_bit; bit > 0; bit >>= 1)
+    if (gsize * at_least(v + bit) > idx) v += bit;
+  const int above = at_least(v + 1), here = at_least(v) - above, k = idx - gsize * above;
+  local = k / here;
+  int j = here - 1 - k % here;      // which of the blocks of this length, counted from the first
+  qb = lo = 0;
+#pragma unroll
+  for (int c = 0; c < kOrderChunks; ++c) {
+    if (64 * c >= p.nqb) break;
+    const uint64_t same = __ballot(len[c] == v);
+    const int n = __popcll(same);
+    if (j >= 0 && j < n) {
+      const bool mine = (same >> lane & 1) != 0 && __popcll(same & ((1ull << lane) - 1)) == j;
+      const int at = __ffsll((unsigned long long)__ballot(mine)) - 1;
+      qb = 64 * c + at;
+      lo = __builtin_amdgcn_readlane(first[c], at);
+    }
+    j -= n;
+  }
+  local = __builtin_amdgcn_readfirstlane(local);
+  qb = __builtin_amdgcn_readfirstlane(qb);
+  lo = __builtin_amdgcn_readfirstlane(lo);
+}
+
 // Workgroup -> (batch*head, query block).  Workgroups are dealt round-robin to the 8 XCDs, each
 // with its own L2: an XCD is given a contiguous group of (batch, head) pairs so that the query
 // blocks sharing K/V rows share an L2.  Inside a group the blocks with a full window of keys
 // come first, pair by pair from the last block down; the n_light shorter blocks at the start of
 // every sequence come last, longest first across the whole group, and fill the tail of the grid.
-__device__ __forceinline__ void workgroup_to_block(const PrefillParams& p, int& bh, int& qb) {
+__device__ __forceinline__ void workgroup_to_block(const PrefillParams& p, int* found, int& bh, int& qb, int& lo) {
   const int nbh = p.B * p.H;
   int group = 0, gsize = nbh, idx = blockIdx.x;
   if ((nbh & 7) == 0) { group = blockIdx.x & 7; gsize = nbh >> 3; idx = blockIdx.x >> 3; }
   const int n_full = p.nqb - p.n_light;
   int local;
-  if (idx < gsize * n_full) {
+  if (p.order_shift >= 0) {
+    if (threadIdx.x < 64) {      // (a load per block touches a cache line each: one wavefront's are enough)
+      block_by_length(p, gsize, idx, local, qb, lo);
+      if (threadIdx.x == 0) { found[0] = local; found[1] = qb; found[2] = lo; }
+    }
+    __syncthreads();
+    local = __builtin_amdgcn_readfirstlane(found[0]);
+    qb = __builtin_amdgcn_readfirstlane(found[1]);
+    lo = __builtin_amdgcn_readfirstlane(found[2]);
+  } else if (idx < gsize * n_full) {
     local = idx / n_full;
     qb = p.nqb - 1 - idx % n_full;
   } else {
@@ -79,6 +142,7 @@ __device__ __forceinline__ void workgroup_to_block(const PrefillParams& p, int& 
     qb = p.n_light - 1 - j / gsize;
     local = j % gsize;
   }
+  if (p.order_shift < 0) lo = row_lo(p, qb * kBM);
   bh = group * gsize + local;
 }
 
@@ -132,8 +196,9 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane & 31, lh = lane >> 5;
 
-  int bh, qb;
-  workgroup_to_block(p, bh, qb);
+  int bh, qb, lo_first;
+  __shared__ int found[3];
+  workgroup_to_block(p, found, bh, qb, lo_first);
   const int h = bh % p.H, b = bh / p.H;
 
   const int q0 = qb * kBM;
@@ -150,7 +215,7 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   // online softmax does not care about the order, and the query blocks of one (batch, head)
   // that run side by side then read the same K/V tile at the same step, so one fetch into the
   // L2 serves all of them.  With no window every range starts at tile 0 and nothing is rotated.
-  const int t_lo = row_lo(p, q0) / kTBN;
+  const int t_lo = lo_first / kTBN;
   const int t_hi = min(q0 + kBM - 1, p.T - 1) / kTBN;
   const int n_tiles = t_hi - t_lo + 1;
   int t_first = t_lo;
@@ -843,6 +908,15 @@ static int fill_prefill_params(PrefillParams& p, const void* q, const int64_t* q
   p.nqb = (T + kBM - 1) / kBM;
   p.period = (window > 0 && window < T) ? (kBM - 1) / kTBN + 1 + (window - 1 + kTBN - 1) / kTBN : 0;
   p.n_light = (window > 0 && window < T) ? min((window - 1 + kBM - 1) / kBM, p.nqb) : 0;
+  p.order_shift = -1; p.order_bit = 0;
+  // Finding the order costs a workgroup about 1 us; the lengths differ enough to pay for it where a window is an eighth of the
+  // row or more (three documents of T = 16384, window 2048: 197 -> 182 us; a mask with a lone document, which
+  // gains nothing, 162.5 -> 165.4 us; at a sixteenth a lone document costs 148 against 146 us, nine of them take 258 against 270 us).
+  if (doc_start != nullptr && p.nqb <= 64 * kOrderChunks && (window <= 0 || (int64_t)window * 8 >= T)) {
+    int longest = (window > 0 && window < T ? window : T) / 32 + 6;     // tiles of a block
+    for (p.order_shift = 0; longest > 255; longest >>= 1) ++p.order_shift;
+    for (p.order_bit = 1; 2 * p.order_bit <= longest; p.order_bit *= 2) {}
+  }
   p.scale_log2e = scale * kLog2e;
   return DAISY_OK;
 }

@@ -140,3 +140,20 @@ def test_prefill_rejects_bad_arguments():
         ops.prefill_attention(q.float(), q.float(), q.float(), window=4)
     with pytest.raises(RuntimeError, match="no CPU path"):
         ops.prefill_attention(q.cpu(), q.cpu(), q.cpu(), window=4)
+
+
+# Documents change the order in which the blocks of 128 queries are worked on: every block once, whatever the lengths.  Rows of more
+# blocks than the order covers, (batch, head) pairs that do and do not divide among the XCDs, documents of one token, one document.
+@pytest.mark.parametrize("B,T,H,D,W,starts", [(1, 8300, 8, 64, 1024, (0, 1, 700, 4000, 4128, 8299)), (1, 8300, 3, 128, None, (0, 2500, 2501, 6000)),
+                                              (2, 3333, 16, 64, 256, (0,)), (1, 65537, 2, 64, 128, (0, 31000)), (1, 65536, 2, 64, 128, (0, 31000)),
+                                              (1, 5000, 5, 128, 300, tuple(range(0, 5000, 61)))])
+def test_documents_equal_their_own_calls(B, T, H, D, W, starts):
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    q, k, v = (torch.randn(B, T, H, D, generator=g, device="cuda").bfloat16() for _ in range(3))
+    bounds = list(starts) + [T]
+    doc = torch.cat([torch.full((b - a,), a, dtype=torch.int32, device="cuda") for a, b in zip(bounds, bounds[1:])])
+    o, _ = ops.prefill_attention(q, k, v, window=W, doc_start=doc)
+    for a, b in zip(bounds, bounds[1:]):
+        ref, _ = ops.prefill_attention(q[:, a:b], k[:, a:b], v[:, a:b], window=W)
+        # two bf16 roundings of the same sums over other tiles of keys, with bf16 probabilities
+        assert ((o[:, a:b].float() - ref.float()).norm() / ref.float().norm()).item() < 1e-2
