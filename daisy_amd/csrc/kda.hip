@@ -84,7 +84,8 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 // operands are stored with their contraction index permuted inside every aligned group of 32 (perm32) so that those 8
 // indices are 8 consecutive elements, one 16-byte load.
 //
-// What bounds it.  The first kernel moves bytes, with the conversions in between: 1.0 GB in 217 us at B4 T8192 H16 (4.7 TB/s);
+// What bounds it.  The first kernel moves bytes, with the conversions in between: 1.29 GB (673 MB of inputs, 612 MB of blocks)
+// in 217 us at B4 T8192 H16 (5.9 TB/s);
 // with chunks of 64 and W = T K, U0 = T V in the workspace (107 KB per 64 positions, from a solve with 256 right-hand
 // sides) it took 355 us.  The second kernel is a serial chain of chunks, bound by the latency of a link: folding T into
 // the two matrices above takes a product and a conversion out of it, and chunks of 32 let three stages of everything the

@@ -279,7 +279,8 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(GatedNormParams p) {
 using namespace daisy;
 
 // A thread walks its steps eight inputs at a time, so a short input, whose threads do not fill the chip, lasts as long as one
-// thread's chain of loads: threads of eight steps there (three more rows read per eight, all cached).FIG
+// thread's chain of loads: threads of eight steps there (three more rows read per eight, all cached).  The KDA layer over 64 rows
+// of 8 heads of 128: 50.5 -> 46.3 us, 300 rows of 12: 65 -> 59.5, 2048 rows of 16: 210.5 -> 208.3; level from a workgroup per compute unit on.
 int daisy::short_conv_group(const ConvPart* parts, int n, int B, int T, int K, int silu, hipStream_t s) {
   DAISY_CHECK_ARG(parts && n >= 1 && n <= 3 && B > 0 && T > 0, "short_conv: %d parts, B=%d, T=%d", n, B, T);
   DAISY_CHECK_SUPPORTED(K >= 2 && K <= 4, "short_conv: kernel size %d not supported (2..4)", K);
