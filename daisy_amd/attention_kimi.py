@@ -236,7 +236,7 @@ class KimiLinearSelfAttention(nn.Module):
             lins = (m["q_proj"], m["k_proj"], m["v_proj"], m["f_proj"]._modules["0"], m["g_proj"]._modules["0"], m["b_proj"],
                     m["f_proj"]._modules["1"], m["o_proj"])
             g1, convs, norm = m["g_proj"]._modules["1"], (m["q_conv1d"], m["k_conv1d"], m["v_conv1d"]), m["o_norm"]
-            if not (_plain(g1, nn.Linear) and _plain(norm, GatedRMSNorm) and all([_plain(c, ShortConvolution) for c in convs])
+            if not (not nn.modules.module._has_any_global_hook() and _plain(g1, nn.Linear) and _plain(norm, GatedRMSNorm) and all([_plain(c, ShortConvolution) for c in convs])
                     and all([l._parameters["bias"] is None for l in lins])):
                 return None
             w = [l._parameters["weight"] for l in lins]

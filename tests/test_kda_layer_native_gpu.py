@@ -73,3 +73,17 @@ def test_products_in_one_launch_equal_separate_ones(M, K, Ns):
         for y, w, b in zip(ys, ws, bs):
             ref = x.float() @ w.float().T + (b.float() if b is not None else 0.0)
             assert ((y.float() - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-3 * K ** 0.5).all(), tile
+
+
+def test_hooks_on_what_the_layer_calls_are_called():
+    m = _layer(4, 64, 1.0, 4, False)
+    x = torch.randn(2, 5, 256, device=DEV).bfloat16()
+    seen = []
+    with torch.no_grad():
+        assert m._fast(x, False) is not None
+        for add in (m.o_norm.register_forward_hook, m.g_proj[1].register_forward_pre_hook, torch.nn.modules.module.register_module_forward_hook):
+            handle = add(lambda *a: seen.append(type(a[0])))
+            m(x, None)
+            handle.remove()
+            assert {"GatedRMSNorm", "Linear"} & {t.__name__ for t in seen}
+            seen.clear()
