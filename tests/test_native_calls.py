@@ -1,0 +1,72 @@
+"""What the modules hand to the one-call path (``daisy_amd/_native.so``) and which calls it serves."""
+import pytest
+import torch
+
+from daisy_amd import CausalSelfAttention, KVCache, WindowMask, _lib
+
+
+class _Recorder:
+    """Stands in for the extension: keeps the arguments and answers like it."""
+
+    def __init__(self, answer):
+        self.answer, self.args = answer, None
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.name, self.args = name, args
+            return self.answer
+        return call
+
+
+def _attn(dim=128, H=2, D=64, ve=True, **kw):
+    torch.manual_seed(0)
+    return CausalSelfAttention(dim, H, D, receives_ve=ve, layer_idx=0, max_seq_len=64, **kw).eval()
+
+
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("ve_dtype", [None, torch.float32, torch.bfloat16])
+def test_activations_reach_the_one_call_path_in_the_weights_dtype(x_dtype, ve_dtype, monkeypatch):
+    attn = _attn(ve=ve_dtype is not None)
+    x = torch.randn(1, 5, 128).to(x_dtype)
+    ve = None if ve_dtype is None else torch.randn(1, 5, 128).to(ve_dtype)
+    kv = torch.zeros(1, 5, 2, 64)
+    ext = _Recorder((x, None, kv, kv))
+    monkeypatch.setattr(_lib, "native", lambda: ext)
+    attn.prefill(x, ve, attn_mask=WindowMask(4))
+    assert ext.name == "layer_prefill" and ext.args[0].dtype == torch.bfloat16 and torch.equal(ext.args[0], x.bfloat16())
+    got_ve = ext.args[8]
+    assert got_ve is None if ve is None else got_ve.dtype == torch.bfloat16 and torch.equal(got_ve, ve.bfloat16())
+    cache = KVCache(L=1, B=1, H=2, W=8, D=64, device="cpu", dtype=torch.bfloat16)
+    ext.answer = (x, None, None)
+    one = None if ve is None else ve[:, :1]
+    attn.step(x[:, :1], cache.ring(0), cache.ring(0), 0, one, 8)
+    assert ext.name == "layer_step" and ext.args[0].dtype == torch.bfloat16
+    assert ext.args[7] is None if ve is None else ext.args[7].dtype == torch.bfloat16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ve", [False, True])
+def test_fp32_activations_equal_the_bf16_ones_they_round_to(ve, monkeypatch):
+    attn = _attn(ve=ve).to("cuda:0")
+    with torch.no_grad():
+        attn.qkvo_w.normal_(std=0.05)
+    g = torch.Generator(device="cuda:0").manual_seed(1)
+    x, vals = (torch.randn(2, 33, 128, generator=g, device="cuda:0") for _ in range(2))
+    served = []
+
+    class Spy:
+        def __getattr__(self, name):
+            return lambda *a: served.append(getattr(ext, name)(*a)) or served[-1]
+
+    ext = _lib.native()
+    monkeypatch.setattr(_lib, "native", Spy)
+    outs = []
+    with torch.no_grad():
+        for xs, vs in ((x, vals), (x.bfloat16(), vals.bfloat16())):
+            cache = KVCache(L=1, B=2, H=2, W=16, D=64, device="cuda:0", dtype=torch.bfloat16)
+            y, k, v = attn.prefill(xs, vs if ve else None, attn_mask=WindowMask(7))
+            s, _, _ = attn.step(xs[:, :1].contiguous(), cache.ring(0), cache.ring(0), 0, vs[:, :1].contiguous() if ve else None, 16)
+            outs.append((y, k, v, s, cache.k, cache.v))
+    assert len(served) == 4 and all(r is not None for r in served)
+    for a, b in zip(*outs):
+        assert a.dtype == b.dtype and torch.equal(a, b)
