@@ -769,7 +769,7 @@ def bench_next_rows(steps, warmup):
         "kv_bytes_per_step": 2 * L * Bs * 8 * min(t_before + 1, W) * 128 * 2}
     del model, cache, recorded
 
-    # ---- training-time block masks as per-row lower bounds: one sequence of 32768, 3 documents ----
+    # ---- training-time block masks as per-row lower bounds (handed over as the module does): one sequence of 32768, 3 documents ----
     with torch.no_grad():
         T, H, D, wblk = 32768, 8, 128, 8          # window of 8 blocks of 128 = 1024 keys
         seq = torch.randint(1, 1000, (T,), device=dev)
@@ -782,7 +782,7 @@ def bench_next_rows(steps, warmup):
             lo = m.doc_start.long()
             pairs = int((torch.arange(T, device=dev) - lo + 1).sum())
             o_buf = torch.empty_like(q)
-            ms, ms_first = time_settled(lambda: ops.prefill_attention(q, k, v, window=None, doc_start=m.doc_start, scale=SCALE, out=o_buf),
+            ms, ms_first = time_settled(lambda: ops.prefill_attention(q, k, v, window=m.span, doc_start=m.doc_start, scale=SCALE, out=o_buf),
                                         max(steps // 2, 5), 3, seconds=0.2)
             fl = 4.0 * D * H * pairs
             rows[name] = {"ms": ms, "ms_first_steps_from_idle": ms_first, "flops": fl, "tflops": fl / ms / 1e9,

@@ -71,6 +71,32 @@ def test_a_library_block_mask_converts_to_the_same_row_bounds(p_eos, w):
     assert torch.equal(mask.doc_start, build_block_window_masks(ids, w, 1, eos_token_id=1, block=block)[0].doc_start)
 
 
+@pytest.mark.parametrize("p_eos", [0.0, 0.01, 0.2])
+@pytest.mark.parametrize("w", [1, 3, 8])
+def test_masks_of_row_bounds_say_how_far_back_a_row_reaches(p_eos, w, monkeypatch):
+    """The attention call gets that as its window (the kernels order their work by it); it hides no key."""
+    from daisy_amd import CausalSelfAttention, WindowMask, _lib
+    T, block = 512, 64
+    ids = _ids(T, p_eos, seed=41 + w)
+    bm = flex_block_mask(ids, w, eos=1, block=block)
+    dense = torch.where(block_mask_pairs(bm), 0.0, float("-inf"))[None, None]
+    most = int(block_mask_pairs(bm).sum(1).max())
+    masks = {"block": block_mask_to_window(bm), "dense": dense_mask_to_window(dense),
+             "closed": build_block_window_masks(ids, w, 1, eos_token_id=1, block=block)[0]}
+    attn = CausalSelfAttention(64, 1, 64, max_seq_len=T)
+    seen = []
+    ext = type("Ext", (), {"layer_prefill": lambda self, *a: seen.append(a[6:8]) or (a[0], None, a[0], a[0])})()
+    monkeypatch.setattr(_lib, "native", lambda: ext)
+    for name, mask in masks.items():
+        assert mask.window is None and (mask.span == most if name != "closed" else most <= mask.span <= w * block), name
+        lo, pos = mask.doc_start.long(), torch.arange(T)
+        assert bool((pos - mask.span + 1 <= lo).all()), name
+        attn(torch.zeros(1, T, 64), None, block_mask=mask)
+        assert seen[-1][0] == mask.span and seen[-1][1] is mask.doc_start, name
+    attn(torch.zeros(1, T, 64), None, attn_mask=WindowMask(100, masks["dense"].doc_start, span=most))    # a window goes first
+    assert seen[-1][0] == 100
+
+
 def test_block_masks_that_are_not_causal_bands_are_refused():
     from torch.nn.attention.flex_attention import create_block_mask
     T = 256
