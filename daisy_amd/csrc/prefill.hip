@@ -125,7 +125,10 @@ __device__ __forceinline__ void workgroup_to_block(const PrefillParams& p, int* 
   if ((nbh & 7) == 0) { group = blockIdx.x & 7; gsize = nbh >> 3; idx = blockIdx.x >> 3; }
   const int n_full = p.nqb - p.n_light;
   int local;
-  if (p.order_shift >= 0) {
+  // (a lone document, which the last row's bound shows, leaves a window's blocks equally long: T = 16384, window 2048, 8 heads of
+  // 128: 145.2 us by length, 142.6 us without, as without documents; one scalar load, which several documents do not feel)
+  const bool by_length = p.order_shift >= 0 && (p.n_light == 0 || p.doc_start[p.T - 1] > 0);
+  if (by_length) {
     if (threadIdx.x < 64) {      // (a load per block touches a cache line each: one wavefront's are enough)
       block_by_length(p, gsize, idx, local, qb, lo);
       if (threadIdx.x == 0) { found[0] = local; found[1] = qb; found[2] = lo; }
@@ -142,7 +145,7 @@ __device__ __forceinline__ void workgroup_to_block(const PrefillParams& p, int* 
     qb = p.n_light - 1 - j / gsize;
     local = j % gsize;
   }
-  if (p.order_shift < 0) lo = row_lo(p, qb * kBM);
+  if (!by_length) lo = row_lo(p, qb * kBM);
   bh = group * gsize + local;
 }
 
@@ -910,8 +913,9 @@ static int fill_prefill_params(PrefillParams& p, const void* q, const int64_t* q
   p.n_light = (window > 0 && window < T) ? min((window - 1 + kBM - 1) / kBM, p.nqb) : 0;
   p.order_shift = -1; p.order_bit = 0;
   // Finding the order costs a workgroup about 1 us; the lengths differ enough to pay for it where a window is an eighth of the
-  // row or more (three documents of T = 16384, window 2048: 197 -> 182 us; a mask with a lone document, which
-  // gains nothing, 162.5 -> 165.4 us; at a sixteenth a lone document costs 148 against 146 us, nine of them take 258 against 270 us).
+  // row or more (three documents of T = 16384, window 2048: 197 -> 182 us; at a sixteenth nine documents take 258 against 270 us).
+  // Without a window they differ also within a lone document (T = 8192, 16 heads of 64: 207 -> 171 us); bounds of rows that all
+  // reach equally far back only pay (8 key blocks of T = 32768: 144 -> 151 us), so a caller who knows how far gives that as the window.
   if (doc_start != nullptr && p.nqb <= 64 * kOrderChunks && (window <= 0 || (int64_t)window * 8 >= T)) {
     int longest = (window > 0 && window < T ? window : T) / 32 + 6;     // tiles of a block
     for (p.order_shift = 0; longest > 255; longest >>= 1) ++p.order_shift;

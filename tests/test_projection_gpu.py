@@ -75,6 +75,22 @@ def test_attention_on_both_sides_of_the_block_rule(D, B, H, T, window, docs):
     assert_close_bf16(o, ref, f"o T={T}")
 
 
+@pytest.mark.parametrize("D,B,H", [(64, 8, 33), (128, 7, 37)])       # many blocks, in XCD groups and not
+@pytest.mark.parametrize("T,window", [(300, 64), (257, 40), (384, 383)])
+def test_a_lone_document_changes_nothing_and_one_that_opens_with_the_last_row_only_that(D, B, H, T, window):
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q, k, v = (torch.randn(B, T, H, D, generator=g, device=DEV).bfloat16() for _ in range(3))
+    plain, _ = ops.prefill_attention(q, k, v, window=window)
+    doc = torch.zeros(T, dtype=torch.int32, device=DEV)
+    assert torch.equal(ops.prefill_attention(q, k, v, window=window, doc_start=doc)[0], plain)
+    doc[-1] = T - 1
+    o, _ = ops.prefill_attention(q, k, v, window=window, doc_start=doc)
+    own = (T - 1) // 32 * 32               # the rows of the last row's wavefront share its rescaling, and with it their rounding:
+    assert torch.equal(o[:, :own], plain[:, :own])
+    want = torch.cat([plain[:, own:-1], v[:, -1:]], 1).float()       # bf16 weights (2^-9) on either side, two roundings of the outputs
+    assert ((o[:, own:].float() - want).abs() <= 2.0 ** -7 * v.float().abs().max()).all()
+
+
 def test_calls_that_something_intercepts_reach_the_library_op():
     """Tangents, subclasses, vmap and autocast of a decode batch's projection (64 rows: above the few-rows kernel)."""
     from daisy_amd.attention import step_linear
