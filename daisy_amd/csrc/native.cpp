@@ -176,8 +176,8 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// linears(x, weights, biases, max_rows, tile): the products of x with several matrices in one launch, as a tuple, or None.
-// Arguments as for linear; weights and biases: tuples (a bias may be None).
+// linears(x, weights, biases, max_rows, tile): the products of x with several matrices in one launch, as a tuple of views of one
+// tensor, or None.  Arguments as for linear; weights and biases: tuples (a bias may be None).
 PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (intercepted() || n != 5 || !is_tensor(a[0]) || !PyTuple_Check(a[1]) || !PyTuple_Check(a[2])) return none();
@@ -200,6 +200,7 @@ PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
     seg[i] = daisy::ProjSegment{r.p, r.stride, (const uint16_t*)ptr(w), w.stride(0), (const uint16_t*)ptr(bias), nullptr, 0, (int)w.size(0), 0};
     pitch += (w.size(0) + 7) / 8 * 8;
   }
+  if (!tile && (max_rows <= 0 || (r.M > max_rows && !daisy::proj_wanted(r.M, (int)pitch, r.K)))) return none();
   Unlocked unlocked;
   Tensor y = empty({(int64_t)r.M, pitch}, at::kBFloat16, x);
   int64_t at = 0;
@@ -213,9 +214,12 @@ PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (rc != DAISY_OK) return none();
   unlocked.end();
   PyObject* res = PyTuple_New(count);
+  c10::SmallVector<int64_t, 5> sizes(x.sizes().begin(), x.sizes().end()), strides(x.dim(), 1);
   at = 0;
   for (Py_ssize_t i = 0; i < count; ++i) {
-    PyTuple_SET_ITEM(res, i, wrap(y.narrow(1, at, seg[i].N)));
+    sizes.back() = seg[i].N;
+    for (int64_t d = x.dim() - 2, step = pitch; d >= 0; step *= sizes[d--]) strides[d] = step;
+    PyTuple_SET_ITEM(res, i, wrap(y.as_strided(sizes, strides, at)));
     at += (seg[i].N + 7) / 8 * 8;
   }
   return res;

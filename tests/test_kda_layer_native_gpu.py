@@ -87,3 +87,27 @@ def test_hooks_on_what_the_layer_calls_are_called():
             handle.remove()
             assert {"GatedRMSNorm", "Linear"} & {t.__name__ for t in seen}
             seen.clear()
+
+
+@pytest.mark.parametrize("B,T,H,D", [(1, 5, 4, 64), (5, 1, 12, 64), (2, 33, 4, 128), (1, 700, 12, 96), (1, 2000, 16, 128)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_input_projections_of_a_layer_on_its_python_path(B, T, H, D, strided):
+    """A layer that receives value embeddings, a padded batch: one launch up to the sizes where the library's products lead."""
+    m = _layer(H, D, 1.0 if D != 96 else 4 / 3, 4, False)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(B, T, 2 * H * D if strided else H * D, generator=g, device=DEV).bfloat16()[..., :H * D]
+    lins = (m.q_proj, m.k_proj, m.v_proj, m.f_proj[0], m.g_proj[0], m.b_proj)
+    with torch.no_grad():
+        served = _lib.native().linears(x, tuple(l.weight for l in lins), (None,) * 6, 4, 0) is not None
+        assert served == (T < 2000)
+        for y, l in zip(m._input_projections(x), lins):
+            ref = x.float() @ l.weight.float().T
+            assert y.shape == ref.shape and y.stride(-1) == 1
+            assert ((y.float() - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-3 * (H * D) ** 0.5).all()
+        mask = torch.ones(B, T, dtype=torch.long, device=DEV)
+        mask[0, :T // 3] = 0
+        if T > 1:
+            y = m(x, None, attn_mask=mask)
+            alone = m(x[:1, T // 3:].contiguous(), None)
+            assert (y[0, :T // 3] == 0).all()
+            assert ((y[:1, T // 3:].float() - alone.float()).norm() / alone.float().norm()).item() < 5e-3
