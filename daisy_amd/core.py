@@ -184,7 +184,7 @@ class GraphedStep:
         self._pos_host: Optional[int] = None      # what self.pos holds, None = unknown
         self._graph: Optional[torch.cuda.CUDAGraph] = None
         self._logits: Optional[Tensor] = None
-        self._recorded_addresses: Optional[tuple] = None
+        self._recorded: Optional[tuple] = None
         self.status = torch.zeros(1, dtype=torch.int32, device=dev)   # raised by the kernels, see check()
         tables = [blk.attn.rotary.cos.shape[0] for blk in model.blocks
                   if getattr(blk, "attn", None) is not None and hasattr(blk.attn, "rotary")]
@@ -196,10 +196,13 @@ class GraphedStep:
                 for t in blk.attn.state_tensors()]
 
     def _addresses(self) -> tuple:
-        """Every address the recorded launches carry besides the parameters: the ring and the layers' own state; and
-        what layers that read a snapshot of their parameters say the snapshot depends on (``replay_guard``)."""
-        guards = tuple(blk.attn.replay_guard() for blk in self.model.blocks if hasattr(getattr(blk, "attn", None), "replay_guard"))
-        return (self.cache.k.data_ptr(), self.cache.v.data_ptr()) + tuple(t.data_ptr() for t in self._stateful_tensors()) + guards
+        """Every address the recorded launches carry besides the parameters: the ring and the layers' own state."""
+        return (self.cache.k.data_ptr(), self.cache.v.data_ptr()) + tuple(t.data_ptr() for t in self._stateful_tensors())
+
+    def _recorded_with(self) -> tuple:
+        """The addresses, and what layers say a recording of theirs depends on besides (``replay_guard``)."""
+        return self._addresses() + tuple(blk.attn.replay_guard() for blk in self.model.blocks
+                                         if hasattr(getattr(blk, "attn", None), "replay_guard"))
 
     def check(self) -> None:
         """Raises what the kernels of the replayed steps reported (a position past the rotary tables).
@@ -236,8 +239,8 @@ class GraphedStep:
         # The graph carries raw addresses.  A layer that made a new state tensor during the walk (no
         # prefill before the first step, a window that could not be shifted in place) would leave the
         # graph pointing at memory that belongs to the capture: refuse to replay such a recording.
-        self._recorded_addresses = self._addresses()
-        if self._recorded_addresses != before:
+        self._recorded = self._recorded_with()
+        if self._addresses() != before:
             self._graph = None
             raise RuntimeError("a recorded step needs layers that update their state in place: run a prefill first "
                                "(the KDA layer creates its state there) and keep the cache's tensors")
@@ -250,7 +253,7 @@ class GraphedStep:
         self.tokens.copy_(token_ids.reshape(-1))
         if self._pos_host != cache.t:
             self.pos.fill_(cache.t)
-        if self._graph is not None and self._addresses() != self._recorded_addresses:
+        if self._graph is not None and self._recorded_with() != self._recorded:
             # A prefill of another batch size, a new cache tensor, a reset that moved a layer's state: the
             # recording points at memory that may have been freed.  Record again at the current addresses.
             self._graph = None

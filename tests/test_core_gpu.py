@@ -304,14 +304,15 @@ def test_recorded_step_with_a_kda_layer():
 
 
 def test_recorded_step_follows_a_weight_that_changes_in_place():
-    """The KDA layer's decode step reads a stacked snapshot of six of its weights; a recording made before one of
-    them changed in place (a state dict loaded into the same model) must not go on replaying the old snapshot."""
+    """A KDA layer whose decode step reads a stacked snapshot of six of its weights (one without convolutions: the
+    one-call step leaves it to the layer's Python path); a recording made before one of them changed in place (a state
+    dict loaded into the same model) must not go on replaying the old snapshot."""
     import copy
     from daisy_amd import KimiLinearSelfAttention
     with torch.no_grad():
         model = _Core(window=48, max_seq_len=512)
         torch.manual_seed(2)
-        model.blocks[0].attn = KimiLinearSelfAttention(256, 2, 512, 128).bfloat16()
+        model.blocks[0].attn = KimiLinearSelfAttention(256, 2, 512, 128, use_short_conv=False).bfloat16()
         model = model.to(DEV)
         twin = copy.deepcopy(model)
         B, T = 1, 20
@@ -324,11 +325,45 @@ def test_recorded_step_follows_a_weight_that_changes_in_place():
         for s in range(4):
             _close(graphed(ids[:, T + s]), core.step(model, ids[:, T + s], eager), f"replay {s}", tol=1e-2)
         first_graph = graphed._graph
+        assert twin.blocks[0].attn._stacked_w is not None
         for m in (model, twin):                      # the same in-place change on both
             m.blocks[0].attn.v_proj.weight.mul_(-1.0)
         for s in range(4, 8):
             _close(graphed(ids[:, T + s]), core.step(model, ids[:, T + s], eager), f"replay {s} after the change", tol=1e-2)
         assert graphed._graph is not first_graph, "the step was recorded again"
+
+
+def test_recorded_one_call_step_reads_the_weights_where_they_are():
+    """No snapshot: a change in place shows in the next replay of the same recording; a weight that was replaced makes a new one."""
+    from daisy_amd import KimiLinearSelfAttention
+    with torch.no_grad():
+        model = _Core(window=48, max_seq_len=512)
+        torch.manual_seed(2)
+        model.blocks[0].attn = layer = KimiLinearSelfAttention(256, 2, 512, 128).bfloat16()
+        model = model.to(DEV)
+        ids = torch.randint(2, 96, (1, 24), generator=torch.Generator().manual_seed(4)).to(DEV)
+        cache = KVCache(4, 1, 2, 48, 128, DEV, torch.bfloat16)
+        graphed = core.GraphedStep(model, cache)
+
+        def both(s):
+            """The token's logits replayed and launched kernel by kernel, from the same states."""
+            held = [t.clone() for t in (cache.k, cache.v, *layer.state_tensors())]
+            got, t0 = graphed(ids[:, s]).clone(), cache.t
+            for t, old in zip((cache.k, cache.v, *layer.state_tensors()), held):
+                t.copy_(old)
+            cache.t = t0 - 1
+            return got, core.step(model, ids[:, s], cache)
+
+        core.prefill(model, ids[:, :20], cache)
+        _close(*both(20), "replay", tol=1e-2)
+        recording = graphed._graph
+        layer.v_proj.weight.mul_(-1.0)
+        _close(*both(21), "after a change in place", tol=1e-2)
+        assert layer._stacked_w is None and graphed._graph is recording
+        old = layer.k_proj.weight                                  # (kept: the recording still names it)
+        layer.k_proj.weight = torch.nn.Parameter(-old)
+        _close(*both(22), "after a replacement", tol=1e-2)
+        assert graphed._graph is not recording
 
 
 def test_generator_single_sequence_with_recorded_steps():

@@ -75,3 +75,19 @@ def test_kimi_layer_constructor_contract():
     for kw in (dict(head_dim=160), dict(head_dim=36), dict(head_dim=128, expand_v=0.75), dict(head_dim=128, conv_size=5)):
         with pytest.raises(ValueError, match="not supported"):
             KimiLinearSelfAttention(256, 2, max_seq_len=64, **kw)
+
+
+@torch.no_grad()
+def test_a_kda_layer_without_a_stacked_copy_guards_addresses_only():
+    from daisy_amd import KimiLinearSelfAttention
+    m = KimiLinearSelfAttention(128, 2, max_seq_len=16, head_dim=64)
+    guard = m.replay_guard()
+    m.v_proj.weight.mul_(-1.0)                           # read where it is by a recorded step
+    assert m.replay_guard() == guard
+    old = m.v_proj.weight
+    m.v_proj.weight = torch.nn.Parameter(-old)
+    assert m.replay_guard() != guard
+    m._stacked_key = m._input_weights()                  # as the Python path leaves it: a snapshot of this version
+    guard = m.replay_guard()
+    m.v_proj.weight.mul_(-1.0)
+    assert m.replay_guard() != guard
