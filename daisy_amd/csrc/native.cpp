@@ -292,7 +292,7 @@ PyObject* py_layer_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!rows_bf16(w, 3, dev) || !w.is_contiguous() || w.size(0) != 4 || w.size(1) != dim || w.size(2) != dim) return none();
   const int64_t B = x.size(0), T = x.size(1);
   if (!rotary_table(cos, T, D / 2, dev) || !rotary_table(sin, T, D / 2, dev)) return none();
-  if (doc && !int32_vector(*doc, T, dev)) return none();
+  if (doc && !(int32_vector(*doc, T, dev) && doc->dim() == 1)) return none();
   if ((ve == nullptr) != (g_ve == nullptr) || (k_out == nullptr) != (v_out == nullptr)) return none();
   if (needs_autograd({&x, &w, ve, g_ve})) return none();
   GateSource gate{nullptr, 0};
@@ -564,7 +564,7 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!matrix(w[6], kd, Dv) || !matrix(w[7], vd, Dv) || (w[8] && !vector(w[8], vd, at::kBFloat16)) || !matrix(w[9], dim, vd)) return none();
   for (int i = 0; i < 3; ++i) {
     if (!vector(w[10 + i], widths[i] * taps, at::kBFloat16) || (w[13 + i] && !vector(w[13 + i], widths[i], at::kBFloat16))) return none();
-    if (win[i] && !(vector(win[i], B * widths[i] * taps, at::kBFloat16) && win[i]->dim() == 3 && win[i]->size(0) == B)) return none();
+    if (win[i] && !(vector(win[i], B * widths[i] * taps, at::kBFloat16) && win[i]->dim() == 3 && win[i]->size(0) == B && win[i]->size(1) == widths[i])) return none();
   }
   if (!vector(w[16], H, at::kFloat) || !vector(w[17], kd, at::kFloat) || !vector(w[18], Dv, at::kBFloat16)) return none();
   if (state && !(vector(state, B * kd * Dv, at::kFloat) && state->dim() == 4 && state->size(0) == B && state->size(1) == H && state->size(2) == Dk)) return none();

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from daisy_amd import CausalSelfAttention, KVCache, WindowMask, _lib
+from daisy_amd import CausalSelfAttention, KimiLinearSelfAttention, KVCache, WindowMask, _lib
 
 
 class _Recorder:
@@ -70,3 +70,22 @@ def test_fp32_activations_equal_the_bf16_ones_they_round_to(ve, monkeypatch):
     assert len(served) == 4 and all(r is not None for r in served)
     for a, b in zip(*outs):
         assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_shapes_that_the_kernels_functions_refuse_are_refused_in_one_call_too():
+    attn = _attn(ve=False).to("cuda:0")
+    x = torch.randn(1, 9, 128, device="cuda:0").bfloat16()
+    bounds = torch.zeros(9, dtype=torch.int32, device="cuda:0")
+    attn.prefill(x, None, attn_mask=WindowMask(4, bounds))
+    for bad in (bounds[None], bounds[:, None], bounds[:8], bounds.long()):
+        with pytest.raises(ValueError, match="doc_start"):
+            attn.prefill(x, None, attn_mask=WindowMask(4, bad))
+    layer = KimiLinearSelfAttention(128, 2, max_seq_len=16, head_dim=64).to("cuda:0").eval()
+    for call in (lambda: layer.prefill(x, None), lambda: layer.step(x[:, :1], None, None, 9, None, None)):
+        layer.reset_history()
+        layer.prefill(x, None)
+        layer._conv_state = tuple(w.transpose(1, 2).contiguous() for w in layer._conv_state)
+        with pytest.raises(ValueError, match="cache must be"):
+            call()
