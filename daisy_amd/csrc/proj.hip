@@ -362,17 +362,20 @@ static int launch_proj(ProjSegmentsParams& p, hipStream_t s) {
 template <int EPI, typename PARAMS>
 static int dispatch_proj(int tile, PARAMS& p, hipStream_t s) {
   for (const ProjTile& t : kProjTiles)
-    DAISY_CHECK_SUPPORTED(t.code != tile || (p.K % t.bk == 0 && !(EPI == 2 && t.bn % 128 != 0)), "proj: tile %d does not serve K=%d", tile, p.K);
+    DAISY_CHECK_SUPPORTED(t.code != tile || (p.K % t.bk == 0 && !(EPI == 2 && t.bn % 128 != 0) && !(EPI == 3 && t.code == 7)),
+                          "proj: tile %d does not serve K=%d with epilogue %d", tile, p.K, EPI);
   if constexpr (EPI != 2) {
     if (tile == 1) return launch_proj<32, 64, 2, 2, 128, 3, EPI>(p, s);
     if (tile == 2) return launch_proj<64, 64, 2, 4, 128, 4, EPI>(p, s);
+  }
+  if constexpr (EPI != 3) {
+    if (tile == 7) return launch_proj<256, 256, 2, 4, 64, 2, EPI>(p, s);
   }
   switch (tile) {
     case 3: return launch_proj<64, 128, 2, 4, 128, 3, EPI>(p, s);
     case 4: return launch_proj<64, 128, 2, 2, 64, 3, EPI>(p, s);
     case 5: return launch_proj<128, 128, 4, 2, 64, 4, EPI>(p, s);
     case 6: return launch_proj<128, 128, 2, 2, 64, 2, EPI>(p, s);
-    case 7: return launch_proj<256, 256, 2, 4, 64, 2, EPI>(p, s);
     default: DAISY_CHECK_SUPPORTED(false, "proj: no tile %d", tile);
   }
 }
@@ -409,14 +412,14 @@ int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, in
     for (int i = 0; i < n; ++i) c += (seg[i].N + bn - 1) / bn;
     return c;
   };
-  if (!tile) tile = proj_tile(M, K, 8, columns);
-  if (!gates) return dispatch_proj<0>(tile, p, s);
+  const int by_size = tile ? tile : proj_tile(M, K, 8, columns);
+  if (!gates) return dispatch_proj<0>(by_size, p, s);
   DAISY_CHECK_ARG(gates->A_log && gates->dt_bias && gates->logits && gates->beta && gates->H > 0 && gates->Dk % 8 == 0 && seg[0].N == gates->H * gates->Dk,
                   "proj_segments: gate of %d heads of %d channels on a product of %d", gates->H, gates->Dk, seg[0].N);
   p.gates = *gates;
-  // (two workgroups to a compute unit: the gate of one runs beside the copies of the other; 32768 rows, whole layer: 1674 against 1680 us)
-  if (tile == 7) tile = 6;
-  return dispatch_proj<3>(tile, p, s);
+  // (no gate with tile 7: of tile 6 two workgroups fit a compute unit, and the gate of one runs beside the copies of the other;
+  // 32768 rows, whole layer: 1674 against 1680 us)
+  return dispatch_proj<3>(!tile && by_size == 7 ? 6 : by_size, p, s);
 }
 
 int proj_qkv(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const QkvEpilogue& e,

@@ -1,4 +1,7 @@
 """What the modules hand to the one-call path (``daisy_amd/_native.so``) and which calls it serves."""
+import ctypes
+from ctypes import c_int, c_int64, c_void_p
+
 import pytest
 import torch
 
@@ -89,3 +92,25 @@ def test_shapes_that_the_kernels_functions_refuse_are_refused_in_one_call_too():
         layer._conv_state = tuple(w.transpose(1, 2).contiguous() for w in layer._conv_state)
         with pytest.raises(ValueError, match="cache must be"):
             call()
+
+
+class _Segment(ctypes.Structure):
+    _fields_ = [("x", c_void_p), ("x_sm", c_int64), ("w", c_void_p), ("w_sn", c_int64), ("bias", c_void_p), ("y", c_void_p),
+                ("y_sm", c_int64), ("N", c_int), ("tile_end", c_int)]
+
+
+class _Gates(ctypes.Structure):
+    _fields_ = [("A_log", c_void_p), ("dt_bias", c_void_p), ("H", c_int), ("Dk", c_int), ("logits", c_void_p),
+                ("logits_row", c_int64), ("beta", c_void_p)]
+
+
+@pytest.mark.parametrize("tile,K", [(7, 128), (8, 128), (1, 64)])
+def test_a_forced_tile_that_does_not_serve_a_gated_product_is_refused(tile, K):
+    """Not replaced by another: refused ahead of any launch (an internal function of the library, called by its C++ name)."""
+    lib = _lib.load()
+    fn = lib._ZN5daisy13proj_segmentsEPKNS_11ProjSegmentEiiiP12ihipStream_tiPKNS_8KdaGatesE
+    fn.argtypes = [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p]
+    p = (ctypes.addressof(ctypes.create_string_buffer(64)) + 15) // 16 * 16        # (never read)
+    seg, gates = _Segment(p, K, p, K, None, p, 128, 128, 0), _Gates(p, p, 2, 64, p, 8, p)
+    assert fn(ctypes.byref(seg), 1, 4, K, None, tile, ctypes.byref(gates)) == -2
+    assert "tile" in lib.daisy_last_error().decode()
