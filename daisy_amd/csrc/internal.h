@@ -129,6 +129,7 @@ struct ConvPart {
 };
 int short_conv_group(const ConvPart* parts, int n, int B, int T, int K, int silu, hipStream_t s);
 bool kda_layer_step_serves(int Dk, int Dv, int taps);
+bool gated_rmsnorm_serves(int D);      // the widths that daisy_gated_rmsnorm_fwd takes
 int kda_layer_step(const KdaLayerStep& p, int B, int Dv, hipStream_t s);
 
 }  // namespace daisy

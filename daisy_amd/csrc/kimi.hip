@@ -274,6 +274,8 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(GatedNormParams p) {
   if (row < p.rows) *reinterpret_cast<u32x4*>(p.out + r * D + 8 * c) = pack8(o);
 }
 
+bool gated_rmsnorm_serves(int D) { return D == 32 || D == 64 || D == 128 || D == 256; }
+
 }  // namespace daisy
 
 using namespace daisy;
@@ -361,7 +363,7 @@ extern "C" int daisy_gated_rmsnorm_fwd(const void* x, const void* gate, const vo
                                        int64_t rows, int D, float eps, void* stream) {
   DAISY_CHECK_ARG(x && gate && weight && out, "gated_rmsnorm: x, gate, weight and out must be non-NULL");
   DAISY_CHECK_ARG(rows > 0, "gated_rmsnorm: rows=%lld must be positive", (long long)rows);
-  DAISY_CHECK_SUPPORTED(D == 32 || D == 64 || D == 128 || D == 256, "gated_rmsnorm: last dim %d not supported (32, 64, 128 or 256)", D);
+  DAISY_CHECK_SUPPORTED(gated_rmsnorm_serves(D), "gated_rmsnorm: last dim %d not supported (32, 64, 128 or 256)", D);
   auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
   DAISY_CHECK_ARG(al16(x) && al16(gate) && al16(weight) && al16(out), "gated_rmsnorm: tensors must be 16-byte aligned");
   GatedNormParams p;

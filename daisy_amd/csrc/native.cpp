@@ -4,7 +4,8 @@
 // walking the same step through Python wrappers, ctypes and tensor views took the host 55 to 120 us.  The functions
 // here take the tensors as they are, check shapes, types and strides in C++, allocate the outputs and launch.  Each
 // returns None for anything out of the ordinary (other dtypes, layouts, devices, autograd, a kernel that refused its
-// arguments): the Python function in front of it then runs its own path, which serves the case or raises.
+// arguments): the Python function in front of it then runs its own path, which serves the case or raises.  What has been
+// written by then it writes again, the same values to the same places; only the KDA layer's states would not bear that.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -111,6 +112,9 @@ class Unlocked {
 };
 
 PyObject* wrap(const Tensor& t) { return THPVariable_Wrap(t); }
+
+// For a kernel behind which a call cannot be given back to the Python function in front of it.
+void must(int rc) { TORCH_CHECK(rc == DAISY_OK, "daisy_amd: a kernel refused its arguments (code ", rc, "): ", daisy_last_error()); }
 
 // The gate logit of a layer with value embeddings; false when it is not a lone fp32 or bf16 number on the GPU.
 bool gate_source(const Tensor& g, int dev, GateSource& out) {
@@ -566,11 +570,13 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!vector(w[10 + i], widths[i] * taps, at::kBFloat16) || (w[13 + i] && !vector(w[13 + i], widths[i], at::kBFloat16))) return none();
     if (win[i] && !(vector(win[i], B * widths[i] * taps, at::kBFloat16) && win[i]->dim() == 3 && win[i]->size(0) == B && win[i]->size(1) == widths[i])) return none();
   }
-  if (!vector(w[16], H, at::kFloat) || !vector(w[17], kd, at::kFloat) || !vector(w[18], Dv, at::kBFloat16)) return none();
+  if (!vector(w[16], H, at::kFloat) || !vector(w[17], kd, at::kFloat) || !vector(w[18], Dv, at::kBFloat16) ||
+      (reinterpret_cast<uintptr_t>(ptr(w[18])) & 15) != 0) return none();
   if (state && !(vector(state, B * kd * Dv, at::kFloat) && state->dim() == 4 && state->size(0) == B && state->size(1) == H && state->size(2) == Dk)) return none();
   const bool step = keep && T == 1 && state;
   const size_t need = step ? 0 : daisy_kda_workspace_bytes((int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64);
-  if (step ? !(win[0] && win[1] && win[2] && daisy::kda_layer_step_serves((int)Dk, (int)Dv, (int)taps)) : (need == 0 || dim % 64 != 0 || Dv % 64 != 0)) return none();
+  if (step ? !(win[0] && win[1] && win[2] && daisy::kda_layer_step_serves((int)Dk, (int)Dv, (int)taps)) : (need == 0 || dim % 64 != 0 || Dv % 64 != 0 || !daisy::gated_rmsnorm_serves((int)Dv)))
+    return none();
 
   // ---- the projections of the input ---------------------------------------------------------------------------------
   Unlocked unlocked;
@@ -602,10 +608,14 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (daisy::proj_segments(seg + 3, 3, (int)M, (int)dim, s) != DAISY_OK) return none();
   }
 
-  // ---- one token: everything up to the output projection in one launch ----------------------------------------------
+  // ---- one token: everything up to the output projection in one launch; a prompt: the convolutions --------------------
   const float scale = (float)(1.0 / std::sqrt((double)Dk));
   constexpr float kL2Eps = 1e-6f;
-  Tensor o, st, new_win[3];
+  Tensor o, conv[3], new_win[3];
+  // Where a state is kept: in its home when that has the shape, else in a new tensor.
+  auto keeper = [&](const Tensor* h, at::IntArrayRef shape, at::ScalarType type) {
+    return h && on_gpu(*h, dev) && h->scalar_type() == type && h->is_contiguous() && h->sizes() == shape ? *h : empty(shape, type, x);
+  };
   if (step) {
     o = empty({B, 1, vd}, at::kBFloat16, x);
     daisy::KdaLayerStep p{seg[0].y, seg[1].y, seg[2].y, seg[3].y, seg[4].y, seg[5].y, seg[0].y_sm, seg[1].y_sm, seg[2].y_sm, seg[3].y_sm,
@@ -615,11 +625,6 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     for (int i = 0; i < 3; ++i) p.window[i] = (uint16_t*)ptr(win[i]);
     if (daisy::kda_layer_step(p, (int)B, (int)Dv, s) != DAISY_OK) return none();
   } else {
-    // Where a state is kept: in its home when that has the shape, else in a new tensor.
-    auto keeper = [&](const Tensor* h, at::IntArrayRef shape, at::ScalarType type) {
-      return h && on_gpu(*h, dev) && h->scalar_type() == type && h->is_contiguous() && h->sizes() == shape ? *h : empty(shape, type, x);
-    };
-    Tensor conv[3];
     daisy::ConvPart parts[3];
     for (int i = 0; i < 3; ++i) {
       conv[i] = empty({B, T, widths[i]}, at::kBFloat16, x);
@@ -632,26 +637,35 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     if (daisy::short_conv_group(parts, 3, (int)B, (int)T, (int)taps, 1, s) != DAISY_OK) return none();
     for (Tensor& t : big) t = Tensor();
-    Tensor g = empty({M, kd}, at::kBFloat16, x), gate = empty({M, vd}, at::kBFloat16, x), beta = empty({M, H}, at::kFloat, x);
-    const daisy::ProjSegment low[2] = {{seg[3].y, seg[3].y_sm, W[6], Dv, nullptr, (uint16_t*)ptr(g), kd, (int)kd, 0},
-                                       {seg[4].y, seg[4].y_sm, W[7], Dv, W[8], (uint16_t*)ptr(gate), vd, (int)vd, 0}};
-    const daisy::KdaGates gates{(const float*)ptr(w[16]), (const float*)ptr(w[17]), (int)H, (int)Dk, seg[5].y, seg[5].y_sm, (float*)ptr(beta)};
-    if (daisy::proj_segments(low, 2, (int)M, (int)Dv, s, 0, &gates) != DAISY_OK) return none();
-    o = empty({B, T, vd}, at::kBFloat16, x);
-    if (keep) st = keeper(home[0], {B, H, Dk, Dv}, at::kFloat);
-    Tensor ws = empty({(int64_t)need}, at::kByte, x);
-    if (daisy_kda_chunk_fwd(ptr(conv[0]), ptr(conv[1]), ptr(conv[2]), ptr(g), 1, (const float*)ptr(beta), (const float*)ptr(state), ptr(o),
-                            keep ? (float*)ptr(st) : nullptr, (int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64, scale, 1, kL2Eps, ptr(ws), need, s) != DAISY_OK)
-      return none();
-    if (daisy_gated_rmsnorm_fwd(ptr(o), ptr(gate), W[18], ptr(o), M * H, (int)Dv, norm_eps, s) != DAISY_OK) return none();
   }
-  Tensor y;
-  if (M <= max_rows || daisy::proj_wanted((int)M, (int)dim, (int)vd)) {
-    y = empty({B, T, dim}, at::kBFloat16, x);
-    if (!own_linear(Rows{(const uint16_t*)ptr(o), vd, (int)M, (int)vd}, W[9], vd, (int)dim, nullptr, (uint16_t*)ptr(y), dim, max_rows, s)) return none();
-  } else {
-    y = at::linear(o, *w[9]);
-  }
+
+  // ---- the rest.  The state of a step, the windows of a prompt may have changed in place by now: there is no way back to the
+  // ---- caller's own path, which would apply the tokens a second time, so a refusal raises (and cannot be returned from here)
+  auto rest = [&]() -> std::array<Tensor, 2> {
+    Tensor st, y;
+    if (!step) {
+      Tensor g = empty({M, kd}, at::kBFloat16, x), gate = empty({M, vd}, at::kBFloat16, x), beta = empty({M, H}, at::kFloat, x);
+      const daisy::ProjSegment low[2] = {{seg[3].y, seg[3].y_sm, W[6], Dv, nullptr, (uint16_t*)ptr(g), kd, (int)kd, 0},
+                                         {seg[4].y, seg[4].y_sm, W[7], Dv, W[8], (uint16_t*)ptr(gate), vd, (int)vd, 0}};
+      const daisy::KdaGates gates{(const float*)ptr(w[16]), (const float*)ptr(w[17]), (int)H, (int)Dk, seg[5].y, seg[5].y_sm, (float*)ptr(beta)};
+      must(daisy::proj_segments(low, 2, (int)M, (int)Dv, s, 0, &gates));
+      o = empty({B, T, vd}, at::kBFloat16, x);
+      if (keep) st = keeper(home[0], {B, H, Dk, Dv}, at::kFloat);
+      Tensor ws = empty({(int64_t)need}, at::kByte, x);
+      must(daisy_kda_chunk_fwd(ptr(conv[0]), ptr(conv[1]), ptr(conv[2]), ptr(g), 1, (const float*)ptr(beta), (const float*)ptr(state), ptr(o),
+                               keep ? (float*)ptr(st) : nullptr, (int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64, scale, 1, kL2Eps, ptr(ws), need, s));
+      must(daisy_gated_rmsnorm_fwd(ptr(o), ptr(gate), W[18], ptr(o), M * H, (int)Dv, norm_eps, s));
+    }
+    if (M <= max_rows || daisy::proj_wanted((int)M, (int)dim, (int)vd)) {
+      y = empty({B, T, dim}, at::kBFloat16, x);
+      must(own_linear(Rows{(const uint16_t*)ptr(o), vd, (int)M, (int)vd}, W[9], vd, (int)dim, nullptr, (uint16_t*)ptr(y), dim, max_rows, s)
+               ? DAISY_OK : DAISY_ERR_UNSUPPORTED);
+    } else {
+      y = at::linear(o, *w[9]);
+    }
+    return {y, st};
+  };
+  const auto [y, st] = rest();
   unlocked.end();
   PyObject* res = PyTuple_New(5);
   PyTuple_SET_ITEM(res, 0, wrap(y));

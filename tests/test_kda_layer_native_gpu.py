@@ -111,3 +111,25 @@ def test_input_projections_of_a_layer_on_its_python_path(B, T, H, D, strided):
             alone = m(x[:1, T // 3:].contiguous(), None)
             assert (y[0, :T // 3] == 0).all()
             assert ((y[:1, T // 3:].float() - alone.float()).norm() / alone.float().norm()).item() < 5e-3
+
+
+@pytest.mark.parametrize("what", ["value width", "norm weight"])
+@torch.no_grad()
+def test_a_call_that_is_given_back_has_not_touched_the_states(what):
+    """A value width that the gated norm does not take, a norm weight off its 16-byte boundary: refused ahead of the
+    convolutions, which write the windows where they are kept."""
+    H, Dk, Dv, B, T = 2, 64, 192 if what == "value width" else 64, 2, 5
+    dim, kd, vd = 128, H * Dk, H * Dv
+    g = torch.Generator(device=DEV).manual_seed(3)
+
+    def rnd(*shape, dtype=torch.bfloat16):
+        return (torch.randn(*shape, generator=g, device=DEV) * 0.1).to(dtype)
+
+    norm_w = rnd(Dv + 1)[1:] if what == "norm weight" else rnd(Dv)
+    weights = (rnd(kd, dim), rnd(kd, dim), rnd(vd, dim), rnd(Dv, dim), rnd(Dv, dim), rnd(H, dim), rnd(kd, Dv), rnd(vd, Dv), rnd(vd), rnd(dim, vd),
+               rnd(kd, 1, 4), rnd(kd, 1, 4), rnd(vd, 1, 4), None, None, None, rnd(H, dtype=torch.float32), rnd(kd, dtype=torch.float32), norm_w)
+    state, windows = rnd(B, H, Dk, Dv, dtype=torch.float32), tuple(rnd(B, c, 4) for c in (kd, kd, vd))
+    before = [t.clone() for t in (state, *windows)]
+    assert _lib.native().kda_layer(rnd(B, T, dim), weights, H, Dk, Dv, 4, state, windows, (state, *windows), True, 1e-5, 4) is None
+    for t, b in zip((state, *windows), before):
+        assert torch.equal(t, b)
