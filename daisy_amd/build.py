@@ -65,16 +65,21 @@ NATIVE_SOURCE = os.path.join(CSRC, "native.cpp")
 NATIVE_PATH = os.path.join(os.path.dirname(CSRC), "_native.so")
 
 
-def _compile_native(verbose: bool) -> str:
+def _native_command() -> list:
+    """The host compiler with the flags of native.cpp: every warning on for our code, headers of others (-isystem) quiet."""
     import sysconfig
     import torch
     from torch.utils.cpp_extension import include_paths
-    obj = os.path.splitext(NATIVE_SOURCE)[0] + ".o"
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wextra", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
     for inc in (*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]):
         cmd += ["-isystem", inc]
-    _run([*cmd, "-c", NATIVE_SOURCE, "-o", obj], "native.cpp", verbose)
+    return cmd
+
+
+def _compile_native(verbose: bool) -> str:
+    obj = os.path.splitext(NATIVE_SOURCE)[0] + ".o"
+    _run([*_native_command(), "-c", NATIVE_SOURCE, "-o", obj], "native.cpp", verbose)
     return obj
 
 
@@ -91,6 +96,8 @@ def _run(cmd, what: str, verbose: bool) -> None:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"building {what} failed:\n{r.stdout}\n{r.stderr}")
+    if verbose and r.stderr.strip():
+        print(r.stderr, flush=True)
 
 
 def _link(objs, out: str, verbose: bool) -> None:
