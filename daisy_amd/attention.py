@@ -437,7 +437,7 @@ class CausalSelfAttention(nn.Module):
             fast = _lib.native().layer_prefill(
                 x, self.qkvo_w, rot.cos, rot.sin, self.num_heads, self.head_dim, window or 0, mask.doc_start,
                 ve, self.g_ve, k_dest, v_dest, float(self.attn_scale), NORM_EPS_BF16,
-                STEP_ROWS_KERNEL_MAX, want_q)
+                STEP_ROWS_KERNEL_MAX, bool(want_q))
             if fast is not None:
                 return fast
             q, k_rot, v = self._project_qkv_fused(x, ve, 0, *(dest or (None, None)))

@@ -47,6 +47,16 @@ def test_activations_reach_the_one_call_path_in_the_weights_dtype(x_dtype, ve_dt
     assert ext.args[7] is None if ve is None else ext.args[7].dtype == torch.bfloat16
 
 
+@pytest.mark.parametrize("debug", [False, True, 0, 1, "yes"])
+def test_debug_taps_are_asked_for_by_truth(debug, monkeypatch):
+    """The extension looks for True itself: any other true value used to leave ``last_q`` empty."""
+    attn, kv = _attn(ve=False), torch.zeros(1, 5, 2, 64)
+    ext = _Recorder((kv, kv, kv, kv))
+    monkeypatch.setattr(_lib, "native", lambda: ext)
+    attn.prefill(torch.randn(1, 5, 128), None, attn_mask=WindowMask(4), debug=debug)
+    assert ext.args[15] is bool(debug)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("ve", [False, True])
 def test_fp32_activations_equal_the_bf16_ones_they_round_to(ve, monkeypatch):
