@@ -24,6 +24,21 @@ def say(msg: str):
     print(msg, flush=True)
 
 
+def check_prefill_of_many_heads(q, k, v, ref, what: str, k_rot=None, **kw):
+    """The attention call again with its heads repeated until there are more blocks of 128 queries than the kernel for few
+    blocks (four wavefronts per 32 queries) is used for: the kernel of 128 queries per workgroup on the same small shape.
+    Every repetition equals the first, the first the reference ``[B, T, H, D]``."""
+    from daisy_amd import ops
+    B, T, H, D = q.shape
+    n = 768 // ((T + 127) // 128 * H * B) + 1
+    o, kr = ops.prefill_attention(*(t.repeat(1, 1, n, 1) for t in (q, k, v)), **kw)
+    for got, want, name in ((o, ref, "o"), (kr, k_rot, "rotated keys")):
+        if want is not None:
+            got = got.view(B, T, n, H, D)
+            assert torch.equal(got, got[:, :, :1].expand_as(got)), f"{what}: {name} of equal heads differ"
+            assert_close_bf16(got[:, :, 0], want, f"{name}, many heads ({what})")
+
+
 def flex_block_mask(ids: torch.Tensor, window_blocks: int, eos: int, block: int = 128):
     """A ``torch.nn.attention.flex_attention.BlockMask`` for document-causal attention with a window
     counted in key blocks, assembled the way the reference's training forward assembles its masks

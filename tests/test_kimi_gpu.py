@@ -402,6 +402,8 @@ def test_stacked_input_projections_equal_the_separate_ones(B):
             assert torch.equal(a, b)
         # the whole step through the stacked matrix equals the step through the separate launches
         xs = torch.randn(B, 6, 256, generator=g).bfloat16().to(DEV)
+        m._fast = lambda x, use_cache: None              # (the one-call step reads no stack)
+        stack = m._stacked_w
         m.reset_history()
         m.prefill(xs[:, :3], None, attn_mask=None)
         y_stacked = [m.step(xs[:, t:t + 1], None, None, t, None, window=None)[0] for t in range(3, 6)]
@@ -409,7 +411,8 @@ def test_stacked_input_projections_equal_the_separate_ones(B):
         m._input_projections = lambda inp: tuple(_project(l, inp) for l in lins)
         m.prefill(xs[:, :3], None, attn_mask=None)
         y_separate = [m.step(xs[:, t:t + 1], None, None, t, None, window=None)[0] for t in range(3, 6)]
-        del m._input_projections
+        del m._input_projections, m._fast
+        assert m._stacked_w is stack
         for a, b in zip(y_stacked, y_separate):
             assert torch.equal(a, b)
         # more rows than the few-rows kernel is used for: the separate library products

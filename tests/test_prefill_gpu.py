@@ -4,7 +4,7 @@ import torch
 
 import oracle
 from daisy_amd import ops
-from helpers import assert_close_bf16, say
+from helpers import assert_close_bf16, check_prefill_of_many_heads, say
 
 pytestmark = pytest.mark.gpu
 
@@ -71,6 +71,10 @@ def test_prefill_matches_oracle(B, T, H, D, window, rope, docs):
                                f"{bad.numel()} differ, max diff {(k_rot.cpu().float() - k_ref.float()).abs().max().item():.3e}")
     else:
         assert k_rot is None
+    if D in (64, 128):
+        check_prefill_of_many_heads(*(t.to(dev) for t in (q, k, v)), ref, "oracle case", k_rot=k_ref if rope else None, window=window,
+                                    cos=None if cos is None else cos.to(dev), sin=None if sin is None else sin.to(dev),
+                                    doc_start=None if doc_start is None else doc_start.to(dev))
 
 
 def test_prefill_strided_views_of_merged_qkv():
@@ -127,6 +131,9 @@ def test_prefill_is_deterministic_and_window_invariant():
     a, _ = ops.prefill_attention(q, k, v, window=None)
     b, _ = ops.prefill_attention(q, k, v, window=T)
     c, _ = ops.prefill_attention(q, k, v, window=T + 1000)
+    assert torch.equal(a, b) and torch.equal(a, c)
+    q, k, v = (t.repeat(1, 1, 200, 1) for t in (q, k, v))      # more query blocks than the kernel for few of them takes
+    a, b, c = (ops.prefill_attention(q, k, v, window=w)[0] for w in (None, T, T + 1000))
     assert torch.equal(a, b) and torch.equal(a, c)
 
 

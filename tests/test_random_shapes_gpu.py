@@ -11,7 +11,7 @@ import torch
 import oracle
 from oracle import kda as okda
 from daisy_amd import chunk_kda, fused_recurrent_kda, ops
-from helpers import assert_close_bf16, say
+from helpers import assert_close_bf16, check_prefill_of_many_heads, say
 
 pytestmark = pytest.mark.gpu
 SCALE = 0.12
@@ -55,6 +55,9 @@ def test_prefill_random_shapes(seed):
         assert_close_bf16(o, ref, f"o (case {it})")
         if rope:
             assert_close_bf16(k_rot, kr, f"rotated keys (case {it})")
+        check_prefill_of_many_heads(qd, kd, vd, ref, f"case {it}", k_rot=kr if rope else None, window=window, scale=SCALE,
+                                    cos=None if cos is None else cos.cuda(), sin=None if sin is None else sin.cuda(),
+                                    doc_start=None if doc_start is None else doc_start.cuda())
 
 
 @pytest.mark.parametrize("seed", [21, 22])

@@ -12,7 +12,7 @@ import torch
 
 import oracle
 from daisy_amd import ops
-from helpers import assert_close_bf16, say
+from helpers import assert_close_bf16, check_prefill_of_many_heads, say
 
 pytestmark = pytest.mark.gpu
 
@@ -47,7 +47,8 @@ def _random_large(B, T, H, D, seed):
 def test_prefill_large_logits(D, window, rise):
     """T = 700: 5.5 query blocks, 22 key tiles; with window 200 the tile order is rotated (every block starts in
     the middle of its range and wraps), so a rising score puts the row maximum in a tile that is visited in the
-    middle of the walk and a falling one in the tile visited right after the wrap."""
+    middle of the walk and a falling one in the tile visited right after the wrap.  Two heads run on the kernel for few query
+    blocks, whose wavefronts take every fourth tile; the repeated heads on the one that walks all of them."""
     if window == 1 and rise not in (5.0, "random"):
         pytest.skip("one key per row: the structure does not matter")
     B, T, H = 1, 700, 2
@@ -58,6 +59,7 @@ def test_prefill_large_logits(D, window, rise):
     say(f"  score range in log2 units: {s.min().item():.0f} .. {s.max().item():.0f}")
     o, _ = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), window=window, scale=1.0)
     assert_close_bf16(o, ref, "o")
+    check_prefill_of_many_heads(q.cuda(), k.cuda(), v.cuda(), ref, f"rise {rise}", window=window, scale=1.0)
 
 
 @pytest.mark.parametrize("D", [64, 128])
@@ -74,6 +76,8 @@ def test_prefill_large_logits_with_rotation_and_documents(D):
     o, _ = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), window=W, scale=1.0, cos=cos.cuda(), sin=sin.cuda(),
                                  doc_start=doc_start.cuda())
     assert_close_bf16(o, ref, "o")
+    check_prefill_of_many_heads(q.cuda(), k.cuda(), v.cuda(), ref, "documents", window=W, scale=1.0, cos=cos.cuda(), sin=sin.cuda(),
+                                doc_start=doc_start.cuda())
 
 
 @pytest.mark.parametrize("D", [64, 128])
