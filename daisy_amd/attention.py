@@ -2,10 +2,11 @@
 
 Mirrors models/daisy/attention.py of the reference: same constructor, same
 state-dict keys (``qkvo_w``, optional ``g_ve``), same ``forward`` / ``prefill`` /
-``step`` / ``reset_history`` signatures, shapes and dtypes.  The QKV and output
-projections and the weightless RMS norms stay PyTorch library calls; RoPE, the
-mask and the attention itself run in ``libdaisy_hip.so``.  Inference only: the
-kernels have no backward.
+``step`` / ``reset_history`` signatures, shapes and dtypes.  With bf16 weights
+a call goes from its tensors to the kernels in one step (``_native.so``): the
+projections, the norms, RoPE, the value mix and the attention, with the library's
+GEMM for products where that leads; anything out of the ordinary takes the path
+below, kernel by kernel.  Inference only: the kernels have no backward.
 
 Masks.  The reference passes a dense additive ``[1, 1, T, T]`` mask built by
 ``build_attn_mask`` (models/daisy/daisy_core.py:53-69).  Here the mask is the
@@ -313,7 +314,8 @@ class Rotary(nn.Module):
 
 
 # Up to this many sequences, a decode step's two projections go through ``ops.linear_rows`` (the weights are read
-# once by a kernel made for a few rows: 4.6 against 9.9 us for a 4608 x 1536 matrix and one row); beyond, the library GEMM.
+# once by a kernel made for a few rows: 4.6 against 9.9 us for a 4608 x 1536 matrix and one row); beyond, the tiled kernel
+# while it leads, then the library GEMM.  0: the library GEMM everywhere.
 STEP_ROWS_KERNEL_MAX = 4
 
 

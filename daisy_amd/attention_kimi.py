@@ -17,7 +17,7 @@ The delta-rule core runs on the HIP kernels (``chunk_kda`` for sequences, ``fuse
 with the state updated in place for single-token steps), and so do the four-tap convolutions
 with their SiLU and the gated norm (one streaming kernel each, ``daisy_short_conv_fwd`` and
 ``daisy_gated_rmsnorm_fwd``; like every op of this package they run on the GPU only and raise
-for CPU tensors); the projections are library GEMMs.  Three pieces of the reference come from the absent
+for CPU tensors); large projections are library GEMMs.  Three pieces of the reference come from the absent
 ``flash-linear-attention`` package and are restated from their documented behaviour, not pinned
 against it: ``ShortConvolution`` (depthwise causal conv + SiLU with a ``[B, C, K]`` state) and
 the gated RMS norm (``FusedRMSNormGated(activation="sigmoid", eps=1e-5)``, the module the
