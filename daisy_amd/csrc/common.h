@@ -136,9 +136,31 @@ __device__ __forceinline__ float group_sum(float x) {
 // gbase + byte_off at LDS address lds_addr + 16*i.  gbase and lds_addr are wavefront-uniform.
 // Issued as inline assembly so that the compiler does not serialise later LDS reads of the
 // OTHER buffer behind it; the caller waits with s_waitcnt vmcnt(0) before publishing the tile.
+template <bool STREAMED = false>
 __device__ __forceinline__ void copy16_to_lds_async(const uint16_t* gbase, int byte_off, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(byte_off), "s"(gbase), "s"(lds_addr) : "memory");
+  if (STREAMED)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" :: "v"(byte_off), "s"(gbase), "s"(lds_addr) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(byte_off), "s"(gbase), "s"(lds_addr) : "memory");
+}
+// N KiB in a row: the instruction's offset moves the global and the LDS address alike, four copies per address.
+template <int N>
+__device__ __forceinline__ void copy_kib_to_lds_async(const char* gbase, int byte_off, uint32_t lds_addr) {
+  if constexpr (N >= 4) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %0, %1 offset:2048\n\tglobal_load_lds_dwordx4 %0, %1 offset:3072"
+                 :: "v"(byte_off), "s"(gbase), "s"(lds_addr) : "memory");
+    if constexpr (N > 4) copy_kib_to_lds_async<N - 4>(gbase + 4096, byte_off, lds_addr + 4096);
+  } else if constexpr (N == 3) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %0, %1 offset:2048"
+                 :: "v"(byte_off), "s"(gbase), "s"(lds_addr) : "memory");
+  } else if constexpr (N == 2) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024"
+                 :: "v"(byte_off), "s"(gbase), "s"(lds_addr) : "memory");
+  } else {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(byte_off), "s"(gbase), "s"(lds_addr) : "memory");
+  }
 }
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(size_t)(__attribute__((address_space(3))) const void*)p;

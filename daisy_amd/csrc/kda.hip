@@ -72,31 +72,30 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 //
 // kda_prep_kernel (all chunks in parallel) produces everything that depends on neither S0 nor V, one block of
 // KdaBlob<KD>::kBytes per chunk, laid out as the other kernel wants it in LDS:
-//   Kg  = -exp(G) (.) K             bf16 [32][KD]   contraction index (channel) permuted
-//   Qg  = scale exp(G) (.) Q        bf16 [32][KD]   channel permuted
-//   Mh + Ml = (exp(G_last - G) (.) K)^T T split into two bf16 terms, [KD][32], column (position) permuted
-//   Ph + Pl = scale tril(P) T       the same, [32][32]
+//   Kg  = -exp(G) (.) K             bf16 [32][KD]
+//   Qg  = scale exp(G) (.) Q        bf16 [32][KD]
+//   Mh + Ml = (exp(G_last - G) (.) K)^T T split into two bf16 terms, [KD][32]: rows in the order of the state's tiles, columns
+//                                   (positions) permuted
+//   Ph + Pl = scale tril(P) T       the same, [32][32], columns permuted
 //   dec = exp(G_last)               fp32 [KD]
 // kda_state_kernel (one workgroup per (batch, head, 32 value columns)) then walks the chunks in order with the fp32
 // state in registers; every product in it is a v_mfma_f32_16x16x32_bf16 whose B operand is an accumulator (S0 or X)
 // converted to bf16 in place: in the 16x16 accumulator layout lane l holds column l%16 and rows 4*(l/16)+r of each
-// tile, so two stacked tiles give the lane 8 contraction indices 16*t + 4*(l/16) + r (t = 0,1; r = 0..3).  The A
-// operands are stored with their contraction index permuted inside every aligned group of 32 (perm32) so that those 8
-// indices are 8 consecutive elements, one 16-byte load.
+// tile, so two stacked tiles give the lane 8 contraction indices, (t, r) with t = 0,1; r = 0..3.  The state's tiles 2 m and 2 m + 1
+// hold channels 32 m + 8 (row/4) + 4 t + row%4, so that a lane's eight are neighbours and one 16-byte piece of Kg or Qg as they
+// are; X's tiles hold positions 16 t + 4 (row/4) + row%4, and M and P are stored with their columns permuted to match.
 //
-// What bounds it.  The first kernel moves bytes, with the conversions in between: 1.29 GB (673 MB of inputs, 612 MB of blocks)
-// in 217 us at B4 T8192 H16 (5.9 TB/s);
-// with chunks of 64 and W = T K, U0 = T V in the workspace (107 KB per 64 positions, from a solve with 256 right-hand
-// sides) it took 355 us.  The second kernel is a serial chain of chunks, bound by the latency of a link: folding T into
-// the two matrices above takes a product and a conversion out of it, and chunks of 32 let three stages of everything the
-// chain needs fit the LDS, so that no computing wavefront waits for global memory (those loads alone were 90 us of 284).
-// It takes 230 us at that size, 0.9 us per chunk; 165 us of them remain without the copies into the LDS.
+// What bounds it.  Of the first kernel, at B4 T8192 H16 with fp32 log-decays, memory: 1.29 GB (673 MB of inputs, 612 MB of blocks) in
+// 222 us; otherwise its vector instructions and their latency.  The second is a serial chain of chunks; what sets the time of a
+// link is not the chain itself (without it the kernel is as fast) but its 39 KB of operands: a compute unit has about 64 KB
+// of requests in flight, 62 GB/s from memory (160 GB/s if they are in the L2).  0.55 us a link at B1 T8192 with 4 heads of
+// 128 (0.75 before the data-moving wavefronts were written as below), 0.4 us with 4 heads of 64 (0.63), 0.87 us with 64 of
+// 128 (0.89), where all compute units ask at once.
 //
 // Numerics: the 16x16 blocks of A and P run on MFMA with both operands referenced to the row before the block (every
 // exponent <= 0 off the diagonal); a diagonal block whose total decay exceeds exp(-80) is referenced to its middle row
-// instead (exponents up to the decay of 8 rows either way), when those go beyond exp(-80) to four rows in four passes, and
-// when four rows do, it is accumulated in fp32 pair by pair with exp(G_i - G_j), j < i (no exponent is ever positive, so
-// strong decays cannot overflow).
+// instead (exponents up to the decay of 8 rows either way); when those go beyond exp(-80) it is taken by halves, of 8, 4, 2 and
+// 1 rows, in two-term bf16 splits: no exponent is ever positive, so strong decays cannot overflow.
 // T is computed in fp32; the products with T, the state update and the output's second term use two-term bf16 splits of
 // both operands (three MFMAs each, relative error ~2^-17), which keeps the state error near fp32.
 // ===========================================================================
@@ -104,11 +103,13 @@ constexpr int KC = 32;    // chunk length
 constexpr int KDMAX = 128;
 constexpr int KVS = 16;   // value columns per state wavefront
 
-// One chunk's block in the workspace: byte offsets of its parts; rows of 16-byte pieces XOR-swizzled (below).
+// One chunk's block in the workspace: byte offsets of its parts (first what the chain reads, then what the outputs read);
+// rows of 16-byte pieces XOR-swizzled (below).
 template <int KD> struct KdaBlob {
-  static constexpr int kKg = 0, kQg = KC * KD * 2, kMh = 2 * KC * KD * 2, kMl = 3 * KC * KD * 2;
-  static constexpr int kPh = 4 * KC * KD * 2, kPl = kPh + KC * KC * 2, kDec = kPl + KC * KC * 2;
-  static constexpr int kBytes = (kDec + KD * 4 + 1023) & ~1023;     // whole 1 KiB copies
+  static constexpr int kKg = 0, kMh = KC * KD * 2, kMl = 2 * KC * KD * 2, kDec = 3 * KC * KD * 2;
+  static constexpr int kChain = (kDec + KD * 4 + 1023) & ~1023;      // whole 1 KiB copies
+  static constexpr int kQg = kChain, kPh = kQg + KC * KD * 2, kPl = kPh + KC * KC * 2;
+  static constexpr int kBytes = kPl + KC * KC * 2, kOut = kBytes - kChain;
 };
 static_assert(KdaBlob<128>::kBytes == 37 * 1024 && KdaBlob<64>::kBytes == 21 * 1024, "");
 // Swizzle of a row's 16-byte pieces: the 16 lanes that a 16-byte LDS read serves together must fall into 16 different slots
@@ -230,20 +231,15 @@ __global__ __launch_bounds__(256) void kda_chunk_table_kernel(const int32_t* cu,
   if (tid == 255) seq_chunk0[n_seq] = min(run, nc_max);   // the last thread's run ends at the total
 }
 
-// Stored position of contraction index x inside its aligned group of 32: bits (4,3,2) -> (3,2,4).
-__host__ __device__ constexpr int perm32(int x) { return (x & ~0x1c) | ((x & 0x0c) << 1) | ((x & 0x10) >> 2); }
-__host__ __device__ constexpr int perm32_inv(int p) { return (p & ~0x1c) | ((p & 0x18) >> 1) | ((p & 0x04) << 2); }
-
 __device__ __forceinline__ f32x4 lds_f4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
-// A float as two bf16 terms (value = hi + lo up to 2^-17 relative).
-__device__ __forceinline__ void split_bf16(float x, float& hi, float& lo) { hi = round_bf16(x); lo = x - hi; }
-// Eight floats as two 16-byte pieces of bf16 terms.
+// Eight floats as two 16-byte pieces of bf16 terms (value = hi + lo up to 2^-17 relative).
 __device__ __forceinline__ void split_pack8(const float* x, u32x4& hi, u32x4& lo) {
   float h[8], l[8];
+  hi = pack8(x);
+  unpack8(hi, h);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) split_bf16(x[e], h[e], l[e]);
-  hi = pack8(h);
+  for (int e = 0; e < 8; ++e) l[e] = x[e] - h[e];
   lo = pack8(l);
 }
 // LDS writes of a wavefront before this point are seen by all of its lanes after it.
@@ -251,406 +247,350 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
-__device__ __forceinline__ uint32_t dpp_xor2(uint32_t x) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, false); }
 
-// A workgroup makes two neighbouring chunk slots (64 rows; they may belong to different sequences).
-template <int KD>
-__global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaParams p) {
+typedef __attribute__((address_space(3))) const char* lds_cptr;
+__device__ __forceinline__ bf16x8 lds_bf16x8(lds_cptr p) {
+  return __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)p);
+}
+__device__ __forceinline__ f32x4 lds_f32x4(lds_cptr p) { return *(const f32x4 __attribute__((address_space(3)))*)p; }
+// LDS transpose read: inside a block of 16 lanes that address, lane i, row i / 4 and columns 4 (i % 4) .. + 3 of a bf16
+// tile, lane i receives column i of the four rows.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x2 lds_column4(lds_cptr p) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)p));
+}
+// The value that another lane of the same 16 holds: lane N of them, or by a pattern inside every quad.
+template <int CTRL> __device__ __forceinline__ float dpp_move(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int N> __device__ __forceinline__ float from_row(float x) { return dpp_move<0x150 + N>(x); }
+__device__ __forceinline__ float sum_over_q4(float x) {       // over the four lanes that share a row of an operand
+  x += __shfl_xor(x, 16);
+  return x + __shfl_xor(x, 32);
+}
+
+// 16 bytes of a block of the workspace, past the caches or into them.
+template <bool STREAMED> __device__ __forceinline__ void store_piece(const u32x4& v, char* to) {
+  if (STREAMED) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(to));
+  else *reinterpret_cast<u32x4*>(to) = v;
+}
+
+// A workgroup makes one chunk, a wavefront one block of 16 rows.  Everything a wavefront does before the triangle's inverse
+// it does in the layout of a matrix operand: lane (row li, q4) holds channels 32 m + 8 q4 + e of its row, of k, of q and of
+// the running log-decay.  The running sum comes in that layout from a product with a triangle of ones on the fp32 matrix
+// instructions (left operand: channels, straight from memory, two of them per load), so g passes through neither LDS nor
+// vector instructions; it is the sum inside the wavefront's own 16 rows, which is the reference the block's products want.
+// Each factor is then one exponential per element for everything it is needed for, and rows 3, 7, 11, 15 that serve as
+// references are lane moves.  Two chunks per workgroup with sums, norms, block rows and operands each in a layout of their own and
+// exponentials taken anew for each were bound by their vector instructions, 27000 cycles per 64 rows: with the layer's log-decays
+// (bf16, half of the diagonal blocks steep) B4 T8192 H16 took 292 us and takes 203, T = 777 of 8 heads 24.5 and 12.
+// *Tried:* both kernels in one launch, two of these wavefronts beside the chain's and blocks shared by flags through the L2: a
+// wavefront alone needs 15000 cycles per block, 2 us a link.  *Tried:* the running sum by adds across lanes (fewer instructions, one
+// more round through the LDS for g): the same time.
+template <int KD, bool STREAMED>
+__global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   using Blob = KdaBlob<KD>;
-  constexpr int CPR = KD / 8, RPP = 256 / CPR, NP = 64 / RPP;         // 16-byte pieces per row, rows per pass, passes
-  constexpr int NM = KD / 32;                                         // contraction groups of 32 channels
-  __shared__ __attribute__((aligned(16))) float G[64][KD + 4];        // inclusive running log-decay (rows 4 banks apart: 16 rows read side by side do not collide)
-  __shared__ __attribute__((aligned(16))) uint16_t Kr[64][KD + 8];    // k as given (bf16)
-  __shared__ __attribute__((aligned(16))) uint16_t Qr[64][KD + 8];    // q as given
-  __shared__ __attribute__((aligned(16))) float Ad[4][16][16];        // diagonal blocks of A, [block][column j][row i]
-  __shared__ __attribute__((aligned(16))) float Ao[2][16][20];        // the block A_10 of either chunk, [row][column]
-  __shared__ __attribute__((aligned(16))) float Td[4][16][20];        // (I + A_II)^-1, [block][row][column]
-  __shared__ __attribute__((aligned(16))) float rk[64], rq[64], bt[64];   // 1/|k|, 1/|q|, beta (0 for padded rows)
-  __shared__ int steep[4];      // per 16-row block: decay beyond exp(-80) over all of it (1), over 8 of its rows (2), over 4 (3)
+  constexpr int NM = KD / 32, ROW = 2 * KD;                           // contraction groups of 32 channels, bytes of a bf16 row
+  // rows[0] / rows[1]: k / q as given; then Kg / Qg on their way out; then the two terms of exp(G_last - G) k.  A
+  // wavefront's 16 rows are its own until the last use.
+  __shared__ __attribute__((aligned(1024))) char rows[2][KC * ROW];
+  __shared__ __attribute__((aligned(16))) char kcol[16 * ROW];        // the first block's columns for block (1, 0)
+  __shared__ __attribute__((aligned(16))) float Et[2][KD];            // decay of either block of 16 rows
+  __shared__ __attribute__((aligned(16))) float Td[2][16][20];        // first A_II as [column j][row i] of 16 x 16, then (I + A_II)^-1 as [row][column]
+  __shared__ __attribute__((aligned(16))) float Ao[16][20];           // A_10, [row][column]
+  __shared__ __attribute__((aligned(16))) float bt[KC], rks[KC];      // beta (0 for padded rows), 1 / |k|
 
   const int h = blockIdx.y;
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  // First token row and live rows of the two chunks.  A slot without a chunk has no live rows and is not stored; its
-  // loads go to the first chunk's first row.
-  int t0[2], n_live[2];
-  int64_t ci[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int slot = 2 * blockIdx.x + c;
-    t0[c] = 0;
-    n_live[c] = 0;
-    int gc = slot;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, q4 = lane >> 4;
+  const int I = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int t0, n_live;
+  int64_t ci;
+  {
+    const int slot = blockIdx.x;
     if (p.n_seq > 0) {
       int rows_end;
       const SeqSpan sp = packed_span(p, slot, true, rows_end);
-      if (sp.nc > 0) {
-        t0[c] = sp.tok0 + (slot - sp.c0) * KC;
-        n_live[c] = min(sp.tok_end - t0[c], KC);
-      }
+      if (sp.nc == 0) return;                    // surplus slots (the grid covers the upper bound)
+      t0 = sp.tok0 + (slot - sp.c0) * KC;
+      n_live = min(sp.tok_end - t0, KC);
+      ci = (int64_t)h * p.nc_total + slot;
     } else {
-      gc = blockIdx.z * p.NC + slot;
-      if (slot < p.NC) {
-        t0[c] = blockIdx.z * p.T + slot * KC;
-        n_live[c] = min((int)(blockIdx.z + 1) * p.T - t0[c], KC);
-      }
+      t0 = blockIdx.z * p.T + slot * KC;
+      n_live = min((int)(blockIdx.z + 1) * p.T - t0, KC);
+      ci = (int64_t)h * p.nc_total + blockIdx.z * p.NC + slot;
     }
-    if (c == 0 && n_live[0] <= 0) return;      // surplus slots (the grid covers the upper bound)
-    if (n_live[c] <= 0) { t0[c] = t0[0]; n_live[c] = 0; }
-    ci[c] = (int64_t)h * p.nc_total + gc;
   }
-  // Addresses: a wavefront-uniform 64-bit base per array and chunk plus a 32-bit offset per lane.
-  const uint32_t row_stride = (uint32_t)p.H * (uint32_t)p.Dk;     // elements between token rows of one head (q, k, g)
-  const int64_t tok_base[2] = {((int64_t)t0[0] * p.H + h) * p.Dk, ((int64_t)t0[1] * p.H + h) * p.Dk};
-  char* const blob[2] = {p.blobs + ci[0] * Blob::kBytes, p.blobs + ci[1] * Blob::kBytes};
+  const bool edge = n_live < KC || p.Dk < KD;     // rows or channels that do not exist: read as copies of others, then zeroed
+  const uint32_t row_stride = (uint32_t)p.H * (uint32_t)p.Dk;         // elements between token rows of one head (q, k, g)
+  const int64_t tok_base = ((int64_t)t0 * p.H + h) * p.Dk;
+  char* const blob = p.blobs + ci * Blob::kBytes;
 
-  // ---- phase 0a: G = cumsum(g) -----------------------------------------------
-  // Every global load of the chunks (g here, then q, k and beta of phase 0b) goes out before the first result is used,
-  // so that the memory latency is paid once.  Inputs are read once and the workspace is written once: both as streaming
-  // (non-temporal) accesses.
-  if (tid < 4) steep[tid] = 0;
-  __syncthreads();
-  const int cc = tid % CPR, r4 = tid / CPR;
-  u32x4 qraw[NP], kraw[NP];
-  float btv[NP];
-  constexpr int GR = 64 * KD / 256;               // rows of one channel per thread: a whole chunk (128) or half of one (64)
+  // ---- every global load goes out at once: g as left operand, k and q rows into the LDS (swizzled), beta ----
+  // g: tile t of group m holds channels 32 m + 8 (row / 4) + 2 (row % 4) + t, so that a lane's two tiles are neighbours and the
+  // product's rows 4 q4 + r are channels 8 q4 + 2 r + t; contraction step s: position 4 s + q4 of the block.
+  const int last = n_live - 1;
+  u32x2 graw[NM][4];
   {
-    const int d = tid % KD, part = __builtin_amdgcn_readfirstlane(tid / KD);   // the row of a g load is wavefront-uniform
-    const int c = part * GR / KC, row0 = part * GR % KC;
-    const bool d_live = d < p.Dk;                 // channels beyond Dk read as zero (their loads re-read the last channel)
-    const int dl = min(d, p.Dk - 1);
-    // Rows past the end re-read the last row (always valid) and are zeroed afterwards, so that the loads carry no
-    // branches and all go out together; the dtype is decided once, outside the loops, for the same reason.  bf16 g: the
-    // two channels of a pair read the same dword (no sub-dword loads) and take their half.
-    const int last = max((c ? n_live[1] : n_live[0]) - 1, 0), live = c ? n_live[1] : n_live[0];
-    const int64_t base = c ? tok_base[1] : tok_base[0];
-    uint32_t graw[GR];
-    if (p.g_bf16) {
+    const int ch = 8 * (li >> 2) + 2 * (li & 3);
 #pragma unroll
-      for (int i = 0; i < GR; ++i) {
-        const uint32_t* row = reinterpret_cast<const uint32_t*>(p.g) + ((base + (uint32_t)min(row0 + i, last) * row_stride) >> 1);
-        graw[i] = __builtin_nontemporal_load(row + (uint32_t)(dl >> 1));
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < GR; ++i) {
-        const uint32_t* row = reinterpret_cast<const uint32_t*>(p.g) + (base + (uint32_t)min(row0 + i, last) * row_stride);
-        graw[i] = __builtin_nontemporal_load(row + (uint32_t)dl);
-      }
-    }
-    const int ccl = min(cc, p.Dk / 8 - 1);
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int r = r4 + RPP * i, rc = r >> 5;    // (a pass of 16 or 32 rows lies inside one chunk)
-      const uint32_t row = (uint32_t)min(r & 31, max((rc ? n_live[1] : n_live[0]) - 1, 0));
-      const int64_t at = (rc ? tok_base[1] : tok_base[0]) + row * row_stride + 8u * ccl;
-      kraw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.k + at));
-      qraw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.q + at));
-      btv[i] = p.beta[(int64_t)((rc ? t0[1] : t0[0]) + row) * p.H + h];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    float gv[GR];
-    const bool g16 = p.g_bf16 != 0, odd = (d & 1) != 0;
-#pragma unroll
-    for (int i = 0; i < GR; ++i) {
-      const float x = g16 ? (odd ? bf16hi_to_f32(graw[i]) : bf16lo_to_f32(graw[i])) : __uint_as_float(graw[i]);
-      gv[i] = (row0 + i < live && d_live) ? x : 0.f;
-    }
-    // G holds the running sum in units of log 2 (g * log2(e)): every exponential below is a bare v_exp_f32.
-    float acc = 0.f;
-#pragma unroll
-    for (int i = 0; i < GR; ++i) {
-      acc += gv[i] * kLog2e;
-      G[part * GR + i][d] = acc;
-    }
-#pragma unroll
-    for (int blk = 0; blk < GR / 16; ++blk) {
-      float t4[4];
-#pragma unroll
-      for (int f = 0; f < 4; ++f) t4[f] = gv[16 * blk + 4 * f] + gv[16 * blk + 4 * f + 1] + gv[16 * blk + 4 * f + 2] + gv[16 * blk + 4 * f + 3];
-      const float lo = t4[0] + t4[1], hi = t4[2] + t4[3];
-      if (__any(lo + hi < -80.f)) {
-        const bool four = __any(fminf(fminf(t4[0], t4[1]), fminf(t4[2], t4[3])) < -80.f), eight = __any(fminf(lo, hi) < -80.f);
-        if ((tid & 63) == 0) atomicMax(&steep[part * GR / 16 + blk], four ? 3 : eight ? 2 : 1);
-      }
-    }
-    if constexpr (GR < KC) {                      // the second half of a chunk continues from the first
-      __syncthreads();
-      if (row0 != 0) {
-        const float add = G[part * GR - 1][d];
-#pragma unroll
-        for (int i = 0; i < GR; ++i) G[part * GR + i][d] += add;
-      }
-    }
-  }
-
-  // ---- phase 0b: raw q, k to LDS, row norms, beta ---------------------------
-  float rkv[NP], rqv[NP];
-#pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int r = r4 + RPP * i;
-    const bool live = (r & 31) < ((r >> 5) ? n_live[1] : n_live[0]);
-    const u32x4 zero4 = {0, 0, 0, 0};
-    if (!live || 8 * cc >= p.Dk) { kraw[i] = zero4; qraw[i] = zero4; }
-    float kf[8], qf[8];
-    unpack8(kraw[i], kf);
-    unpack8(qraw[i], qf);
-    float sk = 0.f, sq = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { sk = fmaf(kf[e], kf[e], sk); sq = fmaf(qf[e], qf[e], sq); }
-    sk = group_sum<CPR>(sk);
-    sq = group_sum<CPR>(sq);
-    rkv[i] = p.l2norm ? rsqrtf(sk + p.l2eps) : 1.f;
-    rqv[i] = p.l2norm ? rsqrtf(sq + p.l2eps) : 1.f;
-    if (cc == 0) {
-      rk[r] = rkv[i];
-      rq[r] = rqv[i];
-      bt[r] = live ? btv[i] : 0.f;
-    }
-    *reinterpret_cast<u32x4*>(&Kr[r][8 * cc]) = kraw[i];
-    *reinterpret_cast<u32x4*>(&Qr[r][8 * cc]) = qraw[i];
-  }
-  __syncthreads();
-
-  // ---- phase 1: Kg = -exp(G) k/|k|, Qg = scale exp(G) q/|q| (channel permuted), dec = exp(G_last) ----
-  {
-    // The stored 16-byte piece a of a group of 32 channels holds channels 4a..+3 and 16 + 4a..+3: lanes cc and cc ^ 2 each
-    // own half of two pieces and swap one half.
-    const int b2 = cc & 3;
-    const bool low = b2 < 2;
-    const int piece = (cc & ~3) + 2 * (b2 & 1) + (low ? 0 : 1);
-    auto join = [&](const u32x4& pk) -> u32x4 {
-      const uint32_t s0 = low ? pk.z : pk.x, s1 = low ? pk.w : pk.y;
-      const uint32_t x0 = dpp_xor2(s0), x1 = dpp_xor2(s1);
-      return low ? u32x4{pk.x, pk.y, x0, x1} : u32x4{x0, x1, pk.z, pk.w};
-    };
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int r = r4 + RPP * i, rc = r >> 5, row = r & 31;
-      float qf[8], kf[8], o8[8], k8[8];
-      unpack8(qraw[i], qf);
-      unpack8(kraw[i], kf);
-      const f32x4 g0 = lds_f4(&G[r][8 * cc]), g1 = lds_f4(&G[r][8 * cc + 4]);
-      const float sq = p.scale * rqv[i], sk = -rkv[i];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float f = __builtin_amdgcn_exp2f(e < 4 ? g0[e & 3] : g1[e & 3]);
-        o8[e] = sq * f * qf[e];
-        k8[e] = sk * f * kf[e];
-      }
-      const uint32_t at = (uint32_t)(row * 2 * KD + 16 * (piece ^ piece_swizzle<2 * KD>(row)));
-      const u32x4 kp = join(pack8(k8)), qp = join(pack8(o8));
-      if (rc == 0 || n_live[1] > 0) {
-        char* dst = (rc ? blob[1] : blob[0]) + at;
-        __builtin_nontemporal_store(kp, reinterpret_cast<u32x4*>(dst + Blob::kKg));
-        __builtin_nontemporal_store(qp, reinterpret_cast<u32x4*>(dst + Blob::kQg));
-      }
-    }
-    if (tid < 2 * KD / 4) {
-      const int c = tid / (KD / 4), d4 = 4 * (tid % (KD / 4));
-      const f32x4 gl = lds_f4(&G[KC * c + KC - 1][d4]);
-      f32x4 dv;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dv[e] = __builtin_amdgcn_exp2f(gl[e]);
-      if (c == 0 || n_live[1] > 0) *reinterpret_cast<f32x4*>((c ? blob[1] : blob[0]) + Blob::kDec + 4 * d4) = dv;
-    }
-  }
-
-  // ---- phase 2: 16x16 blocks of A and P on MFMA --------------------------------
-  // Block rows bi = 0..3 of the 64 rows (chunk bi / 2, I = bi % 2).  Block (I, J), J <= I: both operands are referenced to
-  // the row before block I (the chunk's start for I = 0: G_ref = 0), so the row factor exp(G_i - G_ref) is <= 1 and, for J < I,
-  // so is the column factor exp(G_ref - G_j).  For a diagonal block (J == I) the column factor grows to exp(total decay
-  // of the block); beyond exp(80) the block's middle row is the reference, each factor then growing to the decay of 8 rows
-  // (four passes took 60 us more per 32768 rows of 16 heads with the decays of a freshly initialised layer).
-  // Wavefront w takes block row w: its diagonal block and, in the second block row of a chunk, block (1, 0).
-  const int li = lane & 15, q4 = lane >> 4;
-  const int chunk = wave >> 1, I = wave & 1;
-  const int ri = 16 * wave + li;
-  char* const my_blob = chunk ? blob[1] : blob[0];
-  const bool stored = chunk == 0 || n_live[1] > 0;
-  bf16x8 va[NM], vq[NM];
-  // Row operands k_i f_i, q_i f_i with f_i = exp(G_i - G_ref(i)); `ref` is the lane's reference row (-1: G_ref = 0).
-  auto row_operands = [&](int ref) {
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      const int d0 = 32 * m + 8 * q4;
-      float ki[8], qi[8], ak[8], aq[8];
-      unpack8(*reinterpret_cast<const u32x4*>(&Kr[ri][d0]), ki);
-      unpack8(*reinterpret_cast<const u32x4*>(&Qr[ri][d0]), qi);
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        const f32x4 gi = lds_f4(&G[ri][d0 + 4 * hf]);
-        const f32x4 gr = (ref >= 0) ? lds_f4(&G[max(ref, 0)][d0 + 4 * hf]) : zero;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float fi = __builtin_amdgcn_exp2f(gi[e] - gr[e]);
-          ak[4 * hf + e] = ki[4 * hf + e] * fi;
-          aq[4 * hf + e] = qi[4 * hf + e] * fi;
-        }
-      }
-      va[m] = __builtin_bit_cast(bf16x8, pack8(ak));
-      vq[m] = __builtin_bit_cast(bf16x8, pack8(aq));
-    }
-  };
-  // This wavefront's rows of scale tril(P), as a product's operand wants them: row 16 I + li, columns 4 q4 + r of either
-  // column block.
-  f32x4 P[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  auto mfma_block = [&](int J, int ref) {
-    const int rj = 32 * chunk + 16 * J + li;
-    f32x4 accA = {0.f, 0.f, 0.f, 0.f}, accP = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      const int d0 = 32 * m + 8 * q4;
-      float kj[8], bk[8];
-      unpack8(*reinterpret_cast<const u32x4*>(&Kr[rj][d0]), kj);
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        const f32x4 gj = lds_f4(&G[rj][d0 + 4 * hf]);
-        const f32x4 gr = (ref >= 0) ? lds_f4(&G[max(ref, 0)][d0 + 4 * hf]) : zero;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bk[4 * hf + e] = kj[4 * hf + e] * __builtin_amdgcn_exp2f(gr[e] - gj[e]);
-      }
-      const bf16x8 vb = __builtin_bit_cast(bf16x8, pack8(bk));
-      accA = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[m], vb, accA, 0, 0, 0);
-      // P comes out transposed (operands swapped: both operand layouts hold 8 contraction indices of
-      // one row / column per lane): a lane then owns four consecutive columns of one row of P.
-      accP = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb, vq[m], accP, 0, 0, 0);
-    }
-    // accA: lane holds column j = 16J + li, rows i = 16I + 4*q4 + r
-    const float rkj = rk[rj];
-    f32x4 av;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 16 * wave + 4 * q4 + r;
-      av[r] = bt[i] * rk[i] * rkj * accA[r];
-    }
-    {
-      // accP: lane holds row i = 16I + li, columns j = 16J + 4*q4 + r
-      const int ip = 16 * I + li, jp = 16 * J + 4 * q4;
-      const f32x4 rk4 = lds_f4(&rk[32 * chunk + jp]);
-      const float qs = p.scale * rq[ri];
-      f32x4 pv;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pv[r] = (jp + r <= ip) ? qs * rk4[r] * accP[r] : 0.f;
-      if (J == 0) P[0] = pv; else P[1] = pv;
-    }
-    if (I == J) {
-      *reinterpret_cast<f32x4*>(&Ad[wave][li][4 * q4]) = av;   // entries with i <= j are never read
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) Ao[chunk][4 * q4 + r][li] = av[r];
-    }
-  };
-  // A diagonal block whose decay is too steep for the MFMA path even with a reference row per four rows is accumulated
-  // in fp32 pair by pair with exp(G_i - G_j), j < i, where no exponent is ever positive.
-  auto steep_diagonal = [&]() {
-    const int il = lane >> 2, dq = lane & 3;
-    const int rr = 16 * wave + il;
-    float a[16], pp[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) { a[j] = 0.f; pp[j] = 0.f; }
-#pragma unroll 1
-    for (int dc = 0; dc < KD / 32; ++dc) {
-      const int d0 = (KD / 4) * dq + 8 * dc;
-      float ki[8], qi[8];
-      unpack8(*reinterpret_cast<const u32x4*>(&Kr[rr][d0]), ki);
-      unpack8(*reinterpret_cast<const u32x4*>(&Qr[rr][d0]), qi);
-      const f32x4 gi0 = lds_f4(&G[rr][d0]), gi1 = lds_f4(&G[rr][d0 + 4]);
-#pragma unroll
-      for (int j = 15; j >= 0; --j) {
-        const int rj = 16 * wave + j;
-        float kj[8];
-        unpack8(*reinterpret_cast<const u32x4*>(&Kr[rj][d0]), kj);
-        // exp(G_i - G_j) for j < i: the exponent is a sum of log-decays, never positive; rows at or
-        // above the diagonal take the factor 1 (only j == i is used, by P).
-        const f32x4 gj0 = lds_f4(&G[rj][d0]), gj1 = lds_f4(&G[rj][d0 + 4]);
-        const bool below = j < il;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float diff = (e < 4) ? gi0[e & 3] - gj0[e & 3] : gi1[e & 3] - gj1[e & 3];
-          const float t = kj[e] * (below ? __builtin_amdgcn_exp2f(diff) : 1.f);
-          a[j] = fmaf(ki[e], t, a[j]);
-          pp[j] = fmaf(qi[e], t, pp[j]);
-        }
-      }
-    }
-    const float bi = bt[rr] * rk[rr], qs = p.scale * rq[rr];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      float av = dpp_add<0x4E>(dpp_add<0xB1>(a[j]));         // sum over the 4 channel quarters
-      float pv = dpp_add<0x4E>(dpp_add<0xB1>(pp[j]));
-      const float rkj = rk[16 * wave + j];
-      if ((j & 3) == dq && j < il) Ad[wave][j][il] = bi * rkj * av;
-      if ((j & 3) == dq) Td[wave][il][j] = (j <= il) ? qs * rkj * pv : 0.f;   // (on the way to the operand layout)
-    }
-    wave_lds_fence();
-    if (I == 0) P[0] = lds_f4(&Td[wave][li][4 * q4]); else P[1] = lds_f4(&Td[wave][li][4 * q4]);
-    wave_lds_fence();
-  };
-  // A steep diagonal block on the matrix cores after all: with one reference row per group of four
-  // rows (the row before the group) every row factor exp(G_i - G_ref(i)) is <= 1, and the column
-  // factors exp(G_ref - G_j) are <= 1 for columns of earlier groups and at most the decay of four
-  // rows inside the group.  Pass r multiplies all rows by the columns scaled for the reference of
-  // group r; the accumulator layout gives rows 4r..4r+3 (A) resp. the lanes of those rows (P, transposed) that pass's result.
-  auto steep_diagonal_mfma = [&]() {
-    row_operands((I == 0 && li < 4) ? -1 : 16 * wave + (li & ~3) - 1);
-    f32x4 accA = {0.f, 0.f, 0.f, 0.f}, accP = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int r = 0; r < 4; ++r) {
-      const int ref = (I == 0 && r == 0) ? -1 : 16 * wave + 4 * r - 1;
-      const bool live = (li >> 2) <= r;     // later columns are above the diagonal for every row of the group
-      f32x4 pa = {0.f, 0.f, 0.f, 0.f}, pp = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < 4; ++s) {
+      const uint32_t row = (uint32_t)min(16 * I + 4 * s + q4, last) * row_stride;
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
-        const int d0 = 32 * m + 8 * q4;
-        float kj[8], bk[8];
-        unpack8(*reinterpret_cast<const u32x4*>(&Kr[ri][d0]), kj);
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-          const f32x4 gj = lds_f4(&G[ri][d0 + 4 * hf]);
-          const f32x4 gr = (ref >= 0) ? lds_f4(&G[max(ref, 0)][d0 + 4 * hf]) : zero;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            bk[4 * hf + e] = live ? kj[4 * hf + e] * __builtin_amdgcn_exp2f(fminf(gr[e] - gj[e], 120.f)) : 0.f;
-        }
-        const bf16x8 vb = __builtin_bit_cast(bf16x8, pack8(bk));
-        pa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[m], vb, pa, 0, 0, 0);
-        pp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb, vq[m], pp, 0, 0, 0);
+        const uint32_t at = row + (uint32_t)min(32 * m + ch, p.Dk - 2);
+        if (p.g_bf16) graw[m][s].x = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>((const uint16_t*)p.g + tok_base + at));
+        else graw[m][s] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>((const float*)p.g + tok_base + at));
       }
-      if (q4 == r) accA = pa;               // rows 4 q4 .. of A
-      if ((li >> 2) == r) accP = pp;        // row li of P
     }
-    const float rkj = rk[ri];
-    f32x4 av;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 16 * wave + 4 * q4 + r;
-      av[r] = bt[i] * rk[i] * rkj * accA[r];
-    }
-    *reinterpret_cast<f32x4*>(&Ad[wave][li][4 * q4]) = av;   // entries with i <= j are never read
-    const f32x4 rk4 = lds_f4(&rk[16 * wave + 4 * q4]);
-    const float qs = p.scale * rq[ri];
-    f32x4 pv;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) pv[r] = (4 * q4 + r <= li) ? qs * rk4[r] * accP[r] : 0.f;
-    if (I == 0) P[0] = pv; else P[1] = pv;
-  };
+  }
+  const float beta = p.beta[(int64_t)(t0 + min(16 * I + li, last)) * p.H + h];
+  __builtin_amdgcn_sched_barrier(0);
+  lds_cptr const my_rows[2] = {(lds_cptr)&rows[0][16 * I * ROW], (lds_cptr)&rows[1][16 * I * ROW]};
   {
-    const int sp = __builtin_amdgcn_readfirstlane(steep[wave]), before = I ? 16 * wave - 1 : -1, middle = 16 * wave + 7;
-    if (I == 1 || sp == 0) row_operands(before);
-    if (I == 1) mfma_block(0, before);
-    if (sp == 3) steep_diagonal();
-    else if (sp == 2) steep_diagonal_mfma();
-    else {
-      // With the middle row as reference the entries above the diagonal may overflow; nothing reads them.
-      if (sp == 1) row_operands(middle);
-      mfma_block(I, sp == 1 ? middle : before);
+    constexpr int RPI = 1024 / ROW, PPR = ROW / 16;                   // rows per copy, pieces per row
+#pragma unroll
+    for (int j = 0; j < 16 / RPI; ++j) {
+      const int r = RPI * j + lane / PPR, piece = (lane % PPR) ^ piece_swizzle<ROW>(r);
+      const int off = 2 * (int)((uint32_t)min(16 * I + r, last) * row_stride + 8u * (uint32_t)min(piece, p.Dk / 8 - 1));
+      copy16_to_lds_async<true>(p.k + tok_base, off, (uint32_t)(size_t)my_rows[0] + 1024 * j);
+      copy16_to_lds_async<true>(p.q + tok_base, off, (uint32_t)(size_t)my_rows[1] + 1024 * j);
     }
   }
 
-  // ---- phase 3: T = (I + A)^-1 diag(beta).  The inverse of diagonal block `wave` in fp32, one column per lane (lanes
+  // ---- G: running log-decay inside the block, in units of log 2; element e of group m is G[m][e % 2][e / 2] ----
+  f32x4 G[NM][2];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) G[m][0] = G[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const float ones = (4 * s + q4 <= li) ? kLog2e : 0.f;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      float g0 = p.g_bf16 ? bf16lo_to_f32(graw[m][s].x) : __uint_as_float(graw[m][s].x);
+      float g1 = p.g_bf16 ? bf16hi_to_f32(graw[m][s].x) : __uint_as_float(graw[m][s].y);
+      if (edge && (16 * I + 4 * s + q4 >= n_live || 32 * m + 8 * (li >> 2) >= p.Dk)) g0 = g1 = 0.f;
+      G[m][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(g0, ones, G[m][0], 0, 0, 0);
+      G[m][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g1, ones, G[m][1], 0, 0, 0);
+    }
+  }
+
+  // ---- k and q of the lane's row, and 1 over their norms ----
+  const int swz = piece_swizzle<ROW>(li);
+  int at[NM];                                     // the lane's piece of group m inside its wavefront's rows
+#pragma unroll
+  for (int m = 0; m < NM; ++m) at[m] = li * ROW + 16 * ((4 * m + q4) ^ swz);
+  __builtin_amdgcn_s_waitcnt(0x0F70);             // vmcnt(0): the wavefront's own copies have landed
+  asm volatile("" ::: "memory");
+  float kn[NM][8], qn[NM][8], sk = 0.f, sq = 0.f;
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    u32x4 kr = __builtin_bit_cast(u32x4, lds_bf16x8(my_rows[0] + at[m])), qr = __builtin_bit_cast(u32x4, lds_bf16x8(my_rows[1] + at[m]));
+    if (edge && (16 * I + li >= n_live || 32 * m + 8 * q4 >= p.Dk)) kr = qr = u32x4{0u, 0u, 0u, 0u};
+    unpack8(kr, kn[m]);
+    unpack8(qr, qn[m]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { sk = fmaf(kn[m][e], kn[m][e], sk); sq = fmaf(qn[m][e], qn[m][e], sq); }
+  }
+  // The norms (and scale) come in behind the products of k and q with their factors: where those are 1, no rounding is added.
+  const float rk = p.l2norm ? rsqrtf(sum_over_q4(sk) + p.l2eps) : 1.f;
+  const float rq = p.scale * (p.l2norm ? rsqrtf(sum_over_q4(sq) + p.l2eps) : 1.f);
+
+  // ---- factors.  How steep the block is (wavefront-uniform): 0 while exp(-G) of every element is safe (exponents up to
+  // 80), 1 while that holds with the block's middle row as reference, 2 beyond. ----
+  constexpr float kSafe = 80.f * kLog2e;
+  float far0 = 0.f;
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) far0 = fmaxf(far0, fabsf(G[m][e & 1][e >> 1]));
+  const bool gentle = !__any(far0 > kSafe);
+  // Diagonal block of A and P on MFMA.  accA: lane holds column j = li, rows i = 4 q4 + r of the block.  P comes out
+  // transposed (operands swapped: both operand layouts hold 8 contraction indices of one row / column per lane): row i = li,
+  // columns j = 4 q4 + r.
+  f32x4 accA = {0.f, 0.f, 0.f, 0.f}, accP = {0.f, 0.f, 0.f, 0.f};
+  if (!gentle) {
+    float far7 = 0.f;
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float g = G[m][e & 1][e >> 1];
+        far7 = fmaxf(far7, fabsf(g - from_row<7>(g)));
+      }
+    if (!__any(far7 > kSafe)) {
+      // With the middle row as reference the entries above the diagonal may overflow; nothing reads them.
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        float ak[8], aq[8], bk[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float g = G[m][e & 1][e >> 1], d = g - from_row<7>(g), f = __builtin_amdgcn_exp2f(d);
+          ak[e] = kn[m][e] * f;
+          aq[e] = qn[m][e] * f;
+          bk[e] = kn[m][e] * __builtin_amdgcn_exp2f(-d);
+        }
+        const bf16x8 col = __builtin_bit_cast(bf16x8, pack8(bk));
+        accA = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pack8(ak)), col, accA, 0, 0, 0);
+        accP = __builtin_amdgcn_mfma_f32_16x16x32_bf16(col, __builtin_bit_cast(bf16x8, pack8(aq)), accP, 0, 0, 0);
+      }
+    } else {
+      // Any decay: rows and columns that differ first in bit `lev` of their number meet at the last row of the lower half of
+      // their group of 2 lev rows.  The lane's row is on the row's side of that product or on the column's, never on both,
+      // so a level takes one exponential per element, of a sum of log-decays; entries of other levels are dropped.  Both
+      // operands in two bf16 terms: such blocks used to be summed in fp32 pair by pair, and lose no precision here.
+      float pd = 0.f;
+#pragma unroll
+      for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pd = fmaf(kn[m][e], qn[m][e], pd);
+      pd = sum_over_q4(pd);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) accP[r] = (4 * q4 + r == li) ? pd : 0.f;
+      auto level = [&](auto lev_, auto ref_of) {
+        constexpr int lev = decltype(lev_)::value;
+        const bool low = (li & lev) == 0;
+        f32x4 pa = {0.f, 0.f, 0.f, 0.f}, pp = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+          float wk[8], wq[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float g = G[m][e & 1][e >> 1], d = g - ref_of(g), f = __builtin_amdgcn_exp2f(low ? -d : d);
+            wk[e] = kn[m][e] * f;
+            wq[e] = qn[m][e] * f;
+          }
+          u32x4 kh, kl, qh, ql;
+          split_pack8(wk, kh, kl);
+          split_pack8(wq, qh, ql);
+          auto add = [&](const u32x4& col, const u32x4& row_k, const u32x4& row_q) {
+            pa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, row_k), __builtin_bit_cast(bf16x8, col), pa, 0, 0, 0);
+            pp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, col), __builtin_bit_cast(bf16x8, row_q), pp, 0, 0, 0);
+          };
+          add(kl, kh, qh);
+          add(kh, kl, ql);
+          add(kh, kh, qh);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int x = (4 * q4 + r) ^ li;
+          if (x >= lev && x < 2 * lev) { accA[r] = pa[r]; accP[r] = pp[r]; }
+        }
+      };
+      level(std::integral_constant<int, 8>{}, [&](float g) { return from_row<7>(g); });
+      level(std::integral_constant<int, 4>{}, [&](float g) { const float lower = from_row<3>(g), upper = from_row<11>(g); return (li & 8) ? upper : lower; });
+      level(std::integral_constant<int, 2>{}, [&](float g) { return dpp_move<0x55>(g); });        // row 1 of every quad
+      level(std::integral_constant<int, 1>{}, [&](float g) { return dpp_move<0xA0>(g); });        // the even row of every pair
+    }
+  }
+  // k f and q f with f = exp(G) take the place of k and q, kd = exp(G_15 - G) k that of G.
+  float kd[NM][8];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    float f[8], bk[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float g = G[m][e & 1][e >> 1];
+      f[e] = __builtin_amdgcn_exp2f(g);
+      if (gentle) {
+        bk[e] = kn[m][e] * __builtin_amdgcn_exp2f(-g);
+        kd[m][e] = bk[e] * from_row<15>(f[e]);
+      } else {
+        kd[m][e] = kn[m][e] * __builtin_amdgcn_exp2f(from_row<15>(g) - g);
+      }
+      kn[m][e] *= f[e];
+      qn[m][e] *= f[e];
+    }
+    if (gentle) {
+      const bf16x8 col = __builtin_bit_cast(bf16x8, pack8(bk));
+      accA = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pack8(kn[m])), col, accA, 0, 0, 0);
+      accP = __builtin_amdgcn_mfma_f32_16x16x32_bf16(col, __builtin_bit_cast(bf16x8, pack8(qn[m])), accP, 0, 0, 0);
+    }
+    if (li == 15) {
+      *reinterpret_cast<f32x4*>(&Et[I][32 * m + 8 * q4]) = f32x4{f[0], f[1], f[2], f[3]};
+      *reinterpret_cast<f32x4*>(&Et[I][32 * m + 8 * q4 + 4]) = f32x4{f[4], f[5], f[6], f[7]};
+    }
+    if (I == 0) *reinterpret_cast<u32x4*>(&kcol[at[m]]) = pack8(kd[m]);
+  }
+  if (q4 == 0) {
+    bt[16 * I + li] = (16 * I + li < n_live) ? beta : 0.f;
+    rks[16 * I + li] = rk;
+  }
+  __syncthreads();   // decays, beta and the first block's columns are in place
+
+  f32x4 P[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};          // this wavefront's rows of scale tril(P), either column block
+  {
+    const f32x4 bt4 = lds_f4(&bt[16 * I + 4 * q4]), rk4 = lds_f4(&rks[16 * I + 4 * q4]);
+    f32x4 av, pv;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      av[r] = bt4[r] * rk4[r] * rk * accA[r];     // entries with i <= j are never read
+      pv[r] = (4 * q4 + r <= li) ? rq * rk4[r] * accP[r] : 0.f;
+    }
+    *reinterpret_cast<f32x4*>(&Td[I][0][0] + 16 * li + 4 * q4) = av;
+    if (I == 0) P[0] = pv;
+    else {
+      P[1] = pv;
+      f32x4 a10 = {0.f, 0.f, 0.f, 0.f};           // block (1, 0)
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        const bf16x8 col = lds_bf16x8((lds_cptr)&kcol[0] + at[m]);
+        a10 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pack8(kn[m])), col, a10, 0, 0, 0);
+        P[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(col, __builtin_bit_cast(bf16x8, pack8(qn[m])), P[0], 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Ao[4 * q4 + r][li] = bt4[r] * rk4[r] * rks[li] * a10[r];
+      P[0] *= rq * lds_f4(&rks[4 * q4]);
+    }
+  }
+  // ---- Kg = -exp(G) k, Qg = scale exp(G) q with G from the chunk's start: through the wavefront's rows, whole KiB out ----
+  {
+    char* const kg = &rows[0][16 * I * ROW];
+    char* const qg = &rows[1][16 * I * ROW];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      if (I == 1) {
+        const f32x4 e0 = lds_f4(&Et[0][32 * m + 8 * q4]), e1 = lds_f4(&Et[0][32 * m + 8 * q4 + 4]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float f = e < 4 ? e0[e & 3] : e1[e & 3];
+          kn[m][e] *= -rk * f;
+          qn[m][e] *= rq * f;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { kn[m][e] *= -rk; qn[m][e] *= rq; }
+      }
+      *reinterpret_cast<u32x4*>(kg + at[m]) = pack8(kn[m]);
+      *reinterpret_cast<u32x4*>(qg + at[m]) = pack8(qn[m]);
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int j = 0; j < 16 * ROW / 1024; ++j) {
+      const u32x4 a = *reinterpret_cast<const u32x4*>(kg + 1024 * j + 16 * lane), b = *reinterpret_cast<const u32x4*>(qg + 1024 * j + 16 * lane);
+      store_piece<STREAMED>(a, blob + Blob::kKg + 16 * I * ROW + 1024 * j + 16 * lane);
+      store_piece<STREAMED>(b, blob + Blob::kQg + 16 * I * ROW + 1024 * j + 16 * lane);
+    }
+    wave_lds_fence();
+    if (tid < KD / 4) *reinterpret_cast<f32x4*>(blob + Blob::kDec + 16 * tid) = lds_f4(&Et[0][4 * tid]) * lds_f4(&Et[1][4 * tid]);
+  }
+  // ---- exp(G_last - G) k in two bf16 terms, for the transposing reads below ----
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    if (I == 0) {
+      const f32x4 e0 = lds_f4(&Et[1][32 * m + 8 * q4]), e1 = lds_f4(&Et[1][32 * m + 8 * q4 + 4]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) kd[m][e] *= rk * (e < 4 ? e0[e & 3] : e1[e & 3]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) kd[m][e] *= rk;
+    }
+    u32x4 hi, lo;
+    split_pack8(kd[m], hi, lo);
+    *reinterpret_cast<u32x4*>(&rows[0][16 * I * ROW + at[m]]) = hi;
+    *reinterpret_cast<u32x4*>(&rows[1][16 * I * ROW + at[m]]) = lo;
+  }
+
+  // ---- T = (I + A)^-1 diag(beta).  The inverse of the wavefront's diagonal block in fp32, one column per lane (lanes
   // 16.. repeat the work of lane & 15).
   wave_lds_fence();
   {
@@ -661,29 +601,29 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
     for (int j = 0; j < 15; ++j) {
       f32x4 ar[4];
 #pragma unroll
-      for (int i4 = (j + 1) / 4; i4 < 4; ++i4) ar[i4] = lds_f4(&Ad[wave][j][4 * i4]);
+      for (int i4 = (j + 1) / 4; i4 < 4; ++i4) ar[i4] = lds_f4(&Td[I][0][0] + 16 * j + 4 * i4);
       const float xj = tc[j];
 #pragma unroll
       for (int i = j + 1; i < 16; ++i) tc[i] = fmaf(-ar[i >> 2][i & 3], xj, tc[i]);
     }
+    wave_lds_fence();
     if (lane < 16) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) Td[wave][i][li] = tc[i];
+      for (int i = 0; i < 16; ++i) Td[I][i][li] = tc[i];
     }
   }
-  __syncthreads();   // both inverses and A_10 of either chunk are in place
-  // T_10 = -T_11 (A_10 T_00) in two fp32 matrix products, both wavefronts of a chunk all of it.  As right operand (lane
-  // (column li, rows 4 q4 + e)) and as result the layout is the same, and it is also the one T^T is wanted in below.  (As
-  // multiply-adds from LDS this took 3400 of the workgroup's 27000 cycles.)
+  __syncthreads();   // both inverses, A_10 and the rows are in place
+  // T_10 = -T_11 (A_10 T_00) in two fp32 matrix products, both wavefronts all of it.  As right operand (lane
+  // (column li, rows 4 q4 + e)) and as result the layout is the same, and it is also the one T^T is wanted in below.
   f32x4 t00, t10, t11;
   {
-    const f32x4 a10 = lds_f4(&Ao[chunk][li][4 * q4]), r11 = lds_f4(&Td[2 * chunk + 1][li][4 * q4]);
+    const f32x4 a10 = lds_f4(&Ao[li][4 * q4]), r11 = lds_f4(&Td[1][li][4 * q4]);
     f32x4 m1 = {0.f, 0.f, 0.f, 0.f};
     t10 = m1;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      t00[e] = Td[2 * chunk][4 * q4 + e][li];
-      t11[e] = Td[2 * chunk + 1][4 * q4 + e][li];
+      t00[e] = Td[0][4 * q4 + e][li];
+      t11[e] = Td[1][4 * q4 + e][li];
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) m1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a10[e], t00[e], m1, 0, 0, 0);
@@ -694,7 +634,7 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
   // 16 + 4 q4 + (e - 4) for e >= 4; two bf16 terms.
   bf16x8 th[2], tl[2];
   {
-    const float b0 = bt[32 * chunk + li], b1 = bt[32 * chunk + 16 + li];
+    const float b0 = bt[li], b1 = bt[16 + li];
     float v0[8], v1[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -713,10 +653,7 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
   }
   // Row `row` of (right operand)^T T: the products come out with four consecutive columns of T per lane and column block,
   // which is the stored piece q4 of that row; both terms of it leave from here, 16 whole rows per instruction.
-  auto times_t = [&](const float* r8, char* dst_hi, char* dst_lo, int row) {
-    u32x4 hi, lo;
-    split_pack8(r8, hi, lo);
-    const bf16x8 rh = __builtin_bit_cast(bf16x8, hi), rl = __builtin_bit_cast(bf16x8, lo);
+  auto times_t = [&](const bf16x8& rh, const bf16x8& rl, char* dst_hi, char* dst_lo, int row) {
     float out[8];
 #pragma unroll
     for (int J = 0; J < 2; ++J) {
@@ -727,34 +664,33 @@ __global__ __launch_bounds__(256, KD == 128 ? 2 : 3) void kda_prep_kernel(KdaPar
 #pragma unroll
       for (int r = 0; r < 4; ++r) out[4 * J + r] = acc[r];
     }
+    u32x4 hi, lo;
     split_pack8(out, hi, lo);
-    const int at = row * 64 + 16 * (q4 ^ piece_swizzle<64>(row));
-    if (stored) {
-      __builtin_nontemporal_store(hi, reinterpret_cast<u32x4*>(dst_hi + at));
-      __builtin_nontemporal_store(lo, reinterpret_cast<u32x4*>(dst_lo + at));
-    }
+    const int off = row * 64 + 16 * (q4 ^ piece_swizzle<64>(row));
+    store_piece<STREAMED>(hi, dst_hi + off);
+    store_piece<STREAMED>(lo, dst_lo + off);
   };
   {
     float pv[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) { pv[e] = P[0][e]; pv[4 + e] = P[1][e]; }
-    times_t(pv, my_blob + Blob::kPh, my_blob + Blob::kPl, 16 * I + li);
+    u32x4 hi, lo;
+    split_pack8(pv, hi, lo);
+    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), blob + Blob::kPh, blob + Blob::kPl, 16 * I + li);
   }
-  // ---- phase 4: M = (exp(G_last - G) k/|k|)^T T, half of the chunk's channels per wavefront
-  {
-    const f32x4 r0 = lds_f4(&rk[32 * chunk + 4 * q4]), r1 = lds_f4(&rk[32 * chunk + 16 + 4 * q4]);
+  // ---- M = (exp(G_last - G) k)^T T, half of the chunk's channels per wavefront: row 16 i + li of the block is channel
+  // 32 (i / 2) + 8 (li / 4) + 4 (i % 2) + li % 4, the one that row of the state's tile i stands for
+  const int r0 = 4 * q4 + (li >> 2);
 #pragma unroll
-    for (int i = 0; i < KD / 32; ++i) {
-      const int d = 16 * (KD / 32 * I + i) + li;
-      const float glast = G[32 * chunk + 31][d];
-      float kv[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int r = 32 * chunk + (e < 4 ? 4 * q4 + e : 12 + 4 * q4 + e);
-        kv[e] = __builtin_amdgcn_exp2f(glast - G[r][d]) * bf16lo_to_f32(Kr[r][d]) * (e < 4 ? r0[e & 3] : r1[e & 3]);
-      }
-      times_t(kv, my_blob + Blob::kMh, my_blob + Blob::kMl, d);
-    }
+  for (int n = 0; n < KD / 32; ++n) {
+    const int i = KD / 32 * I + n, piece = 4 * (i >> 1) + (li & 3), half = 8 * (i & 1);
+    const int a0 = r0 * ROW + 16 * (piece ^ piece_swizzle<ROW>(r0)) + half;     // rows 16 apart share a swizzle
+    u32x4 hi, lo;
+    const u32x2 h0 = lds_column4((lds_cptr)&rows[0][0] + a0), h1 = lds_column4((lds_cptr)&rows[0][0] + a0 + 16 * ROW);
+    const u32x2 l0 = lds_column4((lds_cptr)&rows[1][0] + a0), l1 = lds_column4((lds_cptr)&rows[1][0] + a0 + 16 * ROW);
+    hi = u32x4{h0.x, h0.y, h1.x, h1.y};
+    lo = u32x4{l0.x, l0.y, l1.x, l1.y};
+    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), blob + Blob::kMh, blob + Blob::kMl, 16 * i + li);
   }
 }
 
@@ -775,20 +711,8 @@ __device__ __forceinline__ bf16x8 pack_rest2(const f32x4& t0, const f32x4& t1, b
   return pack_acc2(l0, l1);
 }
 
-typedef __attribute__((address_space(3))) const char* lds_cptr;
-__device__ __forceinline__ bf16x8 lds_bf16x8(lds_cptr p) {
-  return __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)p);
-}
-__device__ __forceinline__ f32x4 lds_f32x4(lds_cptr p) { return *(const f32x4 __attribute__((address_space(3)))*)p; }
-// LDS transpose read: inside a block of 16 lanes that address, lane i, row i / 4 and columns 4 (i % 4) .. + 3 of a bf16
-// tile, lane i receives column i of the four rows.
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2 lds_column4(lds_cptr p) {
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)p));
-}
-
 constexpr int KCT = 2;                        // tiles of 16 value columns per workgroup
-constexpr int KPW = 4;                        // data-moving wavefronts per workgroup
+constexpr int KPW = 2;                        // data-moving wavefronts per workgroup
 constexpr int KSTAGES = 3;                    // LDS stages of chunk data
 constexpr int kStateThreads = 64 * (2 * KCT + KPW);
 
@@ -800,24 +724,23 @@ constexpr int kStateThreads = 64 * (2 * KCT + KPW);
 //    both computing X and handing state halves over through LDS, took 250 us instead of 230 (B4 T8192 H16, 128 x 128);
 //  * the outputs are not part of the chain: a second wavefront per tile makes Qg S0 of the chunk from the bf16 state
 //    the first one left in LDS, adds (P T) X when X has arrived, and stores the rows one chunk later;
-//  * neither waits for global memory: four further wavefronts issue the asynchronous copies of the chunk two ahead (the
-//    chunk's block is one linear copy of 37 or 21 KiB, V 32 rows of 64 bytes).
+//  * neither waits for global memory: two further wavefronts issue the asynchronous copies of the chunks ahead.
 template <int KD>
 __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p) {
   using Blob = KdaBlob<KD>;
   constexpr int NM = KD / 32, NS = KD / 16;                    // channel groups of 32, state tiles of 16 rows
   constexpr int kV = Blob::kBytes, kStage = Blob::kBytes + KC * KVS * KCT * 2;
-  constexpr int NCP = Blob::kBytes / 1024;
+  // Links are cut by workgroup barriers.  Interval n between two of them copies the chain's part of chunk n and the outputs'
+  // part of chunk n - 1, the chain reads its part in interval n + 2 and computes link n, beside its outputs, in interval n + 3.
   __shared__ __attribute__((aligned(1024))) char stage[KSTAGES][kStage];
   __shared__ __attribute__((aligned(16))) u32x4 xs[2][KCT][NM][64];           // [chunk parity][column tile][channel group][lane]: S0 as right operand
   __shared__ __attribute__((aligned(16))) u32x4 xx[2][KCT][2][64];            // X as right operand, two terms
   __shared__ __attribute__((aligned(16))) uint16_t ost[KCT][KC][KVS];         // output rows on their way out
 
-  // Keep the column groups of one (batch, head) on one XCD: they read the same chunk data.
-  int vid = blockIdx.x;
-  if ((gridDim.x & 7) == 0) vid = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  // The column groups of one (batch, head) on one XCD, in consecutive workgroups of it: they read the same blocks.
   const int NGRP = (p.Dv + KVS * KCT - 1) / (KVS * KCT);       // groups of 32 value columns
-  const int grp = vid % NGRP, bh = vid / NGRP;
+  const int slot = blockIdx.x >> 3, grp = slot % NGRP, bh = 8 * (slot / NGRP) + (blockIdx.x & 7);
+  if (bh >= (p.n_seq > 0 ? p.n_seq : p.B) * p.H) return;
   const int h = bh % p.H, b = bh / p.H;     // b: batch element, or sequence of a packed batch
   int rows_end;
   const SeqSpan sp = seq_span(p, b, rows_end);
@@ -825,72 +748,75 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
   const int64_t ci0 = (int64_t)h * p.nc_total + sp.c0;
   const int lane = threadIdx.x & 63, ln = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const char* const my_blobs = p.blobs + ci0 * Blob::kBytes;
+  const int ct = wave & 1;                   // chain 0, 1; outputs 2, 3; data 4, 5
 
-  if (wave >= 2 * KCT) {
+  if (wave >> 1 == 2) {
     // ================= data-moving wavefront =================
-    const int pw = wave - 2 * KCT;
+    // Their instructions count: with an address, a branch and an m0 of its own for every KiB (some 250 scalar instructions
+    // per chunk) these wavefronts set the time of a link.  So each takes a run of the chain's part and one of the outputs' part,
+    // KiB after KiB by the instruction's own offset, the KiB with the decays (both of them, the same bytes) and 16 rows of V:
+    // lane i lands at row i / 4, piece i % 4.  Pieces past the last column re-read the last one (columns are independent and dead
+    // ones are not stored).
+    // The column groups of a (batch, head) ask for the same bytes at the same time.  Each begins its run at another place, so that
+    // first requests differ and later ones find the L2 filled (T = 8192: 64 heads of 128 469 -> 455 us, both kernels), and
+    // in turns with a pause between: all at once they delay the other wavefronts' LDS and store traffic (4 heads of 128 215 -> 184 us,
+    // of 64 134 -> 117).  With most compute units at it a longer pause is the better one (456 against 458 us; 192 against 184 the other
+    // way round).  *Tried:* one dword of every line fetched further ahead, by these or by a wavefront of its own, and from the scalar
+    // side: slower, answers come back in order and hits wait behind misses.
+    const int pw = ct;
+    constexpr int NM1 = 3 * KC * KD * 2 / 1024 / KPW, NO1 = Blob::kOut / 1024 / KPW;
+    static_assert(NM1 * KPW * 1024 == Blob::kDec && NO1 * KPW * 1024 == Blob::kOut && Blob::kChain - Blob::kDec == 1024, "runs of whole KiB");
+    constexpr int kTurns = NM1 / 3;
+    const bool crowded = gridDim.x >= 192;
     const uint32_t stage_lds = lds_address(&stage[0][0]);
-    // V: a copy moves 16 rows of 64 bytes; lane i lands at row i / 4, piece i % 4.  Pieces past the last column re-read
-    // the last one (columns are independent and dead ones are not stored).
-    const int v_row = lane >> 2, v_piece = min(KVS * KCT * grp / 8 + (lane & 3), p.Dv / 8 - 1);
-    const char* const my_blobs = p.blobs + ci0 * Blob::kBytes;
-    auto issue_copies = [&](int n, int st) {
-      const uint16_t* src = reinterpret_cast<const uint16_t*>(my_blobs + (int64_t)n * Blob::kBytes);
-      const uint32_t dst = stage_lds + st * kStage;
+    const int n_rows = sp.tok_end - sp.tok0, v_pitch = 2 * p.H * p.Dv;
+    const char* const my_v = (const char*)(p.v + ((int64_t)sp.tok0 * p.H + h) * p.Dv);
+    const int v_row = 16 * pw + (lane >> 2), v_off = 16 * min(KVS * KCT * grp / 8 + (lane & 3), p.Dv / 8 - 1);
+    auto copy_chain = [&](int n, int st) {
+      const char* const block = my_blobs + (int64_t)n * Blob::kBytes;
+      const uint32_t to = stage_lds + st * kStage;
 #pragma unroll
-      for (int j = pw; j < NCP; j += KPW) copy16_to_lds_async(src + 512 * j, 16 * lane, dst + 1024 * j);
-      if (pw >= 2) {
-        const int tok = sp.tok0 + n * KC;
-        const int row = min(16 * (pw - 2) + v_row, sp.tok_end - 1 - tok);
-        copy16_to_lds_async(p.v + ((int64_t)tok * p.H + h) * p.Dv, 2 * (row * p.H * p.Dv + 8 * v_piece), dst + kV + 1024 * (pw - 2));
+      for (int i = 0; i < kTurns; ++i) {
+        const int first = (pw * kTurns + (i + grp) % kTurns) * (NM1 / kTurns) * 1024;
+        copy_kib_to_lds_async<NM1 / kTurns>(block + first, 16 * lane, to + first);
+        if (crowded) __builtin_amdgcn_s_sleep(4); else __builtin_amdgcn_s_sleep(2);
       }
+      copy_kib_to_lds_async<1>(block + Blob::kDec, 16 * lane, to + Blob::kDec);
+      copy_kib_to_lds_async<1>(my_v + (int64_t)n * KC * v_pitch, min(v_row, n_rows - n * KC - 1) * v_pitch + v_off, to + kV + 1024 * pw);
     };
-    // The workgroups of a (batch, head) copy the same blocks at about the same time; each asks for its share of the block
-    // two chunks beyond the copies (one dword per 128-byte line, by wavefronts 0 and 1) so that the copies find it in
-    // the L2.  The target register is tied up for the whole loop.
-    constexpr int kAhead = 4;                 // (6 and 8 gave the same time)
-    uint32_t touched = 0;
-    const int t_line = (64 * pw + lane) * NGRP + grp;
-    const int t_off = 128 * min(t_line, Blob::kBytes / 128 - 1);
-    auto touch_ahead = [&](int n) {
-      asm volatile("global_load_dword %0, %1, %2" : "+v"(touched) : "v"(t_off), "s"(my_blobs + (int64_t)n * Blob::kBytes) : "memory");
+    auto copy_out = [&](int n, int st) {
+      constexpr int first = Blob::kChain;
+      copy_kib_to_lds_async<NO1>(my_blobs + (int64_t)n * Blob::kBytes + first + pw * NO1 * 1024, 16 * lane, stage_lds + st * kStage + first + pw * NO1 * 1024);
     };
-    // Copies of one chunk that this wavefront has in flight: they are its youngest when it waits for the chunk before.
-    static_assert(NCP % KPW == 1 && NCP / KPW + 2 < 16, "copies per wavefront: base + 1 (0), base (1), base + 1 (2, 3: V)");
-    auto older_landed = [&](bool more, bool touching) {
-      constexpr int base = NCP / KPW;
-      if (!more) __builtin_amdgcn_s_waitcnt(0x0F70);
-      else if (pw == 0 && touching) __builtin_amdgcn_s_waitcnt(0x0F70 | (base + 2));
-      else if (pw != 1 || touching) __builtin_amdgcn_s_waitcnt(0x0F70 | (base + 1));
-      else __builtin_amdgcn_s_waitcnt(0x0F70 | base);
+    auto landed = [&](auto still) {           // all copies but the youngest `still` of this wavefront are in the LDS
+      constexpr int N = decltype(still)::value;
+      static_assert(N < 64, "");
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | (N >> 4) << 14);
       asm volatile("" ::: "memory");
     };
-    if (nc > 0) issue_copies(0, 0);
-    if (nc > 1) issue_copies(1, 1);
-    older_landed(nc > 1, false);
-    __syncthreads();
-    int st = 2;                               // stage of chunk n + 2
-    for (int n = 0; n < nc; ++n) {
-      const bool touching = n + kAhead < nc;
-      if (n + 2 < nc) issue_copies(n + 2, st);
-      if (touching && pw < 2) touch_ahead(n + kAhead);
-      older_landed(n + 2 < nc, touching);
+    int st = 0;                               // stage of chunk n
+    for (int n = 0; n < nc + 3; ++n) {
+      const int before = st == 0 ? KSTAGES - 1 : st - 1;
+      if (n < nc) copy_chain(n, st);
+      if (n > 0 && n <= nc) copy_out(n - 1, before);
+      // everything of earlier intervals has landed
+      if (n == 0) landed(std::integral_constant<int, NM1 + 2>{});
+      else if (n < nc) landed(std::integral_constant<int, NM1 + 2 + NO1>{});
+      else landed(std::integral_constant<int, 0>{});
       st = st == KSTAGES - 1 ? 0 : st + 1;
       __syncthreads();
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    asm volatile("" :: "v"(touched));
     return;
   }
 
   // ---- per-lane LDS read offsets (bytes, inside a stage) ------------------------------------
   // A operand of a 16x16x32 MFMA: lane (row ln, k-group q4) reads piece 4m + q4 of its row; rows 16 apart share a swizzle.
-  const int ct = wave % KCT;
   int rdk[NM];
 #pragma unroll
   for (int m = 0; m < NM; ++m) rdk[m] = ln * 2 * KD + 16 * ((4 * m + q4) ^ piece_swizzle<2 * KD>(ln));
   const int rd64 = ln * 64 + 16 * (q4 ^ piece_swizzle<64>(ln));
-  lds_cptr stage0 = (lds_cptr)&stage[0][0];
+  lds_cptr const stage0 = (lds_cptr)&stage[0][0];
   int so = 0;                                 // stage of the chunk at hand
 
   if (wave >= KCT) {
@@ -915,7 +841,7 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
       const int tok = sp.tok0 + n * KC + (lane >> 1);
       if (tok < sp.tok_end && col < p.Dv) *reinterpret_cast<u32x4*>(p.o + ((int64_t)tok * p.H + h) * p.Dv + col) = v;
     };
-    __syncthreads();
+    for (int n = 0; n < 3; ++n) __syncthreads();
     for (int n = 0; n < nc; ++n) {
       lds_cptr sb = stage0 + so;
       so = so == (KSTAGES - 1) * kStage ? 0 : so + kStage;
@@ -945,7 +871,7 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
   // ================= chain wavefront =================
   const int vcol = KVS * (KCT * grp + ct) + ln;
   const int rdv = kV + (4 * q4 + (ln >> 2)) * 64 + 2 * (KVS * ct + 4 * (ln & 3));
-  // State tile i: rows (key channels) 16*i + 4*q4 + r, column vcol; rows beyond Dk and columns beyond Dv do not
+  // State tile i: rows (key channels) 32*(i/2) + 8*q4 + 4*(i%2) + r, column vcol; rows beyond Dk and columns beyond Dv do not
   // exist in the caller's [Dk, Dv] state: they are zero and stay zero.
   const bool col_live = vcol < p.Dv;
   f32x4 S[NS];
@@ -953,83 +879,107 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
   for (int i = 0; i < NS; ++i) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = 16 * i + 4 * q4 + r;
+      const int row = 32 * (i >> 1) + 8 * q4 + 4 * (i & 1) + r;
       S[i][r] = (p.s0 && col_live && row < p.Dk) ? p.s0[((int64_t)bh * p.Dk + row) * p.Dv + vcol] : 0.f;
     }
   }
   bf16x8 Sb[NM];   // the state as right operand, by channel group
+  auto next_operand = [&](int from, int to, int par) {
 #pragma unroll
-  for (int m = 0; m < NM; ++m) {
-    Sb[m] = pack_acc2(S[2 * m], S[2 * m + 1]);
-    xs[0][ct][m][lane] = __builtin_bit_cast(u32x4, Sb[m]);
-  }
+    for (int m = from; m < to; ++m) {
+      Sb[m] = pack_acc2(S[2 * m], S[2 * m + 1]);
+      xs[par][ct][m][lane] = __builtin_bit_cast(u32x4, Sb[m]);
+    }
+  };
+  next_operand(0, NM, 0);
+  __syncthreads();
+  __syncthreads();
+
+  // A link's operands are read during the link before it, each register as soon as its last product has been issued: a 16-byte
+  // LDS read keeps a wavefront's port for 16 cycles and a chunk needs 34 of them, which in front of their use was half of
+  // the link.
+  bf16x8 ka[2][NM], mh[NS], ml[NS];
+  u32x2 vr[2];
+  f32x4 dcc[NS];
+  auto read_v = [&](lds_cptr sb) {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) vr[mt] = lds_column4(sb + rdv + 16 * mt * 64);
+  };
+  auto read_ka = [&](lds_cptr sb, int m) {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) ka[mt][m] = lds_bf16x8(sb + Blob::kKg + 16 * mt * 2 * KD + rdk[m]);
+  };
+  auto read_dec = [&](lds_cptr sb, int i) { dcc[i] = lds_f32x4(sb + Blob::kDec + 4 * (32 * (i >> 1) + 8 * q4 + 4 * (i & 1))); };
+  auto read_ml = [&](lds_cptr sb, int i) { ml[i] = lds_bf16x8(sb + Blob::kMl + 16 * i * 64 + rd64); };
+  auto read_mh = [&](lds_cptr sb, int i) { mh[i] = lds_bf16x8(sb + Blob::kMh + 16 * i * 64 + rd64); };
+  read_v(stage0);
+#pragma unroll
+  for (int m = 0; m < NM; ++m) read_ka(stage0, m);
+#pragma unroll
+  for (int i = 0; i < NS; ++i) { read_dec(stage0, i); read_ml(stage0, i); read_mh(stage0, i); }
   __syncthreads();
 
   for (int n = 0; n < nc; ++n) {
     const int par = n & 1;
-    lds_cptr sb = stage0 + so;
     so = so == (KSTAGES - 1) * kStage ? 0 : so + kStage;
-
-    // A 16-byte LDS read keeps a wavefront's port for 16 cycles and this wavefront needs forty of them per chunk: what
-    // X needs is read first, everything else between the products and the conversions that do not need it.
-    bf16x8 ka[2][NM], mh[NS], ml[NS];
-    u32x2 vr[2];
-    f32x4 dcc[NS];
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt) vr[mt] = lds_column4(sb + rdv + 16 * mt * 64);
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) ka[mt][m] = lds_bf16x8(sb + Blob::kKg + 16 * mt * 2 * KD + rdk[m]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    lds_cptr sb = stage0 + so;                // chunk n + 1 (behind the last one: what the stage holds, never used)
 
     // X = V + (-exp(G) K) S0, row tile mt: positions 16*mt + 4*q4 + r, column vcol
     f32x4 X[2];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) X[mt] = f32x4{bf16lo_to_f32(vr[mt].x), bf16hi_to_f32(vr[mt].x), bf16lo_to_f32(vr[mt].y), bf16hi_to_f32(vr[mt].y)};
+    read_v(sb);
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) X[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[mt][m], Sb[m], X[mt], 0, 0, 0);
+      read_ka(sb, m);
 #pragma unroll
-      for (int i = m * NS / NM; i < (m + 1) * NS / NM; ++i) dcc[i] = lds_f32x4(sb + Blob::kDec + 4 * (16 * i + 4 * q4));
+      for (int i = m * NS / NM; i < (m + 1) * NS / NM; ++i) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[i][r] *= dcc[i][r];
+        read_dec(sb, i);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      ml[i] = lds_bf16x8(sb + Blob::kMl + 16 * i * 64 + rd64);
-      mh[i] = lds_bf16x8(sb + Blob::kMh + 16 * i * 64 + rd64);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S[i][r] *= dcc[i][r];
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // S = exp(G_last) (.) S + M X, both operands split into two bf16 terms
+    // S = exp(G_last) (.) S + M X, both operands split into two bf16 terms; the tiles in two halves, so that the first
+    // one's conversions run beside the second one's products
     const bf16x8 Xh = pack_acc2(X[0], X[1]);
+    bf16x8 Xl;
 #pragma unroll
-    for (int i = 0; i < NS; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ml[i], Xh, S[i], 0, 0, 0);
-    const bf16x8 Xl = pack_rest2(X[0], X[1], Xh);
-    {
-      xx[par][ct][0][lane] = __builtin_bit_cast(u32x4, Xh);
-      xx[par][ct][1][lane] = __builtin_bit_cast(u32x4, Xl);
+    for (int half = 0; half < 2; ++half) {
+      constexpr int HT = NS / 2;
+#pragma unroll
+      for (int i = half * HT; i < (half + 1) * HT; ++i) {
+        S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ml[i], Xh, S[i], 0, 0, 0);
+        read_ml(sb, i);
+      }
+      if (half == 0) {
+        Xl = pack_rest2(X[0], X[1], Xh);
+        xx[par][ct][0][lane] = __builtin_bit_cast(u32x4, Xh);
+        xx[par][ct][1][lane] = __builtin_bit_cast(u32x4, Xl);
+      }
+#pragma unroll
+      for (int i = half * HT; i < (half + 1) * HT; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mh[i], Xh, S[i], 0, 0, 0);
+#pragma unroll
+      for (int i = half * HT; i < (half + 1) * HT; ++i) {
+        S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mh[i], Xl, S[i], 0, 0, 0);
+        read_mh(sb, i);
+      }
+      if (half == 1) next_operand(0, NM / 2, par ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int i = 0; i < NS; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mh[i], Xh, S[i], 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < NS; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mh[i], Xl, S[i], 0, 0, 0);
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      Sb[m] = pack_acc2(S[2 * m], S[2 * m + 1]);
-      xs[par ^ 1][ct][m][lane] = __builtin_bit_cast(u32x4, Sb[m]);
-    }
+    next_operand(NM / 2, NM, par ^ 1);
     __syncthreads();
   }
   if (p.s_out != nullptr && col_live) {
+    int row0 = 8 * q4;
+    asm volatile("" : "+v"(row0));            // (the addresses are worked out here and not kept, spilled, across the loop)
 #pragma unroll
     for (int i = 0; i < NS; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = 16 * i + 4 * q4 + r;
+        const int row = 32 * (i >> 1) + row0 + 4 * (i & 1) + r;
         if (row < p.Dk) p.s_out[((int64_t)bh * p.Dk + row) * p.Dv + vcol] = S[i][r];
       }
   }
@@ -1089,12 +1039,25 @@ extern "C" size_t daisy_kda_varlen_workspace_bytes(int T, int n_seq, int H, int 
   return kda_chunk_slots(1, T, n_seq) * H * kBlobBytes + kda_table_bytes(T, n_seq);
 }
 
+// Blocks of up to this many bytes are stored through the caches (the last level holds 256 MB), where the second kernel finds
+// them: T = 8192, 4 heads of 64 154 -> 117 us, T = 6016, 12 heads of 128 168 -> 156 us; 153 MB of them 118 -> 124 us.
+constexpr int64_t kCachedBytes = (int64_t)128 << 20;
+
 template <int KD>
 static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
   const int groups = (p.Dv + KVS * KCT - 1) / (KVS * KCT);
-  hipLaunchKernelGGL(kda_prep_kernel<KD>, dim3((p.NC + 1) / 2, p.H, p.n_seq > 0 ? 1 : p.B), dim3(256), 0, s, p);
+  const dim3 chunks(p.NC, p.H, p.n_seq > 0 ? 1 : p.B);
+  const int64_t bytes = (int64_t)p.H * p.nc_total * KdaBlob<KD>::kBytes;
+  if (bytes > kCachedBytes) {
+    // Beyond 400 MB 6 KB more of LDS than the kernel uses: five workgroups per compute unit.  A sixth only adds requests where memory
+    // is the bound (B4 T8192 H16, 128 x 128, fp32 log-decays, behind the other kernel: 230 -> 222 us; with four the latency shows,
+    // 329; half of that length 111 and 113 us).
+    hipLaunchKernelGGL((kda_prep_kernel<KD, true>), chunks, dim3(128), KD == 128 && bytes > (int64_t)400 << 20 ? 6144 : 0, s, p);
+  } else {
+    hipLaunchKernelGGL((kda_prep_kernel<KD, false>), chunks, dim3(128), 0, s, p);
+  }
   DAISY_CHECK_LAUNCH("kda_prep_kernel");
-  hipLaunchKernelGGL(kda_state_kernel<KD>, dim3((unsigned)(n_streams * p.H * groups)), dim3(kStateThreads), 0, s, p);
+  hipLaunchKernelGGL(kda_state_kernel<KD>, dim3((unsigned)((n_streams * p.H + 7) / 8 * 8 * groups)), dim3(kStateThreads), 0, s, p);
   DAISY_CHECK_LAUNCH("kda_state_kernel");
   return DAISY_OK;
 }
@@ -1123,7 +1086,7 @@ static int kda_chunk_launch(const void* q, const void* k, const void* v,
     set_error("kda: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
     return DAISY_ERR_WORKSPACE;
   }
-  DAISY_CHECK_ARG(slots <= 0x7fffffff && (int64_t)(n_seq > 0 ? n_seq : B) * H * ((Dv + KVS * KCT - 1) / (KVS * KCT)) <= 0x7fffffff,
+  DAISY_CHECK_ARG(slots <= 0x7fffffff && ((int64_t)(n_seq > 0 ? n_seq : B) * H + 7) * ((Dv + KVS * KCT - 1) / (KVS * KCT)) <= 0x7fffffff,
                   "kda: too many chunks or sequences");
   KdaParams p;
   p.q = (const uint16_t*)q; p.k = (const uint16_t*)k; p.v = (const uint16_t*)v;

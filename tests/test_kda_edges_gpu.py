@@ -1,4 +1,4 @@
-"""Chunked KDA at the edges of its tiling: chunks of 32 positions handled in pairs, key widths of 64 and 128 channels, groups
+"""Chunked KDA at the edges of its tiling: chunks of 32 positions, key widths of 64 and 128 channels, groups
 of 32 value columns, and keys that overlap so strongly that the triangle's inverse carries the result."""
 import pytest
 import torch
@@ -73,3 +73,21 @@ def test_kda_packed_chunk_slots(lengths, behind):
         o_ref, S_ref = oracle.kda_recurrent(*(t[:, a:a + n] for t in (q, k, v, gl, beta)))
         assert_close_bf16(o[:, a:a + n], o_ref, f"sequence {i}: o")
         assert ((S[i:i + 1] - S_ref).norm() / S_ref.norm()).item() <= 1e-3
+
+
+# Blocks of the workspace (37 KiB per chunk and head) beyond 128 and 400 MB are stored past the caches, beyond 400 with fewer
+# workgroups per compute unit; 192 and more workgroups of the second kernel copy at another pace.  Heads are independent: the
+# same bits as from calls on the other side of every line.
+@pytest.mark.parametrize("T,H", [(3712, 32), (8200, 48)])
+def test_kda_workspace_sizes_agree(T, H):
+    assert (T + 31) // 32 * H * 37 * 1024 > (400 << 20 if T > 8000 else 128 << 20)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    q, k, v = (torch.randn(1, T, H, 128, generator=g, device="cuda").bfloat16() for _ in range(3))
+    gl = F.logsigmoid(torch.randn(1, T, H, 128, generator=g, device="cuda"))
+    beta = torch.sigmoid(torch.randn(1, T, H, generator=g, device="cuda"))
+    kw = dict(output_final_state=True, use_qk_l2norm_in_kernel=True)
+    o, S = chunk_kda(q, k, v, gl, beta, **kw)
+    for h in range(0, H, 8):
+        part = [t[:, :, h:h + 8].contiguous() for t in (q, k, v, gl, beta)]
+        o8, S8 = chunk_kda(*part, **kw)
+        assert torch.equal(o[:, :, h:h + 8], o8) and torch.equal(S[:, h:h + 8], S8)
