@@ -166,6 +166,15 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(size_t)(__attribute__((address_space(3))) const void*)p;
 }
 
+// ---- LDS layout ---------------------------------------------------------------
+// Swizzle of a row's 16-byte pieces: the 16 lanes that a 16-byte LDS read serves together must fall into 16 different slots
+// of the 256-byte bank window.  Those are not 16 consecutive lanes but lanes 0-3, 12-15 and 20-27 (and so on): rows 0-3
+// and 12-15 of one k-group with rows 4-11 of the next.  For rows of 64 bytes (row >> 2) & 3 itself puts two of them into every
+// slot (256 of 930 LDS cycles per chunk of the KDA chain); the permutation 0 2 3 1 of it puts one.  Rows of 256, 128 and 64 bytes:
+template <int ROWBYTES> __host__ __device__ constexpr int piece_swizzle(int row) {
+  return ROWBYTES == 256 ? (row & 15) : ROWBYTES == 128 ? ((row >> 1) & 7) : ((row >> 3) & 1) | (((row >> 2) ^ (row >> 3)) & 1) << 1;
+}
+
 // ---- host-side error plumbing --------------------------------------------
 void set_error(const char* fmt, ...);
 

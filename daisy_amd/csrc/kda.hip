@@ -112,14 +112,6 @@ template <int KD> struct KdaBlob {
   static constexpr int kBytes = kPl + KC * KC * 2, kOut = kBytes - kChain;
 };
 static_assert(KdaBlob<128>::kBytes == 37 * 1024 && KdaBlob<64>::kBytes == 21 * 1024, "");
-// Swizzle of a row's 16-byte pieces: the 16 lanes that a 16-byte LDS read serves together must fall into 16 different slots
-// of the 256-byte bank window.  Those are not 16 consecutive lanes but lanes 0-3, 12-15 and 20-27 (and so on): rows 0-3
-// and 12-15 of one k-group with rows 4-11 of the next.  For rows of 64 bytes (row >> 2) & 3 itself puts two of them into every
-// slot (256 of 930 LDS cycles per chunk); the permutation 0 2 3 1 of it puts one.  Rows of 256, 128 and 64 bytes:
-template <int ROWBYTES> __host__ __device__ constexpr int piece_swizzle(int row) {
-  return ROWBYTES == 256 ? (row & 15) : ROWBYTES == 128 ? ((row >> 1) & 7) : ((row >> 3) & 1) | (((row >> 2) ^ (row >> 3)) & 1) << 1;
-}
-
 struct KdaParams {
   const uint16_t* q; const uint16_t* k; const uint16_t* v;
   const void* g; int g_bf16; const float* beta;

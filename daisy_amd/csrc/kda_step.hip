@@ -153,15 +153,17 @@ __global__ __launch_bounds__(256) void kda_recurrent_kernel(KdaStepParams p) {
 // The same step with everything of the KDA layer that lies between its projections.
 //
 // What bounds it: HBM, the state in and out (134 MB for 64 sequences of 16 heads of 128 x 128: 27.6 us at what a copy
-// reaches, 33 us measured).  As separate launches the token passed through eleven kernels (three convolutions, two
+// reaches, 28.6 us measured).  As separate launches the token passed through eleven kernels (three convolutions, two
 // projections from the low rank, gate, two for beta, recurrence, copy, norm), 70 us of GPU time and as much again between them.  Here one
 // workgroup per (sequence, head) requests its inputs, then its state, and does the small work while the state arrives:
 // the two products from the low rank are 32 KB of weights per head and matrix, read through the L2 by all sequences.
+// The state's requests have to leave early: nothing ahead of them converts or branches on what was loaded, which would wait
+// for it, and the weights come in whole rows.  32.8 us at the size above -> 30.0 without the waits, 28.6 with the weights
+// through the LDS.
 // VD / 16 wavefronts; wavefront w owns value columns [32 (w / 2), .. + 32) of half w % 2 of the key channels, lane (dq, jc)
 // channels KD / 16 dq .. of that half and columns 4 jc ..: rows of 128 bytes as in kda_recurrent_kernel (with 64-byte
-// rows the step of 64 sequences took 3 us more), and half as much state per lane, so that the weights fit beside it in
-// 128 registers.  The
-// products run on the matrix cores, weights as left operand straight from memory and all sixteen columns of the right
+// rows the step of 64 sequences took 3 us more), and half as much state per lane, so that two workgroups fit a CU
+// (128 registers).  The products run on the matrix cores, weights as left operand and all sixteen columns of the right
 // operand the same row: fifteen of them are waste, but nothing is unpacked and nothing summed across lanes.
 __device__ __forceinline__ float sum_over_rows(float x) {          // lane bits 3, 4, 5
   x = dpp_add<0x128>(x);                 // row_ror 8
@@ -180,6 +182,8 @@ __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep 
   __shared__ __attribute__((aligned(16))) float eg_gate[SLOTS];   // exp(g), then sigmoid(gate)
   __shared__ __attribute__((aligned(16))) f32x4 part[2][2][VD / 4];   // [half][prediction, read-out][columns]
   __shared__ float red[VD / 32];
+  constexpr int RB = 2 * VD, PPR = RB / 16;                       // bytes and 16-byte pieces of a weight row
+  __shared__ __attribute__((aligned(1024))) char weights[NW * TPW][16 * RB];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = wave & 1, dq = lane >> 3, jc = lane & 7, d0 = KD / 2 * half + ROWS * dq;     // d0: this lane's first key channel
@@ -188,33 +192,40 @@ __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep 
   const int Dk = p.Dk;
 
   // ---- requests: the low-rank rows and weights, the convolutions' inputs, the state --------------------------------
-  u32x4 low_f[KS], low_g[KS], wv[TPW][KS];
+  // Weights: the 16 rows of a tile through the LDS (a wavefront's own), swizzled, in whole rows.  Straight into operand layout,
+  // 16 rows by 64 bytes per load, they kept the address unit busy for 4 us and the state's requests behind them.
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) {
+    const int s0 = 16 * min(wave + NW * t, TILES - 1);            // (surplus tiles redo the last one)
+    const uint16_t* const w = s0 < KD ? p.wf + (int64_t)h * Dk * VD : p.wg + ((int64_t)h * VD + s0 - KD) * VD;
+    const int rows_left = s0 < KD ? Dk - s0 : 16, row0 = s0 < KD ? s0 : 0;    // (channels beyond Dk re-read the last row)
+#pragma unroll
+    for (int j = 0; j < 16 * RB / 1024; ++j) {
+      const int r = 1024 / RB * j + lane / PPR, piece = (lane % PPR) ^ piece_swizzle<RB>(r);
+      copy16_to_lds_async(w, (row0 + min(r, rows_left - 1)) * RB + 16 * piece, lds_address(&weights[wave + NW * t][0]) + 1024 * j);
+    }
+  }
+  u32x4 low_f[KS], low_g[KS];
 #pragma unroll
   for (int m = 0; m < KS; ++m) {
     low_f[m] = *reinterpret_cast<const u32x4*>(p.f + b * p.f_row + 32 * m + 8 * q4);
     low_g[m] = *reinterpret_cast<const u32x4*>(p.g + b * p.g_row + 32 * m + 8 * q4);
   }
-#pragma unroll
-  for (int t = 0; t < TPW; ++t) {
-    const int s0 = 16 * min(wave + NW * t, TILES - 1);            // (surplus tiles redo the last one)
-    const uint16_t* w = s0 < KD ? p.wf + ((int64_t)h * Dk + min(s0 + ln, Dk - 1)) * VD    // (channels beyond Dk re-read the last row)
-                                : p.wg + ((int64_t)h * VD + s0 - KD + ln) * VD;
-#pragma unroll
-    for (int m = 0; m < KS; ++m) wv[t][m] = *reinterpret_cast<const u32x4*>(w + 32 * m + 8 * q4);
-  }
   // Taps and window of a channel as four bf16 aligned at the newest end: tap 3 meets the new input, window entry j tap j - 1.
-  float xin[CROUNDS], cb[CROUNDS];
+  // (Nothing is converted here: that would wait for the load, and the state's requests with it.  Which convolution a channel belongs
+  // to is the same for a whole wavefront, so that its pointers are scalar loads.)
+  static_assert(KD % 64 == 0, "a wavefront's channels belong to one convolution");
+  uint32_t xraw[CROUNDS], braw[CROUNDS];
   u32x2 cw[CROUNDS], win[CROUNDS];
 #pragma unroll
   for (int r = 0; r < CROUNDS; ++r) {
-    const int c = tid + NT * r, kind = c < KD ? 0 : c < 2 * KD ? 1 : 2, d = c - KD * kind, D = kind == 2 ? VD : Dk;
-    xin[r] = 0.f;
-    if (c >= CH || d >= D) continue;                              // (channels beyond Dk: zeros)
-    const int ch = h * D + d;
-    const uint16_t* x = kind == 0 ? p.q + b * p.q_row : kind == 1 ? p.k + b * p.k_row : p.v + b * p.v_row;
+    const int c0 = 64 * wave + NT * r, kind = c0 < KD ? 0 : c0 < 2 * KD ? 1 : 2, D = kind == 2 ? VD : Dk;
+    const int ch = h * D + min(c0 + lane - KD * kind, D - 1);     // (channels beyond the last re-read it)
+    const uint16_t* const x = kind == 0 ? p.q + b * p.q_row : kind == 1 ? p.k + b * p.k_row : p.v + b * p.v_row;
+    const uint16_t* const bias = p.conv_bias[kind];
     const uint16_t *wp = p.conv_w[kind] + (int64_t)ch * p.taps, *cp = p.window[kind] + ((int64_t)b * p.H * D + ch) * p.taps;
-    xin[r] = bf16lo_to_f32(x[ch]);
-    cb[r] = p.conv_bias[kind] != nullptr ? bf16lo_to_f32(p.conv_bias[kind][ch]) : 0.f;
+    xraw[r] = x[ch];
+    braw[r] = (bias != nullptr ? bias : x)[ch];                   // (no branch around a load either; dropped below)
     if (p.taps == 4) {
       cw[r] = *reinterpret_cast<const u32x2*>(wp);
       win[r] = *reinterpret_cast<const u32x2*>(cp);
@@ -224,33 +235,50 @@ __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep 
       win[r] = u32x2{c0 << 16, (uint32_t)cp[p.taps - 2] | (uint32_t)cp[p.taps - 1] << 16};
     }
   }
-  const float b_logit = bf16lo_to_f32(p.b[b * p.b_row + h]);
+  const uint32_t b_logit = p.b[b * p.b_row + h];
   const int col = 32 * (wave >> 1) + 4 * jc;
   float* const state = p.state + ((int64_t)blockIdx.x * Dk + d0) * VD + col;
-  __builtin_amdgcn_sched_barrier(0);
-  f32x4 S[ROWS];
+  // What the products' results meet: lane (ln, q4) has row 4 q4 + ln % 4 of tile ln / 4 of every four.
+  constexpr int ROUNDS = (TPW + 3) / 4;
+  auto slot_of = [&](int r) { return 16 * (wave + NW * (4 * r + (ln >> 2))) + 4 * q4 + (ln & 3); };
+  float dt[ROUNDS];
+  uint32_t gb[ROUNDS];
 #pragma unroll
-  for (int i = 0; i < ROWS; ++i) {
-    S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (d0 + i < Dk) S[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(state + i * VD));
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int slot = slot_of(r);
+    dt[r] = p.dt_bias[h * Dk + min(slot, Dk - 1)];
+    gb[r] = (p.g_bias != nullptr ? p.g_bias + (int64_t)h * VD : p.norm_w)[min(max(slot - KD, 0), VD - 1)];
   }
+  const float a_log = p.A_log[h];
+  const u32x2 nw = *reinterpret_cast<const u32x2*>(p.norm_w + col);
   __builtin_amdgcn_sched_barrier(0);
+  f32x4 S[ROWS];                                  // (rows beyond Dk: read as copies of others, then zeroed)
+  const char* const state_in = (const char*)(p.state + (int64_t)blockIdx.x * Dk * VD);
+  const uint32_t at = 4u * (uint32_t)(min(d0, Dk - ROWS) * VD + col);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) S[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(state_in + at + 4 * VD * i));
+  __builtin_amdgcn_sched_barrier(0);
+
+  __builtin_amdgcn_s_waitcnt(0x0F70 | ROWS);      // everything older than the state has arrived, the weights among it
+  asm volatile("" ::: "memory");
 
   // ---- convolutions ----------------------------------------------------------------------------------------------
 #pragma unroll
   for (int r = 0; r < CROUNDS; ++r) {
-    const int c = tid + NT * r, kind = c < KD ? 0 : c < 2 * KD ? 1 : 2, d = c - KD * kind, D = kind == 2 ? VD : Dk;
+    const int c0 = 64 * wave + NT * r, kind = c0 < KD ? 0 : c0 < 2 * KD ? 1 : 2, D = kind == 2 ? VD : Dk;
+    const int c = c0 + lane, d = c - KD * kind;
     if (c >= CH) continue;
     float a = 0.f;
     if (d < D) {
-      a = cb[r];
+      const float x = bf16lo_to_f32(xraw[r]);
+      a = p.conv_bias[kind] != nullptr ? bf16lo_to_f32(braw[r]) : 0.f;
       a = fmaf(bf16lo_to_f32(cw[r].x), bf16hi_to_f32(win[r].x), a);
       a = fmaf(bf16hi_to_f32(cw[r].x), bf16lo_to_f32(win[r].y), a);
       a = fmaf(bf16lo_to_f32(cw[r].y), bf16hi_to_f32(win[r].y), a);
-      a = round_bf16(fmaf(bf16hi_to_f32(cw[r].y), xin[r], a));
+      a = round_bf16(fmaf(bf16hi_to_f32(cw[r].y), x, a));
       a = round_bf16(a * __builtin_amdgcn_rcpf(1.f + __expf(-a)));
       uint16_t* cp = p.window[kind] + ((int64_t)b * p.H * D + h * D + d) * p.taps;
-      const u32x2 next = {win[r].x >> 16 | win[r].y << 16, win[r].y >> 16 | __float_as_uint(xin[r])};
+      const u32x2 next = {win[r].x >> 16 | win[r].y << 16, win[r].y >> 16 | xraw[r] << 16};
       if (p.taps == 4) *reinterpret_cast<u32x2*>(cp) = next;
       else {
         if (p.taps == 3) cp[0] = (uint16_t)(next.x >> 16);
@@ -260,8 +288,7 @@ __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep 
     }
     qkv[c] = a;
   }
-  // ---- g = f wf^T and gate = g wg^T + bias: every column of a tile is the same; lane (ln, q4) takes row 4 q4 + ln % 4 of
-  // tile ln / 4 of every four
+  // ---- g = f wf^T and gate = g wg^T + bias: every column of a tile is the same
 #pragma unroll
   for (int t0 = 0; t0 < TPW; t0 += 4) {
     f32x4 acc[4];
@@ -272,7 +299,7 @@ __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep 
       const bool decay = 16 * (wave + NW * (t0 + t)) < KD;
 #pragma unroll
       for (int m = 0; m < KS; ++m)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[t0 + t][m]),
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&weights[wave + NW * (t0 + t)][ln * RB + 16 * ((4 * m + q4) ^ piece_swizzle<RB>(ln))]),
                                                          __builtin_bit_cast(bf16x8, decay ? low_f[m] : low_g[m]), acc[t], 0, 0, 0);
     }
     f32x4 mine = acc[0];
@@ -281,22 +308,21 @@ __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep 
     float x = mine[0];
 #pragma unroll
     for (int r = 1; r < 4; ++r) x = (ln & 3) == r ? mine[r] : x;
-    const int t = t0 + (ln >> 2), slot = 16 * (wave + NW * t) + 4 * q4 + (ln & 3);
+    const int t = t0 + (ln >> 2), slot = slot_of(t0 / 4);
     if (t < TPW && slot < SLOTS) {
       float y;
       if (slot < KD) {
         // every intermediate rounded as the tensor that holds it in the layer
-        const int d = min(slot, Dk - 1);
-        const float gl = -expf(p.A_log[h]) * softplus(round_bf16(x) + p.dt_bias[h * Dk + d], 1.f, 20.f, 1.f);
+        const float gl = -expf(a_log) * softplus(round_bf16(x) + dt[t0 / 4], 1.f, 20.f, 1.f);
         y = slot < Dk ? __expf(round_bf16(gl)) : 1.f;
       } else {
-        if (p.g_bias != nullptr) x += bf16lo_to_f32(p.g_bias[h * VD + slot - KD]);
+        if (p.g_bias != nullptr) x += bf16lo_to_f32(gb[t0 / 4]);
         y = __builtin_amdgcn_rcpf(1.f + __expf(-round_bf16(x)));
       }
       eg_gate[slot] = y;
     }
   }
-  const float beta = round_bf16(1.f / (1.f + expf(-b_logit)));
+  const float beta = round_bf16(1.f / (1.f + expf(-bf16lo_to_f32(b_logit))));
   __syncthreads();
 
   // ---- the delta rule; q and k L2-normalised (every wavefront sums for itself) ---------------------------------------
@@ -317,6 +343,10 @@ __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep 
   // S^T q + (k . q) delta: both products over the old state in one pass and one round of cross-lane sums.
   f32x4 pred = {0.f, 0.f, 0.f, 0.f}, out = {0.f, 0.f, 0.f, 0.f};
   float kk[ROWS];
+  if (d0 >= Dk) {
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 #pragma unroll
   for (int i4 = 0; i4 < ROWS / 4; ++i4) {
     const f32x4 e4 = *reinterpret_cast<const f32x4*>(&eg_gate[d0 + 4 * i4]);
@@ -366,7 +396,6 @@ __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep 
   for (int w = 0; w < VD / 32; ++w) ss += red[w];
   const float rstd = rsqrtf(ss / (float)VD + p.norm_eps);
   if (dq == 0 && half == 0) {
-    const u32x2 nw = *reinterpret_cast<const u32x2*>(p.norm_w + col);
     const f32x4 gt = *reinterpret_cast<const f32x4*>(&eg_gate[KD + col]);
     const float w4[4] = {bf16lo_to_f32(nw.x), bf16hi_to_f32(nw.x), bf16lo_to_f32(nw.y), bf16hi_to_f32(nw.y)};
 #pragma unroll

@@ -59,6 +59,13 @@ def test_layer_in_one_call_equals_its_kernels_one_by_one(H, D, expand_v, taps, c
         assert ((a.float() - b.float()).norm() / a.float().norm().clamp_min(1e-9)).item() < 5e-3
 
 
+@pytest.mark.parametrize("H,D,expand_v,taps,conv_bias", [(8, 8, 4.0, 4, True), (8, 72, 32 / 72, 2, True), (8, 120, 64 / 120, 3, False),
+                                                         (16, 56, 128 / 56, 4, False)])
+def test_step_whose_key_channels_end_inside_a_tile(H, D, expand_v, taps, conv_bias, monkeypatch):
+    """Key widths that are no multiple of the 16 weight rows of a tile, from the smallest; every value width."""
+    test_layer_in_one_call_equals_its_kernels_one_by_one(H, D, expand_v, taps, conv_bias, 5, 4, monkeypatch)
+
+
 @pytest.mark.parametrize("M,K,Ns", [(1, 256, (256, 64, 12)), (4, 128, (100, 8, 1)), (5, 64, (64, 200)), (70, 768, (768, 64, 64, 12)),
                                     (300, 128, (2048, 2048)), (513, 2048, (128, 128, 16))])
 def test_products_in_one_launch_equal_separate_ones(M, K, Ns):
