@@ -47,15 +47,28 @@ struct DecodeParams {
   uint16_t* k_rows; uint16_t* v_rows;   // optional: bf16 copies of the new rows, [B, H, D]
 };
 
+// A pointer whose origin the compiler cannot see any more, as one to global memory.
+template <typename T> __device__ __forceinline__ const __attribute__((address_space(1))) T* in_global(const void* ptr) {
+  return (const __attribute__((address_space(1))) T*)ptr;
+}
+
 struct DecodeRange { int n_rows, new_idx, rows_per_split; };
 
-__device__ __forceinline__ DecodeRange decode_range(const DecodeParams& p) {
+// The step's position when it comes from device memory (pos_dev != NULL).
+__device__ __forceinline__ int device_position(const DecodeParams& p) {
+  return max(*(const __attribute__((address_space(4))) int32_t*)p.pos_dev, 0);
+}
+__device__ __forceinline__ DecodeRange decode_range(const DecodeParams& p, int t) {
   DecodeRange r{p.n_rows, p.new_idx, p.rows_per_split};
   if (p.pos_dev != nullptr) {
-    const int t = max(p.pos_dev[0], 0);
-    r.n_rows = min(t + 1, p.ring_rows);
-    r.new_idx = t % p.ring_rows;
-    r.rows_per_split = (r.n_rows + p.nsplit - 1) / p.nsplit;
+    r.new_idx = t;
+    if (t < p.ring_rows - 1) {
+      r.n_rows = t + 1;
+      r.rows_per_split = (r.n_rows + p.nsplit - 1) / p.nsplit;
+    } else {                       // a full ring: the host's split of ring_rows holds
+      r.n_rows = p.ring_rows;
+      r.new_idx = t % p.ring_rows;
+    }
   }
   return r;
 }
@@ -181,15 +194,26 @@ struct SoftmaxState {
   float acc[8];
 };
 
-// Merges `b` into `a` (both may be empty, i.e. m == -inf).
-__device__ __forceinline__ void merge_state(SoftmaxState& a, const SoftmaxState& b) {
-  const float m = fmaxf(a.m, b.m);
-  const float mu = (m == -INFINITY) ? 0.f : m;
-  const float sa = fast_exp2(a.m - mu), sb = fast_exp2(b.m - mu);
-  a.l = a.l * sa + b.l * sb;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) a.acc[i] = a.acc[i] * sa + b.acc[i] * sb;
-  a.m = m;
+// Maximum and sum over the row groups of a wavefront (lanes that agree modulo LPR = 8 or 16).
+template <int LPR, typename OP>
+__device__ __forceinline__ float over_groups(float x, OP op) {
+  if constexpr (LPR == 8) x = op(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false)));   // row_ror 8
+  u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+  x = op(__uint_as_float(t.x), __uint_as_float(t.y));
+  t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+  return op(__uint_as_float(t.x), __uint_as_float(t.y));
+}
+template <int LPR> __device__ __forceinline__ float max_over_groups(float x) {
+  return over_groups<LPR>(x, [](float a, float b) { return fmaxf(a, b); });
+}
+template <int LPR> __device__ __forceinline__ float sum_over_groups(float x) {
+  return over_groups<LPR>(x, [](float a, float b) { return a + b; });
+}
+
+// gate_value of a value that was fetched as two halves (a bf16 logit in the first).
+__device__ __forceinline__ float gate_of_halves(const uint16_t* r, int kind) {
+  const float x = __uint_as_float(kind == GateSource::kLogitBf16 ? (uint32_t)r[0] << 16 : r[0] | (uint32_t)r[1] << 16);
+  return kind == GateSource::kValue ? x : round_bf16(1.f / (1.f + expf(-x)));
 }
 
 // PREP: q, k_new and v_new are rows of the QKV projection output; the kernel normalises, rotates
@@ -201,7 +225,11 @@ __device__ __forceinline__ void merge_state(SoftmaxState& a, const SoftmaxState&
 // loaded again as soon as it has been used.  A wavefront so keeps 2 to 4 * kDecodeUnroll KiB of cache rows
 // in flight from its first instructions to its last row: with a few hundred workgroups on the chip
 // (one sequence, a dozen heads) the launch is a handful of memory round trips long, and every trip
-// spent with nothing in flight shows.
+// spent with nothing in flight shows.  So all arguments are fetched in one go, nothing ahead of the cache rows
+// branches on a loaded value or converts one, an address costs an addition, and the wavefronts' partial
+// results meet in one step at the end: with one sequence, 12 heads of 128 and 8192 rows the cache rows are
+// asked for 1.8 us into the launch, not 2.5, and the kernel takes 10.9 instead of 11.6 us in a recorded
+// step, 11.6 instead of 12.4 launched eagerly (6.5 of them for its 50 MB).
 template <int D, bool PREP, bool F16C = false>
 __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(DecodeParams p) {
   constexpr int LPR = D / 8;        // lanes per cache row
@@ -211,43 +239,58 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(DecodeParams p) 
   constexpr int STRIDE = kDecodeWaves * RB;   // rows the four wavefronts cover with one set each
 
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int sub = lane / LPR;
   const int dl = (lane % LPR) * 8;
+  // Every line of the arguments is asked for at once: fetched where they are used, they were three round trips in a row.
+  asm volatile("" ::"s"(p.q), "s"(p.vn_sb), "s"(p.vc), "s"(p.cos_row), "s"(p.pos_dev), "s"(p.ve), "s"(p.gate.p), "s"(p.k_rows),
+               "s"(p.cos_tab), "s"(p.sin_tab));
 
-  const DecodeRange rg = decode_range(p);
+  const int pos = p.pos_dev != nullptr ? device_position(p) : p.pos_host;
+  const DecodeRange rg = decode_range(p, pos);
   const int new_idx = rg.new_idx;
   const int r0 = split * rg.rows_per_split;
   const int r1 = min(r0 + rg.rows_per_split, rg.n_rows);
   // Only the split that holds the new token's slot needs the new key and value rows.
   const bool holds_new = new_idx >= r0 && new_idx < r0 + rg.rows_per_split;
-  uint16_t* kbase = p.kc + b * p.kc_sb + h * p.kc_sh + dl;
-  uint16_t* vbase = p.vc + b * p.vc_sb + h * p.vc_sh + dl;
-  const uint16_t* q_row = p.q + b * p.q_sb + h * p.q_sh;
-  const uint16_t* kn_row = p.k_new + b * p.kn_sb + h * p.kn_sh;
-  const uint16_t* vn_row = p.v_new + b * p.vn_sb + h * p.vn_sh;
+  const uint64_t uh = blockIdx.y, ub = blockIdx.z;     // (products modulo 2^64: strides may be negative)
+  uint16_t* kcache = p.kc + uh * p.kc_sh;
+  uint16_t* vcache = p.vc + uh * p.vc_sh;
+  const uint16_t* q_row = p.q + uh * p.q_sh;
+  const uint16_t* kn_row = p.k_new + uh * p.kn_sh;
+  const uint16_t* vn_row = p.v_new + uh * p.vn_sh;
+  if (b > 0) {                     // (scalar products in 64 bits are six instructions each)
+    kcache += ub * p.kc_sb;
+    vcache += ub * p.vc_sb;
+    q_row += ub * p.q_sb;
+    kn_row += ub * p.kn_sb;
+    vn_row += ub * p.vn_sb;
+  }
 
   // Raw rows of the new token.
   RawRow q_raw, kn_raw;
   TrigRow trig;
-  u32x4 vn_raw, ve_raw = {0u, 0u, 0u, 0u};
-  float gate = 0.f;
+  u32x4 vn_raw, ve_raw;
+  uint16_t gate_raw[2];
   bool past_tables = false, rotate = true;
   if constexpr (PREP) {
-    const int t = p.pos_dev != nullptr ? max(p.pos_dev[0], 0) : p.pos_host;
     // A position past the rotation tables (possible only when it comes from device memory) reads the
     // last table row, to stay inside the allocation, and is reported: the status word gets its bit and
     // the outputs of the step are NaN, so that the step cannot pass for a valid one.
-    past_tables = t >= p.table_rows;
-    const int64_t trow = (int64_t)min(t, p.table_rows - 1) * (D / 2);
+    past_tables = pos >= p.table_rows;
+    const int64_t trow = (int64_t)min(pos, p.table_rows - 1) * (D / 2);
     trig = load_trig_row<D>(p.cos_tab + trow, p.sin_tab + trow, dl);
     q_raw = load_raw_row<D>(q_row, dl, true);
     kn_raw = load_raw_row<D>(holds_new ? kn_row : q_row, dl, true);
     vn_raw = *reinterpret_cast<const u32x4*>((holds_new ? vn_row : q_row) + dl);
-    if (p.ve != nullptr) {
-      ve_raw = *reinterpret_cast<const u32x4*>((holds_new ? p.ve + b * p.ve_sb + h * p.ve_sh : q_row) + dl);
-      gate = gate_value(p.gate);
-    }
+    // (Without a second value row something readable in its place, and the gate's halves as they lie: a branch or a
+    // conversion here would wait for the loads so far, and the cache rows' requests with it.)
+    const uint16_t* ve_at = holds_new && p.ve != nullptr ? p.ve + b * p.ve_sb + h * p.ve_sh : q_row;
+    const uint16_t* gate_at = p.ve != nullptr ? (const uint16_t*)p.gate.p : q_row;
+    asm volatile("" : "+s"(ve_at), "+s"(gate_at));              // (loads of their own: not q's row taken over in a branch)
+    ve_raw = *in_global<u32x4>(ve_at + dl);
+    gate_raw[0] = *in_global<uint16_t>(gate_at);
+    gate_raw[1] = *in_global<uint16_t>(gate_at + (p.ve == nullptr || p.gate.kind == GateSource::kLogitBf16 ? 0 : 1));
   } else {
     static_assert(!F16C, "fp16 cache rows come with the kernel-side preparation only");
     rotate = p.cos_row != nullptr;
@@ -257,33 +300,39 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(DecodeParams p) 
     vn_raw = *reinterpret_cast<const u32x4*>(vn_row + dl);
   }
 
-  // Lanes whose row is past the range, or is the new token's slot, load a row
-  // that is always readable instead (and are masked / overwritten below).
+  // Lanes whose row is past the range, or is the new token's slot, load a row that is always readable instead (and are
+  // masked / overwritten below): another row of the range or, where there is none, the new rows.  Addresses advance by
+  // uniform steps, so that a row costs an addition and a selection.
   const int safe_row = (r0 != new_idx) ? r0 : r0 + 1;
-  const uint16_t* k_safe = (safe_row < r1) ? kbase + (int64_t)safe_row * p.kc_sr : kn_row + dl;
-  const uint16_t* v_safe = (safe_row < r1) ? vbase + (int64_t)safe_row * p.vc_sr : vn_row + dl;
+  const bool has_rows = safe_row < r1;
+  const int64_t k_step = has_rows ? p.kc_sr * 2 : 0, v_step = has_rows ? p.vc_sr * 2 : 0;     // bytes per row
+  const char* const k_rows = (const char*)(has_rows ? kcache : kn_row) + 2 * dl;
+  const char* const v_rows = (const char*)(has_rows ? vcache : vn_row) + 2 * dl;
+  const char* const k_safe = k_rows + (uint32_t)safe_row * (uint64_t)k_step;
+  const char* const v_safe = v_rows + (uint32_t)safe_row * (uint64_t)v_step;
+  int base = r0 + wave * RB;
+  const char* ka = k_rows + (uint32_t)base * (uint64_t)k_step + (uint32_t)sub * (uint64_t)k_step;
+  const char* va = v_rows + (uint32_t)base * (uint64_t)v_step + (uint32_t)sub * (uint64_t)v_step;
 
-  auto load_set = [&](int base, u32x4* kr, u32x4* vr) {
+  auto load_rows = [&](int ahead, const char* a, int64_t step, const char* safe, u32x4* out) {
+    const int left = r1 - base - sub, to_new = new_idx - base - sub;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int row = base + u * RPW + sub;
-      const uint16_t* a = (row < r1 && row != new_idx) ? kbase + (int64_t)row * p.kc_sr : k_safe;
-      kr[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a));
+    for (int u = 0; u < U; ++u, a += RPW * step) {
+      asm volatile("" : "+v"(a));                               // (a selection below, not a branch around the addition)
+      const int at = ahead + u * RPW;
+      out[u] = __builtin_nontemporal_load(in_global<u32x4>(at < left && at != to_new ? a : safe));
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int row = base + u * RPW + sub;
-      const uint16_t* a = (row < r1 && row != new_idx) ? vbase + (int64_t)row * p.vc_sr : v_safe;
-      vr[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a));
-    }
+  };
+  auto load_set = [&](int ahead, u32x4* kr, u32x4* vr) {       // the set that begins `ahead` rows after `base`
+    load_rows(ahead, ka + ahead * k_step, k_step, k_safe, kr);
+    load_rows(ahead, va + ahead * v_step, v_step, v_safe, vr);
   };
 
   // Two register sets; a set past the end of the range loads the safe row (one cache line) and is not used.
   u32x4 kA[U], vA[U], kB[U], vB[U];
-  int base = r0 + wave * RB;
   __builtin_amdgcn_sched_barrier(0);
-  load_set(base, kA, vA);
-  load_set(base + STRIDE, kB, vB);
+  load_set(0, kA, vA);
+  load_set(STRIDE, kB, vB);
   __builtin_amdgcn_sched_barrier(0);
 
   float qf[8], knf[8];
@@ -301,6 +350,7 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(DecodeParams p) 
     for (int i = 0; i < 8; ++i) { knf[i] = 0.f; vnf[i] = 0.f; }
     if (holds_new) {
       norm_rot_row<D>(kn_raw, trig, dl, p.eps, knf);
+      const float gate = p.ve != nullptr ? gate_of_halves(gate_raw, p.gate.kind) : 0.f;
       norm_mix_row<D>(vn_raw, p.ve != nullptr, ve_raw, gate, p.eps, vnf);
     }
     vn_packed = F16C ? pack8_f16(vnf) : pack8(vnf);
@@ -334,8 +384,8 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(DecodeParams p) 
         kr[u] = kn_packed;
         vr[u] = vn_packed;
         if (p.write_back) {
-          *reinterpret_cast<u32x4*>(kbase + (int64_t)row * p.kc_sr) = kn_packed;
-          *reinterpret_cast<u32x4*>(vbase + (int64_t)row * p.vc_sr) = vn_packed;
+          *reinterpret_cast<u32x4*>(kcache + (int64_t)row * p.kc_sr + dl) = kn_packed;
+          *reinterpret_cast<u32x4*>(vcache + (int64_t)row * p.vc_sr + dl) = vn_packed;
         }
         if (PREP && p.k_rows != nullptr) {
           float f[8];
@@ -374,60 +424,56 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_kernel(DecodeParams p) 
     }
   };
 
-  for (; base < r1; base += 2 * STRIDE) {
+  while (base < r1) {
     consume(base, kA, vA);
-    load_set(base + 2 * STRIDE, kA, vA);
+    load_set(2 * STRIDE, kA, vA);
     if (base + STRIDE < r1) consume(base + STRIDE, kB, vB);
-    load_set(base + 3 * STRIDE, kB, vB);
+    load_set(3 * STRIDE, kB, vB);
+    base += 2 * STRIDE;
+    ka += 2 * STRIDE * k_step;
+    va += 2 * STRIDE * v_step;
   }
 
-  // Merge the row groups of this wavefront (lanes that differ above bit log2(LPR)).
+  // Merge the row groups of this wavefront, then the wavefronts through LDS: both against the common maximum.
+  const float wave_m = max_over_groups<LPR>(st.m);
+  const float scale = fast_exp2(st.m - (wave_m == -INFINITY ? 0.f : wave_m));
+  st.l = sum_over_groups<LPR>(st.l * scale);
 #pragma unroll
-  for (int off = LPR; off < 64; off <<= 1) {
-    SoftmaxState o;
-    o.m = __shfl_xor(st.m, off);
-    o.l = __shfl_xor(st.l, off);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o.acc[i] = __shfl_xor(st.acc[i], off);
-    merge_state(st, o);
-  }
-
-  // Merge the wavefronts through LDS.
+  for (int i = 0; i < 8; ++i) st.acc[i] = sum_over_groups<LPR>(st.acc[i] * scale);
   __shared__ float sm_m[kDecodeWaves], sm_l[kDecodeWaves];
-  __shared__ float sm_acc[kDecodeWaves][D];
+  __shared__ __attribute__((aligned(16))) float sm_acc[kDecodeWaves][D];
   if (lane < LPR) {
     if (lane == 0) {
-      sm_m[wave] = st.m;
+      sm_m[wave] = wave_m;
       sm_l[wave] = st.l;
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sm_acc[wave][dl + i] = st.acc[i];
+    *reinterpret_cast<f32x4*>(&sm_acc[wave][dl]) = f32x4{st.acc[0], st.acc[1], st.acc[2], st.acc[3]};
+    *reinterpret_cast<f32x4*>(&sm_acc[wave][dl + 4]) = f32x4{st.acc[4], st.acc[5], st.acc[6], st.acc[7]};
   }
   __syncthreads();
-  if (wave == 0 && lane < LPR) {
+  if (tid < D / 2) {               // two channels each
+    float m = sm_m[0], l = 0.f, acc[2] = {0.f, 0.f};
 #pragma unroll
-    for (int w = 1; w < kDecodeWaves; ++w) {
-      SoftmaxState o;
-      o.m = sm_m[w];
-      o.l = sm_l[w];
+    for (int w = 1; w < kDecodeWaves; ++w) m = fmaxf(m, sm_m[w]);
+    const float mu = (m == -INFINITY) ? 0.f : m;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o.acc[i] = sm_acc[w][dl + i];
-      merge_state(st, o);
+    for (int w = 0; w < kDecodeWaves; ++w) {
+      const float sc = fast_exp2(sm_m[w] - mu);
+      l = fmaf(sm_l[w], sc, l);
+      acc[0] = fmaf(sm_acc[w][2 * tid], sc, acc[0]);
+      acc[1] = fmaf(sm_acc[w][2 * tid + 1], sc, acc[1]);
     }
     if (p.nsplit == 1) {
-      const float inv = 1.f / st.l;
-      float of[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) of[i] = st.acc[i] * inv;
-      *reinterpret_cast<u32x4*>(p.o + b * p.o_sb + h * p.o_sh + dl) = pack8(of);
+      const float inv = 1.f / l;
+      *reinterpret_cast<uint32_t*>(p.o + b * p.o_sb + h * p.o_sh + 2 * tid) = pack_bf16x2(acc[0] * inv, acc[1] * inv);
     } else {
       float* part = p.partials + (((int64_t)b * p.H + h) * p.nsplit + split) * (D + 2);
-      if (lane == 0) {
-        part[0] = st.m;
-        part[1] = st.l;
+      if (tid == 0) {
+        part[0] = m;
+        part[1] = l;
       }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) part[2 + dl + i] = st.acc[i];
+      part[2 + 2 * tid] = acc[0];
+      part[2 + 2 * tid + 1] = acc[1];
     }
   }
 }
@@ -667,7 +713,7 @@ template <typename E>
 __global__ __launch_bounds__(64) void decode_scalar_kernel(DecodeParams p, int D) {
   const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
   const int half = D / 2;
-  const DecodeRange rg = decode_range(p);
+  const DecodeRange rg = decode_range(p, p.pos_dev != nullptr ? device_position(p) : 0);
   const E* qp = reinterpret_cast<const E*>(p.q) + b * p.q_sb + h * p.q_sh;
   const E* knp = reinterpret_cast<const E*>(p.k_new) + b * p.kn_sb + h * p.kn_sh;
   const E* vnp = reinterpret_cast<const E*>(p.v_new) + b * p.vn_sb + h * p.vn_sh;

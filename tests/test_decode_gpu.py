@@ -186,6 +186,25 @@ def test_attn_step_prepares_rows_and_attends_in_one_launch(B, H, D, W, mix, nspl
         assert_close_bf16(outs[0][0], o2.float(), f"one launch vs two, t={t}", max_abs=8e-3, mean_abs=3e-4)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("W,t,nsplit", [(9, 4, 64), (9, 9, 64), (70, 71, 2), (300, 555, 3)])
+def test_decode_splits_of_a_row_and_caches_of_other_strides(D, W, t, nsplit):
+    """Splits that hold nothing but the new row; rows, heads and sequences of the cache in any order in memory."""
+    test_decode_ring_matches_oracle(2, 3, D, W, t, nsplit)
+    g = torch.Generator(device="cuda").manual_seed(W + D)
+    k, v = (torch.randn(2, 3, W, D, generator=g, device="cuda").bfloat16() for _ in range(2))
+    rows = [torch.randn(2, 3, D, generator=g, device="cuda").bfloat16() for _ in range(3)]
+    n_rows, slot = min(t + 1, W), t % W
+    outs = []
+    for order in ((0, 1, 2, 3), (2, 0, 1, 3), (1, 2, 0, 3)):
+        back = [order.index(i) for i in range(4)]
+        kc, vc = (x.permute(order).contiguous().permute(back) for x in (k, v))
+        o = ops.decode_attention(*rows, kc, vc, n_rows=n_rows, new_idx=slot, write_back=True, nsplit=nsplit)
+        outs.append((o, kc, vc))
+    for got in outs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got, outs[0]))
+
+
 def test_decode_rejects_bad_arguments():
     z = torch.zeros(1, 1, 128, dtype=torch.bfloat16, device="cuda:0")
     rows = torch.zeros(1, 1, 4, 128, dtype=torch.bfloat16, device="cuda:0")
