@@ -113,9 +113,21 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 
 // ---- cross-lane sums with DPP (no LDS traffic) -------------------------------
 template <int CTRL>
-__device__ __forceinline__ float dpp_add(float x) {
-  int y = __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false);
-  return x + __int_as_float(y);
+__device__ __forceinline__ float dpp_move(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) { return x + dpp_move<CTRL>(x); }
+
+// x and its value in the neighbouring row of 16 lanes (rows 0 and 1, 2 and 3) or in the other half of the wavefront.
+struct LanePair { float x, y; };
+__device__ __forceinline__ LanePair row_pair(float x) {
+  const u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+  return {__uint_as_float(t.x), __uint_as_float(t.y)};
+}
+__device__ __forceinline__ LanePair half_pair(float x) {
+  const u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
+  return {__uint_as_float(t.x), __uint_as_float(t.y)};
 }
 
 // Sum over the LPR consecutive lanes that share a cache row; every lane of the
@@ -126,8 +138,12 @@ __device__ __forceinline__ float group_sum(float x) {
   x = dpp_add<0x4E>(x);                     // quad_perm [2,3,0,1]   (xor 2)
   if (LPR >= 8) x = dpp_add<0x141>(x);      // row_half_mirror       (joins the two quads of 8 lanes)
   if (LPR >= 16) x = dpp_add<0x128>(x);     // row_ror 8             (joins the two halves of 16 lanes)
-  if (LPR >= 32) x += __shfl_xor(x, 16);    // the neighbouring row of 16 lanes
+  if (LPR >= 32) { const LanePair t = row_pair(x); x = t.x + t.y; }
   return x;
+}
+__device__ __forceinline__ float wave_sum(float x) {
+  const LanePair t = half_pair(group_sum<32>(x));
+  return t.x + t.y;
 }
 
 // ---- asynchronous global -> LDS copies ------------------------------------------

@@ -197,11 +197,10 @@ struct SoftmaxState {
 // Maximum and sum over the row groups of a wavefront (lanes that agree modulo LPR = 8 or 16).
 template <int LPR, typename OP>
 __device__ __forceinline__ float over_groups(float x, OP op) {
-  if constexpr (LPR == 8) x = op(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false)));   // row_ror 8
-  u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-  x = op(__uint_as_float(t.x), __uint_as_float(t.y));
-  t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-  return op(__uint_as_float(t.x), __uint_as_float(t.y));
+  if constexpr (LPR == 8) x = op(x, dpp_move<0x128>(x));   // row_ror 8
+  const LanePair r = row_pair(x);
+  const LanePair t = half_pair(op(r.x, r.y));
+  return op(t.x, t.y);
 }
 template <int LPR> __device__ __forceinline__ float max_over_groups(float x) {
   return over_groups<LPR>(x, [](float a, float b) { return fmaxf(a, b); });
@@ -548,11 +547,13 @@ __global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(DecodeP
 // sequence both kernels are a memory round trip each, and so is the gap between them.  Every workgroup combines the whole row o
 // into LDS (a thread four channels), and each of its wavefronts multiplies it with one weight row.  What bounds it is what a
 // compute unit pulls out of the L2 (98 KB of partials for 12 heads of 128 and 16 splits), so all of a thread's partials and its
-// pieces of the weight row are requested first, and the splits' weights are worked out meanwhile, once per workgroup
-// (a first version, every thread on its own, took 1.5 us longer).  Sums in the order of decode_combine_kernel and
+// pieces of the weight row are requested first, the splits' maxima and sums ahead of them.  The splits' weights come out of those:
+// a lane looks after one split of its head, eight lanes hold a group, the maxima meet in cross-lane moves and the results go round
+// a wavefront's own corner of the LDS, without a barrier.  (Worked out once per workgroup, by loops over the splits between three
+// barriers, they were done 1.5 us after the maxima had arrived, now 0.2.)  Sums in the order of decode_combine_kernel and
 // linear_rows_kernel: the results are the same bits.
-// 12 heads of 128, ring of 8192: one layer's step launched eagerly 22.6 to 24.9 -> 21.4 us; twelve of them in a recorded step
-// 381.3 -> 381.0 us (6.1 us for this kernel where the two took 2.5 and 3.3 and a gap: a graph's nodes follow each other closely).
+// 12 heads of 128, ring of 8192: one layer's step launched eagerly 20.6 -> 19.5 us, twelve of them in a recorded step 372 -> 355 us
+// (two kernels in its place: 22 to 24 us a layer).
 struct CombineProjectParams {
   const float* partials;     // [H, nsplit, D + 2]
   int HD, nsplit;
@@ -566,21 +567,33 @@ constexpr int kProjectSplits = 32;                         // and H nsplit at mo
 template <int D, int G>
 __global__ __launch_bounds__(kProjectThreads) void decode_combine_project_kernel(CombineProjectParams p) {
   constexpr int S = 8 * G, PIECES = kProjectChannels / 8 / 64;
+  constexpr int T = D / 4, HEADS = 64 / T, REP = (S + T - 1) / T;   // threads of a head, heads of a wavefront, splits of a thread
   __shared__ __attribute__((aligned(16))) uint32_t row[kProjectChannels / 2];
-  __shared__ f32x2 ml[kProjectThreads];                 // [H][nsplit] maximum and sum of a split
-  __shared__ float ws[kProjectChannels / D * S];        // [H][S] weight of a split in its group (0: no such split)
-  __shared__ float wg[kProjectChannels / D * (G + 1)];  // [H][G + 1] weight of a group; the sum
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // Of a wavefront's heads, by group and split in it: weight in the group (0: no such split) and sum; weight of the group.
+  __shared__ __attribute__((aligned(16))) float ws[kProjectRows][HEADS][S], ls[kProjectRows][HEADS][S], wg[kProjectRows][HEADS][4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  asm volatile("" ::"s"(p.partials), "s"(p.HD), "s"(p.out.w), "s"(p.out.N));   // (one fetch of the arguments)
   const int H = p.HD / D, ns = p.nsplit, pieces = p.HD / 8;
-  const f32x2 my_ml = *reinterpret_cast<const f32x2*>(p.partials + (int64_t)min(tid, H * ns - 1) * (D + 2));
-  const int c = min(4 * tid, p.HD - 4), h = c / D;      // (threads past the end redo the last channels)
-  const float* part = p.partials + (int64_t)h * ns * (D + 2) + 2 + c % D;
-  f32x2 as[S][2];
+  const bool combines = 256 * wave < p.HD;
+  const int h = min(tid / T, H - 1), j = lane % T, hw = lane / T;   // (threads past the end redo the last head)
+  const uint32_t head = 4u * (uint32_t)(h * ns * (D + 2));          // bytes
+  f32x2 ml[REP];
+  f32x4 as[S];
+  if (combines) {
+    // Thread j looks after split u of group g for its head, with group g's in eight consecutive lanes.
 #pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const float* at = part + min(s, ns - 1) * (D + 2);  // 8-byte aligned
-    as[s][0] = *reinterpret_cast<const f32x2*>(at);
-    as[s][1] = *reinterpret_cast<const f32x2*>(at + 2);
+    for (int r = 0; r < REP; ++r) {
+      const int e = j + T * r, sp = (e / 8) % G + (e % 8) * G;
+      ml[r] = *reinterpret_cast<const f32x2*>((const char*)p.partials + (head + 4u * (uint32_t)(min(sp, ns - 1) * (D + 2))));
+    }
+    typedef f32x4 __attribute__((aligned(8))) f32x4_8;              // (a partial is D + 2 floats)
+    const char* at = (const char*)p.partials + 8;
+    const uint32_t mine = head + 16u * (uint32_t)j;
+#pragma unroll
+    for (int sp = 0; sp < S; ++sp) {
+      as[sp] = *reinterpret_cast<const f32x4_8*>(at + mine);
+      at += sp + 1 < ns ? 4 * (D + 2) : 0;
+    }
   }
   const int n = blockIdx.x * kProjectRows + wave;
   const uint16_t* wr = p.out.w + (int64_t)min(n, p.out.N - 1) * p.out.w_sn;
@@ -590,59 +603,64 @@ __global__ __launch_bounds__(kProjectThreads) void decode_combine_project_kernel
   for (int j = 0; j < PIECES; ++j) wv[j] = lane + 64 * j < pieces ? *reinterpret_cast<const u32x4*>(wr + 8 * (lane + 64 * j)) : zero;
   __builtin_amdgcn_sched_barrier(0);
 
-  // The barriers wait for LDS only: the loads stay in flight.
-  auto publish = [] {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-  if (tid < H * ns) ml[tid] = my_ml;
-  publish();
-  for (int i = tid; i < H * S; i += kProjectThreads) {
-    const int hh = i / S, s = i % S, g = s % G;
-    float m = -INFINITY;
-    for (int u = g; u < ns; u += G) m = fmaxf(m, ml[hh * ns + u][0]);
-    const float mu = (m == -INFINITY) ? 0.f : m;
-    ws[i] = s < ns ? fast_exp2(ml[hh * ns + s][0] - mu) : 0.f;
-    if (s < G) {
-      float mt = m;
-      for (int u = 0; u < ns; ++u) mt = fmaxf(mt, ml[hh * ns + u][0]);
-      const float mut = (mt == -INFINITY) ? 0.f : mt;
-      wg[hh * (G + 1) + s] = fast_exp2(m - mut);
+  if (combines) {
+    float m[REP], mt = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < REP; ++r) {
+      const int e = j + T * r, sp = (e / 8) % G + (e % 8) * G;
+      if (sp >= ns) ml[r] = f32x2{-INFINITY, 0.f};
+      m[r] = ml[r][0];
+      m[r] = fmaxf(m[r], dpp_move<0xB1>(m[r]));                     // over eight lanes
+      m[r] = fmaxf(m[r], dpp_move<0x4E>(m[r]));
+      m[r] = fmaxf(m[r], dpp_move<0x141>(m[r]));
+      mt = fmaxf(mt, m[r]);
     }
-  }
-  publish();
-  if (tid < H) {
-    float lt = 0.f;
+    mt = fmaxf(mt, dpp_move<0x128>(mt));                            // over the head's lanes
+    if (T == 32) {
+      const LanePair t = row_pair(mt);
+      mt = fmaxf(t.x, t.y);
+    }
+    const float mut = (mt == -INFINITY) ? 0.f : mt;
+#pragma unroll
+    for (int r = 0; r < REP; ++r) {
+      const int e = j + T * r, g = (e / 8) % G, sp = g + (e % 8) * G, slot = 8 * g + e % 8;
+      const float mu = (m[r] == -INFINITY) ? 0.f : m[r];
+      ws[wave][hw][slot] = sp < ns ? fast_exp2(ml[r][0] - mu) : 0.f;
+      ls[wave][hw][slot] = ml[r][1];
+      wg[wave][hw][g] = fast_exp2(m[r] - mut);
+    }
+    if (ns < S) {                       // (an infinite value of the last split must not meet a weight of 0)
+#pragma unroll
+      for (int sp = 0; sp < S; ++sp)
+        if (sp >= ns) as[sp] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    asm volatile("" ::: "memory");      // (a wavefront's LDS accesses are carried out in order)
+    float t[4] = {0.f, 0.f, 0.f, 0.f}, lt = 0.f;
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      float l = 0.f;
-      for (int u = g; u < ns; u += G) l = fmaf(ml[tid * ns + u][1], ws[tid * S + u], l);
-      lt = G > 1 ? fmaf(l, wg[tid * (G + 1) + g], lt) : l;
-    }
-    wg[tid * (G + 1) + G] = lt;
-  }
-  publish();
-
-  float t[4] = {0.f, 0.f, 0.f, 0.f};
+      float a[4] = {0.f, 0.f, 0.f, 0.f}, l = 0.f;
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float a[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int u4 = 0; u4 < 2; ++u4) {
+        const f32x4 w4 = *reinterpret_cast<const f32x4*>(&ws[wave][hw][8 * g + 4 * u4]);
+        const f32x4 l4 = *reinterpret_cast<const f32x4*>(&ls[wave][hw][8 * g + 4 * u4]);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int s = g + u * G;
-      const float w = ws[h * S + s];
-      if (s < ns) {          // (an infinite value of the last split must not meet a weight of 0)
+        for (int u = 0; u < 4; ++u) {
+          l = fmaf(l4[u], w4[u], l);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a[e] = fmaf(as[s][e / 2][e % 2], w, a[e]);
+          for (int e = 0; e < 4; ++e) a[e] = fmaf(as[g + (4 * u4 + u) * G][e], w4[u], a[e]);
+        }
       }
-    }
+      const float wgg = wg[wave][hw][g];
+      lt = G > 1 ? fmaf(l, wgg, lt) : l;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) t[e] = G > 1 ? fmaf(a[e], wg[h * (G + 1) + g], t[e]) : a[e];
+      for (int e = 0; e < 4; ++e) t[e] = G > 1 ? fmaf(a[e], wgg, t[e]) : a[e];
+    }
+    if (4 * tid < p.HD) *reinterpret_cast<u32x2*>(&row[2 * tid]) = u32x2{pack_bf16x2(t[0] / lt, t[1] / lt), pack_bf16x2(t[2] / lt, t[3] / lt)};
   }
-  const float lt = wg[h * (G + 1) + G];
-  if (4 * tid < p.HD) *reinterpret_cast<u32x2*>(&row[2 * tid]) = u32x2{pack_bf16x2(t[0] / lt, t[1] / lt), pack_bf16x2(t[2] / lt, t[3] / lt)};
-  publish();
+  // The barrier waits for LDS only: the weights stay in flight.
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
   float acc = 0.f;
 #pragma unroll
   for (int j = 0; j < PIECES; ++j) {
@@ -653,8 +671,7 @@ __global__ __launch_bounds__(kProjectThreads) void decode_combine_project_kernel
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc = fmaf(wf[i], xf[i], acc);
   }
-  acc = group_sum<32>(acc);
-  acc += __shfl_xor(acc, 32);
+  acc = wave_sum(acc);
   if (lane == 0 && n < p.out.N) p.out.y[n] = (uint16_t)(pack_bf16x2(acc, 0.f) & 0xffffu);
 }
 

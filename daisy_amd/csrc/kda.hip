@@ -252,9 +252,6 @@ __device__ __forceinline__ u32x2 lds_column4(lds_cptr p) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)p));
 }
 // The value that another lane of the same 16 holds: lane N of them, or by a pattern inside every quad.
-template <int CTRL> __device__ __forceinline__ float dpp_move(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
-}
 template <int N> __device__ __forceinline__ float from_row(float x) { return dpp_move<0x150 + N>(x); }
 __device__ __forceinline__ float sum_over_q4(float x) {       // over the four lanes that share a row of an operand
   x += __shfl_xor(x, 16);

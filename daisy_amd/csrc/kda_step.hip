@@ -166,11 +166,9 @@ __global__ __launch_bounds__(256) void kda_recurrent_kernel(KdaStepParams p) {
 // (128 registers).  The products run on the matrix cores, weights as left operand and all sixteen columns of the right
 // operand the same row: fifteen of them are waste, but nothing is unpacked and nothing summed across lanes.
 __device__ __forceinline__ float sum_over_rows(float x) {          // lane bits 3, 4, 5
-  x = dpp_add<0x128>(x);                 // row_ror 8
-  u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-  x = __uint_as_float(t.x) + __uint_as_float(t.y);
-  t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false));
-  return __uint_as_float(t.x) + __uint_as_float(t.y);
+  const LanePair r = row_pair(dpp_add<0x128>(x));                   // row_ror 8
+  const LanePair t = half_pair(r.x + r.y);
+  return t.x + t.y;
 }
 template <int KD, int VD>
 __global__ __launch_bounds__(4 * VD, 4) void kda_layer_step_kernel(KdaLayerStep p) {

@@ -29,11 +29,6 @@ struct LinearSegmentsParams {
 
 constexpr int kLinearMaxRows = 8;
 
-__device__ __forceinline__ float wave_sum(float x) {
-  x = group_sum<32>(x);
-  return x + __shfl_xor(x, 32);
-}
-
 // M activation rows, R weight rows per wavefront, P 16-byte pieces of every row in flight per lane; one wavefront
 // per workgroup.
 template <int M, int R, int P, bool SEGMENTS>
