@@ -339,6 +339,13 @@ def _as_bf16(t: Optional[Tensor]) -> Optional[Tensor]:
     return t if t is None or t.dtype is torch.bfloat16 else t.to(torch.bfloat16)
 
 
+def _held(store: dict, module: nn.Module, name: str):
+    """``module.name`` for a parameter, buffer or submodule, straight from the dictionary that holds it: by way of
+    ``nn.Module.__getattr__`` the five names of a one-call step cost the host more than a microsecond."""
+    held = store.get(name)
+    return getattr(module, name) if held is None else held
+
+
 class CausalSelfAttention(nn.Module):
     """Merged-QKVO sliding-window causal self-attention (models/daisy/attention.py:73-202)."""
 
@@ -399,7 +406,7 @@ class CausalSelfAttention(nn.Module):
 
     def _fused_prep_ok(self) -> bool:
         # The one-pass norm + RoPE + ve-mix kernel works on bf16 rows of 64 or 128 channels.
-        return self.fused_prep and self.qkvo_w.dtype == torch.bfloat16 and self.head_dim in (64, 128)
+        return self.fused_prep and self.head_dim in (64, 128) and _held(self._parameters, self, "qkvo_w").dtype is torch.bfloat16
 
     def _project_qkv_fused(self, x: Tensor, ve: Optional[Tensor], pos0: int, k_out=None, v_out=None):
         """QKV projection, then norm + RoPE (rows ``pos0 + t``) + ve mix in one kernel; ``[B, T, H, D]``.
@@ -433,12 +440,13 @@ class CausalSelfAttention(nn.Module):
         window = mask.window or mask.span
         dest = kv_out if kv_out is not None else mask.kv_out
         if self._fused_prep_ok():
-            rot = self.rotary
+            rot = _held(self._modules, self, "rotary")
             k_dest, v_dest = dest if dest is not None else (None, None)
             x, ve = _as_bf16(x), _as_bf16(ve) if self.receives_ve else None
             fast = _lib.native().layer_prefill(
-                x, self.qkvo_w, rot.cos, rot.sin, self.num_heads, self.head_dim, window or 0, mask.doc_start,
-                ve, self.g_ve, k_dest, v_dest, float(self.attn_scale), NORM_EPS_BF16,
+                x, _held(self._parameters, self, "qkvo_w"), _held(rot._buffers, rot, "cos"), _held(rot._buffers, rot, "sin"),
+                self.num_heads, self.head_dim, window or 0, mask.doc_start,
+                ve, _held(self._parameters, self, "g_ve") if self.receives_ve else None, k_dest, v_dest, float(self.attn_scale), NORM_EPS_BF16,
                 STEP_ROWS_KERNEL_MAX, bool(want_q))
             if fast is not None:
                 return fast
@@ -589,9 +597,10 @@ class CausalSelfAttention(nn.Module):
         rows' way into slot ``pos % W`` and the attention over the ring all happen in
         ``ops.attn_step``.  Returns the new rows as views of the ring, or ``None, None`` when only
         the device knows the position."""
-        rot = self.rotary
+        rot = _held(self._modules, self, "rotary")
         x, ve = _as_bf16(x), _as_bf16(ve) if self.receives_ve else None
-        fast = _lib.native().layer_step(x, self.qkvo_w, ring.k, ring.v, pos, rot.cos, rot.sin, ve, self.g_ve,
+        fast = _lib.native().layer_step(x, _held(self._parameters, self, "qkvo_w"), ring.k, ring.v, pos, _held(rot._buffers, rot, "cos"),
+                                        _held(rot._buffers, rot, "sin"), ve, _held(self._parameters, self, "g_ve") if self.receives_ve else None,
                                         ring.status if isinstance(pos, Tensor) else None, float(self.attn_scale),
                                         NORM_EPS_BF16, STEP_ROWS_KERNEL_MAX)
         if fast is not None:
