@@ -309,8 +309,15 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
 // 17.9 us in the library; M = 64, N = 6144, K = 2048: 7.3 us with 32 x 64, 9.7 us in the library (a KDA decode step's six input projections in
 // one launch: 8.3 us, one by one 42 us); M = 8192,
 // N = 6144, K = 2048: 155 us with 256 x 256, 178 us with 128 x 128, 141 us in the library.)
+// The two smallest are for products whose 32 x 64 tiles leave most compute units idle: what a workgroup then waits for is its own
+// K * (bm + bn) operands, at the 60 to 150 GB/s that one compute unit pulls, and smaller tiles on more of them have less of it
+// each (weights from memory: M = 64, N = K = 2048: 9.6 us with 32 x 64, 7.1 with 32 x 32, 6.7 with 16 x 32; M = 128: 9.4, 7.1, 9.0;
+// M = 16, N = 4608, K = 1536: 8.2, 6.35, 6.2; M = N = K = 256: 2.65, 2.5, 2.4).  16 rows only while all rows of tiles are one panel:
+// beyond, the weights are read twice (M = 200, N = K = 512: 3.2, 3.0, 3.3).
 struct ProjTile { int code, bm, bn, bk, per_cu; float one, full; };
 constexpr ProjTile kProjTiles[] = {
+    {9, 16, 32, 128, 3, 3.6f, 6.6f},      // 2 wavefronts, 4 stages
+    {10, 32, 32, 128, 2, 4.0f, 6.6f},     // 4 wavefronts, 4 stages
     {1, 32, 64, 128, 2, 5.8f, 8.0f},      // 4 wavefronts, 3 stages
     {2, 64, 64, 128, 1, 7.2f, 7.2f},      // 8 wavefronts, 4 stages
     {3, 64, 128, 128, 1, 10.3f, 10.3f},   // 8 wavefronts, 3 stages
@@ -325,6 +332,7 @@ static int proj_tile(int M, int K, int head, COLUMNS columns) {
   float least = 0.f;
   for (const ProjTile& t : kProjTiles) {
     if (K % t.bk != 0 || t.bn % head != 0) continue;    // (head: a tile of the QKV projection holds whole heads)
+    if (t.bm == 16 && M > 8 * t.bm) continue;
     const int64_t n = (int64_t)((M + t.bm - 1) / t.bm) * columns(t.bn), round = 256 * t.per_cu;
     const int64_t tail = n % round;
     const float cost = (float)(n / round) * t.full + (tail > 256 ? t.full : tail > 0 ? t.one : 0.f);
@@ -362,10 +370,14 @@ static int launch_proj(ProjSegmentsParams& p, hipStream_t s) {
 template <int EPI, typename PARAMS>
 static int dispatch_proj(int tile, PARAMS& p, hipStream_t s) {
   for (const ProjTile& t : kProjTiles)
-    DAISY_CHECK_SUPPORTED(t.code != tile || (p.K % t.bk == 0 && !(EPI == 2 && t.bn % 128 != 0) && !(EPI == 3 && t.code == 7)),
+    DAISY_CHECK_SUPPORTED(t.code != tile || (p.K % t.bk == 0 && !(EPI == 2 && t.bn % 128 != 0) && !(EPI == 1 && t.bn % 64 != 0) && !(EPI == 3 && t.code == 7)),
                           "proj: tile %d does not serve K=%d with epilogue %d", tile, p.K, EPI);
   if constexpr (EPI != 2) {
     if (tile == 1) return launch_proj<32, 64, 2, 2, 128, 3, EPI>(p, s);
+    if constexpr (EPI != 1) {
+      if (tile == 10) return launch_proj<32, 32, 2, 2, 128, 4, EPI>(p, s);
+      if (tile == 9) return launch_proj<16, 32, 1, 2, 128, 4, EPI>(p, s);
+    }
     if (tile == 2) return launch_proj<64, 64, 2, 4, 128, 4, EPI>(p, s);
   }
   if constexpr (EPI != 3) {

@@ -28,6 +28,25 @@ def test_tiles_against_fp64(tile, K, M, N):
         assert (err <= r.abs() * 2 ** -8 + K ** 0.5 * 1e-5 + 1e-3).all(), err.max().item()
 
 
+@pytest.mark.parametrize("tile,K", [(10, 128), (10, 640), (9, 256), (9, 512)])
+@pytest.mark.parametrize("M,N", [(1, 8), (15, 32), (17, 40), (33, 200), (130, 72)])
+def test_smallest_tiles_against_fp64(tile, K, M, N):
+    """Remainders of tiles of 16 and 32 rows and 32 columns; fewer K steps than stages, and more."""
+    test_tiles_against_fp64(tile, K, M, N)
+
+
+@pytest.mark.parametrize("M", [5, 16, 17, 100, 128, 129, 200])
+def test_products_on_both_sides_of_the_smallest_tiles_rule(M):
+    """The rule by sizes gives the bits of the tiles it picks among (same order of the sums in all of them)."""
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, 512, generator=g, device=DEV).bfloat16()
+    w = torch.randn(520, 512, generator=g, device=DEV).bfloat16()
+    with torch.no_grad():
+        y = _lib.native().linear(x, w, None, 4, 0)
+        for tile in (1, 9, 10):
+            assert torch.equal(y, _lib.native().linear(x, w, None, 4, tile))
+
+
 @pytest.mark.parametrize("H,D", [(2, 128), (6, 64), (3, 64)])
 @pytest.mark.parametrize("B,T", [(1, 5), (2, 64), (1, 129), (3, 200), (1, 1100)])
 @pytest.mark.parametrize("ve", [False, True])
