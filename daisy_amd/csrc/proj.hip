@@ -313,13 +313,16 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
 // K * (bm + bn) operands, at the 60 to 150 GB/s that one compute unit pulls, and smaller tiles on more of them have less of it
 // each (weights from memory: M = 64, N = K = 2048: 9.6 us with 32 x 64, 7.1 with 32 x 32, 6.7 with 16 x 32; M = 128: 9.4, 7.1, 9.0;
 // M = 16, N = 4608, K = 1536: 8.2, 6.35, 6.2; M = N = K = 256: 2.65, 2.5, 2.4).  16 rows only while all rows of tiles are one panel:
-// beyond, the weights are read twice (M = 200, N = K = 512: 3.2, 3.0, 3.3).
+// beyond, the weights are read twice (M = 200, N = K = 512: 3.2, 3.0, 3.3).  32 x 128 does the same for the QKV projection, whose
+// narrower tiles would not hold a head of 128 (a layer of 12 heads, 100 tokens: 21.2 us with 64 x 128, 19.5; 160 tokens: 22.6, 21.1; in
+// two rounds it loses: 256 tokens 23.7, 28.1); with heads of 64, 32 x 64 stays ahead of it (16 heads, 100 tokens: 14.7, 15.4).
 struct ProjTile { int code, bm, bn, bk, per_cu; float one, full; };
 constexpr ProjTile kProjTiles[] = {
     {9, 16, 32, 128, 3, 3.6f, 6.6f},      // 2 wavefronts, 4 stages
     {10, 32, 32, 128, 2, 4.0f, 6.6f},     // 4 wavefronts, 4 stages
     {1, 32, 64, 128, 2, 5.8f, 8.0f},      // 4 wavefronts, 3 stages
     {2, 64, 64, 128, 1, 7.2f, 7.2f},      // 8 wavefronts, 4 stages
+    {11, 32, 128, 128, 1, 8.3f, 8.3f},    // 8 wavefronts, 3 stages; QKV projection with heads of 128 only
     {3, 64, 128, 128, 1, 10.3f, 10.3f},   // 8 wavefronts, 3 stages
     {4, 64, 128, 64, 2, 12.3f, 19.0f},    // 4 wavefronts, 3 stages
     {5, 128, 128, 64, 1, 15.8f, 15.8f},   // 8 wavefronts, 4 stages
@@ -332,7 +335,7 @@ static int proj_tile(int M, int K, int head, COLUMNS columns) {
   float least = 0.f;
   for (const ProjTile& t : kProjTiles) {
     if (K % t.bk != 0 || t.bn % head != 0) continue;    // (head: a tile of the QKV projection holds whole heads)
-    if (t.bm == 16 && M > 8 * t.bm) continue;
+    if ((t.bm == 16 && M > 8 * t.bm) || (t.code == 11 && head != 128)) continue;
     const int64_t n = (int64_t)((M + t.bm - 1) / t.bm) * columns(t.bn), round = 256 * t.per_cu;
     const int64_t tail = n % round;
     const float cost = (float)(n / round) * t.full + (tail > 256 ? t.full : tail > 0 ? t.one : 0.f);
@@ -370,7 +373,7 @@ static int launch_proj(ProjSegmentsParams& p, hipStream_t s) {
 template <int EPI, typename PARAMS>
 static int dispatch_proj(int tile, PARAMS& p, hipStream_t s) {
   for (const ProjTile& t : kProjTiles)
-    DAISY_CHECK_SUPPORTED(t.code != tile || (p.K % t.bk == 0 && !(EPI == 2 && t.bn % 128 != 0) && !(EPI == 1 && t.bn % 64 != 0) && !(EPI == 3 && t.code == 7)),
+    DAISY_CHECK_SUPPORTED(t.code != tile || (p.K % t.bk == 0 && !(EPI == 2 && t.bn % 128 != 0) && !(EPI == 1 && t.bn % 64 != 0) && !(EPI != 2 && t.code == 11) && !(EPI == 3 && t.code == 7)),
                           "proj: tile %d does not serve K=%d with epilogue %d", tile, p.K, EPI);
   if constexpr (EPI != 2) {
     if (tile == 1) return launch_proj<32, 64, 2, 2, 128, 3, EPI>(p, s);
@@ -379,6 +382,9 @@ static int dispatch_proj(int tile, PARAMS& p, hipStream_t s) {
       if (tile == 9) return launch_proj<16, 32, 1, 2, 128, 4, EPI>(p, s);
     }
     if (tile == 2) return launch_proj<64, 64, 2, 4, 128, 4, EPI>(p, s);
+  }
+  if constexpr (EPI == 2) {
+    if (tile == 11) return launch_proj<32, 128, 2, 4, 128, 3, EPI>(p, s);
   }
   if constexpr (EPI != 3) {
     if (tile == 7) return launch_proj<256, 256, 2, 4, 64, 2, EPI>(p, s);
