@@ -35,6 +35,21 @@ def test_smallest_tiles_against_fp64(tile, K, M, N):
     test_tiles_against_fp64(tile, K, M, N)
 
 
+@pytest.mark.parametrize("M", [2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("N,K", [(1024, 192), (2048, 64), (2056, 128), (5464, 128), (8200, 64), (16392, 72), (1024, 72)])
+def test_few_rows_on_both_sides_of_the_rule_against_fp64(M, N, K):
+    """Rows and columns on either side of where the weight-streaming kernel hands over to the tiled one, and sizes that one refuses."""
+    g = torch.Generator().manual_seed(M * N)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), torch.randn(N, K, generator=g).bfloat16()
+    with torch.no_grad():
+        y = _lib.native().linear(x.to(DEV), w.to(DEV), None, 4, 0)
+    assert (y is None) == (M > 4 and K % 64 != 0)
+    if y is not None:
+        r = x.double() @ w.double().t()
+        err = (y.cpu().double() - r).abs()
+        assert (err <= r.abs() * 2 ** -8 + K ** 0.5 * 1e-5 + 1e-3).all(), err.max().item()
+
+
 @pytest.mark.parametrize("M", [5, 16, 17, 100, 128, 129, 200])
 def test_products_on_both_sides_of_the_smallest_tiles_rule(M):
     """The rule by sizes gives the bits of the tiles it picks among (same order of the sums in all of them)."""
