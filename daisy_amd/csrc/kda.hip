@@ -95,7 +95,8 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 // Numerics: the 16x16 blocks of A and P run on MFMA with both operands referenced to the row before the block (every
 // exponent <= 0 off the diagonal); a diagonal block whose total decay exceeds exp(-80) is referenced to its middle row
 // instead (exponents up to the decay of 8 rows either way); when those go beyond exp(-80) it is taken by halves, of 8, 4, 2 and
-// 1 rows, in two-term bf16 splits: no exponent is ever positive, so strong decays cannot overflow.
+// 1 rows: no exponent is ever positive, so strong decays cannot overflow.  These products are in two-term bf16 splits (2^-17)
+// and, where four rows alone decay beyond exp(-80), in fp32.
 // T is computed in fp32; the products with T, the state update and the output's second term use two-term bf16 splits of
 // both operands (three MFMAs each, relative error ~2^-17), which keeps the state error near fp32.
 // ===========================================================================
@@ -384,8 +385,8 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   const float rk = p.l2norm ? rsqrtf(sum_over_q4(sk) + p.l2eps) : 1.f;
   const float rq = p.scale * (p.l2norm ? rsqrtf(sum_over_q4(sq) + p.l2eps) : 1.f);
 
-  // ---- factors.  How steep the block is (wavefront-uniform): 0 while exp(-G) of every element is safe (exponents up to
-  // 80), 1 while that holds with the block's middle row as reference, 2 beyond. ----
+  // ---- factors.  How steep the block is (wavefront-uniform): `gentle` while exp(-G) of every element is safe (exponents up to
+  // 80); else with the block's middle row as reference while that is; else, or where a group of four rows is `steepest`, by halves. ----
   constexpr float kSafe = 80.f * kLog2e;
   float far0 = 0.f;
 #pragma unroll
@@ -398,15 +399,17 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   // columns j = 4 q4 + r.
   f32x4 accA = {0.f, 0.f, 0.f, 0.f}, accP = {0.f, 0.f, 0.f, 0.f};
   if (!gentle) {
-    float far7 = 0.f;
+    float far7 = 0.f, far4 = 0.f;
 #pragma unroll
     for (int m = 0; m < NM; ++m)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float g = G[m][e & 1][e >> 1];
         far7 = fmaxf(far7, fabsf(g - from_row<7>(g)));
+        far4 = fmaxf(far4, fabsf(g - dpp_move<0x114>(g)));      // row_shr 4, zero for the first four: in row 4 n + 3 the sum of rows 4 n ..
       }
-    if (!__any(far7 > kSafe)) {
+    const bool steepest = __any((li & 3) == 3 && far4 > kSafe);
+    if (!steepest && !__any(far7 > kSafe)) {
       // With the middle row as reference the entries above the diagonal may overflow; nothing reads them.
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
@@ -426,7 +429,9 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
       // Any decay: rows and columns that differ first in bit `lev` of their number meet at the last row of the lower half of
       // their group of 2 lev rows.  The lane's row is on the row's side of that product or on the column's, never on both,
       // so a level takes one exponential per element, of a sum of log-decays; entries of other levels are dropped.  Both
-      // operands in two bf16 terms: such blocks used to be summed in fp32 pair by pair, and lose no precision here.
+      // operands in two bf16 terms, 2^-18 of either; in a block with a steepest group of four as they are, on the fp32 instructions
+      // (27 % of the blocks of 6001 rows, 12 heads of 64, with a layer's first gates: both kernels 45.3 us in two terms, 47.5 with
+      // products of 16 x 16 at every level, 46.2 with those of 4 x 4 below).
       float pd = 0.f;
 #pragma unroll
       for (int m = 0; m < NM; ++m)
@@ -435,8 +440,9 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
       pd = sum_over_q4(pd);
 #pragma unroll
       for (int r = 0; r < 4; ++r) accP[r] = (4 * q4 + r == li) ? pd : 0.f;
-      auto level = [&](auto lev_, auto ref_of) {
+      auto level = [&](auto lev_, auto exact_, auto ref_of) {
         constexpr int lev = decltype(lev_)::value;
+        constexpr bool exact = decltype(exact_)::value;
         const bool low = (li & lev) == 0;
         f32x4 pa = {0.f, 0.f, 0.f, 0.f}, pp = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -448,16 +454,40 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
             wk[e] = kn[m][e] * f;
             wq[e] = qn[m][e] * f;
           }
-          u32x4 kh, kl, qh, ql;
-          split_pack8(wk, kh, kl);
-          split_pack8(wq, qh, ql);
-          auto add = [&](const u32x4& col, const u32x4& row_k, const u32x4& row_q) {
-            pa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, row_k), __builtin_bit_cast(bf16x8, col), pa, 0, 0, 0);
-            pp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, col), __builtin_bit_cast(bf16x8, row_q), pp, 0, 0, 0);
-          };
-          add(kl, kh, qh);
-          add(kh, kl, ql);
-          add(kh, kh, qh);
+          if constexpr (exact && lev <= 4) {
+            // Inside four rows, and of four rows with the four before them (row_shr 4): a product per group of four and q4, in a
+            // quarter of the 16 x 16 one's time.
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float col = lev == 4 ? dpp_move<0x114>(wk[e]) : wk[e];
+              pa = __builtin_amdgcn_mfma_f32_4x4x1f32(wk[e], col, pa, 0, 0, 0);
+              pp = __builtin_amdgcn_mfma_f32_4x4x1f32(col, wq[e], pp, 0, 0, 0);
+            }
+          } else if constexpr (exact) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              pa = __builtin_amdgcn_mfma_f32_16x16x4f32(wk[e], wk[e], pa, 0, 0, 0);
+              pp = __builtin_amdgcn_mfma_f32_16x16x4f32(wk[e], wq[e], pp, 0, 0, 0);
+            }
+          } else {
+            u32x4 kh, kl, qh, ql;
+            split_pack8(wk, kh, kl);
+            split_pack8(wq, qh, ql);
+            auto add = [&](const u32x4& col, const u32x4& row_k, const u32x4& row_q) {
+              pa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, row_k), __builtin_bit_cast(bf16x8, col), pa, 0, 0, 0);
+              pp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, col), __builtin_bit_cast(bf16x8, row_q), pp, 0, 0, 0);
+            };
+            add(kl, kh, qh);
+            add(kh, kl, ql);
+            add(kh, kh, qh);
+          }
+        }
+        if constexpr (exact && lev <= 4) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            pa[r] = sum_over_q4(lev == 4 ? dpp_move<0x104>(pa[r]) : pa[r]);        // (row_shl 4: back to the column's lane)
+            pp[r] = sum_over_q4(pp[r]);
+          }
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -465,10 +495,13 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
           if (x >= lev && x < 2 * lev) { accA[r] = pa[r]; accP[r] = pp[r]; }
         }
       };
-      level(std::integral_constant<int, 8>{}, [&](float g) { return from_row<7>(g); });
-      level(std::integral_constant<int, 4>{}, [&](float g) { const float lower = from_row<3>(g), upper = from_row<11>(g); return (li & 8) ? upper : lower; });
-      level(std::integral_constant<int, 2>{}, [&](float g) { return dpp_move<0x55>(g); });        // row 1 of every quad
-      level(std::integral_constant<int, 1>{}, [&](float g) { return dpp_move<0xA0>(g); });        // the even row of every pair
+      auto levels = [&](auto exact) {
+        level(std::integral_constant<int, 8>{}, exact, [&](float g) { return from_row<7>(g); });
+        level(std::integral_constant<int, 4>{}, exact, [&](float g) { const float lower = from_row<3>(g), upper = from_row<11>(g); return (li & 8) ? upper : lower; });
+        level(std::integral_constant<int, 2>{}, exact, [&](float g) { return dpp_move<0x55>(g); });        // row 1 of every quad
+        level(std::integral_constant<int, 1>{}, exact, [&](float g) { return dpp_move<0xA0>(g); });        // the even row of every pair
+      };
+      if (steepest) levels(std::true_type{}); else levels(std::false_type{});
     }
   }
   // k f and q f with f = exp(G) take the place of k and q, kd = exp(G_15 - G) k that of G.

@@ -91,3 +91,32 @@ def test_kda_workspace_sizes_agree(T, H):
         part = [t[:, :, h:h + 8].contiguous() for t in (q, k, v, gl, beta)]
         o8, S8 = chunk_kda(*part, **kw)
         assert torch.equal(o[:, :, h:h + 8], o8) and torch.equal(S[:, h:h + 8], S8)
+
+
+# One key channel carries everything and decays by a step whose factor two bf16 terms hold worst (2^-18 off, the same way in every
+# link), beta = -2: errors of A add up over the links of the triangle's inverse.  Eight other channels make the block steep.  What every
+# block leaves: three splits in two terms and a dropped product of the lower ones, 2^-18 each, and fp32's roundings over 16 links.
+# Blocks whose steep rows lie eight apart have A's operands in two terms too: three times 2^-18 in each link.
+FP32_LINKS, TWO_TERM_LINKS = 4 * 2 ** -18 + 16 * 2 ** -22, 4 * 2 ** -18 + 16 * 3 * 2 ** -18
+
+
+@pytest.mark.parametrize("Dk", [64, 128])
+@pytest.mark.parametrize("steep,bound", [
+    (lambda g: g.fill_(-25.), FP32_LINKS),              # every group of four rows beyond exp(-80)
+    (lambda g: g[:, 0].fill_(-100.), FP32_LINKS),       # the first row alone
+    (lambda g: g[:, 6].fill_(-100.), FP32_LINKS),
+    (lambda g: g[:, 15].fill_(-100.), FP32_LINKS),      # the last one, on no side of any difference of the block
+    (lambda g: g.fill_(-12.), TWO_TERM_LINKS),          # eight rows beyond it, four not
+], ids=["all", "first", "one", "last", "eight"])
+def test_kda_steep_blocks_against_fp64(Dk, steep, bound):
+    q, k, v, _, _ = _inputs(1, 16, 2, Dk, 32, seed=Dk)
+    k.zero_()[..., 0] = 1
+    gl = torch.zeros(1, 16, 2, Dk)
+    gl[..., 0] = -0.2197265625
+    steep(gl[..., -8:])
+    beta = torch.full((1, 16, 2), -2.)
+    _, S_ref = oracle.kda_recurrent(q, k, v, gl, beta, use_qk_l2norm=False, dtype=torch.float64)
+    _, S = chunk_kda(q.cuda(), k.cuda(), v.cuda(), gl.cuda(), beta.cuda(), output_final_state=True)
+    err = ((S.cpu().double() - S_ref).norm() / S_ref.norm()).item()
+    print(f"state error {err:.2e} of {bound:.2e}")
+    assert err <= bound
