@@ -348,6 +348,9 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   }
 
   // ---- G: running log-decay inside the block, in units of log 2; element e of group m is G[m][e % 2][e / 2] ----
+  // The product multiplies rows behind a position by 0, which an infinite log-decay must not meet: one below kForgets counts as that,
+  // whose exponential is 0 in fp32 already (and sums over many such rows keep the bits of the mild ones).  NaN stays NaN.
+  constexpr float kForgets = -104.f;
   f32x4 G[NM][2];
 #pragma unroll
   for (int m = 0; m < NM; ++m) G[m][0] = G[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -358,6 +361,8 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     for (int m = 0; m < NM; ++m) {
       float g0 = p.g_bf16 ? bf16lo_to_f32(graw[m][s].x) : __uint_as_float(graw[m][s].x);
       float g1 = p.g_bf16 ? bf16hi_to_f32(graw[m][s].x) : __uint_as_float(graw[m][s].y);
+      g0 = __builtin_elementwise_maximum(g0, kForgets);
+      g1 = __builtin_elementwise_maximum(g1, kForgets);
       if (edge && (16 * I + 4 * s + q4 >= n_live || 32 * m + 8 * (li >> 2) >= p.Dk)) g0 = g1 = 0.f;
       G[m][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(g0, ones, G[m][0], 0, 0, 0);
       G[m][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g1, ones, G[m][1], 0, 0, 0);

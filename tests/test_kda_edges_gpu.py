@@ -120,3 +120,24 @@ def test_kda_steep_blocks_against_fp64(Dk, steep, bound):
     err = ((S.cpu().double() - S_ref).norm() / S_ref.norm()).item()
     print(f"state error {err:.2e} of {bound:.2e}")
     assert err <= bound
+
+
+# A log-decay of minus infinity forgets its channel.  Rows at either side of the blocks of 16 and the chunks of 32.
+@pytest.mark.parametrize("Dk", [64, 128])
+@pytest.mark.parametrize("rows", [(31,), (0,), (15, 16), (32, 63), (5, 6, 40), (62, 63)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_kda_infinite_decays(Dk, rows, dtype):
+    for T in (32, 64):
+        at = [r for r in rows if r < T]
+        if not at:
+            continue
+        q, k, v, gl, beta = _inputs(1, T, 2, Dk, 32, seed=T + rows[0])
+        gl = gl.to(dtype)
+        gl[:, at, 0, ::3] = -torch.inf       # a third of the channels of one head, all of the other
+        gl[:, at, 1] = -torch.inf
+        o_ref, S_ref = oracle.kda_recurrent(q, k, v, gl, beta)
+        o, S = _run(q, k, v, gl, beta)
+        assert_close_bf16(o, o_ref, f"T = {T}: o")
+        assert ((S - S_ref).norm() / S_ref.norm()).item() <= 1e-3
+    gl[:, T // 2, 0, 0] = torch.nan          # not taken for a decay
+    assert _run(q, k, v, gl, beta)[1][:, 0].isnan().any()
