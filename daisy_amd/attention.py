@@ -314,9 +314,8 @@ class Rotary(nn.Module):
 
 
 # Up to this many sequences, a decode step's two projections go through ``ops.linear_rows`` (the weights are read
-# once by a kernel made for a few rows: 4.6 against 9.9 us for a 4608 x 1536 matrix and one row) where the tiled kernel does not
-# lead already (the native call's rule by rows and columns, which also keeps up to 8 rows there for short matrices); beyond, the
-# tiled kernel while it leads, then the library GEMM.  0: the library GEMM everywhere.
+# once by a kernel made for a few rows: 4.6 against 9.9 us for a 4608 x 1536 matrix and one row); beyond, the tiled kernel
+# while it leads, then the library GEMM.  0: the library GEMM everywhere.
 STEP_ROWS_KERNEL_MAX = 4
 
 

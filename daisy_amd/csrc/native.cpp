@@ -141,23 +141,14 @@ bool as_rows(const Tensor& x, int dev, Rows& r) {
   return stride % 8 == 0 && (reinterpret_cast<uintptr_t>(r.p) & 15) == 0;
 }
 
-// Whether a product of a few rows is better off with the weight-streaming kernel than with the tiled one.  Its fp32 products grow with
-// M N, the tiled kernel's time hardly does: level at M N of 12 to 18 thousand (weights from memory, K = N or N / 3; us, streamed / tiled:
-// N = 1536, M = 5: 4.1 / 5.0, M = 8: 5.0 / 5.0; N = 2048, M = 8: 6.2 / 6.6; N = 4608, M = 2: 5.0 / 6.1, M = 4: 6.3 / 6.1, M = 8: 8.7 / 6.1;
-// N = 8192, M = 4: 8.3 / 6.8).  One and two rows always, and the longest matrices (four weight rows a wavefront: N = 50304, M = 3:
-// 16.4 / 17.3).
-bool streams_rows(int M, int N) { return M <= 2 || N >= 16384 || (int64_t)M * N <= 16384; }
-constexpr int kStreamedRows = 8;        // as many as that kernel takes
-
-// y = x w^T for one of this library's kernels: a few rows (up to max_rows whatever the other kernel serves) through the weight-streaming
-// kernel, larger products through the tiled one where the sizes favour it.  False: the library GEMM is the better choice.
+// y = x w^T for one of this library's kernels: up to max_rows rows through the weight-streaming kernel, larger
+// products through the tiled one where the sizes favour it.  False: the library GEMM is the better choice.
 bool own_linear(const Rows& x, const uint16_t* w, int64_t w_sn, int N, const uint16_t* bias, uint16_t* y, int64_t y_sm,
                 int max_rows, hipStream_t s) {
   if (max_rows <= 0) return false;
-  const bool tiled = daisy::proj_wanted(x.M, N, x.K), few = x.M <= max_rows && !bias;
-  const bool streamed = few ? !tiled || streams_rows(x.M, N) : tiled && !bias && x.M <= kStreamedRows && N < 16384 && streams_rows(x.M, N);
-  if (!streamed && tiled && daisy::proj_linear(x.p, x.stride, w, w_sn, bias, y, y_sm, x.M, N, x.K, s) == DAISY_OK) return true;
-  return (streamed || few) && daisy_linear_rows_fwd(x.p, x.stride, w, w_sn, y, y_sm, x.M, N, x.K, s) == DAISY_OK;
+  if (x.M <= max_rows && !bias) return daisy_linear_rows_fwd(x.p, x.stride, w, w_sn, y, y_sm, x.M, N, x.K, s) == DAISY_OK;
+  if (!daisy::proj_wanted(x.M, N, x.K)) return false;
+  return daisy::proj_linear(x.p, x.stride, w, w_sn, bias, y, y_sm, x.M, N, x.K, s) == DAISY_OK;
 }
 
 // linear(x, w, bias, max_rows, tile): x w^T (+ bias) through an own kernel, or None.  tile != 0 forces the tiled kernel

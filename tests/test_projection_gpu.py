@@ -38,7 +38,7 @@ def test_smallest_tiles_against_fp64(tile, K, M, N):
 @pytest.mark.parametrize("M", [2, 3, 4, 5, 8, 9])
 @pytest.mark.parametrize("N,K", [(1024, 192), (2048, 64), (2056, 128), (5464, 128), (8200, 64), (16392, 72), (1024, 72)])
 def test_few_rows_on_both_sides_of_the_rule_against_fp64(M, N, K):
-    """Rows and columns on either side of where the weight-streaming kernel hands over to the tiled one, and sizes that one refuses."""
+    """Few rows on either side of the limit where the weight-streaming kernel hands over to the tiled one, and sizes that one refuses."""
     g = torch.Generator().manual_seed(M * N)
     x, w = torch.randn(M, K, generator=g).bfloat16(), torch.randn(N, K, generator=g).bfloat16()
     with torch.no_grad():
@@ -144,3 +144,27 @@ def test_calls_that_something_intercepts_reach_the_library_op():
         assert type(step_linear(x.as_subclass(Sub), w)) is Sub
         with torch.autocast("cuda", torch.float16):
             assert step_linear(x, w).dtype == torch.float16
+
+
+@pytest.mark.parametrize("limit", [1, 4, 8])
+@pytest.mark.parametrize("N,K", [(1024, 512), (4608, 512), (8200, 448)])
+def test_the_limit_of_rows_chooses_the_kernel(N, K, limit):
+    """Up to that many rows go to the weight-streaming kernel (a row's bits do not depend on how many there are), more to the tiled
+    one, whatever the columns."""
+    g = torch.Generator().manual_seed(N)
+    x, w = torch.randn(9, K // 2, generator=g), torch.randn(N, K // 2, generator=g)
+    # (sums that nearly cancel, so that their order shows in bf16)
+    x, w = torch.cat([x, x], 1).bfloat16().to(DEV), torch.cat([w, 0.01 * torch.randn(N, K // 2, generator=g) - w], 1).bfloat16().to(DEV)
+    with torch.no_grad():
+        rows, tiled = ops.linear_rows(x[:8], w), _lib.native().linear(x, w, None, 4, 4)
+        assert not torch.equal(rows, tiled[:8])            # (so that bits tell the kernels apart)
+        for M in (1, 3, 4, 5, 8, 9):
+            y = _lib.native().linear(x[:M], w, None, limit, 0)
+            assert torch.equal(y, rows[:M] if M <= limit else tiled[:M]), M
+
+
+def test_tiled_product_of_one_row_broadcast():
+    x, w = torch.randn(1, 128, device=DEV).bfloat16(), torch.randn(1024, 128, device=DEV).bfloat16()
+    with torch.no_grad():
+        y = _lib.native().linear(x.expand(6, 128), w, None, 4, 0)
+        assert torch.equal(y, _lib.native().linear(x.repeat(6, 1), w, None, 4, 0))
