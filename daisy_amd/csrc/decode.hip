@@ -566,7 +566,11 @@ struct CombineProjectParams {
 constexpr int kProjectThreads = 512;
 constexpr int kProjectRows = kProjectThreads / 64;
 constexpr int kProjectChannels = 4 * kProjectThreads;      // H D at most
-constexpr int kProjectSplits = 32;                         // and H nsplit at most kProjectThreads
+constexpr int kProjectSplits = 32;
+// Partial rows (H nsplit) at most: every workgroup reads all of them, and beyond this the two kernels are ahead (a layer's step, heads of
+// 64, two kernels / one: 18 heads x 32 splits 23.4 / 23.8 us, 24 x 32 26.6 / 26.9, 32 x 18 26.6 / 28.2, 32 x 32 33.4 / 35.4; up to it
+// one kernel: 12 heads of 128 x 16 above).
+constexpr int kProjectPartials = 512;
 // G groups of up to eight splits, as decode_combine_kernel forms them: split s belongs to group s % G.
 template <int D, int G>
 __global__ __launch_bounds__(kProjectThreads) void decode_combine_project_kernel(CombineProjectParams p) {
@@ -711,7 +715,7 @@ static int resolve_nsplit(int B, int H, int n_rows, int nsplit) {
 bool step_projects(int B, int H, int D, int n_rows) {
   if (B != 1 || (D != 64 && D != 128) || H * D > kProjectChannels) return false;
   const int ns = resolve_nsplit(B, H, n_rows, 0);
-  return ns > 1 && ns <= kProjectSplits && H * ns <= kProjectThreads;
+  return ns > 1 && ns <= kProjectSplits && H * ns <= kProjectPartials;
 }
 template <int D, int G>
 static void launch_combine_project(const DecodeParams& p, const StepProjection& out, hipStream_t s) {
