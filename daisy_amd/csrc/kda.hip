@@ -1075,10 +1075,13 @@ static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
   const dim3 chunks(p.NC, p.H, p.n_seq > 0 ? 1 : p.B);
   const int64_t bytes = (int64_t)p.H * p.nc_total * KdaBlob<KD>::kBytes;
   if (bytes > kCachedBytes) {
-    // Beyond 400 MB 6 KB more of LDS than the kernel uses: five workgroups per compute unit.  A sixth only adds requests where memory
-    // is the bound (B4 T8192 H16, 128 x 128, fp32 log-decays, behind the other kernel: 230 -> 222 us; with four the latency shows,
-    // 329; half of that length 111 and 113 us).
-    hipLaunchKernelGGL((kda_prep_kernel<KD, true>), chunks, dim3(128), KD == 128 && bytes > (int64_t)400 << 20 ? 6144 : 0, s, p);
+    // fp32 log-decays beyond 400 MB: 6 KB more of LDS than the kernel uses, five workgroups per compute unit.  Where memory is the bound a sixth
+    // only adds requests.  16 heads of 128, T = 8192, B = 3 / 4 / 6, both kernels, six workgroups -> five: mild fp32 log-decays 375 to 381 -> 374 to 376,
+    // 442 to 450 -> 442 to 448, 742 -> 735 us (with four the latency shows: 329 us for the first kernel, B = 4, where it takes 222); steep fp32 ones 390 -> 396, 466 ->
+    // 472, 756 -> 766.  With half the bytes to read the vector instructions are: mild bf16 ones 364 / 364, 416 / 415, 690 / 688,
+    // steep ones (a layer's first gates) 377 / 387, 450 / 468, 729 / 749, so those keep all six.
+    const bool memory_bound = KD == 128 && !p.g_bf16 && bytes > (int64_t)400 << 20;
+    hipLaunchKernelGGL((kda_prep_kernel<KD, true>), chunks, dim3(128), memory_bound ? 6144 : 0, s, p);
   } else {
     hipLaunchKernelGGL((kda_prep_kernel<KD, false>), chunks, dim3(128), 0, s, p);
   }
