@@ -75,15 +75,16 @@ def test_kda_packed_chunk_slots(lengths, behind):
         assert ((S[i:i + 1] - S_ref).norm() / S_ref.norm()).item() <= 1e-3
 
 
-# Blocks of the workspace (37 KiB per chunk and head) beyond 128 and 400 MB are stored past the caches, beyond 400 with fewer
-# workgroups per compute unit; 192 and more workgroups of the second kernel copy at another pace.  Heads are independent: the
-# same bits as from calls on the other side of every line.
-@pytest.mark.parametrize("T,H", [(3712, 32), (8200, 48)])
-def test_kda_workspace_sizes_agree(T, H):
-    assert (T + 31) // 32 * H * 37 * 1024 > (400 << 20 if T > 8000 else 128 << 20)
+# Blocks of the workspace (37 KiB per chunk and head, 21 for up to 64 key channels) beyond 128 MB are stored past the caches, those of
+# 128 channels with fp32 log-decays beyond 400 with fewer workgroups per compute unit; 192 and more workgroups of the second
+# kernel copy at another pace.  Heads are independent: the same bits as from calls on the other side of every line.
+@pytest.mark.parametrize("T,H,Dk", [(3712, 32, 128), (8200, 48, 128), (6560, 48, 64)])
+def test_kda_workspace_sizes_agree(T, H, Dk):
+    assert (T + 31) // 32 * H * (37 if Dk > 64 else 21) * 1024 > (400 << 20 if T > 8000 else 128 << 20)
+    assert (H + 7) // 8 * 8 * 4 >= 192 or T < 4000      # (four groups of value columns per head)
     g = torch.Generator(device="cuda").manual_seed(T)
-    q, k, v = (torch.randn(1, T, H, 128, generator=g, device="cuda").bfloat16() for _ in range(3))
-    gl = F.logsigmoid(torch.randn(1, T, H, 128, generator=g, device="cuda"))
+    q, k, v = (torch.randn(1, T, H, d, generator=g, device="cuda").bfloat16() for d in (Dk, Dk, 128))
+    gl = F.logsigmoid(torch.randn(1, T, H, Dk, generator=g, device="cuda"))
     beta = torch.sigmoid(torch.randn(1, T, H, generator=g, device="cuda"))
     kw = dict(output_final_state=True, use_qk_l2norm_in_kernel=True)
     o, S = chunk_kda(q, k, v, gl, beta, **kw)
