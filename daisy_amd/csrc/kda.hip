@@ -788,7 +788,9 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
     // first requests differ and later ones find the L2 filled (T = 8192: 64 heads of 128 469 -> 455 us, both kernels), and
     // in turns with a pause between: all at once they delay the other wavefronts' LDS and store traffic (4 heads of 128 215 -> 184 us,
     // of 64 134 -> 117).  With most compute units at it a longer pause is the better one (456 against 458 us; 192 against 184 the other
-    // way round).  *Tried:* one dword of every line fetched further ahead, by these or by a wavefront of its own, and from the scalar
+    // way round).  The first chunks, which nothing computes beside, are asked for without a pause, and the last outputs' part is not waited
+    // for in the interval that asks for it (64 sequences of 64 rows, 16 heads of 64: 52.1 -> 50.4 us; 4 of 100
+    // rows, 24 heads of 128: 32.5 -> 31.0).  *Tried:* one dword of every line fetched further ahead, by these or by a wavefront of its own, and from the scalar
     // side: slower, answers come back in order and hits wait behind misses.
     const int pw = ct;
     constexpr int NM1 = 3 * KC * KD * 2 / 1024 / KPW, NO1 = Blob::kOut / 1024 / KPW;
@@ -806,6 +808,7 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
       for (int i = 0; i < kTurns; ++i) {
         const int first = (pw * kTurns + (i + grp) % kTurns) * (NM1 / kTurns) * 1024;
         copy_kib_to_lds_async<NM1 / kTurns>(block + first, 16 * lane, to + first);
+        if (n < KSTAGES) continue;
         if (crowded) __builtin_amdgcn_s_sleep(4); else __builtin_amdgcn_s_sleep(2);
       }
       copy_kib_to_lds_async<1>(block + Blob::kDec, 16 * lane, to + Blob::kDec);
@@ -829,6 +832,7 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
       // everything of earlier intervals has landed
       if (n == 0) landed(std::integral_constant<int, NM1 + 2>{});
       else if (n < nc) landed(std::integral_constant<int, NM1 + 2 + NO1>{});
+      else if (n == nc) landed(std::integral_constant<int, NO1>{});
       else landed(std::integral_constant<int, 0>{});
       st = st == KSTAGES - 1 ? 0 : st + 1;
       __syncthreads();
