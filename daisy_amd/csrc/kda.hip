@@ -259,11 +259,20 @@ __device__ __forceinline__ float sum_over_q4(float x) {       // over the four l
   return x + __shfl_xor(x, 32);
 }
 
-// 16 bytes of a block of the workspace, past the caches or into them.
-template <bool STREAMED> __device__ __forceinline__ void store_piece(const u32x4& v, char* to) {
-  if (STREAMED) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(to));
-  else *reinterpret_cast<u32x4*>(to) = v;
-}
+// A chunk's block in the workspace, stored in pieces of 16 bytes past the caches or through them: there the cache policy sc1 writes
+// through the L2 at once.  Left dirty there, all blocks of a launch of a few rounds are written back at its end (512 chunks x heads of
+// 128: 16.7 us, 13.3 written through).  As buffer stores, which take the policy as an argument.
+constexpr int kWriteThrough = 16;             // sc1
+constexpr int kBufferWord3 = 0x00020000;      // an untyped buffer of bytes
+template <bool STREAMED> struct BlockOut {
+  char* base;
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ BlockOut(char* b, int bytes) : base(b), rsrc(__builtin_amdgcn_make_buffer_rsrc(b, 0, bytes, kBufferWord3)) {}
+  __device__ __forceinline__ void store(const u32x4& v, int at, int part) const {        // byte `at` (the lane's) of the part at byte `part`
+    if (STREAMED) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(base + part + at));
+    else __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, at, part, kWriteThrough);
+  }
+};
 
 // A workgroup makes one chunk, a wavefront one block of 16 rows.  Everything a wavefront does before the triangle's inverse
 // it does in the layout of a matrix operand: lane (row li, q4) holds channels 32 m + 8 q4 + e of its row, of k, of q and of
@@ -313,7 +322,7 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   const bool edge = n_live < KC || p.Dk < KD;     // rows or channels that do not exist: read as copies of others, then zeroed
   const uint32_t row_stride = (uint32_t)p.H * (uint32_t)p.Dk;         // elements between token rows of one head (q, k, g)
   const int64_t tok_base = ((int64_t)t0 * p.H + h) * p.Dk;
-  char* const blob = p.blobs + ci * Blob::kBytes;
+  const BlockOut<STREAMED> block(p.blobs + ci * Blob::kBytes, Blob::kBytes);
 
   // ---- every global load goes out at once: g as left operand, k and q rows into the LDS (swizzled), beta ----
   // g: tile t of group m holds channels 32 m + 8 (row / 4) + 2 (row % 4) + t, so that a lane's two tiles are neighbours and the
@@ -593,11 +602,11 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
 #pragma unroll
     for (int j = 0; j < 16 * ROW / 1024; ++j) {
       const u32x4 a = *reinterpret_cast<const u32x4*>(kg + 1024 * j + 16 * lane), b = *reinterpret_cast<const u32x4*>(qg + 1024 * j + 16 * lane);
-      store_piece<STREAMED>(a, blob + Blob::kKg + 16 * I * ROW + 1024 * j + 16 * lane);
-      store_piece<STREAMED>(b, blob + Blob::kQg + 16 * I * ROW + 1024 * j + 16 * lane);
+      block.store(a, 16 * lane, Blob::kKg + 16 * I * ROW + 1024 * j);
+      block.store(b, 16 * lane, Blob::kQg + 16 * I * ROW + 1024 * j);
     }
     wave_lds_fence();
-    if (tid < KD / 4) *reinterpret_cast<f32x4*>(blob + Blob::kDec + 16 * tid) = lds_f4(&Et[0][4 * tid]) * lds_f4(&Et[1][4 * tid]);
+    if (tid < KD / 4) *reinterpret_cast<f32x4*>(block.base + Blob::kDec + 16 * tid) = lds_f4(&Et[0][4 * tid]) * lds_f4(&Et[1][4 * tid]);
   }
   // ---- exp(G_last - G) k in two bf16 terms, for the transposing reads below ----
 #pragma unroll
@@ -679,7 +688,7 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   }
   // Row `row` of (right operand)^T T: the products come out with four consecutive columns of T per lane and column block,
   // which is the stored piece q4 of that row; both terms of it leave from here, 16 whole rows per instruction.
-  auto times_t = [&](const bf16x8& rh, const bf16x8& rl, char* dst_hi, char* dst_lo, int row) {
+  auto times_t = [&](const bf16x8& rh, const bf16x8& rl, int part_hi, int part_lo, int row) {
     float out[8];
 #pragma unroll
     for (int J = 0; J < 2; ++J) {
@@ -693,8 +702,8 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     u32x4 hi, lo;
     split_pack8(out, hi, lo);
     const int off = row * 64 + 16 * (q4 ^ piece_swizzle<64>(row));
-    store_piece<STREAMED>(hi, dst_hi + off);
-    store_piece<STREAMED>(lo, dst_lo + off);
+    block.store(hi, off, part_hi);
+    block.store(lo, off, part_lo);
   };
   {
     float pv[8];
@@ -702,7 +711,7 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     for (int e = 0; e < 4; ++e) { pv[e] = P[0][e]; pv[4 + e] = P[1][e]; }
     u32x4 hi, lo;
     split_pack8(pv, hi, lo);
-    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), blob + Blob::kPh, blob + Blob::kPl, 16 * I + li);
+    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), Blob::kPh, Blob::kPl, 16 * I + li);
   }
   // ---- M = (exp(G_last - G) k)^T T, half of the chunk's channels per wavefront: row 16 i + li of the block is channel
   // 32 (i / 2) + 8 (li / 4) + 4 (i % 2) + li % 4, the one that row of the state's tile i stands for
@@ -716,7 +725,7 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     const u32x2 l0 = lds_column4((lds_cptr)&rows[1][0] + a0), l1 = lds_column4((lds_cptr)&rows[1][0] + a0 + 16 * ROW);
     hi = u32x4{h0.x, h0.y, h1.x, h1.y};
     lo = u32x4{l0.x, l0.y, l1.x, l1.y};
-    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), blob + Blob::kMh, blob + Blob::kMl, 16 * i + li);
+    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), Blob::kMh, Blob::kMl, 16 * i + li);
   }
 }
 
@@ -789,9 +798,9 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
     // in turns with a pause between: all at once they delay the other wavefronts' LDS and store traffic (4 heads of 128 215 -> 184 us,
     // of 64 134 -> 117).  With most compute units at it a longer pause is the better one (456 against 458 us; 192 against 184 the other
     // way round).  The first chunks, which nothing computes beside, are asked for without a pause, and the last outputs' part is not waited
-    // for in the interval that asks for it (64 sequences of 64 rows, 16 heads of 64: 52.1 -> 50.4 us; 4 of 100
-    // rows, 24 heads of 128: 32.5 -> 31.0).  *Tried:* one dword of every line fetched further ahead, by these or by a wavefront of its own, and from the scalar
-    // side: slower, answers come back in order and hits wait behind misses.
+    // for in the interval that asks for it (64 sequences of 64 rows, 16 heads of 64: 52.1 -> 50.4 us; 4 of 100 rows, 24 heads of 128:
+    // 32.5 -> 31.0).  *Tried:* one dword of every line fetched further ahead, by these or by a wavefront of its own, and from the
+    // scalar side: slower, answers come back in order and hits wait behind misses.
     const int pw = ct;
     constexpr int NM1 = 3 * KC * KD * 2 / 1024 / KPW, NO1 = Blob::kOut / 1024 / KPW;
     static_assert(NM1 * KPW * 1024 == Blob::kDec && NO1 * KPW * 1024 == Blob::kOut && Blob::kChain - Blob::kDec == 1024, "runs of whole KiB");
@@ -1069,8 +1078,9 @@ extern "C" size_t daisy_kda_varlen_workspace_bytes(int T, int n_seq, int H, int 
   return kda_chunk_slots(1, T, n_seq) * H * kBlobBytes + kda_table_bytes(T, n_seq);
 }
 
-// Blocks of up to this many bytes are stored through the caches (the last level holds 256 MB), where the second kernel finds
-// them: T = 8192, 4 heads of 64 154 -> 117 us, T = 6016, 12 heads of 128 168 -> 156 us; 153 MB of them 118 -> 124 us.
+// Blocks of up to this many bytes are stored through the caches (the last level holds 256 MB), where the second kernel finds them.  Both
+// kernels, past / through them: 21 MB (T = 8192, 4 heads of 64) 155 / 114 us, 81 MB (T = 6016, 12 heads of 128) 168 / 158, 126 MB (T = 8192,
+// 24 heads of 64) 198 / 143; 296 MB (T = 8192, 32 heads of 128) 310 / 333.
 constexpr int64_t kCachedBytes = (int64_t)128 << 20;
 
 template <int KD>
