@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 // are; X's tiles hold positions 16 t + 4 (row/4) + row%4, and M and P are stored with their columns permuted to match.
 //
 // What bounds it.  Of the first kernel, at B4 T8192 H16 with fp32 log-decays, memory: 1.29 GB (673 MB of inputs, 612 MB of blocks) in
-// 222 us; otherwise its vector instructions and their latency.  The second is a serial chain of chunks; what sets the time of a
+// 216 us (208 at the fastest); otherwise its vector instructions and their latency.  The second is a serial chain of chunks; what sets the time of a
 // link is not the chain itself (without it the kernel is as fast) but its 39 KB of operands: a compute unit has about 64 KB
 // of requests in flight, 62 GB/s from memory (160 GB/s if they are in the L2).  0.55 us a link at B1 T8192 with 4 heads of
 // 128 (0.75 before the data-moving wavefronts were written as below), 0.4 us with 4 heads of 64 (0.63), 0.87 us with 64 of
@@ -95,8 +95,8 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 // Numerics: the 16x16 blocks of A and P run on MFMA with both operands referenced to the row before the block (every
 // exponent <= 0 off the diagonal); a diagonal block whose total decay exceeds exp(-80) is referenced to its middle row
 // instead (exponents up to the decay of 8 rows either way); when those go beyond exp(-80) it is taken by halves, of 8, 4, 2 and
-// 1 rows: no exponent is ever positive, so strong decays cannot overflow.  These products are in two-term bf16 splits (2^-17)
-// and, where four rows alone decay beyond exp(-80), in fp32.
+// 1 rows: no exponent is ever positive, so strong decays cannot overflow.  These products are in two-term bf16 splits (2^-18 of
+// either operand) and, where four rows alone decay beyond exp(-80), in fp32.
 // T is computed in fp32; the products with T, the state update and the output's second term use two-term bf16 splits of
 // both operands (three MFMAs each, relative error ~2^-17), which keeps the state error near fp32.
 // ===========================================================================
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void kda_chunk_table_kernel(const int32_t* cu,
 
 __device__ __forceinline__ f32x4 lds_f4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
-// Eight floats as two 16-byte pieces of bf16 terms (value = hi + lo up to 2^-17 relative).
+// Eight floats as two 16-byte pieces of bf16 terms (value = hi + lo up to 2^-18 relative).
 __device__ __forceinline__ void split_pack8(const float* x, u32x4& hi, u32x4& lo) {
   float h[8], l[8];
   hi = pack8(x);
@@ -252,7 +252,7 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ u32x2 lds_column4(lds_cptr p) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)p));
 }
-// The value that another lane of the same 16 holds: lane N of them, or by a pattern inside every quad.
+// The value that lane N of the same 16 holds.
 template <int N> __device__ __forceinline__ float from_row(float x) { return dpp_move<0x150 + N>(x); }
 __device__ __forceinline__ float sum_over_q4(float x) {       // over the four lanes that share a row of an operand
   const LanePair r = row_pair(x);
@@ -1092,7 +1092,7 @@ static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
   if (bytes > kCachedBytes) {
     // fp32 log-decays beyond 400 MB: 6 KB more of LDS than the kernel uses, five workgroups per compute unit.  Where memory is the bound a sixth
     // only adds requests.  16 heads of 128, T = 8192, B = 3 / 4 / 6, both kernels, six workgroups -> five: mild fp32 log-decays 375 to 381 -> 374 to 376,
-    // 442 to 450 -> 442 to 448, 742 -> 735 us (with four the latency shows: 329 us for the first kernel, B = 4, where it takes 222); steep fp32 ones 390 -> 396, 466 ->
+    // 442 to 450 -> 442 to 448, 742 -> 735 us (with four the latency shows: 329 us for the first kernel, B = 4, where it takes 216); steep fp32 ones 390 -> 396, 466 ->
     // 472, 756 -> 766.  With half the bytes to read the vector instructions are: mild bf16 ones 364 / 364, 416 / 415, 690 / 688,
     // steep ones (a layer's first gates) 377 / 387, 450 / 468, 729 / 749, so those keep all six.
     const bool memory_bound = KD == 128 && !p.g_bf16 && bytes > (int64_t)400 << 20;
