@@ -276,6 +276,179 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(GatedNormParams p) {
 
 bool gated_rmsnorm_serves(int D) { return D == 32 || D == 64 || D == 128 || D == 256; }
 
+// ---- the low-rank products of the KDA layer with what follows them ---------------------------------------------
+// y [M, N] = x [M, K] w [N, K]^T with K = 64 or 128, the width of a value head: two or four products deep, so that it is all operands and
+// results.  A workgroup keeps its columns of w (a head's, or 128) in the LDS as operands, and each of its wavefronts takes block after block
+// of 16 rows of x, straight from memory, the next block's while the present one is worked on.  The rows of w are dealt to the accumulators
+// such that a lane ends with 8 consecutive columns of a row; rounded to bf16 they pass through a corner of the LDS, 4 KB, and what follows
+// works on whole rows, 4 of them per access (straight from the accumulators' layout, 64 bytes of 16 rows per access, 134 MB were stored in
+// 75 us).
+// EPI 0: the decay gate, and beta.  EPI 1: the output gate, and with it the gated RMS norm of the rows of o, in place; the gate itself is
+// not written.
+// 32768 rows of 16 heads of 128: the two products as tiles of 128 x 128 with the gate in their epilogue and gated_rmsnorm_kernel behind them took
+// 115 + 62 us; these take 61 (134 MB written, 36 us of vector instructions) and 61 us (276 MB).  Beta is shared out among the groups of columns: as
+// the first group's it came last in the launch, a chain of loads of 25 us.
+// Nothing in the loop is conditional: rows and columns past the end are the last ones over again, stored as such.  (Behind a branch around
+// a store the next block's operands are waited for together with the stores.)
+struct LowRankParams {
+  const uint16_t* x; int64_t x_sm;
+  const uint16_t* w;
+  int M, N, groups;                    // groups of columns
+  KdaGates gates; uint16_t* y;         // EPI 0
+  const uint16_t* bias; const uint16_t* weight; uint16_t* o; float eps;      // EPI 1: bias [N] or NULL, norm weight [K], o [M, N]
+};
+constexpr int kLowRankWaves = 4;
+template <int K, int EPI>
+__global__ __launch_bounds__(64 * kLowRankWaves, 3) void low_rank_kernel(LowRankParams p) {
+  constexpr int COLS = EPI == 0 ? 128 : K, NG = COLS / 32, KS = K / 32;        // columns of a wavefront, groups of 32 of them, products per sum
+  constexpr int LPR = COLS / 8, RPA = 64 / LPR, NR = 16 / RPA;                 // lanes per row, rows per access, accesses per block
+  __shared__ __attribute__((aligned(16))) u32x4 ws[2 * NG][KS][64];
+  __shared__ __attribute__((aligned(16))) u32x4 turn[kLowRankWaves][16][LPR];
+  __shared__ __attribute__((aligned(16))) float bs[COLS];                      // EPI 1: the gate's bias
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, q4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int piece = lane % LPR, row_in = lane / LPR;                           // the lane's place in whole rows
+  // The columns of a walker's rows in consecutive workgroups of one XCD, whose L2 then holds these rows of x.
+  const int in_xcd = blockIdx.x >> 3, n0 = in_xcd % p.groups * COLS;
+  const int walker = (in_xcd / p.groups * 8 + (blockIdx.x & 7)) * kLowRankWaves + wave, walkers = gridDim.x / p.groups * kLowRankWaves;
+  const int blocks = (p.M + 15) / 16;
+  const int col8 = min(n0 + 8 * piece, p.N - 8);
+
+  auto load_x = [&](int block, u32x4* xv) {
+    const uint16_t* row = p.x + (int64_t)min(16 * block + li, p.M - 1) * p.x_sm + 8 * q4;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) xv[s] = *reinterpret_cast<const u32x4*>(row + 32 * s);
+  };
+  auto row_at = [&](int block, int j) { return (int64_t)min(16 * block + RPA * j + row_in, p.M - 1) * p.N + col8; };
+  auto load_o = [&](int block, u32x4* ov) {
+#pragma unroll
+    for (int j = 0; j < NR; ++j) ov[j] = *reinterpret_cast<const u32x4*>(p.o + row_at(block, j));
+  };
+  u32x4 xv[KS], ov[EPI == 1 ? NR : 1];
+  load_x(min(walker, blocks - 1), xv);
+  if constexpr (EPI == 1) load_o(min(walker, blocks - 1), ov);
+  // Row a of tile 2 m + u is column 32 m + 8 (a / 4) + 4 u + a % 4: a lane's rows of the two tiles are columns 32 m + 8 q4 ..
+#pragma unroll
+  for (int t = wave; t < 2 * NG; t += kLowRankWaves) {
+    const int col = min(n0 + 32 * (t >> 1) + 8 * (li >> 2), p.N - 8) + 4 * (t & 1) + (li & 3);
+    const uint16_t* row = p.w + (int64_t)col * K + 8 * q4;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) ws[t][s][lane] = *reinterpret_cast<const u32x4*>(row + 32 * s);
+  }
+  if (EPI == 1 && tid < COLS) bs[tid] = p.bias != nullptr ? bf16lo_to_f32(p.bias[n0 + tid]) : 0.f;
+  // What goes with the lane's columns: the decay gate's bias and scale, or the norm's weight.
+  float c8[8], scale = 1.f;
+  if constexpr (EPI == 0) {
+    scale = -expf(p.gates.A_log[col8 / p.gates.Dk]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) c8[e] = p.gates.dt_bias[col8 + e];
+  } else {
+    unpack8(*reinterpret_cast<const u32x4*>(p.weight + 8 * piece), c8);
+  }
+  __syncthreads();
+
+  for (int block = walker; block < blocks; block += walkers) {
+    f32x4 acc[2 * NG];
+#pragma unroll
+    for (int t = 0; t < 2 * NG; ++t)
+      acc[t] = EPI == 1 ? *reinterpret_cast<const f32x4*>(&bs[32 * (t >> 1) + 8 * q4 + 4 * (t & 1)]) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const bf16x8 xs = __builtin_bit_cast(bf16x8, xv[s]);
+#pragma unroll
+      for (int t = 0; t < 2 * NG; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ws[t][s][lane]), xs, acc[t], 0, 0, 0);
+    }
+    const int next = min(block + walkers, blocks - 1);
+    load_x(next, xv);
+#pragma unroll
+    for (int m = 0; m < NG; ++m)
+      turn[wave][li][(4 * m + q4) ^ (li & (LPR - 1))] =
+          u32x4{pack_bf16x2(acc[2 * m][0], acc[2 * m][1]), pack_bf16x2(acc[2 * m][2], acc[2 * m][3]),
+                pack_bf16x2(acc[2 * m + 1][0], acc[2 * m + 1][1]), pack_bf16x2(acc[2 * m + 1][2], acc[2 * m + 1][3])};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    u32x4 of[EPI == 1 ? NR : 1];
+    if constexpr (EPI == 1) {
+#pragma unroll
+      for (int j = 0; j < NR; ++j) of[j] = ov[j];
+      load_o(next, ov);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+      const int r = RPA * j + row_in;
+      float y[8], f[8];
+      unpack8(turn[wave][r][piece ^ (r & (LPR - 1))], y);
+      if constexpr (EPI == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = scale * softplus(y[e] + c8[e]);
+        *reinterpret_cast<u32x4*>(p.y + row_at(block, j)) = pack8(f);
+      } else {
+        float x[8], ss = 0.f;
+        unpack8(of[j], x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
+        ss = group_sum<LPR>(ss);
+        const float rstd = rsqrtf(ss / (float)K + p.eps);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = x[e] * rstd * c8[e] * __builtin_amdgcn_rcpf(1.f + __expf(-y[e]));
+        *reinterpret_cast<u32x4*>(p.o + row_at(block, j)) = pack8(f);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (EPI == 0) {                      // beta of the walker's rows, a block in turn by every group of columns
+    for (int block = walker + walkers * (in_xcd % p.groups); block < blocks; block += walkers * p.groups) {
+      const int count = min(16, p.M - 16 * block) * p.gates.H;
+      for (int i = lane; i < count; i += 64) {
+        const float logit = bf16lo_to_f32(p.gates.logits[(int64_t)(16 * block + i / p.gates.H) * p.gates.logits_row + i % p.gates.H]);
+        p.gates.beta[(int64_t)16 * block * p.gates.H + i] = round_bf16(1.f / (1.f + expf(-logit)));
+      }
+    }
+  }
+}
+
+// Three workgroups fit a compute unit; every wavefront walks the rows as often as that takes.
+template <int K, int EPI>
+static int launch_low_rank(LowRankParams& p, hipStream_t s) {
+  p.groups = EPI == 0 ? (p.N + 127) / 128 : p.N / K;
+  const int wanted = (p.M + 16 * kLowRankWaves - 1) / (16 * kLowRankWaves), fit = 768 / p.groups;
+  const int walkers = ((wanted < fit ? wanted : fit) + 7) / 8 * 8;
+  hipLaunchKernelGGL((low_rank_kernel<K, EPI>), dim3((unsigned)(walkers * p.groups)), dim3(64 * kLowRankWaves), 0, s, p);
+  DAISY_CHECK_LAUNCH("low_rank_kernel");
+  return DAISY_OK;
+}
+// From about four million outputs on.  Below, a workgroup's own latencies (its columns into the LDS, a block or two, beta) are what the call waits
+// for, and tiles have fewer of them: a layer's call, tiles and the gated norm / these kernels, 64 rows of 8 heads of 128 41.5 / 47.8 us, 200 of 16
+// 62 / 67, 777 of 12 89.5 / 91.5, 2048 of 16 175 / 175, 8000 of 8 222 / 218, 32768 of 8 of 64 420 / 404, 40000 of 16 of 128 2190 / 2120.
+bool low_rank_wanted(int M, int N, int K) { return (K == 64 || K == 128) && (int64_t)M * N >= 4000000; }
+static int low_rank_check(const LowRankParams& p, int K) {
+  auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
+  DAISY_CHECK_SUPPORTED(K == 64 || K == 128, "low_rank: K=%d (64 or 128)", K);
+  DAISY_CHECK_ARG(p.x && p.w && p.M > 0 && p.N >= 8 && p.N % 8 == 0 && al16(p.x) && al16(p.w) && p.x_sm % 8 == 0 && p.x_sm >= K,
+                  "low_rank: M=%d, N=%d, rows %lld elements apart on 16-byte boundaries", p.M, p.N, (long long)p.x_sm);
+  return DAISY_OK;
+}
+int low_rank_gate(const uint16_t* x, int64_t x_sm, const uint16_t* w, const KdaGates& gates, uint16_t* y, int M, int N, int K, hipStream_t s) {
+  LowRankParams p{};
+  p.x = x; p.x_sm = x_sm; p.w = w; p.M = M; p.N = N; p.gates = gates; p.y = y;
+  if (const int rc = low_rank_check(p, K); rc != DAISY_OK) return rc;
+  DAISY_CHECK_ARG(y && gates.A_log && gates.dt_bias && gates.logits && gates.beta && gates.H > 0 && gates.Dk % 8 == 0 && N == gates.H * gates.Dk &&
+                      (reinterpret_cast<uintptr_t>(y) & 15) == 0, "low_rank_gate: %d heads of %d channels on a product of %d", gates.H, gates.Dk, N);
+  return K == 64 ? launch_low_rank<64, 0>(p, s) : launch_low_rank<128, 0>(p, s);
+}
+int low_rank_norm(const uint16_t* x, int64_t x_sm, const uint16_t* w, const uint16_t* bias, const uint16_t* norm_weight, uint16_t* o, float eps,
+                  int M, int N, int K, hipStream_t s) {
+  LowRankParams p{};
+  p.x = x; p.x_sm = x_sm; p.w = w; p.M = M; p.N = N; p.bias = bias; p.weight = norm_weight; p.o = o; p.eps = eps;
+  if (const int rc = low_rank_check(p, K); rc != DAISY_OK) return rc;
+  auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
+  DAISY_CHECK_ARG(o && norm_weight && N % K == 0 && al16(o) && al16(bias) && al16(norm_weight), "low_rank_norm: N=%d in heads of %d, tensors on 16-byte boundaries", N, K);
+  return K == 64 ? launch_low_rank<64, 1>(p, s) : launch_low_rank<128, 1>(p, s);
+}
+
 }  // namespace daisy
 
 using namespace daisy;

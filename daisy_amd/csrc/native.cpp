@@ -644,17 +644,22 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   auto rest = [&]() -> std::array<Tensor, 2> {
     Tensor st, y;
     if (!step) {
-      Tensor g = empty({M, kd}, at::kBFloat16, x), gate = empty({M, vd}, at::kBFloat16, x), beta = empty({M, H}, at::kFloat, x);
+      // the low-rank products: with the decay gate and beta ahead of the delta rule, with the gated norm behind it
+      const bool own_low = daisy::low_rank_wanted((int)M, (int)kd, (int)Dv) && (!w[8] || (reinterpret_cast<uintptr_t>(W[8]) & 15) == 0);
+      Tensor g = empty({M, kd}, at::kBFloat16, x), gate, beta = empty({M, H}, at::kFloat, x);
+      if (!own_low) gate = empty({M, vd}, at::kBFloat16, x);
       const daisy::ProjSegment low[2] = {{seg[3].y, seg[3].y_sm, W[6], Dv, nullptr, (uint16_t*)ptr(g), kd, (int)kd, 0},
-                                         {seg[4].y, seg[4].y_sm, W[7], Dv, W[8], (uint16_t*)ptr(gate), vd, (int)vd, 0}};
+                                         {seg[4].y, seg[4].y_sm, W[7], Dv, W[8], own_low ? nullptr : (uint16_t*)ptr(gate), vd, (int)vd, 0}};
       const daisy::KdaGates gates{(const float*)ptr(w[16]), (const float*)ptr(w[17]), (int)H, (int)Dk, seg[5].y, seg[5].y_sm, (float*)ptr(beta)};
-      must(daisy::proj_segments(low, 2, (int)M, (int)Dv, s, 0, &gates));
+      must(own_low ? daisy::low_rank_gate(seg[3].y, seg[3].y_sm, W[6], gates, (uint16_t*)ptr(g), (int)M, (int)kd, (int)Dv, s)
+                   : daisy::proj_segments(low, 2, (int)M, (int)Dv, s, 0, &gates));
       o = empty({B, T, vd}, at::kBFloat16, x);
       if (keep) st = keeper(home[0], {B, H, Dk, Dv}, at::kFloat);
       Tensor ws = empty({(int64_t)need}, at::kByte, x);
       must(daisy_kda_chunk_fwd(ptr(conv[0]), ptr(conv[1]), ptr(conv[2]), ptr(g), 1, (const float*)ptr(beta), (const float*)ptr(state), ptr(o),
                                keep ? (float*)ptr(st) : nullptr, (int)B, (int)T, (int)H, (int)Dk, (int)Dv, 64, scale, 1, kL2Eps, ptr(ws), need, s));
-      must(daisy_gated_rmsnorm_fwd(ptr(o), ptr(gate), W[18], ptr(o), M * H, (int)Dv, norm_eps, s));
+      must(own_low ? daisy::low_rank_norm(seg[4].y, seg[4].y_sm, W[7], W[8], W[18], (uint16_t*)ptr(o), norm_eps, (int)M, (int)vd, (int)Dv, s)
+                   : daisy_gated_rmsnorm_fwd(ptr(o), ptr(gate), W[18], ptr(o), M * H, (int)Dv, norm_eps, s));
     }
     if (M <= max_rows || daisy::proj_wanted((int)M, (int)dim, (int)vd)) {
       y = empty({B, T, dim}, at::kBFloat16, x);

@@ -72,7 +72,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
   [[maybe_unused]] bool gated = false;
   if constexpr (SEGMENTS) {
     // gated and plain columns of tiles in turn: the gate's arithmetic runs beside the other workgroups' stores (32768 rows of 16
-    // heads of 128: 146 -> 134 us)
+    // heads of 128, which low_rank_kernel takes by now: 146 -> 134 us)
     if (EPI == 3 && p.NT == 2 * p.seg[0].tile_end) nt = (nt >> 1) + (nt & 1) * p.seg[0].tile_end;
     int i = 0;
     while (i + 1 < p.n && nt >= p.seg[i].tile_end) ++i;

@@ -140,3 +140,21 @@ def test_a_call_that_is_given_back_has_not_touched_the_states(what):
     assert _lib.native().kda_layer(rnd(B, T, dim), weights, H, Dk, Dv, 4, state, windows, (state, *windows), True, 1e-5, 4) is None
     for t, b in zip((state, *windows), before):
         assert torch.equal(t, b)
+
+
+@pytest.mark.parametrize("B,T,H,D,expand_v", [(1, 4099, 16, 64, 1.0), (2, 2061, 8, 128, 1.0), (1, 6251, 16, 40, 1.6), (1, 16385, 2, 128, 1.0)])
+def test_long_rows_take_the_low_rank_kernels(B, T, H, D, expand_v, monkeypatch):
+    """Rows that are no multiple of the 16 of a block, 640 columns (no multiple of 128) for the decay gate, fewer columns than an XCD has
+    workgroups; against the layer's own path, which makes the products as tiles and the norm by itself."""
+    m = _layer(H, D, expand_v, 4, False)
+    assert B * T * H * D >= 4000000
+    x = torch.randn(B, T, H * D, generator=torch.Generator(device=DEV).manual_seed(T), device=DEV).bfloat16()
+    with torch.no_grad():
+        got = [m.prefill(x, None)[0]] + [t.clone() for t in m.state_tensors()]
+        m.reset_history()
+        monkeypatch.setattr(KimiLinearSelfAttention, "_fast", lambda self, *a: None)
+        ref = [m.prefill(x, None)[0]] + [t.clone() for t in m.state_tensors()]
+    # the same products and gates; the norm's sum of squares in another order (fp32) ahead of one rounding to bf16
+    for a, b in zip(ref, got):
+        assert ((a.float() - b.float()).norm() / a.float().norm()).item() < 1e-3
+        assert (a.float() - b.float()).abs().max().item() <= 2 ** -7 * a.float().abs().max().item()
