@@ -46,7 +46,8 @@ struct PrefillParams {
   uint16_t* o; int64_t o_sb, o_st, o_sh;
   uint16_t* k_out; int64_t ko_sb, ko_st, ko_sh;
   int B, T, H, D, window, nqb;
-  int period;    // 32-key tiles in a full window's range (0 = no window): the rotation period of the tile order
+  int keys;      // key rows per tile
+  int period;    // tiles in a full window's range (0 = no window): the rotation period of the tile order
   int n_light;   // leading query blocks that see fewer keys than a full window (0 = order by block only)
   int order_shift;   // documents: query blocks in the order of their lengths, in units of 2^order_shift tiles; -1: by block
   int order_bit;     // the highest bit of such a length
@@ -179,11 +180,16 @@ __device__ __forceinline__ u32x2 lds_read_tr16_as3(lds_u16_ptr p) {
 // on the diagonal is masked per element.  The Q block at the start and the O block at the end pass
 // through an LDS area of the wavefront's own, so that every global access of the kernel covers whole
 // rows (a CU's memory path, shared by its three workgroups, is busy per cache line touched).
-constexpr int kTBN = 32;   // key rows per tile of prefill_tile_kernel
-template <int D>
-__global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(PrefillParams p) {
+//
+// KEYS = 64 (prefill_wide_tile_kernel, head dim 64): a tile is two products side by side, with one maximum, one check of the reference and
+// one barrier for both (120 registers and 32 KiB, still four workgroups per CU: the Q and O blocks fit Ks[1] and Vs[1]).
+constexpr int kTBN = 32;   // key rows of a product
+template <int D, int KEYS>
+__device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
   constexpr int NS = D / 16, NDT = D / 32, HALF = D / 2, CPR = D / 8;
-  constexpr int RPL = 64 / CPR, NLD = kTBN / RPL / 4, TILE = kTBN * D;
+  constexpr int SUB = KEYS / kTBN;               // products of a tile
+  static_assert(SUB == 1 || (SUB == 2 && D == 64), "");
+  constexpr int RPL = 64 / CPR, NLD = KEYS / RPL / 4, TILE = KEYS * D;
   static_assert(NLD >= 1, "a tile is at least one copy per wavefront");
   auto swz_k = [](int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); };
   auto swz_v = [](int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
@@ -193,7 +199,7 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   // Two more tile-sized areas: with Ks[1] and Vs[1] they give every wavefront 32 rows x D of its own for
   // turning the row-major Q block into operand fragments at the start (while the first K/V tile lands in
   // Ks[0] / Vs[0]) and the accumulators into row-major O at the end.
-  __shared__ __attribute__((aligned(1024))) uint16_t Xs[2][TILE];
+  __shared__ __attribute__((aligned(1024))) uint16_t Xs[SUB == 1 ? 2 : 1][SUB == 1 ? TILE : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -218,8 +224,8 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   // online softmax does not care about the order, and the query blocks of one (batch, head)
   // that run side by side then read the same K/V tile at the same step, so one fetch into the
   // L2 serves all of them.  With no window every range starts at tile 0 and nothing is rotated.
-  const int t_lo = lo_first / kTBN;
-  const int t_hi = min(q0 + kBM - 1, p.T - 1) / kTBN;
+  const int t_lo = lo_first / KEYS;
+  const int t_hi = min(q0 + kBM - 1, p.T - 1) / KEYS;
   const int n_tiles = t_hi - t_lo + 1;
   int t_first = t_lo;
   if (p.period > 0) {
@@ -244,15 +250,15 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   // The copies walk the tiles in visiting order; the source pointers move by one tile per step and go
   // back to the first tile of the range once (kept incrementally: the scalar unit would otherwise
   // rebuild two 64-bit products per step).
-  const int64_t k_step = (int64_t)kTBN * p.k_st, v_step = (int64_t)kTBN * p.v_st;
+  const int64_t k_step = (int64_t)KEYS * p.k_st, v_step = (int64_t)KEYS * p.v_st;
   const uint16_t* const k_lo = kbase + t_lo * k_step;
   const uint16_t* const v_lo = vbase + t_lo * v_step;
   int t_cp = t_first;                                   // tile the next copy_tiles() call fetches
   const uint16_t* kt = kbase + t_first * k_step;
   const uint16_t* vt = vbase + t_first * v_step;
   auto copy_tiles = [&](int buf) {
-    const int kv0 = t_cp * kTBN;
-    if (kv0 + kTBN <= p.T) {
+    const int kv0 = t_cp * KEYS;
+    if (kv0 + KEYS <= p.T) {
 #pragma unroll
       for (int i = 0; i < NLD; ++i) {
         copy16_to_lds_async(kt + (int64_t)(4 * RPL * i) * p.k_st, k_off, ks_lds + 2 * (buf * TILE) + 4096 * i);
@@ -289,8 +295,8 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   constexpr int CH = HALF / 8;          // pair chunks per row
   constexpr int QRI = 64 / CH;          // rows per load instruction
   constexpr int QT = 32 / QRI;          // loads of each kind per lane
-  const uint32_t x_lds = wave == 0 ? lds_address(&Ks[1][0]) : wave == 1 ? lds_address(&Vs[1][0])
-                                                                         : lds_address(&Xs[wave - 2][0]);
+  const uint32_t x_lds = SUB > 1 ? lds_address(wave < 2 ? &Ks[1][0] : &Vs[1][0]) + 2 * kTBN * D * (wave & 1)
+                         : wave == 0 ? lds_address(&Ks[1][0]) : wave == 1 ? lds_address(&Vs[1][0]) : lds_address(&Xs[SUB > 1 ? 0 : wave - 2][0]);
   bf16x8 qreg[NS];
   {
     const int qr = lane / CH, qc = lane % CH;
@@ -361,22 +367,25 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   // copy of the accumulators across the join.
   auto process_tile = [&](auto buf_tag, int kv0, bool masked) {
     constexpr int buf = decltype(buf_tag)::value;
-    f32x16 sacc;
+    f32x16 sacc[SUB];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
+    for (int u = 0; u < SUB; ++u)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sacc[u][r] = 0.f;
     // K fragments: four reads ahead of the products (an LDS read takes about as long as four MFMAs;
     // left alone the compiler keeps one fragment register set and waits for every read in turn).
     {
-      bf16x8 kf[NS];
+      constexpr int N = NS * SUB;
+      bf16x8 kf[N];
 #pragma unroll
-      for (int s = 0; s < NS; ++s)
-        kf[s] = __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)(size_t)((k_a0 ^ (32u * s)) + 2 * buf * TILE));
+      for (int s = 0; s < N; ++s)
+        kf[s] = __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)(size_t)((k_a0 ^ (32u * (s / SUB))) + 2 * (buf * TILE + s % SUB * kTBN * D)));
 #pragma unroll
-      for (int s = 0; s < NS; ++s) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qreg[s], sacc, 0, 0, 0);
-      constexpr int AHEAD = NS < 4 ? NS : 4;
+      for (int s = 0; s < N; ++s) sacc[s % SUB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qreg[s / SUB], sacc[s % SUB], 0, 0, 0);
+      constexpr int AHEAD = N < 4 ? N : 4;
       __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);          // DS reads
 #pragma unroll
-      for (int s = 0; s < NS - AHEAD; ++s) {
+      for (int s = 0; s < N - AHEAD; ++s) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);            // MFMA
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
@@ -387,10 +396,12 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
       const int hi = qrow - (kv0 + 4 * lh);
       const int lo = lo_q - (kv0 + 4 * lh);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int c = 8 * (r >> 2) + (r & 3);
-        if (c > hi || c < lo) sacc[r] = -INFINITY;
-      }
+      for (int u = 0; u < SUB; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int c = kTBN * u + 8 * (r >> 2) + (r & 3);
+          if (c > hi || c < lo) sacc[u][r] = -INFINITY;
+        }
     }
     // Online softmax (log2 domain, lazy rescale): the reference maximum m_run only moves when some
     // query of the wavefront sees a score more than 8 (log2 units) above it; until then
@@ -398,7 +409,9 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
     // touched.
     float mt = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[r]);
+    for (int u = 0; u < SUB; ++u)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[u][r]);
     mt = pair_max(mt) * p.scale_log2e;
     if (__builtin_amdgcn_ballot_w64(mt > m_run + 8.f) != 0) {
       const float m_new = fmaxf(m_run, mt);
@@ -412,14 +425,14 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
         for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
     }
     const float mu = (m_run == -INFINITY) ? 0.f : m_run;
-    bf16x8 pfrag[2];
+    bf16x8 pfrag[2 * SUB];
     float lsum = 0.f;
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < 2 * SUB; ++m) {
       float pv[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        pv[e] = fast_exp2(fmaf(sacc[8 * m + e], p.scale_log2e, -mu));
+        pv[e] = fast_exp2(fmaf(sacc[m >> 1][8 * (m & 1) + e], p.scale_log2e, -mu));
         lsum += pv[e];
       }
       pfrag[m] = __builtin_bit_cast(bf16x8, pack8(pv));
@@ -427,7 +440,7 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
     l_run += lsum;
     // O^T += V^T P^T
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < 2 * SUB; ++m) {
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) {
         lds_u16_ptr vp = (lds_u16_ptr)(size_t)((v_a0 ^ (64u * dt)) + 2 * (buf * TILE + 16 * m * D));
@@ -446,10 +459,10 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
   auto iteration = [&](int n, auto buf_tag) {
     constexpr int buf = decltype(buf_tag)::value;
     if (n + 1 < n_tiles) copy_tiles(buf ^ 1);
-    const int kv0 = t_cur * kTBN;
+    const int kv0 = t_cur * KEYS;
     t_cur = t_cur < t_hi ? t_cur + 1 : t_lo;
-    if (wave_live && kv0 <= q_w_max && kv0 + kTBN - 1 >= lo_w_min) {
-      const bool clean = kv0 + kTBN - 1 <= q_w_min && kv0 >= lo_w_max;
+    if (wave_live && kv0 <= q_w_max && kv0 + KEYS - 1 >= lo_w_min) {
+      const bool clean = kv0 + KEYS - 1 <= q_w_min && kv0 >= lo_w_max;
       process_tile(buf_tag, kv0, !clean);
     }
     copies_landed();
@@ -487,6 +500,10 @@ __global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(Prefil
     if (qw0 + r < p.T) __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(obase + (int64_t)(qw0 + r) * p.o_st));
   }
 }
+
+template <int D>
+__global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(PrefillParams p) { prefill_tiles<D, kTBN>(p); }
+__global__ __launch_bounds__(kPrefillThreads, 4) void prefill_wide_tile_kernel(PrefillParams p) { prefill_tiles<64, 2 * kTBN>(p); }
 
 // Few workgroups (a prompt of one or two thousand tokens of one sequence): blocks of 128 queries leave most compute
 // units idle and the last block walks all of its keys with one step in flight.  Here a workgroup is 32 queries, its
@@ -881,7 +898,8 @@ static int launch_mfma(PrefillParams p, hipStream_t s) {
     DAISY_CHECK_LAUNCH("prefill_split_kernel");
     return DAISY_OK;
   }
-  hipLaunchKernelGGL((prefill_tile_kernel<D>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
+  if (D == 64 && p.keys > kTBN) hipLaunchKernelGGL(prefill_wide_tile_kernel, dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
+  else hipLaunchKernelGGL((prefill_tile_kernel<D>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
   DAISY_CHECK_LAUNCH("prefill_tile_kernel");
   return DAISY_OK;
 }
@@ -909,7 +927,13 @@ static int fill_prefill_params(PrefillParams& p, const void* q, const int64_t* q
   p.ko_sb = k_out ? k_out_strides[0] : 0; p.ko_st = k_out ? k_out_strides[1] : 0; p.ko_sh = k_out ? k_out_strides[2] : 0;
   p.B = B; p.T = T; p.H = H; p.D = D; p.window = window;
   p.nqb = (T + kBM - 1) / kBM;
-  p.period = (window > 0 && window < T) ? (kBM - 1) / kTBN + 1 + (window - 1 + kTBN - 1) / kTBN : 0;
+  // Head dim 64: tiles of 64 keys, but for short windows, of which the tiles at their edges are a larger part.  32 / 64 keys a tile, us:
+  // T = 16384, 12 heads, no window 605 / 558; T = 32768, 32 heads 4440 / 4344; window 8192, five documents of T = 65536, 4 heads 425 / 412; window
+  // 4096, seven of T = 20001, 16 heads 154.5 / 154.2; 2048, T = 32768, 16 heads 300 / 293; 1024, 8 x 4096, 16 heads 147 / 145.5; 384, T = 32768, 8 heads
+  // 48.2 / 45.5; 256, 4 x 8192, 16 heads 66.6 / 67; 128, 16 x 2048, 8 heads 26.6 / 27.
+  const bool windowed = window > 0 && window < T;
+  const int keys = p.keys = D == 64 && !(windowed && window < 384) ? 2 * kTBN : kTBN;
+  p.period = (window > 0 && window < T) ? (kBM - 1) / keys + 1 + (window - 1 + keys - 1) / keys : 0;
   p.n_light = (window > 0 && window < T) ? min((window - 1 + kBM - 1) / kBM, p.nqb) : 0;
   p.order_shift = -1; p.order_bit = 0;
   // Finding the order costs a workgroup about 1 us; the lengths differ enough to pay for it where a window is an eighth of the

@@ -124,6 +124,20 @@ def test_prefill_long_sequence_sampled_rows():
     assert_close_bf16(o[:, rows.cuda()], ref, "o[rows]")
 
 
+@pytest.mark.parametrize("T,window,docs", [(63, None, False), (64, None, False), (65, None, True), (193, 383, False), (1000, 384, False), (1000, 385, True),
+                                           (1025, 575, False), (777, 640, True)])
+def test_prefill_tiles_of_64_keys(T, window, docs):
+    """Head dim 64 takes 64 keys per tile from a window of 384 on: rows that end before, at and behind a tile's and a product's end,
+    windows whose first key lies in either half of a tile, documents that start anywhere in one."""
+    q, k, v = _inputs(1, T, 3, 64, seed=T)
+    doc_start = None
+    if docs:
+        doc_start = oracle.doc_start_from_ids(torch.randint(0, 60, (T,), generator=torch.Generator().manual_seed(2)), 3)
+    ref, _ = _oracle(q, k, v, window, doc_start=doc_start)
+    check_prefill_of_many_heads(q.cuda(), k.cuda(), v.cuda(), ref, f"T{T} W{window}", window=window,
+                                doc_start=None if doc_start is None else doc_start.cuda())
+
+
 def test_prefill_is_deterministic_and_window_invariant():
     """A window >= T equals full causal attention bit for bit; repeated calls agree."""
     B, T, H, D = 1, 320, 2, 128
