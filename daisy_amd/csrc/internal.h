@@ -96,6 +96,10 @@ int attn_step_launch(const void* q, const int64_t* q_strides, const void* k, con
                      int B, int H, int D, int ring_rows, const int32_t* pos_dev, float scale, int nsplit,
                      void* workspace, size_t workspace_bytes, void* stream, const StepPrep& prep);
 
+// y [rows, C] = x rsqrt(mean(x^2) + eps), bf16, contiguous; the sizes that it takes.
+bool rms_rows_serves(int64_t rows, int64_t C);
+int rms_rows(const uint16_t* x, uint16_t* y, int rows, int C, float eps, hipStream_t s);
+
 // qkv_prep_kernel with the gate as the layer holds it.
 int prep_launch(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
                 const void* v, const int64_t* v_strides, const void* ve, const int64_t* ve_strides, GateSource gate,

@@ -180,6 +180,25 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// norm(x, eps): the weightless RMS norm over the last dim of contiguous bf16 rows, or None.
+PyObject* py_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 2 || intercepted() || !is_tensor(a[0])) return none();
+  const Tensor& x = THPVariable_Unpack(a[0]);
+  const float eps = (float)PyFloat_AsDouble(a[1]);
+  if (PyErr_Occurred()) { PyErr_Clear(); return none(); }
+  const int dev = gpu_of(x);
+  if (dev < 0 || !bf16(x) || x.dim() < 1 || !x.is_contiguous() || x.numel() == 0 || needs_autograd({&x})) return none();
+  const int64_t C = x.size(-1), rows = x.numel() / C;
+  if (!daisy::rms_rows_serves(rows, C) || (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) != 0) return none();
+  Unlocked unlocked;
+  Tensor y = empty(x.sizes(), at::kBFloat16, x);
+  const bool ok = daisy::rms_rows((const uint16_t*)ptr(x), (uint16_t*)ptr(y), (int)rows, (int)C, eps, stream_of(dev)) == DAISY_OK;
+  unlocked.end();
+  return ok ? wrap(y) : none();
+  END_HANDLE_TH_ERRORS
+}
+
 // linears(x, weights, biases, max_rows, tile): the products of x with several matrices in one launch, as a tuple of views of one
 // tensor, or None.  Arguments as for linear; weights and biases: tuples (a bias may be None).
 PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -687,7 +706,7 @@ PyObject* call(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   return r;
 }
 #define FAST(name) {#name, (PyCFunction)(void (*)(void))call<py_##name>, METH_FASTCALL, nullptr}
-PyMethodDef kMethods[] = {FAST(linear), FAST(linears), FAST(prefill_attention), FAST(layer_prefill), FAST(layer_step), FAST(kda_chunk), FAST(kda_layer),
+PyMethodDef kMethods[] = {FAST(linear), FAST(norm), FAST(linears), FAST(prefill_attention), FAST(layer_prefill), FAST(layer_step), FAST(kda_chunk), FAST(kda_layer),
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -1,9 +1,11 @@
-"""Elementwise helpers that stay in PyTorch (library routines on either side)."""
+"""The norm in front of a model's layers, and a weight initialiser."""
 from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
 from torch import Tensor
+
+from . import _lib
 
 
 def norm(x: Tensor) -> Tensor:
@@ -11,8 +13,13 @@ def norm(x: Tensor) -> Tensor:
 
     Same call as the reference's ``norm`` (models/daisy/functional.py:6-7): no eps is passed, and torch 2.10
     then adds the machine epsilon of its accumulation type -- fp32's for bf16 and fp32 inputs alike, on the
-    CPU and on the GPU -- not ``finfo(x.dtype).eps`` (see ``NORM_EPS_BF16`` below).
+    CPU and on the GPU -- not ``finfo(x.dtype).eps`` (see ``NORM_EPS_BF16`` below).  The few bf16 rows of a
+    decode step take this package's kernel (same arithmetic, another order of the sum), everything else the library's.
     """
+    if x.is_cuda and x.dtype is torch.bfloat16 and not torch.compiler.is_compiling():
+        y = _lib.native().norm(x, NORM_EPS_BF16)
+        if y is not None:
+            return y
     return F.rms_norm(x, (x.size(-1),))
 
 

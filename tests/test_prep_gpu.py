@@ -124,3 +124,33 @@ def test_prep_rejects_bad_arguments():
     cos = torch.zeros(3, 64, device=DEV)
     with pytest.raises(Exception, match="Rotary buffers too small"):
         ops.qkv_prep(q, q, q, eps=1e-7, cos=cos, sin=cos)
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (3, 64), (1, 1, 72), (2, 5, 512), (1, 1, 1536), (32, 520), (33, 520), (2, 8192), (1, 8200)])
+def test_norm_rows(shape):
+    """Rows of one thread to rows of all of them, with idle threads in the last wavefront; longer ones and more go to the library."""
+    from daisy_amd import norm
+    x = (torch.randn(shape, generator=torch.Generator().manual_seed(shape[-1])) * 3).bfloat16()
+    x[..., 0] = 1e18                                  # squares beyond bf16's exactness, not beyond fp32
+    ref = x.double() * (x.double().pow(2).mean(-1, keepdim=True) + NORM_EPS_BF16).rsqrt()
+    got = norm(x.cuda())
+    assert got.dtype == torch.bfloat16 and got.is_contiguous()
+    # one rounding to bf16 of a value known to fp32's precision
+    assert ((got.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() * 1.001).all()
+
+
+def test_norm_leaves_to_the_library_what_it_does_not_take():
+    from daisy_amd import norm
+    lib = lambda t: torch.nn.functional.rms_norm(t, (t.size(-1),))
+    x = torch.randn(4, 96, device="cuda").bfloat16()
+    for t in (x.float(), x[:, 1:65], x.t(), x.view(-1)[1:97], x.half(), x[:, :7].contiguous()):
+        assert torch.equal(norm(t), lib(t))
+    bad = x.clone()
+    bad[1, 3], bad[2, 5] = float("nan"), float("inf")
+    assert torch.equal(norm(bad).isnan(), lib(bad).isnan()) and torch.equal(norm(bad)[0], lib(bad)[0])
+    w = x.clone().requires_grad_()
+    norm(w).sum().backward()
+    assert w.grad is not None
+    assert norm(torch.empty(0, 64, device="cuda", dtype=torch.bfloat16)).shape == (0, 64)
+    out = torch.func.vmap(norm)(x)
+    assert torch.equal(out, lib(x))
