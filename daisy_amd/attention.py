@@ -430,10 +430,9 @@ class CausalSelfAttention(nn.Module):
                             k_out=k_out, v_out=v_out)
 
     def _attend(self, x: Tensor, ve: Optional[Tensor], attn_mask, kv_out=None, want_q: bool = False):
-        """Returns ``y [B, T, dim]`` and q (rotated), k (rotated), v as ``[B, T, H, D]``.  Where the kernels
+        """Returns ``y [B, T, dim]``, q (rotated) as ``[B, T, H, D]`` and k (rotated), v as ``[B, H, T, D]``.  Where the kernels
         rotate q themselves, the rotated q is computed for the caller only when ``want_q`` asks for it
         (``prefill(debug=True)``), and is ``None`` otherwise."""
-        B, T = x.size(0), x.size(1)
         mask = _as_window_mask(attn_mask)
         if mask.doc_start is not None and mask.doc_start.device != x.device:    # e.g. converted from a mask built on the CPU
             mask = replace(mask, doc_start=mask.doc_start.to(x.device))
@@ -450,11 +449,13 @@ class CausalSelfAttention(nn.Module):
                 STEP_ROWS_KERNEL_MAX, bool(want_q))
             if fast is not None:
                 return fast
+            B, T = x.size(0), x.size(1)
             q, k_rot, v = self._project_qkv_fused(x, ve, 0, *(dest or (None, None)))
             o, _ = ops.prefill_attention(q, k_rot, v, window=window, scale=self.attn_scale, doc_start=mask.doc_start)
             y = F.linear(o.view(B, T, self.m_dim), self.qkvo_w[3])
-            return y, q, k_rot, v
+            return y, q, k_rot.transpose(1, 2), v.transpose(1, 2)
         torch._assert(dest is None, "writing keys and values to a destination needs the fused pre-attention kernel")
+        B, T = x.size(0), x.size(1)
         q, k, v = self._project_qkv(x)
         dtype = q.dtype
         v = self._mix_ve(v, ve)
@@ -466,14 +467,14 @@ class CausalSelfAttention(nn.Module):
             o, k_rot = ops.prefill_attention_f32(q, k, v, window=window, scale=self.attn_scale, cos=cos, sin=sin,
                                                  doc_start=mask.doc_start)
             y = F.linear(o.view(B, T, self.m_dim), self.qkvo_w[3])
-            return y, q_rot, k_rot, v
+            return y, q_rot, k_rot.transpose(1, 2), v.transpose(1, 2)
         o, k_rot = ops.prefill_attention(
             self._kernel_dtype(q), self._kernel_dtype(k), self._kernel_dtype(v),
             window=window, scale=self.attn_scale, cos=cos, sin=sin, doc_start=mask.doc_start)
         y = o.view(B, T, self.m_dim).to(dtype)
         y = F.linear(y, self.qkvo_w[3])
         q_rot = _apply_rope(q, cos[None, :, None, :], sin[None, :, None, :]) if want_q else None
-        return y, q_rot, k_rot.to(dtype), v
+        return y, q_rot, k_rot.to(dtype).transpose(1, 2), v.transpose(1, 2)
 
     # -- reference interface -----------------------------------------------
     def forward(self, x: Tensor, ve: Optional[Tensor], block_mask=None, attn_mask: MaskLike = None):
@@ -497,8 +498,9 @@ class CausalSelfAttention(nn.Module):
         if debug:
             aliased = kv_out is not None or getattr(_as_window_mask(attn_mask), "kv_out", None) is not None
             self.last_q = q
-            self.last_k = k.clone() if aliased else k
-        return y, k.transpose(1, 2), v.transpose(1, 2)
+            k_rows = k.transpose(1, 2)
+            self.last_k = k_rows.clone() if aliased else k_rows
+        return y, k, v
 
     def step(self, x, k_ctx: Union[Tensor, RingContext], v_ctx: Union[Tensor, RingContext], pos: Union[int, Tensor],
              ve: Optional[Tensor], window: Optional[int]):

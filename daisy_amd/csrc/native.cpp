@@ -291,7 +291,7 @@ PyObject* py_prefill_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // layer_prefill(x, qkvo_w, cos, sin, H, D, window, doc_start, ve, g_ve, k_out, v_out, scale, eps, max_rows, want_q)
-//   -> (y [B, T, dim], q or None, k, v [B, T, H, D])
+//   -> (y [B, T, dim], q [B, T, H, D] or None, k, v [B, H, T, D])   (rows of a token side by side in memory all the same)
 // CausalSelfAttention.prefill on bf16 weights: QKV projection, norm + RoPE + value mix, attention, output projection.
 PyObject* py_layer_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -328,8 +328,15 @@ PyObject* py_layer_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const uint16_t* wp = (const uint16_t*)ptr(w);
   const std::array<int64_t, 4> shape{B, T, H, D};
   const int64_t full[3] = {T * dim, dim, D};
-  Tensor k = k_out ? *k_out : empty(shape, at::kBFloat16, x), v = v_out ? *v_out : empty(shape, at::kBFloat16, x);
-  const Strides3 ks(k), vs(v);
+  // (made as the caller gets them: two views from Python cost the host a sixth of a small layer's call)
+  const std::array<int64_t, 4> by_head{B, H, T, D}, by_head_strides{T * dim, D, dim, 1};
+  auto rows = [&] { return Tensor(at::detail::empty_strided_cuda(by_head, by_head_strides, at::kBFloat16, x.device())); };
+  Tensor k = k_out ? *k_out : rows(), v = v_out ? *v_out : rows();
+  Strides3 ks, vs;
+  for (int i = 0; i < 3; ++i) {
+    ks.s[i] = k_out ? k_out->stride(i) : full[i];
+    vs.s[i] = v_out ? v_out->stride(i) : full[i];
+  }
   Tensor q = empty(shape, at::kBFloat16, x);
   if (max_rows > 0 && r.M > max_rows && daisy::proj_qkv_wanted(r.M, 3 * dim, dim)) {
     daisy::QkvEpilogue e{(uint16_t*)ptr(q), full[0], full[1], full[2], (uint16_t*)ptr(k), ks.s[0], ks.s[1], ks.s[2],
@@ -368,8 +375,8 @@ PyObject* py_layer_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
   PyObject* res = PyTuple_New(4);
   PyTuple_SET_ITEM(res, 0, wrap(y));
   PyTuple_SET_ITEM(res, 1, want_q ? wrap(q) : new_none());
-  PyTuple_SET_ITEM(res, 2, wrap(k));
-  PyTuple_SET_ITEM(res, 3, wrap(v));
+  PyTuple_SET_ITEM(res, 2, wrap(k_out ? k.transpose(1, 2) : k));
+  PyTuple_SET_ITEM(res, 3, wrap(v_out ? v.transpose(1, 2) : v));
   return res;
   END_HANDLE_TH_ERRORS
 }
