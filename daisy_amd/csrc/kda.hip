@@ -747,6 +747,17 @@ __device__ __forceinline__ bf16x8 pack_rest2(const f32x4& t0, const f32x4& t1, b
   return pack_acc2(l0, l1);
 }
 
+// Tiles I .. N - 1 of a state times the decays of their rows: dec[i] those of tile i, or one register set of which lane i of 16 holds
+// tile i's (a lane move in the product's operand).  `behind(i)`: what follows tile i.
+template <int I, int N, int SETS, typename F> __device__ __forceinline__ void decay_tiles(f32x4* S, const f32x4 (&dec)[SETS], F behind) {
+  if constexpr (I < N) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[I][r] *= SETS == 1 ? from_row<I>(dec[0][r]) : dec[I % SETS][r];
+    behind(I);
+    decay_tiles<I + 1, N>(S, dec, behind);
+  }
+}
+
 constexpr int KCT = 2;                        // tiles of 16 value columns per workgroup
 constexpr int KPW = 2;                        // data-moving wavefronts per workgroup
 constexpr int KSTAGES = 3;                    // LDS stages of chunk data
@@ -797,8 +808,8 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
     // The column groups of a (batch, head) ask for the same bytes at the same time.  Each begins its run at another place, so that
     // first requests differ and later ones find the L2 filled (T = 8192: 64 heads of 128 469 -> 455 us, both kernels), and
     // in turns with a pause between: all at once they delay the other wavefronts' LDS and store traffic (4 heads of 128 215 -> 184 us,
-    // of 64 134 -> 117).  With most compute units at it a longer pause is the better one (456 against 458 us; 192 against 184 the other
-    // way round).  The first chunks, which nothing computes beside, are asked for without a pause, and the last outputs' part is not waited
+    // of 64 134 -> 117).  With most compute units at it, once, a longer pause is the better one (456 against 458 us; 192 against 184 the other
+    // way round; 384 workgroups, 8 x 1000 rows, 12 heads of 128: 94.2 us, 88.4 with the shorter one).  The first chunks, which nothing computes beside, are asked for without a pause, and the last outputs' part is not waited
     // for in the interval that asks for it (64 sequences of 64 rows, 16 heads of 64: 52.1 -> 50.4 us; 4 of 100 rows, 24 heads of 128:
     // 32.5 -> 31.0).  *Tried:* one dword of every line fetched further ahead, by these or by a wavefront of its own, and from the
     // scalar side: slower, answers come back in order and hits wait behind misses.
@@ -806,7 +817,7 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
     constexpr int NM1 = 3 * KC * KD * 2 / 1024 / KPW, NO1 = Blob::kOut / 1024 / KPW;
     static_assert(NM1 * KPW * 1024 == Blob::kDec && NO1 * KPW * 1024 == Blob::kOut && Blob::kChain - Blob::kDec == 1024, "runs of whole KiB");
     constexpr int kTurns = NM1 / 3;
-    const bool crowded = gridDim.x >= 192;
+    const bool crowded = gridDim.x >= 192 && gridDim.x <= 256;
     const uint32_t stage_lds = lds_address(&stage[0][0]);
     const int n_rows = sp.tok_end - sp.tok0, v_pitch = 2 * p.H * p.Dv;
     const char* const my_v = (const char*)(p.v + ((int64_t)sp.tok0 * p.H + h) * p.Dv);
@@ -940,7 +951,10 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
   // the link.
   bf16x8 ka[2][NM], mh[NS], ml[NS];
   u32x2 vr[2];
-  f32x4 dcc[NS];
+  // The decays of a lane's rows of all tiles are the same for 16 lanes.  With 8 tiles each lane reads those of one of them (8 heads of 128 of
+  // 2 x 1000 rows 37.9 -> 37.4 us, 4 of 8192 181.5 -> 175.3), with 4 all of them (4 heads of 64 of 8192 rows 112.8 us, 114.4 with one).
+  constexpr int DECS = KD == 128 ? 1 : NS;
+  f32x4 dec[DECS];
   auto read_v = [&](lds_cptr sb) {
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) vr[mt] = lds_column4(sb + rdv + 16 * mt * 64);
@@ -949,14 +963,19 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) ka[mt][m] = lds_bf16x8(sb + Blob::kKg + 16 * mt * 2 * KD + rdk[m]);
   };
-  auto read_dec = [&](lds_cptr sb, int i) { dcc[i] = lds_f32x4(sb + Blob::kDec + 4 * (32 * (i >> 1) + 8 * q4 + 4 * (i & 1))); };
+  auto read_dec = [&](lds_cptr sb, int set) {
+    const int i = DECS == 1 ? ln & (NS - 1) : set;
+    dec[set] = lds_f32x4(sb + Blob::kDec + 4 * (32 * (i >> 1) + 8 * q4 + 4 * (i & 1)));
+  };
   auto read_ml = [&](lds_cptr sb, int i) { ml[i] = lds_bf16x8(sb + Blob::kMl + 16 * i * 64 + rd64); };
   auto read_mh = [&](lds_cptr sb, int i) { mh[i] = lds_bf16x8(sb + Blob::kMh + 16 * i * 64 + rd64); };
   read_v(stage0);
 #pragma unroll
   for (int m = 0; m < NM; ++m) read_ka(stage0, m);
 #pragma unroll
-  for (int i = 0; i < NS; ++i) { read_dec(stage0, i); read_ml(stage0, i); read_mh(stage0, i); }
+  for (int i = 0; i < DECS; ++i) read_dec(stage0, i);
+#pragma unroll
+  for (int i = 0; i < NS; ++i) { read_ml(stage0, i); read_mh(stage0, i); }
   __syncthreads();
 
   for (int n = 0; n < nc; ++n) {
@@ -969,18 +988,21 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) X[mt] = f32x4{bf16lo_to_f32(vr[mt].x), bf16hi_to_f32(vr[mt].x), bf16lo_to_f32(vr[mt].y), bf16hi_to_f32(vr[mt].y)};
     read_v(sb);
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
+    auto group = [&](auto which) {
+      constexpr int m = decltype(which)::value;
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) X[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[mt][m], Sb[m], X[mt], 0, 0, 0);
       read_ka(sb, m);
-#pragma unroll
-      for (int i = m * NS / NM; i < (m + 1) * NS / NM; ++i) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) S[i][r] *= dcc[i][r];
-        read_dec(sb, i);
-      }
+      decay_tiles<m * NS / NM, (m + 1) * NS / NM>(S, dec, [&](int i) {
+        if (DECS > 1 || i == NS - 1) read_dec(sb, DECS > 1 ? i : 0);
+      });
       __builtin_amdgcn_sched_barrier(0);
+    };
+    group(std::integral_constant<int, 0>{});
+    group(std::integral_constant<int, 1>{});
+    if constexpr (NM > 2) {
+      group(std::integral_constant<int, 2>{});
+      group(std::integral_constant<int, NM - 1>{});
     }
     // S = exp(G_last) (.) S + M X, both operands split into two bf16 terms; the tiles in two halves, so that the first
     // one's conversions run beside the second one's products
