@@ -507,19 +507,19 @@ __global__ __launch_bounds__(kPrefillThreads, 4) void prefill_wide_tile_kernel(P
 
 // Few workgroups (a prompt of one or two thousand tokens of one sequence): blocks of 128 queries leave most compute
 // units idle and the last block walks all of its keys with one step in flight.  Here a workgroup is 32 queries, its
-// four wavefronts take every fourth key tile each -- tiles of their own, copied into LDS areas of their own, no
-// barrier in the loop -- and the four partial results (maximum, sum, O^T) meet in LDS at the end.  K(n+1) is copied
+// W wavefronts (four, or eight: eight_wavefronts) take every W-th key tile each -- tiles of their own, copied into LDS areas of their own, no
+// barrier in the loop -- and the partial results (maximum, sum, O^T) meet in LDS at the end.  K(n+1) is copied
 // while the softmax and the second product of tile n run, V(n+1) while the scores of tile n+1 do (in-order vmcnt:
 // at most one tensor's copies stay outstanding).  A tile is fetched once per 32 queries instead of once per 128, so
 // long grids are better off with prefill_tile_kernel (the rule stands at launch_mfma).
-template <int D>
-__global__ __launch_bounds__(kPrefillThreads, 2) void prefill_split_kernel(PrefillParams p) {
+template <int D, int W>
+__global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kernel(PrefillParams p) {
   constexpr int NS = D / 16, NDT = D / 32, HALF = D / 2, CPR = D / 8;
   constexpr int RPL = 64 / CPR, NCP = kTBN / RPL, TILE = kTBN * D;    // NCP copies of 1 KiB per tile
   auto swz_k = [](int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); };
   auto swz_v = [](int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
-  __shared__ __attribute__((aligned(1024))) uint16_t tiles[4][2][TILE];   // [wavefront][K, V]; the fp32 partial O at the end
-  __shared__ float part_m[4][32], part_l[4][32];
+  __shared__ __attribute__((aligned(1024))) uint16_t tiles[W][2][TILE];   // [wavefront][K, V]; the fp32 partial O at the end
+  __shared__ float part_m[W][32], part_l[W][32];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -631,9 +631,9 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_split_kernel(Prefi
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
 
-  for (; t <= t_hi; t += 4) {
+  for (; t <= t_hi; t += W) {
     const int kv0 = t * kTBN;
-    const bool more = t + 4 <= t_hi;
+    const bool more = t + W <= t_hi;
     // K(n) has landed when only V(n)'s copies are outstanding
     __builtin_amdgcn_s_waitcnt(0x0F70 | NCP);
     asm volatile("" ::: "memory");
@@ -646,7 +646,7 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_split_kernel(Prefi
       kf[s] = __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)(size_t)(k_a0 ^ (32u * s)));
     __builtin_amdgcn_s_waitcnt(0xC07F);    // lgkmcnt(0): the fragments are out of LDS, the area takes the next tile
     asm volatile("" ::: "memory");
-    if (more) copy_k(t + 4);
+    if (more) copy_k(t + W);
 #pragma unroll
     for (int s = 0; s < NS; ++s) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qreg[s], sacc, 0, 0, 0);
     if (!(kv0 + kTBN - 1 <= min(q0, p.T - 1) && kv0 >= lo_max)) {
@@ -701,7 +701,7 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_split_kernel(Prefi
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);    // the V fragments are out of LDS
     asm volatile("" ::: "memory");
-    if (more) copy_v(t + 4);
+    if (more) copy_v(t + W);
   }
 
   // Partial results: each lane of a pair holds its share of the row sum; O^T as [query][channel] fp32 in the
@@ -721,17 +721,18 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_split_kernel(Prefi
   __syncthreads();
   // 8 channels per thread and pass
 #pragma unroll
-  for (int it = 0; it < 32 * CPR / kPrefillThreads; ++it) {
-    const int idx = tid + kPrefillThreads * it, row = idx / CPR, c = idx % CPR;
+  for (int it = 0; it < (32 * CPR + 64 * W - 1) / (64 * W); ++it) {
+    const int idx = tid + 64 * W * it, row = idx / CPR, c = idx % CPR;
+    if (32 * CPR < 64 * W && idx >= 32 * CPR) break;
     float m = part_m[0][row];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) m = fmaxf(m, part_m[w][row]);
+    for (int w = 1; w < W; ++w) m = fmaxf(m, part_m[w][row]);
     const float mu = (m == -INFINITY) ? 0.f : m;
     float l = 0.f, acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < W; ++w) {
       const float a = fast_exp2(part_m[w][row] - mu);
       l = fmaf(part_l[w][row], a, l);
       const float* src = reinterpret_cast<const float*>(&tiles[w][0][0]) + row * D;
@@ -876,6 +877,20 @@ static int64_t split_limit(const PrefillParams& p) {
   return full && p.T >= 1024 ? 384 : p.window <= 0 || p.window >= 1024 ? 192 : 144;
 }
 
+// When those are eight wavefronts: while a compute unit has no second workgroup to run and the longest block has more key tiles than four of them
+// take in two turns (us, four / eight; heads of 128, no window: 12 heads x 384 rows 7.0 / 6.6, 8 x 1024 11.3 / 10.1, 4 x 2048 18.3 / 14.9, 2 x 4096 31 / 23;
+// window 1024, 4 x 2048 12.7 / 10.3; 256, 8 x 1024 7.5 / 7.0; 128, 32 x 256 6.6 / 6.1; heads of 64, 4 x 2048 13.3 / 10.1; 128 rows 5.0 / 5.2, 256 5.9 / 6.0;
+// window 1024, 6 x 2048 14.0 / 16.7).  Causal blocks differ in length, so that long ones gain with twice the workgroups too (heads of 64, 16 x 1024 8.9 /
+// 8.8, 8 x 2048 13.8 / 12.2; of 128, 12 x 1024 12.4 / 12.9, 8 x 1536 15.8 / 13.9, 4 x 4096 35 / 30).  Documents' lengths are not known here.
+template <int D>
+static bool eight_wavefronts(const PrefillParams& p, int64_t workgroups) {
+  if (p.doc_start != nullptr) return false;
+  const bool full = p.window <= 0 || p.window >= p.T;
+  const int tiles = full ? (p.T + kTBN - 1) / kTBN : (p.window - 2 + kTBN) / kTBN + 1;      // of the longest block
+  if (workgroups <= 256) return tiles >= (full ? 9 : 5);
+  return full && workgroups <= 512 && tiles >= (D == 64 ? 32 : 48);
+}
+
 template <int D>
 static int launch_mfma(PrefillParams p, hipStream_t s) {
   const int64_t nwg = (int64_t)p.nqb * p.H * p.B;
@@ -894,7 +909,8 @@ static int launch_mfma(PrefillParams p, hipStream_t s) {
   }
   if (nwg <= split_limit<D>(p)) {
     const int64_t nsw = (int64_t)((p.T + 31) / 32) * p.H * p.B;
-    hipLaunchKernelGGL((prefill_split_kernel<D>), dim3((unsigned)nsw), dim3(kPrefillThreads), 0, s, p);
+    if (eight_wavefronts<D>(p, nsw)) hipLaunchKernelGGL((prefill_split_kernel<D, 8>), dim3((unsigned)nsw), dim3(512), 0, s, p);
+    else hipLaunchKernelGGL((prefill_split_kernel<D, 4>), dim3((unsigned)nsw), dim3(kPrefillThreads), 0, s, p);
     DAISY_CHECK_LAUNCH("prefill_split_kernel");
     return DAISY_OK;
   }

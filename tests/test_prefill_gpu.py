@@ -138,6 +138,18 @@ def test_prefill_tiles_of_64_keys(T, window, docs):
                                 doc_start=None if doc_start is None else doc_start.cuda())
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,T,H,window", [(1, 257, 1, None), (1, 288, 3, None), (1, 289, 2, None), (2, 161, 2, 97), (1, 200, 3, 98), (1, 1023, 8, 128),
+                                          (1, 1025, 8, 128), (1, 1030, 12, None), (1, 1537, 9, None), (3, 31, 2, None)])
+def test_few_query_blocks_on_both_sides_of_eight_wavefronts(B, T, H, window, D):
+    """Wavefronts with no tile, one, and several; the last tile short; as many workgroups as either rule allows, and more."""
+    q, k, v = _inputs(B, T, H, D, seed=T)
+    rows = None if T <= 1100 else torch.cat([torch.arange(40), torch.arange(T - 70, T)])
+    ref, _ = _oracle(q, k, v, window, rows=rows)
+    o, _ = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), window=window)
+    assert_close_bf16(o if rows is None else o[:, rows.cuda()], ref, f"T{T} H{H} W{window}")
+
+
 def test_prefill_is_deterministic_and_window_invariant():
     """A window >= T equals full causal attention bit for bit; repeated calls agree."""
     B, T, H, D = 1, 320, 2, 128
