@@ -648,10 +648,8 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
       for (int i = j + 1; i < 16; ++i) tc[i] = fmaf(-ar[i >> 2][i & 3], xj, tc[i]);
     }
     wave_lds_fence();
-    if (lane < 16) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) Td[I][i][li] = tc[i];
-    }
+    for (int i = 0; i < 16; ++i) Td[I][i][li] = tc[i];      // (all lanes, four the same: in a branch around this the sums would go there, behind all of their operands)
   }
   __syncthreads();   // both inverses, A_10 and the rows are in place
   // T_10 = -T_11 (A_10 T_00) in two fp32 matrix products, both wavefronts all of it.  As right operand (lane
