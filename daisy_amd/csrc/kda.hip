@@ -263,7 +263,9 @@ __device__ __forceinline__ float sum_over_q4(float x) {       // over the four l
 
 // A chunk's block in the workspace, stored in pieces of 16 bytes past the caches or through them: there the cache policy sc1 writes
 // through the L2 at once.  Left dirty there, all blocks of a launch of a few rounds are written back at its end (512 chunks x heads of
-// 128: 16.7 us, 13.3 written through).  As buffer stores, which take the policy as an argument.
+// 128: 16.7 us, 13.3 written through).  As buffer stores, which take the policy as an argument.  The whole offset is the lane's: the
+// instruction behind a store of 16 bytes must not write its data registers yet, and with an offset in a scalar register the compiler
+// does not keep it from that (the first word of a piece was then, in some 20 of 928 blocks, what the next instruction had put there).
 constexpr int kWriteThrough = 16;             // sc1
 constexpr int kBufferWord3 = 0x00020000;      // an untyped buffer of bytes
 template <bool CACHED> struct BlockOut {      // CACHED: all of them through the caches
@@ -273,7 +275,7 @@ template <bool CACHED> struct BlockOut {      // CACHED: all of them through the
   __device__ __forceinline__ BlockOut(char* b, int bytes, bool past) : base(b), rsrc(__builtin_amdgcn_make_buffer_rsrc(b, 0, bytes, kBufferWord3)), streamed(past) {}
   __device__ __forceinline__ void store(const u32x4& v, int at, int part) const {        // byte `at` (the lane's) of the part at byte `part`
     if (!CACHED && streamed) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(base + part + at));
-    else __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, at, part, kWriteThrough);
+    else __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, at + part, 0, kWriteThrough);
   }
 };
 
@@ -649,7 +651,8 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     }
     wave_lds_fence();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) Td[I][i][li] = tc[i];      // (all lanes, four the same: in a branch around this the sums would go there, behind all of their operands)
+    for (int i = 0; i < 16; ++i) Td[I][i][li] = tc[i];      // all lanes, four the same: into a branch around this the compiler moves the sums, behind
+                                                            // all of their operands (heads of 64: 164 registers instead of 126, three wavefronts a SIMD)
   }
   __syncthreads();   // both inverses, A_10 and the rows are in place
   // T_10 = -T_11 (A_10 T_00) in two fp32 matrix products, both wavefronts all of it.  As right operand (lane
@@ -690,9 +693,10 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     th[1] = __builtin_bit_cast(bf16x8, hi);
     tl[1] = __builtin_bit_cast(bf16x8, lo);
   }
-  // Row `row` of (right operand)^T T: the products come out with four consecutive columns of T per lane and column block,
+  // Row 16 tile + li of (right operand)^T T: the products come out with four consecutive columns of T per lane and column block,
   // which is the stored piece q4 of that row; both terms of it leave from here, 16 whole rows per instruction.
-  auto times_t = [&](const bf16x8& rh, const bf16x8& rl, int part_hi, int part_lo, int row) {
+  const int t_at = li * 64 + 16 * (q4 ^ piece_swizzle<64>(li));       // (rows 16 apart share a swizzle)
+  auto times_t = [&](const bf16x8& rh, const bf16x8& rl, int part_hi, int part_lo, int tile) {
     float out[8];
 #pragma unroll
     for (int J = 0; J < 2; ++J) {
@@ -705,9 +709,8 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     }
     u32x4 hi, lo;
     split_pack8(out, hi, lo);
-    const int off = row * 64 + 16 * (q4 ^ piece_swizzle<64>(row));
-    block.store(hi, off, part_hi);
-    block.store(lo, off, part_lo);
+    block.store(hi, t_at, part_hi + 1024 * tile);
+    block.store(lo, t_at, part_lo + 1024 * tile);
   };
   {
     float pv[8];
@@ -715,7 +718,7 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     for (int e = 0; e < 4; ++e) { pv[e] = P[0][e]; pv[4 + e] = P[1][e]; }
     u32x4 hi, lo;
     split_pack8(pv, hi, lo);
-    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), Blob::kPh, Blob::kPl, 16 * I + li);
+    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), Blob::kPh, Blob::kPl, I);
   }
   // ---- M = (exp(G_last - G) k)^T T, half of the chunk's channels per wavefront: row 16 i + li of the block is channel
   // 32 (i / 2) + 8 (li / 4) + 4 (i % 2) + li % 4, the one that row of the state's tile i stands for
@@ -729,7 +732,7 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     const u32x2 l0 = lds_column4((lds_cptr)&rows[1][0] + a0), l1 = lds_column4((lds_cptr)&rows[1][0] + a0 + 16 * ROW);
     hi = u32x4{h0.x, h0.y, h1.x, h1.y};
     lo = u32x4{l0.x, l0.y, l1.x, l1.y};
-    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), Blob::kMh, Blob::kMl, 16 * i + li);
+    times_t(__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, lo), Blob::kMh, Blob::kMl, i);
   }
 }
 

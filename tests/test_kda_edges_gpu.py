@@ -5,7 +5,7 @@ import torch
 import torch.nn.functional as F
 
 import oracle
-from daisy_amd import chunk_kda
+from daisy_amd import _lib, chunk_kda
 from helpers import assert_close_bf16
 
 pytestmark = pytest.mark.gpu
@@ -113,6 +113,22 @@ def test_kda_blocks_through_and_past_the_caches(T, H, D, packed, mb):
             part, state = chunk_kda(*(t[:, lo:hi].contiguous() for t in (q, k, v, gl, beta)), initial_state=state, **kw)
             assert torch.equal(part, o[:, lo:hi]), (lo, hi)
         assert torch.equal(state[0], S[i])
+
+
+# The blocks themselves, all of their bytes, from call to call: a 16-byte store's data registers written again by the next instruction
+# changed the low terms of rows 28 .. 31 of M in 2 % of the blocks, which only those of the last chunk show in a result, and by an ulp.
+@pytest.mark.parametrize("T,H,D", [(3712, 8, 128), (3712, 12, 64)])
+def test_kda_blocks_are_the_same_in_every_call(T, H, D):
+    lib = _lib.load()
+    q, k, v, gl, beta = (t.cuda() for t in _inputs(1, T, H, D, D, seed=T))
+    n = lib.daisy_kda_workspace_bytes(1, T, H, D, D, 64)
+    blocks = [torch.zeros(n, dtype=torch.uint8, device="cuda") for _ in range(4)]
+    o, S = torch.empty(1, T, H, D, dtype=torch.bfloat16, device="cuda"), torch.empty(1, H, D, D, device="cuda")
+    assert q.dtype == torch.bfloat16 and gl.dtype == beta.dtype == torch.float32 and all(t.is_contiguous() for t in (q, k, v, gl, beta))
+    for ws in blocks:
+        assert lib.daisy_kda_chunk_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), gl.data_ptr(), 0, beta.data_ptr(), None, o.data_ptr(), S.data_ptr(),
+                                       1, T, H, D, D, 64, D ** -0.5, 1, 1e-6, ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream) == 0
+    assert blocks[0].any() and all(torch.equal(ws, blocks[0]) for ws in blocks[1:])
 
 
 # One key channel carries everything and decays by a step whose factor two bf16 terms hold worst (2^-18 off, the same way in every
