@@ -301,6 +301,129 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
   }
 }
 
+// Several narrow products of the same rows of x in one tile of 128 rows and up to 288 columns, so that x is read once: with a column of
+// tiles of its own per product, two or three of 128, every one of them pulls x again.  M = 32768, K = 2048, N = 128 + 128 + 16: 52.9 us with
+// 128 x 128 -> 39.0 (3.7 TB/s of x and results).  A step of 64 elements of K takes 1.0 us even of a single workgroup: reads of the LDS, products
+// and waits in a row.  Eight wavefronts of 32 rows x 144 columns.  *Tried:* 64 x 80 (fewer LDS reads): 40.9; only the copies that narrower products
+// need: 39.4, and 35.5 instead of 32.4 for a single workgroup.
+constexpr int kJoinedRows = 128, kJoinedColumns = 288;
+__global__ __launch_bounds__(512) void proj_joined_kernel(ProjSegmentsParams p) {
+  constexpr int BM = kJoinedRows, BN = kJoinedColumns, BK = 64, STAGES = 3, NW = 8;
+  constexpr int WM = 32, WN = 144, MI = WM / 16, NI = WN / 16, KK = BK / 32;
+  constexpr int RB = 2 * BK, ABYTES = BM * RB, STAGE = (BM + BN) * RB;
+  constexpr int CA = BM / 8 / NW, CB = (BN / 8 + NW - 1) / NW, CPW = CA + CB;       // copies of 8 rows per wavefront and step
+  __shared__ __attribute__((aligned(1024))) char smem[STAGES * STAGE];
+  auto swz = [](int r) { return (r >> 1) & 7; };
+
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 15, q4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 3, wn = wave >> 2;
+  const int m0 = blockIdx.x * BM;
+
+  // Eight rows of W per copy, of one product: each begins at a multiple of eight columns (tile_end: of the last one behind it).  Copies past
+  // the last column, and the ones that the last wavefronts do not have, repeat the last one that there is, into the same place.
+  const int cr = lane / 8, cp = lane % 8;
+  int offa[CA], offb[CB], to[CB];
+  const uint16_t* wb[CB];
+  const uint16_t* xa = p.seg[0].x + (int64_t)m0 * p.seg[0].x_sm;
+#pragma unroll
+  for (int j = 0; j < CA; ++j) {
+    const int r = 8 * (wave + NW * j) + cr;
+    offa[j] = 2 * (int)((min(m0 + r, p.M - 1) - m0) * p.seg[0].x_sm) + 16 * (cp ^ swz(r));
+  }
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    const int c8 = 8 * min(wave + NW * j, p.NT - 1);
+    int i = 0;
+    while (i + 1 < p.n && c8 >= p.seg[i].tile_end) ++i;
+    const int row0 = c8 - (i > 0 ? p.seg[i - 1].tile_end : 0);
+    wb[j] = p.seg[i].w + (int64_t)row0 * p.seg[i].w_sn;
+    offb[j] = 2 * (int)((min(row0 + cr, p.seg[i].N - 1) - row0) * p.seg[i].w_sn) + 16 * (cp ^ swz(c8 + cr));
+    to[j] = ABYTES + c8 * RB;
+  }
+  const uint32_t lds0 = lds_address(smem);
+  auto issue = [&](int st) {
+    const uint32_t dst = lds0 + st * STAGE;
+#pragma unroll
+    for (int j = 0; j < CB; ++j) { copy16_to_lds_async(wb[j], offb[j], dst + to[j]); wb[j] += BK; }
+#pragma unroll
+    for (int j = 0; j < CA; ++j) copy16_to_lds_async(xa, offa[j], dst + 1024 * (wave + NW * j));
+    xa += BK;
+  };
+
+  f32x4 acc[NI][MI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MI; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int nk = p.K / BK;
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < nk) issue(s);
+  // (columns that no product has are multiplied from what the LDS holds and not stored)
+  const uint32_t fa = lds0 + (WM * wm + ln) * RB + 16 * (q4 ^ swz(ln));
+  const uint32_t fb = lds0 + ABYTES + (WN * wn + ln) * RB + 16 * (q4 ^ swz(ln));
+  auto frag = [&](uint32_t a) { return __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)(size_t)a); };
+
+  int st = 0;
+  for (int k = 0; k < nk; ++k) {
+    if (k + 1 == nk) wait_vmcnt<0>(); else wait_vmcnt<CPW>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint32_t so = st * STAGE;
+    bf16x8 a[KK][NI], b[KK][MI];
+#pragma unroll
+    for (int j = 0; j < MI; ++j) b[0][j] = frag(fa + so + 16 * RB * j);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) a[0][i] = frag(fb + so + 16 * RB * i);
+    __builtin_amdgcn_sched_barrier(0);
+    // every wavefront is done with step k - 1: its stage takes step k + 2
+    if (k + STAGES - 1 < nk) issue(st == 0 ? STAGES - 1 : st - 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      if (kk + 1 < KK) {
+#pragma unroll
+        for (int j = 0; j < MI; ++j) b[kk + 1][j] = frag((fa ^ (64u * (kk + 1))) + so + 16 * RB * j);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) a[kk + 1][i] = frag((fb ^ (64u * (kk + 1))) + so + 16 * RB * i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < MI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][i], b[kk][j], acc[i][j], 0, 0, 0);
+    }
+    st = st + 1 == STAGES ? 0 : st + 1;
+  }
+  __syncthreads();
+
+  // Output tile [BM][BN] bf16 in LDS, its pieces in fours swizzled by the row, then whole rows of every product.
+  constexpr int CHN = BN / 8;
+  auto tile_at = [&](int m, int c) { return smem + m * (2 * BN) + 16 * (c ^ (m & 3)); };
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int n = WN * wn + 16 * i + 4 * q4;
+#pragma unroll
+    for (int j = 0; j < MI; ++j)
+      *reinterpret_cast<u32x2*>(tile_at(WM * wm + 16 * j + ln, n >> 3) + 2 * (n & 7)) =
+          u32x2{pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
+  }
+  __syncthreads();
+  for (int idx = tid; idx < BM * CHN; idx += 64 * NW) {
+    const int m = idx / CHN, c = idx % CHN;
+    if (m0 + m >= p.M || c >= p.NT) continue;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(tile_at(m, c));
+    uint16_t* y = p.seg[0].y + (int64_t)(m0 + m) * p.seg[0].y_sm + 8 * c;
+#pragma unroll
+    for (int i = 1; i < kMaxSegments; ++i)
+      if (i < p.n && 8 * c >= p.seg[i - 1].tile_end) y = p.seg[i].y + (int64_t)(m0 + m) * p.seg[i].y_sm + 8 * c - p.seg[i - 1].tile_end;
+    *reinterpret_cast<u32x4*>(y) = v;
+  }
+}
+
 // The tile shapes, and what choosing one costs.  `per_cu` workgroups of a shape fit a compute unit; one round of a
 // workgroup on every compute unit takes `one` us at K = 2048 (measured with the operands behind the L2; the time is
 // proportional to K), a round with all of them `full`.  A product of n tiles then costs about 1.5 us plus its rounds, and
@@ -329,8 +452,9 @@ constexpr ProjTile kProjTiles[] = {
     {6, 128, 128, 64, 2, 20.2f, 25.3f},   // 4 wavefronts, 2 stages
     {7, 256, 256, 64, 1, 42.0f, 42.0f},   // 8 wavefronts, 2 stages
 };
+constexpr float kJoinedRound = 30.0f;         // the joined tile, 128 x 288, in the same units
 template <typename COLUMNS>      // columns(bn): columns of tiles of that width
-static int proj_tile(int M, int K, int head, COLUMNS columns) {
+static int proj_tile(int M, int K, int head, COLUMNS columns, float* its_cost = nullptr) {
   int best = 0;
   float least = 0.f;
   for (const ProjTile& t : kProjTiles) {
@@ -341,6 +465,7 @@ static int proj_tile(int M, int K, int head, COLUMNS columns) {
     const float cost = (float)(n / round) * t.full + (tail > 256 ? t.full : tail > 0 ? t.one : 0.f);
     if (best == 0 || cost < least) { best = t.code; least = cost; }
   }
+  if (its_cost) *its_cost = least;
   return best;
 }
 
@@ -430,7 +555,29 @@ int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, in
     for (int i = 0; i < n; ++i) c += (seg[i].N + bn - 1) / bn;
     return c;
   };
-  const int by_size = tile ? tile : proj_tile(M, K, 8, columns);
+  // All products in one tile across (code 12): the same rows of x, no bias, together at most a tile wide.  By cost, which is a round of its
+  // workgroups (30 at K = 2048, as proj_tile counts); 128 + 128 + 16 columns, the best other tile / this one: K = 2048 and 20000 rows 31.5 / 34.8,
+  // 22000 48.5 / 35.5, 40000 59.3 / 68.1, 45000 75.5 / 69.1, 131072 224 / 183 us; K = 1024, 24000 rows 26.2 / 22.6, 65536 50.8 / 46.7.  Of
+  // short rows the fixed part of a round is too much: K = 512, 32768 rows 19.6 / 17.1, but 45000 26.3 / 28.2; K = 256, 131072 37.5 / 44.9.
+  int across = 0;
+  bool joined = !gates && ((!tile && K >= 1024) || tile == 12);
+  for (int i = 0; i < n; ++i) {
+    across += (seg[i].N + 7) & ~7;
+    joined = joined && seg[i].x == seg[0].x && seg[i].x_sm == seg[0].x_sm && !seg[i].bias;
+  }
+  joined = joined && across <= kJoinedColumns;
+  DAISY_CHECK_SUPPORTED(joined || tile != 12, "proj_segments: tile 12 does not serve these products");
+  float cost = 0.f;
+  const int by_size = tile ? tile : proj_tile(M, K, 8, columns, &cost);
+  const int row_tiles = (M + kJoinedRows - 1) / kJoinedRows;
+  if (joined && (tile || kJoinedRound * ((row_tiles + 255) / 256) < cost)) {
+    int at = 0;
+    for (int i = 0; i < n; ++i) p.seg[i].tile_end = at += (seg[i].N + 7) & ~7;
+    p.NT = across / 8;
+    hipLaunchKernelGGL(proj_joined_kernel, dim3((unsigned)row_tiles), dim3(512), 0, s, p);
+    DAISY_CHECK_LAUNCH("proj_joined_kernel");
+    return DAISY_OK;
+  }
   if (!gates) return dispatch_proj<0>(by_size, p, s);
   DAISY_CHECK_ARG(gates->A_log && gates->dt_bias && gates->logits && gates->beta && gates->H > 0 && gates->Dk % 8 == 0 && seg[0].N == gates->H * gates->Dk,
                   "proj_segments: gate of %d heads of %d channels on a product of %d", gates->H, gates->Dk, seg[0].N);

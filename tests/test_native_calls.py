@@ -124,3 +124,34 @@ def test_a_forced_tile_that_does_not_serve_a_gated_product_is_refused(tile, K):
     seg, gates = _Segment(p, K, p, K, None, p, 128, 128, 0), _Gates(p, p, 2, 64, p, 8, p)
     assert fn(ctypes.byref(seg), 1, 4, K, None, tile, ctypes.byref(gates)) == -2
     assert "tile" in lib.daisy_last_error().decode()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,widths", [(1, 64, (13,)), (127, 128, (128, 128, 16)), (129, 192, (64, 5, 8, 3, 100, 72)), (300, 256, (256, 32)), (24001, 1024, (64, 20, 8))])
+def test_narrow_products_in_one_tile_across(M, K, widths):
+    """One tile for all columns (code 12) against tiles of 128 x 128 (6), which sum over K in the same order: the same bits; by rule at
+    24001 rows; nothing behind a product's rows or columns is written.  Products that one tile does not hold are refused."""
+    lib = _lib.load()
+    fn = lib._ZN5daisy13proj_segmentsEPKNS_11ProjSegmentEiiiP12ihipStream_tiPKNS_8KdaGatesE
+    fn.argtypes = [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p]
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").bfloat16()[:, :K]
+    w = [torch.randn(n, K, generator=g, device="cuda").bfloat16() for n in widths]
+
+    def call(tile, bias=None):
+        y = [torch.full((M + 1, (n + 7) // 8 * 8 + 8), 7.0, dtype=torch.bfloat16, device="cuda") for n in widths]
+        segs = (_Segment * len(widths))(*(_Segment(x.data_ptr(), K + 8, a.data_ptr(), K, bias, b.data_ptr(), b.shape[1], n, 0)
+                                          for a, b, n in zip(w, y, widths)))
+        return fn(ctypes.addressof(segs), len(widths), M, K, torch.cuda.current_stream().cuda_stream, tile, None), y
+
+    results = [call(tile) for tile in (12, 6, 0)]
+    assert [rc for rc, _ in results] == [0, 0, 0]
+    for i, n in enumerate(widths):
+        assert all(torch.equal(y[i][:M, :n], results[1][1][i][:M, :n]) for _, y in results)
+        assert all((y[i][M] == 7).all() and (y[i][:, (n + 7) // 8 * 8:] == 7).all() for _, y in results)
+        ref = x.float() @ w[i].float().T
+        assert (results[0][1][i][:M, :n] - ref).abs().max() <= 2 ** -8 * ref.abs().max()
+    assert call(12, bias=w[0].data_ptr())[0] == -2
+    widths = (128, 128, 40)
+    w = [torch.zeros(n, K, dtype=torch.bfloat16, device="cuda") for n in widths]
+    assert call(12)[0] == -2
