@@ -137,9 +137,10 @@ struct SeqSpan { int tok0, tok_end, c0, nc; };
 // gets the end of the last sequence.  Bounds = the caller's, forced to start at 0, to stay within 0..T and not to decrease
 // (whatever was passed, no kernel then leaves the tensors); chunk slots = running sum of ceil(len / 32).  A lane per
 // sequence, two scans: about 0.5 us in every workgroup of both kernels instead of a launch of one workgroup in front of
-// them (6 us).
+// them (6 us).  BY_LENGTH: `key` counts from the longest one on, equal ones in their order (a lane per sequence only); it becomes
+// the sequence's number.
 constexpr int kScanSeqs = 64;
-__device__ __forceinline__ SeqSpan packed_span(const KdaParams& p, int key, bool by_slot, int& rows_end) {
+template <bool BY_LENGTH = false> __device__ __forceinline__ SeqSpan packed_span(const KdaParams& p, int& key, bool by_slot, int& rows_end) {
   SeqSpan s{0, 0, 0, 0};
   if (p.bounds != nullptr) {
     rows_end = p.bounds[p.n_seq];
@@ -174,12 +175,22 @@ __device__ __forceinline__ SeqSpan packed_span(const KdaParams& p, int key, bool
     if (owner == 0) return s;
     key = __builtin_ctzll(owner);
   }
+  if constexpr (BY_LENGTH) {
+    const int before = __shfl_up(nc, 1);
+    if (__ballot(nc > before && lane > 0) != 0) {                     // (not in that order already)
+      const uint32_t mine = ((uint32_t)nc << 6) + 63 - lane;          // (no two the same)
+      int ahead = 0;
+#pragma unroll 4
+      for (int j = 0; j < p.n_seq; ++j) ahead += (uint32_t)__builtin_amdgcn_readlane((int)mine, j) > mine ? 1 : 0;
+      key = __builtin_ctzll(__ballot(lane < p.n_seq && ahead == key));
+    }
+  }
   s.tok0 = __builtin_amdgcn_readlane(begin, key); s.tok_end = __builtin_amdgcn_readlane(end, key);
   s.nc = __builtin_amdgcn_readlane(nc, key); s.c0 = __builtin_amdgcn_readlane(upto, key) - s.nc;
   return s;
 }
-__device__ __forceinline__ SeqSpan seq_span(const KdaParams& p, int seq, int& rows_end) {
-  if (p.n_seq > 0) return packed_span(p, seq, false, rows_end);
+template <bool BY_LENGTH> __device__ __forceinline__ SeqSpan seq_span(const KdaParams& p, int& seq, int& rows_end) {
+  if (p.n_seq > 0) return packed_span<BY_LENGTH>(p, seq, false, rows_end);
   rows_end = p.B * p.T;
   return SeqSpan{seq * p.T, (seq + 1) * p.T, seq * p.NC, p.NC};
 }
@@ -313,8 +324,8 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   {
     const int slot = blockIdx.x;
     if (p.n_seq > 0) {
-      int rows_end;
-      const SeqSpan sp = packed_span(p, slot, true, rows_end);
+      int seq = slot, rows_end;
+      const SeqSpan sp = packed_span(p, seq, true, rows_end);
       if (sp.nc == 0) return;                    // surplus slots (the grid covers the upper bound)
       t0 = sp.tok0 + (slot - sp.c0) * KC;
       n_live = min(sp.tok_end - t0, KC);
@@ -778,7 +789,8 @@ constexpr int kStateThreads = 64 * (2 * KCT + KPW);
 //  * the outputs are not part of the chain: a second wavefront per tile makes Qg S0 of the chunk from the bf16 state
 //    the first one left in LDS, adds (P T) X when X has arrived, and stores the rows one chunk later;
 //  * neither waits for global memory: two further wavefronts issue the asynchronous copies of the chunks ahead.
-template <int KD>
+// BY_LENGTH: packed sequences from the longest one on (a kernel of its own: with that code ahead of their loop other calls' chains are 1 to 2 % slower).
+template <int KD, bool BY_LENGTH>
 __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p) {
   using Blob = KdaBlob<KD>;
   constexpr int NM = KD / 32, NS = KD / 16;                    // channel groups of 32, state tiles of 16 rows
@@ -792,11 +804,13 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
 
   // The column groups of one (batch, head) on one XCD, in consecutive workgroups of it: they read the same blocks.
   const int NGRP = (p.Dv + KVS * KCT - 1) / (KVS * KCT);       // groups of 32 value columns
-  const int slot = blockIdx.x >> 3, grp = slot % NGRP, bh = 8 * (slot / NGRP) + (blockIdx.x & 7);
+  const int slot = blockIdx.x >> 3, grp = slot % NGRP;
+  int bh = 8 * (slot / NGRP) + (blockIdx.x & 7);
   if (bh >= (p.n_seq > 0 ? p.n_seq : p.B) * p.H) return;
-  const int h = bh % p.H, b = bh / p.H;     // b: batch element, or sequence of a packed batch
-  int rows_end;
-  const SeqSpan sp = seq_span(p, b, rows_end);
+  const int h = bh % p.H;
+  int b = bh / p.H, rows_end;               // b: batch element, or sequence of a packed batch
+  const SeqSpan sp = seq_span<BY_LENGTH>(p, b, rows_end);
+  if constexpr (BY_LENGTH) bh = b * p.H + h;
   const int nc = sp.nc;                      // chunks of this sequence (0 for an empty one)
   const int64_t ci0 = (int64_t)h * p.nc_total + sp.c0;
   const int lane = threadIdx.x & 63, ln = lane & 15, q4 = lane >> 4;
@@ -1131,7 +1145,14 @@ static int kda_launch_width(KdaParams p, int n_streams, hipStream_t s) {
   if (bytes <= kCachedBytes) hipLaunchKernelGGL((kda_prep_kernel<KD, true>), chunks, dim3(128), 0, s, p);
   else hipLaunchKernelGGL((kda_prep_kernel<KD, false>), chunks, dim3(128), memory_bound ? 6144 : 0, s, p);
   DAISY_CHECK_LAUNCH("kda_prep_kernel");
-  hipLaunchKernelGGL(kda_state_kernel<KD>, dim3((unsigned)((n_streams * p.H + 7) / 8 * 8 * groups)), dim3(kStateThreads), 0, s, p);
+  const unsigned chains = (unsigned)((n_streams * p.H + 7) / 8 * 8 * groups);
+  // A chain fills a compute unit: where there are more than 256, a long sequence that starts late ends alone.  Longest first, cut at random places, both
+  // kernels: 10 sequences of T = 4689, 16 heads of 128 102 -> 87 us, 7 of 3000, 12 heads 53 -> 44.4, 7 of 6164, 16 of 64 67.3 -> 56; 40 such batches 4 % on
+  // average.  Where the longest one comes early anyway ranking costs (12 of 12000, 16 of 64 95.5 -> 97.3): 0.03 us a sequence in every workgroup, so
+  // only up to a tenth of a mean chain (else 16 of T = 2088, 8 heads of 128 34.5 -> 35.5, 13 of 148, 12 heads 18.2 -> 19.8); not where they are in that order.
+  const bool by_length = chains > 256 && p.n_seq > 1 && p.n_seq <= kScanSeqs && p.NC >= p.n_seq * p.n_seq;
+  if (by_length) hipLaunchKernelGGL((kda_state_kernel<KD, true>), dim3(chains), dim3(kStateThreads), 0, s, p);
+  else hipLaunchKernelGGL((kda_state_kernel<KD, false>), dim3(chains), dim3(kStateThreads), 0, s, p);
   DAISY_CHECK_LAUNCH("kda_state_kernel");
   return DAISY_OK;
 }

@@ -115,6 +115,26 @@ def test_kda_blocks_through_and_past_the_caches(T, H, D, packed, mb):
         assert torch.equal(state[0], S[i])
 
 
+# More chains than compute units: packed sequences start longest first (a lane per sequence, few enough of them for their rows), unless they
+# are in that order.  Each one's rows and states are those of a call of its own, from a state of its own.
+@pytest.mark.parametrize("lengths", [(40, 33, 512, 0, 512, 130), (600, 300, 300, 20, 1), (1, 31, 700, 64, 65, 64, 1000, 0)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_kda_packed_longest_first(lengths, D):
+    H, n, T = 16, len(lengths), sum(lengths)
+    q, k, v, gl, beta = _inputs(1, T + 5, H, D, 128, seed=T)
+    s0 = torch.randn(n, H, D, 128, generator=torch.Generator().manual_seed(n))
+    cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32)
+    assert n * H * 4 > 256 and T // 32 + n >= n * n
+    o, S = _run(q, k, v, gl, beta, cu_seqlens=cu.cuda(), initial_state=s0.cuda())
+    assert not o[:, T:].any()
+    for i, m in enumerate(lengths):
+        if m == 0:
+            assert torch.equal(S[i], s0[i])
+            continue
+        o1, S1 = _run(*(t[:, cu[i]:cu[i] + m].contiguous() for t in (q, k, v, gl, beta)), initial_state=s0[i:i + 1].cuda())
+        assert torch.equal(o[:, cu[i]:cu[i] + m], o1) and torch.equal(S[i:i + 1], S1)
+
+
 # The blocks themselves, all of their bytes, from call to call: a 16-byte store's data registers written again by the next instruction
 # changed the low terms of rows 28 .. 31 of M in 2 % of the blocks, which only those of the last chunk show in a result, and by an ulp.
 @pytest.mark.parametrize("T,H,D", [(3712, 8, 128), (3712, 12, 64)])
