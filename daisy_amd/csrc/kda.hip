@@ -125,7 +125,6 @@ struct KdaParams {
   // wavefront finds its way by itself (packed_span); beyond, kda_chunk_table_kernel writes bounds [n_seq + 1] = sanitised
   // running lengths, seq_chunk0 [n_seq + 1] = first chunk slot of every sequence, chunk_seq [NC] = sequence of every slot.
   int n_seq; const int32_t* cu; const int32_t* bounds; const int32_t* seq_chunk0; const int32_t* chunk_seq;
-  int cached;     // 1024ths of a sequence's blocks, from its start, that are stored through the caches
   int nc_total;   // chunk slots per head in the workspace: B * NC, or NC for a packed batch
 };
 
@@ -279,13 +278,12 @@ __device__ __forceinline__ float sum_over_q4(float x) {       // over the four l
 // does not keep it from that (the first word of a piece was then, in some 20 of 928 blocks, what the next instruction had put there).
 constexpr int kWriteThrough = 16;             // sc1
 constexpr int kBufferWord3 = 0x00020000;      // an untyped buffer of bytes
-template <bool CACHED> struct BlockOut {      // CACHED: all of them through the caches
+template <bool STREAMED> struct BlockOut {
   char* base;
   __amdgpu_buffer_rsrc_t rsrc;
-  bool streamed;
-  __device__ __forceinline__ BlockOut(char* b, int bytes, bool past) : base(b), rsrc(__builtin_amdgcn_make_buffer_rsrc(b, 0, bytes, kBufferWord3)), streamed(past) {}
+  __device__ __forceinline__ BlockOut(char* b, int bytes) : base(b), rsrc(__builtin_amdgcn_make_buffer_rsrc(b, 0, bytes, kBufferWord3)) {}
   __device__ __forceinline__ void store(const u32x4& v, int at, int part) const {        // byte `at` (the lane's) of the part at byte `part`
-    if (!CACHED && streamed) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(base + part + at));
+    if (STREAMED) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(base + part + at));
     else __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, at + part, 0, kWriteThrough);
   }
 };
@@ -302,7 +300,7 @@ template <bool CACHED> struct BlockOut {      // CACHED: all of them through the
 // *Tried:* both kernels in one launch, two of these wavefronts beside the chain's and blocks shared by flags through the L2: a
 // wavefront alone needs 15000 cycles per block, 2 us a link.  *Tried:* the running sum by adds across lanes (fewer instructions, one
 // more round through the LDS for g): the same time.
-template <int KD, bool CACHED>
+template <int KD, bool STREAMED>
 __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   using Blob = KdaBlob<KD>;
   constexpr int NM = KD / 32, ROW = 2 * KD;                           // contraction groups of 32 channels, bytes of a bf16 row
@@ -320,7 +318,6 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   const int I = __builtin_amdgcn_readfirstlane(tid >> 6);
   int t0, n_live;
   int64_t ci;
-  bool streamed;
   {
     const int slot = blockIdx.x;
     if (p.n_seq > 0) {
@@ -330,18 +327,16 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
       t0 = sp.tok0 + (slot - sp.c0) * KC;
       n_live = min(sp.tok_end - t0, KC);
       ci = (int64_t)h * p.nc_total + slot;
-      streamed = (int64_t)(slot - sp.c0) * 1024 >= (int64_t)sp.nc * p.cached;
     } else {
       t0 = blockIdx.z * p.T + slot * KC;
       n_live = min((int)(blockIdx.z + 1) * p.T - t0, KC);
       ci = (int64_t)h * p.nc_total + blockIdx.z * p.NC + slot;
-      streamed = (int64_t)slot * 1024 >= (int64_t)p.NC * p.cached;
     }
   }
   const bool edge = n_live < KC || p.Dk < KD;     // rows or channels that do not exist: read as copies of others, then zeroed
   const uint32_t row_stride = (uint32_t)p.H * (uint32_t)p.Dk;         // elements between token rows of one head (q, k, g)
   const int64_t tok_base = ((int64_t)t0 * p.H + h) * p.Dk;
-  const BlockOut<CACHED> block(p.blobs + ci * Blob::kBytes, Blob::kBytes, streamed);
+  const BlockOut<STREAMED> block(p.blobs + ci * Blob::kBytes, Blob::kBytes);
 
   // ---- every global load goes out at once: g as left operand, k and q rows into the LDS (swizzled), beta ----
   // g: tile t of group m holds channels 32 m + 8 (row / 4) + 2 (row % 4) + t, so that a lane's two tiles are neighbours and the
@@ -1121,29 +1116,30 @@ extern "C" size_t daisy_kda_varlen_workspace_bytes(int T, int n_seq, int H, int 
   return kda_chunk_slots(1, T, n_seq) * H * kBlobBytes + kda_table_bytes(T, n_seq);
 }
 
-// Blocks of up to kCachedBytes are stored through the caches (the last level holds 256 MB), where the second kernel finds them.  Both
+// Blocks of up to this many bytes are stored through the caches (the last level holds 256 MB), where the second kernel finds them.  Both
 // kernels, past / through them: 21 MB (T = 8192, 4 heads of 64) 155 / 114 us, 81 MB (T = 6016, 12 heads of 128) 168 / 158, 126 MB (T = 8192,
-// 24 heads of 64) 198 / 143; 148 MB (T = 8192, 16 heads of 128) 242 / 217, (4 x 2048) 119 / 109; 168 MB (4 x 8192, 8 heads of 64) 221 / 154, (2 x 16384)
-// 369 / 253; 173 MB (4 x 2400, 16 heads of 128) 132 / 133; 204 MB (8 x 1400) 157 / 162; 296 MB (T = 16384) 474 / 502.
-// Up to kPartlyCachedBytes the first blocks of every sequence are, as many as kCachedPart bytes hold: 181 MB (T = 10000, 16 heads of 128) 290 -> 264 us,
-// 206 MB (8 x 5000, 8 heads of 64) 177.6 -> 171, 226 MB (T = 12500, 16 of 128) 361 -> 355.6, 231 MB (8 x 1600) 176 -> 174; 252 MB (4 x 8192, 12 of 64)
-// 244 -> 245.5, 296 MB (4 x 4096, 16 of 128) 229 -> 232.
-constexpr int64_t kCachedBytes = (int64_t)170 << 20, kPartlyCachedBytes = (int64_t)240 << 20, kCachedPart = (int64_t)128 << 20;
+// 24 heads of 64) 198 / 143; 296 MB (T = 8192, 32 heads of 128) 310 / 333.
+// *Tried:* 170 MB, and up to 240 MB the first 128 of every sequence's: with the same inputs in every call 3 to 30 % faster, with others in every call,
+// which pass through the same caches, 4 x 2048 rows, 16 heads of 128 124.6 -> 127.7, 10104 in 4 sequences, 12 heads 134.7 -> 138.5, 15500 in 6, 16 of 64 by 128
+// 168 -> 176, against 2 x 7500, 8 heads of 128 260 -> 252.
+constexpr int64_t kCachedBytes = (int64_t)128 << 20;
 
 template <int KD>
-static int kda_launch_width(KdaParams p, int n_streams, hipStream_t s) {
+static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
   const int groups = (p.Dv + KVS * KCT - 1) / (KVS * KCT);
   const dim3 chunks(p.NC, p.H, p.n_seq > 0 ? 1 : p.B);
   const int64_t bytes = (int64_t)p.H * p.nc_total * KdaBlob<KD>::kBytes;
-  p.cached = bytes <= kPartlyCachedBytes ? (int)(kCachedPart * 1024 / bytes) : 0;
-  // fp32 log-decays beyond 400 MB: 6 KB more of LDS than the kernel uses, five workgroups per compute unit.  Where memory is the bound a sixth
-  // only adds requests.  16 heads of 128, T = 8192, B = 3 / 4 / 6, both kernels, six workgroups -> five: mild fp32 log-decays 375 to 381 -> 374 to 376,
-  // 442 to 450 -> 442 to 448, 742 -> 735 us (with four the latency shows: 329 us for the first kernel, B = 4, where it takes 216); steep fp32 ones 390 -> 396, 466 ->
-  // 472, 756 -> 766.  With half the bytes to read the vector instructions are: mild bf16 ones 364 / 364, 416 / 415, 690 / 688,
-  // steep ones (a layer's first gates) 377 / 387, 450 / 468, 729 / 749, so those keep all six.
-  const bool memory_bound = KD == 128 && !p.g_bf16 && bytes > (int64_t)400 << 20;
-  if (bytes <= kCachedBytes) hipLaunchKernelGGL((kda_prep_kernel<KD, true>), chunks, dim3(128), 0, s, p);
-  else hipLaunchKernelGGL((kda_prep_kernel<KD, false>), chunks, dim3(128), memory_bound ? 6144 : 0, s, p);
+  if (bytes > kCachedBytes) {
+    // fp32 log-decays beyond 400 MB: 6 KB more of LDS than the kernel uses, five workgroups per compute unit.  Where memory is the bound a sixth
+    // only adds requests.  16 heads of 128, T = 8192, B = 3 / 4 / 6, both kernels, six workgroups -> five: mild fp32 log-decays 375 to 381 -> 374 to 376,
+    // 442 to 450 -> 442 to 448, 742 -> 735 us (with four the latency shows: 329 us for the first kernel, B = 4, where it takes 216); steep fp32 ones 390 -> 396, 466 ->
+    // 472, 756 -> 766.  With half the bytes to read the vector instructions are: mild bf16 ones 364 / 364, 416 / 415, 690 / 688,
+    // steep ones (a layer's first gates) 377 / 387, 450 / 468, 729 / 749, so those keep all six.
+    const bool memory_bound = KD == 128 && !p.g_bf16 && bytes > (int64_t)400 << 20;
+    hipLaunchKernelGGL((kda_prep_kernel<KD, true>), chunks, dim3(128), memory_bound ? 6144 : 0, s, p);
+  } else {
+    hipLaunchKernelGGL((kda_prep_kernel<KD, false>), chunks, dim3(128), 0, s, p);
+  }
   DAISY_CHECK_LAUNCH("kda_prep_kernel");
   const unsigned chains = (unsigned)((n_streams * p.H + 7) / 8 * 8 * groups);
   // A chain fills a compute unit: where there are more than 256, a long sequence that starts late ends alone.  Longest first, cut at random places, both
