@@ -4,6 +4,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 from torch import Tensor
+from torch.nn import Parameter
 
 from . import _lib
 
@@ -16,10 +17,12 @@ def norm(x: Tensor) -> Tensor:
     CPU and on the GPU -- not ``finfo(x.dtype).eps`` (see ``NORM_EPS_BF16`` below).  The few bf16 rows of a
     decode step take this package's kernel (same arithmetic, another order of the sum), everything else the library's.
     """
-    if x.is_cuda and x.dtype is torch.bfloat16 and not torch.compiler.is_compiling():
-        y = _lib.native().norm(x, NORM_EPS_BF16)
-        if y is not None:
-            return y
+    # A stand-in of a symbolic trace and a tensor subclass have no device or dtype to ask for here, a script cannot call the extension.
+    if not torch.jit.is_scripting():
+        if type(x) in (Tensor, Parameter) and x.is_cuda and x.dtype is torch.bfloat16 and not torch.compiler.is_compiling():
+            y = _lib.native().norm(x, NORM_EPS_BF16)
+            if y is not None:
+                return y
     return F.rms_norm(x, (x.size(-1),))
 
 

@@ -5,7 +5,7 @@ from ctypes import c_int, c_int64, c_void_p
 import pytest
 import torch
 
-from daisy_amd import CausalSelfAttention, KimiLinearSelfAttention, KVCache, WindowMask, _lib
+from daisy_amd import CausalSelfAttention, KimiLinearSelfAttention, KVCache, WindowMask, _lib, norm
 
 
 class _Recorder:
@@ -155,3 +155,18 @@ def test_narrow_products_in_one_tile_across(M, K, widths):
     widths = (128, 128, 40)
     w = [torch.zeros(n, K, dtype=torch.bfloat16, device="cuda") for n in widths]
     assert call(12)[0] == -2
+
+
+class _Normed(torch.nn.Module):
+    def forward(self, x):
+        return norm(x)
+
+
+@pytest.mark.parametrize("record", [torch.fx.symbolic_trace, torch.jit.script], ids=["symbolic_trace", "script"])
+@pytest.mark.parametrize("of", ["function", "module"])
+def test_norm_is_recorded_as_the_librarys_call(record, of):
+    """A stand-in for a tensor has no device and no dtype to ask for, and a script no extension to call."""
+    recorded = record(norm if of == "function" else _Normed())
+    assert "rms_norm" in str(getattr(recorded, "inlined_graph", recorded.graph))
+    for x in (torch.randn(3, 24), torch.randn(2, 1, 40).bfloat16()):
+        assert torch.equal(recorded(x), torch.nn.functional.rms_norm(x, (x.size(-1),)))
