@@ -133,6 +133,7 @@ struct ConvPart {
 };
 // The KDA layer's low-rank products, x [M, K] w [N, K]^T with K = 64 or 128, a value head's width: through the decay gate into y [M, N],
 // with beta; or as the gate of the gated RMS norm over the N / K heads of o [M, N], in place (bias [N] or NULL, norm_weight [K]).
+int low_rank_walkers(int M, int groups);       // their workgroups per group of columns
 bool low_rank_wanted(int M, int N, int K);     // whether they are the better choice than proj_segments and gated_rmsnorm_kernel
 int low_rank_gate(const uint16_t* x, int64_t x_sm, const uint16_t* w, const KdaGates& gates, uint16_t* y, int M, int N, int K, hipStream_t s);
 int low_rank_norm(const uint16_t* x, int64_t x_sm, const uint16_t* w, const uint16_t* bias, const uint16_t* norm_weight, uint16_t* o, float eps,

@@ -410,13 +410,16 @@ __global__ __launch_bounds__(64 * kLowRankWaves, 3) void low_rank_kernel(LowRank
   }
 }
 
-// Three workgroups fit a compute unit; every wavefront walks the rows as often as that takes.
+// Workgroups per group of columns.  Three workgroups fit a compute unit; every wavefront walks the rows as often as that takes.  Whole
+// eights, one per XCD, and never none: a layer of more than 768 heads has more groups than fit.
+int low_rank_walkers(int M, int groups) {
+  const int wanted = (M + 16 * kLowRankWaves - 1) / (16 * kLowRankWaves), fit = 768 / groups > 1 ? 768 / groups : 1;
+  return ((wanted < fit ? wanted : fit) + 7) / 8 * 8;
+}
 template <int K, int EPI>
 static int launch_low_rank(LowRankParams& p, hipStream_t s) {
   p.groups = EPI == 0 ? (p.N + 127) / 128 : p.N / K;
-  const int wanted = (p.M + 16 * kLowRankWaves - 1) / (16 * kLowRankWaves), fit = 768 / p.groups;
-  const int walkers = ((wanted < fit ? wanted : fit) + 7) / 8 * 8;
-  hipLaunchKernelGGL((low_rank_kernel<K, EPI>), dim3((unsigned)(walkers * p.groups)), dim3(64 * kLowRankWaves), 0, s, p);
+  hipLaunchKernelGGL((low_rank_kernel<K, EPI>), dim3((unsigned)(low_rank_walkers(p.M, p.groups) * p.groups)), dim3(64 * kLowRankWaves), 0, s, p);
   DAISY_CHECK_LAUNCH("low_rank_kernel");
   return DAISY_OK;
 }

@@ -170,3 +170,62 @@ def test_norm_is_recorded_as_the_librarys_call(record, of):
     assert "rms_norm" in str(getattr(recorded, "inlined_graph", recorded.graph))
     for x in (torch.randn(3, 24), torch.randn(2, 1, 40).bfloat16()):
         assert torch.equal(recorded(x), torch.nn.functional.rms_norm(x, (x.size(-1),)))
+
+
+@pytest.mark.parametrize("groups", [1, 2, 5, 8, 10, 16, 40, 95, 96, 97, 768, 769, 800, 4000])
+def test_low_rank_products_always_have_workgroups(groups):
+    """Whole eights, one per XCD; of more groups of columns than fit the chip too."""
+    fn = _lib.load()._ZN5daisy16low_rank_walkersEii
+    for M in (1, 64, 65, 1000, 40000):
+        walkers = fn(M, groups)
+        assert walkers >= 8 and walkers % 8 == 0 and walkers * groups * 256 < 2 ** 31
+        assert walkers <= (M + 511) // 512 * 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,H,Dk", [(1, 64, 3, 64), (15, 128, 2, 128), (16, 64, 16, 40), (17, 128, 5, 8), (129, 64, 4, 128), (70, 64, 800, 128),
+                                      (2100, 128, 10, 64)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_low_rank_products_with_what_follows_them(M, K, H, Dk, bias):
+    """The decay gate with beta, and the gated norm: rows that end inside a block of 16, columns inside a group of 128, more groups of columns
+    than workgroups fit the chip.  Against 64 bits: one rounding of the product to bf16, one of the result; nothing behind the rows is written."""
+    lib = _lib.load()
+    gate = lib._ZN5daisy13low_rank_gateEPKtlS1_RKNS_8KdaGatesEPtiiiP12ihipStream_t
+    gate.argtypes = [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]
+    norm_of = lib._ZN5daisy13low_rank_normEPKtlS1_S1_S1_PtfiiiP12ihipStream_t
+    norm_of.argtypes = [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_float, c_int, c_int, c_int, c_void_p]
+    g = torch.Generator(device="cuda").manual_seed(M + H)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+
+    # (u: half the spacing of bf16 numbers, 7 bits behind the first)
+    stream, u, x = torch.cuda.current_stream().cuda_stream, 2.0 ** -8, rnd(M, K + 16).bfloat16()
+
+    def product(w, b):                                       # in 64 bits, and how far its bf16 value may be from it
+        z, size = x[:, :K].double() @ w.double().T + b, x[:, :K].double().abs() @ w.double().abs().T + abs(b)
+        return z, u * z.abs() + K * 2.0 ** -24 * size
+
+    w, logits = (rnd(H * Dk, K) / K ** 0.5).bfloat16(), rnd(M, (H + 7) // 8 * 8).bfloat16()
+    A_log, dt_bias, beta = rnd(H), rnd(H * Dk), torch.full((M + 1, H), 7.0, device="cuda")
+    y = torch.full((M + 1, H * Dk), 7.0, device="cuda").bfloat16()
+    gates = _Gates(A_log.data_ptr(), dt_bias.data_ptr(), H, Dk, logits.data_ptr(), logits.shape[1], beta.data_ptr())
+    assert gate(x.data_ptr(), K + 16, w.data_ptr(), ctypes.addressof(gates), y.data_ptr(), M, H * Dk, K, stream) == 0, lib.daisy_last_error()
+    z, dz = product(w, 0.0)
+    scale = A_log.double().exp().repeat_interleave(Dk)
+    ref = -scale * torch.nn.functional.softplus(z + dt_bias.double())
+    assert ((y[:M] - ref).abs() - (scale * dz + (u + 1e-5) * ref.abs()) * 1.01).max() <= 0   # (the gate's slope is at most its scale)
+    ref = logits[:, :H].double().sigmoid()
+    assert ((beta[:M] - ref).abs() - (u + 1e-5) * ref).max() <= 0
+    assert (y[M] == 7).all() and (beta[M] == 7).all()
+
+    w, weight, b = (rnd(H * K, K) / K ** 0.5).bfloat16(), rnd(K).bfloat16(), rnd(H * K).bfloat16() if bias else None
+    o = torch.full((M + 1, H * K), 7.0, device="cuda").bfloat16()
+    o[:M] = rnd(M, H * K)
+    before = o[:M].double().view(M, H, K)
+    assert norm_of(x.data_ptr(), K + 16, w.data_ptr(), b.data_ptr() if bias else None, weight.data_ptr(), o.data_ptr(), 1e-5, M, H * K, K, stream) == 0
+    z, dz = product(w, b.double() if bias else 0.0)
+    rows = (before * (before.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt() * weight.double()).view(M, H * K)
+    ref = rows * z.sigmoid()
+    assert ((o[:M] - ref).abs() - (rows.abs() * dz / 4 + (u + 1e-5) * ref.abs()) * 1.01).max() <= 0   # (the sigmoid's slope is at most 1 / 4)
+    assert (o[M] == 7).all()
