@@ -182,6 +182,16 @@ def test_low_rank_products_always_have_workgroups(groups):
         assert walkers <= (M + 511) // 512 * 8
 
 
+def test_low_rank_products_walk_in_one_round():
+    """Heads whose number does not divide 96: of 768 places no more workgroups than fit, where that fills five sixths of them."""
+    fn = _lib.load()._ZN5daisy16low_rank_walkersEii
+    for groups in range(1, 97):
+        whole = 768 // groups // 8 * 8
+        walkers = fn(1 << 20, groups)
+        assert walkers == whole if whole * groups > 640 else whole <= walkers <= whole + 8
+    assert [fn(40000, n) * n for n in (5, 7, 8, 10, 14, 16)] == [760, 728, 768, 720, 672, 768]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,H,Dk", [(1, 64, 3, 64), (15, 128, 2, 128), (16, 64, 16, 40), (17, 128, 5, 8), (129, 64, 4, 128), (70, 64, 800, 128),
                                       (2100, 128, 10, 64)])
