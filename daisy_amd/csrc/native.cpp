@@ -180,7 +180,7 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// norm(x, eps): the weightless RMS norm over the last dim of contiguous bf16 rows, or None.
+// norm(x, eps): the weightless RMS norm over the last dim of contiguous bf16 rows, one token per sequence ([.., 1, C]), or None.
 PyObject* py_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 2 || intercepted() || !is_tensor(a[0])) return none();
@@ -188,7 +188,7 @@ PyObject* py_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const float eps = (float)PyFloat_AsDouble(a[1]);
   if (PyErr_Occurred()) { PyErr_Clear(); return none(); }
   const int dev = gpu_of(x);
-  if (dev < 0 || !bf16(x) || x.dim() < 1 || !x.is_contiguous() || x.numel() == 0 || needs_autograd({&x})) return none();
+  if (dev < 0 || !bf16(x) || x.dim() < 2 || x.size(-2) != 1 || !x.is_contiguous() || x.numel() == 0 || needs_autograd({&x})) return none();
   const int64_t C = x.size(-1), rows = x.numel() / C;
   if (!daisy::rms_rows_serves(rows, C) || (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) != 0) return none();
   Unlocked unlocked;

@@ -187,10 +187,11 @@ int prep_launch(const void* q, const int64_t* q_strides, const void* k, const in
 // y = x * rsqrt(mean(x^2) + eps) over rows of C bf16, one rounding at the end: the norms in front of the layers of a model.  In a decode step
 // a launch is its arguments, one memory round trip and the sum, so a workgroup takes a row, every thread one piece of 16 bytes that it keeps for
 // the second use, and the wavefronts' sums meet in the LDS behind the only barrier.  Against the library's kernel in a recorded chain of them:
-// 1 row of 1536 2.76 -> 1.80 us, 16 rows 3.03 -> 2.00, 1 row of 8192 5.16 -> 2.04; from Python 6.9 -> 4.3 us a call.
-// Prompts stay with the library, although this kernel would be ahead there too (256 rows of 1536 3.1 and 2.1 us, 32768 of 1024 34 and 20): the order
-// of the sum is another one, so that some ten elements in a million come out one bf16 step away, and a prompt's rows stay in caches.
-constexpr int64_t kNormRows = 32;
+// 1 row of 1536 2.81 -> 2.00 us, 32 rows 3.23 -> 2.19, 1 row of 8192 5.26 -> 2.18; from Python 6.9 -> 4.3 us a call.
+// For one token per sequence, of any number of sequences (64 rows of 1536 3.24 -> 2.2 us): its caller looks at the shape.  Prompts stay with the
+// library, although this kernel would be ahead there too (2048 rows of 1536 5.20 and 3.54 us, 32768 66.7 and 36.1): the order of the sum is another one,
+// three elements in a million come out one bf16 step away (the error against 64 bits is the same to 8 digits), and a prompt's row
+// is then the same whatever the number of tokens.
 constexpr int kNormThreads = 1024;
 __global__ __launch_bounds__(kNormThreads) void rms_row_kernel(const uint16_t* x, uint16_t* y, int C, float eps) {
   __shared__ float part[kNormThreads / 64];
@@ -212,11 +213,15 @@ __global__ __launch_bounds__(kNormThreads) void rms_row_kernel(const uint16_t* x
   if (live) *reinterpret_cast<u32x4*>(y + at) = pack8(f);
 }
 
-bool rms_rows_serves(int64_t rows, int64_t C) { return rows >= 1 && rows <= kNormRows && C >= 8 && C % 8 == 0 && C <= 8 * kNormThreads; }
+static int rms_threads(int64_t C) { return (int)((C / 8 + 63) / 64 * 64); }
+// (fewer than 2^31 threads: 33 million rows of 512)
+bool rms_rows_serves(int64_t rows, int64_t C) {
+  return rows >= 1 && C >= 8 && C % 8 == 0 && C <= 8 * kNormThreads && rows < ((int64_t)1 << 31) / rms_threads(C);
+}
 int rms_rows(const uint16_t* x, uint16_t* y, int rows, int C, float eps, hipStream_t s) {
   DAISY_CHECK_ARG(x && y && rms_rows_serves(rows, C) && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0,
                   "rms_rows: %d rows of %d on 16-byte boundaries", rows, C);
-  hipLaunchKernelGGL(rms_row_kernel, dim3((unsigned)rows), dim3((unsigned)((C / 8 + 63) / 64 * 64)), 0, s, x, y, C, eps);
+  hipLaunchKernelGGL(rms_row_kernel, dim3((unsigned)rows), dim3((unsigned)rms_threads(C)), 0, s, x, y, C, eps);
   DAISY_CHECK_LAUNCH("rms_row_kernel");
   return DAISY_OK;
 }

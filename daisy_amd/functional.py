@@ -14,8 +14,10 @@ def norm(x: Tensor) -> Tensor:
 
     Same call as the reference's ``norm`` (models/daisy/functional.py:6-7): no eps is passed, and torch 2.10
     then adds the machine epsilon of its accumulation type -- fp32's for bf16 and fp32 inputs alike, on the
-    CPU and on the GPU -- not ``finfo(x.dtype).eps`` (see ``NORM_EPS_BF16`` below).  The few bf16 rows of a
-    decode step take this package's kernel (same arithmetic, another order of the sum), everything else the library's.
+    CPU and on the GPU -- not ``finfo(x.dtype).eps`` (see ``NORM_EPS_BF16`` below).  The bf16 rows of a
+    decode step, one token per sequence (``[B, 1, C]``), take this package's kernel: same arithmetic, another order of
+    the sum, so that a few elements in a million are one bf16 step away.  Everything else is the library's, prompts of
+    any length among it.
     """
     # A stand-in of a symbolic trace and a tensor subclass have no device or dtype to ask for here, a script cannot call the extension.
     if not torch.jit.is_scripting():

@@ -139,6 +139,28 @@ def test_norm_rows(shape):
     assert ((got.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() * 1.001).all()
 
 
+def test_norm_of_a_prompt_is_the_librarys_whatever_its_length():
+    """Few rows are no decode step: the order of the sum, hence here and there a bf16 step, would depend on the number of tokens."""
+    from daisy_amd import norm
+    g = torch.Generator(device="cuda").manual_seed(5)
+    for shape in [(1, 32, 1536), (16, 2, 1536), (1, 2, 16, 1024), (32, 1536), (1, 33, 1536)]:
+        for _ in range(100):
+            x = torch.randn(shape, generator=g, device="cuda").bfloat16()
+            assert torch.equal(norm(x), torch.nn.functional.rms_norm(x, (x.size(-1),))), shape
+
+
+@pytest.mark.parametrize("C", [64, 520, 1536, 8192])
+def test_norm_of_a_decode_step_does_not_depend_on_the_batch(C):
+    from daisy_amd import norm
+    x = torch.randn(2000, 1, C, generator=torch.Generator(device="cuda").manual_seed(C), device="cuda").bfloat16()
+    whole = norm(x)
+    assert whole.shape == x.shape
+    ref = x.double() * (x.double().pow(2).mean(-1, keepdim=True) + NORM_EPS_BF16).rsqrt()
+    assert ((whole - ref).abs() - 2.0 ** -8 * ref.abs() * 1.001).max() <= 0
+    for n in (1, 32, 33, 64):
+        assert all(torch.equal(norm(x[at:at + n]), whole[at:at + n]) for at in range(0, 2000, n))
+
+
 def test_norm_leaves_to_the_library_what_it_does_not_take():
     from daisy_amd import norm
     lib = lambda t: torch.nn.functional.rms_norm(t, (t.size(-1),))
