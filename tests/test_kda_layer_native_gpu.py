@@ -9,10 +9,10 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def _layer(H, D, expand_v, taps, conv_bias):
+def _layer(H, D, expand_v, taps, conv_bias, dim=None):
     torch.manual_seed(H * D + taps)
     with torch.device(DEV):
-        m = KimiLinearSelfAttention(H * D, H, max_seq_len=1024, head_dim=D, expand_v=expand_v, conv_size=taps, conv_bias=conv_bias)
+        m = KimiLinearSelfAttention(dim or H * D, H, max_seq_len=1024, head_dim=D, expand_v=expand_v, conv_size=taps, conv_bias=conv_bias)
     with torch.no_grad():
         m.dt_bias.normal_()
         m.g_proj[1].bias.normal_(std=0.3)
@@ -142,15 +142,19 @@ def test_a_call_that_is_given_back_has_not_touched_the_states(what):
         assert torch.equal(t, b)
 
 
-@pytest.mark.parametrize("B,T,H,D,expand_v", [(1, 4099, 16, 64, 1.0), (2, 2061, 8, 128, 1.0), (1, 6251, 16, 40, 1.6), (1, 16385, 2, 128, 1.0)])
-def test_long_rows_take_the_low_rank_kernels(B, T, H, D, expand_v, monkeypatch):
+@pytest.mark.parametrize("B,T,H,D,expand_v,dim", [(1, 4099, 16, 64, 1.0, 1024), (2, 2061, 8, 128, 1.0, 1024), (1, 6251, 16, 40, 1.6, 640),
+                                                  (1, 16385, 2, 128, 1.0, 256), (1, 81, 800, 64, 1.0, 64)])
+def test_long_rows_take_the_low_rank_kernels(B, T, H, D, expand_v, dim, monkeypatch):
     """Rows that are no multiple of the 16 of a block, 640 columns (no multiple of 128) for the decay gate, fewer columns than an XCD has
-    workgroups; against the layer's own path, which makes the products as tiles and the norm by itself."""
-    m = _layer(H, D, expand_v, 4, False)
-    assert B * T * H * D >= 4000000
-    x = torch.randn(B, T, H * D, generator=torch.Generator(device=DEV).manual_seed(T), device=DEV).bfloat16()
+    workgroups, more heads than workgroups fit the chip; against the layer's own path, which makes the products as tiles and the norm by itself."""
+    m = _layer(H, D, expand_v, 4, False, dim)
+    assert _lib.load()._ZN5daisy15low_rank_wantedEiii(B * T, H * D, m.head_v_dim) & 1
+    x = torch.randn(B, T, dim, generator=torch.Generator(device=DEV).manual_seed(T), device=DEV).bfloat16()
+    whole, taken = KimiLinearSelfAttention._fast, []
     with torch.no_grad():
+        monkeypatch.setattr(KimiLinearSelfAttention, "_fast", lambda self, *a: taken.append(whole(self, *a)) or taken[-1])
         got = [m.prefill(x, None)[0]] + [t.clone() for t in m.state_tensors()]
+        assert len(taken) == 1 and taken[0] is not None, "the one-call path gave the call back"
         m.reset_history()
         monkeypatch.setattr(KimiLinearSelfAttention, "_fast", lambda self, *a: None)
         ref = [m.prefill(x, None)[0]] + [t.clone() for t in m.state_tensors()]

@@ -126,17 +126,23 @@ def test_prep_rejects_bad_arguments():
         ops.qkv_prep(q, q, q, eps=1e-7, cos=cos, sin=cos)
 
 
-@pytest.mark.parametrize("shape", [(1, 8), (3, 64), (1, 1, 72), (2, 5, 512), (1, 1, 1536), (32, 520), (33, 520), (2, 8192), (1, 8200)])
-def test_norm_rows(shape):
-    """Rows of one thread to rows of all of them, with idle threads in the last wavefront; longer ones and more go to the library."""
+@pytest.mark.parametrize("rows,C", [(1, 8), (3, 64), (1, 72), (10, 512), (7, 520), (1, 1024), (33, 1536), (5, 2056), (2, 8192), (1, 8200)])
+def test_norm_rows(rows, C):
+    """Rows of one thread to rows of all of them, with idle threads in the last wavefront; longer ones go to the library.  Ordinary values, and
+    rows whose sum of squares is one element's, at either end of every wavefront's 512 and of the row: whatever is left out of the
+    sum, or in it twice, is the result's error."""
     from daisy_amd import norm
-    x = (torch.randn(shape, generator=torch.Generator().manual_seed(shape[-1])) * 3).bfloat16()
-    x[..., 0] = 1e18                                  # squares beyond bf16's exactness, not beyond fp32
-    ref = x.double() * (x.double().pow(2).mean(-1, keepdim=True) + NORM_EPS_BF16).rsqrt()
-    got = norm(x.cuda())
-    assert got.dtype == torch.bfloat16 and got.is_contiguous()
-    # one rounding to bf16 of a value known to fp32's precision
-    assert ((got.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() * 1.001).all()
+    g = torch.Generator().manual_seed(C)
+    last = (C - 1) // 512 * 512
+    for at in [None] + sorted({0, 7, C - 1, last} | {i for w in range(0, C, 512) for i in (w, min(w + 511, C - 1))}):
+        x = torch.randn(rows, 1, C, generator=g).mul(3 if at is None else 2.0 ** -10).bfloat16()
+        if at is not None:
+            x[..., at] = 1e18 if at == 7 else 40.0            # (1e18: squares beyond bf16's exactness, not beyond fp32)
+        ref = x.double() * (x.double().pow(2).mean(-1, keepdim=True) + NORM_EPS_BF16).rsqrt()
+        got = norm(x.cuda())
+        assert got.dtype == torch.bfloat16 and got.is_contiguous()
+        # one rounding to bf16 of a value known to fp32's precision
+        assert ((got.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() * 1.001).all(), at
 
 
 def test_norm_of_a_prompt_is_the_librarys_whatever_its_length():
@@ -164,15 +170,15 @@ def test_norm_of_a_decode_step_does_not_depend_on_the_batch(C):
 def test_norm_leaves_to_the_library_what_it_does_not_take():
     from daisy_amd import norm
     lib = lambda t: torch.nn.functional.rms_norm(t, (t.size(-1),))
-    x = torch.randn(4, 96, device="cuda").bfloat16()
-    for t in (x.float(), x[:, 1:65], x.t(), x.view(-1)[1:97], x.half(), x[:, :7].contiguous()):
+    x = torch.randn(4, 1, 96, generator=torch.Generator(device="cuda").manual_seed(4), device="cuda").bfloat16()
+    for t in (x.float(), x[..., 1:65], x.transpose(0, 2), x.view(-1)[1:97].view(1, 1, 96), x.half(), x[..., :7].contiguous(), x[0, 0]):
         assert torch.equal(norm(t), lib(t))
     bad = x.clone()
-    bad[1, 3], bad[2, 5] = float("nan"), float("inf")
-    assert torch.equal(norm(bad).isnan(), lib(bad).isnan()) and torch.equal(norm(bad)[0], lib(bad)[0])
+    bad[1, 0, 3], bad[2, 0, 5] = float("nan"), float("inf")
+    assert torch.equal(norm(bad).isnan(), lib(bad).isnan()) and torch.equal(norm(bad)[0], norm(x)[0])
     w = x.clone().requires_grad_()
     norm(w).sum().backward()
     assert w.grad is not None
-    assert norm(torch.empty(0, 64, device="cuda", dtype=torch.bfloat16)).shape == (0, 64)
+    assert norm(torch.empty(0, 1, 64, device="cuda", dtype=torch.bfloat16)).shape == (0, 1, 64)
     out = torch.func.vmap(norm)(x)
     assert torch.equal(out, lib(x))
