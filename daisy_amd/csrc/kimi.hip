@@ -430,6 +430,9 @@ static int launch_low_rank(LowRankParams& p, hipStream_t s) {
 // From about four million outputs on.  Below, a workgroup's own latencies (its columns into the LDS, a block or two, beta) are what the call waits
 // for, and tiles have fewer of them: a layer's call, tiles and the gated norm / these kernels, 64 rows of 8 heads of 128 41.5 / 47.8 us, 200 of 16
 // 62 / 67, 777 of 12 89.5 / 91.5, 2048 of 16 175 / 175, 8000 of 8 222 / 218, 32768 of 8 of 64 420 / 404, 40000 of 16 of 128 2190 / 2120.
+// Asked of the gate's outputs for both kernels, also where values are wider or narrower than keys: from four million on the pair is ahead of tiles and norm
+// at every ratio (in a recorded chain, 16 heads, keys by values: 128 by 64, 2001 rows 16.8 / 13.9, 64 by 128, 4003 rows 27.1 / 23.6, 256 by 64, 1000 rows
+// 14.3 / 12.0), and one of them with tiles for the other is a launch more than either (17.8, 31.2, 15.6 with the gate's own kernel).
 bool low_rank_wanted(int M, int N, int K) { return (K == 64 || K == 128) && (int64_t)M * N >= 4000000; }
 static int low_rank_check(const LowRankParams& p, int K) {
   auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };

@@ -878,7 +878,7 @@ static int64_t split_limit(const PrefillParams& p) {
 }
 
 // When those are eight wavefronts: while a compute unit has no second workgroup to run and the longest block has more key tiles than four of them
-// take in two turns (us, four / eight; heads of 128, no window: 12 heads x 384 rows 7.0 / 6.6, 8 x 1024 11.3 / 10.1, 4 x 2048 18.3 / 14.9, 2 x 4096 31 / 23;
+// take in two turns, in one where a window makes most blocks as long as the longest (us, four / eight; heads of 128, no window: 12 heads x 384 rows 7.0 / 6.6, 8 x 1024 11.3 / 10.1, 4 x 2048 18.3 / 14.9, 2 x 4096 31 / 23;
 // window 1024, 4 x 2048 12.7 / 10.3; 256, 8 x 1024 7.5 / 7.0; 128, 32 x 256 6.6 / 6.1; heads of 64, 4 x 2048 13.3 / 10.1; 128 rows 5.0 / 5.2, 256 5.9 / 6.0;
 // window 1024, 6 x 2048 14.0 / 16.7).  Causal blocks differ in length, so that long ones gain with twice the workgroups too (heads of 64, 16 x 1024 8.9 /
 // 8.8, 8 x 2048 13.8 / 12.2; of 128, 12 x 1024 12.4 / 12.9, 8 x 1536 15.8 / 13.9, 4 x 4096 35 / 30).  Documents' lengths are not known here.

@@ -557,7 +557,9 @@ int proj_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s, in
   };
   // All products in one tile across (code 12): the same rows of x, no bias, together at most a tile wide.  By cost, which is a round of its
   // workgroups (30 at K = 2048, as proj_tile counts); 128 + 128 + 16 columns, the best other tile / this one: K = 2048 and 20000 rows 31.5 / 34.8,
-  // 22000 48.5 / 35.5, 40000 59.3 / 68.1, 45000 75.5 / 69.1, 131072 224 / 183 us; K = 1024, 24000 rows 26.2 / 22.6, 65536 50.8 / 46.7.  Of
+  // 22000 48.5 / 35.5, 40000 59.3 / 68.1, 45000 75.5 / 69.1, 131072 224 / 183 us; K = 1024, 24000 rows 26.2 / 22.6, 65536 50.8 / 46.7: ahead where
+  // the others need another round, from some 21000 rows to 32768 and again from some 45000, level between, where they are taken.  Narrower ones alike (K = 2048,
+  // 24000 rows, 64 + 64 + 16 columns 41.8 / 34.9, a lone product of 280 46.1 / 34.9; of 128 or 256 the others are never dearer and are taken).  Of
   // short rows the fixed part of a round is too much: K = 512, 32768 rows 19.6 / 17.1, but 45000 26.3 / 28.2; K = 256, 131072 37.5 / 44.9.
   int across = 0;
   bool joined = !gates && ((!tile && K >= 1024) || tile == 12);
