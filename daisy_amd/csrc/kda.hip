@@ -1,6 +1,7 @@
 // Kernel 3: chunked Kimi Delta Attention forward and its log-decay gate (gfx950).
 #include "common.h"
 #include <type_traits>
+#include <utility>
 
 namespace daisy {
 
@@ -59,7 +60,7 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 // Chunked forward.  Per (batch, head), chunk of C = 32 positions.  The kernels work on KD = 64 or 128 key
 // channels; a smaller Dk (a multiple of 8) is served by reading the missing channels as zeros (zero channels of q, k
 // and g change nothing: they add nothing to any dot product or norm, and their state rows stay zero), and value
-// columns are independent of each other, so any Dv (a multiple of 8) is served in groups of 32.
+// columns are independent of each other, so any Dv (a multiple of 8) is served in groups of 32 or 64.
 //
 // With G_i the inclusive running sum of the log-decay g inside the chunk (per channel), S0 the state at the chunk
 // start, and (per channel products written with (.)):
@@ -71,14 +72,14 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 //   S' = diag(exp(G_last)) S0 + ((exp(G_last - G) (.) K)^T T) X
 //
 // kda_prep_kernel (all chunks in parallel) produces everything that depends on neither S0 nor V, one block of
-// KdaBlob<KD>::kBytes per chunk, laid out as the other kernel wants it in LDS:
+// KdaBlob<KD>::kBytes per chunk, whose KiB are operands as the lanes of the other kernel hold them (piece i of 16 bytes is lane i's):
 //   Kg  = -exp(G) (.) K             bf16 [32][KD]
 //   Qg  = scale exp(G) (.) Q        bf16 [32][KD]
 //   Mh + Ml = (exp(G_last - G) (.) K)^T T split into two bf16 terms, [KD][32]: rows in the order of the state's tiles, columns
 //                                   (positions) permuted
 //   Ph + Pl = scale tril(P) T       the same, [32][32], columns permuted
 //   dec = exp(G_last)               fp32 [KD]
-// kda_state_kernel (one workgroup per (batch, head, 32 value columns)) then walks the chunks in order with the fp32
+// kda_state_kernel (one workgroup per (batch, head, 32 or 64 value columns)) then walks the chunks in order with the fp32
 // state in registers; every product in it is a v_mfma_f32_16x16x32_bf16 whose B operand is an accumulator (S0 or X)
 // converted to bf16 in place: in the 16x16 accumulator layout lane l holds column l%16 and rows 4*(l/16)+r of each
 // tile, so two stacked tiles give the lane 8 contraction indices, (t, r) with t = 0,1; r = 0..3.  The state's tiles 2 m and 2 m + 1
@@ -86,11 +87,11 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 // are; X's tiles hold positions 16 t + 4 (row/4) + row%4, and M and P are stored with their columns permuted to match.
 //
 // What bounds it.  Of the first kernel, at B4 T8192 H16 with fp32 log-decays, memory: 1.29 GB (673 MB of inputs, 612 MB of blocks) in
-// 216 us (208 at the fastest); otherwise its vector instructions and their latency.  The second is a serial chain of chunks; what sets the time of a
+// 203 us (6.3 TB/s); otherwise its vector instructions and their latency.  The second is a serial chain of chunks; what sets the time of a
 // link is not the chain itself (without it the kernel is as fast) but its 39 KB of operands: a compute unit has about 64 KB
-// of requests in flight, 62 GB/s from memory (160 GB/s if they are in the L2).  0.55 us a link at B1 T8192 with 4 heads of
-// 128 (0.75 before the data-moving wavefronts were written as below), 0.4 us with 4 heads of 64 (0.63), 0.87 us with 64 of
-// 128 (0.89), where all compute units ask at once.
+// of requests in flight, 62 GB/s from memory (160 GB/s if they are in the L2).  0.57 us a link at T = 8192 with 4 heads of
+// 128 (0.63 before operands lay in the lanes' order and the outputs' came past the LDS), 0.39 us with 4 heads of 64, 0.67 us with 16 of 128,
+// whose blocks come from memory and not from the last-level cache (0.70), 0.88 us with 64 of 128 (0.93), where all compute units ask at once.
 //
 // Numerics: the 16x16 blocks of A and P run on MFMA with both operands referenced to the row before the block (every
 // exponent <= 0 off the diagonal); a diagonal block whose total decay exceeds exp(-80) is referenced to its middle row
@@ -104,13 +105,12 @@ constexpr int KC = 32;    // chunk length
 constexpr int KDMAX = 128;
 constexpr int KVS = 16;   // value columns per state wavefront
 
-// One chunk's block in the workspace: byte offsets of its parts (first what the chain reads, then what the outputs read);
-// rows of 16-byte pieces XOR-swizzled (below).
+// One chunk's block in the workspace: byte offsets of its parts (first what the chain reads, then what the outputs read).
 template <int KD> struct KdaBlob {
   static constexpr int kKg = 0, kMh = KC * KD * 2, kMl = 2 * KC * KD * 2, kDec = 3 * KC * KD * 2;
   static constexpr int kChain = (kDec + KD * 4 + 1023) & ~1023;      // whole 1 KiB copies
   static constexpr int kQg = kChain, kPh = kQg + KC * KD * 2, kPl = kPh + KC * KC * 2;
-  static constexpr int kBytes = kPl + KC * KC * 2, kOut = kBytes - kChain;
+  static constexpr int kBytes = kPl + KC * KC * 2;
 };
 static_assert(KdaBlob<128>::kBytes == 37 * 1024 && KdaBlob<64>::kBytes == 21 * 1024, "");
 struct KdaParams {
@@ -119,7 +119,7 @@ struct KdaParams {
   const float* s0; uint16_t* o; float* s_out;
   int B, T, H, NC; float scale; int l2norm; float l2eps;
   int Dk, Dv;     // the tensors' own widths: Dk <= KD key channels, Dv value columns
-  char* blobs;    // [H][nc_total][KdaBlob<KD>::kBytes]
+  char* blobs;    // [nc_total][H][KdaBlob<KD>::kBytes]
   // Sequences packed along the token axis of a batch of one (B == 1, T = all tokens): n_seq > 0, cu [n_seq + 1] = the
   // caller's running lengths; NC is the host's upper bound T / 32 + n_seq on the chunk slots.  Up to kScanSeqs sequences a
   // wavefront finds its way by itself (packed_span); beyond, kda_chunk_table_kernel writes bounds [n_seq + 1] = sanitised
@@ -304,7 +304,7 @@ template <int KD, bool STREAMED>
 __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   using Blob = KdaBlob<KD>;
   constexpr int NM = KD / 32, ROW = 2 * KD;                           // contraction groups of 32 channels, bytes of a bf16 row
-  // rows[0] / rows[1]: k / q as given; then Kg / Qg on their way out; then the two terms of exp(G_last - G) k.  A
+  // rows[0] / rows[1]: k / q as given; then the two terms of exp(G_last - G) k.  A
   // wavefront's 16 rows are its own until the last use.
   __shared__ __attribute__((aligned(1024))) char rows[2][KC * ROW];
   __shared__ __attribute__((aligned(16))) char kcol[16 * ROW];        // the first block's columns for block (1, 0)
@@ -313,24 +313,33 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
   __shared__ __attribute__((aligned(16))) float Ao[16][20];           // A_10, [row][column]
   __shared__ __attribute__((aligned(16))) float bt[KC], rks[KC];      // beta (0 for padded rows), 1 / |k|
 
-  const int h = blockIdx.y;
+  // 32 chunks of a head in neighbouring workgroups, then as many of the next head: what runs at a time reads and writes neighbouring memory, token
+  // rows as much as blocks, whose order in the workspace is the tokens'; and workgroups of one head, which differ in how steep their decays
+  // are, run side by side.  T = 8192, 16 heads, all chunks of a head (and of its blocks) in a row / 32 / 1: mild fp32 log-decays B = 1 62 / 57 / 57 us, 2
+  // 115 / 105 / 104, 3 168 / 151 / 152, 4 213 / 204 / 203; a layer's first gates (bf16) B = 2 121 / 116 / 132, 4 251 / 248 / 273.
+  int h, slot;
+  {
+    constexpr uint32_t kRun = 32;
+    const uint32_t run = blockIdx.x / (kRun * p.H), at = blockIdx.x % (kRun * p.H), n = min(kRun, p.NC - kRun * run);
+    h = (int)(at / n);
+    slot = (int)(kRun * run + at % n);
+  }
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, q4 = lane >> 4;
   const int I = __builtin_amdgcn_readfirstlane(tid >> 6);
   int t0, n_live;
   int64_t ci;
   {
-    const int slot = blockIdx.x;
     if (p.n_seq > 0) {
       int seq = slot, rows_end;
       const SeqSpan sp = packed_span(p, seq, true, rows_end);
       if (sp.nc == 0) return;                    // surplus slots (the grid covers the upper bound)
       t0 = sp.tok0 + (slot - sp.c0) * KC;
       n_live = min(sp.tok_end - t0, KC);
-      ci = (int64_t)h * p.nc_total + slot;
+      ci = (int64_t)slot * p.H + h;
     } else {
       t0 = blockIdx.z * p.T + slot * KC;
       n_live = min((int)(blockIdx.z + 1) * p.T - t0, KC);
-      ci = (int64_t)h * p.nc_total + blockIdx.z * p.NC + slot;
+      ci = ((int64_t)blockIdx.z * p.NC + slot) * p.H + h;
     }
   }
   const bool edge = n_live < KC || p.Dk < KD;     // rows or channels that do not exist: read as copies of others, then zeroed
@@ -591,37 +600,25 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
       P[0] *= rq * lds_f4(&rks[4 * q4]);
     }
   }
-  // ---- Kg = -exp(G) k, Qg = scale exp(G) q with G from the chunk's start: through the wavefront's rows, whole KiB out ----
-  {
-    char* const kg = &rows[0][16 * I * ROW];
-    char* const qg = &rows[1][16 * I * ROW];
+  // ---- Kg = -exp(G) k, Qg = scale exp(G) q with G from the chunk's start: as the lanes hold them, whole KiB out ----
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      if (I == 1) {
-        const f32x4 e0 = lds_f4(&Et[0][32 * m + 8 * q4]), e1 = lds_f4(&Et[0][32 * m + 8 * q4 + 4]);
+  for (int m = 0; m < NM; ++m) {
+    if (I == 1) {
+      const f32x4 e0 = lds_f4(&Et[0][32 * m + 8 * q4]), e1 = lds_f4(&Et[0][32 * m + 8 * q4 + 4]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float f = e < 4 ? e0[e & 3] : e1[e & 3];
-          kn[m][e] *= -rk * f;
-          qn[m][e] *= rq * f;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) { kn[m][e] *= -rk; qn[m][e] *= rq; }
+      for (int e = 0; e < 8; ++e) {
+        const float f = e < 4 ? e0[e & 3] : e1[e & 3];
+        kn[m][e] *= -rk * f;
+        qn[m][e] *= rq * f;
       }
-      *reinterpret_cast<u32x4*>(kg + at[m]) = pack8(kn[m]);
-      *reinterpret_cast<u32x4*>(qg + at[m]) = pack8(qn[m]);
-    }
-    wave_lds_fence();
+    } else {
 #pragma unroll
-    for (int j = 0; j < 16 * ROW / 1024; ++j) {
-      const u32x4 a = *reinterpret_cast<const u32x4*>(kg + 1024 * j + 16 * lane), b = *reinterpret_cast<const u32x4*>(qg + 1024 * j + 16 * lane);
-      block.store(a, 16 * lane, Blob::kKg + 16 * I * ROW + 1024 * j);
-      block.store(b, 16 * lane, Blob::kQg + 16 * I * ROW + 1024 * j);
+      for (int e = 0; e < 8; ++e) { kn[m][e] *= -rk; qn[m][e] *= rq; }
     }
-    wave_lds_fence();
-    if (tid < KD / 4) *reinterpret_cast<f32x4*>(block.base + Blob::kDec + 16 * tid) = lds_f4(&Et[0][4 * tid]) * lds_f4(&Et[1][4 * tid]);
+    block.store(pack8(kn[m]), 16 * lane, Blob::kKg + 1024 * (NM * I + m));
+    block.store(pack8(qn[m]), 16 * lane, Blob::kQg + 1024 * (NM * I + m));
   }
+  if (tid < KD / 4) *reinterpret_cast<f32x4*>(block.base + Blob::kDec + 16 * tid) = lds_f4(&Et[0][4 * tid]) * lds_f4(&Et[1][4 * tid]);
   // ---- exp(G_last - G) k in two bf16 terms, for the transposing reads below ----
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
@@ -700,8 +697,7 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     tl[1] = __builtin_bit_cast(bf16x8, lo);
   }
   // Row 16 tile + li of (right operand)^T T: the products come out with four consecutive columns of T per lane and column block,
-  // which is the stored piece q4 of that row; both terms of it leave from here, 16 whole rows per instruction.
-  const int t_at = li * 64 + 16 * (q4 ^ piece_swizzle<64>(li));       // (rows 16 apart share a swizzle)
+  // which is the piece the lane's place in an operand wants; both terms of it leave from here, a KiB per instruction.
   auto times_t = [&](const bf16x8& rh, const bf16x8& rl, int part_hi, int part_lo, int tile) {
     float out[8];
 #pragma unroll
@@ -715,8 +711,8 @@ __global__ __launch_bounds__(128, 3) void kda_prep_kernel(KdaParams p) {
     }
     u32x4 hi, lo;
     split_pack8(out, hi, lo);
-    block.store(hi, t_at, part_hi + 1024 * tile);
-    block.store(lo, t_at, part_lo + 1024 * tile);
+    block.store(hi, 16 * lane, part_hi + 1024 * tile);
+    block.store(lo, 16 * lane, part_lo + 1024 * tile);
   };
   {
     float pv[8];
@@ -770,35 +766,38 @@ template <int I, int N, int SETS, typename F> __device__ __forceinline__ void de
   }
 }
 
-constexpr int KCT = 2;                        // tiles of 16 value columns per workgroup
-constexpr int KPW = 2;                        // data-moving wavefronts per workgroup
+constexpr int KPW = 2;                        // data-moving wavefronts per workgroup, and as many for the outputs
+template <typename F, int... I> __device__ __forceinline__ void each_constant(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
 constexpr int KSTAGES = 3;                    // LDS stages of chunk data
-constexpr int kStateThreads = 64 * (2 * KCT + KPW);
+constexpr int KSETS = 4;                      // register sets of an output wavefront
+template <int KCT> constexpr int kStateThreads = 64 * (KCT + 2 * KPW);
 
 // The chunk-to-chunk chain sets the time of this kernel once its data are there, and next to it what the CU's LDS can
-// deliver (about 110 KB of operands and copies per chunk).  So:
+// deliver, 128 bytes a clock (about 130 KB of operands and copies per chunk with two column tiles, KCT = 2, 240 KB with four, which
+// sets their link).  So:
 //  * one wavefront owns one tile of 16 value columns with all of its state rows: the state never leaves its registers
 //    (as right operand it is the accumulators converted in place), nothing of the chain waits for another wavefront,
 //    and every operand of the chain is read once per column tile.  Two wavefronts per tile with half of the state each,
 //    both computing X and handing state halves over through LDS, took 250 us instead of 230 (B4 T8192 H16, 128 x 128);
-//  * the outputs are not part of the chain: a second wavefront per tile makes Qg S0 of the chunk from the bf16 state
-//    the first one left in LDS, adds (P T) X when X has arrived, and stores the rows one chunk later;
-//  * neither waits for global memory: two further wavefronts issue the asynchronous copies of the chunks ahead.
+//  * the outputs are not part of the chain: two more wavefronts, with 16 of the chunk's positions each, make Qg S0 from the bf16 state
+//    that the chain left in LDS, add (P T) X when X has arrived, and store the rows one chunk later.  Their operands come from memory
+//    into registers, KSETS - 1 chunks ahead, once for all column tiles; a wavefront per tile, with operands through the LDS: T = 8192,
+//    up to 8 heads of 128 162 -> 145 us, 16 heads 180 -> 172, 64 heads 237 -> 226 (two sets fewer or more: level);
+//  * the chain does not wait for global memory: two further wavefronts issue the asynchronous copies of the chunks ahead.
 // BY_LENGTH: packed sequences from the longest one on (a kernel of its own: with that code ahead of their loop other calls' chains are 1 to 2 % slower).
-template <int KD, bool BY_LENGTH>
-__global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p) {
+template <int KD, int KCT, bool BY_LENGTH>
+__global__ __launch_bounds__(kStateThreads<KCT>, 1) void kda_state_kernel(KdaParams p) {
   using Blob = KdaBlob<KD>;
   constexpr int NM = KD / 32, NS = KD / 16;                    // channel groups of 32, state tiles of 16 rows
-  constexpr int kV = Blob::kBytes, kStage = Blob::kBytes + KC * KVS * KCT * 2;
-  // Links are cut by workgroup barriers.  Interval n between two of them copies the chain's part of chunk n and the outputs'
-  // part of chunk n - 1, the chain reads its part in interval n + 2 and computes link n, beside its outputs, in interval n + 3.
+  constexpr int kV = Blob::kChain, kStage = kV + KC * KVS * KCT * 2;
+  // Links are cut by workgroup barriers.  Interval n between two of them copies the chain's part of chunk n; the chain reads it in
+  // interval n + 2 and computes link n, beside its outputs, in interval n + 3.
   __shared__ __attribute__((aligned(1024))) char stage[KSTAGES][kStage];
-  __shared__ __attribute__((aligned(16))) u32x4 xs[2][KCT][NM][64];           // [chunk parity][column tile][channel group][lane]: S0 as right operand
-  __shared__ __attribute__((aligned(16))) u32x4 xx[2][KCT][2][64];            // X as right operand, two terms
-  __shared__ __attribute__((aligned(16))) uint16_t ost[KCT][KC][KVS];         // output rows on their way out
+  __shared__ __attribute__((aligned(16))) u32x4 xs[2][KCT][NM][64];           // [chunk parity][column tile][channel group][lane]: S0 as operand
+  __shared__ __attribute__((aligned(16))) u32x4 xx[2][KCT][2][64];            // X as operand, two terms
 
   // The column groups of one (batch, head) on one XCD, in consecutive workgroups of it: they read the same blocks.
-  const int NGRP = (p.Dv + KVS * KCT - 1) / (KVS * KCT);       // groups of 32 value columns
+  const int NGRP = (p.Dv + KVS * KCT - 1) / (KVS * KCT);
   const int slot = blockIdx.x >> 3, grp = slot % NGRP;
   int bh = 8 * (slot / NGRP) + (blockIdx.x & 7);
   if (bh >= (p.n_seq > 0 ? p.n_seq : p.B) * p.H) return;
@@ -807,52 +806,50 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
   const SeqSpan sp = seq_span<BY_LENGTH>(p, b, rows_end);
   if constexpr (BY_LENGTH) bh = b * p.H + h;
   const int nc = sp.nc;                      // chunks of this sequence (0 for an empty one)
-  const int64_t ci0 = (int64_t)h * p.nc_total + sp.c0;
+  const int64_t ci0 = (int64_t)sp.c0 * p.H + h, step = (int64_t)p.H * Blob::kBytes;
   const int lane = threadIdx.x & 63, ln = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const char* const my_blobs = p.blobs + ci0 * Blob::kBytes;
-  const int ct = wave & 1;                   // chain 0, 1; outputs 2, 3; data 4, 5
+  const int col0 = KVS * KCT * grp;          // the workgroup's first value column
 
-  if (wave >> 1 == 2) {
+  if (wave >= KCT + KPW) {
     // ================= data-moving wavefront =================
     // Their instructions count: with an address, a branch and an m0 of its own for every KiB (some 250 scalar instructions
-    // per chunk) these wavefronts set the time of a link.  So each takes a run of the chain's part and one of the outputs' part,
-    // KiB after KiB by the instruction's own offset, the KiB with the decays (both of them, the same bytes) and 16 rows of V:
+    // per chunk) these wavefronts set the time of a link.  So each takes a run of the chain's part, KiB after KiB by the instruction's own offset, the KiB with the decays (both of them, the same bytes) and 16 rows of V:
     // lane i lands at row i / 4, piece i % 4.  Pieces past the last column re-read the last one (columns are independent and dead
     // ones are not stored).
     // The column groups of a (batch, head) ask for the same bytes at the same time.  Each begins its run at another place, so that
     // first requests differ and later ones find the L2 filled (T = 8192: 64 heads of 128 469 -> 455 us, both kernels), and
-    // in turns with a pause between: all at once they delay the other wavefronts' LDS and store traffic (4 heads of 128 215 -> 184 us,
-    // of 64 134 -> 117).  With most compute units at it, once, a longer pause is the better one (456 against 458 us; 192 against 184 the other
-    // way round; 384 workgroups, 8 x 1000 rows, 12 heads of 128: 94.2 us, 88.4 with the shorter one).  The first chunks, which nothing computes beside, are asked for without a pause, and the last outputs' part is not waited
-    // for in the interval that asks for it (64 sequences of 64 rows, 16 heads of 64: 52.1 -> 50.4 us; 4 of 100 rows, 24 heads of 128:
-    // 32.5 -> 31.0).  *Tried:* one dword of every line fetched further ahead, by these or by a wavefront of its own, and from the
-    // scalar side: slower, answers come back in order and hits wait behind misses.
-    const int pw = ct;
-    constexpr int NM1 = 3 * KC * KD * 2 / 1024 / KPW, NO1 = Blob::kOut / 1024 / KPW;
-    static_assert(NM1 * KPW * 1024 == Blob::kDec && NO1 * KPW * 1024 == Blob::kOut && Blob::kChain - Blob::kDec == 1024, "runs of whole KiB");
+    // in turns with a pause between: all at once they delay the other wavefronts' LDS and store traffic.  The pause in units of 64
+    // clocks: 0 / 1 / 2 / 4 with few chains of T = 8192, heads of 128, 147 / 145 / 147 / 169 us, with 256 workgroups 231 / 229.5 / 233 (3) / 231.
+    // The first chunks, which nothing computes beside, are asked for without (64 sequences of 64 rows, 16 heads of 64: 52.1 -> 50.4
+    // us; 4 of 100 rows, 24 heads of 128: 32.5 -> 31.0).  *Tried:* a fourth stage: level.  *Tried:* one dword of every line fetched further
+    // ahead, by these or by a wavefront of its own, and from the scalar side: slower, answers come back in order and hits wait behind misses.
+    const int pw = wave - KCT - KPW;
+    constexpr int NM1 = 3 * KC * KD * 2 / 1024 / KPW;
+    static_assert(NM1 * KPW * 1024 == Blob::kDec && Blob::kChain - Blob::kDec == 1024, "runs of whole KiB");
     constexpr int kTurns = NM1 / 3;
-    const bool crowded = gridDim.x >= 192 && gridDim.x <= 256;
     const uint32_t stage_lds = lds_address(&stage[0][0]);
     const int n_rows = sp.tok_end - sp.tok0, v_pitch = 2 * p.H * p.Dv;
     const char* const my_v = (const char*)(p.v + ((int64_t)sp.tok0 * p.H + h) * p.Dv);
-    const int v_row = 16 * pw + (lane >> 2), v_off = 16 * min(KVS * KCT * grp / 8 + (lane & 3), p.Dv / 8 - 1);
+    const int v_row = 16 * pw + (lane >> 2);
+    int v_off[KCT / 2];
+#pragma unroll
+    for (int u = 0; u < KCT / 2; ++u) v_off[u] = 16 * min(col0 / 8 + 4 * u + (lane & 3), p.Dv / 8 - 1);
     auto copy_chain = [&](int n, int st) {
-      const char* const block = my_blobs + (int64_t)n * Blob::kBytes;
+      const char* const block = my_blobs + n * step;
       const uint32_t to = stage_lds + st * kStage;
 #pragma unroll
       for (int i = 0; i < kTurns; ++i) {
         const int first = (pw * kTurns + (i + grp) % kTurns) * (NM1 / kTurns) * 1024;
         copy_kib_to_lds_async<NM1 / kTurns>(block + first, 16 * lane, to + first);
         if (n < KSTAGES) continue;
-        if (crowded) __builtin_amdgcn_s_sleep(4); else __builtin_amdgcn_s_sleep(2);
+        __builtin_amdgcn_s_sleep(1);
       }
       copy_kib_to_lds_async<1>(block + Blob::kDec, 16 * lane, to + Blob::kDec);
-      copy_kib_to_lds_async<1>(my_v + (int64_t)n * KC * v_pitch, min(v_row, n_rows - n * KC - 1) * v_pitch + v_off, to + kV + 1024 * pw);
-    };
-    auto copy_out = [&](int n, int st) {
-      constexpr int first = Blob::kChain;
-      copy_kib_to_lds_async<NO1>(my_blobs + (int64_t)n * Blob::kBytes + first + pw * NO1 * 1024, 16 * lane, stage_lds + st * kStage + first + pw * NO1 * 1024);
+#pragma unroll
+      for (int u = 0; u < KCT / 2; ++u)
+        copy_kib_to_lds_async<1>(my_v + (int64_t)n * KC * v_pitch, min(v_row, n_rows - n * KC - 1) * v_pitch + v_off[u], to + kV + 2048 * u + 1024 * pw);
     };
     auto landed = [&](auto still) {           // all copies but the youngest `still` of this wavefront are in the LDS
       constexpr int N = decltype(still)::value;
@@ -861,82 +858,92 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
       asm volatile("" ::: "memory");
     };
     int st = 0;                               // stage of chunk n
-    for (int n = 0; n < nc + 3; ++n) {
-      const int before = st == 0 ? KSTAGES - 1 : st - 1;
-      if (n < nc) copy_chain(n, st);
-      if (n > 0 && n <= nc) copy_out(n - 1, before);
-      // everything of earlier intervals has landed
-      if (n == 0) landed(std::integral_constant<int, NM1 + 2>{});
-      else if (n < nc) landed(std::integral_constant<int, NM1 + 2 + NO1>{});
-      else if (n == nc) landed(std::integral_constant<int, NO1>{});
-      else landed(std::integral_constant<int, 0>{});
+    for (int n = 0; n < nc + KSTAGES; ++n) {
+      if (n < nc) {
+        copy_chain(n, st);
+        landed(std::integral_constant<int, (KSTAGES - 2) * (NM1 + 1 + KCT / 2)>{});
+      } else {
+        landed(std::integral_constant<int, 0>{});
+      }
       st = st == KSTAGES - 1 ? 0 : st + 1;
       __syncthreads();
     }
     return;
   }
 
-  // ---- per-lane LDS read offsets (bytes, inside a stage) ------------------------------------
-  // A operand of a 16x16x32 MFMA: lane (row ln, k-group q4) reads piece 4m + q4 of its row; rows 16 apart share a swizzle.
-  int rdk[NM];
-#pragma unroll
-  for (int m = 0; m < NM; ++m) rdk[m] = ln * 2 * KD + 16 * ((4 * m + q4) ^ piece_swizzle<2 * KD>(ln));
-  const int rd64 = ln * 64 + 16 * (q4 ^ piece_swizzle<64>(ln));
-  lds_cptr const stage0 = (lds_cptr)&stage[0][0];
-  int so = 0;                                 // stage of the chunk at hand
-
   if (wave >= KCT) {
-    // ================= output wavefront =================
-    const int piece = lane & 1, col = KVS * (KCT * grp + ct) + 8 * piece;
-    f32x4 O[2];
-    bf16x8 ph[2], pl[2];
-    // O(n) += (P T) X, then the 32 rows of 32 bytes leave: two lanes per row
-    auto finish = [&](int n) {
-      const bf16x8 Xh = __builtin_bit_cast(bf16x8, xx[n & 1][ct][0][lane]), Xl = __builtin_bit_cast(bf16x8, xx[n & 1][ct][1][lane]);
+    // ================= output wavefront: 16 positions of every chunk, all columns =================
+    // Its rows of Qg and P come straight into registers, as operands, KSETS - 1 links ahead; the products are O^T, so that a lane has
+    // four neighbouring columns of one position per tile and, of the tiles 2 u and 2 u + 1, eight.
+    const int mt = wave - KCT;
+    const char* const my_q = my_blobs + Blob::kQg + 1024 * NM * mt + 16 * lane;
+    const char* const my_p = my_blobs + Blob::kPh + 1024 * mt + 16 * lane;
+    bf16x8 qg[KSETS][NM], pt[KSETS][2];
+    auto fetch = [&](auto set, int n) {
+      constexpr int s = decltype(set)::value;
+      const int64_t at = n * step;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[mt], Xh, O[mt], 0, 0, 0);
-        O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph[mt], Xl, O[mt], 0, 0, 0);
-        O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph[mt], Xh, O[mt], 0, 0, 0);
+      for (int m = 0; m < NM; ++m) qg[s][m] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(my_q + at + 1024 * m));
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ost[ct][16 * mt + 4 * q4 + r][ln] = (uint16_t)(pack_bf16x2(O[mt][r], 0.f) & 0xffffu);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      const u32x4 v = *reinterpret_cast<const u32x4*>(&ost[ct][lane >> 1][8 * piece]);
-      const int tok = sp.tok0 + n * KC + (lane >> 1);
-      if (tok < sp.tok_end && col < p.Dv) *reinterpret_cast<u32x4*>(p.o + ((int64_t)tok * p.H + h) * p.Dv + col) = v;
+      for (int t = 0; t < 2; ++t) pt[s][t] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(my_p + at + (Blob::kPl - Blob::kPh) * t));
     };
-    for (int n = 0; n < 3; ++n) __syncthreads();
-    for (int n = 0; n < nc; ++n) {
-      lds_cptr sb = stage0 + so;
-      so = so == (KSTAGES - 1) * kStage ? 0 : so + kStage;
-      if (n > 0) finish(n - 1);
+    f32x4 O[KCT];
+    uint16_t* const my_o = p.o + ((int64_t)(sp.tok0 + 16 * mt + ln) * p.H + h) * p.Dv + col0 + 8 * q4;
+    // O(n) += (P T) X, then the rows leave
+    auto finish = [&](auto set, int n) {
+      constexpr int s = decltype(set)::value;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        ph[mt] = lds_bf16x8(sb + Blob::kPh + 16 * mt * 64 + rd64);
-        pl[mt] = lds_bf16x8(sb + Blob::kPl + 16 * mt * 64 + rd64);
-        O[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int ct = 0; ct < KCT; ++ct) {
+        const bf16x8 Xh = __builtin_bit_cast(bf16x8, xx[n & 1][ct][0][lane]), Xl = __builtin_bit_cast(bf16x8, xx[n & 1][ct][1][lane]);
+        O[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Xh, pt[s][1], O[ct], 0, 0, 0);
+        O[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Xl, pt[s][0], O[ct], 0, 0, 0);
+        O[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Xh, pt[s][0], O[ct], 0, 0, 0);
       }
+      const bool live = sp.tok0 + n * KC + 16 * mt + ln < sp.tok_end;
 #pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        const bf16x8 Sb = __builtin_bit_cast(bf16x8, xs[n & 1][ct][m][lane]);
+      for (int u = 0; u < KCT / 2; ++u) {
+        const u32x4 v = {pack_bf16x2(O[2 * u][0], O[2 * u][1]), pack_bf16x2(O[2 * u][2], O[2 * u][3]),
+                         pack_bf16x2(O[2 * u + 1][0], O[2 * u + 1][1]), pack_bf16x2(O[2 * u + 1][2], O[2 * u + 1][3])};
+        if (live && col0 + 32 * u + 8 * q4 < p.Dv) *reinterpret_cast<u32x4*>(my_o + (int64_t)n * KC * p.H * p.Dv + 32 * u) = v;
+      }
+    };
+    auto link = [&](auto set, int n) {
+      constexpr int s = decltype(set)::value, before = (s + KSETS - 1) % KSETS;
+      if (n > 0) finish(std::integral_constant<int, before>{}, n - 1);
+      fetch(std::integral_constant<int, before>{}, min(n + KSETS - 1, nc - 1));
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-          O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lds_bf16x8(sb + Blob::kQg + 16 * mt * 2 * KD + rdk[m]), Sb, O[mt], 0, 0, 0);
+      for (int ct = 0; ct < KCT; ++ct) {
+        O[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+          O[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xs[n & 1][ct][m][lane]), qg[s][m], O[ct], 0, 0, 0);
       }
       __syncthreads();
-    }
-    if (nc > 0) finish(nc - 1);
+    };
+    auto each_set = [](auto f) { each_constant(f, std::make_integer_sequence<int, KSETS>{}); };
+    if (nc > 0) each_set([&](auto set) { if constexpr (decltype(set)::value < KSETS - 1) fetch(set, min((int)decltype(set)::value, nc - 1)); });
+    for (int i = 0; i < KSTAGES; ++i) __syncthreads();
+    for (int n = 0; n < nc; n += KSETS)
+      each_set([&](auto set) {
+        constexpr int s = decltype(set)::value;
+        if (n + s < nc) link(set, n + s);
+        if (n + s == nc - 1) finish(set, n + s);
+      });
     // rows behind the last sequence of a packed batch belong to none: zeros
-    if (p.n_seq > 0 && b == p.n_seq - 1 && col < p.Dv)
-      for (int tok = rows_end + (lane >> 1); tok < p.T; tok += 32) *reinterpret_cast<u32x4*>(p.o + ((int64_t)tok * p.H + h) * p.Dv + col) = u32x4{0u, 0u, 0u, 0u};
+    if (p.n_seq > 0 && b == p.n_seq - 1)
+      for (int u = 0; u < KCT / 2; ++u)
+        for (int tok = rows_end + 16 * mt + ln; tok < p.T; tok += 32)
+          if (col0 + 32 * u + 8 * q4 < p.Dv) *reinterpret_cast<u32x4*>(p.o + ((int64_t)tok * p.H + h) * p.Dv + col0 + 32 * u + 8 * q4) = u32x4{0u, 0u, 0u, 0u};
     return;
   }
 
   // ================= chain wavefront =================
-  const int vcol = KVS * (KCT * grp + ct) + ln;
-  const int rdv = kV + (4 * q4 + (ln >> 2)) * 64 + 2 * (KVS * ct + 4 * (ln & 3));
+  // Column ln of tile ct: the tiles 2 u and 2 u + 1 take turns in the fours of 32 columns, for the outputs' sake.
+  const int ct = wave, vcol = col0 + 32 * (ct >> 1) + 8 * (ln >> 2) + 4 * (ct & 1) + (ln & 3);
+  const int rdv = kV + 2048 * (ct >> 1) + (4 * q4 + (ln >> 2)) * 64 + 2 * (8 * (ln & 3) + 4 * (ct & 1));
+  const int rd = 16 * lane;                   // a lane's piece of a KiB of operands
+  lds_cptr const stage0 = (lds_cptr)&stage[0][0];
+  int so = 0;                                 // stage of the chunk at hand
   // State tile i: rows (key channels) 32*(i/2) + 8*q4 + 4*(i%2) + r, column vcol; rows beyond Dk and columns beyond Dv do not
   // exist in the caller's [Dk, Dv] state: they are zero and stay zero.
   const bool col_live = vcol < p.Dv;
@@ -958,8 +965,7 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
     }
   };
   next_operand(0, NM, 0);
-  __syncthreads();
-  __syncthreads();
+  for (int i = 0; i < KSTAGES - 1; ++i) __syncthreads();
 
   // A link's operands are read during the link before it, each register as soon as its last product has been issued: a 16-byte
   // LDS read keeps a wavefront's port for 16 cycles and a chunk needs 34 of them, which in front of their use was half of
@@ -976,14 +982,14 @@ __global__ __launch_bounds__(kStateThreads, 1) void kda_state_kernel(KdaParams p
   };
   auto read_ka = [&](lds_cptr sb, int m) {
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) ka[mt][m] = lds_bf16x8(sb + Blob::kKg + 16 * mt * 2 * KD + rdk[m]);
+    for (int mt = 0; mt < 2; ++mt) ka[mt][m] = lds_bf16x8(sb + Blob::kKg + 1024 * (NM * mt + m) + rd);
   };
   auto read_dec = [&](lds_cptr sb, int set) {
     const int i = DECS == 1 ? ln & (NS - 1) : set;
     dec[set] = lds_f32x4(sb + Blob::kDec + 4 * (32 * (i >> 1) + 8 * q4 + 4 * (i & 1)));
   };
-  auto read_ml = [&](lds_cptr sb, int i) { ml[i] = lds_bf16x8(sb + Blob::kMl + 16 * i * 64 + rd64); };
-  auto read_mh = [&](lds_cptr sb, int i) { mh[i] = lds_bf16x8(sb + Blob::kMh + 16 * i * 64 + rd64); };
+  auto read_ml = [&](lds_cptr sb, int i) { ml[i] = lds_bf16x8(sb + Blob::kMl + 1024 * i + rd); };
+  auto read_mh = [&](lds_cptr sb, int i) { mh[i] = lds_bf16x8(sb + Blob::kMh + 1024 * i + rd); };
   read_v(stage0);
 #pragma unroll
   for (int m = 0; m < NM; ++m) read_ka(stage0, m);
@@ -1124,31 +1130,35 @@ extern "C" size_t daisy_kda_varlen_workspace_bytes(int T, int n_seq, int H, int 
 // 168 -> 176, against 2 x 7500, 8 heads of 128 260 -> 252.
 constexpr int64_t kCachedBytes = (int64_t)128 << 20;
 
-template <int KD>
-static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
+template <int KD, int KCT>
+static void launch_chains(const KdaParams& p, int n_streams, hipStream_t s) {
   const int groups = (p.Dv + KVS * KCT - 1) / (KVS * KCT);
-  const dim3 chunks(p.NC, p.H, p.n_seq > 0 ? 1 : p.B);
-  const int64_t bytes = (int64_t)p.H * p.nc_total * KdaBlob<KD>::kBytes;
-  if (bytes > kCachedBytes) {
-    // fp32 log-decays beyond 400 MB: 6 KB more of LDS than the kernel uses, five workgroups per compute unit.  Where memory is the bound a sixth
-    // only adds requests.  16 heads of 128, T = 8192, B = 3 / 4 / 6, both kernels, six workgroups -> five: mild fp32 log-decays 375 to 381 -> 374 to 376,
-    // 442 to 450 -> 442 to 448, 742 -> 735 us (with four the latency shows: 329 us for the first kernel, B = 4, where it takes 216); steep fp32 ones 390 -> 396, 466 ->
-    // 472, 756 -> 766.  With half the bytes to read the vector instructions are: mild bf16 ones 364 / 364, 416 / 415, 690 / 688,
-    // steep ones (a layer's first gates) 377 / 387, 450 / 468, 729 / 749, so those keep all six.
-    const bool memory_bound = KD == 128 && !p.g_bf16 && bytes > (int64_t)400 << 20;
-    hipLaunchKernelGGL((kda_prep_kernel<KD, true>), chunks, dim3(128), memory_bound ? 6144 : 0, s, p);
-  } else {
-    hipLaunchKernelGGL((kda_prep_kernel<KD, false>), chunks, dim3(128), 0, s, p);
-  }
-  DAISY_CHECK_LAUNCH("kda_prep_kernel");
   const unsigned chains = (unsigned)((n_streams * p.H + 7) / 8 * 8 * groups);
   // A chain fills a compute unit: where there are more than 256, a long sequence that starts late ends alone.  Longest first, cut at random places, both
   // kernels: 10 sequences of T = 4689, 16 heads of 128 102 -> 87 us, 7 of 3000, 12 heads 53 -> 44.4, 7 of 6164, 16 of 64 67.3 -> 56; 40 such batches 4 % on
   // average.  Where the longest one comes early anyway ranking costs (12 of 12000, 16 of 64 95.5 -> 97.3): 0.03 us a sequence in every workgroup, so
   // only up to a tenth of a mean chain (else 16 of T = 2088, 8 heads of 128 34.5 -> 35.5, 13 of 148, 12 heads 18.2 -> 19.8); not where they are in that order.
   const bool by_length = chains > 256 && p.n_seq > 1 && p.n_seq <= kScanSeqs && p.NC >= p.n_seq * p.n_seq;
-  if (by_length) hipLaunchKernelGGL((kda_state_kernel<KD, true>), dim3(chains), dim3(kStateThreads), 0, s, p);
-  else hipLaunchKernelGGL((kda_state_kernel<KD, false>), dim3(chains), dim3(kStateThreads), 0, s, p);
+  if (by_length) hipLaunchKernelGGL((kda_state_kernel<KD, KCT, true>), dim3(chains), dim3(kStateThreads<KCT>), 0, s, p);
+  else hipLaunchKernelGGL((kda_state_kernel<KD, KCT, false>), dim3(chains), dim3(kStateThreads<KCT>), 0, s, p);
+}
+
+template <int KD>
+static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
+  const dim3 chunks((unsigned)p.NC * (unsigned)p.H, 1, p.n_seq > 0 ? 1 : p.B);
+  const int64_t bytes = (int64_t)p.H * p.nc_total * KdaBlob<KD>::kBytes;
+  if (bytes > kCachedBytes) {
+    hipLaunchKernelGGL((kda_prep_kernel<KD, true>), chunks, dim3(128), 0, s, p);
+  } else {
+    hipLaunchKernelGGL((kda_prep_kernel<KD, false>), chunks, dim3(128), 0, s, p);
+  }
+  DAISY_CHECK_LAUNCH("kda_prep_kernel");
+  // Where groups of 32 value columns are more than the compute units, groups of 64: a link of 64 columns takes longer (0.8 us against 0.57 with few chains,
+  // by its LDS reads), but one round of them less than two.  Chains of T = 4096, 32 / 64 columns, us: heads of 128, 256 groups of 32 167 / 183, 320 206 /
+  // 140, 384 210 / 155, 512 228 / 187, T = 2048 1024 229 / 187; key heads of 64 256 114 / 125, 320 156 / 106, 512 172 / 128, 64 sequences of 64 rows 22 / 20.  Packed
+  // sequences likewise, of equal lengths or not (16 of 17 batches 1 to 18 % faster with 64, both kernels; 11 cut at random places, the longest 2.6 means, 108 / 120).
+  const int64_t groups = (int64_t)n_streams * p.H * ((p.Dv + 2 * KVS - 1) / (2 * KVS));
+  if (groups > 256 && p.Dv > 2 * KVS) launch_chains<KD, 4>(p, n_streams, s); else launch_chains<KD, 2>(p, n_streams, s);
   DAISY_CHECK_LAUNCH("kda_state_kernel");
   return DAISY_OK;
 }
@@ -1177,7 +1187,7 @@ static int kda_chunk_launch(const void* q, const void* k, const void* v,
     set_error("kda: workspace of %zu bytes needed, got %zu", need, workspace_bytes);
     return DAISY_ERR_WORKSPACE;
   }
-  DAISY_CHECK_ARG(slots <= 0x7fffffff && ((int64_t)(n_seq > 0 ? n_seq : B) * H + 7) * ((Dv + KVS * KCT - 1) / (KVS * KCT)) <= 0x7fffffff,
+  DAISY_CHECK_ARG((int64_t)slots * H <= 0x1ffffff && ((int64_t)(n_seq > 0 ? n_seq : B) * H + 7) * ((Dv + 2 * KVS - 1) / (2 * KVS)) <= 0x7fffffff,
                   "kda: too many chunks or sequences");
   KdaParams p;
   p.q = (const uint16_t*)q; p.k = (const uint16_t*)k; p.v = (const uint16_t*)v;

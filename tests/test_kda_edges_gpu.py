@@ -75,9 +75,8 @@ def test_kda_packed_chunk_slots(lengths, behind):
         assert ((S[i:i + 1] - S_ref).norm() / S_ref.norm()).item() <= 1e-3
 
 
-# Blocks of the workspace (37 KiB per chunk and head, 21 for up to 64 key channels) beyond 128 MB are stored past the caches, those of
-# 128 channels with fp32 log-decays beyond 400 with fewer workgroups per compute unit; 192 to 256 workgroups of the second
-# kernel copy at another pace.  Heads are independent: the same bits as from calls on the other side of every line.
+# Blocks of the workspace (37 KiB per chunk and head, 21 for up to 64 key channels) beyond 128 MB are stored past the caches.  Heads are
+# independent: the same bits as from calls on the other side of the line.
 @pytest.mark.parametrize("T,H,Dk", [(3712, 32, 128), (8200, 48, 128), (6560, 48, 64)])
 def test_kda_workspace_sizes_agree(T, H, Dk):
     assert (T + 31) // 32 * H * (37 if Dk > 64 else 21) * 1024 > (400 << 20 if T > 8000 else 128 << 20)
@@ -112,6 +111,40 @@ def test_kda_packed_longest_first(lengths, D):
             continue
         o1, S1 = _run(*(t[:, cu[i]:cu[i] + m].contiguous() for t in (q, k, v, gl, beta)), initial_state=s0[i:i + 1].cuda())
         assert torch.equal(o[:, cu[i]:cu[i] + m], o1) and torch.equal(S[i:i + 1], S1)
+
+
+# More groups of 32 value columns than compute units: groups of 64, whole ones, with a dead half, and with columns that end inside a
+# half.  Sequences are independent: the same bits as from a call of one of them, in groups of 32.
+@pytest.mark.parametrize("B,T,H,Dk,Dv", [(40, 33, 8, 64, 40), (9, 97, 16, 128, 96), (33, 1, 8, 72, 64), (17, 160, 8, 128, 72), (12, 129, 12, 64, 128)])
+def test_kda_wide_column_groups(B, T, H, Dk, Dv):
+    assert B * H * ((Dv + 31) // 32) > 256 >= (H + 7) // 8 * 8 * ((Dv + 31) // 32)
+    q, k, v, gl, beta = _inputs(B, T, H, Dk, Dv, seed=B + T)
+    s0 = torch.randn(B, H, Dk, Dv, generator=torch.Generator().manual_seed(B))
+    o, S = _run(q, k, v, gl, beta, initial_state=s0.cuda())
+    for b in (0, B // 2, B - 1):
+        part = [t[b:b + 1].contiguous() for t in (q, k, v, gl, beta)]
+        o1, S1 = _run(*part, initial_state=s0[b:b + 1].cuda())
+        assert torch.equal(o[b:b + 1], o1) and torch.equal(S[b:b + 1], S1)
+    o_ref, S_ref = oracle.kda_recurrent(*part, initial_state=s0[B - 1:])
+    assert_close_bf16(o[B - 1:], o_ref, "o")
+    assert ((S[B - 1:] - S_ref).norm() / S_ref.norm()).item() <= 1e-3
+
+
+# ... of which there are more than compute units too: packed sequences start longest first.
+@pytest.mark.parametrize("D,Dv", [(64, 128), (128, 96)])
+def test_kda_packed_wide_column_groups_longest_first(D, Dv):
+    lengths, H = (40, 33, 512, 0, 512, 130, 700, 64, 513), 16
+    n, T = len(lengths), sum(lengths)
+    assert n * H * ((Dv + 63) // 64) > 256 and T // 32 + n >= n * n
+    q, k, v, gl, beta = _inputs(1, T + 5, H, D, Dv, seed=T)
+    cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32)
+    torch.full((T + 5, H, Dv), float("nan"), dtype=torch.bfloat16, device="cuda")
+    o, S = _run(q, k, v, gl, beta, cu_seqlens=cu.cuda())
+    assert not o[:, T:].any()
+    for i, m in enumerate(lengths):
+        if m:
+            o1, S1 = _run(*(t[:, cu[i]:cu[i] + m].contiguous() for t in (q, k, v, gl, beta)))
+            assert torch.equal(o[:, cu[i]:cu[i] + m], o1) and torch.equal(S[i:i + 1], S1)
 
 
 # The blocks themselves, all of their bytes, from call to call: a 16-byte store's data registers written again by the next instruction
