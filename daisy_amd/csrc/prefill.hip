@@ -160,6 +160,64 @@ __device__ __forceinline__ float pair_sum(float x) {
   return __int_as_float(r[0]) + __int_as_float(r[1]);
 }
 
+// Online softmax of a tile (log2 domain): its probabilities as operands, against the wavefront's reference maxima, which move only
+// when some query's share of the tile's sum exceeds kMost.  Until then no probability does, which bf16 and the fp32 sums hold
+// without loss, and neither the tile's maxima are looked for nor is O touched: the scores' exponentials come straight behind their
+// products.  A reference that is not set yet (no key of that query seen) takes the long way too.  The tile kernels are bound by their vector
+// instructions (head dim 64: 855 cycles of them per 64 keys against 512 of the matrix pipe) and by power, which fewer of them
+// spare: with the maxima of every tile worked out and compared (a reference moved at 2^8) 65536 rows, 16 heads of 128, full causal took 15.00 ms, now
+// 14.56; 20001 rows in seven documents, 16 heads of 64, 178.6 us, now 171.4; a layer of 8 x 4096 rows, 8 heads of 128, window 1024, 406.2 and 403.8.
+struct SoftmaxRef {
+  float m = -INFINITY, minus = 0.f;   // reference (scaled), the same in both lanes of a query; what is added to the scaled scores
+  float l = 0.f;                      // this lane's share of the running sum
+  bool unset = true;                  // some query of the wavefront has no reference
+};
+constexpr float kMost = 4096.f;
+template <int SUB, int NDT>
+__device__ __forceinline__ void softmax_tile(const f32x16 (&sacc)[SUB], float scale_log2e, SoftmaxRef& ref, f32x16 (&oacc)[NDT],
+                                             bf16x8 (&pfrag)[2 * SUB]) {
+  float lsum;
+  auto exponentials = [&]() {
+    lsum = 0.f;
+#pragma unroll
+    for (int m = 0; m < 2 * SUB; ++m) {
+      float pv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        pv[e] = fast_exp2(fmaf(sacc[m >> 1][8 * (m & 1) + e], scale_log2e, ref.minus));
+        lsum += pv[e];
+      }
+      pfrag[m] = __builtin_bit_cast(bf16x8, pack8(pv));
+    }
+  };
+  bool longer = ref.unset;
+  if (!longer) {
+    exponentials();
+    longer = __builtin_amdgcn_ballot_w64(lsum > kMost) != 0;
+  }
+  if (longer) {
+    float mt = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < SUB; ++u)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[u][r]);
+    mt = pair_max(mt) * scale_log2e;
+    const float m_new = fmaxf(ref.m, mt);
+    const float mu = (m_new == -INFINITY) ? 0.f : m_new;
+    const float alpha = fast_exp2(ref.m - mu);
+    ref.m = m_new;
+    ref.minus = -mu;
+    ref.unset = __builtin_amdgcn_ballot_w64(m_new == -INFINITY) != 0;
+    ref.l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+    exponentials();
+  }
+  ref.l += lsum;
+}
+
 // LDS transpose read (ds_read_b64_tr_b16); semantics in the header comment.
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const uint16_t* lds_u16_ptr;
@@ -359,8 +417,7 @@ __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
-  float m_run = -INFINITY;  // reference maximum (scaled, log2 domain) of this lane's query
-  float l_run = 0.f;        // this lane's share of the running sum
+  SoftmaxRef ref;
 
   // One tile of 32 keys.  There is ONE code path for clean and masked tiles (the mask is a small
   // conditional region): two instantiations of the products would make the compiler keep a second
@@ -403,41 +460,8 @@ __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
           if (c > hi || c < lo) sacc[u][r] = -INFINITY;
         }
     }
-    // Online softmax (log2 domain, lazy rescale): the reference maximum m_run only moves when some
-    // query of the wavefront sees a score more than 8 (log2 units) above it; until then
-    // probabilities are at most 2^8, which bf16 and the fp32 sums hold without loss, and O is not
-    // touched.
-    float mt = -INFINITY;
-#pragma unroll
-    for (int u = 0; u < SUB; ++u)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[u][r]);
-    mt = pair_max(mt) * p.scale_log2e;
-    if (__builtin_amdgcn_ballot_w64(mt > m_run + 8.f) != 0) {
-      const float m_new = fmaxf(m_run, mt);
-      const float mu = (m_new == -INFINITY) ? 0.f : m_new;
-      const float alpha = fast_exp2(m_run - mu);
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-    }
-    const float mu = (m_run == -INFINITY) ? 0.f : m_run;
     bf16x8 pfrag[2 * SUB];
-    float lsum = 0.f;
-#pragma unroll
-    for (int m = 0; m < 2 * SUB; ++m) {
-      float pv[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pv[e] = fast_exp2(fmaf(sacc[m >> 1][8 * (m & 1) + e], p.scale_log2e, -mu));
-        lsum += pv[e];
-      }
-      pfrag[m] = __builtin_bit_cast(bf16x8, pack8(pv));
-    }
-    l_run += lsum;
+    softmax_tile<SUB, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
     // O^T += V^T P^T
 #pragma unroll
     for (int m = 0; m < 2 * SUB; ++m) {
@@ -476,7 +500,7 @@ __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
   // Epilogue: normalise, turn the accumulators (a lane holds four channels of one query per register
   // group) into row-major bf16 through this wavefront's LDS area, and store 16 bytes per lane with whole
   // rows per group of lanes.  The tile buffers are free: the loop ends with a barrier.
-  const float l_tot = pair_sum(l_run);
+  const float l_tot = pair_sum(ref.l);
   const float inv = 1.f / l_tot;
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) {
@@ -629,7 +653,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+  SoftmaxRef ref;
 
   for (; t <= t_hi; t += W) {
     const int kv0 = t * kTBN;
@@ -637,9 +661,9 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
     // K(n) has landed when only V(n)'s copies are outstanding
     __builtin_amdgcn_s_waitcnt(0x0F70 | NCP);
     asm volatile("" ::: "memory");
-    f32x16 sacc;
+    f32x16 sacc[1];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
+    for (int r = 0; r < 16; ++r) sacc[0][r] = 0.f;
     bf16x8 kf[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s)
@@ -648,43 +672,17 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
     asm volatile("" ::: "memory");
     if (more) copy_k(t + W);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qreg[s], sacc, 0, 0, 0);
+    for (int s = 0; s < NS; ++s) sacc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qreg[s], sacc[0], 0, 0, 0);
     if (!(kv0 + kTBN - 1 <= min(q0, p.T - 1) && kv0 >= lo_max)) {
       const int hi = qrow - (kv0 + 4 * lh), lo = lo_q - (kv0 + 4 * lh);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int c = 8 * (r >> 2) + (r & 3);
-        if (c > hi || c < lo) sacc[r] = -INFINITY;
+        if (c > hi || c < lo) sacc[0][r] = -INFINITY;
       }
     }
-    // online softmax with the lazy rescale of prefill_tile_kernel
-    float mt = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[r]);
-    mt = pair_max(mt) * p.scale_log2e;
-    if (__builtin_amdgcn_ballot_w64(mt > m_run + 8.f) != 0) {
-      const float m_new = fmaxf(m_run, mt);
-      const float mu = (m_new == -INFINITY) ? 0.f : m_new;
-      const float alpha = fast_exp2(m_run - mu);
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-    }
-    const float mu = (m_run == -INFINITY) ? 0.f : m_run;
     bf16x8 pfrag[2];
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      float pv[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pv[e] = fast_exp2(fmaf(sacc[8 * m + e], p.scale_log2e, -mu));
-        l_run += pv[e];
-      }
-      pfrag[m] = __builtin_bit_cast(bf16x8, pack8(pv));
-    }
+    softmax_tile<1, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
     // V(n) has landed when only K(n + 1)'s copies are outstanding
     if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | NCP);
     else __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -706,8 +704,8 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
 
   // Partial results: each lane of a pair holds its share of the row sum; O^T as [query][channel] fp32 in the
   // wavefront's own tile area, 16-byte pieces swizzled by the query.
-  const float l_tot = pair_sum(l_run);
-  if (lh == 0) { part_m[wave][lq] = m_run; part_l[wave][lq] = l_tot; }
+  const float l_tot = pair_sum(ref.l);
+  if (lh == 0) { part_m[wave][lq] = ref.m; part_l[wave][lq] = l_tot; }
   float* const po = reinterpret_cast<float*>(&tiles[wave][0][0]);
   constexpr int PC = D / 4;
 #pragma unroll

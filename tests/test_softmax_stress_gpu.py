@@ -63,6 +63,25 @@ def test_prefill_large_logits(D, window, rise):
 
 
 @pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("above", [11.0, 11.9, 12.1, 15.0, 140.0])
+@pytest.mark.parametrize("at", [130, 400, 639])
+def test_prefill_one_key_above_the_reference(D, above, at):
+    """All scores 0 but those of one key, `above` log2 units higher for every third query (for the others lower): on either side of
+    2^12, the share of a tile's sum that makes the reference move, and past what fp32 holds without it.  The key lies behind the tiles
+    that set the references; a lane holds it alone in a tile, so that it is the sum."""
+    T, H = 700, 2
+    g = torch.Generator().manual_seed(D + at)
+    q, k = torch.zeros(1, T, H, D), torch.zeros(1, T, H, D)
+    q[..., 3] = torch.where(torch.arange(T) % 3 == 0, 4.0, -4.0).view(1, T, 1)
+    k[:, at, :, 3] = above / LOG2E / 4.0
+    q, k, v = q.bfloat16(), k.bfloat16(), torch.randn(1, T, H, D, generator=g).bfloat16()
+    ref = oracle.windowed_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), None, 1.0).transpose(1, 2)
+    o, _ = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), window=None, scale=1.0)
+    assert_close_bf16(o, ref, "o")
+    check_prefill_of_many_heads(q.cuda(), k.cuda(), v.cuda(), ref, f"{above} above", window=None, scale=1.0)
+
+
+@pytest.mark.parametrize("D", [64, 128])
 def test_prefill_large_logits_with_rotation_and_documents(D):
     """The same with RoPE in the call and document bounds (masked tiles take the same softmax path)."""
     B, T, H, W = 2, 515, 2, 300
