@@ -745,7 +745,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] *= inv;
     if (q0 + row < p.T)
-      *reinterpret_cast<u32x4*>(p.o + b * p.o_sb + (int64_t)(q0 + row) * p.o_st + h * p.o_sh + 8 * c) = pack8(acc);
+      store_through(p.o + b * p.o_sb + (int64_t)(q0 + row) * p.o_st + h * p.o_sh + 8 * c, pack8(acc));
   }
 }
 

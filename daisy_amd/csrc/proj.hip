@@ -221,7 +221,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
       const int idx = tid + NTHR * it, m = idx / CHN, c = idx % CHN;
       if (BM * CHN % NTHR != 0 && m >= BM) break;
       const u32x4 v = *reinterpret_cast<const u32x4*>(tile_at(m, c));
-      if (m0 + m < p.M && n0 + 8 * c < g.N) *reinterpret_cast<u32x4*>(g.y + (int64_t)(m0 + m) * g.y_sm + n0 + 8 * c) = v;
+      if (m0 + m < p.M && n0 + 8 * c < g.N) store_through(g.y + (int64_t)(m0 + m) * g.y_sm + n0 + 8 * c, v);
     }
   } else {
     constexpr int D = EPI == 1 ? 64 : 128, HALF = D / 2, LPR = D / 16, HPT = BN / D;
@@ -293,8 +293,8 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
           dst = e.v + b * e.v_sb + t * e.v_st + h * e.v_sh;
         }
         if (live) {
-          *reinterpret_cast<u32x4*>(dst + 8 * c) = pack8(lo);
-          *reinterpret_cast<u32x4*>(dst + 8 * c + HALF) = pack8(hi);
+          store_through(dst + 8 * c, pack8(lo));
+          store_through(dst + 8 * c + HALF, pack8(hi));
         }
       }
     }
