@@ -5,10 +5,9 @@
 // tiles to give every compute unit several workgroups, so nothing hides a workgroup's own latencies: with one K step in
 // flight, a step lasts a memory round trip (about 0.7 us) where its matrix instructions take 0.2 us.  The kernel
 // keeps up to three K steps in flight (asynchronous global -> LDS copies; a wavefront waits with vmcnt for the oldest
-// step only), reads the operands of a step before it issues the next copies, and the tile shape follows the number of
+// step only), reads the operands of the next products beside the ones at hand, and the tile shape follows the number of
 // tiles (kProjTiles).  Large products are bound by the matrix cores and by what the compute units can pull through the
-// L2, hence the order of the tiles (below).  Reading the operands of a step ahead of the barrier in front of it
-// was tried: 10 % slower on the small shapes, no different on the large ones.
+// L2, hence the order of the tiles (below).
 //
 // Operands: both x [M, K] and W [N, K] have K contiguous, so both tiles are rows of 64 or 128 bf16 in LDS, their
 // 16-byte chunks XOR-swizzled so that 16 rows read side by side fall into 16 different slots of the 256-byte bank
@@ -128,41 +127,81 @@ __global__ __launch_bounds__(64 * WVM * WVN) void proj_kernel(std::conditional_t
   const uint32_t fb = lds_address(smem) + ABYTES + (WN * wn + ln) * RB + 16 * (q4 ^ swz(ln));
   auto frag = [&](uint32_t a) { return __builtin_bit_cast(bf16x8, *(const u32x4 __attribute__((address_space(3)))*)(size_t)a); };
 
-  int st = 0;
-  for (int k = 0; k < nk; ++k) {
-    // the copies of step k have landed when at most those of the steps behind it are outstanding
-    const int behind = nk - 1 - k;
-    if (STAGES == 2 || behind == 0) wait_vmcnt<0>();
+  // The copies of a step have landed when at most those of the `behind` steps after it are outstanding.
+  auto landed = [&](int behind) {
+    if (STAGES == 2 || behind <= 0) wait_vmcnt<0>();
     else if (behind >= STAGES - 2) wait_vmcnt<CPW * (STAGES - 2)>();
     else wait_vmcnt<CPW>();                  // STAGES <= 4: one step behind
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const uint32_t so = st * STAGE;
-    bf16x8 a[KK][NI], b[KK][MI];
+  };
+  bf16x8 a[2][NI], b[2][MI];                 // operands of 32 elements of K, and the next ones
+  auto read = [&](int kk, uint32_t so) {
 #pragma unroll
-    for (int i = 0; i < NI; ++i) a[0][i] = frag(fb + so + 16 * RB * i);
+    for (int i = 0; i < NI; ++i) a[kk & 1][i] = frag((fb ^ (64u * kk)) + so + 16 * RB * i);
 #pragma unroll
-    for (int j = 0; j < MI; ++j) b[0][j] = frag(fa + so + 16 * RB * j);
+    for (int j = 0; j < MI; ++j) b[kk & 1][j] = frag((fa ^ (64u * kk)) + so + 16 * RB * j);
+  };
+  auto multiply = [&](int kk) {
     __builtin_amdgcn_sched_barrier(0);
-    // every wavefront is done with step k - 1: its stage takes step k + STAGES - 1
-    if (k + STAGES - 1 < nk) issue(st == 0 ? STAGES - 1 : st - 1);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < MI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk & 1][i], b[kk & 1][j], acc[i][j], 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
+  };
+  static_assert(KK % 2 == 0, "a step ends on the second set");
+  int st = 0;
+  if constexpr (STAGES == 2) {
+    for (int k = 0; k < nk; ++k) {
+      landed(0);
+      const uint32_t so = st * STAGE;
+      read(0, so);
+      __builtin_amdgcn_sched_barrier(0);
+      // every wavefront is done with step k - 1: its stage takes step k + 1
+      if (k + 1 < nk) issue(st ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      if (kk + 1 < KK) {
-#pragma unroll
-        for (int i = 0; i < NI; ++i) a[kk + 1][i] = frag((fb ^ (64u * (kk + 1))) + so + 16 * RB * i);
-#pragma unroll
-        for (int j = 0; j < MI; ++j) b[kk + 1][j] = frag((fa ^ (64u * (kk + 1))) + so + 16 * RB * j);
-        __builtin_amdgcn_sched_barrier(0);
+      for (int kk = 0; kk < KK; ++kk) {
+        if (kk + 1 < KK) read(kk + 1, so);
+        multiply(kk);
       }
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < MI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][i], b[kk][j], acc[i][j], 0, 0, 0);
+      st ^= 1;
     }
-    st = st + 1 == STAGES ? 0 : st + 1;
+  } else {
+    // The operands of a step's first products are read beside the last ones of the step before, so that only the barrier lies between
+    // two steps' products, not the reads (0.2 of 0.41 us a step of 128 x 128 x 64 on eight wavefronts; its matrix instructions take 0.32 at the
+    // clock that they are granted).  us, before / now: 16 x 4608 x 1536 (tile 9) 5.21 / 4.89, 64 x 2048 x 2048 6.03 / 5.44; 128 x 2048 x 2048 (10) 6.38 /
+    // 5.78; 128 x 6144 x 2048 (2) 9.25 / 8.80; 777 x 4608 x 1536 (5) 15.4 / 14.9; tiles 1, 3 and 4 level; with two stages it loses (6: 1500 x 4608 x 1536 23.4 /
+    // 27.6; 7: a layer of 8 x 4096 rows 403 / 411).
+    // `inside`: there are STAGES more steps; else `behind` of them after the next one, -1: no next one.
+    uint32_t so = 0;
+    auto step = [&](auto inside, int behind) {
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) {
+        if (kk + 1 < KK) {
+          read(kk + 1, so);
+        } else if (inside || behind >= 0) {
+          // the step's last operands are in registers, of all wavefronts behind the barrier: its stage takes the step STAGES ahead
+          landed(inside ? STAGES - 2 : behind);
+          so = st + 1 == STAGES ? 0 : so + STAGE;
+          read(0, so);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (inside) issue(st);
+          st = st + 1 == STAGES ? 0 : st + 1;
+        }
+        multiply(kk);
+      }
+    };
+    landed(min(STAGES - 1, nk) - 1);
+    if (STAGES - 1 < nk) issue(STAGES - 1);
+    read(0, 0);
+    // (with a scalar load pending here the compiler, which cannot tell their order, would wait for every LDS read ahead of the products)
+    __builtin_amdgcn_s_waitcnt(0xC07F);       // lgkmcnt(0)
+    int k = 0;
+    for (; k + STAGES < nk; ++k) step(std::true_type{}, 0);
+    for (; k < nk; ++k) step(std::false_type{}, nk - 2 - k);
   }
   __syncthreads();
 

@@ -35,6 +35,14 @@ def test_smallest_tiles_against_fp64(tile, K, M, N):
     test_tiles_against_fp64(tile, K, M, N)
 
 
+@pytest.mark.parametrize("tile,bk,stages", [(1, 128, 3), (2, 128, 4), (3, 128, 3), (4, 64, 3), (5, 64, 4), (6, 64, 2), (9, 128, 4), (10, 128, 4)])
+@pytest.mark.parametrize("more", [-2, -1, 0, 1, 2, 5])
+def test_tiles_around_as_many_steps_as_stages_against_fp64(tile, bk, stages, more):
+    """From fewer steps of K than there are stages, where every step is one of the last, to a few more, where stages are reused."""
+    K = bk * max(stages + more, 1)
+    test_tiles_against_fp64(tile, K, 70, 136)
+
+
 @pytest.mark.parametrize("M", [2, 3, 4, 5, 8, 9])
 @pytest.mark.parametrize("N,K", [(1024, 192), (2048, 64), (2056, 128), (5464, 128), (8200, 64), (16392, 72), (1024, 72)])
 def test_few_rows_on_both_sides_of_the_rule_against_fp64(M, N, K):
