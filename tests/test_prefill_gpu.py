@@ -190,3 +190,15 @@ def test_documents_equal_their_own_calls(B, T, H, D, W, starts):
         ref, _ = ops.prefill_attention(q[:, a:b], k[:, a:b], v[:, a:b], window=W)
         # two bf16 roundings of the same sums over other tiles of keys, with bf16 probabilities
         assert ((o[:, a:b].float() - ref.float()).norm() / ref.float().norm()).item() < 1e-2
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H", [1, 2, 3, 4, 6, 12])
+@pytest.mark.parametrize("B,T", [(1, 1), (2, 37), (1, 300)])
+def test_rotated_keys_are_the_oracles_bits(D, H, B, T):
+    """One, two and four heads a thread; counts of rows that leave surplus lanes in the last workgroup; keys at strides of their own."""
+    q, k, v = _inputs(B, T, H, D, seed=H + T)
+    cos, sin = oracle.rope_tables(D, T)
+    kd = torch.zeros(B, T, H, D + 8, dtype=torch.bfloat16, device="cuda")[..., :D].copy_(k)
+    _, kr = ops.prefill_attention(q.cuda(), kd, v.cuda(), window=None, cos=cos.cuda(), sin=sin.cuda())
+    assert torch.equal(kr.cpu(), oracle.apply_rope(k, cos, sin))
