@@ -223,7 +223,7 @@ PyObject* py_linears(PyObject*, PyObject* const* a, Py_ssize_t n) {
     seg[i] = daisy::ProjSegment{r.p, r.stride, (const uint16_t*)ptr(w), w.stride(0), (const uint16_t*)ptr(bias), nullptr, 0, (int)w.size(0), 0};
     pitch += (w.size(0) + 7) / 8 * 8;
   }
-  if (!tile && (max_rows <= 0 || (r.M > max_rows && !daisy::proj_wanted(r.M, (int)pitch, r.K)))) return none();
+  if (!tile && (max_rows <= 0 || (r.M > max_rows && !daisy::proj_segments_wanted(r.M, (int)pitch, r.K)))) return none();
   Unlocked unlocked;
   Tensor y = empty({(int64_t)r.M, pitch}, at::kBFloat16, x);
   int64_t at = 0;
@@ -610,7 +610,7 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const uint16_t* W[kWeights];
   for (int i = 0; i < kWeights; ++i) W[i] = (const uint16_t*)ptr(w[i]);
   const int64_t pitch = (2 * kd + vd + 2 * Dv + H + 7) / 8 * 8, small = (2 * Dv + H + 7) / 8 * 8;
-  const bool rows_kernel = M <= max_rows, together = rows_kernel || daisy::proj_wanted((int)M, (int)pitch, (int)dim);
+  const bool rows_kernel = M <= max_rows, together = rows_kernel || daisy::proj_segments_wanted((int)M, (int)pitch, (int)dim);
   Tensor proj, big[3];
   daisy::ProjSegment seg[6];
   proj = empty({M, together ? pitch : small}, at::kBFloat16, x);

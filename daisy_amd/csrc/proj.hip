@@ -513,7 +513,15 @@ static int proj_tile(int M, int K, int head, COLUMNS columns, float* its_cost = 
 // (another read and write of every row, 62 us of 228 us at M = 32768, N = 3072, K = 1024).  That pass is a fixed price per
 // output and the library's lead grows with K: ahead at every M up to K = 1536 (whole layer, M = 32768: 640 against 655 us),
 // behind from K = 2048 on where the product is large (M = 32768: 1014 against 981 us; M = 8192: 251 against 257 us).
-bool proj_wanted(int M, int N, int K) { return K % 64 == 0 && N % 8 == 0 && (K <= 512 || (int64_t)M * N <= 4300000); }
+bool proj_segments_wanted(int M, int N, int K) { return K % 64 == 0 && N % 8 == 0 && (K <= 512 || (int64_t)M * N <= 4300000); }
+// One product also where its tiles of 128 x 128, of which two fit a compute unit, nearly fill one round: 384 to 512 of them.  Library / this, us:
+// 4096 x 1536 x 1536 21.9 / 21.8, 8192 x 768 x 768 14.5 / 13.1, 8192 x 1024 x 1024 19.6 / 16.8, 7000 x 1024 x 1024 18.9 / 17.0, 4096 x 2048 x 2048 32.3 / 30.8,
+// 1400 x 4608 x 1536 26.0 / 22.4; with fewer tiles either may be ahead (288: 16.7 / 12.7 and 13.3 / 13.7, 352: 25.4 / 28.5), with more the library is (516: 27.8 /
+// 36.3, 17.8 / 21.3).  K up to 2048 and M from 1000 are what was measured.
+bool proj_wanted(int M, int N, int K) {
+  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+  return proj_segments_wanted(M, N, K) || (K % 64 == 0 && N % 8 == 0 && K <= 2048 && M >= 1000 && tiles >= 384 && tiles <= 512);
+}
 bool proj_qkv_wanted(int M, int N, int K) { return K % 64 == 0 && (K <= 1536 || (int64_t)M * N <= 80000000); }
 
 template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI>

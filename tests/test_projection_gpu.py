@@ -70,6 +70,22 @@ def test_products_on_both_sides_of_the_smallest_tiles_rule(M):
             assert torch.equal(y, _lib.native().linear(x, w, None, 4, tile))
 
 
+@pytest.mark.parametrize("M,N,own", [(999, 6144, False), (1000, 6144, True), (6009, 1024, False), (6017, 1024, True), (8192, 1024, True), (8193, 1024, False)])
+def test_large_products_on_both_sides_of_the_rule(M, N, own):
+    """From 384 to 512 tiles of 128 x 128 and 1000 rows on; the few rows compared are the first, the last and some of every row of tiles."""
+    K = 576
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), torch.randn(N, K, generator=g).bfloat16()
+    with torch.no_grad():
+        y = _lib.native().linear(x.to(DEV), w.to(DEV), None, 4, 0)
+    assert (y is not None) == own
+    if own:
+        rows = torch.cat([torch.arange(0, M, 61), torch.tensor([M - 1])])
+        r = x[rows].double() @ w.double().t()
+        err = (y[rows.to(DEV)].cpu().double() - r).abs()
+        assert (err <= r.abs() * 2 ** -8 + K ** 0.5 * 1e-5 + 1e-3).all(), err.max().item()
+
+
 @pytest.mark.parametrize("H,D", [(2, 128), (6, 64), (3, 64)])
 @pytest.mark.parametrize("B,T", [(1, 5), (2, 64), (1, 129), (3, 200), (1, 1100)])
 @pytest.mark.parametrize("ve", [False, True])
