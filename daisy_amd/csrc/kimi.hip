@@ -49,6 +49,15 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvGroup group) {
   const int t0 = blockIdx.y * group.seg;
   const int t1 = min(t0 + group.seg, T);
 
+  // The rows ahead of the first step are asked for beside the weights, without a branch around any (ahead of the sequence: its first row, put
+  // right below): behind a branch each was waited for by itself, 6.6 -> 5.6 us for 3 x 235 rows of 3 x 512 channels.  (The first steps' rows
+  // with them: the same there, 32768 rows of 3 x 2048 channels 130.3 -> 132.3.)
+  constexpr int U = 8;   // steps whose inputs are in flight together
+  auto load_row = [&](int t) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.x + b * p.x_sb + (int64_t)t * p.x_st + c0)); };
+  u32x4 before[K - 1], raw[U];
+#pragma unroll
+  for (int j = 0; j < K - 1; ++j) before[j] = load_row(max(t0 - (K - 1) + j, 0));
+  __builtin_amdgcn_sched_barrier(0);
   float w[K][8], acc0[8];
   {
     // channel c's taps are K consecutive values; 8 channels = 8K consecutive bf16
@@ -85,11 +94,9 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvGroup group) {
       for (int j = 0; j < K; ++j) { carried[j][2 * v] = f[j % 8]; carried[j][2 * v + 1] = f[(4 + j) % 8]; }
     }
   }
-  // Input at time ti (may be negative: carried window or zero).
-  auto input_at = [&](int ti, float* f) {
-    if (ti >= 0) {
-      unpack8(__builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.x + b * p.x_sb + (int64_t)ti * p.x_st + c0)), f);
-    } else if (p.cache_in != nullptr) {
+  // Input at time ti < 0: carried window or zero.
+  auto input_ahead = [&](int ti, float* f) {
+    if (p.cache_in != nullptr) {
       if (K == 4) {
 #pragma unroll
         for (int j = 1; j < K; ++j)
@@ -109,15 +116,13 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvGroup group) {
 
   float win[K - 1][8];   // win[j] = input at t - (K-1) + j for the step t about to be computed
 #pragma unroll
-  for (int j = 0; j < K - 1; ++j) input_at(t0 - (K - 1) + j, win[j]);
-  constexpr int U = 8;   // steps whose inputs are in flight together
+  for (int j = 0; j < K - 1; ++j) {
+    unpack8(before[j], win[j]);
+    if (t0 - (K - 1) + j < 0) input_ahead(t0 - (K - 1) + j, win[j]);
+  }
   for (int tb = t0; tb < t1; tb += U) {
-    u32x4 raw[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int t = min(tb + u, T - 1);   // steps past the end re-read the last row and are not stored
-      raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.x + b * p.x_sb + (int64_t)t * p.x_st + c0));
-    }
+    for (int u = 0; u < U; ++u) raw[u] = load_row(min(tb + u, T - 1));
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       float xin[8], out[8];
@@ -144,7 +149,10 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvGroup group) {
   if (p.cache_out != nullptr && t1 == T) {
     float last[K][8];
 #pragma unroll
-    for (int j = 0; j < K; ++j) input_at(T - K + j, last[j]);
+    for (int j = 0; j < K; ++j) {
+      if (T - K + j >= 0) unpack8(load_row(T - K + j), last[j]);
+      else input_ahead(T - K + j, last[j]);
+    }
     if (K == 4) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
