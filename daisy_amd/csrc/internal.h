@@ -60,6 +60,7 @@ int linear_segments(const ProjSegment* seg, int n, int M, int K, hipStream_t s);
 // the library GEMM with qkv_prep_kernel behind it).
 bool proj_wanted(int M, int N, int K);              // one product
 bool proj_segments_wanted(int M, int N, int K);     // several, N columns in all
+bool proj_layer_wanted(int M, int N, int K);        // the KDA layer's six, N columns in all
 bool proj_qkv_wanted(int M, int N, int K);
 // The QKV projection of x [B * T, K] with its epilogue.
 int proj_qkv(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const QkvEpilogue& e,

@@ -610,7 +610,7 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const uint16_t* W[kWeights];
   for (int i = 0; i < kWeights; ++i) W[i] = (const uint16_t*)ptr(w[i]);
   const int64_t pitch = (2 * kd + vd + 2 * Dv + H + 7) / 8 * 8, small = (2 * Dv + H + 7) / 8 * 8;
-  const bool rows_kernel = M <= max_rows, together = rows_kernel || daisy::proj_segments_wanted((int)M, (int)pitch, (int)dim);
+  const bool rows_kernel = M <= max_rows, together = rows_kernel || daisy::proj_layer_wanted((int)M, (int)pitch, (int)dim);
   Tensor proj, big[3];
   daisy::ProjSegment seg[6];
   proj = empty({M, together ? pitch : small}, at::kBFloat16, x);
@@ -627,7 +627,12 @@ PyObject* py_kda_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (daisy::proj_segments(seg, 6, (int)M, (int)dim, s) != DAISY_OK) return none();
   } else {
     for (int i = 0; i < 3; ++i) {
-      big[i] = at::linear(x, *w[i]);
+      if (daisy::proj_wanted((int)M, (int)widths[i], (int)dim)) {
+        big[i] = empty({B, T, widths[i]}, at::kBFloat16, x);
+        if (!own_linear(r, W[i], dim, (int)widths[i], nullptr, (uint16_t*)ptr(big[i]), widths[i], max_rows, s)) return none();
+      } else {
+        big[i] = at::linear(x, *w[i]);
+      }
       seg[i].y = (uint16_t*)ptr(big[i]);
       seg[i].y_sm = widths[i];
     }

@@ -522,6 +522,12 @@ bool proj_wanted(int M, int N, int K) {
   const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
   return proj_segments_wanted(M, N, K) || (K % 64 == 0 && N % 8 == 0 && K <= 2048 && M >= 1000 && tiles >= 384 && tiles <= 512);
 }
+// A KDA layer's six products of the same rows, N columns in all, in one launch rather than the three large ones by themselves (this kernel's or
+// the library's) and the rest in another: one launch for four, and whole rounds of tiles for four that end in part of one.  Layers of 12 heads
+// of 64, 8, 12 and 16 of 128, us apart / in one: 3000 rows 128.4 / 114.0; 2300 137.1 / 119.9, 4100 206.6 / 185.1, 7000 (19 million) 282.3 / 276.7;
+// 900 104.9 / 93.2, 2800 210.6 / 182.4, 4900 (23 million) 277.9 / 271.5; 1280 148.8 / 126.0, 2300 220.9 / 190.1, 3700 (24 million) 281.9 / 276.0.  Beyond, either
+// may be ahead: 8 heads 8100 (26 million) 307 / 310, 9000 385 / 354; 16 heads 4090 (26 million) 296 / 301, 4400 353 / 325, 6000 409 / 422.
+bool proj_layer_wanted(int M, int N, int K) { return proj_segments_wanted(M, N, K) || (K % 64 == 0 && N % 8 == 0 && K <= 2048 && (int64_t)M * N <= 25000000); }
 bool proj_qkv_wanted(int M, int N, int K) { return K % 64 == 0 && (K <= 1536 || (int64_t)M * N <= 80000000); }
 
 template <int BM, int BN, int WVM, int WVN, int BK, int STAGES, int EPI>

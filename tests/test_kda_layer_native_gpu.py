@@ -120,6 +120,21 @@ def test_input_projections_of_a_layer_on_its_python_path(B, T, H, D, strided):
             assert ((y[:1, T // 3:].float() - alone.float()).norm() / alone.float().norm()).item() < 5e-3
 
 
+@pytest.mark.parametrize("B,T,H,D", [(1, 680, 16, 128), (2, 1031, 8, 128), (1, 3896, 16, 128), (1, 3897, 16, 128), (1, 5201, 12, 64), (1, 7700, 8, 128)])
+def test_input_projections_of_the_one_call_on_every_route(B, T, H, D, monkeypatch):
+    """The six products in one launch (up to 25 million columns and rows: 3896 rows of 16 heads of 128), and beyond it the large ones by
+    themselves, this library's (3897 rows) and the tensor library's (7700); against the layer's Python path."""
+    m = _layer(H, D, 1.0, 4, False)
+    x = torch.randn(B, T, H * D, generator=torch.Generator(device=DEV).manual_seed(T), device=DEV).bfloat16()
+    with torch.no_grad():
+        got = m._fast(x, False)
+        assert got is not None
+        monkeypatch.setattr(KimiLinearSelfAttention, "_fast", lambda self, *a: None)
+        ref = m(x, None)
+    # the same products with sums in another order ahead of their rounding to bf16, through the layer
+    assert ((got.float() - ref.float()).norm() / ref.float().norm()).item() < 5e-3
+
+
 @pytest.mark.parametrize("what", ["value width", "norm weight"])
 @torch.no_grad()
 def test_a_call_that_is_given_back_has_not_touched_the_states(what):
