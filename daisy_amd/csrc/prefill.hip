@@ -51,6 +51,7 @@ struct PrefillParams {
   int n_light;   // leading query blocks that see fewer keys than a full window (0 = order by block only)
   int order_shift;   // documents: query blocks in the order of their lengths, in units of 2^order_shift tiles; -1: by block
   int order_bit;     // the highest bit of such a length
+  int runs;          // prefill_split_kernel: neighbouring blocks to one XCD, else (batch, head) pairs in turn
   float scale_log2e;
 };
 
@@ -556,6 +557,10 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
     const int g = nbh >> 3, idx = blockIdx.x >> 3;
     bh = (blockIdx.x & 7) * g + idx % g;
     qb = nqb - 1 - idx / g;
+  } else if (p.runs) {               // an XCD takes a run of neighbouring blocks
+    const int runs = (nbh * nqb) & ~7, i = blockIdx.x, at = i < runs ? (i & 7) * (runs >> 3) + (i >> 3) : i;
+    bh = at / nqb;
+    qb = nqb - 1 - at % nqb;
   } else {
     bh = blockIdx.x % nbh;
     qb = nqb - 1 - blockIdx.x / nbh;
@@ -861,16 +866,32 @@ __global__ __launch_bounds__(64) void prefill_scalar_kernel(PrefillParams p) {
   }
 }
 
-// Up to how many blocks of 128 queries the kernel with four wavefronts per 32 queries is the faster one.  From a sweep
-// over B * H = 4 ... 64, T = 64 ... 8192, windows of 128, 1024 and 8192, both head dims: 1.4 to 2.4 times as fast
+// Up to how many blocks of 128 queries the kernel with four wavefronts per 32 queries is the faster one.  From sweeps
+// over B * H = 4 ... 64, T = 64 ... 30000, windows of 128 to 8192 and none, two to nine documents, both head dims: 1.4 to 2.4 times as fast
 // while the blocks leave compute units idle (12 heads of 128, T = 777: 19.4 -> 11.0 us; 8 heads of 64, T = 2048:
-// 32.7 -> 14.4 us), level at the limits below and slower beyond (it fetches every key tile four times as often).  Full
-// causal blocks differ in length, which favours it longer than windowed ones; wide heads less than narrow ones.
+// 32.7 -> 14.4 us), level at the limits below and slower beyond (it fetches every key tile four times as often).  Blocks of different lengths, full
+// causal or in documents, favour it longer than those of a window; wide heads less than narrow ones.  us, 128 queries / 32 (blocks of 128):
+// heads of 128, windows: 1600 rows x 16 heads (208), 200 / 800 keys 14.6 / 13.6, 24.9 / 21.6; 5 x 700 x 8 (240), 400 18.0 / 16.2; 2000 x 16 (256), 400 / 800 18.5 /
+// 19.7, 25.2 / 24.1; 6000 x 6 (282), 800 29.8 / 37.0; half of the row or more: 2 x 5000 x 4 (320), 4096 88 / 78, 3000 x 12 (288), 1500 42.0 / 41.5; documents: 4283 x 6
+// (204) 44 / 31, 7000 x 8 (440), four 73.6 / 53.6, with 1500 keys 60 / 61 and 59 / 52 (two, four; but bounds may also be a mask that reaches 1500 keys back everywhere: 320 for these), with 500 30 / 39; 16000 x 4 (500), four 155 / 114, with 1500 71 / 76; 5000 x 16 (640), four 58 / 61.
+// Heads of 64, windows: 12000 x 4 (376), 200 / 1500 14.6 / 11.8, 35.8 / 33.5; 10 x 700 x 8 (480), 200 / 400 14.3 / 12.3, 14.8 / 14.9; 5000 x 12 (480), 1500 37 / 42;
+// documents: 4000 x 16 (512), three 37 / 27, 5000 x 16 (640), four 38.9 / 32.6, with 1500 36.6 / 32.5, with 500 24.6 / 25.2; 8000 x 16 (1008) 64 / 69.
 template <int D>
 static int64_t split_limit(const PrefillParams& p) {
-  const bool full = p.doc_start == nullptr && (p.window <= 0 || p.window >= p.T);
-  if (D == 64) return full ? 768 : 320;
-  return full && p.T >= 1024 ? 384 : p.window <= 0 || p.window >= 1024 ? 192 : 144;
+  const bool windowed = p.window > 0 && p.window < p.T, docs = p.doc_start != nullptr;
+  if (docs && (!windowed || p.window >= 1024)) return D == 64 ? 700 : !windowed || p.window >= 4096 ? 512 : 320;
+  if (!windowed) return D == 64 ? 768 : p.T >= 1024 ? 384 : 288;
+  if (D == 64) return 448;
+  return 2 * (int64_t)p.window >= p.T ? 320 : p.window >= 600 ? 256 : 240;
+}
+// Its (batch, head) pairs, where they are no multiple of eight, go round the XCDs in turn, so that an XCD meets pairs / gcd(pairs, 8) of them.  When the keys
+// and values of those leave its L2 (4 MB) and a window makes blocks equally long, it takes a run of neighbouring blocks instead: 4000 rows, 5
+// heads of 128 (10 MB), window 200 / 800 / 1500 18.1 / 34.7 / 42.5 -> 13.0 / 22.8 / 33.9 us; 4283 rows, 6 heads (6.6 MB), 200 / 1500 19.2 / 37.9 -> 14.9 / 37.5; but 3000
+// rows, 12 heads (4.6 MB), 1500 41.5 -> 45.7.
+static bool runs_of_blocks(const PrefillParams& p) {
+  const int pairs = p.B * p.H, eighth = pairs & -pairs;              // (the largest power of two in it)
+  if (p.doc_start != nullptr || p.window <= 0 || 2 * (int64_t)p.window > p.T || eighth >= 8) return false;
+  return (int64_t)(pairs / eighth) * p.T * p.D * 4 > (5 << 20);
 }
 
 // When those are eight wavefronts: while a compute unit has no second workgroup to run and the longest block has more key tiles than four of them
@@ -908,6 +929,7 @@ static int launch_mfma(PrefillParams p, hipStream_t s) {
   }
   if (nwg <= split_limit<D>(p)) {
     const int64_t nsw = (int64_t)((p.T + 31) / 32) * p.H * p.B;
+    p.runs = runs_of_blocks(p);
     if (eight_wavefronts<D>(p, nsw)) hipLaunchKernelGGL((prefill_split_kernel<D, 8>), dim3((unsigned)nsw), dim3(512), 0, s, p);
     else hipLaunchKernelGGL((prefill_split_kernel<D, 4>), dim3((unsigned)nsw), dim3(kPrefillThreads), 0, s, p);
     DAISY_CHECK_LAUNCH("prefill_split_kernel");
