@@ -207,7 +207,7 @@ def test_rotated_keys_are_the_oracles_bits(D, H, B, T):
 @pytest.mark.parametrize("T,H,D,window,docs", [
     (4001, 5, 128, 200, 0), (4100, 3, 128, 1500, 0), (6500, 5, 64, 130, 0), (4224, 6, 128, 129, 0),   # runs of blocks, their remainder among them
     (2048, 15, 128, 300, 0), (2049, 15, 128, 300, 0), (2048, 16, 128, 600, 0), (5120, 8, 128, 2560, 0), (5121, 8, 128, 2560, 0),
-    (7168, 8, 64, 200, 0), (7169, 8, 64, 200, 0),
+    (7168, 8, 64, 200, 0), (7169, 8, 64, 200, 0), (3100, 13, 128, 200, 0), (5000, 13, 64, 700, 0), (2700, 12, 128, 1300, 0),
     (5120, 8, 128, None, 3), (8192, 8, 128, 4096, 3), (8193, 8, 128, 4096, 3), (5120, 8, 128, 1100, 3), (5121, 8, 128, 1100, 3),
     (5600, 16, 64, None, 3), (5633, 16, 64, None, 3),
 ])
