@@ -130,9 +130,24 @@ __device__ __forceinline__ void workgroup_to_block(const PrefillParams& p, int* 
   // Pairs that are no multiple of eight: an XCD takes a run of neighbouring blocks with a full window (the shorter ones fill the tail as they come).  Dealt to
   // the XCDs one by one, every L2 fetched every key: 3 x 5000 rows, 12 heads of 128, window 800 98.9 -> 80.7 us; 16384 rows, 12 heads, 1024 127.8 -> 118.8,
   // 4096 335 -> 332; 60000 rows, 4 heads, 1427 196.7 -> 185.9; heads of 64, 30000 rows, 12 heads, 1000 126.4 -> 115.1, but 20000 rows, 4 heads, 4096 95.1 / 96.6.
+  // Of documents under a short window each XCD takes an eighth of every pair's full-window blocks, of each pair another one, because documents make parts of a
+  // row cheap: 16384 rows, 12 heads, window 1024, six documents / one 121.9 / 125.9 -> 106.1 / 108.0 us, half the row in documents of 200 96.1 -> 82.6; 20000 rows, 10
+  // heads, 2000 186.7 / 196.4 -> 178.1 / 192.1; 30000 rows, 4 heads, 1000 98.6 / 99.0 -> 79.7 / 75.5; heads of 64, 60000 rows, 4 heads, 1024 89.5 / 94.1 -> 77.8 / 81.9.
+  // (Runs of an eighth of all blocks: 30000 rows, 4 heads, 2000, half in short ones 84.9 -> 111.9.)  Fewer pairs cannot make up for a cheap part (4 heads, 3072
+  // 169.9 -> 193.1; two, 1000 61.9 -> 73.6), nor can blocks that all run at once (7 heads, 14200 rows, 1500 63.5 -> 70.7; 5, 9000, 1000 42.7 -> 45.2;
+  // three fit a compute unit, four of heads of 64).
   if ((nbh & 7) != 0 && p.period > 0 && p.doc_start == nullptr && p.window < 64 * p.D) {
     const int runs = (nbh * n_full) & ~7;
     if (idx < runs) idx = (idx & 7) * (runs >> 3) + (idx >> 3);
+  } else if ((nbh & 7) != 0 && nbh >= 4 && p.period > 0 && p.doc_start != nullptr && p.order_shift < 0 && p.window <= (nbh >= 8 ? 2048 : 1024) && nbh * p.nqb > (p.D == 64 ? 1024 : 768)) {
+    const int m = n_full >> 3, rest = n_full & 7, runs = nbh * m * 8;
+    if (idx < runs) {
+      const int pair = (idx >> 3) / m, turn = (pair & 1) * 4 + (pair & 2) + (pair >> 2 & 1);
+      idx = pair * n_full + ((idx + turn) & 7) * m + (idx >> 3) % m;
+    } else if (idx < nbh * n_full) {
+      idx -= runs;
+      idx = idx / rest * n_full + 8 * m + idx % rest;
+    }
   }
   // (a lone document, which the last row's bound shows, leaves a window's blocks equally long: T = 16384, window 2048, 8 heads of
   // 128: 145.2 us by length, 142.6 us without, as without documents; one scalar load, which several documents do not feel)

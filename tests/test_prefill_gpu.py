@@ -210,6 +210,7 @@ def test_rotated_keys_are_the_oracles_bits(D, H, B, T):
     (7168, 8, 64, 200, 0), (7169, 8, 64, 200, 0), (3100, 13, 128, 200, 0), (5000, 13, 64, 700, 0), (2700, 12, 128, 1300, 0),
     (5120, 8, 128, None, 3), (8192, 8, 128, 4096, 3), (8193, 8, 128, 4096, 3), (5120, 8, 128, 1100, 3), (5121, 8, 128, 1100, 3),
     (5600, 16, 64, None, 3), (5633, 16, 64, None, 3),
+    (7700, 13, 128, 200, 3), (7400, 14, 128, 200, 3), (12000, 12, 64, 1000, 3), (1000, 110, 128, 120, 3),      # eighths of a pair, with and without a remainder, none
 ])
 def test_prefill_on_both_sides_of_the_block_size_rule(T, H, D, window, docs):
     """Sizes around the numbers of blocks at which the kernel with 32 queries per workgroup hands over to the one with 128, and pairs
