@@ -251,7 +251,7 @@ __device__ __forceinline__ u32x2 lds_read_tr16_as3(lds_u16_ptr p) {
 
 // Main kernel (keys already rotated, or no RoPE on keys).  32-key tiles, and nothing of a step is
 // overlapped inside a wavefront: scores, softmax and the product of one tile follow each other.  The
-// kernel is small instead -- 167 VGPRs and 48 KiB of LDS at D = 128 -- so that THREE workgroups fit a
+// kernel is small instead -- 158 VGPRs and 48 KiB of LDS at D = 128 -- so that THREE workgroups fit a
 // CU, three wavefronts a SIMD, and the latencies of one wavefront's step (the issue of its tile
 // copies, the LDS operand reads, the softmax chain, the barrier) are covered by the other two: matrix
 // instructions of one wavefront and vector instructions of another do run side by side on a SIMD.
