@@ -786,7 +786,10 @@ __global__ __launch_bounds__(256) void rope_k_kernel(PrefillParams p) {
   constexpr int HALF = D / 2, CPR = D / 8;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int HG = p.H / HPT;
-  const int64_t rows = (int64_t)p.B * p.T * HG, row = min(idx / CPR, rows - 1);     // (surplus lanes redo the last row: whole rows exchange)
+  // Surplus lanes read the last row as well, since whole rows exchange, and store nothing: k_out may be k, and another wavefront's lanes
+  // own that row.
+  const int64_t rows = (int64_t)p.B * p.T * HG, row = min(idx / CPR, rows - 1);
+  const bool live = idx / CPR < rows;
   const int ch = (int)(idx % CPR), hg = (int)(row % HG), t = (int)(row / HG % p.T), b = (int)(row / HG / p.T);
   u32x4 own[HPT];
   // The unrotated keys are not needed again: read them past the caches, so that q, v and the
@@ -814,7 +817,7 @@ __global__ __launch_bounds__(256) void rope_k_kernel(PrefillParams p) {
     unpack8(other, o);
 #pragma unroll
     for (int e = 0; e < 8; ++e) y[e] = lower ? rope_lo(x[e], o[e], c[e], sn[e]) : rope_hi(o[e], x[e], c[e], sn[e]);
-    *reinterpret_cast<u32x4*>(p.k_out + b * p.ko_sb + (int64_t)t * p.ko_st + (hg + j * HG) * p.ko_sh + 8 * ch) = pack8(y);
+    if (live) *reinterpret_cast<u32x4*>(p.k_out + b * p.ko_sb + (int64_t)t * p.ko_st + (hg + j * HG) * p.ko_sh + 8 * ch) = pack8(y);
   }
 }
 

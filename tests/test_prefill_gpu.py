@@ -204,6 +204,23 @@ def test_rotated_keys_are_the_oracles_bits(D, H, B, T):
     assert torch.equal(kr.cpu(), oracle.apply_rope(k, cos, sin))
 
 
+@pytest.mark.parametrize("D,H,T,surplus", [(128, 12, 45, 0), (128, 12, 42, 1), (128, 12, 44, 2), (128, 12, 43, 3), (128, 3, 89, 1), (128, 3, 86, 3),
+                                           (64, 12, 170, 0), (64, 12, 177, 1), (64, 12, 174, 2), (64, 12, 171, 3), (64, 6, 171, 3), (64, 1, 513, 3)])
+@pytest.mark.parametrize("pad", [0, 8])
+def test_keys_rotated_in_place(D, H, T, surplus, pad):
+    """``k_out`` is ``k``: every row is rotated once, by the lanes that own it.  A lane takes 16 bytes of one, two or four heads; lengths that
+    leave none to three whole wavefronts of the last workgroup without rows."""
+    heads = 4 if D == 64 and H % 4 == 0 else 2 if H % 2 == 0 else 1
+    assert -(T * H // heads * D // 8) % 256 // 64 == surplus
+    q, k, v = _inputs(1, T, H, D, seed=T + H)
+    cos, sin = oracle.rope_tables(D, T)
+    kd = torch.zeros(1, T, H, D + pad, dtype=torch.bfloat16, device="cuda")[..., :D].copy_(k)
+    o_ref, k_ref = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), window=None, cos=cos.cuda(), sin=sin.cuda())
+    o, kr = ops.prefill_attention(q.cuda(), kd, v.cuda(), window=None, cos=cos.cuda(), sin=sin.cuda(), k_out=kd)
+    assert kr.data_ptr() == kd.data_ptr()
+    assert torch.equal(kr.cpu(), oracle.apply_rope(k, cos, sin)) and torch.equal(kr, k_ref) and torch.equal(o, o_ref)
+
+
 @pytest.mark.parametrize("T,H,D,window,docs", [
     (4001, 5, 128, 200, 0), (4100, 3, 128, 1500, 0), (6500, 5, 64, 130, 0), (4224, 6, 128, 129, 0),   # runs of blocks, their remainder among them
     (2048, 15, 128, 300, 0), (2049, 15, 128, 300, 0), (2048, 16, 128, 600, 0), (5120, 8, 128, 2560, 0), (5121, 8, 128, 2560, 0),
