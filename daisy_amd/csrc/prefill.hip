@@ -33,6 +33,7 @@
 // Algorithmic work: 4*D flops per visible (query, key) pair.
 #include "common.h"
 
+#include <cfloat>
 #include <type_traits>
 
 namespace daisy {
@@ -186,14 +187,17 @@ __device__ __forceinline__ float pair_sum(float x) {
 // Online softmax of a tile (log2 domain): its probabilities as operands, against the wavefront's reference maxima, which move only
 // when some query's share of the tile's sum exceeds kMost.  Until then no probability does, which bf16 and the fp32 sums hold
 // without loss, and neither the tile's maxima are looked for nor is O touched: the scores' exponentials come straight behind their
-// products.  A reference that is not set yet (no key of that query seen) takes the long way too.  The tile kernels are bound by their vector
+// products.  A query that has seen no key has -FLT_MAX for a reference: what it does not see stays 0, its first key overflows the sum and sets it.  (Behind
+// a document's start the queries of a wavefront wait through every tile of the document ahead.  While any of them did, each tile took the long way: 20000
+// rows in seven documents, 4 heads of 128 172 us, 24545 in twenty, 8 heads 211, 5900 in three, 16 of 64 52.4; now 149, 186 and 49.8, with the maxima of every tile
+// 147, 185 and 49.2.)  A wavefront's first tile takes it at once, so that short rows do not work out its exponentials twice.  The tile kernels are bound by their vector
 // instructions (head dim 64: 855 cycles of them per 64 keys against 512 of the matrix pipe) and by power, which fewer of them
 // spare: with the maxima of every tile worked out and compared (a reference moved at 2^8) 65536 rows, 16 heads of 128, full causal took 15.00 ms, now
 // 14.56; 20001 rows in seven documents, 16 heads of 64, 178.6 us, now 171.4; a layer of 8 x 4096 rows, 8 heads of 128, window 1024, 406.2 and 403.8.
 struct SoftmaxRef {
-  float m = -INFINITY, minus = 0.f;   // reference (scaled), the same in both lanes of a query; what is added to the scaled scores
-  float l = 0.f;                      // this lane's share of the running sum
-  bool unset = true;                  // some query of the wavefront has no reference
+  float minus = FLT_MAX;   // less the reference (scaled), the same in both lanes of a query: what is added to the scaled scores
+  float l = 0.f;           // this lane's share of the running sum
+  bool first = true;       // the wavefront has seen no tile
 };
 constexpr float kMost = 4096.f;
 template <int SUB, int NDT>
@@ -213,24 +217,21 @@ __device__ __forceinline__ void softmax_tile(const f32x16 (&sacc)[SUB], float sc
       pfrag[m] = __builtin_bit_cast(bf16x8, pack8(pv));
     }
   };
-  bool longer = ref.unset;
-  if (!longer) {
+  bool moves = ref.first;
+  if (!moves) {
     exponentials();
-    longer = __builtin_amdgcn_ballot_w64(lsum > kMost) != 0;
+    moves = __builtin_amdgcn_ballot_w64(lsum > kMost) != 0;
   }
-  if (longer) {
+  if (moves) {
+    ref.first = false;
     float mt = -INFINITY;
 #pragma unroll
     for (int u = 0; u < SUB; ++u)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[u][r]);
     mt = pair_max(mt) * scale_log2e;
-    const float m_new = fmaxf(ref.m, mt);
-    const float mu = (m_new == -INFINITY) ? 0.f : m_new;
-    const float alpha = fast_exp2(ref.m - mu);
-    ref.m = m_new;
-    ref.minus = -mu;
-    ref.unset = __builtin_amdgcn_ballot_w64(m_new == -INFINITY) != 0;
+    const float minus = fminf(ref.minus, -mt), alpha = fast_exp2(minus - ref.minus);
+    ref.minus = minus;
     ref.l *= alpha;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
@@ -732,7 +733,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
   // Partial results: each lane of a pair holds its share of the row sum; O^T as [query][channel] fp32 in the
   // wavefront's own tile area, 16-byte pieces swizzled by the query.
   const float l_tot = pair_sum(ref.l);
-  if (lh == 0) { part_m[wave][lq] = ref.m; part_l[wave][lq] = l_tot; }
+  if (lh == 0) { part_m[wave][lq] = -ref.minus; part_l[wave][lq] = l_tot; }
   float* const po = reinterpret_cast<float*>(&tiles[wave][0][0]);
   constexpr int PC = D / 4;
 #pragma unroll
@@ -752,13 +753,12 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
     float m = part_m[0][row];
 #pragma unroll
     for (int w = 1; w < W; ++w) m = fmaxf(m, part_m[w][row]);
-    const float mu = (m == -INFINITY) ? 0.f : m;
     float l = 0.f, acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;
 #pragma unroll
     for (int w = 0; w < W; ++w) {
-      const float a = fast_exp2(part_m[w][row] - mu);
+      const float a = fast_exp2(part_m[w][row] - m);
       l = fmaf(part_l[w][row], a, l);
       const float* src = reinterpret_cast<const float*>(&tiles[w][0][0]) + row * D;
 #pragma unroll

@@ -82,6 +82,27 @@ def test_prefill_one_key_above_the_reference(D, above, at):
 
 
 @pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("window", [None, 200])
+@pytest.mark.parametrize("levels", [(0.0, 200.0, -200.0, 140.0, -140.0), (-300.0, 300.0, 0.0, -13.0, 11.0)])
+def test_prefill_documents_that_start_inside_a_wavefront(D, window, levels):
+    """Queries on both sides of a document's start in one wavefront: those behind it have no reference while the tiles of the document
+    ahead pass, and get one at their first key, however far their scores (of one level per document, in log2 units) lie from 0."""
+    T, H, starts = 700, 2, (0, 45, 333, 334, 499)
+    g = torch.Generator().manual_seed(D)
+    q, k = (0.3 * torch.randn(1, T, H, D, generator=g) for _ in range(2))
+    q[..., 3] = 4.0
+    doc_start = torch.zeros(T, dtype=torch.int32)
+    for at, level in zip(starts, levels):
+        k[:, at:, :, 3] = level / LOG2E / 4.0
+        doc_start[at:] = at
+    q, k, v = q.bfloat16(), k.bfloat16(), torch.randn(1, T, H, D, generator=g).bfloat16()
+    ref = oracle.windowed_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), window, 1.0, doc_start).transpose(1, 2)
+    o, _ = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), window=window, scale=1.0, doc_start=doc_start.cuda())
+    assert_close_bf16(o, ref, "o")
+    check_prefill_of_many_heads(q.cuda(), k.cuda(), v.cuda(), ref, "documents", window=window, scale=1.0, doc_start=doc_start.cuda())
+
+
+@pytest.mark.parametrize("D", [64, 128])
 def test_prefill_large_logits_with_rotation_and_documents(D):
     """The same with RoPE in the call and document bounds (masked tiles take the same softmax path)."""
     B, T, H, W = 2, 515, 2, 300
