@@ -190,7 +190,11 @@ __device__ __forceinline__ float pair_sum(float x) {
 // products.  A query that has seen no key has -FLT_MAX for a reference: what it does not see stays 0, its first key overflows the sum and sets it.  (Behind
 // a document's start the queries of a wavefront wait through every tile of the document ahead.  While any of them did, each tile took the long way: 20000
 // rows in seven documents, 4 heads of 128 172 us, 24545 in twenty, 8 heads 211, 5900 in three, 16 of 64 52.4; now 149, 186 and 49.8, with the maxima of every tile
-// 147, 185 and 49.2.)  A wavefront's first tile takes it at once, so that short rows do not work out its exponentials twice.  The tile kernels are bound by their vector
+// 147, 185 and 49.2.)  
+// FIRST: a wavefront's first tile takes the long way at once, so that short rows do not work out its exponentials twice; the branch costs the tile
+// kernel for heads of 128 more where it is bound by latency, two or three blocks to a compute unit: 9000 rows, 8 heads 202.5 us with the maxima of every
+// tile, 208.7 with the branch, 203.8 without; 20000 in documents that start with a block, 4 heads 113.5, 115.8, 114.6.  (Heads of 64 need it: 128 registers
+// do not hold both ends of the block that the products and the exponentials then share.)  The tile kernels are bound by their vector
 // instructions (head dim 64: 855 cycles of them per 64 keys against 512 of the matrix pipe) and by power, which fewer of them
 // spare: with the maxima of every tile worked out and compared (a reference moved at 2^8) 65536 rows, 16 heads of 128, full causal took 15.00 ms, now
 // 14.56; 20001 rows in seven documents, 16 heads of 64, 178.6 us, now 171.4; a layer of 8 x 4096 rows, 8 heads of 128, window 1024, 406.2 and 403.8.
@@ -200,7 +204,7 @@ struct SoftmaxRef {
   bool first = true;       // the wavefront has seen no tile
 };
 constexpr float kMost = 4096.f;
-template <int SUB, int NDT>
+template <bool FIRST, int SUB, int NDT>
 __device__ __forceinline__ void softmax_tile(const f32x16 (&sacc)[SUB], float scale_log2e, SoftmaxRef& ref, f32x16 (&oacc)[NDT],
                                              bf16x8 (&pfrag)[2 * SUB]) {
   float lsum;
@@ -217,7 +221,7 @@ __device__ __forceinline__ void softmax_tile(const f32x16 (&sacc)[SUB], float sc
       pfrag[m] = __builtin_bit_cast(bf16x8, pack8(pv));
     }
   };
-  bool moves = ref.first;
+  bool moves = FIRST && ref.first;
   if (!moves) {
     exponentials();
     moves = __builtin_amdgcn_ballot_w64(lsum > kMost) != 0;
@@ -485,7 +489,7 @@ __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
         }
     }
     bf16x8 pfrag[2 * SUB];
-    softmax_tile<SUB, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
+    softmax_tile<D == 64, SUB, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
     // O^T += V^T P^T
 #pragma unroll
     for (int m = 0; m < 2 * SUB; ++m) {
@@ -710,7 +714,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
       }
     }
     bf16x8 pfrag[2];
-    softmax_tile<1, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
+    softmax_tile<true, 1, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
     // V(n) has landed when only K(n + 1)'s copies are outstanding
     if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | NCP);
     else __builtin_amdgcn_s_waitcnt(0x0F70);
