@@ -31,6 +31,8 @@ struct QkvEpilogue {
   float eps;
 };
 
+// Whether prefill attention of so many (batch, head) pairs takes the kernel with 32 queries per workgroup.
+bool prefill_split_wanted(int pairs, int T, int D, int window, bool docs);
 // y [M, N] = x [M, K] w [N, K]^T (+ bias), fp32 accumulation, one rounding.  tile: 0 = by the sizes.
 int proj_linear(const uint16_t* x, int64_t x_sm, const uint16_t* w, int64_t w_sn, const uint16_t* bias,
                 uint16_t* y, int64_t y_sm, int M, int N, int K, hipStream_t s, int tile = 0);

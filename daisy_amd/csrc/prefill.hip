@@ -33,6 +33,7 @@
 // Algorithmic work: 4*D flops per visible (query, key) pair.
 #include "common.h"
 
+#include <algorithm>
 #include <cfloat>
 #include <type_traits>
 
@@ -895,32 +896,44 @@ __global__ __launch_bounds__(64) void prefill_scalar_kernel(PrefillParams p) {
   }
 }
 
-// Up to how many blocks of 128 queries the kernel with four wavefronts per 32 queries is the faster one.  From sweeps
-// over B * H = 4 ... 64, T = 64 ... 30000, windows of 128 to 8192 and none, two to nine documents, both head dims: 1.4 to 2.4 times as fast
+// Bytes of keys and values that an XCD meets in the kernel with 32 queries per workgroup, whose (batch, head) pairs go round the XCDs in turn:
+// those of pairs / gcd(pairs, 8) of them, which find their blocks' neighbours in its L2 (4 MB) or not.
+static int64_t met_bytes(int pairs, int T, int D) { return (int64_t)pairs / std::min(pairs & -pairs, 8) * T * D * 4; }
+constexpr int64_t kMetBytes = 5 << 20;
+// Whether the kernel with four wavefronts per 32 queries is the faster one: up to so many blocks of 128 queries.  It is 1.4 to 2.4 times as fast
 // while the blocks leave compute units idle (12 heads of 128, T = 777: 19.4 -> 11.0 us; 8 heads of 64, T = 2048:
-// 32.7 -> 14.4 us), level at the limits below and slower beyond (it fetches every key tile four times as often).  Blocks of different lengths, full
-// causal or in documents, favour it longer than those of a window; wide heads less than narrow ones.  us, 128 queries / 32 (blocks of 128):
-// heads of 128, windows: 1600 rows x 16 heads (208), 200 / 800 keys 14.6 / 13.6, 24.9 / 21.6; 5 x 700 x 8 (240), 400 18.0 / 16.2; 2000 x 16 (256), 400 / 800 18.5 /
-// 19.7, 25.2 / 24.1; 6000 x 6 (282), 800 29.8 / 37.0; half of the row or more: 2 x 5000 x 4 (320), 4096 88 / 78, 3000 x 12 (288), 1500 42.0 / 41.5; documents: 4283 x 6
-// (204) 44 / 31, 7000 x 8 (440), four 73.6 / 53.6, with 1500 keys 60 / 61 and 59 / 52 (two, four; but bounds may also be a mask that reaches 1500 keys back everywhere: 320 for these), with 500 30 / 39; 16000 x 4 (500), four 155 / 114, with 1500 71 / 76; 5000 x 16 (640), four 58 / 61.
-// Heads of 64, windows: 12000 x 4 (376), 200 / 1500 14.6 / 11.8, 35.8 / 33.5; 10 x 700 x 8 (480), 200 / 400 14.3 / 12.3, 14.8 / 14.9; 5000 x 12 (480), 1500 37 / 42;
-// documents: 4000 x 16 (512), three 37 / 27, 5000 x 16 (640), four 38.9 / 32.6, with 1500 36.6 / 32.5, with 500 24.6 / 25.2; 8000 x 16 (1008) 64 / 69.
-template <int D>
-static int64_t split_limit(const PrefillParams& p) {
-  const bool windowed = p.window > 0 && p.window < p.T, docs = p.doc_start != nullptr;
-  if (docs && (!windowed || p.window >= 1024)) return D == 64 ? 700 : !windowed || p.window >= 4096 ? 512 : 320;
-  if (!windowed) return D == 64 ? 768 : p.T >= 1024 ? 384 : 288;
-  if (D == 64) return 448;
-  return 2 * (int64_t)p.window >= p.T ? 320 : p.window >= 600 ? 256 : 240;
+// 32.7 -> 14.4 us) and slower beyond (it fetches every key tile four times as often).  From sweeps over 3 to 24 (batch, head) pairs, 145 to 780
+// blocks, windows of 120 to 8192 and none, one to hundreds of documents.  us, 128 queries / 32 (heads x rows, blocks of 128):
+// Documents, whose lengths the host does not know.  Heads of 128: 12 x 3000 (288) in documents of 20 to 200 tokens 17.7 / 18.0, 200 to 900 32.3 / 23.0, one 68.9 /
+// 51.2; 8 x 5100 (320) likewise 18.2 / 20.0, 30.3 / 27.4, 109 / 80; 8 x 8100 (512) 18.5 / 27.4, 34.0 / 40.2, 184 / 181: to 288, from where short ones lose, though long ones
+// gain for longer.  With a window under 1024, 8 x 3100 (200), 400 keys 22.4 / 17.8, 8 x 4096 (256) 20.9 / 22.1.  Heads of 64: 12 x 5000 (480) 14.4 / 13.1,
+// 21.6 / 18.9; 8 x 8100 (512), 1500 keys 23.9 / 21.9, but one document, a window's mask, 35.7 / 39.6; 24 x 3670 (696) two 39.6 / 43.9.
+// Keys past an XCD's L2 and no runs of blocks (below) to help, that is documents, or a window of more than a fourth of the row: heads of 128: 7 x 4000 (224), 1500
+// keys, one document 41.0 / 59.7, no window 84.5 / 52.1; 5 x 6000 (235), 1500 keys 41.3 / 67.9, no window, documents of 20 to 200 17.2 / 18.0; 7 x 8000 (441), 4096 keys 102 / 227.
+// Heads of 64: 5 x 9000 (355), 4096 keys 57.5 / 68.6; 9 x 4816 (342), 2017 32.8 / 37.9; no window, 9 x 6884 (486) one document 92.2 / 95.2, 7 x 8000 (441) documents of 200 to
+// 900 25.9 / 23.2.
+// Windows, heads of 128: 8 x 3100 (200), 150 / 400 keys 14.7 / 13.9, 19.7 / 17.8, but 4 x 6472 (204), 236 16.9 / 19.1, 12 x 2491 (240), 438 20.4 / 21.7; 2000 x 16 (256), 800 25.2 /
+// 24.1; half of the row or more: 3000 x 12 (288), 1500 42.0 / 41.5, 2 x 5000 x 4 (320), 4096 88 / 78.  Heads of 64: 12000 x 4 (376), 200 / 1500 14.6 / 11.8, 35.8 / 33.5; 10 x 700 x 8
+// (480), 400 14.8 / 14.9; 5000 x 12 (480), 1500 37 / 42.
+bool prefill_split_wanted(int pairs, int T, int D, int window, bool docs) {
+  const bool windowed = window > 0 && window < T, far = !windowed || window >= 1024;
+  const bool near = met_bytes(pairs, T, D) <= kMetBytes || (!docs && 4 * (int64_t)window <= T);
+  int64_t limit;
+  if (!windowed && !docs) limit = D == 64 ? 768 : T >= 1024 ? 384 : 288;
+  else if (D == 64) limit = near ? (docs && far ? 500 : 448) : windowed ? 320 : 440;
+  else if (windowed && window < 600) limit = pairs % 8 == 0 ? 208 : 144;
+  else if (!near) limit = windowed ? 192 : 224;
+  else if (docs) limit = far ? 288 : 208;
+  else limit = 2 * (int64_t)window >= T ? 320 : 256;
+  return (int64_t)pairs * ((T + kBM - 1) / kBM) <= limit;
 }
-// Its (batch, head) pairs, where they are no multiple of eight, go round the XCDs in turn, so that an XCD meets pairs / gcd(pairs, 8) of them.  When the keys
-// and values of those leave its L2 (4 MB) and a window makes blocks equally long, it takes a run of neighbouring blocks instead: 4000 rows, 5
+// When the keys and values that an XCD meets leave its L2 and a window makes blocks equally long, it takes a run of neighbouring blocks instead: 4000 rows, 5
 // heads of 128 (10 MB), window 200 / 800 / 1500 18.1 / 34.7 / 42.5 -> 13.0 / 22.8 / 33.9 us; 4283 rows, 6 heads (6.6 MB), 200 / 1500 19.2 / 37.9 -> 14.9 / 37.5; but 3000
 // rows, 12 heads (4.6 MB), 1500 41.5 -> 45.7.
 static bool runs_of_blocks(const PrefillParams& p) {
-  const int pairs = p.B * p.H, eighth = pairs & -pairs;              // (the largest power of two in it)
-  if (p.doc_start != nullptr || p.window <= 0 || 2 * (int64_t)p.window > p.T || eighth >= 8) return false;
-  return (int64_t)(pairs / eighth) * p.T * p.D * 4 > (5 << 20);
+  const int pairs = p.B * p.H;
+  if (p.doc_start != nullptr || p.window <= 0 || 2 * (int64_t)p.window > p.T || pairs % 8 == 0) return false;
+  return met_bytes(pairs, p.T, p.D) > kMetBytes;
 }
 
 // When those are eight wavefronts: while a compute unit has no second workgroup to run and the longest block has more key tiles than four of them
@@ -956,7 +969,7 @@ static int launch_mfma(PrefillParams p, hipStream_t s) {
     DAISY_CHECK_LAUNCH("rope_k_kernel");
     p.k = p.k_out; p.k_sb = p.ko_sb; p.k_st = p.ko_st; p.k_sh = p.ko_sh;
   }
-  if (nwg <= split_limit<D>(p)) {
+  if (prefill_split_wanted(p.B * p.H, p.T, D, p.window, p.doc_start != nullptr)) {
     const int64_t nsw = (int64_t)((p.T + 31) / 32) * p.H * p.B;
     p.runs = runs_of_blocks(p);
     if (eight_wavefronts<D>(p, nsw)) hipLaunchKernelGGL((prefill_split_kernel<D, 8>), dim3((unsigned)nsw), dim3(512), 0, s, p);

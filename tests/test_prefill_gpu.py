@@ -1,9 +1,11 @@
 """Kernel 1 parity: HIP prefill attention vs the fp32 oracle (through the C ABI)."""
+import ctypes
+
 import pytest
 import torch
 
 import oracle
-from daisy_amd import ops
+from daisy_amd import _lib, ops
 from helpers import assert_close_bf16, check_prefill_of_many_heads, say
 
 pytestmark = pytest.mark.gpu
@@ -221,17 +223,32 @@ def test_keys_rotated_in_place(D, H, T, surplus, pad):
     assert torch.equal(kr.cpu(), oracle.apply_rope(k, cos, sin)) and torch.equal(kr, k_ref) and torch.equal(o, o_ref)
 
 
-@pytest.mark.parametrize("T,H,D,window,docs", [
-    (4001, 5, 128, 200, 0), (4100, 3, 128, 1500, 0), (6500, 5, 64, 130, 0), (4224, 6, 128, 129, 0),   # runs of blocks, their remainder among them
-    (2048, 15, 128, 300, 0), (2049, 15, 128, 300, 0), (2048, 16, 128, 600, 0), (5120, 8, 128, 2560, 0), (5121, 8, 128, 2560, 0),
-    (7168, 8, 64, 200, 0), (7169, 8, 64, 200, 0), (3100, 13, 128, 200, 0), (5000, 13, 64, 700, 0), (2700, 12, 128, 1300, 0),
-    (5120, 8, 128, None, 3), (8192, 8, 128, 4096, 3), (8193, 8, 128, 4096, 3), (5120, 8, 128, 1100, 3), (5121, 8, 128, 1100, 3),
-    (5600, 16, 64, None, 3), (5633, 16, 64, None, 3),
-    (7700, 13, 128, 200, 3), (7400, 14, 128, 200, 3), (12000, 12, 64, 1000, 3), (1000, 110, 128, 120, 3),      # eighths of a pair, with and without a remainder, none
+@pytest.mark.parametrize("T,H,D,window,docs,split", [
+    # no window
+    (4096, 12, 128, None, 0, True), (4097, 12, 128, None, 0, False), (1000, 36, 128, None, 0, True), (1000, 37, 128, None, 0, False),
+    (6144, 16, 64, None, 0, True), (6145, 16, 64, None, 0, False),
+    # a window; with runs of blocks, their remainder among them; keys past an XCD's L2
+    (4001, 5, 128, 800, 0, True), (4100, 3, 128, 1000, 0, True), (4300, 3, 128, 200, 0, True), (6500, 5, 64, 130, 0, True),
+    (3328, 8, 128, 200, 0, True), (3329, 8, 128, 200, 0, False), (3072, 6, 128, 200, 0, True), (3073, 6, 128, 200, 0, False),
+    (2048, 16, 128, 800, 0, True), (2049, 16, 128, 800, 0, False), (5120, 8, 128, 2560, 0, True), (5121, 8, 128, 2561, 0, False),
+    (4096, 6, 128, 2000, 0, True), (4097, 6, 128, 2000, 0, False),
+    (7168, 8, 64, 200, 0, True), (7169, 8, 64, 200, 0, False), (8192, 5, 64, 4000, 0, True), (8193, 5, 64, 4000, 0, False),
+    (3100, 13, 128, 200, 0, False), (5000, 13, 64, 700, 0, False), (2700, 12, 128, 1300, 0, False), (2700, 12, 128, 1350, 0, True),
+    # documents
+    (4608, 8, 128, None, 3, True), (4609, 8, 128, None, 3, False), (4608, 8, 128, 1100, 3, True), (4609, 8, 128, 1100, 3, False),
+    (3328, 8, 128, 800, 3, True), (3329, 8, 128, 800, 3, False), (3072, 6, 128, 200, 3, True), (3073, 6, 128, 200, 3, False),
+    (4096, 6, 128, 2000, 3, True), (4097, 6, 128, 2000, 3, False), (4096, 7, 128, None, 3, True), (4097, 7, 128, None, 3, False),
+    (3200, 20, 64, None, 3, True), (3201, 20, 64, None, 3, False), (7168, 8, 64, 700, 3, True), (7169, 8, 64, 700, 3, False),
+    (8192, 5, 64, 700, 3, True), (8193, 5, 64, 700, 3, False), (11264, 5, 64, None, 3, True), (11265, 5, 64, None, 3, False),
+    # eighths of a pair, with and without a remainder, none
+    (7700, 13, 128, 200, 3, False), (7400, 14, 128, 200, 3, False), (12000, 12, 64, 1000, 3, False), (1000, 110, 128, 120, 3, False),
 ])
-def test_prefill_on_both_sides_of_the_block_size_rule(T, H, D, window, docs):
-    """Sizes around the numbers of blocks at which the kernel with 32 queries per workgroup hands over to the one with 128, and pairs
-    that are no multiple of eight; the first rows, some of every block and the last ones against the oracle."""
+def test_prefill_on_both_sides_of_the_block_size_rule(T, H, D, window, docs, split):
+    """Sizes around the numbers of blocks at which the kernel with 32 queries per workgroup hands over to the one with 128 (the rule itself is
+    asked which), and pairs that are no multiple of eight; the first rows, some of every block and the last ones against the oracle."""
+    wanted = _lib.load()._ZN5daisy20prefill_split_wantedEiiiib
+    wanted.restype = ctypes.c_bool
+    assert wanted(H, T, D, window or 0, bool(docs)) == split
     q, k, v = _inputs(1, T, H, D, seed=T + H, normalise=True)
     doc_start = None
     if docs:
