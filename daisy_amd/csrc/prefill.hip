@@ -191,7 +191,7 @@ __device__ __forceinline__ float pair_sum(float x) {
 // products.  A query that has seen no key has -FLT_MAX for a reference: what it does not see stays 0, its first key overflows the sum and sets it.  (Behind
 // a document's start the queries of a wavefront wait through every tile of the document ahead.  While any of them did, each tile took the long way: 20000
 // rows in seven documents, 4 heads of 128 172 us, 24545 in twenty, 8 heads 211, 5900 in three, 16 of 64 52.4; now 149, 186 and 49.8, with the maxima of every tile
-// 147, 185 and 49.2.)  
+// 147, 185 and 49.2.)
 // FIRST: a wavefront's first tile takes the long way at once, so that short rows do not work out its exponentials twice; the branch costs the tile
 // kernel for heads of 128 more where it is bound by latency, two or three blocks to a compute unit: 9000 rows, 8 heads 202.5 us with the maxima of every
 // tile, 208.7 with the branch, 203.8 without; 20000 in documents that start with a block, 4 heads 113.5, 115.8, 114.6.  (Heads of 64 need it: 128 registers
@@ -257,7 +257,7 @@ __device__ __forceinline__ u32x2 lds_read_tr16_as3(lds_u16_ptr p) {
 
 // Main kernel (keys already rotated, or no RoPE on keys).  32-key tiles, and nothing of a step is
 // overlapped inside a wavefront: scores, softmax and the product of one tile follow each other.  The
-// kernel is small instead -- 158 VGPRs and 48 KiB of LDS at D = 128 -- so that THREE workgroups fit a
+// kernel is small instead -- 167 VGPRs and 48 KiB of LDS at D = 128 -- so that THREE workgroups fit a
 // CU, three wavefronts a SIMD, and the latencies of one wavefront's step (the issue of its tile
 // copies, the LDS operand reads, the softmax chain, the barrier) are covered by the other two: matrix
 // instructions of one wavefront and vector instructions of another do run side by side on a SIMD.
@@ -490,16 +490,26 @@ __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
         }
     }
     bf16x8 pfrag[2 * SUB];
+    auto v_frag = [&](int m, int dt) {
+      lds_u16_ptr vp = (lds_u16_ptr)(size_t)((v_a0 ^ (64u * dt)) + 2 * (buf * TILE + 16 * m * D));
+      const u32x2 a0 = lds_read_tr16_as3(vp);            // keys 16m + 4lh + 0..3
+      const u32x2 a1 = lds_read_tr16_as3(vp + 8 * D);    // keys 16m + 8 + 4lh + 0..3
+      return u32x4{a0.x, a0.y, a1.x, a1.y};
+    };
+    // The first V fragments are asked for ahead of the exponentials: behind the branch at their end, where the reads of all but those stand, each tile
+    // waits for the first one, which shows where a SIMD has one or two wavefronts.  As many as the registers hold (167 and 128).  us, none / these: 9000 rows, 8
+    // heads of 128, no window 205.9 / 201.8, 5900 x 12 in documents that start with a block 99.3 / 97.2, x 16 of 64 in three 50.4 / 49.8.
+    constexpr int EARLY = D == 128 ? 2 : 1;
+    u32x4 early[EARLY];
+#pragma unroll
+    for (int i = 0; i < EARLY; ++i) early[i] = v_frag(0, i);
     softmax_tile<D == 64, SUB, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
     // O^T += V^T P^T
 #pragma unroll
     for (int m = 0; m < 2 * SUB; ++m) {
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) {
-        lds_u16_ptr vp = (lds_u16_ptr)(size_t)((v_a0 ^ (64u * dt)) + 2 * (buf * TILE + 16 * m * D));
-        const u32x2 a0 = lds_read_tr16_as3(vp);            // keys 16m + 4lh + 0..3
-        const u32x2 a1 = lds_read_tr16_as3(vp + 8 * D);    // keys 16m + 8 + 4lh + 0..3
-        const u32x4 av = {a0.x, a0.y, a1.x, a1.y};
+        const u32x4 av = m == 0 && dt < EARLY ? early[dt] : v_frag(m, dt);
         oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), pfrag[m], oacc[dt], 0, 0, 0);
       }
     }
