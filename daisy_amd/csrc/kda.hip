@@ -139,9 +139,54 @@ struct SeqSpan { int tok0, tok_end, c0, nc; };
 // them (6 us).  BY_LENGTH: `key` counts from the longest one on, equal ones in their order (a lane per sequence only); it becomes
 // the sequence's number.
 constexpr int kScanSeqs = 64;
-template <bool BY_LENGTH = false> __device__ __forceinline__ SeqSpan packed_span(const KdaParams& p, int& key, bool by_slot, int& rows_end) {
+struct SeqScan { int begin, end, nc, upto; };      // a sequence per lane: token rows, chunks, chunks up to its end
+__device__ __forceinline__ SeqScan packed_scan(const KdaParams& p) {
+  const int lane = threadIdx.x & 63;
+  SeqScan c;
+  c.end = min(max(p.cu[min(lane + 1, p.n_seq)], p.cu[0]), p.T);
+  c.end = max(c.end, 0);
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int left = __shfl_up(c.end, off);
+    if (lane >= off) c.end = max(c.end, left);
+  }
+  c.begin = __shfl_up(c.end, 1);
+  c.begin = lane == 0 ? 0 : c.begin;
+  c.nc = lane < p.n_seq ? (c.end - c.begin + KC - 1) / KC : 0;
+  c.upto = c.nc;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int left = __shfl_up(c.upto, off);
+    if (lane >= off) c.upto += left;
+  }
+  return c;
+}
+template <bool BY_LENGTH> __device__ __forceinline__ SeqSpan scanned_span(const KdaParams& p, const SeqScan& c, int& key, bool by_slot, int& rows_end) {
   SeqSpan s{0, 0, 0, 0};
+  const int lane = threadIdx.x & 63;
+  rows_end = __builtin_amdgcn_readlane(c.end, 63);     // (lanes past the last sequence repeat its end)
+  if (by_slot) {
+    const uint64_t owner = __ballot(key >= c.upto - c.nc && key < c.upto);
+    if (owner == 0) return s;
+    key = __builtin_ctzll(owner);
+  }
+  if constexpr (BY_LENGTH) {
+    const int before = __shfl_up(c.nc, 1);
+    if (__ballot(c.nc > before && lane > 0) != 0) {                     // (not in that order already)
+      const uint32_t mine = ((uint32_t)c.nc << 6) + 63 - lane;          // (no two the same)
+      int ahead = 0;
+#pragma unroll 4
+      for (int j = 0; j < p.n_seq; ++j) ahead += (uint32_t)__builtin_amdgcn_readlane((int)mine, j) > mine ? 1 : 0;
+      key = __builtin_ctzll(__ballot(lane < p.n_seq && ahead == key));
+    }
+  }
+  s.tok0 = __builtin_amdgcn_readlane(c.begin, key); s.tok_end = __builtin_amdgcn_readlane(c.end, key);
+  s.nc = __builtin_amdgcn_readlane(c.nc, key); s.c0 = __builtin_amdgcn_readlane(c.upto, key) - s.nc;
+  return s;
+}
+template <bool BY_LENGTH = false> __device__ __forceinline__ SeqSpan packed_span(const KdaParams& p, int& key, bool by_slot, int& rows_end) {
   if (p.bounds != nullptr) {
+    SeqSpan s{0, 0, 0, 0};
     rows_end = p.bounds[p.n_seq];
     if (by_slot) {
       if (key >= p.seq_chunk0[p.n_seq]) return s;
@@ -151,42 +196,7 @@ template <bool BY_LENGTH = false> __device__ __forceinline__ SeqSpan packed_span
     s.c0 = p.seq_chunk0[key]; s.nc = p.seq_chunk0[key + 1] - s.c0;
     return s;
   }
-  const int lane = threadIdx.x & 63;
-  int end = min(max(p.cu[min(lane + 1, p.n_seq)], p.cu[0]), p.T);
-  end = max(end, 0);
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int left = __shfl_up(end, off);
-    if (lane >= off) end = max(end, left);
-  }
-  int begin = __shfl_up(end, 1);
-  begin = lane == 0 ? 0 : begin;
-  const int nc = lane < p.n_seq ? (end - begin + KC - 1) / KC : 0;
-  int upto = nc;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int left = __shfl_up(upto, off);
-    if (lane >= off) upto += left;
-  }
-  rows_end = __builtin_amdgcn_readlane(end, 63);     // (lanes past the last sequence repeat its end)
-  if (by_slot) {
-    const uint64_t owner = __ballot(key >= upto - nc && key < upto);
-    if (owner == 0) return s;
-    key = __builtin_ctzll(owner);
-  }
-  if constexpr (BY_LENGTH) {
-    const int before = __shfl_up(nc, 1);
-    if (__ballot(nc > before && lane > 0) != 0) {                     // (not in that order already)
-      const uint32_t mine = ((uint32_t)nc << 6) + 63 - lane;          // (no two the same)
-      int ahead = 0;
-#pragma unroll 4
-      for (int j = 0; j < p.n_seq; ++j) ahead += (uint32_t)__builtin_amdgcn_readlane((int)mine, j) > mine ? 1 : 0;
-      key = __builtin_ctzll(__ballot(lane < p.n_seq && ahead == key));
-    }
-  }
-  s.tok0 = __builtin_amdgcn_readlane(begin, key); s.tok_end = __builtin_amdgcn_readlane(end, key);
-  s.nc = __builtin_amdgcn_readlane(nc, key); s.c0 = __builtin_amdgcn_readlane(upto, key) - s.nc;
-  return s;
+  return scanned_span<BY_LENGTH>(p, packed_scan(p), key, by_slot, rows_end);
 }
 template <bool BY_LENGTH> __device__ __forceinline__ SeqSpan seq_span(const KdaParams& p, int& seq, int& rows_end) {
   if (p.n_seq > 0) return packed_span<BY_LENGTH>(p, seq, false, rows_end);
@@ -784,17 +794,20 @@ template <int KCT> constexpr int kStateThreads = 64 * (KCT + 2 * KPW);
 //    into registers, KSETS - 1 chunks ahead, once for all column tiles; a wavefront per tile, with operands through the LDS: T = 8192,
 //    up to 8 heads of 128 162 -> 145 us, 16 heads 180 -> 172, 64 heads 237 -> 226 (two sets fewer or more: level);
 //  * the chain does not wait for global memory: two further wavefronts issue the asynchronous copies of the chunks ahead.
-// BY_LENGTH: packed sequences from the longest one on (a kernel of its own: with that code ahead of their loop other calls' chains are 1 to 2 % slower).
-template <int KD, int KCT, bool BY_LENGTH>
-__global__ __launch_bounds__(kStateThreads<KCT>, 1) void kda_state_kernel(KdaParams p) {
+
+// What a chain keeps in the LDS, in arrays of their own so that the compiler can tell their accesses apart.
+template <int KD, int KCT> constexpr int kStageBytes = KdaBlob<KD>::kChain + KC * KVS * KCT * 2;
+template <int KD, int KCT> using StageLds = char[KSTAGES][kStageBytes<KD, KCT>];
+template <int KD, int KCT> using StateLds = u32x4[2][KCT][KD / 32][64];       // [chunk parity][column tile][channel group][lane]: S0 as operand
+template <int KCT> using XLds = u32x4[2][KCT][2][64];                         // X as operand, two terms
+// The chain of this workgroup.  span_of(b, rows_end): where sequence b lives; BY_LENGTH: b counts from the longest one on and becomes the sequence's number.
+template <int KD, int KCT, bool BY_LENGTH, typename SPAN>
+__device__ __forceinline__ void kda_chain(const KdaParams& p, StageLds<KD, KCT>& stage, StateLds<KD, KCT>& xs, XLds<KCT>& xx, SPAN span_of) {
   using Blob = KdaBlob<KD>;
   constexpr int NM = KD / 32, NS = KD / 16;                    // channel groups of 32, state tiles of 16 rows
-  constexpr int kV = Blob::kChain, kStage = kV + KC * KVS * KCT * 2;
+  constexpr int kV = Blob::kChain, kStage = kStageBytes<KD, KCT>;
   // Links are cut by workgroup barriers.  Interval n between two of them copies the chain's part of chunk n; the chain reads it in
   // interval n + 2 and computes link n, beside its outputs, in interval n + 3.
-  __shared__ __attribute__((aligned(1024))) char stage[KSTAGES][kStage];
-  __shared__ __attribute__((aligned(16))) u32x4 xs[2][KCT][NM][64];           // [chunk parity][column tile][channel group][lane]: S0 as operand
-  __shared__ __attribute__((aligned(16))) u32x4 xx[2][KCT][2][64];            // X as operand, two terms
 
   // The column groups of one (batch, head) on one XCD, in consecutive workgroups of it: they read the same blocks.
   const int NGRP = (p.Dv + KVS * KCT - 1) / (KVS * KCT);
@@ -803,7 +816,7 @@ __global__ __launch_bounds__(kStateThreads<KCT>, 1) void kda_state_kernel(KdaPar
   if (bh >= (p.n_seq > 0 ? p.n_seq : p.B) * p.H) return;
   const int h = bh % p.H;
   int b = bh / p.H, rows_end;               // b: batch element, or sequence of a packed batch
-  const SeqSpan sp = seq_span<BY_LENGTH>(p, b, rows_end);
+  const SeqSpan sp = span_of(b, rows_end);
   if constexpr (BY_LENGTH) bh = b * p.H + h;
   const int nc = sp.nc;                      // chunks of this sequence (0 for an empty one)
   const int64_t ci0 = (int64_t)sp.c0 * p.H + h, step = (int64_t)p.H * Blob::kBytes;
@@ -1068,6 +1081,43 @@ __global__ __launch_bounds__(kStateThreads<KCT>, 1) void kda_state_kernel(KdaPar
   }
 }
 
+// BY_LENGTH: packed sequences from the longest one on (a kernel of its own: with that code ahead of their loop other calls' chains are 1 to 2 % slower).
+template <int KD, int KCT, bool BY_LENGTH>
+__global__ __launch_bounds__(kStateThreads<KCT>, 1) void kda_state_kernel(KdaParams p) {
+  __shared__ __attribute__((aligned(1024))) StageLds<KD, KCT> stage;
+  __shared__ __attribute__((aligned(16))) StateLds<KD, KCT> xs;
+  __shared__ __attribute__((aligned(16))) XLds<KCT> xx;
+  kda_chain<KD, KCT, BY_LENGTH>(p, stage, xs, xx, [&](int& b, int& rows_end) { return seq_span<BY_LENGTH>(p, b, rows_end); });
+}
+
+// Up to kScanSeqs packed sequences in groups of 64 columns or of 32, as their lengths, which only the device knows, want it: 64 where the
+// longest chain, whose links they lengthen, is no more than three quarters of the links of 32 that fall to a compute unit, each chain counted for four more that it
+// takes to start.  Columns come in whole groups of 64; the grid is that of 32.  us, 32 / 64 columns (that ratio), heads of 128: 16 sequences, 16 heads, T = 6000,
+// equal (0.18) 91.9 / 82.5, the longest a fifth (0.57) 93.1 / 88.7, cut at random (0.78) 97.4 / 99.5, the longest two fifths (1.1) 95.6 / 120, nearly all (2.8) 149 / 204;
+// T = 16000, cut at random (0.68) 238 / 228, 8 heads (1.4) 142 / 159; 33 sequences, T = 6000, at random (0.53) 114 / 95, the longest two fifths (0.89) 118 / 123, 8 heads,
+// at random (1.0) 62 / 72, T = 16000 (0.64) 151 / 149.  (Not for key heads of 64: of their groups of 32 two workgroups fit a compute unit, of this kernel one.)
+template <bool BY_LENGTH>
+__global__ __launch_bounds__(kStateThreads<4>, 1) void kda_packed_state_kernel(KdaParams p) {
+  constexpr int KD = 128;
+  __shared__ __attribute__((aligned(1024))) StageLds<KD, 4> stage;
+  __shared__ __attribute__((aligned(16))) StateLds<KD, 4> xs;
+  __shared__ __attribute__((aligned(16))) XLds<4> xx;
+  const SeqScan scan = packed_scan(p);
+  int longest = scan.nc;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
+  longest = __builtin_amdgcn_readfirstlane(longest);
+  const int64_t links = (int64_t)(__builtin_amdgcn_readlane(scan.upto, 63) + 4 * p.n_seq) * p.H * (p.Dv / (2 * KVS));
+  auto chain = [&](auto columns) {
+    constexpr int KCT = decltype(columns)::value;
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= kStateThreads<KCT>) return;
+    kda_chain<KD, KCT, BY_LENGTH>(p, reinterpret_cast<StageLds<KD, KCT>&>(stage), reinterpret_cast<StateLds<KD, KCT>&>(xs), reinterpret_cast<XLds<KCT>&>(xx),
+                                  [&](int& b, int& rows_end) { return scanned_span<BY_LENGTH>(p, scan, b, false, rows_end); });
+  };
+  if (longest * (int64_t)(256 * 4) <= 3 * links) chain(std::integral_constant<int, 4>{});
+  else chain(std::integral_constant<int, 2>{});
+}
+
 }  // namespace daisy
 
 using namespace daisy;
@@ -1130,19 +1180,6 @@ extern "C" size_t daisy_kda_varlen_workspace_bytes(int T, int n_seq, int H, int 
 // 168 -> 176, against 2 x 7500, 8 heads of 128 260 -> 252.
 constexpr int64_t kCachedBytes = (int64_t)128 << 20;
 
-template <int KD, int KCT>
-static void launch_chains(const KdaParams& p, int n_streams, hipStream_t s) {
-  const int groups = (p.Dv + KVS * KCT - 1) / (KVS * KCT);
-  const unsigned chains = (unsigned)((n_streams * p.H + 7) / 8 * 8 * groups);
-  // A chain fills a compute unit: where there are more than 256, a long sequence that starts late ends alone.  Longest first, cut at random places, both
-  // kernels: 10 sequences of T = 4689, 16 heads of 128 102 -> 87 us, 7 of 3000, 12 heads 53 -> 44.4, 7 of 6164, 16 of 64 67.3 -> 56; 40 such batches 4 % on
-  // average.  Where the longest one comes early anyway ranking costs (12 of 12000, 16 of 64 95.5 -> 97.3): 0.03 us a sequence in every workgroup, so
-  // only up to a tenth of a mean chain (else 16 of T = 2088, 8 heads of 128 34.5 -> 35.5, 13 of 148, 12 heads 18.2 -> 19.8); not where they are in that order.
-  const bool by_length = chains > 256 && p.n_seq > 1 && p.n_seq <= kScanSeqs && p.NC >= p.n_seq * p.n_seq;
-  if (by_length) hipLaunchKernelGGL((kda_state_kernel<KD, KCT, true>), dim3(chains), dim3(kStateThreads<KCT>), 0, s, p);
-  else hipLaunchKernelGGL((kda_state_kernel<KD, KCT, false>), dim3(chains), dim3(kStateThreads<KCT>), 0, s, p);
-}
-
 template <int KD>
 static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
   const dim3 chunks((unsigned)p.NC * (unsigned)p.H, 1, p.n_seq > 0 ? 1 : p.B);
@@ -1153,12 +1190,32 @@ static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
     hipLaunchKernelGGL((kda_prep_kernel<KD, false>), chunks, dim3(128), 0, s, p);
   }
   DAISY_CHECK_LAUNCH("kda_prep_kernel");
-  // Where groups of 32 value columns are more than the compute units, groups of 64: a link of 64 columns takes longer (0.8 us against 0.57 with few chains,
-  // by its LDS reads), but one round of them less than two.  Chains of T = 4096, 32 / 64 columns, us: heads of 128, 256 groups of 32 167 / 183, 320 206 /
-  // 140, 384 210 / 155, 512 228 / 187, T = 2048 1024 229 / 187; key heads of 64 256 114 / 125, 320 156 / 106, 512 172 / 128, 64 sequences of 64 rows 22 / 20.  Packed
-  // sequences likewise, of equal lengths or not (16 of 17 batches 1 to 18 % faster with 64, both kernels; 11 cut at random places, the longest 2.6 means, 108 / 120).
-  const int64_t groups = (int64_t)n_streams * p.H * ((p.Dv + 2 * KVS - 1) / (2 * KVS));
-  if (groups > 256 && p.Dv > 2 * KVS) launch_chains<KD, 4>(p, n_streams, s); else launch_chains<KD, 2>(p, n_streams, s);
+  // A chain fills a compute unit.  Groups of 64 value columns where they take fewer rounds of 256 than groups of 32: a link of 64 columns takes longer (0.8 us
+  // against 0.57 with few chains, by its LDS reads), but one round of them less than two.  Chains of T = 4096, 32 / 64 columns, us: heads of 128, 256 groups of 32 167 /
+  // 183, 320 206 / 140, 384 210 / 155, 512 228 / 187, T = 2048 1024 229 / 187; key heads of 64 256 114 / 125, 320 156 / 106, 512 172 / 128, 64 sequences of 64 rows 22 / 20.
+  // Both kernels, T = 2048, where a dead half makes the rounds as many: 9 x 16 heads of 128 x 96 (432 / 288 groups) 242 / 270, 10 x 16 of 64 x 96 160 / 176; T = 1024, 6 x 16
+  // of 128 x 160 (480 / 288) 93 / 107; as many or fewer: 11 x 16 of 128 x 96 (528 / 352) 314 / 299, 20 x 16 (960 / 640) level, 17 x 16 of 128 x 40 (544 / 272) 219 / 220.
+  const int64_t streams = (int64_t)n_streams * p.H;
+  const int narrow = (p.Dv + 2 * KVS - 1) / (2 * KVS), wide = (p.Dv + 4 * KVS - 1) / (4 * KVS);
+  const unsigned chains = (unsigned)((streams + 7) / 8 * 8 * narrow);
+  if (p.n_seq == 0) {
+    if ((streams * wide + 255) / 256 < (streams * narrow + 255) / 256) {
+      hipLaunchKernelGGL((kda_state_kernel<KD, 4, false>), dim3((unsigned)((streams + 7) / 8 * 8 * wide)), dim3(kStateThreads<4>), 0, s, p);
+    } else {
+      hipLaunchKernelGGL((kda_state_kernel<KD, 2, false>), dim3(chains), dim3(kStateThreads<2>), 0, s, p);
+    }
+  } else {
+    // Where there are more than 256, a long sequence that starts late ends alone.  Longest first, cut at random places, both
+    // kernels: 10 sequences of T = 4689, 16 heads of 128 102 -> 87 us, 7 of 3000, 12 heads 53 -> 44.4, 7 of 6164, 16 of 64 67.3 -> 56; 40 such batches 4 % on
+    // average.  Where the longest one comes early anyway ranking costs (12 of 12000, 16 of 64 95.5 -> 97.3): 0.03 us a sequence in every workgroup, so
+    // only up to a tenth of a mean chain (else 16 of T = 2088, 8 heads of 128 34.5 -> 35.5, 13 of 148, 12 heads 18.2 -> 19.8); not where they are in that order.
+    const bool by_length = chains > 256 && p.n_seq > 1 && p.n_seq <= kScanSeqs && p.NC >= p.n_seq * p.n_seq;
+    const bool either = KD == 128 && p.n_seq <= kScanSeqs && streams * narrow > 256 && p.Dv % (4 * KVS) == 0;
+    if (either && by_length) hipLaunchKernelGGL(kda_packed_state_kernel<true>, dim3(chains), dim3(kStateThreads<4>), 0, s, p);
+    else if (either) hipLaunchKernelGGL(kda_packed_state_kernel<false>, dim3(chains), dim3(kStateThreads<4>), 0, s, p);
+    else if (by_length) hipLaunchKernelGGL((kda_state_kernel<KD, 2, true>), dim3(chains), dim3(kStateThreads<2>), 0, s, p);
+    else hipLaunchKernelGGL((kda_state_kernel<KD, 2, false>), dim3(chains), dim3(kStateThreads<2>), 0, s, p);
+  }
   DAISY_CHECK_LAUNCH("kda_state_kernel");
   return DAISY_OK;
 }
