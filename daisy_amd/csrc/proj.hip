@@ -514,13 +514,16 @@ static int proj_tile(int M, int K, int head, COLUMNS columns, float* its_cost = 
 // output and the library's lead grows with K: ahead at every M up to K = 1536 (whole layer, M = 32768: 640 against 655 us),
 // behind from K = 2048 on where the product is large (M = 32768: 1014 against 981 us; M = 8192: 251 against 257 us).
 bool proj_segments_wanted(int M, int N, int K) { return K % 64 == 0 && N % 8 == 0 && (K <= 512 || (int64_t)M * N <= 4300000); }
-// One product also where its tiles of 128 x 128, of which two fit a compute unit, nearly fill one round: 384 to 512 of them.  Library / this, us:
-// 4096 x 1536 x 1536 21.9 / 21.8, 8192 x 768 x 768 14.5 / 13.1, 8192 x 1024 x 1024 19.6 / 16.8, 7000 x 1024 x 1024 18.9 / 17.0, 4096 x 2048 x 2048 32.3 / 30.8,
-// 1400 x 4608 x 1536 26.0 / 22.4; with fewer tiles either may be ahead (288: 16.7 / 12.7 and 13.3 / 13.7, 352: 25.4 / 28.5), with more the library is (516: 27.8 /
-// 36.3, 17.8 / 21.3).  K up to 2048 and M from 1000 are what was measured.
+// One product also where its tiles of 128 x 128, of which two fit a compute unit, nearly fill one round: 384 to 512 of them, from 440 for rows of more
+// than 1024, none of more than 1536, of which the library's tiles make better use.  Library / this, us (200 sizes, M from 1000, K from 576): 8192 x 1024 x 576 15.0 / 12.1, 8192 x
+// 1024 x 1024 19.6 / 16.8, 7000 x 1024 x 1024 18.9 / 17.0, 2176 x 3072 x 1024 (408) 18.8 / 17.9, 29212 x 256 x 1024 20.3 / 19.0, 5760 x 1280 x 1536 (450) 26.3 / 25.4, but 4096
+// x 1536 x 1536 (384) 21.9 / 21.8, 1472 x 4096 x 1536 (384) 22.4 / 24.1, 3072 x 2048 x 1280 (384) 20.0 / 21.4; 4096 x 2048 x 2048 32.3 / 30.8, but 6144 x 1024 x 2048 (384) 26.7 /
+// 29.1, 25756 x 256 x 1792 30.5 / 38.2; one column of tiles 49152 x 128 x 1024 26.5 / 28.9, 60159 x 128 x 1536 44.9 / 45.9.  With fewer tiles either may be ahead (288: 16.7 /
+// 12.7 and 13.3 / 13.7, 352: 25.4 / 28.5), with more the library is (516: 27.8 / 36.3, 17.8 / 21.3).
 bool proj_wanted(int M, int N, int K) {
   const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  return proj_segments_wanted(M, N, K) || (K % 64 == 0 && N % 8 == 0 && K <= 2048 && M >= 1000 && tiles >= 384 && tiles <= 512);
+  return proj_segments_wanted(M, N, K) ||
+         (K % 64 == 0 && N % 8 == 0 && K <= 1536 && N >= 256 && M >= 1000 && tiles >= (K <= 1024 ? 384 : 440) && tiles <= 512);
 }
 // A KDA layer's six products of the same rows, N columns in all, in one launch rather than the three large ones by themselves (this kernel's or
 // the library's) and the rest in another: one launch for four, and whole rounds of tiles for four that end in part of one.  Layers of 12 heads
