@@ -971,11 +971,13 @@ static int launch_mfma(PrefillParams p, hipStream_t s) {
     // Pre-pass: rotate K once into k_out, then attend over k_out.
     // (four heads a thread, four 16-byte accesses under way: heads of 128 are better off with two, whose rotation is twice as long: 77.9 and 78.8 us
     // for 8 x 4096 rows, 8 heads, with the attention)
-    const int hpt = D == 64 && p.H % 4 == 0 ? 4 : p.H % 2 == 0 ? 2 : 1;
+    constexpr int kHeads = D == 64 ? 4 : 2;
+    const int hpt = p.H % kHeads == 0 ? kHeads : p.H % 2 == 0 ? 2 : 1;
     const int64_t total = (int64_t)p.B * p.T * (p.H / hpt) * (D / 8);
-    if (hpt == 4) hipLaunchKernelGGL((rope_k_kernel<D, 4>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p);
-    else if (hpt == 2) hipLaunchKernelGGL((rope_k_kernel<D, 2>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((rope_k_kernel<D, 1>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p);
+    const dim3 grid((unsigned)((total + 255) / 256));
+    if (hpt == kHeads) hipLaunchKernelGGL((rope_k_kernel<D, kHeads>), grid, dim3(256), 0, s, p);
+    else if (hpt == 2) hipLaunchKernelGGL((rope_k_kernel<D, 2>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((rope_k_kernel<D, 1>), grid, dim3(256), 0, s, p);
     DAISY_CHECK_LAUNCH("rope_k_kernel");
     p.k = p.k_out; p.k_sb = p.ko_sb; p.k_st = p.ko_st; p.k_sh = p.ko_sh;
   }
