@@ -261,6 +261,6 @@ def test_prefill_on_both_sides_of_the_block_size_rule(T, H, D, window, docs, spl
         lo = torch.maximum(lo, doc_start.long())
     o, _ = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), window=window, doc_start=None if doc_start is None else doc_start.cuda())
     visible = (torch.arange(T)[None] <= rows[:, None]) & (torch.arange(T)[None] >= lo[rows][:, None])
-    for h in range(0, H, max(H // 3, 1)):
+    for h in range(H) if H <= 20 else (*range(8), *range(H - 8, H)):      # (every remainder by eight: the order of blocks depends on it)
         s = (q[0, rows, h].float() @ k[0, :, h].float().T * 0.12).masked_fill(~visible, float("-inf"))
         assert_close_bf16(o[0, rows.cuda(), h], s.softmax(-1) @ v[0, :, h].float(), f"o, head {h}")

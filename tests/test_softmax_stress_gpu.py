@@ -3,8 +3,9 @@
 The ordinary parity cases use scale 0.12 on unit-variance inputs: scores a few log2 units wide, so the
 rescale of the running sums almost never fires after a row's first tile.  Here scale = 1 and the keys are
 built so that the score of a (query, key) pair grows (or falls) steadily with the key's position: the row
-maximum rises tile after tile by a chosen amount -- below the kernels' lazy-rescale threshold (2^8), just
-above it, and far above it (old contributions scaled by ~2^-40) -- or sits in the first / last key a query
+maximum rises tile after tile by a chosen amount -- 5, 12 or 40 log2 units: a prefill kernel moves its reference
+when a lane's share of a tile's sum exceeds 2^12, some tiles late, about each, or in each (old contributions
+scaled by ~2^-40); decode follows the maximum -- or sits in the first / last key a query
 sees.  Checked against the fp32 oracle at the usual bf16 tolerances.
 """
 import pytest
