@@ -192,12 +192,15 @@ __device__ __forceinline__ float pair_sum(float x) {
 // a document's start the queries of a wavefront wait through every tile of the document ahead.  While any of them did, each tile took the long way: 20000
 // rows in seven documents, 4 heads of 128 172 us, 24545 in twenty, 8 heads 211, 5900 in three, 16 of 64 52.4; now 149, 186 and 49.8, with the maxima of every tile
 // 147, 185 and 49.2.)
-// FIRST: a wavefront's first tile takes the long way at once, so that short rows do not work out its exponentials twice; the branch costs the tile
-// kernel for heads of 128 more where it is bound by latency, two or three blocks to a compute unit: 9000 rows, 8 heads 202.5 us with the maxima of every
-// tile, 208.7 with the branch, 203.8 without; 20000 in documents that start with a block, 4 heads 113.5, 115.8, 114.6.  (Heads of 64 need it: 128 registers
-// do not hold both ends of the block that the products and the exponentials then share.)  The tile kernels are bound by their vector
-// instructions (head dim 64: 855 cycles of them per 64 keys against 512 of the matrix pipe) and by power, which fewer of them
-// spare: with the maxima of every tile worked out and compared (a reference moved at 2^8) 65536 rows, 16 heads of 128, full causal took 15.00 ms, now
+// kFirst: a wavefront's first tile takes the long way at once, so that short rows do not work out its exponentials twice; the branch costs the tile
+// kernel for heads of 128 more where it is bound by latency, two or three blocks to a compute unit, so there it is kSums: 9000 rows, 8 heads 202.5 us with the
+// maxima of every tile, 208.7 with the branch, 203.8 without; 20000 in documents that start with a block, 4 heads 113.5, 115.8, 114.6.  (Heads of 64 need it: 128
+// registers do not hold both ends of the block that the products and the exponentials then share.)
+// kMaxima: the maxima of every tile ahead of its exponentials, a reference moves at 2^8.  For windows of a few tiles, most of which are some query's first or last:
+// sums / maxima, us, heads of 128: 8 x 4096 rows, window 100 / 256 / 383 / 450 15.0 / 14.2, 17.1 / 16.2, 19.2 / 18.4, 20.7 / 20.1, 16 x 30000 102 / 100, 121 / 119, 146.8 / 146.6, 163.6 /
+// 165.3; heads of 64: 12 x 2 x 8192, 100 / 200 / 300 26.5 / 24.8, 29.1 / 28.1, 31.8 / 31.9, 16 x 30000 57.3 / 56.6, 63.8 / 64.0, 71.5 / 73.5.
+// The tile kernels are bound by their vector instructions (head dim 64: 855 cycles of them per 64 keys against 512 of the matrix pipe) and by power, which fewer of
+// them spare: with the maxima of every tile worked out and compared (a reference moved at 2^8) 65536 rows, 16 heads of 128, full causal took 15.00 ms, now
 // 14.56; 20001 rows in seven documents, 16 heads of 64, 178.6 us, now 171.4; a layer of 8 x 4096 rows, 8 heads of 128, window 1024, 406.2 and 403.8.
 struct SoftmaxRef {
   float minus = FLT_MAX;   // less the reference (scaled), the same in both lanes of a query: what is added to the scaled scores
@@ -205,7 +208,8 @@ struct SoftmaxRef {
   bool first = true;       // the wavefront has seen no tile
 };
 constexpr float kMost = 4096.f;
-template <bool FIRST, int SUB, int NDT>
+enum SoftmaxMode { kSums, kFirst, kMaxima };
+template <SoftmaxMode MODE, int SUB, int NDT>
 __device__ __forceinline__ void softmax_tile(const f32x16 (&sacc)[SUB], float scale_log2e, SoftmaxRef& ref, f32x16 (&oacc)[NDT],
                                              bf16x8 (&pfrag)[2 * SUB]) {
   float lsum;
@@ -222,7 +226,7 @@ __device__ __forceinline__ void softmax_tile(const f32x16 (&sacc)[SUB], float sc
       pfrag[m] = __builtin_bit_cast(bf16x8, pack8(pv));
     }
   };
-  bool moves = FIRST && ref.first;
+  bool moves = MODE == kMaxima || (MODE == kFirst && ref.first);
   if (!moves) {
     exponentials();
     moves = __builtin_amdgcn_ballot_w64(lsum > kMost) != 0;
@@ -235,13 +239,15 @@ __device__ __forceinline__ void softmax_tile(const f32x16 (&sacc)[SUB], float sc
 #pragma unroll
       for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[u][r]);
     mt = pair_max(mt) * scale_log2e;
-    const float minus = fminf(ref.minus, -mt), alpha = fast_exp2(minus - ref.minus);
-    ref.minus = minus;
-    ref.l *= alpha;
+    if (MODE != kMaxima || __builtin_amdgcn_ballot_w64(mt > 8.f - ref.minus) != 0) {
+      const float minus = fminf(ref.minus, -mt), alpha = fast_exp2(minus - ref.minus);
+      ref.minus = minus;
+      ref.l *= alpha;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
+      for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+    }
     exponentials();
   }
   ref.l += lsum;
@@ -271,7 +277,7 @@ __device__ __forceinline__ u32x2 lds_read_tr16_as3(lds_u16_ptr p) {
 // KEYS = 64 (prefill_wide_tile_kernel, head dim 64): a tile is two products side by side, with one maximum, one check of the reference and
 // one barrier for both (120 registers and 32 KiB, still four workgroups per CU: the Q and O blocks fit Ks[1] and Vs[1]).
 constexpr int kTBN = 32;   // key rows of a product
-template <int D, int KEYS>
+template <int D, int KEYS, SoftmaxMode MODE>
 __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
   constexpr int NS = D / 16, NDT = D / 32, HALF = D / 2, CPR = D / 8;
   constexpr int SUB = KEYS / kTBN;               // products of a tile
@@ -499,11 +505,11 @@ __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
     // The first V fragments are asked for ahead of the exponentials: behind the branch at their end, where the reads of all but those stand, each tile
     // waits for the first one, which shows where a SIMD has one or two wavefronts.  As many as the registers hold (167 and 128).  us, none / these: 9000 rows, 8
     // heads of 128, no window 205.9 / 201.8, 5900 x 12 in documents that start with a block 99.3 / 97.2, x 16 of 64 in three 50.4 / 49.8.
-    constexpr int EARLY = D == 128 ? 2 : 1;
-    u32x4 early[EARLY];
+    constexpr int EARLY = MODE == kMaxima ? 0 : D == 128 ? 2 : 1;
+    u32x4 early[EARLY + 1];
 #pragma unroll
     for (int i = 0; i < EARLY; ++i) early[i] = v_frag(0, i);
-    softmax_tile<D == 64, SUB, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
+    softmax_tile<MODE, SUB, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
     // O^T += V^T P^T
 #pragma unroll
     for (int m = 0; m < 2 * SUB; ++m) {
@@ -564,9 +570,9 @@ __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
   }
 }
 
-template <int D>
-__global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(PrefillParams p) { prefill_tiles<D, kTBN>(p); }
-__global__ __launch_bounds__(kPrefillThreads, 4) void prefill_wide_tile_kernel(PrefillParams p) { prefill_tiles<64, 2 * kTBN>(p); }
+template <int D, SoftmaxMode MODE>
+__global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(PrefillParams p) { prefill_tiles<D, kTBN, MODE>(p); }
+__global__ __launch_bounds__(kPrefillThreads, 4) void prefill_wide_tile_kernel(PrefillParams p) { prefill_tiles<64, 2 * kTBN, kFirst>(p); }
 
 // Few workgroups (a prompt of one or two thousand tokens of one sequence): blocks of 128 queries leave most compute
 // units idle and the last block walks all of its keys with one step in flight.  Here a workgroup is 32 queries, its
@@ -725,7 +731,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : W / 4) void prefill_split_kern
       }
     }
     bf16x8 pfrag[2];
-    softmax_tile<true, 1, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
+    softmax_tile<kFirst, 1, NDT>(sacc, p.scale_log2e, ref, oacc, pfrag);
     // V(n) has landed when only K(n + 1)'s copies are outstanding
     if (more) __builtin_amdgcn_s_waitcnt(0x0F70 | NCP);
     else __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -990,7 +996,8 @@ static int launch_mfma(PrefillParams p, hipStream_t s) {
     return DAISY_OK;
   }
   if (D == 64 && p.keys > kTBN) hipLaunchKernelGGL(prefill_wide_tile_kernel, dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
-  else hipLaunchKernelGGL((prefill_tile_kernel<D>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
+  else if (p.period > 0 && p.window < (D == 64 ? 256 : 384)) hipLaunchKernelGGL((prefill_tile_kernel<D, kMaxima>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
+  else hipLaunchKernelGGL((prefill_tile_kernel<D, D == 64 ? kFirst : kSums>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
   DAISY_CHECK_LAUNCH("prefill_tile_kernel");
   return DAISY_OK;
 }
