@@ -188,7 +188,8 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 // Stores 16 bytes through the L2 at once (policy sc1).  What a kernel leaves dirty in the L2 is written back at its end, behind its last
 // workgroup: its last round's results, all of them for a launch of one round.  The store's data registers are free one wait state
 // behind it, which the block holds.  us, a plain store / this: a layer's prefill of 777 rows, 12 heads of 128, QKV projection 37.5 / 37.0,
-// attention output and output projection 36.8 / 36.5; of 8 x 4096 rows, 8 heads, 400 / 396; 4096 x 2048 x 512 17.2 / 16.0.
+// attention output and output projection 36.8 / 36.5; of 8 x 4096 rows, 8 heads, 400 / 396; 4096 x 2048 x 512 17.2 / 16.0; products of a decode
+// batch, 9 to 512 rows, level (0.99 to 1.02) up to 2048 columns, 128 to 512 rows of 8192 x 1536 3 % ahead.
 __device__ __forceinline__ void store_through(void* at, const u32x4& v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(at), "v"(v) : "memory");
 }

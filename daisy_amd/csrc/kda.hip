@@ -86,8 +86,8 @@ __global__ __launch_bounds__(256) void kda_gate_kernel(const void* g, const floa
 // hold channels 32 m + 8 (row/4) + 4 t + row%4, so that a lane's eight are neighbours and one 16-byte piece of Kg or Qg as they
 // are; X's tiles hold positions 16 t + 4 (row/4) + row%4, and M and P are stored with their columns permuted to match.
 //
-// What bounds it.  Of the first kernel, at B4 T8192 H16 with fp32 log-decays, memory: 1.29 GB (673 MB of inputs, 612 MB of blocks) in
-// 203 us (6.3 TB/s); otherwise its vector instructions and their latency.  The second is a serial chain of chunks; what sets the time of a
+// What bounds it.  Of the first kernel, at B4 T8192 H16 with fp32 log-decays, mostly memory: 1.15 GB (539 MB of inputs, 612 MB of blocks) in
+// 203 us, 5.7 TB/s where the streaming kernels reach 6.3; otherwise its vector instructions and their latency.  The second is a serial chain of chunks; what sets the time of a
 // link is not the chain itself (without it the kernel is as fast) but its 39 KB of operands: a compute unit has about 64 KB
 // of requests in flight, 62 GB/s from memory (160 GB/s if they are in the L2).  0.57 us a link at T = 8192 with 4 heads of
 // 128 (0.63 before operands lay in the lanes' order and the outputs' came past the LDS), 0.39 us with 4 heads of 64, 0.67 us with 16 of 128,
@@ -783,8 +783,8 @@ constexpr int KSETS = 4;                      // register sets of an output wave
 template <int KCT> constexpr int kStateThreads = 64 * (KCT + 2 * KPW);
 
 // The chunk-to-chunk chain sets the time of this kernel once its data are there, and next to it what the CU's LDS can
-// deliver, 128 bytes a clock (about 130 KB of operands and copies per chunk with two column tiles, KCT = 2, 240 KB with four, which
-// sets their link).  So:
+// deliver, 128 bytes a clock (heads of 128: some 116 KB of operands and copies per chunk with two column tiles, KCT = 2, 206 KB with four,
+// which sets their link).  So:
 //  * one wavefront owns one tile of 16 value columns with all of its state rows: the state never leaves its registers
 //    (as right operand it is the accumulators converted in place), nothing of the chain waits for another wavefront,
 //    and every operand of the chain is read once per column tile.  Two wavefronts per tile with half of the state each,
@@ -981,8 +981,8 @@ __device__ __forceinline__ void kda_chain(const KdaParams& p, StageLds<KD, KCT>&
   for (int i = 0; i < KSTAGES - 1; ++i) __syncthreads();
 
   // A link's operands are read during the link before it, each register as soon as its last product has been issued: a 16-byte
-  // LDS read keeps a wavefront's port for 16 cycles and a chunk needs 34 of them, which in front of their use was half of
-  // the link.
+  // LDS read keeps a wavefront's port for 16 cycles and a chunk needs 25 of them (heads of 64: 16), which in front of their use, 34 with the
+  // decays of all tiles read by every lane, was half of the link.
   bf16x8 ka[2][NM], mh[NS], ml[NS];
   u32x2 vr[2];
   // The decays of a lane's rows of all tiles are the same for 16 lanes.  With 8 tiles each lane reads those of one of them (8 heads of 128 of

@@ -27,7 +27,7 @@
 // lanes L/4, L/4+4, L/4+8, L/4+12; with lane i of a block addressing key i/4,
 // channels 4*(i%4)..+3, lane i receives channel i of four consecutive keys.
 //
-// Keys reach prefill_tile_kernel rotated: by the caller, or by rope_k_kernel, a
+// Keys reach the tile kernels rotated: by the caller, or by rope_k_kernel, a
 // pre-pass that writes the rotated keys the reference's prefill returns anyway.
 //
 // Algorithmic work: 4*D flops per visible (query, key) pair.
@@ -275,7 +275,7 @@ __device__ __forceinline__ u32x2 lds_read_tr16_as3(lds_u16_ptr p) {
 // rows (a CU's memory path, shared by its three workgroups, is busy per cache line touched).
 //
 // KEYS = 64 (prefill_wide_tile_kernel, head dim 64): a tile is two products side by side, with one maximum, one check of the reference and
-// one barrier for both (120 registers and 32 KiB, still four workgroups per CU: the Q and O blocks fit Ks[1] and Vs[1]).
+// one barrier for both (128 registers and 32 KiB, still four workgroups per CU: the Q and O blocks fit Ks[1] and Vs[1]).
 constexpr int kTBN = 32;   // key rows of a product
 template <int D, int KEYS, SoftmaxMode MODE>
 __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
@@ -570,8 +570,10 @@ __device__ __forceinline__ void prefill_tiles(const PrefillParams& p) {
   }
 }
 
-template <int D, SoftmaxMode MODE>
-__global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(PrefillParams p) { prefill_tiles<D, kTBN, MODE>(p); }
+template <int D>
+__global__ __launch_bounds__(kPrefillThreads, 3) void prefill_tile_kernel(PrefillParams p) { prefill_tiles<D, kTBN, D == 64 ? kFirst : kSums>(p); }
+template <int D>
+__global__ __launch_bounds__(kPrefillThreads, 3) void prefill_short_window_kernel(PrefillParams p) { prefill_tiles<D, kTBN, kMaxima>(p); }
 __global__ __launch_bounds__(kPrefillThreads, 4) void prefill_wide_tile_kernel(PrefillParams p) { prefill_tiles<64, 2 * kTBN, kFirst>(p); }
 
 // Few workgroups (a prompt of one or two thousand tokens of one sequence): blocks of 128 queries leave most compute
@@ -996,8 +998,8 @@ static int launch_mfma(PrefillParams p, hipStream_t s) {
     return DAISY_OK;
   }
   if (D == 64 && p.keys > kTBN) hipLaunchKernelGGL(prefill_wide_tile_kernel, dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
-  else if (p.period > 0 && p.window < (D == 64 ? 256 : 384)) hipLaunchKernelGGL((prefill_tile_kernel<D, kMaxima>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
-  else hipLaunchKernelGGL((prefill_tile_kernel<D, D == 64 ? kFirst : kSums>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
+  else if (p.period > 0 && p.window < (D == 64 ? 256 : 384)) hipLaunchKernelGGL((prefill_short_window_kernel<D>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
+  else hipLaunchKernelGGL((prefill_tile_kernel<D>), dim3((unsigned)nwg), dim3(kPrefillThreads), 0, s, p);
   DAISY_CHECK_LAUNCH("prefill_tile_kernel");
   return DAISY_OK;
 }
