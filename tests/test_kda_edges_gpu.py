@@ -113,13 +113,11 @@ def test_kda_packed_longest_first(lengths, D):
         assert torch.equal(o[:, cu[i]:cu[i] + m], o1) and torch.equal(S[i:i + 1], S1)
 
 
-# Groups of 64 value columns where they take fewer rounds of 256 workgroups than groups of 32: whole ones, with a dead half, and with columns
-# that end inside a half; and as many rounds because of the dead half.  Sequences are independent: the same bits as from a call of one of them, in groups of 32.
-@pytest.mark.parametrize("B,T,H,Dk,Dv,wide", [(40, 33, 8, 64, 40, True), (11, 97, 16, 128, 96, True), (33, 1, 8, 72, 64, True), (22, 160, 8, 128, 72, True),
-                                              (12, 129, 12, 64, 128, True), (9, 97, 16, 128, 96, False), (6, 65, 16, 64, 160, False)])
-def test_kda_wide_column_groups(B, T, H, Dk, Dv, wide):
-    groups, half = B * H * ((Dv + 31) // 32), B * H * ((Dv + 63) // 64)
-    assert groups > 256 >= (H + 7) // 8 * 8 * ((Dv + 31) // 32) and ((half + 255) // 256 < (groups + 255) // 256) == wide
+# More groups of 32 value columns than compute units: groups of 64, whole ones, with a dead half, and with columns that end inside a
+# half.  Sequences are independent: the same bits as from a call of one of them, in groups of 32.
+@pytest.mark.parametrize("B,T,H,Dk,Dv", [(40, 33, 8, 64, 40), (9, 97, 16, 128, 96), (33, 1, 8, 72, 64), (17, 160, 8, 128, 72), (12, 129, 12, 64, 128)])
+def test_kda_wide_column_groups(B, T, H, Dk, Dv):
+    assert B * H * ((Dv + 31) // 32) > 256 >= (H + 7) // 8 * 8 * ((Dv + 31) // 32)
     q, k, v, gl, beta = _inputs(B, T, H, Dk, Dv, seed=B + T)
     s0 = torch.randn(B, H, Dk, Dv, generator=torch.Generator().manual_seed(B))
     o, S = _run(q, k, v, gl, beta, initial_state=s0.cuda())
@@ -130,6 +128,31 @@ def test_kda_wide_column_groups(B, T, H, Dk, Dv, wide):
     o_ref, S_ref = oracle.kda_recurrent(*part, initial_state=s0[B - 1:])
     assert_close_bf16(o[B - 1:], o_ref, "o")
     assert ((S[B - 1:] - S_ref).norm() / S_ref.norm()).item() <= 1e-3
+
+
+# Groups of 64 where they take fewer rounds of 256 workgroups than groups of 32, and as many rounds because of a dead half.
+@pytest.mark.parametrize("B,T,H,Dk,Dv,wide", [(40, 33, 8, 64, 40, True), (11, 97, 16, 128, 96, True), (22, 160, 8, 128, 72, True), (17, 160, 8, 128, 72, False),
+                                              (9, 97, 16, 128, 96, False), (6, 65, 16, 64, 160, False)])
+def test_kda_column_groups_by_rounds(B, T, H, Dk, Dv, wide):
+    assert ((B * H * ((Dv + 63) // 64) + 255) // 256 < (B * H * ((Dv + 31) // 32) + 255) // 256) == wide
+    test_kda_wide_column_groups(B, T, H, Dk, Dv)
+
+
+# ... of which there are more than compute units too: packed sequences start longest first.
+@pytest.mark.parametrize("D,Dv", [(64, 128), (128, 96)])
+def test_kda_packed_wide_column_groups_longest_first(D, Dv):
+    lengths, H = (40, 33, 512, 0, 512, 130, 700, 64, 513), 16
+    n, T = len(lengths), sum(lengths)
+    assert n * H * ((Dv + 63) // 64) > 256 and T // 32 + n >= n * n
+    q, k, v, gl, beta = _inputs(1, T + 5, H, D, Dv, seed=T)
+    cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32)
+    torch.full((T + 5, H, Dv), float("nan"), dtype=torch.bfloat16, device="cuda")
+    o, S = _run(q, k, v, gl, beta, cu_seqlens=cu.cuda())
+    assert not o[:, T:].any()
+    for i, m in enumerate(lengths):
+        if m:
+            o1, S1 = _run(*(t[:, cu[i]:cu[i] + m].contiguous() for t in (q, k, v, gl, beta)))
+            assert torch.equal(o[:, cu[i]:cu[i] + m], o1) and torch.equal(S[i:i + 1], S1)
 
 
 # Packed sequences of more groups of 32 than compute units, of both shapes that the kernel chooses from on the device, 64 columns (chains of like

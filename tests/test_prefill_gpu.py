@@ -223,6 +223,34 @@ def test_keys_rotated_in_place(D, H, T, surplus, pad):
     assert torch.equal(kr.cpu(), oracle.apply_rope(k, cos, sin)) and torch.equal(kr, k_ref) and torch.equal(o, o_ref)
 
 
+@pytest.mark.parametrize("T,H,D,window,docs", [
+    (4001, 5, 128, 200, 0), (4100, 3, 128, 1500, 0), (6500, 5, 64, 130, 0), (4224, 6, 128, 129, 0),   # runs of blocks, their remainder among them
+    (2048, 15, 128, 300, 0), (2049, 15, 128, 300, 0), (2048, 16, 128, 600, 0), (5120, 8, 128, 2560, 0), (5121, 8, 128, 2560, 0),
+    (7168, 8, 64, 200, 0), (7169, 8, 64, 200, 0), (3100, 13, 128, 200, 0), (5000, 13, 64, 700, 0), (2700, 12, 128, 1300, 0),
+    (5120, 8, 128, None, 3), (8192, 8, 128, 4096, 3), (8193, 8, 128, 4096, 3), (5120, 8, 128, 1100, 3), (5121, 8, 128, 1100, 3),
+    (5600, 16, 64, None, 3), (5633, 16, 64, None, 3),
+    (7700, 13, 128, 200, 3), (7400, 14, 128, 200, 3), (12000, 12, 64, 1000, 3), (1000, 110, 128, 120, 3),      # eighths of a pair, with and without a remainder, none
+])
+def test_prefill_on_both_sides_of_the_block_size_rule(T, H, D, window, docs):
+    """Sizes around the numbers of blocks at which the kernel with 32 queries per workgroup hands over to the one with 128, and pairs
+    that are no multiple of eight; the first rows, some of every block and the last ones against the oracle."""
+    q, k, v = _inputs(1, T, H, D, seed=T + H, normalise=True)
+    doc_start = None
+    if docs:
+        ids = torch.ones(T, dtype=torch.long)
+        ids[[T // 5, T // 2 + 3]] = 0
+        doc_start = oracle.doc_start_from_ids(ids, 0)
+    rows = torch.cat([torch.arange(0, T, 97), torch.arange(T - 3, T)]).unique()
+    lo = torch.zeros(T, dtype=torch.long) if window is None else (torch.arange(T) - window + 1).clamp(min=0)
+    if doc_start is not None:
+        lo = torch.maximum(lo, doc_start.long())
+    o, _ = ops.prefill_attention(q.cuda(), k.cuda(), v.cuda(), window=window, doc_start=None if doc_start is None else doc_start.cuda())
+    visible = (torch.arange(T)[None] <= rows[:, None]) & (torch.arange(T)[None] >= lo[rows][:, None])
+    for h in range(0, H, max(H // 3, 1)):
+        s = (q[0, rows, h].float() @ k[0, :, h].float().T * 0.12).masked_fill(~visible, float("-inf"))
+        assert_close_bf16(o[0, rows.cuda(), h], s.softmax(-1) @ v[0, :, h].float(), f"o, head {h}")
+
+
 @pytest.mark.parametrize("T,H,D,window,docs,split", [
     # no window
     (4096, 12, 128, None, 0, True), (4097, 12, 128, None, 0, False), (1000, 36, 128, None, 0, True), (1000, 37, 128, None, 0, False),
@@ -243,7 +271,7 @@ def test_keys_rotated_in_place(D, H, T, surplus, pad):
     # eighths of a pair, with and without a remainder, none
     (7700, 13, 128, 200, 3, False), (7400, 14, 128, 200, 3, False), (12000, 12, 64, 1000, 3, False), (1000, 110, 128, 120, 3, False),
 ])
-def test_prefill_on_both_sides_of_the_block_size_rule(T, H, D, window, docs, split):
+def test_prefill_block_size_rule_and_every_head(T, H, D, window, docs, split):
     """Sizes around the numbers of blocks at which the kernel with 32 queries per workgroup hands over to the one with 128 (the rule itself is
     asked which), and pairs that are no multiple of eight; the first rows, some of every block and the last ones against the oracle."""
     wanted = _lib.load()._ZN5daisy20prefill_split_wantedEiiiib

@@ -70,10 +70,25 @@ def test_products_on_both_sides_of_the_smallest_tiles_rule(M):
             assert torch.equal(y, _lib.native().linear(x, w, None, 4, tile))
 
 
-@pytest.mark.parametrize("M,N,K,own", [(999, 6144, 576, False), (1000, 6144, 576, True), (6009, 1024, 576, False), (6017, 1024, 576, True), (8192, 1024, 576, True),
-                                       (8193, 1024, 576, False), (6017, 1024, 1024, True), (4608, 1536, 1088, False), (4609, 1536, 1088, True), (4609, 1536, 1536, True),
+@pytest.mark.parametrize("M,N,own", [(999, 6144, False), (1000, 6144, True), (6009, 1024, False), (6017, 1024, True), (8192, 1024, True), (8193, 1024, False)])
+def test_large_products_on_both_sides_of_the_rule(M, N, own):
+    """From 384 to 512 tiles of 128 x 128 and 1000 rows on; the few rows compared are the first, the last and some of every row of tiles."""
+    K = 576
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g).bfloat16(), torch.randn(N, K, generator=g).bfloat16()
+    with torch.no_grad():
+        y = _lib.native().linear(x.to(DEV), w.to(DEV), None, 4, 0)
+    assert (y is not None) == own
+    if own:
+        rows = torch.cat([torch.arange(0, M, 61), torch.tensor([M - 1])])
+        r = x[rows].double() @ w.double().t()
+        err = (y[rows.to(DEV)].cpu().double() - r).abs()
+        assert (err <= r.abs() * 2 ** -8 + K ** 0.5 * 1e-5 + 1e-3).all(), err.max().item()
+
+
+@pytest.mark.parametrize("M,N,K,own", [(6017, 1024, 1024, True), (4608, 1536, 1088, False), (4609, 1536, 1088, True), (4609, 1536, 1536, True),
                                        (4609, 1536, 1600, False), (4096, 2048, 2048, False), (24576, 256, 1024, True), (49152, 128, 1024, False)])
-def test_large_products_on_both_sides_of_the_rule(M, N, K, own):
+def test_large_products_of_long_rows_and_one_column_of_tiles(M, N, K, own):
     """From 384 (rows of more than 1024: 440) to 512 tiles of 128 x 128, two columns of them and 1000 rows on; the few rows compared are the
     first, the last and some of every row of tiles."""
     g = torch.Generator().manual_seed(M)
