@@ -1096,9 +1096,8 @@ __global__ __launch_bounds__(kStateThreads<KCT>, 1) void kda_state_kernel(KdaPar
 // equal (0.18) 91.9 / 82.5, the longest a fifth (0.57) 93.1 / 88.7, cut at random (0.78) 97.4 / 99.5, the longest two fifths (1.1) 95.6 / 120, nearly all (2.8) 149 / 204;
 // T = 16000, cut at random (0.68) 238 / 228, 8 heads (1.4) 142 / 159; 33 sequences, T = 6000, at random (0.53) 114 / 95, the longest two fifths (0.89) 118 / 123, 8 heads,
 // at random (1.0) 62 / 72, T = 16000 (0.64) 151 / 149.  (Not for key heads of 64: of their groups of 32 two workgroups fit a compute unit, of this kernel one.)
-template <bool BY_LENGTH>
+template <int KD, bool BY_LENGTH>
 __global__ __launch_bounds__(kStateThreads<4>, 1) void kda_packed_state_kernel(KdaParams p) {
-  constexpr int KD = 128;
   __shared__ __attribute__((aligned(1024))) StageLds<KD, 4> stage;
   __shared__ __attribute__((aligned(16))) StateLds<KD, 4> xs;
   __shared__ __attribute__((aligned(16))) XLds<4> xx;
@@ -1210,9 +1209,9 @@ static int kda_launch_width(const KdaParams& p, int n_streams, hipStream_t s) {
     // average.  Where the longest one comes early anyway ranking costs (12 of 12000, 16 of 64 95.5 -> 97.3): 0.03 us a sequence in every workgroup, so
     // only up to a tenth of a mean chain (else 16 of T = 2088, 8 heads of 128 34.5 -> 35.5, 13 of 148, 12 heads 18.2 -> 19.8); not where they are in that order.
     const bool by_length = chains > 256 && p.n_seq > 1 && p.n_seq <= kScanSeqs && p.NC >= p.n_seq * p.n_seq;
-    const bool either = KD == 128 && p.n_seq <= kScanSeqs && streams * narrow > 256 && p.Dv % (4 * KVS) == 0;
-    if (either && by_length) hipLaunchKernelGGL(kda_packed_state_kernel<true>, dim3(chains), dim3(kStateThreads<4>), 0, s, p);
-    else if (either) hipLaunchKernelGGL(kda_packed_state_kernel<false>, dim3(chains), dim3(kStateThreads<4>), 0, s, p);
+    const bool either = p.n_seq <= kScanSeqs && streams * narrow > 256 && p.Dv % (4 * KVS) == 0;
+    if (either && by_length) hipLaunchKernelGGL((kda_packed_state_kernel<KD, true>), dim3(chains), dim3(kStateThreads<4>), 0, s, p);
+    else if (either) hipLaunchKernelGGL((kda_packed_state_kernel<KD, false>), dim3(chains), dim3(kStateThreads<4>), 0, s, p);
     else if (by_length) hipLaunchKernelGGL((kda_state_kernel<KD, 2, true>), dim3(chains), dim3(kStateThreads<2>), 0, s, p);
     else hipLaunchKernelGGL((kda_state_kernel<KD, 2, false>), dim3(chains), dim3(kStateThreads<2>), 0, s, p);
   }
