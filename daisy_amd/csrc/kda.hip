@@ -161,6 +161,17 @@ __device__ __forceinline__ SeqScan packed_scan(const KdaParams& p) {
   }
   return c;
 }
+// A lane's sequence's rank by length, the longest has 0, equal ones in their order; the sequence of a rank.
+__device__ __forceinline__ int length_rank(const KdaParams& p, const SeqScan& c) {
+  const uint32_t mine = ((uint32_t)c.nc << 6) + 63 - (threadIdx.x & 63);          // (no two the same)
+  int ahead = 0;
+#pragma unroll 4
+  for (int j = 0; j < p.n_seq; ++j) ahead += (uint32_t)__builtin_amdgcn_readlane((int)mine, j) > mine ? 1 : 0;
+  return ahead;
+}
+__device__ __forceinline__ int sequence_ranked(const KdaParams& p, int rank, int which) {
+  return __builtin_ctzll(__ballot((int)(threadIdx.x & 63) < p.n_seq && rank == which));
+}
 template <bool BY_LENGTH> __device__ __forceinline__ SeqSpan scanned_span(const KdaParams& p, const SeqScan& c, int& key, bool by_slot, int& rows_end) {
   SeqSpan s{0, 0, 0, 0};
   const int lane = threadIdx.x & 63;
@@ -172,13 +183,7 @@ template <bool BY_LENGTH> __device__ __forceinline__ SeqSpan scanned_span(const 
   }
   if constexpr (BY_LENGTH) {
     const int before = __shfl_up(c.nc, 1);
-    if (__ballot(c.nc > before && lane > 0) != 0) {                     // (not in that order already)
-      const uint32_t mine = ((uint32_t)c.nc << 6) + 63 - lane;          // (no two the same)
-      int ahead = 0;
-#pragma unroll 4
-      for (int j = 0; j < p.n_seq; ++j) ahead += (uint32_t)__builtin_amdgcn_readlane((int)mine, j) > mine ? 1 : 0;
-      key = __builtin_ctzll(__ballot(lane < p.n_seq && ahead == key));
-    }
+    if (__ballot(c.nc > before && lane > 0) != 0) key = sequence_ranked(p, length_rank(p, c), key);      // (not in that order already)
   }
   s.tok0 = __builtin_amdgcn_readlane(c.begin, key); s.tok_end = __builtin_amdgcn_readlane(c.end, key);
   s.nc = __builtin_amdgcn_readlane(c.nc, key); s.c0 = __builtin_amdgcn_readlane(c.upto, key) - s.nc;
@@ -1092,10 +1097,14 @@ __global__ __launch_bounds__(kStateThreads<KCT>, 1) void kda_state_kernel(KdaPar
 
 // Up to kScanSeqs packed sequences in groups of 64 columns or of 32, as their lengths, which only the device knows, want it: 64 where the
 // longest chain, whose links they lengthen, is no more than three quarters of the links of 32 that fall to a compute unit, each chain counted for four more that it
-// takes to start.  Columns come in whole groups of 64; the grid is that of 32.  us, 32 / 64 columns (that ratio), heads of 128: 16 sequences, 16 heads, T = 6000,
+// takes to start, or three quarters of the 256th and 257th longest together, one of which has to wait for the other (with up to one and a half rounds of chains, where that
+// is more than the share, and where ranking them, 1 us, is worth it: 9 sequences, 16 heads of 64 x 64, T = 16000, equal, 288 chains of 32, 139 -> 117, T = 9000 67.2 -> 58.9, 12 of
+// 14000, 8 heads of 128 114 -> 105; with it at 512 chains 16 of 3000, 16 heads of 64 x 64, at random 31.9 -> 34.1).  Columns come in whole groups of 64; the grid is that of 32.  us, 32 / 64 columns (that ratio), heads of 128: 16 sequences, 16 heads, T = 6000,
 // equal (0.18) 91.9 / 82.5, the longest a fifth (0.57) 93.1 / 88.7, cut at random (0.78) 97.4 / 99.5, the longest two fifths (1.1) 95.6 / 120, nearly all (2.8) 149 / 204;
 // T = 16000, cut at random (0.68) 238 / 228, 8 heads (1.4) 142 / 159; 33 sequences, T = 6000, at random (0.53) 114 / 95, the longest two fifths (0.89) 118 / 123, 8 heads,
-// at random (1.0) 62 / 72, T = 16000 (0.64) 151 / 149.  (Not for key heads of 64: of their groups of 32 two workgroups fit a compute unit, of this kernel one.)
+// at random (1.0) 62 / 72, T = 16000 (0.64) 151 / 149.  Key heads of 64, of whose groups of 32 two workgroups fit a compute unit, of this kernel one (32 by their own
+// kernel / 64 / this kernel): 16 sequences, 16 heads of 64 x 128, T = 16000, equal 147 / 126 / 127, the longest two fifths 177 / 199 / 177, nearly all 298 / 343 / 299; 12 heads, T = 9000, cut
+// at random 65.8 / 72.5 / 66.7, a fourth 65.8 / 76.9 / 68.2; T = 3000, equal 30.3 / 29.3 / 29.9, a fourth 31.8 / 32.6 / 34.2.
 template <int KD, bool BY_LENGTH>
 __global__ __launch_bounds__(kStateThreads<4>, 1) void kda_packed_state_kernel(KdaParams p) {
   __shared__ __attribute__((aligned(1024))) StageLds<KD, 4> stage;
@@ -1106,14 +1115,20 @@ __global__ __launch_bounds__(kStateThreads<4>, 1) void kda_packed_state_kernel(K
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) longest = max(longest, __shfl_xor(longest, off));
   longest = __builtin_amdgcn_readfirstlane(longest);
-  const int64_t links = (int64_t)(__builtin_amdgcn_readlane(scan.upto, 63) + 4 * p.n_seq) * p.H * (p.Dv / (2 * KVS));
+  const int groups = p.H * (p.Dv / (2 * KVS));       // a sequence's chains of 32 columns
+  int64_t share = (int64_t)(__builtin_amdgcn_readlane(scan.upto, 63) + 4 * p.n_seq) * groups;       // 256 times
+  if (BY_LENGTH && p.n_seq * groups <= 384) {
+    const int rank = length_rank(p, scan);
+    share = max(share, (int64_t)256 * (__builtin_amdgcn_readlane(scan.nc, sequence_ranked(p, rank, 255 / groups)) +
+                                       __builtin_amdgcn_readlane(scan.nc, sequence_ranked(p, rank, 256 / groups))));
+  }
   auto chain = [&](auto columns) {
     constexpr int KCT = decltype(columns)::value;
     if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= kStateThreads<KCT>) return;
     kda_chain<KD, KCT, BY_LENGTH>(p, reinterpret_cast<StageLds<KD, KCT>&>(stage), reinterpret_cast<StateLds<KD, KCT>&>(xs), reinterpret_cast<XLds<KCT>&>(xx),
                                   [&](int& b, int& rows_end) { return scanned_span<BY_LENGTH>(p, scan, b, false, rows_end); });
   };
-  if (longest * (int64_t)(256 * 4) <= 3 * links) chain(std::integral_constant<int, 4>{});
+  if (longest * (int64_t)(256 * 4) <= 3 * share) chain(std::integral_constant<int, 4>{});
   else chain(std::integral_constant<int, 2>{});
 }
 

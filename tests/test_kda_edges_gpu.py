@@ -176,6 +176,14 @@ def test_kda_packed_wide_column_groups(lengths, H, D, Dv):
             assert not S[i].any()
 
 
+# ... of one to one and a half rounds, where the 256th and 257th longest chain decide too: alike, all but one alike, one long.
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("lengths", [(300, 310, 290, 305, 333, 300, 281, 299, 320), (300,) * 4 + (7,) + (410,) * 4, (90, 0, 150, 2000, 33, 64, 100, 31, 160)])
+def test_kda_packed_wide_column_groups_of_two_rounds(lengths, D):
+    assert 256 < len(lengths) * 16 * 2 <= 384 and sum((m + 31) // 32 for m in lengths) >= len(lengths) ** 2
+    test_kda_packed_wide_column_groups(lengths, 16, D, 64)
+
+
 # The blocks themselves, all of their bytes, from call to call: a 16-byte store's data registers written again by the next instruction
 # changed the low terms of rows 28 .. 31 of M in 2 % of the blocks, which only those of the last chunk show in a result, and by an ulp.
 @pytest.mark.parametrize("T,H,D", [(3712, 8, 128), (3712, 12, 64)])
