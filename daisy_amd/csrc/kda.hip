@@ -1097,7 +1097,7 @@ __global__ __launch_bounds__(kStateThreads<KCT>, 1) void kda_state_kernel(KdaPar
 
 // Up to kScanSeqs packed sequences in groups of 64 columns or of 32, as their lengths, which only the device knows, want it: 64 where the
 // longest chain, whose links they lengthen, is no more than three quarters of the links of 32 that fall to a compute unit, each chain counted for four more that it
-// takes to start, or three quarters of the 256th and 257th longest together, one of which has to wait for the other (with up to one and a half rounds of chains, where that
+// takes to start, or three quarters of the 256th and 257th longest together, one of which has to wait for the other and then start (with up to one and a half rounds of chains, where that
 // is more than the share, and where ranking them, 1 us, is worth it: 9 sequences, 16 heads of 64 x 64, T = 16000, equal, 288 chains of 32, 139 -> 117, T = 9000 67.2 -> 58.9, 12 of
 // 14000, 8 heads of 128 114 -> 105; with it at 512 chains 16 of 3000, 16 heads of 64 x 64, at random 31.9 -> 34.1).  Columns come in whole groups of 64; the grid is that of 32.  us, 32 / 64 columns (that ratio), heads of 128: 16 sequences, 16 heads, T = 6000,
 // equal (0.18) 91.9 / 82.5, the longest a fifth (0.57) 93.1 / 88.7, cut at random (0.78) 97.4 / 99.5, the longest two fifths (1.1) 95.6 / 120, nearly all (2.8) 149 / 204;
@@ -1119,7 +1119,7 @@ __global__ __launch_bounds__(kStateThreads<4>, 1) void kda_packed_state_kernel(K
   int64_t share = (int64_t)(__builtin_amdgcn_readlane(scan.upto, 63) + 4 * p.n_seq) * groups;       // 256 times
   if (BY_LENGTH && p.n_seq * groups <= 384) {
     const int rank = length_rank(p, scan);
-    share = max(share, (int64_t)256 * (__builtin_amdgcn_readlane(scan.nc, sequence_ranked(p, rank, 255 / groups)) +
+    share = max(share, (int64_t)256 * (4 + __builtin_amdgcn_readlane(scan.nc, sequence_ranked(p, rank, 255 / groups)) +
                                        __builtin_amdgcn_readlane(scan.nc, sequence_ranked(p, rank, 256 / groups))));
   }
   auto chain = [&](auto columns) {
